@@ -4,7 +4,7 @@
  * Same conventions as ntk.h: plain pointers and sizes, stream ordered, no allocation, NTK_OK or a negative NTK_E_* code.  Nothing here knows a
  * model: every size and constant is a parameter.  Two precisions of one operator set:
  *   weights NTK_DT_BF16 : matrix products on the bf16 matrix cores (activations rounded to bfloat16 at the product's input, F32 accumulation);
- *   weights NTK_DT_F32  : every product in true F32 (FMA on the vector units).
+ *   weights NTK_DT_F32  : every product in true F32 (32-bit matrix instructions; a few rows: FMA on the vector units).
  * Norms, rotary angles, attention scores and weights, routers and the residual sum are F32 in both.
  */
 #ifndef NTK_LAYERS_H
@@ -53,6 +53,9 @@ typedef struct ntk_dense_desc {
      * launch: what a sublayer still owes to the stream joins it on the way into the next sublayer's first product */
     const float* add_y; int ld_add; const float* add_w; float add_eps, add_mult;
     float* x_out; int ldxo;
+    /* room for partial sums (16-byte aligned, scratch_bytes of it; NULL: none): with more than ntk_dense_few_rows() rows the inputs of a product may be cut into pieces that
+     * run side by side, as many as the room holds ([pieces][T][N] floats).  Products on different streams need scratch of their own. */
+    float* scratch; size_t scratch_bytes;
 } ntk_dense_desc;
 #define NTK_ACT_NONE 0
 #define NTK_ACT_RELU2 1

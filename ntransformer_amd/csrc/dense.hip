@@ -1,23 +1,18 @@
 // dense.hip -- products with dense weight matrices (bfloat16 or float32, row-major [out][in]) for the layer-list model families.
 //
-// One entry point for a product (ntk_dense) with three kernel forms behind it:
-//   * dense_mfma_kernel   bf16 weights, more than kGemvRows rows: 128 x 128 / 64 x 128 / 64 x 64 output tiles on v_mfma_f32_16x16x32_bf16; the F32 activations are rounded
-//                         to bfloat16 (nearest even) on their way into LDS, sums stay F32 in the accumulators;
-//   * dense_fma_kernel    float32 weights, more than kGemvRows rows: the same tiling with plain F32 FMAs, k ascending (true 32-bit);
+// One entry point for a product (ntk_dense) with two kernel forms behind it:
+//   * gemm_tile_kernel    more than kGemvRows rows (gemm_tile.hip.h): bf16 weights on v_mfma_f32_16x16x32_bf16, the F32 activations rounded to bfloat16 (nearest even) on
+//                         their way into LDS; float32 weights on v_mfma_f32_16x16x4_f32 (true 32-bit products and sums);
 //   * dense_gemv_kernel   up to kGemvRows rows (decoding): every wave streams a few weight rows at once, 16 bytes per lane and row, the activation
 //                         row sits in LDS; bf16 weights are widened exactly and multiplied in F32.  What runs inside the launch on the way in: what the row is still owed (a
 //                         sublayer's normed output), an RMS norm; on the way out: a gated unit or an activation.
 // Rows can be grouped (a mixture of experts: sorted rows of group g take matrix g) and gathered (row r reads activation row rows[r] / row_div).
 // Group sizes live on the device, so the grid covers the worst case and workgroups outside their group's range leave at once.
 // A second entry point (ntk_moe_few) runs all of a few tokens' chosen experts, the shared unit and their weighted sum in two row-streaming launches.
-#include "common.hip.h"
+#include "gemm_tile.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float floatx4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t uintx4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {   // round to nearest even; NaN stays NaN
     uint32_t u = __float_as_uint(f);
@@ -40,197 +35,9 @@ struct DenseArgs {
     const float* add_y; int ld_add; const float* add_w; float add_eps, add_mult; float* x_out; int ldxo;   // few-row form only: see ntk_dense_desc
 };
 
-__device__ __forceinline__ bool group_range(const DenseArgs& a, int g, int& r0, int& r1) {
-    if (a.offsets) { r0 = a.offsets[g]; r1 = a.offsets[g + 1]; } else { r0 = 0; r1 = a.T; }
-    return r1 > r0;
-}
-
 __device__ __forceinline__ float activate(float v, int act) {
     if (act == NTK_ACT_RELU2) { const float p = fmaxf(v, 0.0f); return p * p; }
     return v;
-}
-
-// ---------------------------------------------------------------------------------------------------------------- bf16, matrix cores
-// A workgroup of four waves (2 x 2) owns a TM x TN tile of Y; a wave owns (TM / 2) x (TN / 2) of it as 16 x 16 accumulator tiles.  K goes by in chunks
-// of 32: the NEXT chunk's operands are requested into registers before the current one is multiplied out of LDS (global latency behind the MFMAs),
-// activations are rounded to bfloat16 (nearest even, the hardware conversion) on their way into LDS.
-constexpr int BK = 32, LDSK = BK + 8;   // LDS rows of 40 bf16 = 80 bytes: 16-byte aligned operand reads, rows 20 banks apart
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float floatx2_t __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    const bf16x2_t v = __builtin_convertvector(floatx2_t{a, b}, bf16x2_t);
-    uint32_t u;
-    __builtin_memcpy(&u, &v, 4);
-    return u;
-}
-
-template <int TM, int TN, bool VEC>
-__global__ __launch_bounds__(256) void dense_mfma_kernel(const DenseArgs a) {
-    constexpr int PX = TM / 64, PW = TN / 64;        // loader passes of 64 rows
-    constexpr int MI = TM / 32, NJ = TN / 32;        // 16 x 16 tiles per wave
-    int r0, r1;
-    if (!group_range(a, blockIdx.z, r0, r1)) return;
-    const int row_base = r0 + blockIdx.y * TM;
-    if (row_base >= r1) return;
-    const int n_base = blockIdx.x * TN;
-    const uint16_t* W = (const uint16_t*)a.W + (long long)blockIdx.z * a.wstride;
-    __shared__ __attribute__((aligned(16))) uint16_t Xs[TM][LDSK];
-    __shared__ __attribute__((aligned(16))) uint16_t Ws[TN][LDSK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    // loader: thread -> (row tid / 4 + 64 * pass, eight k from (tid & 3) * 8)
-    const int lr = tid >> 2, lk = (tid & 3) * 8;
-    const float* xrow[PX];
-    const uint16_t* wrow[PW];
-#pragma unroll
-    for (int p = 0; p < PX; ++p) {
-        const int xr = row_base + lr + 64 * p;
-        xrow[p] = xr < r1 ? a.X + (long long)(a.rows ? a.rows[xr] / a.row_div : xr) * a.ldx : nullptr;
-    }
-#pragma unroll
-    for (int p = 0; p < PW; ++p) {
-        const int wr = n_base + lr + 64 * p;
-        wrow[p] = wr < a.N ? W + (long long)wr * a.K : nullptr;
-    }
-    floatx4_t acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    uintx4_t xreg[PX], wreg[PW];
-    auto fetch = [&](int k0) {
-        const int k = k0 + lk;
-#pragma unroll
-        for (int p = 0; p < PX; ++p) {
-            xreg[p] = uintx4_t{0u, 0u, 0u, 0u};
-            if (xrow[p]) {
-                if (VEC) {
-                    if (k < a.K) {
-                        const float4 v0 = *reinterpret_cast<const float4*>(xrow[p] + k), v1 = *reinterpret_cast<const float4*>(xrow[p] + k + 4);
-                        xreg[p] = uintx4_t{pack_bf16(v0.x, v0.y), pack_bf16(v0.z, v0.w), pack_bf16(v1.x, v1.y), pack_bf16(v1.z, v1.w)};
-                    }
-                } else {
-                    float v[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) v[j] = k + j < a.K ? xrow[p][k + j] : 0.0f;
-                    xreg[p] = uintx4_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
-                }
-            }
-        }
-#pragma unroll
-        for (int p = 0; p < PW; ++p) {
-            wreg[p] = uintx4_t{0u, 0u, 0u, 0u};
-            if (wrow[p]) {
-                if (VEC) {
-                    if (k < a.K) wreg[p] = *reinterpret_cast<const uintx4_t*>(wrow[p] + k);
-                } else {
-                    uint32_t v[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) v[j] = k + j < a.K ? (uint32_t)wrow[p][k + j] : 0u;
-                    wreg[p] = uintx4_t{v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
-                }
-            }
-        }
-    };
-    fetch(0);
-    for (int k0 = 0; k0 < a.K; k0 += BK) {
-        __syncthreads();   // the previous chunk's operand reads are done
-#pragma unroll
-        for (int p = 0; p < PX; ++p) *reinterpret_cast<uintx4_t*>(&Xs[lr + 64 * p][lk]) = xreg[p];
-#pragma unroll
-        for (int p = 0; p < PW; ++p) *reinterpret_cast<uintx4_t*>(&Ws[lr + 64 * p][lk]) = wreg[p];
-        __syncthreads();
-        if (k0 + BK < a.K) fetch(k0 + BK);
-        bf16x8_t af[MI], bfr[NJ];
-#pragma unroll
-        for (int i = 0; i < MI; ++i) af[i] = *reinterpret_cast<const bf16x8_t*>(&Xs[wm * (TM / 2) + i * 16 + (lane & 15)][(lane >> 4) * 8]);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) bfr[j] = *reinterpret_cast<const bf16x8_t*>(&Ws[wn * (TN / 2) + j * 16 + (lane & 15)][(lane >> 4) * 8]);
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    }
-    // accumulator lane map: row 4 * (lane / 16) + r, column lane % 16.  What a sum is added onto is requested for a whole strip of tiles before the first store.
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        const int row = row_base + wm * (TM / 2) + i * 16 + (lane >> 4) * 4;
-        float* y = a.Y + (long long)row * a.ldy + n_base + wn * (TN / 2) + (lane & 15);
-        const int n_left = a.N - (n_base + wn * (TN / 2) + (lane & 15));
-        if (a.accumulate) {                                  // (uniform over the launch)
-            float old[NJ][4];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) old[j][r] = row + r < r1 && j * 16 < n_left ? y[(long long)r * a.ldy + j * 16] : 0.0f;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][j][r] += old[j][r];
-        }
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (row + r < r1 && j * 16 < n_left) y[(long long)r * a.ldy + j * 16] = activate(acc[i][j][r], a.act);
-    }
-}
-
-// ---------------------------------------------------------------------------------------------------------------- float32, vector FMA
-constexpr int FK = 16, TM = 64, TN = 64;
-__global__ __launch_bounds__(256) void dense_fma_kernel(const DenseArgs a) {
-    int r0, r1;
-    if (!group_range(a, blockIdx.z, r0, r1)) return;
-    const int row_base = r0 + blockIdx.y * TM;
-    if (row_base >= r1) return;
-    const int n_base = blockIdx.x * TN;
-    const float* W = (const float*)a.W + (long long)blockIdx.z * a.wstride;
-    __shared__ __attribute__((aligned(16))) float Xs[FK][TM + 4];
-    __shared__ __attribute__((aligned(16))) float Ws[FK][TN + 4];
-    const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-    const int lr = tid >> 2, lk = (tid & 3) * 4;
-    const int xr = row_base + lr;
-    const bool x_ok = xr < r1;
-    const float* xrow = nullptr;
-    if (x_ok) xrow = a.X + (long long)(a.rows ? a.rows[xr] / a.row_div : xr) * a.ldx;
-    const int wr = n_base + lr;
-    const bool w_ok = wr < a.N;
-    const float* wrow = W + (long long)wr * a.K;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < a.K; k0 += FK) {
-        float xv[4], wv[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int k = k0 + lk + j;
-            xv[j] = (x_ok && k < a.K) ? xrow[k] : 0.0f;
-            wv[j] = (w_ok && k < a.K) ? wrow[k] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { Xs[lk + j][lr] = xv[j]; Ws[lk + j][lr] = wv[j]; }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < FK; ++k) {
-            const float4 xa = *reinterpret_cast<const float4*>(&Xs[k][ty * 4]);
-            const float4 wa = *reinterpret_cast<const float4*>(&Ws[k][tx * 4]);
-            const float xs[4] = {xa.x, xa.y, xa.z, xa.w}, ws[4] = {wa.x, wa.y, wa.z, wa.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(xs[i], ws[j], acc[i][j]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = row_base + ty * 4 + i, col = n_base + tx * 4 + j;
-            if (row < r1 && col < a.N) {
-                float* y = a.Y + (long long)row * a.ldy + col;
-                *y = a.accumulate ? *y + acc[i][j] : activate(acc[i][j], a.act);
-            }
-        }
 }
 
 // ---------------------------------------------------------------------------------------------------------------- few rows: waves stream weight rows
@@ -674,27 +481,31 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
         else launch_gemv<float, false>(a, d->T, s);
         return last_launch_status();
     }
-    if (d->wdtype == NTK_DT_BF16) {
-        const bool vec = (d->K % 8 == 0) && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->W & 15) && (d->wstride % 8 == 0);
-        // 128 x 128 tiles where a group has the rows and the launch still fills the chip; 64-row tiles for short groups (experts, short portions)
-        const int rows_per_group = d->T / G;
-        const bool big = rows_per_group >= 192 && d->N >= 128 && (long long)((d->T + 127) / 128) * ((d->N + 127) / 128) >= 224;
-        if (big) {
-            const dim3 grid((d->N + 127) / 128, (d->T + 127) / 128, G);
-            if (vec) hipLaunchKernelGGL((dense_mfma_kernel<128, 128, true>), grid, dim3(256), 0, s, a);
-            else hipLaunchKernelGGL((dense_mfma_kernel<128, 128, false>), grid, dim3(256), 0, s, a);
-        } else if (d->N >= 128) {
-            const dim3 grid((d->N + 127) / 128, (d->T + 63) / 64, G);
-            if (vec) hipLaunchKernelGGL((dense_mfma_kernel<64, 128, true>), grid, dim3(256), 0, s, a);
-            else hipLaunchKernelGGL((dense_mfma_kernel<64, 128, false>), grid, dim3(256), 0, s, a);
-        } else {
-            const dim3 grid((d->N + 63) / 64, (d->T + 63) / 64, G);
-            if (vec) hipLaunchKernelGGL((dense_mfma_kernel<64, 64, true>), grid, dim3(256), 0, s, a);
-            else hipLaunchKernelGGL((dense_mfma_kernel<64, 64, false>), grid, dim3(256), 0, s, a);
-        }
+    const bool bf = d->wdtype == NTK_DT_BF16;
+    TileArgs t{};
+    t.Y = d->Y; t.ldy = d->ldy; t.X = d->X; t.ldx = d->ldx; t.W = d->W; t.wstride = d->wstride; t.offsets = d->offsets; t.G = G; t.rows = d->rows; t.row_div = a.row_div;
+    t.T = d->T; t.N = d->N; t.K = d->K; t.accumulate = d->accumulate; t.act = d->act; t.part = d->scratch;
+    const int align = bf ? 8 : 4;
+    const bool vec = (d->K % align == 0) && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->W & 15) && (d->wstride % align == 0);
+    if (!vec) {                            // (odd sizes and addresses: element by element into the same tiles)
+        if (bf) launch_tiles<TileBf16, 64, 64, 2, 2, 2, false>(t, 1, s);
+        else launch_tiles<TileF32, 64, 64, 2, 2, 2, false>(t, 1, s);
+        return last_launch_status();
+    }
+    // (no pieces for grouped rows: rows that belong to no group stay untouched)
+    const long long room = d->scratch && !((uintptr_t)d->scratch & 15) && !d->offsets && d->T <= 65535 ? (long long)(d->scratch_bytes / sizeof(float)) : 0;
+    if (bf) {
+        static const TileForm forms[] = {{128, 128, 32, 0.65f, 0.43f}, {64, 128, 64, 0.80f, 0.68f}, {64, 64, 64, 0.70f, 0.35f}, {32, 64, 64, 0.60f, 0.22f}};
+        const TilePlan p = plan_tiles(forms, 4, d->T, G, d->N, d->K, room);
+        if (p.form == 0) launch_tiles<TileBf16, 128, 128, 1, 4, 2, true>(t, p.splits, s);
+        else if (p.form == 1) launch_tiles<TileBf16, 64, 128, 2, 2, 4, true>(t, p.splits, s);
+        else if (p.form == 2) launch_tiles<TileBf16, 64, 64, 2, 2, 2, true>(t, p.splits, s);
+        else launch_tiles<TileBf16, 32, 64, 2, 2, 2, true>(t, p.splits, s);
     } else {
-        const dim3 grid((d->N + TN - 1) / TN, (d->T + TM - 1) / TM, G);
-        hipLaunchKernelGGL(dense_fma_kernel, grid, dim3(256), 0, s, a);
+        static const TileForm forms[] = {{64, 64, 32, 0.78f, 0.70f}, {32, 64, 32, 0.52f, 0.36f}};
+        const TilePlan p = plan_tiles(forms, 2, d->T, G, d->N, d->K, room);
+        if (p.form == 0) launch_tiles<TileF32, 64, 64, 2, 2, 2, true>(t, p.splits, s);
+        else launch_tiles<TileF32, 32, 64, 2, 2, 2, true>(t, p.splits, s);
     }
     return last_launch_status();
 }

@@ -1001,6 +1001,9 @@ int LayerStackModel::alloc_buffers() {
              fl(&cv_, C * std::max(max_conv_, 1)) && fl(&vfirst_, C * std::max(max_gv_, 1));
     if (form_.post_norm) ok = ok && fl(&ff_, C * W) && fl(&zf_, C * std::max(max_ffn_, 1)) && fl(&gu2_, C * 2 * std::max(max_ffn_, 1)) && fl(&wscratch_, wsc) && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_) && fl(&rz_, (size_t)ntk_dense_few_rows() * (max_e_ + 1));
     if (form_.dense_parallel) ok = ok && fl(&gu2_, C * 2 * std::max(max_ffn_, 1)) && fl(&wscratch_, wsc);
+    // four pieces of a whole pass's rows, and no less than sixteen of a short one's
+    pscratch_bytes_ = std::max<size_t>(4 * C * W, (size_t)1 << 22) * sizeof(float);
+    ok = ok && fl(&pscratch_, pscratch_bytes_ / sizeof(float));
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
     h_stage_ = (int*)nt_hip_malloc_host(2 * C * sizeof(int));
     ok = ok && h_stage_ != nullptr;
@@ -1062,7 +1065,7 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
         d.Y = q_; d.ldy = H * qd; d.X = few ? a_ : cq_; d.ldx = few ? na : m.q_rank; d.W = m.uq.ptr; d.wdtype = m.uq.dtype; d.N = H * qd; d.K = m.q_rank;
         if (few) { d.norm_w = m.q_norm; d.norm_offset = 0.0f; }
         else LS_TRY(ntk_rmsnorm_offset(cq_, m.q_norm, nullptr, nullptr, m.q_rank, a_, na, T, m.q_rank, eps_, 0.0f, stream_));
-        LS_TRY(ntk_dense(&d, stream_));
+        LS_TRY(product(d));
         q = q_;
         ldq = H * qd;
     }
@@ -1079,14 +1082,14 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
     } else {
         const int key0 = m.window > 0 ? std::max(0, pos0 - m.window + 1) : 0;
         const int nkeys = pos0 + T - key0;
-        LS_TRY(ntk_dense_linear(kx_, H * m.dim, cache + (size_t)key0 * row, row, m.uk.ptr, m.uk.dtype, nkeys, H * m.dim, m.kv_rank, 0, stream_));
-        LS_TRY(ntk_dense_linear(vx_, hv, cache + (size_t)key0 * row, row, m.uv.ptr, m.uv.dtype, nkeys, hv, m.kv_rank, 0, stream_));
+        LS_TRY(linear(kx_, H * m.dim, cache + (size_t)key0 * row, row, m.uk.ptr, m.uk.dtype, nkeys, H * m.dim, m.kv_rank, 0));
+        LS_TRY(linear(vx_, hv, cache + (size_t)key0 * row, row, m.uv.ptr, m.uv.dtype, nkeys, hv, m.kv_rank, 0));
         LS_TRY(ntk_latent_attention(att_, hv, q, ldq, kx_, H * m.dim, vx_, hv, cache, row, m.kv_rank, m.rot_dim, H, m.dim, m.vdim, 0, pos0, T, key0, m.window, m.scale,
                                     nullptr, stream_));
         if (m.head_gate) LS_TRY(ntk_head_gate(att_, hv, a_ + m.g_off, na, T, H, m.vdim, stream_));
         else LS_TRY(ntk_sigmoid_gate(att_, hv, a_ + m.g_off, na, T, hv, stream_));
     }
-    return ntk_dense_linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0, stream_);
+    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
 // the window mixer: one product for [q | k | v], rotation and cache rows, attention over the window, output projection -> mix_
@@ -1097,7 +1100,7 @@ int LayerStackModel::run_window(const StackLayer& L, const float* h, float* cach
     d.Y = a_; d.ldy = na; d.X = h; d.ldx = W; d.W = m.in.ptr; d.wdtype = m.in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = na; d.K = W;
     LS_TRY(first_product(d));
     LS_TRY(window_heads(m, cache, att_, hv, T, pos0));
-    return ntk_dense_linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0, stream_);
+    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
 // what lies between the window mixer's two products: norms, rotation and cache rows, then the attention with its gate -> out [T][heads * vdim]
@@ -1136,33 +1139,33 @@ int LayerStackModel::dense_parallel_layer(const Run& run, const StackLayer& L, i
     ntk_dense_desc d{};
     d.Y = a_; d.ldy = na; d.X = few ? x_ : h1_; d.ldx = W; d.W = m.in.ptr; d.wdtype = m.in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = na; d.K = W;
     if (few) { d.norm_w = L.norm1.w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }
-    LS_TRY(ntk_dense(&d, stream_));
+    LS_TRY(product(d));
     if (ff) {
         d.W = L.cff.gate_up.ptr; d.wdtype = L.cff.gate_up.dtype; d.N = 2 * ff;
         if (few) {
             d.Y = att_ + hv; d.ldy = no; d.norm_w = L.norm2.w;
             d.glu_ff = ff; d.glu_limit = L.cff.limit; d.glu_alpha = 1.0f; d.glu_up_offset = 0.0f;
-            LS_TRY(ntk_dense(&d, stream_));
+            LS_TRY(product(d));
         } else {
             d.Y = gu2_; d.ldy = 2 * ff; d.X = h2_;
-            LS_TRY(ntk_dense(&d, stream_));
+            LS_TRY(product(d));
             LS_TRY(ntk_glu_rows(att_ + hv, no, gu2_, 2 * ff, T, ff, L.cff.limit, 1.0f, 0.0f, 0.0f, stream_));
         }
     }
     LS_TRY(window_heads(m, run.cache + (size_t)slot * opt_.max_context * m.row(), att_, no, T, pos0));
-    if (L.out.ptr) return ntk_dense_linear(x_, W, att_, no, L.out.ptr, L.out.dtype, T, W, no, 1, stream_);
-    LS_TRY(ntk_dense_linear(x_, W, att_, no, m.o.ptr, m.o.dtype, T, W, hv, 1, stream_));
-    return ff ? ntk_dense_linear(x_, W, att_ + hv, no, L.cff.down.ptr, L.cff.down.dtype, T, W, ff, 1, stream_) : NTK_OK;
+    if (L.out.ptr) return linear(x_, W, att_, no, L.out.ptr, L.out.dtype, T, W, no, 1);
+    LS_TRY(linear(x_, W, att_, no, m.o.ptr, m.o.dtype, T, W, hv, 1));
+    return ff ? linear(x_, W, att_ + hv, no, L.cff.down.ptr, L.cff.down.dtype, T, W, ff, 1) : NTK_OK;
 }
 
 // the lightning mixer: one product for [q | k | v | gate], the recurrence (silu on the way in), gated RMS norm over the joined heads, output projection -> mix_
 int LayerStackModel::run_lightning(const StackLayer& L, float* state, int T, int pos0) {
     const LightningMixer& m = L.lin;
     const int W = info_.width, na = (int)m.in.out_f, hv = m.heads * m.vdim;
-    LS_TRY(ntk_dense_linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0, stream_));
+    LS_TRY(linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0));
     LS_TRY(ntk_lightning_attention(att_, hv, a_, na, a_ + m.k_off, na, a_ + m.v_off, na, m.log_decay, state, m.heads, m.dim, m.vdim, 1, pos0, T, lscratch_, stream_));
     LS_TRY(ntk_gated_rmsnorm(att_, hv, att_, hv, m.norm, a_ + m.g_off, na, T, hv, eps_, stream_));
-    return ntk_dense_linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0, stream_);
+    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
 int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top) {
@@ -1179,13 +1182,13 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
         LS_TRY(first_product(d));
         d.glu_ff = 0;
     } else {
-        LS_TRY(ntk_dense(&d, stream_));
+        LS_TRY(product(d));
         LS_TRY(ntk_glu(act, gu, rows, ex.ff, ex.limit, glu_alpha, glu_up_offset, stream_));
     }
     d.add_y = nullptr;
     d.Y = out; d.ldy = W; d.X = act; d.ldx = ex.ff; d.W = ex.down.ptr; d.wstride = ex.down.stride(); d.wdtype = ex.down.dtype;
     d.rows = nullptr; d.row_div = 1; d.N = W; d.K = ex.ff;
-    return ntk_dense(&d, stream_);
+    return product(d);
 }
 
 // router, grouping, the experts' products; then either straight into the stream together with the mixer's output (parallel form) or as a sum of its own
@@ -1227,9 +1230,9 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
 int LayerStackModel::run_dense_ff(const StackLayer& L, int T) {
     const DenseFeedForward& D = L.ffn;
     const int W = info_.width;
-    LS_TRY(ntk_dense_linear(zf_, D.ff, h2_, W, D.up.ptr, D.up.dtype, T, D.ff, W, 0, stream_));
+    LS_TRY(linear(zf_, D.ff, h2_, W, D.up.ptr, D.up.dtype, T, D.ff, W, 0));
     LS_TRY(ntk_polynorm(zf_, D.ff, zf_, D.ff, D.act, T, D.ff, eps_, stream_));
-    return ntk_dense_linear(ff_, W, zf_, D.ff, D.down.ptr, D.down.dtype, T, W, D.ff, 0, stream_);
+    return linear(ff_, W, zf_, D.ff, D.down.ptr, D.down.dtype, T, W, D.ff, 0);
 }
 
 // the dense gated unit (the experts' unit with one member, clipped or plain): gate and up in one product (decoding: the activation inside its launch), down -> ff_
@@ -1243,7 +1246,7 @@ int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T) {
 int LayerStackModel::run_gated_delta(const StackLayer& L, float* state, int T, int pos0) {
     const GatedDeltaMixer& m = L.gdl;
     const int W = info_.width, na = (int)m.in.out_f, nc = m.channels(), hv = m.heads * m.vdim;
-    LS_TRY(ntk_dense_linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0, stream_));
+    LS_TRY(linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0));
     ntk_gated_recurrence_desc d{};
     if (T == 1) {   // a decoded token: the convolutions run inside the recurrence's pre-pass
         d.q = a_; d.ldq = na; d.k = a_ + m.k_off; d.ldk = na; d.v = a_ + m.v_off; d.ldv = na;
@@ -1259,7 +1262,7 @@ int LayerStackModel::run_gated_delta(const StackLayer& L, float* state, int T, i
     d.state = state; d.H = m.heads; d.dn = m.dim; d.dv = m.vdim; d.q_scale = 1.0f / std::sqrt((float)m.dim); d.pos0 = pos0; d.T = T; d.scratch = rscratch_;
     LS_TRY(ntk_gated_recurrence(&d, stream_));
     LS_TRY(ntk_head_rmsnorm_gate(att_, hv, att_, hv, m.norm, 0, a_ + m.g_off, na, 2, 1.0f, T, m.heads, m.vdim, eps_, stream_));
-    return ntk_dense_linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0, stream_);
+    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
 // the seam in front of a sublayer of the scaled form: what the stream is still owed joins it (RMS norm, weight, the residual factor), then the norm of the row
@@ -1283,13 +1286,24 @@ int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot,
     return NTK_OK;
 }
 
+// every product of the model: with room for the partial sums of a product whose inputs are cut into pieces
+int LayerStackModel::product(ntk_dense_desc& d) {
+    d.scratch = pscratch_; d.scratch_bytes = pscratch_bytes_;
+    return ntk_dense(&d, stream_);
+}
+int LayerStackModel::linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate) {
+    ntk_dense_desc d{};
+    d.Y = Y; d.ldy = ldy; d.X = X; d.ldx = ldx; d.W = W; d.wdtype = wdtype; d.G = 1; d.row_div = 1; d.T = T; d.N = N; d.K = K; d.accumulate = accumulate;
+    return product(d);
+}
+
 // The first product of a sublayer.  In the post-norm form it reads the stream itself: with few rows, what the stream is still owed joins it inside this launch, which
 // leaves the new stream in the other buffer (its workgroups all read the old one).
 int LayerStackModel::first_product(ntk_dense_desc& d) {
-    if (!form_.post_norm || !owed_.y || d.X != x_) return ntk_dense(&d, stream_);
+    if (!form_.post_norm || !owed_.y || d.X != x_) return product(d);
     const int W = info_.width;
     d.add_y = owed_.y; d.ld_add = W; d.add_w = owed_.nb.w; d.add_eps = eps_; d.add_mult = residual_mult_; d.x_out = x0_; d.ldxo = W;
-    LS_TRY(ntk_dense(&d, stream_));
+    LS_TRY(product(d));
     std::swap(x_, x0_);
     owed_.y = nullptr;
     return NTK_OK;
@@ -1316,15 +1330,15 @@ int LayerStackModel::post_norm_layer(const Run& run, const StackLayer& L, int sl
 int LayerStackModel::run_gla(const StackLayer& L, float* state, int T, int pos0) {
     const GlaMixer& m = L.gla;
     const int W = info_.width, na = (int)m.in.out_f, hq = m.heads * m.dim, hv = m.heads * m.vdim;
-    LS_TRY(ntk_dense_linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0, stream_));
-    LS_TRY(ntk_dense_linear(zq_, hq, a_ + m.a_off, na, m.a2.ptr, m.a2.dtype, T, hq, m.rank, 0, stream_));
+    LS_TRY(linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0));
+    LS_TRY(linear(zq_, hq, a_ + m.a_off, na, m.a2.ptr, m.a2.dtype, T, hq, m.rank, 0));
     ntk_gated_recurrence_desc d{};
     d.out = att_; d.ldo = hv; d.q = a_; d.ldq = na; d.k = a_ + m.k_off; d.ldk = na; d.v = a_ + m.v_off; d.ldv = na;
     d.wz = zq_; d.ldw = hq; d.wb = m.a2_b; d.decay_form = NTK_DECAY_SIGMOID_ROOT; d.decay_param = m.tau;
     d.state = state; d.H = m.heads; d.dn = m.dim; d.dv = m.vdim; d.q_scale = 1.0f / std::sqrt((float)m.dim); d.pos0 = pos0; d.T = T; d.scratch = rscratch_;
     LS_TRY(ntk_gated_recurrence(&d, stream_));
     LS_TRY(ntk_head_rmsnorm_gate(att_, hv, att_, hv, m.norm, 0, a_ + m.g_off, na, 2, 1.0f, T, m.heads, m.vdim, eps_, stream_));
-    return ntk_dense_linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0, stream_);
+    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
 // two mixers over the same input: one product for all their projections and the residual gate; left: biases and the query temperature on the way into the
@@ -1335,7 +1349,7 @@ int LayerStackModel::run_parallel(const StackLayer& L, float* cache, float* stat
     const BiasedAttention& a = m.left;
     const DeltaMixer& r = m.right;
     const int W = info_.width, na = (int)m.in.out_f, hv = a.heads * a.vdim, hd = r.heads * r.dim, no = hv + hd;
-    LS_TRY(ntk_dense_linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0, stream_));
+    LS_TRY(linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0));
     // ---- left
     ntk_rotary rot{nullptr, 1.0f, 0};
     LS_TRY(ntk_window_prepare_biased(cache, a.row(), a_ + a.q_off, na, a_ + a.k_off, na, a_ + a.v_off, na, a.heads, a.kv_heads, 1, a.dim, a.vdim, &rot, a.q_b, a.k_b, a.v_b,
@@ -1348,7 +1362,7 @@ int LayerStackModel::run_parallel(const StackLayer& L, float* cache, float* stat
     LS_TRY(ntk_sigmoid_gate_scaled(att_, no, a_ + a.g_off, na, nullptr, m.left_scale, T, hv, stream_));
     // ---- right
     LS_TRY(ntk_tanh_rows(a_ + r.w1_off, na, T, r.rank, stream_));
-    LS_TRY(ntk_dense_linear(zq_, hd, a_ + r.w1_off, na, r.w2.ptr, r.w2.dtype, T, hd, r.rank, 0, stream_));
+    LS_TRY(linear(zq_, hd, a_ + r.w1_off, na, r.w2.ptr, r.w2.dtype, T, hd, r.rank, 0));
     ntk_gated_recurrence_desc g{};
     g.out = att_ + hv; g.ldo = no; g.q = a_ + r.r_off; g.ldq = na; g.k = a_ + r.k_off; g.ldk = na; g.v = a_ + r.v_off; g.ldv = na;
     g.wz = zq_; g.ldw = hd; g.wb = r.w0; g.decay_form = NTK_DECAY_EXP_SIGMOID; g.decay_param = kDeltaDecayRate;
@@ -1356,7 +1370,7 @@ int LayerStackModel::run_parallel(const StackLayer& L, float* cache, float* stat
     g.state = state; g.H = r.heads; g.dn = r.dim; g.dv = r.dim; g.q_scale = 1.0f; g.pos0 = pos0; g.T = T; g.scratch = rscratch_;
     LS_TRY(ntk_gated_recurrence(&g, stream_));
     LS_TRY(ntk_head_rmsnorm_gate(att_ + hv, no, att_ + hv, no, r.norm, r.dim, a_ + r.g_off, na, 1, m.right_scale, T, r.heads, r.dim, eps_, stream_));
-    return ntk_dense_linear(mix_, W, att_, no, m.o.ptr, m.o.dtype, T, W, no, 0, stream_);
+    return linear(mix_, W, att_, no, m.o.ptr, m.o.dtype, T, W, no, 0);
 }
 
 // gate and up (decoding: the gated unit inside the product's launch) and the residual gate's rows, down -> ff_; the residual gate stays in gu2_ behind them
@@ -1367,14 +1381,14 @@ int LayerStackModel::run_gated_ff(const StackLayer& L, int T) {
         ntk_dense_desc d{};
         d.Y = zf_; d.ldy = ff; d.X = h2_; d.ldx = W; d.W = G.in.ptr; d.wdtype = G.in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = 2 * ff; d.K = W;
         d.glu_ff = ff; d.glu_limit = INFINITY; d.glu_alpha = kGeluAlpha; d.glu_cubic = kGeluCubic; d.glu_up_offset = 0.0f;
-        LS_TRY(ntk_dense(&d, stream_));
+        LS_TRY(product(d));
         const size_t es = G.in.dtype == NTK_DT_BF16 ? 2 : 4;
-        LS_TRY(ntk_dense_linear(gu2_ + 2 * ff, n2, h2_, W, (const char*)G.in.ptr + (size_t)2 * ff * W * es, G.in.dtype, T, W, W, 0, stream_));
+        LS_TRY(linear(gu2_ + 2 * ff, n2, h2_, W, (const char*)G.in.ptr + (size_t)2 * ff * W * es, G.in.dtype, T, W, W, 0));
     } else {
-        LS_TRY(ntk_dense_linear(gu2_, n2, h2_, W, G.in.ptr, G.in.dtype, T, n2, W, 0, stream_));
+        LS_TRY(linear(gu2_, n2, h2_, W, G.in.ptr, G.in.dtype, T, n2, W, 0));
         LS_TRY(ntk_glu_cubic(zf_, gu2_, n2, T, ff, INFINITY, kGeluAlpha, kGeluCubic, 0.0f, stream_));
     }
-    return ntk_dense_linear(ff_, W, zf_, ff, G.down.ptr, G.down.dtype, T, W, ff, 0, stream_);
+    return linear(ff_, W, zf_, ff, G.down.ptr, G.down.dtype, T, W, ff, 0);
 }
 
 // A layer of the gated form.  h1_ holds the first norm of the stream already (the embedding's launch or the previous layer's last seam wrote it).  Every
@@ -1482,7 +1496,7 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, in
         if (x_is_x0 && !run.enters) { LS_TRY(ntk_rows_copy(x_, x0_, (long long)T * W, stream_)); x_is_x0 = false; }
         if (run.enters) {
             LS_TRY(ntk_concat_rows(cat_, x_is_x0 ? x0_ : x_, x0_, T, W, stream_));
-            LS_TRY(ntk_dense_linear(x_, W, cat_, 2 * W, loop_in_.ptr, loop_in_.dtype, T, W, 2 * W, 0, stream_));
+            LS_TRY(linear(x_, W, cat_, 2 * W, loop_in_.ptr, loop_in_.dtype, T, W, 2 * W, 0));
             x_is_x0 = false;
         }
         if (form_.gated) {
@@ -1516,7 +1530,7 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, in
         else if (final_norm_.b) { LS_TRY(ntk_layernorm(hn_, W, rows, W, final_norm_.w, final_norm_.b, n_want, W, eps_, 0, stream_)); d.X = hn_; }
         else if (n_want <= ntk_dense_few_rows()) { d.norm_w = final_norm_.w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }   // the output norm inside the head's launch
         else { LS_TRY(ntk_rmsnorm_offset(hn_, final_norm_.w, nullptr, nullptr, W, rows, W, n_want, W, eps_, norm_offset_, stream_)); d.X = hn_; }
-        LS_TRY(ntk_dense(&d, stream_));
+        LS_TRY(product(d));
         if (logit_softcap_ > 0.0f) LS_TRY(ntk_softcap_rows(logits_out, info_.vocab, logit_softcap_, n_want, info_.vocab, stream_));
         if (logit_scale_ != 1.0f) LS_TRY(ntk_scale(logits_out, (long long)n_want * info_.vocab, logit_scale_, stream_));
     }

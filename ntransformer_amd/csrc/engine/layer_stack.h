@@ -338,6 +338,8 @@ private:
     int norm_conv(const NormW& nw, const float* canon, float* conv_state, float* out, int T, int pos0);
     int settle(int T);
     int first_product(ntk_dense_desc& d);
+    int product(ntk_dense_desc& d);
+    int linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate);
     int sequential_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
 
@@ -376,7 +378,8 @@ private:
     float *x_ = nullptr, *x0_ = nullptr, *cat_ = nullptr, *h1_ = nullptr, *h2_ = nullptr, *a_ = nullptr, *cq_ = nullptr, *q_ = nullptr, *qf_ = nullptr, *lat_ = nullptr,
           *att_ = nullptr, *kx_ = nullptr, *vx_ = nullptr, *mix_ = nullptr, *wts_ = nullptr, *sg_ = nullptr, *gu_ = nullptr, *act_ = nullptr, *dn_ = nullptr,
           *sgu_ = nullptr, *sact_ = nullptr, *sdn_ = nullptr, *scratch_ = nullptr, *xw_ = nullptr, *hn_ = nullptr, *hist_ = nullptr, *ff_ = nullptr, *zf_ = nullptr, *wscratch_ = nullptr, *lscratch_ = nullptr,
-          *results_ = nullptr, *zq_ = nullptr, *gu2_ = nullptr, *rscratch_ = nullptr, *cv_ = nullptr, *vfirst_ = nullptr, *mid_ = nullptr, *rz_ = nullptr;   // gated form: the layer results of the pass [runs + 1][chunk][width], decay pre-activations, [gate | up | residual gate]
+          *results_ = nullptr, *zq_ = nullptr, *gu2_ = nullptr, *rscratch_ = nullptr, *cv_ = nullptr, *vfirst_ = nullptr, *mid_ = nullptr, *rz_ = nullptr, *pscratch_ = nullptr;   // gated form: the layer results of the pass [runs + 1][chunk][width], decay pre-activations, [gate | up | residual gate]
+    size_t pscratch_bytes_ = 0;                  // pscratch_: partial sums of products (ntk_dense_desc::scratch)
     size_t max_mid_ = 0;              // (post-norm form: the experts' activations of a token side by side)
     int max_rec_ = 0, max_gu2_ = 0, max_conv_ = 0, max_gv_ = 0;   // (scaled form: convolution channels, key heads x value size of the blending attention layers)
     int *ids_ = nullptr, *offsets_ = nullptr, *order_ = nullptr, *where_ = nullptr, *tokens_dev_ = nullptr, *want_dev_ = nullptr;
