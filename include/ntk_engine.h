@@ -209,6 +209,13 @@ int ntk_reduce_rmsnorm_prepare_x(float* hidden, const ntk_gemm_partials* partial
 int ntk_silu_mul_prepare_x(float* output, const float* gate, const float* up, int n_tokens, int width, void* workspace, void* stream);
 int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials, void* workspace, void* stream);
 
+/* Y[t][0..out) (+)= W . X[t] for the tokens of a prompt over IEEE-half weights ([out][in] row-major), one pass over W: the batched form of n_tokens ntk_gemv calls.
+ * row_max: the tokens' largest |X| where their producer left it (ntk_rmsnorm_rowmax ...), NULL: taken here.  workspace (16-byte aligned): without row_max at least
+ * ntk_gemm_half_workspace_bytes(n_tokens), else NULL is enough; what it holds beyond that is used for partial sums. */
+size_t ntk_gemm_half_workspace_bytes(int n_tokens);
+int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
+                  size_t workspace_bytes, void* stream);
+
 /* Dequantise rows of a (quantised) embedding table on the device: out[t,:] = table[tokens[t],:].
  * Same arithmetic as the host loop in reference src/model/transformer.cpp:419-599; Q5_K is zero-filled
  * exactly as the reference does (:595-598).  tokens is a DEVICE int array. */

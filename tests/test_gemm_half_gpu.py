@@ -1,0 +1,72 @@
+"""ntk_gemm_half (prompt projections over half-precision weights) at the edges of its tiles, chunks and pieces, against float64 sums.  Bound: an activation is off by 2^-24 of its
+value at most, every product and addition rounds to 32 bits once: |error| <= (K + 18) * 2^-24 * sum |x w|."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from ntransformer_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def run(x, w, y0=None, room=0, given_max=False):
+    L = _lib.lib()
+    L.ntk_gemm_half_workspace_bytes.restype = C.c_size_t
+    L.ntk_gemm_half.argtypes = [C.c_void_p] * 3 + [C.c_int] * 4 + [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
+    T, K = x.shape
+    N = w.shape[0]
+    need = int(L.ntk_gemm_half_workspace_bytes(T))
+    xb, wb = ops.DeviceBuffer.from_numpy(x.astype(np.float32)), ops.DeviceBuffer.from_numpy(w.astype(np.float16))
+    yb = ops.DeviceBuffer.from_numpy(y0 if y0 is not None else np.full((T, N), 7.0, np.float32))
+    ws = ops.DeviceBuffer(need + room * 4)
+    mb = ops.DeviceBuffer.from_numpy(np.abs(x).max(1).astype(np.float32)) if given_max else None
+    _lib.check(L.ntk_gemm_half(yb.ptr, wb.ptr, xb.ptr, T, N, K, int(y0 is not None), mb.ptr if mb else None, ws.ptr, need + room * 4, None), "ntk_gemm_half")
+    return yb.numpy(np.float32, T * N).reshape(T, N)
+
+
+def within_bound(y, x, w, y0=0.0):
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    return np.all(np.abs(y - (y0 + x @ w.T)) <= (x.shape[1] + 18) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T + np.abs(y0)) + 1e-37)
+
+
+def values(T, N, K, seed):
+    g = np.random.default_rng(seed)
+    return g.standard_normal((T, K)).astype(np.float32), (g.standard_normal((N, K)) / np.sqrt(K)).astype(np.float16).astype(np.float32)
+
+
+@pytest.mark.parametrize("T,N,K", [(2, 64, 64), (3, 1, 8), (16, 1024, 4096), (31, 65, 72), (33, 516, 520), (65, 128, 2048), (129, 300, 40), (200, 2048, 1024), (257, 512, 96), (5, 70, 37),
+                                   (2, 28672, 128), (1030, 260, 264)])
+def test_edges_of_tiles_chunks_and_pieces(T, N, K):
+    x, w = values(T, N, K, T + N)
+    for room in (0, 16 * T * N):
+        assert within_bound(run(x, w, room=room), x, w)
+        y0 = np.random.default_rng(2).standard_normal((T, N)).astype(np.float32)
+        assert within_bound(run(x, w, y0=y0, room=room, given_max=True), x, w, y0)
+
+
+def test_rows_of_every_magnitude():
+    x, w = values(40, 96, 256, 9)
+    x *= np.logspace(-30, 30, 40).astype(np.float32)[:, None]
+    x[:, ::16] *= 4000.0                       # a few channels tower over the others
+    x[7] = 0.0
+    assert within_bound(run(x, w), x, w)
+
+
+def test_infinities_stay_in_their_row():
+    x, w = values(9, 64, 128, 4)
+    x[3, 5], x[6, 9] = np.inf, np.nan
+    y = run(x, w)
+    rows = [r for r in range(9) if r not in (3, 6)]
+    assert within_bound(y[rows], x[rows], w) and np.isnan(y[6]).all()
+    assert np.array_equal(y[3], np.where(w[:, 5] == 0, np.nan, np.sign(w[:, 5]) * np.inf).astype(np.float32), equal_nan=True)
+
+
+def test_what_it_refuses():
+    L = _lib.lib()
+    b = ops.DeviceBuffer(4096)
+    f = L.ntk_gemm_half
+    f.argtypes = [C.c_void_p] * 3 + [C.c_int] * 4 + [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
+    assert f(b.ptr, b.ptr, None, 2, 8, 8, 0, None, b.ptr, 4096, None) == -5
+    assert f(b.ptr, b.ptr, b.ptr, 2, 8, 8, 0, None, None, 0, None) == -5 and f(b.ptr, b.ptr, b.ptr, 9, 8, 8, 0, None, b.ptr, 32, None) == -2
+    assert f(b.ptr, b.ptr, b.ptr, 2, 0, 8, 0, None, b.ptr, 4096, None) == -2 and f(b.ptr, b.ptr, b.ptr, 0, 8, 8, 0, None, b.ptr, 4096, None) == 0
