@@ -9,7 +9,7 @@
 // Expanded: a workgroup owns 16 tokens of one head and walks the visible keys in chunks of 64 -- lane = key for the scores (key slabs of 64 entries in
 // LDS), online softmax per row in F32, lane = value column for the weighted sum.  Shared: a workgroup owns 16 (token, head) rows and whole tiles of 32
 // cache rows; the tiles go round up to 128 workgroups and a second launch merges their (max, sum, vector) states.
-#include "common.hip.h"
+#include "attention_tile.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -532,6 +532,13 @@ int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const flo
     a.keyA0 = key0;
     const int rows = T;
     if (a.nV > 8 * SLAB) return NTK_E_SHAPE;
+    if (rows >= 32 && attention_tile_takes(a.nA + a.nB, a.nV)) {       // (fewer rows leave most of a tile of 32 empty)
+        TileAttnArgs t{};
+        t.out = out; t.ldo = ldo; t.q = q; t.ldq = ldq; t.kA = a.kA; t.ldA = a.ldA; t.nA = a.nA; t.hA = a.hA; t.kB = a.kB; t.ldB = a.ldB; t.nB = a.nB;
+        t.v = a.v; t.ldV = a.ldV; t.nV = a.nV; t.hV = a.hV; t.key0 = key0; t.H = H; t.G = H; t.pos0 = pos0; t.T = T; t.window = window; t.scale = scale; t.out_scale = 1.0f;
+        launch_attention_tile(t, s);
+        return last_launch_status();
+    }
     const int DKP = (a.nA + a.nB + 3) & ~3;
     const size_t lds = ((size_t)QROWS * DKP + KCH * (SLAB + 1) + QROWS * KCH) * sizeof(float);
     if (lds > 150 * 1024) return NTK_E_SHAPE;

@@ -12,7 +12,7 @@
 // in LDS), online softmax per row and map, lane = value column for the weighted sums (the value slab is loaded once for both maps).  When few rows
 // face many keys (decoding), the chunks go round `splits` workgroups and a second launch merges their (max, sum, vector) states.
 #include <algorithm>
-#include "common.hip.h"
+#include "attention_tile.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -493,10 +493,20 @@ int ntk_window_attention(const ntk_window_attention_desc* d, void* stream) {
     a.scratch = d->scratch;
     a.rel = d->rel; a.bucket_of = d->bucket_of; a.n_dist = d->n_dist;
     if (a.rel && (!a.bucket_of || a.n_dist <= 0)) return NTK_E_NULL;
+    hipStream_t s = resolve_stream(stream);
+    // one map, one part per row, enough rows for the matrix instructions' tiles of 32 (a prompt's portion; decoded tokens split their keys instead)
+    if (d->maps == 1 && a.splits == 1 && !d->sub_norm && (long long)d->T * (d->H / d->G) >= 64 && attention_tile_takes(d->dn, d->dv)) {
+        TileAttnArgs t{};
+        t.out = a.out; t.ldo = a.ldo; t.q = a.q; t.ldq = a.ldq; t.kA = a.cache; t.ldA = a.row; t.nA = a.dn; t.hA = a.dn; t.kB = a.cache; t.ldB = a.row;
+        t.v = a.cache + (long long)a.G * a.dn; t.ldV = a.row; t.nV = a.dv; t.hV = a.dv; t.H = a.H; t.G = a.G; t.pos0 = a.pos0; t.T = a.T;
+        t.window = a.window; t.chunks = a.chunks; t.keep = a.keep; t.scale = a.scale; t.softcap = a.softcap; t.out_scale = a.out_scale; t.sink = a.sink; t.sinks = a.sinks;
+        t.slopes = a.slopes; t.rel = a.rel; t.bucket_of = a.bucket_of; t.n_dist = a.n_dist; t.gate = a.gate; t.ldg = a.ldg; t.head_gate = a.head_gate;
+        launch_attention_tile(t, s);
+        return last_launch_status();
+    }
     const int DNP = (d->dn + 3) & ~3;
     const size_t lds = ((size_t)WROWS * d->maps * DNP + WKCH * (WSLAB + 1) + (size_t)d->maps * WROWS * WKCH) * sizeof(float);
     if (lds > 150 * 1024) return NTK_E_SHAPE;
-    hipStream_t s = resolve_stream(stream);
     const dim3 grid((d->T * (d->H / d->G) + WROWS - 1) / WROWS, d->G, a.splits);
     if (lds > 48 * 1024) {
         static bool raised = false;   // (idempotent: a race sets the same attribute twice)
