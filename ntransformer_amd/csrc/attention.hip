@@ -739,7 +739,8 @@ __global__ __launch_bounds__(256) void rope_kv_store_rows_kernel(float* __restri
     const int cp = start_pos + sp, per_pos = n_kv_heads * head_dim;
     const bool store = cp < max_seq;   // reference attention.cu:336
     const int total = (n_heads + n_kv_heads) * half_dim;
-    for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
+    const int first = blockIdx.y * blockDim.x + threadIdx.x, stride = gridDim.y * blockDim.x;
+    for (int idx = first; idx < total; idx += stride) {
         const int pair = idx % half_dim, head = idx / half_dim;
         const int i0 = interleaved ? 2 * pair : pair, i1 = interleaved ? 2 * pair + 1 : pair + half_dim;
         const float c = cs[0][pair], sn = cs[1][pair];
@@ -760,7 +761,7 @@ __global__ __launch_bounds__(256) void rope_kv_store_rows_kernel(float* __restri
         }
     }
     if (store)
-        for (int e = threadIdx.x; e < per_pos; e += blockDim.x) vc[(size_t)cp * per_pos + e] = f2h(v[(size_t)sp * per_pos + e]);
+        for (int e = first; e < per_pos; e += stride) vc[(size_t)cp * per_pos + e] = f2h(v[(size_t)sp * per_pos + e]);
 }
 
 __global__ void kv_store_kernel(uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, const float* __restrict__ k,
@@ -854,7 +855,9 @@ int ntk_rope_kv_store(float* q, const float* k, const float* v, const int* posit
     if (!q || !k || !v || !positions || !k_cache || !v_cache) return NTK_E_NULL;
     if (seq_len < 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim <= 0 || (head_dim & 1) || head_dim > 256 || start_pos < 0 || max_seq <= 0) return NTK_E_SHAPE;
     if (seq_len == 0) return NTK_OK;
-    hipLaunchKernelGGL(ntk::rope_kv_store_rows_kernel, dim3(seq_len), dim3(256), 0, ntk::resolve_stream(stream), q, k, v, positions, n_heads, n_kv_heads,
+    // (a short prompt: several workgroups on a token's heads, each with its own table -- 16 tokens of 32 + 8 heads 7.6 us with one, 4.8 with four)
+    const int parts = seq_len <= 64 ? 4 : 1;
+    hipLaunchKernelGGL(ntk::rope_kv_store_rows_kernel, dim3(seq_len, parts), dim3(256), 0, ntk::resolve_stream(stream), q, k, v, positions, n_heads, n_kv_heads,
                        head_dim, theta_base, freq_scale, interleaved, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), start_pos, max_seq);
     return ntk::last_launch_status();
 }

@@ -320,7 +320,7 @@ __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, i
 static inline int split_pad_tokens(int T) { return T <= 32 ? (T + 15) / 16 * 16 : (T + GB_TOK - 1) / GB_TOK * GB_TOK; }
 
 // X[T][in] (any producer) -> workspace: row maximum + split, one workgroup per token (instead of row_scale_kernel + split_x_kernel)
-__global__ __launch_bounds__(256) void rowmax_split_kernel(const float* __restrict__ X, int T, int in, uint8_t* __restrict__ ws) {
+__global__ __launch_bounds__(1024) void rowmax_split_kernel(const float* __restrict__ X, int T, int in, uint8_t* __restrict__ ws) {
     __shared__ float red[16];
     const int t = (int)blockIdx.x;
     const float* row = t < T ? X + (size_t)t * in : nullptr;
@@ -1843,13 +1843,18 @@ __global__ __launch_bounds__(256) void reduce_splits_kernel(const ReduceArgs a) 
     if (sg == 2) { Y = a.Y[2]; part = a.part[2]; out = a.out[2]; }
     const size_t idx = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (idx >= (size_t)a.T * out) return;
-    float4 v = *reinterpret_cast<const float4*>(part + idx);
-    for (int s = 1; s < a.nsplit; ++s) {
-        const float4 q = *reinterpret_cast<const float4*>(part + (size_t)s * a.T * out + idx);
-        v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
+    float4 v = *reinterpret_cast<const float4*>(part + idx), rs{0.0f, 0.0f, 0.0f, 0.0f};
+    if (a.resid) rs = *reinterpret_cast<const float4*>(a.resid + idx);
+    for (int s = 1; s < a.nsplit; s += 4) {                  // (four splits' requests under way, the additions in split order)
+        float4 q[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = *reinterpret_cast<const float4*>(part + (size_t)min(s + j, a.nsplit - 1) * a.T * out + idx);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (s + j < a.nsplit) { v.x += q[j].x; v.y += q[j].y; v.z += q[j].z; v.w += q[j].w; }
     }
     if (a.resid) {
-        const float4 q = *reinterpret_cast<const float4*>(a.resid + idx);
+        const float4 q = rs;
         v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
     }
     *reinterpret_cast<float4*>(Y + idx) = v;
@@ -1862,11 +1867,59 @@ __global__ __launch_bounds__(1024) void reduce_rmsnorm_rowmax_kernel(float* __re
                                                                      const float* __restrict__ weight, float eps, float* __restrict__ x_out,
                                                                      float* __restrict__ row_max, float* __restrict__ zero, uint8_t* __restrict__ ws) {
     __shared__ float red[16];
+    extern __shared__ __attribute__((aligned(16))) float xs[];   // the normalised row (launches with ws whose row fits the threads' registers)
     if ((int)blockIdx.x >= T) { split_row(nullptr, 0u, (int)blockIdx.x, H, ws); return; }   // (ws launches only: the padding tokens' zero records)
     const size_t row = (size_t)blockIdx.x * H, plane = (size_t)T * H;
     float* h = hidden + row;
     const int bd = (int)blockDim.x, tid = (int)threadIdx.x;
     float ssq = 0.0f;
+    if (H <= 8 * bd) {
+        // One round trip for everything (up to nine splits, the residual, the norm's weights), the row in registers up to its norm and in LDS for its split: the walk below
+        // reads its own row back twice -- 9.9 us a launch at 16 tokens of 4096 with eight splits, 6.8 this way.  The same elements, sums and orders: identical bits.
+        float v[8], r[8], w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { const int i = min(tid + k * bd, H - 1); v[k] = part[row + i]; r[k] = h[i]; w[k] = weight[i]; }
+        for (int sp = 1; sp < nsplit; sp += 8) {
+            float q[8][8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const size_t at = (size_t)min(sp + j, nsplit - 1) * plane + row;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) q[j][k] = part[at + min(tid + k * bd, H - 1)];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (sp + j < nsplit) {   // (uniform)
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] += q[j][k];
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (tid + k * bd < H) {
+                v[k] += r[k];
+                h[tid + k * bd] = v[k];
+                ssq = fmaf(v[k], v[k], ssq);
+            }
+        const float tot = block_sum(ssq, red);
+        const float rms_inv = 1.0f / sqrtf(tot / (float)H + eps);
+        uint32_t mb = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (tid + k * bd < H) {
+                const float y = v[k] * rms_inv * w[k];
+                x_out[row + tid + k * bd] = y;
+                if (ws) xs[tid + k * bd] = y;
+                mb = max(mb, __float_as_uint(y) & 0x7FFFFFFFu);
+            }
+        const float m = block_max(__uint_as_float(mb <= 0x7F800000u ? mb : 0x7F800000u), red);   // (its barriers also put the row into LDS)
+        if (ws) { split_row(xs, __float_as_uint(m), (int)blockIdx.x, H, ws); return; }
+        if (tid == 0) {
+            row_max[blockIdx.x] = m;
+            if (zero) zero[blockIdx.x] = 0.0f;
+        }
+        return;
+    }
     // the thread's elements tid, tid + bd, ... (rmsnorm_kernel's assignment and accumulation order), eight at a time, the splits four at a time:
     // 32 independent loads in flight, the additions in split order (a rolled loop over the splits is one dependent load per addition:
     // 20 us per launch at 64 tokens x 8 splits, profiles/r05_prefill_row_max_ab.txt)
@@ -2425,7 +2478,7 @@ static int prepare_x_check(const void* X, int n_tokens, int in, const void* work
 int ntk_gemm_prepare_x(const float* X, int n_tokens, int in_features, void* workspace, void* stream) {
     const int st = prepare_x_check(X, n_tokens, in_features, workspace);
     if (st != NTK_OK || n_tokens == 0) return st;
-    hipLaunchKernelGGL(ntk::rowmax_split_kernel, dim3(ntk::split_pad_tokens(n_tokens)), dim3(256), 0, ntk::resolve_stream(stream), X, n_tokens, in_features,
+    hipLaunchKernelGGL(ntk::rowmax_split_kernel, dim3(ntk::split_pad_tokens(n_tokens)), dim3(in_features >= 4096 ? 1024 : 256), 0, ntk::resolve_stream(stream), X, n_tokens, in_features,
                        static_cast<uint8_t*>(workspace));
     return ntk::last_launch_status();
 }
@@ -2457,8 +2510,8 @@ int ntk_reduce_rmsnorm_prepare_x(float* hidden, const ntk_gemm_partials* p, cons
         hipLaunchKernelGGL(ntk::rmsnorm_split_kernel, dim3(ntk::split_pad_tokens(T)), block, 0, st, x_out, hidden, weight, T, H, eps, static_cast<uint8_t*>(workspace));
         return ntk::last_launch_status();
     }
-    hipLaunchKernelGGL(ntk::reduce_rmsnorm_rowmax_kernel, dim3(ntk::split_pad_tokens(T)), block, 0, st, hidden, p->part[0], p->nsplit, T, H, weight, eps, x_out,
-                       static_cast<float*>(nullptr), static_cast<float*>(nullptr), static_cast<uint8_t*>(workspace));
+    hipLaunchKernelGGL(ntk::reduce_rmsnorm_rowmax_kernel, dim3(ntk::split_pad_tokens(T)), block, H <= 8 * (int)block.x ? (size_t)H * sizeof(float) : 0, st, hidden, p->part[0], p->nsplit, T, H,
+                       weight, eps, x_out, static_cast<float*>(nullptr), static_cast<float*>(nullptr), static_cast<uint8_t*>(workspace));
     return ntk::last_launch_status();
 }
 int ntk_silu_mul_prepare_x(float* output, const float* gate, const float* up, int n_tokens, int width, void* workspace, void* stream) {

@@ -236,6 +236,30 @@ def test_gemm_quant_f16_split_sums_folded_into_the_consuming_launch(qname, T, ro
     if T > 1024: assert ns == 1 and ns2 == 1
 
 
+@pytest.mark.parametrize("T,H,nsplit", [(1, 48, 2), (3, 1040, 9), (16, 2048, 8), (5, 4096, 10), (2, 4112, 7), (4, 8192, 17), (3, 8224, 3)])
+def test_reduce_rmsnorm_rowmax_sums_in_split_order(T, H, nsplit):
+    """rows that fit the threads' registers and rows that do not, more splits than one round of requests: the sums in split order, the residual last, bit for bit"""
+    import ctypes as C
+    r = rng(T + H + nsplit)
+    part, h0 = r.standard_normal((nsplit, T, H)).astype(np.float32), r.standard_normal((T, H)).astype(np.float32)
+    nw = (1.0 + 0.1 * r.standard_normal(H)).astype(np.float32)
+    want = part[0].copy()
+    for q in part[1:]:
+        want += q
+    want += h0
+    pd, hd, nd, xd, rm, other = DB.from_numpy(part), DB.from_numpy(h0), DB.from_numpy(nw), DB.zeros(T * H * 4), DB.zeros(T * 4), DB.zeros(T * H * 4)
+    pt = _lib.GemmPartials()
+    pt.part[0], pt.y[0], pt.rows[0], pt.nseg, pt.n_tokens, pt.nsplit = pd.ptr, other.ptr, H, 1, T, nsplit
+    f = _lib.lib().ntk_reduce_rmsnorm_rowmax
+    f.argtypes = [C.c_void_p, C.POINTER(_lib.GemmPartials), C.c_void_p, C.c_float, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+    assert f(hd.ptr, C.byref(pt), nd.ptr, 1e-5, xd.ptr, rm.ptr, None, None) == 0
+    x1 = DB.zeros(T * H * 4)
+    ops.launch_rmsnorm(x1, DB.from_numpy(want), nd, T, H, 1e-5)
+    X = x1.numpy(np.float32).reshape(T, H)
+    assert np.array_equal(hd.numpy(np.float32).reshape(T, H), want) and np.array_equal(xd.numpy(np.float32).reshape(T, H), X)
+    assert np.array_equal(rm.numpy(np.float32), np.abs(X).max(axis=1))
+
+
 @pytest.mark.parametrize("qname", ["Q8_0", "Q4_K", "Q6_K"])
 @pytest.mark.parametrize("T,rows,in_f", [(1, 16, 256), (5, 64, 512), (16, 256, 4096), (20, 128, 2048), (64, 1024, 2048), (70, 48, 1024), (200, 256, 1024), (1024, 32, 256)])
 def test_gemm_quant_f16_planes_written_by_the_launch_that_produces_x(qname, T, rows, in_f):
