@@ -204,11 +204,13 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const AttnArgs a)
 }
 
 // ------------------------------------------------------------------------------------------------------------------- the shared form (decoding)
-// Keys and values are the cache rows themselves, so a workgroup loads a tile of KB = 32 rows [latent | rotated] ONCE (all requests in flight together) and
-// uses it for every (token, head) row of its tile of 16: thread (key, row pair) forms two scores over the whole row, sixteen threads run the online softmax
-// of their row, then thread r sums the weighted latents column r of all 16 rows.  The tiles of 32 keys go round `splits` workgroups; each leaves one
-// (max, sum, vector) state per row and latent_attention_merge_kernel adds them.
-constexpr int KB = 32, SROWS = 16;
+// Keys and values are the cache rows themselves, so a workgroup loads a tile of KB = 32 rows [latent | rotated] ONCE (a thread's requests in flight together) and uses it for
+// every (token, head) row of its tile of 16, on the F32 matrix instructions: wave w forms the scores of 16 rows x 32 keys over every fourth step of 16 entries (queries as
+// operands in registers, straight from memory), the four parts meet in LDS, sixteen threads run the online softmax of their row, then wave w sums the weighted latents
+// of a quarter of the columns.  The tiles of 32 keys go round `splits` workgroups; each leaves one (max, sum, vector) state per row and latent_attention_merge_kernel adds
+// them.  Latency bounds it: launch, one round trip for tile and queries, ~70 matrix instructions, softmax, ~64 more, the states out.  With the products on the vector
+// units (one LDS read per two FMAs) and the tile in three round trips 1100 positions took 21.4 us, now 12.2.
+constexpr int KB = 32, SROWS = 16, SSTEPS = 13;    // keys of (latent + rotated) up to 4 * 16 * SSTEPS = 832 entries
 struct SharedArgs {
     const float* q; int ldq;          // [T][H][R + dr], ldq floats between tokens
     const float* cache; int row;      // cache rows
@@ -218,175 +220,184 @@ struct SharedArgs {
 };
 
 __global__ __launch_bounds__(256) void latent_attention_shared_kernel(const SharedArgs a) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int DK = a.R + a.dr;
-    const int DKP = ((DK + 3) & ~3) + 4;           // rows 16-byte aligned, 4 banks apart
+    constexpr int PP = KB + 4;
+    const int DK = a.R + a.dr, D16 = (DK + 15) & ~15, DKP = D16 + 4;      // rows 16-byte aligned, 4 banks apart; zero behind DK
     float* Ks = lds;                               // [KB][DKP]
-    float* Qs = Ks + KB * DKP;                     // [SROWS][DKP]
-    float* Ps = Qs + SROWS * DKP;                  // [SROWS][KB]
-    float* ms = Ps + SROWS * KB;                   // [SROWS] running max
+    float* Sp = Ks + KB * DKP;                     // [4][SROWS][PP] parts of the scores
+    float* Ps = Sp + 4 * SROWS * PP;               // [SROWS][PP]
+    float* ms = Ps + SROWS * PP;                   // [SROWS] running max
     float* ls = ms + SROWS;                        // [SROWS] running sum
     float* cr = ls + SROWS;                        // [SROWS] correction of this tile
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, g4 = lane >> 4;
     const int n_rows = a.T * a.H, row0 = blockIdx.x * SROWS;
     const int last_row = min(row0 + SROWS, n_rows) - 1;
     const int pmin = a.pos0 + row0 / a.H, pmax = a.pos0 + last_row / a.H;
     const int jlo = a.window > 0 ? max(0, pmin - a.window + 1) : 0, jhi = pmax;
-    for (int d = tid; d < DKP; d += 256) {          // the 16 query rows: all requests of a pass in flight before the first is stored
-        float qv[SROWS];
+    const bool vec4 = (DK % 4 == 0) && (a.row % 4 == 0) && !((uintptr_t)a.cache & 15);
+    // the wave's part of the queries: row i16, entries 16 s + 4 g4 .. of the steps s = wave, wave + 4, ...
+    f4 qf[SSTEPS];
+    {
+        const int r = min(row0 + i16, n_rows - 1);
+        const float* q = a.q + (long long)(r / a.H) * a.ldq + (long long)(r % a.H) * DK;
+        const bool qv = (DK % 4 == 0) && (a.ldq % 4 == 0) && !((uintptr_t)a.q & 15);
 #pragma unroll
-        for (int i = 0; i < SROWS; ++i) {
-            const int r = row0 + i;
-            qv[i] = (r < n_rows && d < DK) ? a.q[(long long)(r / a.H) * a.ldq + (long long)(r % a.H) * DK + d] : 0.0f;
+        for (int u = 0; u < SSTEPS; ++u) {
+            const int d = 16 * (wave + 4 * u) + 4 * g4;
+            qf[u] = f4{0.f, 0.f, 0.f, 0.f};
+            if (d < DK) {
+                if (qv) qf[u] = *reinterpret_cast<const f4*>(q + d);
+                else
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) qf[u][c] = d + c < DK ? q[d + c] : 0.0f;
+            }
         }
-#pragma unroll
-        for (int i = 0; i < SROWS; ++i) Qs[i * DKP + d] = qv[i];
     }
     if (tid < SROWS) { ms[tid] = -INFINITY; ls[tid] = 0.0f; }
-    const int lane = tid & 63, wave = tid >> 6;
-    const int key = tid % KB, rg = tid / KB;       // scores: rows 2 rg, 2 rg + 1
-    const int rpos0 = row0 + 2 * rg < n_rows ? a.pos0 + (row0 + 2 * rg) / a.H : -1;
-    const int rpos1 = row0 + 2 * rg + 1 < n_rows ? a.pos0 + (row0 + 2 * rg + 1) / a.H : -1;
-    constexpr int RC = 2;                          // latent columns per thread: R <= 512
-    float acc[RC][SROWS];
+    const int srow = tid >> 4, sub = tid & 15;     // softmax: sixteen threads per row, two keys each
+    const int rpos = row0 + srow < n_rows ? a.pos0 + (row0 + srow) / a.H : -1;
+    constexpr int CT = 8;                          // tiles of 16 columns per wave: R <= 512
+    f4 acc[CT];
 #pragma unroll
-    for (int c = 0; c < RC; ++c)
-#pragma unroll
-        for (int i = 0; i < SROWS; ++i) acc[c][i] = 0.0f;
-    const bool vec4 = (DK % 4 == 0) && (a.row % 4 == 0) && !((uintptr_t)a.cache & 15);
+    for (int t = 0; t < CT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+    const int col0 = wave * ((((a.R + 15) / 16 + 3) / 4) * 16);           // the wave's columns
+    const int n_ct = min(max(((a.R + 15) / 16) - col0 / 16, 0), ((a.R + 15) / 16 + 3) / 4);
     int tile = 0;
     for (int j0 = jlo; j0 <= jhi; j0 += KB, ++tile) {
         if (tile % a.splits != (int)blockIdx.y) continue;
         const int nk = min(KB, jhi + 1 - j0);
-        __syncthreads();                           // the previous tile is used up (and Qs / ms are written)
-        if (vec4) {                                // 16 bytes per request, eight requests of a thread in flight before the first is stored
-            const int q4 = DK / 4, total = KB * q4, dk = 256 / q4, dc = 256 % q4;
-            int k = tid / q4, c = tid % q4;
-            for (int base = tid; base < total; base += 256 * 8) {
-                float4 v[8];
-                int at[8];
+        const int lk = tid >> 3, lc = tid & 7;     // thread -> (key, every eighth quad)
+        __syncthreads();                           // the previous tile is used up (and ms is written)
+        const float* src = a.cache + (long long)(j0 + min(lk, nk - 1)) * a.row;     // (keys past the last re-read it; their weight is zero)
+        if (vec4) {
+            for (int c0 = lc; 4 * c0 < D16; c0 += 8 * 20) {
+                f4 v[20];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    at[u] = k * DKP + 4 * c;
-                    v[u] = float4{0.f, 0.f, 0.f, 0.f};
-                    if (base + 256 * u < total && k < nk) v[u] = *reinterpret_cast<const float4*>(a.cache + (long long)(j0 + k) * a.row + 4 * c);
-                    c += dc; k += dk;
-                    if (c >= q4) { c -= q4; ++k; }
+                for (int u = 0; u < 20; ++u) {
+                    const int d = 4 * (c0 + 8 * u);
+                    v[u] = f4{0.f, 0.f, 0.f, 0.f};
+                    if (d < DK) v[u] = *reinterpret_cast<const f4*>(src + d);
                 }
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (base + 256 * u < total) *reinterpret_cast<float4*>(Ks + at[u]) = v[u];
+                for (int u = 0; u < 20; ++u)
+                    if (4 * (c0 + 8 * u) < D16) *reinterpret_cast<f4*>(&Ks[lk * DKP + 4 * (c0 + 8 * u)]) = v[u];
             }
         } else {
-            for (int k = wave; k < KB; k += 4)
-                for (int d = lane; d < DKP; d += 64) Ks[k * DKP + d] = (k < nk && d < DK) ? a.cache[(long long)(j0 + k) * a.row + d] : 0.0f;
+            for (int d = lc; d < D16; d += 8) Ks[lk * DKP + d] = d < DK ? src[d] : 0.0f;
         }
         __syncthreads();
-        // ---- scores
-        float s0 = 0.0f, s1 = 0.0f;
-        const float* kr = Ks + key * DKP;
-        const float* qa = Qs + (2 * rg) * DKP;
-        const float* qb = qa + DKP;
-        for (int d = 0; d < DK; d += 4) {          // (entries past DK are zero on both sides)
-            const float4 kv = *reinterpret_cast<const float4*>(kr + d), xa = *reinterpret_cast<const float4*>(qa + d), xb = *reinterpret_cast<const float4*>(qb + d);
-            s0 = fmaf(xa.x, kv.x, s0); s0 = fmaf(xa.y, kv.y, s0); s0 = fmaf(xa.z, kv.z, s0); s0 = fmaf(xa.w, kv.w, s0);
-            s1 = fmaf(xb.x, kv.x, s1); s1 = fmaf(xb.y, kv.y, s1); s1 = fmaf(xb.z, kv.z, s1); s1 = fmaf(xb.w, kv.w, s1);
+        // ---- scores: this wave's steps
+        f4 s0{0.f, 0.f, 0.f, 0.f}, s1{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < SSTEPS; ++u) {
+            const int st = wave + 4 * u;
+            if (16 * st >= D16) continue;          // (uniform over the wave)
+            const f4 k0 = *reinterpret_cast<const f4*>(&Ks[i16 * DKP + 16 * st + 4 * g4]), k1 = *reinterpret_cast<const f4*>(&Ks[(16 + i16) * DKP + 16 * st + 4 * g4]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], k0[c], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], k1[c], s1, 0, 0, 0);
+            }
         }
-        const int j = j0 + key;
-        const bool v0 = key < nk && rpos0 >= 0 && j <= rpos0 && (a.window <= 0 || rpos0 - j < a.window);
-        const bool v1 = key < nk && rpos1 >= 0 && j <= rpos1 && (a.window <= 0 || rpos1 - j < a.window);
-        Ps[(2 * rg) * KB + key] = v0 ? s0 * a.scale : -INFINITY;
-        Ps[(2 * rg + 1) * KB + key] = v1 ? s1 * a.scale : -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            Sp[(wave * SROWS + 4 * g4 + r) * PP + i16] = s0[r];
+            Sp[(wave * SROWS + 4 * g4 + r) * PP + 16 + i16] = s1[r];
+        }
         __syncthreads();
-        // ---- online softmax: 16 lanes per row, two keys each
+        // ---- online softmax
         {
-            const int row = tid >> 4, sub = tid & 15;
-            float* p = Ps + row * KB;
-            const float a0 = p[sub], a1 = p[sub + 16];
-            float mc = fmaxf(a0, a1);
+            float sv[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int key = sub + 16 * e, j = j0 + key;
+                const float* sp = Sp + srow * PP + key;
+                const float sum = (sp[0] + sp[SROWS * PP]) + (sp[2 * SROWS * PP] + sp[3 * SROWS * PP]);
+                const bool vis = key < nk && rpos >= 0 && j <= rpos && (a.window <= 0 || rpos - j < a.window);
+                sv[e] = vis ? sum * a.scale : -INFINITY;
+            }
+            float mc = fmaxf(sv[0], sv[1]);
 #pragma unroll
             for (int o = 8; o >= 1; o >>= 1) mc = fmaxf(mc, __shfl_xor(mc, o, 16));
-            const float mo = ms[row];
+            const float mo = ms[srow];
             const float mn = fmaxf(mo, mc), msafe = mn == -INFINITY ? 0.0f : mn;
-            const float e0 = a0 == -INFINITY ? 0.0f : expf(a0 - msafe), e1 = a1 == -INFINITY ? 0.0f : expf(a1 - msafe);
+            const float e0 = sv[0] == -INFINITY ? 0.0f : expf(sv[0] - msafe), e1 = sv[1] == -INFINITY ? 0.0f : expf(sv[1] - msafe);
             float sum = e0 + e1;
 #pragma unroll
             for (int o = 8; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 16);
-            p[sub] = e0;
-            p[sub + 16] = e1;
-            __syncthreads();                       // every lane has read ms[row]
-            if (sub == 0) {
+            Ps[srow * PP + sub] = e0;
+            Ps[srow * PP + 16 + sub] = e1;
+            if (sub == 0) {                        // (the row's sixteen lanes are of one wave: all have read ms)
                 const float corr = mo == -INFINITY ? 0.0f : expf(mo - msafe);
-                ls[row] = ls[row] * corr + sum;
-                ms[row] = mn;
-                cr[row] = corr;
+                ls[srow] = ls[srow] * corr + sum;
+                ms[srow] = mn;
+                cr[srow] = corr;
             }
         }
         __syncthreads();
-        // ---- weighted latents: thread -> column tid (+ 256)
+        // ---- weighted latents: this wave's columns
+        float corr[4];
 #pragma unroll
-        for (int c = 0; c < RC; ++c) {
-            const int r = tid + 256 * c;
-            if (r < a.R) {
+        for (int r = 0; r < 4; ++r) corr[r] = cr[4 * g4 + r];
+        const f4 p0 = *reinterpret_cast<const f4*>(&Ps[i16 * PP + 4 * g4]), p1 = *reinterpret_cast<const f4*>(&Ps[i16 * PP + 16 + 4 * g4]);
 #pragma unroll
-                for (int i = 0; i < SROWS; ++i) acc[c][i] *= cr[i];
-                for (int k = 0; k < KB; k += 4) {
-                    const float x0 = Ks[(k + 0) * DKP + r], x1 = Ks[(k + 1) * DKP + r], x2 = Ks[(k + 2) * DKP + r], x3 = Ks[(k + 3) * DKP + r];
+        for (int t = 0; t < CT; ++t) {
+            if (t >= n_ct) continue;               // (uniform over the wave)
+            const float* vf = &Ks[(4 * g4) * DKP + col0 + 16 * t + i16];
 #pragma unroll
-                    for (int i = 0; i < SROWS; ++i) {
-                        const float4 p4 = *reinterpret_cast<const float4*>(Ps + i * KB + k);
-                        acc[c][i] = fmaf(p4.x, x0, acc[c][i]); acc[c][i] = fmaf(p4.y, x1, acc[c][i]);
-                        acc[c][i] = fmaf(p4.z, x2, acc[c][i]); acc[c][i] = fmaf(p4.w, x3, acc[c][i]);
-                    }
-                }
+            for (int r = 0; r < 4; ++r) acc[t][r] *= corr[r];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {          // component c of the weights belongs to key 4 g4 + c
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[c], vf[c * DKP], acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[c], vf[(16 + c) * DKP], acc[t], 0, 0, 0);
             }
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < SROWS; ++i) {              // (unrolled: the sums stay in registers)
-        if (row0 + i < n_rows) {
-            float* st = a.scratch + ((long long)(row0 + i) * a.splits + blockIdx.y) * (2 + a.R);
-            if (tid == 0) { st[0] = ms[i]; st[1] = ls[i]; }
+    for (int r = 0; r < 4; ++r) {
+        const int i = 4 * g4 + r;
+        if (row0 + i >= n_rows) continue;
+        float* st = a.scratch + ((long long)(row0 + i) * a.splits + blockIdx.y) * (2 + a.R);
+        if (wave == 0 && i16 == 0) { st[0] = ms[i]; st[1] = ls[i]; }
 #pragma unroll
-            for (int c = 0; c < RC; ++c)
-                if (tid + 256 * c < a.R) st[2 + tid + 256 * c] = acc[c][i];
-        }
+        for (int t = 0; t < CT; ++t)
+            if (t < n_ct && col0 + 16 * t + i16 < a.R) st[2 + col0 + 16 * t + i16] = acc[t][r];
     }
 }
 
-// merge of the partial states of one (token, head) row: weights of the states first, then every thread sums its columns over the states
+// merge of the partial states of one (token, head) row: weights of the states first, then a workgroup sums 64 columns over them, a quarter of the states per wave (one
+// workgroup per row walked all columns over all states: 7.0 us at 35 states of 512, 4.1 this way)
 __global__ __launch_bounds__(256) void latent_attention_merge_kernel(float* out, int ldo, const float* scratch, int splits, int nV, int H) {
     __shared__ float wt[256];
     __shared__ float red[16];
-    const int r = blockIdx.x;   // r = t * H + h
+    __shared__ float part[4][64];
+    const int r = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;   // r = t * H + h
     const float* st = scratch + (long long)r * splits * (2 + nV);
-    float mx = -INFINITY;
-    for (int s = threadIdx.x; s < splits; s += 256) mx = fmaxf(mx, st[(long long)s * (2 + nV)]);
-    mx = block_max(mx, red);
-    float den = 0.0f;
-    for (int s = threadIdx.x; s < splits; s += 256) {
-        const float m = st[(long long)s * (2 + nV)];
-        const float w = m == -INFINITY ? 0.0f : expf(m - mx);
-        wt[s] = w;
-        den += w * st[(long long)s * (2 + nV) + 1];
-    }
-    den = block_sum(den, red);   // (its barriers publish wt)
+    const long long step = 2 + nV;
+    const int v = blockIdx.y * 64 + lane, each = (splits + 3) / 4, s0 = wave * each, s1 = min(s0 + each, splits);
+    float x[8];                                    // the wave's first eight states requested together with the maxima
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = s0 + u < s1 && v < nV ? st[(s0 + u) * step + 2 + v] : 0.0f;
+    const int mine = threadIdx.x;                  // (at most 128 states)
+    const float m = mine < splits ? st[mine * step] : -INFINITY, l = mine < splits ? st[mine * step + 1] : 0.0f;
+    const float mx = block_max(m, red);
+    const float w = m == -INFINITY ? 0.0f : expf(m - mx);
+    wt[threadIdx.x] = w;
+    const float den = block_sum(w * l, red);       // (its barriers publish wt)
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-    float* o = out + (long long)(r / H) * ldo + (long long)(r % H) * nV;
-    for (int v = threadIdx.x; v < nV; v += 256) {
-        float s2 = 0.0f;
-        int s = 0;
-        for (; s + 8 <= splits; s += 8) {          // eight states requested together, added in order
-            float x[8];
+    float sum = 0.0f;
+    for (int s = s0; s < s1; s += 8) {             // states in order
 #pragma unroll
-            for (int u = 0; u < 8; ++u) x[u] = st[(long long)(s + u) * (2 + nV) + 2 + v];
+        for (int u = 0; u < 8; ++u)
+            if (s + u < s1) sum = fmaf(x[u], wt[s + u], sum);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) s2 = fmaf(x[u], wt[s + u], s2);
-        }
-        for (; s < splits; ++s) s2 = fmaf(st[(long long)s * (2 + nV) + 2 + v], wt[s], s2);
-        o[v] = s2 * inv;
+        for (int u = 0; u < 8; ++u) x[u] = s + 8 + u < s1 && v < nV ? st[(s + 8 + u) * step + 2 + v] : 0.0f;
     }
+    part[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0 && v < nV) out[(long long)(r / H) * ldo + (long long)(r % H) * nV + v] = ((part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane])) * inv;
 }
 
 // ------------------------------------------------------------------------------------------------------------------- fold / unfold
@@ -511,15 +522,15 @@ int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const flo
         sa.scale = scale; sa.scratch = scratch;
         const int nkeys = window > 0 ? (window + T - 1 < pos0 + T ? window + T - 1 : pos0 + T) : pos0 + T;
         sa.splits = shared_splits(nkeys);
-        const int rows = T * H, DKP = ((kv_rank + rot_dim + 3) & ~3) + 4;
-        const size_t lds = ((size_t)(KB + SROWS) * DKP + SROWS * KB + 3 * SROWS) * sizeof(float);
-        if (lds > 156 * 1024) return NTK_E_SHAPE;
+        const int rows = T * H, DK = kv_rank + rot_dim;
+        if (((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) > 156 * 1024) return NTK_E_SHAPE;     // (keys of up to 812 entries)
+        const size_t lds = ((size_t)KB * (((DK + 15) & ~15) + 4) + 5 * SROWS * (KB + 4) + 3 * SROWS) * sizeof(float);
         static bool raised_s = false;   // (idempotent: a race sets the same attribute twice)
         if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
         hipLaunchKernelGGL(latent_attention_shared_kernel, dim3((rows + SROWS - 1) / SROWS, sa.splits), dim3(256), lds, s, sa);
         int st = last_launch_status();
         if (st != NTK_OK) return st;
-        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(rows), dim3(256), 0, s, out, ldo, (const float*)scratch, sa.splits, kv_rank, H);
+        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(rows, (kv_rank + 63) / 64), dim3(256), 0, s, out, ldo, (const float*)scratch, sa.splits, kv_rank, H);
         return last_launch_status();
     }
     if (dn <= 0 || dv <= 0) return NTK_E_SHAPE;
