@@ -372,6 +372,11 @@ typedef struct ntk_moe_few_desc {
     int wdtype, act;
     float* mid;
     int T, n;
+    /* glu != 0 (act must be NTK_ACT_NONE): gated units -- `up` and `shared_up` hold a unit's ff gate rows, then its ff up rows, and the unit's activation is
+     * g' * sigmoid(glu_alpha * g') * (u' + glu_up_offset) with g' = min(gate, limit), u' = clamp(up, -limit, limit); limit = glu_limit, the shared unit's shared_limit */
+    int glu; float glu_limit, shared_limit, glu_alpha, glu_up_offset;
+    /* mix != NULL (rows ld_mix floats apart): out += mix + the sum, instead of out = the sum */
+    const float* mix; int ld_mix;
 } ntk_moe_few_desc;
 int ntk_moe_few(const ntk_moe_few_desc* d, void* stream);
 /* Stable grouping of the T*top (token, slot) pairs by expert: offsets [E+1], order [T*top] (pair index t*top+slot of every sorted row),

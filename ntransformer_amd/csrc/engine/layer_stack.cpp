@@ -999,11 +999,12 @@ int LayerStackModel::alloc_buffers() {
     if (form_.scaled)
         ok = ok && fl(&ff_, C * W) && fl(&zf_, C * std::max(max_ffn_, 1)) && fl(&gu2_, C * 2 * std::max(max_ffn_, 1)) && fl(&wscratch_, wsc) && fl(&rscratch_, rsc) &&
              fl(&cv_, C * std::max(max_conv_, 1)) && fl(&vfirst_, C * std::max(max_gv_, 1));
-    if (form_.post_norm) ok = ok && fl(&ff_, C * W) && fl(&zf_, C * std::max(max_ffn_, 1)) && fl(&gu2_, C * 2 * std::max(max_ffn_, 1)) && fl(&wscratch_, wsc) && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_) && fl(&rz_, (size_t)ntk_dense_few_rows() * (max_e_ + 1));
+    if (form_.post_norm) ok = ok && fl(&ff_, C * W) && fl(&zf_, C * std::max(max_ffn_, 1)) && fl(&gu2_, C * 2 * std::max(max_ffn_, 1)) && fl(&wscratch_, wsc) && fl(&rz_, (size_t)ntk_dense_few_rows() * (max_e_ + 1));
     if (form_.dense_parallel) ok = ok && fl(&gu2_, C * 2 * std::max(max_ffn_, 1)) && fl(&wscratch_, wsc);
     // four pieces of a whole pass's rows, and no less than sixteen of a short one's
     pscratch_bytes_ = std::max<size_t>(4 * C * W, (size_t)1 << 22) * sizeof(float);
     ok = ok && fl(&pscratch_, pscratch_bytes_ / sizeof(float));
+    if (max_mid_ > 0) ok = ok && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_);
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
     h_stage_ = (int*)nt_hip_malloc_host(2 * C * sizeof(int));
     ok = ok && h_stage_ != nullptr;
@@ -1219,6 +1220,18 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
         owed_.y = nullptr;
     }
     LS_TRY(ntk_moe_route_ex(ids_, wts_, sgate, h, W, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
+    if (!M.routed.plain && T <= ntk_dense_few_rows() && mid <= NTK_MOE_FEW_MID && W <= NTK_MOE_FEW_MID && !(into_stream && M.identity)) {
+        // decoding: all of a token's gated units in two launches instead of six (grouping, two products each for the chosen and the shared units, their sum: 47 us a token and layer
+        // at 6 of 32 bf16 experts of 2048 x 1408 and a shared unit of 2816, 29 this way)
+        ntk_moe_few_desc d{};
+        d.out = into_stream ? x_ : ff_; d.ldo = W; d.h = h; d.ldh = W; d.ids = ids_; d.wts = wts_; d.top = M.top; d.experts = M.experts;
+        d.up = M.routed.gate_up.ptr; d.down = M.routed.down.ptr; d.ff = M.routed.ff;
+        if (M.has_shared) { d.shared_up = M.shared.gate_up.ptr; d.shared_down = M.shared.down.ptr; d.shared_ff = M.shared.ff; d.sgate = sgate; d.shared_limit = M.shared.limit; }
+        d.wdtype = M.routed.down.dtype; d.act = NTK_ACT_NONE; d.mid = mid_; d.T = T; d.n = W;
+        d.glu = 1; d.glu_limit = M.routed.limit; d.glu_alpha = M.glu_alpha; d.glu_up_offset = M.glu_up_offset;
+        if (into_stream) { d.mix = mix_; d.ld_mix = W; }
+        return ntk_moe_few(&d, stream_);
+    }
     LS_TRY(ntk_moe_group(offsets_, order_, where_, ids_, T, M.top, choices, stream_));     // (identity experts come last: rows behind offsets_[experts], which no product visits)
     LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.routed, h, gu_, act_, dn_, T * M.top, offsets_, order_, M.top));
     if (M.has_shared) LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.shared, h, sgu_, sact_, sdn_, T, nullptr, nullptr, 1));

@@ -74,7 +74,8 @@ class RouteDesc(C.Structure):
 class MoeFewDesc(C.Structure):
     _fields_ = [("out", C.c_void_p), ("ldo", C.c_int), ("h", C.c_void_p), ("ldh", C.c_int), ("ids", C.c_void_p), ("wts", C.c_void_p), ("top", C.c_int), ("experts", C.c_int),
                 ("up", C.c_void_p), ("down", C.c_void_p), ("ff", C.c_int), ("shared_up", C.c_void_p), ("shared_down", C.c_void_p), ("shared_ff", C.c_int), ("sgate", C.c_void_p),
-                ("wdtype", C.c_int), ("act", C.c_int), ("mid", C.c_void_p), ("T", C.c_int), ("n", C.c_int)]
+                ("wdtype", C.c_int), ("act", C.c_int), ("mid", C.c_void_p), ("T", C.c_int), ("n", C.c_int),
+                ("glu", C.c_int), ("glu_limit", C.c_float), ("shared_limit", C.c_float), ("glu_alpha", C.c_float), ("glu_up_offset", C.c_float), ("mix", C.c_void_p), ("ld_mix", C.c_int)]
 
 
 ACT_NONE, ACT_RELU2 = 0, 1
@@ -698,19 +699,26 @@ def moe_pick(z: np.ndarray, E: int, top: int, score: int = 0, groups: int = 1, k
     return ids.numpy(np.int32, T * top).reshape(T, top), wts.numpy(np.float32, T * top).reshape(T, top), (sg.numpy(np.float32, T) if sg else None)
 
 
-def moe_few(h: np.ndarray, ids, wts, up: np.ndarray, down: np.ndarray, shared_up=None, shared_down=None, sgate=None, act: int = ACT_RELU2, dtype: str = "float32") -> np.ndarray:
-    """h [T, n], ids / wts [T, top], up [E, ff, n], down [E, n, ff], shared_up [sff, n], shared_down [n, sff], sgate [T] -> the weighted sum of the chosen units [T, n]"""
+def moe_few(h: np.ndarray, ids, wts, up: np.ndarray, down: np.ndarray, shared_up=None, shared_down=None, sgate=None, act: int = ACT_RELU2, dtype: str = "float32",
+            glu=None, mix: Optional[np.ndarray] = None, out0: Optional[np.ndarray] = None) -> np.ndarray:
+    """h [T, n], ids / wts [T, top], up [E, ff, n], down [E, n, ff], shared_up [sff, n], shared_down [n, sff], sgate [T] -> the weighted sum of the chosen units [T, n];
+    glu = (limit, shared limit, alpha, up offset): gated units, up [E, 2 ff, n] and shared_up [2 sff, n]; mix, out0 [T, n]: both join the sum"""
     L = _bind()
     T, n = h.shape
-    E, ff = up.shape[:2]
-    top, sff = ids.shape[1], (shared_up.shape[0] if shared_up is not None else 0)
+    E, ff = up.shape[0], down.shape[2]
+    top, sff = ids.shape[1], (shared_down.shape[1] if shared_down is not None else 0)
     hb, ib, tb = _f(h), _i(ids), _f(wts)
     (ub, dt), (db, _) = weight_buffer(up, dtype), weight_buffer(down, dtype)
     su, sd = (weight_buffer(w, dtype)[0] if w is not None else None for w in (shared_up, shared_down))
     gb = _f(sgate) if sgate is not None else None
-    out, mid = DeviceBuffer.zeros(T * n * 4), DeviceBuffer.from_numpy(np.full(T * (top * ff + sff), np.nan, np.float32))
-    d = MoeFewDesc(out.ptr, n, hb.ptr, n, ib.ptr, tb.ptr, top, E, ub.ptr, db.ptr, ff, su.ptr if su else None, sd.ptr if sd else None, sff, gb.ptr if gb else None, dt, act,
+    out, mid = _f(out0) if out0 is not None else DeviceBuffer.zeros(T * n * 4), DeviceBuffer.from_numpy(np.full(T * (top * ff + sff), np.nan, np.float32))
+    d = MoeFewDesc(out.ptr, n, hb.ptr, n, ib.ptr, tb.ptr, top, E, ub.ptr, db.ptr, ff, su.ptr if su else None, sd.ptr if sd else None, sff, gb.ptr if gb else None, dt, ACT_NONE if glu else act,
                    mid.ptr, T, n)
+    if glu:
+        d.glu, (d.glu_limit, d.shared_limit, d.glu_alpha, d.glu_up_offset) = 1, glu
+    if mix is not None:
+        mb = _f(mix)
+        d.mix, d.ld_mix = mb.ptr, n
     check(L.ntk_moe_few(C.byref(d), None), "ntk_moe_few")
     return out.numpy(np.float32, T * n).reshape(T, n)
 

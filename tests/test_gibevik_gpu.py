@@ -332,6 +332,35 @@ def test_a_few_tokens_experts_in_two_launches(dtype, T, n, E, ff, top, sff):
         assert rel(Lr.moe_few(h, ids, wts, up, down, su, sd, sg, dtype=dtype), ref) < 1e-5, identity
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,n,E,ff,top,sff", [(1, 32, 4, 16, 2, 24), (8, 41, 6, 9, 3, 0), (3, 33, 5, 7, 4, 11), (2, 600, 3, 520, 3, 1032), (1, 2048, 9, 1408, 6, 2816), (2, 8, 1, 2056, 1, 8)])
+def test_a_few_tokens_gated_experts_into_a_stream(dtype, T, n, E, ff, top, sff):
+    from ntransformer_amd import layers as Lr
+    g = np.random.default_rng(n + ff)
+    h = f32(g.standard_normal((T, n)))
+    up, down = O.to_bf16(g.standard_normal((E, 2 * ff, n)) * 2 / math.sqrt(n)), O.to_bf16(g.standard_normal((E, n, ff)) / math.sqrt(ff))
+    su, sd = (O.to_bf16(g.standard_normal((2 * sff, n)) * 2 / math.sqrt(n)), O.to_bf16(g.standard_normal((n, sff)) / math.sqrt(sff))) if sff else (None, None)
+    mix, out0 = f32(g.standard_normal((T, n))), f32(g.standard_normal((T, n)))
+    limit, shared_limit, alpha, offset = 1.5, 2.0, 1.702, 1.0
+
+    def unit(gu, x, lim):
+        z = gu @ x
+        gate, lin = np.minimum(z[:len(z) // 2], lim), np.clip(z[len(z) // 2:], -lim, lim)
+        return gate / (1 + np.exp(-alpha * gate)) * (lin + offset)
+    for identity in (0, 1):
+        ids = np.stack([g.permutation(E + (2 if identity else 0))[:top] for _ in range(T)])
+        wts = f32(g.uniform(0.1, 1, (T, top)))
+        ref = (mix.astype(F64) + out0) if not identity else np.zeros((T, n))
+        for t in range(T):
+            x = h[t].astype(F64)
+            for e, wt in zip(ids[t], wts[t]):
+                ref[t] += wt * (down[e] @ unit(up[e], x, limit) if e < E else x)
+            if sff:
+                ref[t] += sd @ unit(su, x, shared_limit)
+        got = Lr.moe_few(h, ids, wts, up, down, su, sd, None, dtype=dtype, glu=(limit, shared_limit, alpha, offset), **({} if identity else {"mix": mix, "out0": out0}))
+        assert rel(got, ref) < 1e-5, identity     # (the bound of the ungated form: products of at most 11 264 terms in 32 bits)
+
+
 def test_weighted_sum_with_identity_experts():
     from ntransformer_amd import layers as Lr
     g = np.random.default_rng(6)
