@@ -381,6 +381,20 @@ def test_weighted_sum_with_identity_experts():
         assert rel(Lr.moe_sum(plain, None, wts), np.einsum("ts,tsn->tn", wts.astype(F64), plain.reshape(T, top, n))) < 1e-6
 
 
+@pytest.mark.parametrize("T,top,E,n", [(1, 1, 1, 4), (64, 1, 2, 8), (129, 8, 255, 3), (1024, 6, 32, 132), (1500, 9, 200, 5)])
+def test_grouping_and_sums_at_the_edges(T, top, E, n):
+    """stable order over runs of 64 pairs, one expert, many experts, pairs past the ends; the sum over one slot, odd slots, columns with and without four in a row"""
+    from ntransformer_amd import layers as Lr
+    g = np.random.default_rng(T + E)
+    ids = g.integers(0, E, (T, top)).astype(np.int32)
+    off, order, where = Lr.moe_group(ids, E)
+    want = np.argsort(ids.reshape(-1), kind="stable")
+    assert list(order) == list(want) and all(where[want] == np.arange(T * top))
+    assert list(off) == [0] + list(np.cumsum(np.bincount(ids.reshape(-1), minlength=E)))
+    d, wts = f32(g.standard_normal((T * top, n))), f32(g.uniform(0, 1, (T, top)))
+    assert rel(Lr.moe_sum(d, where, wts), np.einsum("ts,tsn->tn", wts.astype(F64), d.astype(F64)[where].reshape(T, top, n))) < 1e-6
+
+
 # ====================================================================================================================== whole models
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("n", [60, 5])
