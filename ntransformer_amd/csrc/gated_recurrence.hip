@@ -70,6 +70,10 @@ __device__ __forceinline__ float decay_of(float z, int form, float param) {
     return z;
 }
 
+}  // namespace ntk
+#include "delta_chunk.hip.h"
+namespace ntk {
+
 // the per-token vectors of one (token, head), ready for the walk: one wave each
 template <bool DELTA>
 __global__ __launch_bounds__(64) void gated_recurrence_prepare_kernel(const RecArgs a) {
@@ -619,7 +623,8 @@ size_t ntk_gated_recurrence_scratch(int T, int H, int dn, int dv, int removal) {
 
 size_t ntk_gated_recurrence_scratch_ex(const ntk_gated_recurrence_desc* d) {
     if (!d || d->T <= 0 || d->H <= 0 || d->dn <= 0 || d->dv <= 0) return 0;
-    return rec_scratch(d->T, d->H, d->dn, d->dv, d->az != nullptr, rec_needs_prepass(d), d->write_gated != 0 || d->conv_w != nullptr);
+    const size_t walk = rec_scratch(d->T, d->H, d->dn, d->dv, d->az != nullptr, rec_needs_prepass(d), d->write_gated != 0 || d->conv_w != nullptr);
+    return d->write_gated && d->T >= kDeltaChunk ? std::max(walk, delta_chunk_floats(d->T, d->H, d->dn, d->dv)) : walk;
 }
 
 int ntk_gated_recurrence(const ntk_gated_recurrence_desc* d, void* stream) {
@@ -653,6 +658,7 @@ int ntk_gated_recurrence(const ntk_gated_recurrence_desc* d, void* stream) {
         }
     }
     hipStream_t s = resolve_stream(stream);
+    if (a.packed && delta_chunked(a)) return d->dn == 64 ? launch_delta_chunks<64>(a, s) : launch_delta_chunks<128>(a, s);
     // 16 lanes share a column (their sums meet in DPP steps inside a 16-lane row, no trip through LDS on the chain from token to token); rows per lane: the
     // smallest of 4 / 8 / 16 / 32 that covers the head's channels; beyond 512 channels 32 lanes per column.
     if (d->dn <= 16 * 4) return launch_rec<16, 4>(a, s);

@@ -297,6 +297,27 @@ def test_delta_rule_long_portions_walked_in_segments(H, G, dn, dv):
     assert rel(np.concatenate([a, b]), ref.reshape(T, H * dv)) < 1e-4 and rel(st, S) < 1e-4
 
 
+@pytest.mark.parametrize("H,G,dn,dv,T", [(1, 1, 64, 16, 32), (4, 2, 64, 48, 33), (2, 2, 128, 128, 63), (6, 3, 128, 16, 64), (2, 1, 128, 144, 65), (16, 16, 128, 128, 513)])
+def test_delta_rule_in_chunks_on_the_matrix_instructions(H, G, dn, dv, T):
+    """one chunk, partial last chunks, both widths; strong decay (products that underflow) and none; a portion behind a state; and what comes before a NaN stays clean"""
+    from ntransformer_amd import layers as Lr
+    g = np.random.default_rng(T + dn)
+    q, k, v, az, wz, rates, bias = _delta_inputs(g, T + 40, H, G, dn, dv)
+    for scale in (1.0, 60.0, 0.0):
+        r = (rates * scale).astype(np.float32)
+        ref, S = _delta_reference(q, k, v, az, wz, r, bias, H, G, dn, dv)
+        ref = ref.reshape(T + 40, H * dv)
+        kw = dict(decay_form=Lr.DECAY_EXP_SOFTPLUS, wb=bias, decay_rates=r, G=G, unit_q=True, unit_k=True, head_gates=True, write_gated=True, q_scale=dn ** -0.5)
+        a, st = Lr.gated_recurrence(q[:T], k[:T], v[:T], wz[:T], H, dn, dv, 0, az=az[:T], **kw)
+        b, st = Lr.gated_recurrence(q[T:], k[T:], v[T:], wz[T:], H, dn, dv, T, az=az[T:], state=st, **kw)
+        # 32-bit sums of 128 + 32 terms per token; the state keeps what a token left for as long as the decay lets it: the bound of the walk at 45 tokens
+        assert rel(np.concatenate([a, b]), ref) < 1e-5 and rel(st, S) < 1e-5, scale
+    at = T - 7
+    v[at] = np.nan
+    a, st = Lr.gated_recurrence(q[:T], k[:T], v[:T], wz[:T], H, dn, dv, 0, az=az[:T], **kw)
+    assert rel(a[:at], ref[:at]) < 1e-5 and np.isnan(a[at:]).all() and np.isnan(st).all()
+
+
 @pytest.mark.parametrize("H,G,dn,dv,taps", [(4, 2, 8, 8, 4), (6, 3, 32, 64, 4), (3, 3, 13, 7, 2), (2, 1, 70, 130, 5), (5, 1, 16, 300, 1), (2, 2, 128, 96, 16)])
 def test_decoded_tokens_pass_their_convolutions_inside_the_recurrence(H, G, dn, dv, taps):
     """raw q, k, v of one token at a time, the short convolutions inside the pre-pass's launch: the same outputs, state and carried inputs as the convolution as an
