@@ -10,7 +10,8 @@
 //
 // Everything that does not know S_0 is one launch over all chunks and heads at once (delta_chunk_solve_kernel: unit vectors and gates from the raw projections, the two
 // 32 x 32 products, forward substitution on [diag(a) V | diag(a W) U] with a thread per column); what is left from chunk to chunk is four small products per head
-// and 16 value columns (delta_chunk_walk_kernel), the state in the accumulators of its waves all the way.
+// and 16 value columns (delta_chunk_walk_kernel), the state in the accumulators of its waves all the way.  1024 tokens of 16 heads of 128 x 128: 93 us, where the walk
+// token by token, its pre-pass and the settling of its segments took 277.
 #pragma once
 
 namespace ntk {
@@ -21,7 +22,7 @@ typedef float deltax4_t __attribute__((ext_vector_type(4)));
 struct DeltaArgs {
     RecArgs r;
     int chunks;
-    float *vt, *ut, *qw, *udt, *pm, *wc;   // per (chunk, head): [32][dv], [32][dn], [32][dn], [dn][32], [32][32], one number
+    float *vt, *ut, *qw, *udt, *pm, *wc;   // per (chunk, head): [dv][32], [32][dn], [32][dn], [dn][32], [32][32], one number
 };
 
 // floats of DeltaArgs' buffers
@@ -30,11 +31,13 @@ inline size_t delta_chunk_floats(int T, int H, int dn, int dv) {
     return blocks * ((size_t)kDeltaChunk * (dv + 3 * dn + kDeltaChunk) + 4);
 }
 
-// grid (chunks, H).  A chain of short steps (loads, norms, products, 31 dependent rows of the substitution) that needs several workgroups a CU, hence 40 KB of LDS.
+// grid (chunks, H).  A chain of short steps (loads, norms, products, substitution) on a launch of one or two workgroups a CU, so every instruction is fetched cold: the
+// code stays small.  The substitution goes four rows at a time in a loop, the solved rows of a thread's column in LDS; unrolled over all 32 rows with the column in
+// registers it was 20 KB of straight-line code, and 47 us at 32 chunks of 16 heads (24 us at 5) against 21 (16).
 template <int DN>
 __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(const DeltaArgs A) {
     constexpr int C = kDeltaChunk, LD = DN + 4, LA = C + 4;
-    __shared__ __attribute__((aligned(16))) float us[C * LD], qs[C * LD], am[C * LA];
+    __shared__ __attribute__((aligned(16))) float us[C * LD], qs[C * LD], am[C * LA], xs[C][256];
     __shared__ float rm[C][C + 1], wv[C], av[C], cw[C];
     const RecArgs& a = A.r;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.y;
@@ -94,7 +97,7 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(const DeltaArgs 
         if (tile >= 6) break;
         const float* x = (tile < 3 ? us : qs) + (16 * ti + m) * LD + 4 * g;
         const float* y = us + (16 * tj + m) * LD + 4 * g;
-#pragma unroll
+#pragma unroll 2
         for (int k = 0; k < DN; k += 16) {
             const float4 x4 = *reinterpret_cast<const float4*>(x + k), y4 = *reinterpret_cast<const float4*>(y + k);
             acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x4.x, y4.x, acc[u], 0, 0, 0);
@@ -119,78 +122,97 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(const DeltaArgs 
     pm[(tid / 16) * C + 16 + tid % 16] = 0.0f;                // the tile above the diagonal (256 threads: 16 x 16)
     __syncthreads();
     // W q, and the keys with what decays behind them, a channel's 32 tokens in a row
-    for (int e = tid; e < C * DN; e += 256) A.qw[blk * C * DN + e] = cw[e / DN] * qs[(e / DN) * LD + e % DN];
-    for (int e = tid; e < C * DN; e += 256) A.udt[blk * C * DN + e] = rm[C - 1][e % C] * us[(e % C) * LD + e / C];
+#pragma unroll 2
+    for (int e = tid; e < C * DN / 4; e += 256) {
+        const int t = e / (DN / 4), d = e % (DN / 4) * 4;
+        const float4 q4 = *reinterpret_cast<const float4*>(qs + t * LD + d);
+        *reinterpret_cast<float4*>(A.qw + blk * C * DN + 4 * e) = float4{cw[t] * q4.x, cw[t] * q4.y, cw[t] * q4.z, cw[t] * q4.w};
+    }
+#pragma unroll 2
+    for (int e = tid; e < C * DN / 4; e += 256) {
+        const int t = e % (C / 4) * 4, d = e / (C / 4);
+        const float* u = us + t * LD + d;
+        const float* w = rm[C - 1] + t;
+        *reinterpret_cast<float4*>(A.udt + blk * C * DN + 4 * e) = float4{w[0] * u[0], w[1] * u[LD], w[2] * u[2 * LD], w[3] * u[3 * LD]};
+    }
     // forward substitution, a column a thread: the values', then the keys'
     for (int c = tid; c < a.dv + DN; c += 256) {
-        float x[C];
-        if (c < a.dv) {
-            const float* v = a.v + (long long)t0 * a.ldv + (long long)h * a.dv + c;
+        const bool value = c < a.dv;
+        const float* v = a.v + (long long)t0 * a.ldv + (long long)h * a.dv + c;
+        auto right = [&](int t) -> float { return value ? (t < nt ? v[(long long)t * a.ldv] : 0.0f) : t < C ? cw[t] * us[t * LD + c - a.dv] : 0.0f; };
+        float next[4];
 #pragma unroll
-            for (int t = 0; t < C; ++t) x[t] = t < nt ? v[(long long)t * a.ldv] * av[t] : 0.0f;
-        } else {
+        for (int i = 0; i < 4; ++i) next[i] = right(i);
+        for (int t = 0; t < C; t += 4) {
+            float x[4], y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int t = 0; t < C; ++t) x[t] = av[t] * cw[t] * us[t * LD + c - a.dv];
-        }
-#pragma unroll
-        for (int t = 1; t < C; ++t) {
-            float s0 = 0.0f, s1 = 0.0f;
-#pragma unroll
+            for (int i = 0; i < 4; ++i) { x[i] = next[i] * av[t + i]; next[i] = right(t + 4 + i); }
+#pragma unroll 2
             for (int s = 0; s < t; s += 4) {
-                const float4 a4 = *reinterpret_cast<const float4*>(am + t * LA + s);
-                s0 = fmaf(a4.x, x[s], s0);
-                if (s + 1 < t) s1 = fmaf(a4.y, x[s + 1], s1);
-                if (s + 2 < t) s0 = fmaf(a4.z, x[s + 2], s0);
-                if (s + 3 < t) s1 = fmaf(a4.w, x[s + 3], s1);
-            }
-            x[t] -= s0 + s1;
-        }
-        float* out = c < a.dv ? A.vt + blk * C * a.dv + c : A.ut + blk * C * DN + c - a.dv;
-        const int ld = c < a.dv ? a.dv : DN;
+                float xv[4];
 #pragma unroll
-        for (int t = 0; t < C; ++t) out[t * ld] = x[t];
+                for (int j = 0; j < 4; ++j) xv[j] = xs[s + j][tid];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float4 a4 = *reinterpret_cast<const float4*>(am + (t + i) * LA + s);
+                    y[i] = fmaf(a4.x, xv[0], y[i]); y[i] = fmaf(a4.y, xv[1], y[i]); y[i] = fmaf(a4.z, xv[2], y[i]); y[i] = fmaf(a4.w, xv[3], y[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int j = 0; j < i; ++j) y[i] = fmaf(am[(t + i) * LA + t + j], x[j], y[i]);
+                x[i] -= y[i];
+                xs[t + i][tid] = x[i];
+            }
+            if (value) *reinterpret_cast<float4*>(A.vt + (blk * a.dv + c) * C + t) = float4{x[0], x[1], x[2], x[3]};
+            else
+#pragma unroll
+                for (int i = 0; i < 4; ++i) A.ut[(blk * C + t + i) * DN + c - a.dv] = x[i];
+        }
     }
 }
 
-// grid (dv / 16, H), a wave per 16 key channels.  Wave w's accumulators are rows 16 w ... of the 16 columns of the state; a matrix instruction's four k entries may be
+// grid (H, dv / 16) -- the column blocks of a head, which read the same operands, fall on the same L2 where H is a multiple of the eight --, a wave per 16 key channels.  Wave w's accumulators are rows 16 w ... of the 16 columns of the state; a matrix instruction's four k entries may be
 // any four as long as both operands agree, so register r of the accumulators (rows 16 w + 4 g + r of lane group g) is the state's operand as it stands.  Per chunk:
 // every wave's share of U' S_0 and W Q S_0 meets in LDS, one wave per 16 x 16 tile of the two sums it, D = V' - U' S_0 goes to all, then the state's update everywhere
-// and the outputs' product with D in two waves.  Bound by this chain (two barriers a chunk); the next chunk's operands are requested a chunk ahead.
+// and the outputs' product with D in two waves.  Bound by this chain (two barriers a chunk, 1600 of 5200 cycles in matrix instructions); operands are requested two
+// chunks ahead (one: 76 us instead of 72 for 1024 tokens of 16 heads of 128 x 128).
 template <int DN>
-__global__ __launch_bounds__(4 * DN) void delta_chunk_walk_kernel(const DeltaArgs A) {
+__global__ __launch_bounds__(4 * DN, DN / 64) void delta_chunk_walk_kernel(const DeltaArgs A) {
     constexpr int C = kDeltaChunk, NW = DN / 16, LD = 18;     // (18: the four lane groups' rows of D fall into different banks)
     static_assert(NW >= 4, "a wave per summed tile");
     __shared__ __attribute__((aligned(16))) deltax4_t part[NW][4][64];
     __shared__ float dl[C * LD];
     const RecArgs& a = A.r;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m = lane & 15, g = lane >> 4;
-    const int h = blockIdx.y, c0 = blockIdx.x * 16;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x, c0 = blockIdx.y * 16;
     float* st = a.state + ((long long)h * DN + 16 * wave + 4 * g) * a.dv + c0 + m;
     deltax4_t S;
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[r] = a.pos0 > 0 ? st[(long long)r * a.dv] : 0.0f;
-    struct Operands { deltax4_t ut[2], qw[2], ud[2], x[2]; float wc; } cur, next;   // x: V' of waves 0 and 1 (x[0]), the outputs' product of waves 2 and 3
+    // x: V' of waves 0 and 1, the outputs' product of waves 2 and 3; every wave requests the same number of pieces at addresses that only advance from chunk to chunk
+    struct Operands { deltax4_t ut[2], qw[2], ud[2], x[2]; float wc; } op[3];
+    const long long b0 = h, xstep = (long long)a.H * C * (wave < 2 ? a.dv : C);
+    const float* utp = A.ut + (b0 * C + m) * DN + 16 * wave + 4 * g;
+    const float* qwp = A.qw + (b0 * C + m) * DN + 16 * wave + 4 * g;
+    const float* udp = A.udt + (b0 * DN + 16 * wave + m) * C + 8 * g;
+    const float* xp = wave < 2 ? A.vt + (b0 * a.dv + c0 + m) * C + 16 * wave + 4 * g : A.pm + (b0 * C + 16 * (wave & 1) + m) * C + 8 * g;
+    const int x1 = wave < 2 ? 0 : 4;
     auto request = [&](Operands& o, int n) {
-        const long long blk = (long long)n * a.H + h;
+        const long long at = (long long)n * a.H * C * DN;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            o.ut[i] = *reinterpret_cast<const deltax4_t*>(A.ut + (blk * C + 16 * i + m) * DN + 16 * wave + 4 * g);
-            o.qw[i] = *reinterpret_cast<const deltax4_t*>(A.qw + (blk * C + 16 * i + m) * DN + 16 * wave + 4 * g);
-            o.ud[i] = *reinterpret_cast<const deltax4_t*>(A.udt + (blk * DN + 16 * wave + m) * C + 8 * g + 4 * i);
+            o.ut[i] = *reinterpret_cast<const deltax4_t*>(utp + at + 16 * i * DN);
+            o.qw[i] = *reinterpret_cast<const deltax4_t*>(qwp + at + 16 * i * DN);
+            o.ud[i] = *reinterpret_cast<const deltax4_t*>(udp + at + 4 * i);
+            o.x[i] = *reinterpret_cast<const deltax4_t*>(xp + n * xstep + i * x1);
         }
-        o.wc = A.wc[blk];
-        if (wave < 2) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o.x[0][r] = A.vt[(blk * C + 16 * wave + 4 * g + r) * a.dv + c0 + m];
-        } else if (wave < 4) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) o.x[i] = *reinterpret_cast<const deltax4_t*>(A.pm + (blk * C + 16 * (wave - 2) + m) * C + 8 * g + 4 * i);
-        }
+        o.wc = A.wc[(long long)n * a.H + h];
     };
     auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };   // (requests to memory stay under way)
-    request(cur, 0);
-    for (int n = 0; n < A.chunks; ++n) {
-        if (n + 1 < A.chunks) request(next, n + 1);
+    deltax4_t o;
+    auto chunk = [&](const Operands& cur) {
         deltax4_t p[4] = {};
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -204,8 +226,11 @@ __global__ __launch_bounds__(4 * DN) void delta_chunk_walk_kernel(const DeltaArg
         meet();
         deltax4_t sum = {};
         if (wave < 4) {                                       // (uniform over the wave)
+            deltax4_t q[NW];
 #pragma unroll
-            for (int w = 0; w < NW; ++w) sum += part[w][wave][lane];
+            for (int w = 0; w < NW; ++w) q[w] = part[w][wave][lane];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) sum += q[w];
             if (wave < 2)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) dl[(16 * wave + 4 * g + r) * LD + m] = cur.x[0][r] - sum[r];
@@ -224,23 +249,45 @@ __global__ __launch_bounds__(4 * DN) void delta_chunk_walk_kernel(const DeltaArg
 #pragma unroll
             for (int j = 7; j >= 0; --j)
                 if (!(fabsf(d[j]) < INFINITY)) { bad = 8 * g + j; d[j] = 0.0f; }
-            bad = min(bad, __shfl_xor(bad, 16, 64));
-            bad = min(bad, __shfl_xor(bad, 32, 64));
+            if (__ballot(bad < C)) {
+                bad = min(bad, __shfl_xor(bad, 16, 64));
+                bad = min(bad, __shfl_xor(bad, 32, 64));
+            }
 #pragma unroll
             for (int j = 0; j < 8; ++j) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.x[j / 4][j % 4], d[j], sum, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * (wave - 2) + 4 * g + r, t = n * C + row;
-                if (t < a.T) a.out[(long long)t * a.ldo + (long long)h * a.dv + c0 + m] = row >= bad ? NAN : sum[r];
-            }
+            for (int r = 0; r < 4; ++r) o[r] = 16 * (wave - 2) + 4 * g + r >= bad ? NAN : sum[r];
         }
-        cur = next;
+    };
+    // a chunk's outputs are stored at the next one's start: the wait for its operands also waits for the stores before them, which are then long gone
+    auto store = [&](int n) {
+        if (wave != 2 && wave != 3) return;
+        float* p = a.out + (long long)n * C * a.ldo + (long long)h * a.dv + c0 + m;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * (wave - 2) + 4 * g + r;
+            if (n * C + row < a.T) p[(long long)row * a.ldo] = o[r];
+        }
+    };
+    const int last = A.chunks - 1;
+    request(op[0], 0);
+    request(op[1], min(1, last));
+    for (int n = 0; n <= last; n += 3) {
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            if (n + u > last) break;
+            if (n + u) store(n + u - 1);
+            request(op[(u + 2) % 3], min(n + u + 2, last));
+            chunk(op[u]);
+        }
     }
+    store(A.chunks - 1);
 #pragma unroll
     for (int r = 0; r < 4; ++r) st[(long long)r * a.dv] = S[r];
 }
 
-// The chunks take portions of at least one chunk whose rows can be read four floats at a time; everything else walks token by token.
+// The chunks take portions of at least one chunk whose rows can be read four floats at a time (150 tokens of the heads above: 33 us against 100);
+// everything else walks token by token.
 inline bool delta_chunked(const RecArgs& a) {
     return a.az && a.head_gates && a.write_gated && a.unit_k && !a.conv_w && a.T >= kDeltaChunk && (a.dn == 64 || a.dn == 128) && a.dv % 16 == 0 && a.ldq % 4 == 0 && a.ldk % 4 == 0 &&
            !(((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.packed) & 15) && a.H <= 65535;
@@ -259,7 +306,7 @@ static int launch_delta_chunks(const RecArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(delta_chunk_solve_kernel<DN>, dim3(A.chunks, a.H), dim3(256), 0, s, A);
     const int st = last_launch_status();
     if (st != NTK_OK) return st;
-    hipLaunchKernelGGL(delta_chunk_walk_kernel<DN>, dim3(a.dv / 16, a.H), dim3(4 * DN), 0, s, A);
+    hipLaunchKernelGGL(delta_chunk_walk_kernel<DN>, dim3(a.H, a.dv / 16), dim3(4 * DN), 0, s, A);
     return last_launch_status();
 }
 

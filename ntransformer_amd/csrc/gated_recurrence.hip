@@ -22,7 +22,8 @@
 //
 // The delta rule with one gate per head is the same walk with other vectors: S' = w S, S = S' - a u (u^T S') + a k v^T with a scalar w and a per head is
 // S = w S - (a u) ((w u)^T S) + k (a v)^T, so the pre-pass leaves (w u) where the walk takes the sum, (a u) where it removes, and a copy of the values
-// times a.  Unit queries and keys, q / k heads shared by several state heads and the per-head decay forms are the pre-pass's too.
+// times a.  Unit queries and keys, q / k heads shared by several state heads and the per-head decay forms are the pre-pass's too.  Longer portions of it, at the
+// widths models have, go 32 tokens at a time over the matrix instructions instead (delta_chunk.hip.h).
 #include <algorithm>
 #include "common.hip.h"
 #include "../../include/ntk_layers.h"

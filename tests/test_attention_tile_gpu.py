@@ -71,3 +71,21 @@ def test_a_towering_key_and_huge_scores():
     want = reference(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), 0, 1.0)
     err = np.abs(got.reshape(T, H, dv) - want)
     assert np.isfinite(got).all() and err.max() < 2e-3      # (scores up to ~500: 2^-24 * 68 * sum |q k| = 5e-3 of a weight between near-ties)
+
+
+@pytest.mark.parametrize("R,dr,H", [(12, 0, 1), (16, 4, 3), (500, 30, 16), (512, 64, 16), (64, 8, 17)])
+@pytest.mark.parametrize("T,pos0,window", [(1, 0, 0), (1, 63, 0), (1, 1300, 0), (1, 700, 129), (2, 64, 1), (7, 300, 64)])
+def test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, window):
+    """the form whose keys are the latents themselves: ranks off the operand sizes, no rotated part, one head and more heads than a tile, one key, windows, many splits"""
+    g = np.random.default_rng(R + T + pos0)
+    n = pos0 + T
+    q, cache = g.standard_normal((T, H, R + dr)).astype(np.float32), g.standard_normal((n, R + dr)).astype(np.float32)
+    scale = (R + dr) ** -0.5
+    got = Lr.latent_attention(q.reshape(T, -1), cache, R, dr, H, pos0, window, scale).reshape(T, H, R)
+    for t in range(T):
+        lo = max(0, pos0 + t - window + 1) if window else 0
+        keys = cache[lo:pos0 + t + 1].astype(np.float64)
+        s = q[t].astype(np.float64) @ keys.T * scale
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        want = (p / p.sum(axis=1, keepdims=True)) @ keys[:, :R]
+        assert np.abs(got[t] - want).max() < 2e-5 * np.abs(keys).max()
