@@ -361,7 +361,7 @@ int ntk_moe_pick(int* ids, float* wts, float* sgate, const float* z, int ldz, in
  *   out[t] = sum_s wts[t][s] * D_e act(U_e h[t])  (e = ids[t][s]; e >= experts: wts[t][s] * h[t])  + sgate[t] * Ds act(Us h[t])   (shared_up may be NULL; sgate NULL: 1)
  * up [experts][ff][n], down [experts][n][ff], shared_up [shared_ff][n], shared_down [n][shared_ff], all of dtype wdtype; mid: work space F32 [T][top * ff + shared_ff].
  * The first launch streams the chosen experts' and the shared unit's first matrices as one; the second walks a token's chosen second matrices as ONE row per output:
- * the activations, each times its expert's weight, sit side by side in LDS (top * ff + shared_ff <= NTK_MOE_FEW_MID). */
+ * the activations, each times its expert's weight, sit side by side in mid (top * ff + shared_ff <= NTK_MOE_FEW_MID). */
 #define NTK_MOE_FEW_MID 36864
 typedef struct ntk_moe_few_desc {
     float* out; int ldo;

@@ -230,8 +230,8 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(const DenseArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------- a few tokens' experts
-// Two launches for everything between a router and the sum of its experts (see ntk_moe_few).  Both stream weight rows like dense_gemv_kernel: a wave owns RW rows, the
-// next pass's 16 bytes per lane and row are requested before the current ones are used, the first ones ahead of the activations' way into LDS.
+// Two launches for everything between a router and the sum of its experts (see ntk_moe_few).  The first streams weight rows like dense_gemv_kernel: a wave
+// owns RW rows (pairs of rows), the next pass's 16 bytes per lane and row are requested before the current ones are used, the first ones ahead of the row's way into LDS.
 struct MoeFewArgs {
     float* out; int ldo;
     const float* h; int ldh;
