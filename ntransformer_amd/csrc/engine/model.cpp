@@ -674,6 +674,11 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
     const bool with_max = batched && bf16_now && row_max_ != nullptr && prefill_row_max_;
     float* rm_a = with_max ? row_max_ : nullptr;
     float* rm_b = with_max ? row_max_ + cfg_.max_seq_len : nullptr;
+    // what a projection may take from them: NULL unless the launch that wrote ITS input wrote (rm_b: and an earlier one of this layer cleared) the array -- a launch that
+    // splits its rows itself (below) does neither, and a matrix of another format that shares the input would scale by another pass's maxima
+    const float* max_a = nullptr;
+    const float* max_b = nullptr;
+    bool b_clear = false;
     // (round 6) ... or split X themselves: the projection then needs no pre-pass launch at all
     // (up to 64 tokens: a producer that owns a whole token per workgroup writes its planes in 16-byte pieces a kilobyte apart -- at 1024 tokens the pass
     // measured 5 % SLOWER than with the GEMM's own pre-pass, 8B Q8_0 28 010 -> 26 460 tok/s; at 16 - 64 tokens it is 2 - 5 % faster)
@@ -696,8 +701,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
     // to 64 bits as the one-token products' (1.6e-7 of the result both, 2.3e-7 against 2.8e-7 at 14336); at 1024 the latter are closer (0.95e-7 against 1.3e-7)
     auto project_half = [&](float* Y, const DevTensor& w, const float* X, size_t ystride, size_t xstride, bool accumulate, const float* rm) -> bool {
         if (!bf16_now || !w.ptr || w.dtype != NTK_DT_F16 || w.in_f < 4096 || ystride != (size_t)w.out_f || xstride != (size_t)w.in_f) return false;
-        ok(ntk_gemm_half(Y, w.ptr, X, T, (int)w.out_f, (int)w.in_f, accumulate ? 1 : 0, rm, gemm_ws_, gemm_ws_bytes_, s));
-        planes_of = nullptr;               // (the workspace held them)
+        void* ws = cur_ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_;   // (not the one that holds the planes of a quantised matrix's input)
+        if (!ws) { ws = cur_ws; planes_of = nullptr; }
+        ok(ntk_gemm_half(Y, w.ptr, X, T, (int)w.out_f, (int)w.in_f, accumulate ? 1 : 0, rm, ws, gemm_ws_bytes_, s));
         return true;
     };
     auto project = [&](float* Y, const DevTensor& w, const float* X, size_t ystride, size_t xstride, const float* rm) {
@@ -778,11 +784,19 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         project(residual_, w, X, H, xstride, rm);
         ok(ntk_add_inplace(hidden_, residual_, T * H, s));
     };
+    auto left_max = [&](bool written, bool zero_b) {   // a norm has written residual_ (zero_b: the layer's first, which clears rm_b if it leaves maxima at all)
+        max_a = written ? rm_a : nullptr;
+        if (zero_b) b_clear = written && rm_b;
+    };
     auto norm = [&](const DevTensor& nw, bool zero_b, const DevTensor& next_w) {
         if (fuse_split && f16_ok(next_w) && (int)next_w.in_f == H) {
             ok(ntk_rmsnorm_prepare_x(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, flip_ws(), s));
             planes_ready = residual_;
-        } else if (with_max) ok(ntk_rmsnorm_rowmax(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, rm_a, zero_b ? rm_b : nullptr, s));
+            left_max(false, zero_b);
+            return;
+        }
+        left_max(with_max, zero_b);
+        if (with_max) ok(ntk_rmsnorm_rowmax(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, rm_a, zero_b ? rm_b : nullptr, s));
         else ok(ntk_rmsnorm(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, s));
     };
     // hidden += W . X followed by the NEXT RMSNorm (nw; into residual_, with the token maxima) as one consumer launch of the projection's K splits
@@ -808,8 +822,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         if (st == NTK_OK && fuse_split && f16_ok(next_w) && (int)next_w.in_f == H) {   // (the partial sums lie in cur_ws: the planes go to the other one)
             st = ntk_reduce_rmsnorm_prepare_x(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, flip_ws(), s);
             planes_ready = residual_;
+            left_max(false, zero_b);
         } else
-        if (st == NTK_OK) st = ntk_reduce_rmsnorm_rowmax(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, rm_a, zero_b ? rm_b : nullptr, s);
+        if (st == NTK_OK) left_max(true, zero_b), st = ntk_reduce_rmsnorm_rowmax(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, rm_a, zero_b ? rm_b : nullptr, s);
         ok(st);
         return true;
     };
@@ -825,7 +840,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         {
             float* const ys[3] = {q_buf, k_buf, v_buf};
             const DevTensor* const ws[3] = {&L.wq, &L.wk, &L.wv};
-            project_many(ys, ws, 3, residual_, rm_a);
+            project_many(ys, ws, 3, residual_, max_a);
         }
         if (with_max && T >= 4 && hd <= 256) {   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
             ok(ntk_rope_kv_store(q_buf, k_buf, v_buf, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc,
@@ -845,6 +860,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         // gate | up and SiLU x up (per token in the reference, ffn.cpp:127: the same elementwise op): with the token maxima, the gate | up launch's K
         // splits are summed by the SiLU launch itself (ntk_gemm_quant_f16 with `partials` + ntk_reduce_silu_mul_rowmax)
         bool ffn_done = false;
+        max_b = nullptr;
         if (with_max && rm_b && tp_world_ == 1 && L.w_gate.dtype == L.w_up.dtype && is_quant(L.w_gate.dtype) && L.w_gate.in_f == L.w_up.in_f &&
             (size_t)L.w_gate.out_f == (size_t)I && (size_t)L.w_up.out_f == (size_t)I && I % 4 == 0) {
             const bool both_rp = rp_only(L.w_gate) && rp_only(L.w_up);
@@ -852,13 +868,13 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
             ntk_gemv_seg segs[2] = {{both_rp ? L.w_gate.rp : raw_of(L.w_gate), gate_buf, (int)I, L.w_gate.dtype},
                                     {both_rp ? L.w_up.rp : raw_of(L.w_up), up_buf, (int)I, L.w_up.dtype}};
             ntk_gemm_partials pt;
-            int st = gemm_f16(segs, 2, residual_, (int)L.w_gate.in_f, nullptr, residual_ == planes_of ? 1 : 0, rm_a, &pt, both_rp);
+            int st = gemm_f16(segs, 2, residual_, (int)L.w_gate.in_f, nullptr, residual_ == planes_of ? 1 : 0, max_a, &pt, both_rp);
             if (st != NTK_E_DTYPE && st != NTK_E_SHAPE && st != NTK_E_ALIGN) {   // (those three: nothing was launched)
                 if (st == NTK_OK && fuse_split && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I) {
                     st = ntk_reduce_silu_mul_prepare_x(gate_buf, &pt, flip_ws(), s);
                     planes_ready = gate_buf;
                 } else
-                if (st == NTK_OK) st = ntk_reduce_silu_mul_rowmax(gate_buf, &pt, rm_b, s);
+                if (st == NTK_OK) st = ntk_reduce_silu_mul_rowmax(gate_buf, &pt, rm_b, s), max_b = b_clear ? rm_b : nullptr;
                 ok(st);
                 ffn_done = true;
             }
@@ -866,8 +882,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         if (!ffn_done) {
             float* const ys[2] = {gate_buf, up_buf};
             const DevTensor* const ws[2] = {&L.w_gate, &L.w_up};
-            project_many(ys, ws, 2, residual_, rm_a);
+            project_many(ys, ws, 2, residual_, max_a);
             int st_silu = with_max && rm_b ? ntk_silu_mul_rowmax(gate_buf, gate_buf, up_buf, T, I, rm_b, s) : NTK_E_SHAPE;
+            if (st_silu == NTK_OK && b_clear) max_b = rm_b;
             if (fuse_split && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I && tp_world_ == 1) {
                 st_silu = ntk_silu_mul_prepare_x(gate_buf, gate_buf, up_buf, T, I, flip_ws(), s);
                 if (st_silu == NTK_OK) planes_ready = gate_buf;
@@ -878,8 +895,8 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         planes_of = planes_ready;
         planes_ready = nullptr;
         // down projection + residual, and the NEXT layer's first RMSNorm in the same consumer launch when there is a next layer in this pass
-        if (i + 1 < last_layer && project_add_norm(L.w_down, gate_buf, rm_b, layers_[i + 1].attn_norm, true, layers_[i + 1].wq)) normed_ahead = true;
-        else project_add(L.w_down, gate_buf, I, rm_b);
+        if (i + 1 < last_layer && project_add_norm(L.w_down, gate_buf, max_b, layers_[i + 1].attn_norm, true, layers_[i + 1].wq)) normed_ahead = true;
+        else project_add(L.w_down, gate_buf, I, max_b);
         if (rc != NTK_OK) break;
     }
     if (raw_err_ != NTK_OK) { rc = raw_err_; raw_err_ = NTK_OK; }   // what raw_of() could not report through its pointer (it precedes the consumer's NTK_E_NULL)
