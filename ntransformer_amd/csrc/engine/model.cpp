@@ -883,11 +883,13 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
             float* const ys[2] = {gate_buf, up_buf};
             const DevTensor* const ws[2] = {&L.w_gate, &L.w_up};
             project_many(ys, ws, 2, residual_, max_a);
-            int st_silu = with_max && rm_b ? ntk_silu_mul_rowmax(gate_buf, gate_buf, up_buf, T, I, rm_b, s) : NTK_E_SHAPE;
-            if (st_silu == NTK_OK && b_clear) max_b = rm_b;
+            int st_silu = NTK_E_SHAPE;   // (in place: exactly one of these launches runs)
             if (fuse_split && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I && tp_world_ == 1) {
                 st_silu = ntk_silu_mul_prepare_x(gate_buf, gate_buf, up_buf, T, I, flip_ws(), s);
                 if (st_silu == NTK_OK) planes_ready = gate_buf;
+            } else if (with_max && rm_b) {
+                st_silu = ntk_silu_mul_rowmax(gate_buf, gate_buf, up_buf, T, I, rm_b, s);
+                if (st_silu == NTK_OK && b_clear) max_b = rm_b;
             }
             if (st_silu == NTK_E_SHAPE || st_silu == NTK_E_ALIGN) { st_silu = ntk_silu_mul(gate_buf, gate_buf, up_buf, T * I, s); rm_b = nullptr; }   // (then for the rest of the pass)
             ok(st_silu);

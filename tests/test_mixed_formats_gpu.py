@@ -72,3 +72,18 @@ def test_a_prompt_does_not_depend_on_the_prompts_before_it(formats, boost, tmp_p
     eng = loaded(path, batched_prefill=0)
     assert near(fresh, eng.forward(short, 0))
     eng.close()
+
+
+@pytest.mark.parametrize("gate,up", [("Q8_0", "Q4_0"), ("Q4_K", "Q6_K"), ("F16", "F16"), ("F32", "Q8_0")])
+@pytest.mark.parametrize("T", [2, 40, 64, 65])
+def test_gate_and_up_of_two_formats_in_front_of_a_quantised_down(gate, up, T, tmp_path, monkeypatch):
+    """the gated activation is formed once, whichever launch forms it"""
+    path = str(tmp_path / "m.gguf")
+    make(path, G.SMALL, ("Q8_0", "Q8_0", "Q8_0", "Q8_0", gate, up, "Q8_0"), monkeypatch)
+    prompt = list(range(1, T + 1))
+    got = []
+    for batched in (1, 0):
+        eng = loaded(path, batched_prefill=batched)
+        got.append(eng.forward(prompt, 0))
+        eng.close()
+    assert near(*got)
