@@ -514,8 +514,13 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
     t.T = d->T; t.N = d->N; t.K = d->K; t.accumulate = d->accumulate; t.act = d->act; t.part = d->scratch;
     const int align = bf ? 8 : 4;
     const bool vec = (d->K % align == 0) && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->W & 15) && (d->wstride % align == 0);
-    if (!vec) {                            // (odd sizes and addresses: element by element into the same tiles)
-        if (bf) launch_tiles<TileBf16, 64, 64, 2, 2, 2, false>(t, 1, s);
+    if (!vec) {
+        // odd sizes and addresses, element by element into the tiles.  bf16: from three 64 x 64 tiles a CU on, twice the tile -- fewer element-wise readings of either operand: us at
+        // K = 2047 with 64 x 64 / 128 x 128: 1024 x 7488 556 / 346, 400 x 7488 (819 tiles) 269 / 201, 800 x 2048 (416) 147 / 197, 1024 x 2048 (512) 156 / 199; in 16
+        // groups of 2815 outputs 1600 rows 369 / 332, 600 rows 187 / 280
+        const int row_tiles = G > 1 ? d->T / 64 + (G + 1) / 2 : (d->T + 63) / 64;
+        if (bf && (long long)row_tiles * ((d->N + 63) / 64) > 768) launch_tiles<TileBf16, 128, 128, 1, 4, 2, false>(t, 1, s);
+        else if (bf) launch_tiles<TileBf16, 64, 64, 2, 2, 2, false>(t, 1, s);
         else launch_tiles<TileF32, 64, 64, 2, 2, 2, false>(t, 1, s);
         return last_launch_status();
     }

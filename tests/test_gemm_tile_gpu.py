@@ -51,6 +51,22 @@ def test_groups_of_every_size(dtype, sizes):
         assert within_bound(y[s], xr[order[s]], w[g]), g
 
 
+@pytest.mark.parametrize("T,N,K", [(833, 3841, 33), (1025, 3329, 40), (1600, 2049, 67)])
+def test_odd_sizes_in_many_tiles(T, N, K):
+    """element by element into the larger tiles (K = 40: rows that do not start on 16 bytes), alone and over rows in groups"""
+    x, w, xr = values("bfloat16", T, N, K, T)
+    if K == 40:
+        x = np.concatenate([x, np.full((T, 1), np.nan, np.float32)], axis=1)
+    assert within_bound(Lr.dense(x, w, "bfloat16"), xr, w)
+    sizes = (T // 2 + 3, 0, 129, T - T // 2 - 132)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    ws = bf16(np.random.default_rng(8).standard_normal((4, N, K)))
+    y = Lr.dense(x, ws, "bfloat16", offsets=off)
+    for g in range(4):
+        s = slice(off[g], off[g + 1])
+        assert within_bound(y[s], xr[s], ws[g]), g
+
+
 def test_an_activation_on_sums_of_pieces():
     x, w, xr = values("bfloat16", 40, 256, 4096, 1)
     y = Lr.dense(x, w, "bfloat16", act=Lr.ACT_RELU2, scratch_floats=16 * 40 * 256)
