@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const AttnArgs a)
 // of a quarter of the columns.  The tiles of 32 keys go round `splits` workgroups; each leaves one (max, sum, vector) state per row and latent_attention_merge_kernel adds
 // them.  Latency bounds it: launch, one round trip for tile and queries, ~70 matrix instructions, softmax, ~64 more, the states out.  With the products on the vector
 // units (one LDS read per two FMAs) and the tile in three round trips 1100 positions took 21.4 us, now 12.2.
-constexpr int KB = 32, SROWS = 16, SSTEPS = 13;    // keys of (latent + rotated) up to 4 * 16 * SSTEPS = 832 entries
+constexpr int KB = 32, SROWS = 16;
 struct SharedArgs {
     const float* q; int ldq;          // [T][H][R + dr], ldq floats between tokens
     const float* cache; int row;      // cache rows
@@ -219,7 +219,12 @@ struct SharedArgs {
     float* scratch;                   // [rows][splits][2 + R]
 };
 
+// SSTEPS: keys of (latent + rotated) up to 64 * SSTEPS entries; CT: ranks up to 64 * CT.  Three sizes of it: registers for 832 entries leave a SIMD one wave, which is enough for
+// the few workgroups of a decoded token but not where many rows walk a long context.  8 tokens of 64 heads at 8000 positions, latents of 32 + 8: 293 us in the largest
+// size, 121 in the smallest (vector form 158); 256 + 32: 338 -> 156 (262); one token of 16 heads of 64 + 16: 25.7 -> 22.2 (30.5).
+template <int SSTEPS, int CT>
 __global__ __launch_bounds__(256) void latent_attention_shared_kernel(const SharedArgs a) {
+    constexpr int LOADS = 2 * SSTEPS < 20 ? 2 * SSTEPS : 20;       // quads of a row that a thread requests together
     typedef float f4 __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int PP = KB + 4;
@@ -257,8 +262,7 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(const Shar
     if (tid < SROWS) { ms[tid] = -INFINITY; ls[tid] = 0.0f; }
     const int srow = tid >> 4, sub = tid & 15;     // softmax: sixteen threads per row, two keys each
     const int rpos = row0 + srow < n_rows ? a.pos0 + (row0 + srow) / a.H : -1;
-    constexpr int CT = 8;                          // tiles of 16 columns per wave: R <= 512
-    f4 acc[CT];
+    f4 acc[CT];                                    // tiles of 16 columns per wave
 #pragma unroll
     for (int t = 0; t < CT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
     const int col0 = wave * ((((a.R + 15) / 16 + 3) / 4) * 16);           // the wave's columns
@@ -271,16 +275,16 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(const Shar
         __syncthreads();                           // the previous tile is used up (and ms is written)
         const float* src = a.cache + (long long)(j0 + min(lk, nk - 1)) * a.row;     // (keys past the last re-read it; their weight is zero)
         if (vec4) {
-            for (int c0 = lc; 4 * c0 < D16; c0 += 8 * 20) {
-                f4 v[20];
+            for (int c0 = lc; 4 * c0 < D16; c0 += 8 * LOADS) {
+                f4 v[LOADS];
 #pragma unroll
-                for (int u = 0; u < 20; ++u) {
+                for (int u = 0; u < LOADS; ++u) {
                     const int d = 4 * (c0 + 8 * u);
                     v[u] = f4{0.f, 0.f, 0.f, 0.f};
                     if (d < DK) v[u] = *reinterpret_cast<const f4*>(src + d);
                 }
 #pragma unroll
-                for (int u = 0; u < 20; ++u)
+                for (int u = 0; u < LOADS; ++u)
                     if (4 * (c0 + 8 * u) < D16) *reinterpret_cast<f4*>(&Ks[lk * DKP + 4 * (c0 + 8 * u)]) = v[u];
             }
         } else {
@@ -526,8 +530,11 @@ int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const flo
         if (((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) > 156 * 1024) return NTK_E_SHAPE;     // (keys of up to 812 entries)
         const size_t lds = ((size_t)KB * (((DK + 15) & ~15) + 4) + 5 * SROWS * (KB + 4) + 3 * SROWS) * sizeof(float);
         static bool raised_s = false;   // (idempotent: a race sets the same attribute twice)
-        if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
-        hipLaunchKernelGGL(latent_attention_shared_kernel, dim3((rows + SROWS - 1) / SROWS, sa.splits), dim3(256), lds, s, sa);
+        if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel<13, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
+        const dim3 grid((rows + SROWS - 1) / SROWS, sa.splits);
+        if (DK <= 128) hipLaunchKernelGGL((latent_attention_shared_kernel<2, 2>), grid, dim3(256), lds, s, sa);
+        else if (DK <= 320) hipLaunchKernelGGL((latent_attention_shared_kernel<5, 5>), grid, dim3(256), lds, s, sa);
+        else hipLaunchKernelGGL((latent_attention_shared_kernel<13, 8>), grid, dim3(256), lds, s, sa);
         int st = last_launch_status();
         if (st != NTK_OK) return st;
         hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(rows, (kv_rank + 63) / 64), dim3(256), 0, s, out, ldo, (const float*)scratch, sa.splits, kv_rank, H);

@@ -89,3 +89,10 @@ def test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, wind
         p = np.exp(s - s.max(axis=1, keepdims=True))
         want = (p / p.sum(axis=1, keepdims=True)) @ keys[:, :R]
         assert np.abs(got[t] - want).max() < 2e-5 * np.abs(keys).max()
+
+
+@pytest.mark.parametrize("R,dr", [(128, 0), (120, 8), (129, 0), (125, 4), (320, 0), (256, 64), (321, 0), (300, 21)])
+@pytest.mark.parametrize("T,H,pos0,window", [(1, 1, 0, 0), (3, 5, 95, 0), (8, 16, 200, 70)])
+def test_shared_latents_at_the_limits_of_the_operand_sizes(R, dr, H, T, pos0, window):
+    """keys of 128 and 320 entries and one past them, with and without a rotated part"""
+    test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, window)
