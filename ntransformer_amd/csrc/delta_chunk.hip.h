@@ -286,10 +286,11 @@ __global__ __launch_bounds__(4 * DN, DN / 64) void delta_chunk_walk_kernel(const
     for (int r = 0; r < 4; ++r) st[(long long)r * a.dv] = S[r];
 }
 
-// The chunks take portions of at least one chunk whose rows can be read four floats at a time (150 tokens of the heads above: 33 us against 100);
-// everything else walks token by token.
+// The chunks take portions whose rows can be read four floats at a time (150 tokens of the heads above: 33 us against 100); everything else walks token by token.
+// From a chunk and a half on: the two launches take 17 - 25 us however short the portion is (us, walk / chunks: 32 tokens of 16 heads of 128 x 128 20.1 / 21.9, 33: 21.6 / 23.9, 48:
+// 26.3 / 24.1, 64: 32.9 / 24.5; 64 x 128 15.3 / 17.7, 48: 19.7 / 19.0), from two on with wider values, whose substitution goes more than one round (256: 48 tokens 24.8 / 29.6, 64: 30.8 / 30.1).
 inline bool delta_chunked(const RecArgs& a) {
-    return a.az && a.head_gates && a.write_gated && a.unit_k && !a.conv_w && a.T >= kDeltaChunk && (a.dn == 64 || a.dn == 128) && a.dv % 16 == 0 && a.ldq % 4 == 0 && a.ldk % 4 == 0 &&
+    return a.az && a.head_gates && a.write_gated && a.unit_k && !a.conv_w && a.T >= (a.dv > 128 ? 2 * kDeltaChunk : kDeltaChunk * 3 / 2) && (a.dn == 64 || a.dn == 128) && a.dv % 16 == 0 && a.ldq % 4 == 0 && a.ldk % 4 == 0 &&
            !(((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.packed) & 15) && a.H <= 65535;
 }
 

@@ -318,6 +318,12 @@ def test_delta_rule_in_chunks_on_the_matrix_instructions(H, G, dn, dv, T):
     assert rel(a[:at], ref[:at]) < 1e-5 and np.isnan(a[at:]).all() and np.isnan(st).all()
 
 
+@pytest.mark.parametrize("H,G,dn,dv,T", [(2, 1, 64, 48, 47), (2, 1, 64, 48, 48), (3, 3, 128, 128, 49), (2, 2, 128, 144, 63), (2, 2, 128, 144, 64), (1, 1, 64, 256, 97)])
+def test_delta_rule_where_chunks_take_over_from_the_walk(H, G, dn, dv, T):
+    """portions around the length from which the chunks are taken, for values up to 128 and wider, against the reference and behind a state"""
+    test_delta_rule_in_chunks_on_the_matrix_instructions(H, G, dn, dv, T)
+
+
 @pytest.mark.parametrize("H,G,dn,dv,taps", [(4, 2, 8, 8, 4), (6, 3, 32, 64, 4), (3, 3, 13, 7, 2), (2, 1, 70, 130, 5), (5, 1, 16, 300, 1), (2, 2, 128, 96, 16)])
 def test_decoded_tokens_pass_their_convolutions_inside_the_recurrence(H, G, dn, dv, taps):
     """raw q, k, v of one token at a time, the short convolutions inside the pre-pass's launch: the same outputs, state and carried inputs as the convolution as an
