@@ -9,7 +9,7 @@ from ntransformer_amd import layers as Lr
 pytestmark = pytest.mark.gpu
 
 
-def reference(q, k, v, pos0, scale, window=0, chunks=False, keep=0, cap=0.0, sinks=None, slopes=None):
+def reference(q, k, v, pos0, scale, window=0, chunks=False, keep=0, cap=0.0, sinks=None, slopes=None, rel=None, bucket_of=None):
     T, H, _ = q.shape
     G = k.shape[1]
     out = np.zeros((T, H, v.shape[2]))
@@ -21,6 +21,8 @@ def reference(q, k, v, pos0, scale, window=0, chunks=False, keep=0, cap=0.0, sin
             vis &= ((j // window == p // window) if chunks else (p - j < window)) | (j < keep)
         for h in range(H):
             s = (k[:, h // (H // G)] @ q[t, h]) * scale
+            if rel is not None:
+                s = s + rel[bucket_of[np.clip(p - j, 0, len(bucket_of) - 1)], h]
             if slopes is not None:
                 s = s - slopes[h] * (p - j)
             if cap:
@@ -96,3 +98,62 @@ def test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, wind
 def test_shared_latents_at_the_limits_of_the_operand_sizes(R, dr, H, T, pos0, window):
     """keys of 128 and 320 entries and one past them, with and without a rotated part"""
     test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, window)
+
+
+@pytest.mark.parametrize("what", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("H,G,dn,dv,window,keep,option", [(2, 2, 64, 64, 0, 0, ""), (4, 1, 33, 17, 0, 0, "gate"), (2, 1, 128, 128, 20, 3, "cap_sink"), (3, 3, 192, 100, 33, 0, "slopes"),
+                                                          (4, 2, 40, 64, 48, 0, "chunks"), (2, 1, 16, 33, 0, 0, "rel"), (3, 1, 128, 36, 37, 0, "head_gate")])
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(H, G, dn, dv, window, keep, option, what):
+    """a position's value reaches the tokens it is visible to and no other, whatever shares their tiles, under every option of the scores and of the result; a visible one follows the
+    arithmetic (inf - inf, 0 * inf)"""
+    T, pos0 = 90, 7
+    q, k, v = values(T, pos0, H, G, dn, dv, 3)
+    g = np.random.default_rng(4)
+    k[60] -= 40.0 * q[55].mean(0)              # (a weight that may vanish in 32 bits)
+    for at, col in ((60, 1), (60, 9), (77, 16), (2, 4)):
+        v[at, 0, col] = what
+    v[61, 0, 9] = -what
+    kw, ref, factor = {}, {}, np.ones((T, H, dv))
+    if option == "cap_sink":
+        sk = g.standard_normal(H).astype(np.float32)
+        kw, ref = {"softcap": 3.0, "sinks": sk}, {"cap": 3.0, "sinks": sk.astype(np.float64)}
+    elif option == "slopes":
+        sl = np.exp2(-8.0 * (np.arange(H) + 1) / H).astype(np.float32)
+        kw, ref = {"slopes": sl}, {"slopes": sl.astype(np.float64)}
+    elif option == "rel":
+        kw = {"rel": g.standard_normal((5, H)).astype(np.float32), "bucket_of": np.minimum(np.arange(40) // 3, 4).astype(np.int32)}
+        ref = {"rel": kw["rel"].astype(np.float64), "bucket_of": kw["bucket_of"]}
+    elif "gate" in option:
+        gt = g.standard_normal((T, H if option == "head_gate" else H * dv)).astype(np.float32)
+        kw = {"gate": gt, "head_gate": option == "head_gate"}
+        factor = np.broadcast_to(1.0 / (1.0 + np.exp(-gt.astype(np.float64))).reshape(T, H, -1), (T, H, dv))
+    chunks = option == "chunks"
+    cache = np.concatenate([k.reshape(k.shape[0], -1), v.reshape(v.shape[0], -1)], 1)
+    got = Lr.window_attention(q.reshape(T, -1), cache, H, G, 1, dn, dv, pos0, window, 1.0 / np.sqrt(dn), split=False, keep_first=keep, chunks=chunks, **kw).reshape(T, H, dv)
+    clean = np.where(np.isfinite(v), v, 0.0).astype(np.float64)
+    want = reference(q.astype(np.float64), k.astype(np.float64), clean, pos0, 1.0 / np.sqrt(dn), window, chunks, keep, **ref) * factor
+    j = np.arange(pos0 + T)
+    for t in range(T):
+        p = pos0 + t
+        seen = (j <= p) & (((j // window == p // window) if chunks else (p - j < window)) | (j < keep) if window else True)
+        for h in range(H):
+            bad = (~np.isfinite(v[:, h // (H // G)]) & seen[:, None]).any(axis=0)
+            assert np.abs(got[t, h, ~bad] - want[t, h, ~bad]).max() < 2e-5 * np.abs(clean).max(), (t, h)
+            assert not np.isfinite(got[t, h, bad]).any(), (t, h)
+
+
+@pytest.mark.parametrize("what", [np.nan, np.inf])
+def test_latent_values_that_are_not_finite_stay_with_the_rows_that_see_them(what):
+    """the two-part keys of the expanded latent form, behind a first position that is not zero"""
+    T, pos0, key0, H, R, dr, dn, dv = 70, 50, 9, 2, 24, 8, 40, 48
+    g = np.random.default_rng(5)
+    f = lambda *s: g.standard_normal(s).astype(np.float32)
+    q, cache, k, v = f(T, H, dn + dr), f(pos0 + T, R + dr), f(pos0 + T - key0, H, dn), f(pos0 + T - key0, H, dv)
+    v[77 - key0, 1, 20] = what
+    got = Lr.latent_attention(q.reshape(T, -1), cache, R, dr, H, pos0, 42, (dn + dr) ** -0.5, K=k.reshape(len(k), -1), V=v.reshape(len(v), -1), key0=key0).reshape(T, H, dv)
+    keys = np.concatenate([np.zeros((key0, H, dn + dr)), np.concatenate([k, np.repeat(cache[key0:, None, R:], H, 1)], 2)]).astype(np.float64)
+    clean = np.concatenate([np.zeros((key0, H, dv)), np.where(np.isfinite(v), v, 0.0)]).astype(np.float64)
+    want = reference(q.astype(np.float64), keys, clean, pos0, (dn + dr) ** -0.5, 42)
+    hit = np.zeros(got.shape, bool)
+    hit[77 - pos0:77 - pos0 + 42, 1, 20] = True
+    assert np.abs(got[~hit] - want[~hit]).max() < 2e-5 * np.abs(clean).max() and not np.isfinite(got[hit]).any()
