@@ -3,7 +3,7 @@
  *
  * Same conventions as ntk.h: plain pointers and sizes, stream ordered, no allocation, NTK_OK or a negative NTK_E_* code.  Nothing here knows a
  * model: every size and constant is a parameter.  Two precisions of one operator set:
- *   weights NTK_DT_BF16 : matrix products on the bf16 matrix cores (activations rounded to bfloat16 at the product's input, F32 accumulation);
+ *   weights NTK_DT_BF16 : matrix products on the bf16 matrix cores (activations rounded to bfloat16 at the product's input, F32 accumulation; a few rows: F32 activations);
  *   weights NTK_DT_F32  : every product in true F32 (32-bit matrix instructions; a few rows: FMA on the vector units).
  * Norms, rotary angles, attention scores and weights, routers and the residual sum are F32 in both.
  */
@@ -56,6 +56,9 @@ typedef struct ntk_dense_desc {
     /* room for partial sums (16-byte aligned, scratch_bytes of it; NULL: none): with more than ntk_dense_few_rows() rows the inputs of a product may be cut into pieces that
      * run side by side, as many as the room holds ([pieces][T][N] floats).  Products on different streams need scratch of their own. */
     float* scratch; size_t scratch_bytes;
+    /* full_x != 0: activations keep their 32 bits beside bfloat16 weights with more than ntk_dense_few_rows() rows, too (three matrix instructions in place of one; meant for
+     * the experts of a few tokens, whose other products are of the few-row form) */
+    int full_x;
 } ntk_dense_desc;
 #define NTK_ACT_NONE 0
 #define NTK_ACT_RELU2 1

@@ -514,6 +514,11 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
     t.T = d->T; t.N = d->N; t.K = d->K; t.accumulate = d->accumulate; t.act = d->act; t.part = d->scratch;
     const int align = bf ? 8 : 4;
     const bool vec = (d->K % align == 0) && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->W & 15) && (d->wstride % align == 0);
+    if (bf && d->full_x) {                 // (a few tokens' rows: one small tile)
+        if (vec) launch_tiles<TileBf16x3, 32, 64, 2, 2, 2, true>(t, 1, s);
+        else launch_tiles<TileBf16x3, 32, 64, 2, 2, 2, false>(t, 1, s);
+        return last_launch_status();
+    }
     if (!vec) {
         // odd sizes and addresses, element by element into the tiles.  bf16: from three 64 x 64 tiles a CU on, twice the tile -- fewer element-wise readings of either operand: us at
         // K = 2047 with 64 x 64 / 128 x 128: 1024 x 7488 556 / 346, 400 x 7488 (819 tiles) 269 / 201, 800 x 2048 (416) 147 / 197, 1024 x 2048 (512) 156 / 199; in 16

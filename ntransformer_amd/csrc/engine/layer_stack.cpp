@@ -1169,9 +1169,11 @@ int LayerStackModel::run_lightning(const StackLayer& L, float* state, int T, int
     return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
-int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top) {
+int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
+                                 int full_x) {
     const int W = info_.width;
     ntk_dense_desc d{};
+    d.full_x = full_x;
     d.Y = gu; d.ldy = ex.in_rows(); d.X = h; d.ldx = W; d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype;
     d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top; d.T = rows; d.N = ex.in_rows(); d.K = W; d.accumulate = 0;
     if (ex.plain) {                       // the activation inside the product, whatever its form
@@ -1187,9 +1189,24 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
         LS_TRY(ntk_glu(act, gu, rows, ex.ff, ex.limit, glu_alpha, glu_up_offset, stream_));
     }
     d.add_y = nullptr;
+    d.full_x = full_x;
     d.Y = out; d.ldy = W; d.X = act; d.ldx = ex.ff; d.W = ex.down.ptr; d.wstride = ex.down.stride(); d.wdtype = ex.down.dtype;
     d.rows = nullptr; d.row_div = 1; d.N = W; d.K = ex.ff;
     return product(d);
+}
+
+// A few tokens' gated experts: two launches that read a matrix once per (token, choice), or six (grouping, two products each for the chosen and the shared units, their sum) that
+// read it once per chosen expert -- how many those are is taken as for choices that spread evenly.  The constants are us and bytes per us of both, fitted to 1 .. 8 tokens of
+// 2 .. 8 choices among 8 .. 128 experts of 1024 x 512 .. 4096 x 1408, with and without a shared unit, both weight types: the choice is the faster of the two within 12 % everywhere,
+// 0.2 % on average.  us in two launches / in six, bf16 experts of 2048 x 1408: 1 token of 6 among 32 24 / 31, 8 of 2 among 8 43 / 59, 4 of 4 among 8 44 / 60, 4 of 6 among 8
+// 63 / 60, 8 of 6 among 8 113 / 62, 8 of 6 among 16 118 / 83.
+static bool in_two_launches(const MoeFeedForward& M, int T, int W) {
+    const bool bf = M.routed.down.dtype == NTK_DT_BF16;
+    const double unit = 3.0 * W * (bf ? 2 : 4), share = (double)M.experts / (M.experts + M.identity), shared = M.has_shared ? M.shared.ff : 0;
+    const double chosen = M.experts * (1.0 - std::pow(1.0 - (double)M.top / (M.experts + M.identity), T));
+    const double two = 9.0 + unit * T * (M.top * share * M.routed.ff + shared) / 7.8e6;
+    const double six = 16.0 + unit * M.routed.ff * chosen / (bf ? 3.5e6 : 4.8e6) + (shared > 0 ? 11.0 + unit * T * shared / 9.0e6 : 0.0);
+    return two <= six;
 }
 
 // router, grouping, the experts' products; then either straight into the stream together with the mixer's output (parallel form) or as a sum of its own
@@ -1220,9 +1237,8 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
         owed_.y = nullptr;
     }
     LS_TRY(ntk_moe_route_ex(ids_, wts_, sgate, h, W, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
-    if (!M.routed.plain && T <= ntk_dense_few_rows() && mid <= NTK_MOE_FEW_MID && W <= NTK_MOE_FEW_MID && !(into_stream && M.identity)) {
-        // decoding: all of a token's gated units in two launches instead of six (grouping, two products each for the chosen and the shared units, their sum: 47 us a token and layer
-        // at 6 of 32 bf16 experts of 2048 x 1408 and a shared unit of 2816, 29 this way)
+    const bool few = !M.routed.plain && T <= ntk_dense_few_rows() && mid <= NTK_MOE_FEW_MID && W <= NTK_MOE_FEW_MID && !(into_stream && M.identity);
+    if (few && in_two_launches(M, T, W)) {
         ntk_moe_few_desc d{};
         d.out = into_stream ? x_ : ff_; d.ldo = W; d.h = h; d.ldh = W; d.ids = ids_; d.wts = wts_; d.top = M.top; d.experts = M.experts;
         d.up = M.routed.gate_up.ptr; d.down = M.routed.down.ptr; d.ff = M.routed.ff;
@@ -1233,8 +1249,8 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
         return ntk_moe_few(&d, stream_);
     }
     LS_TRY(ntk_moe_group(offsets_, order_, where_, ids_, T, M.top, choices, stream_));     // (identity experts come last: rows behind offsets_[experts], which no product visits)
-    LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.routed, h, gu_, act_, dn_, T * M.top, offsets_, order_, M.top));
-    if (M.has_shared) LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.shared, h, sgu_, sact_, sdn_, T, nullptr, nullptr, 1));
+    LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.routed, h, gu_, act_, dn_, T * M.top, offsets_, order_, M.top, few));
+    if (M.has_shared) LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.shared, h, sgu_, sact_, sdn_, T, nullptr, nullptr, 1, 0));
     if (into_stream) return ntk_moe_combine(x_, mix_, dn_, where_, wts_, M.has_shared ? sdn_ : nullptr, sgate, T, M.top, W, stream_);
     return ntk_moe_sum_ex(ff_, dn_, where_, M.identity ? ids_ : nullptr, M.experts, h, W, wts_, M.has_shared ? sdn_ : nullptr, sgate, T, M.top, W, stream_);
 }
@@ -1250,7 +1266,7 @@ int LayerStackModel::run_dense_ff(const StackLayer& L, int T) {
 
 // the dense gated unit (the experts' unit with one member, clipped or plain): gate and up in one product (decoding: the activation inside its launch), down -> ff_
 int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T) {
-    return run_experts(form_.clipped_glu ? kGluAlpha : 1.0f, form_.clipped_glu ? 1.0f : 0.0f, L.cff, h, gu2_, zf_, ff_, T, nullptr, nullptr, 1);
+    return run_experts(form_.clipped_glu ? kGluAlpha : 1.0f, form_.clipped_glu ? 1.0f : 0.0f, L.cff, h, gu2_, zf_, ff_, T, nullptr, nullptr, 1, 0);
 }
 
 // the delta rule with per-head gates: one product for [q | k | v | gate | beta | decay], the short convolutions of q, k and v (+ silu) with their carried

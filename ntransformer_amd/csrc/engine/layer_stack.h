@@ -334,7 +334,8 @@ private:
     int run_lightning(const StackLayer& L, float* state, int T, int pos0);
     int run_moe(const StackLayer& L, const float* h, int T, bool into_stream);
     int run_dense_ff(const StackLayer& L, int T);
-    int run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top);
+    int run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
+                    int full_x);
     int norm_conv(const NormW& nw, const float* canon, float* conv_state, float* out, int T, int pos0);
     int settle(int T);
     int first_product(ntk_dense_desc& d);

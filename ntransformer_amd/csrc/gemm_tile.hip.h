@@ -1,4 +1,4 @@
-// gemm_tile.hip.h -- one tiled product Y[r][n] = sum_k X[r][k] W[n][k] for three precisions of the same walk (F32 activations, dense row-major weights).
+// gemm_tile.hip.h -- one tiled product Y[r][n] = sum_k X[r][k] W[n][k] for four precisions of the same walk (F32 activations, dense row-major weights).
 //
 // A workgroup of WM x WN waves owns a TM x TN tile.  K goes by in chunks of 64 * SUB bytes per weight row: operands travel HBM / L2 -> registers (two chunks
 // requested ahead) -> LDS (two buffers, one barrier per chunk) -> matrix cores; activations are converted on their way into LDS.  What bounds such a product at a
@@ -45,20 +45,43 @@ struct TileArgs {
     const float* row_max;                           // TileHalf2: largest |x| of every activation row (no gathered rows then)
 };
 
-// ---- the three precisions: WT the stored weight, KE weights per 64 bytes, PIECES how many values stand for one activation.  RUN: the accumulators are added
+// ---- the four precisions: WT the stored weight, KE weights per 64 bytes, PIECES how many values stand for one activation.  RUN: the accumulators are added
 // onto a second set and start again from zero every RUN inputs -- as one chain of 32-bit additions a product of 4096 (14336) halves is off by 6e-7 (1.1e-6) of the result, in
 // runs of 128 by 1.6e-7 (2.3e-7), like the sums over 64 lanes of the one-token products (1.6e-7, 2.8e-7); 0: one chain (inputs rounded to eight bits dwarf it)
 struct TileBf16 {                                   // activations rounded to bfloat16
     using WT = uint16_t;
     static constexpr int KE = 32, EP = 8, PIECES = 1, RUN = 0;
+    static constexpr bool SCALED = false;
     __device__ static void convert(const float (&v)[EP], float, uintx4_t (&out)[PIECES]) {
         out[0] = uintx4_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
     }
     __device__ static floatx4_t mma(uintx4_t a, uintx4_t b, floatx4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bits_as<bf16x8_t>(a), bits_as<bf16x8_t>(b), c, 0, 0, 0); }
 };
+struct TileBf16x3 {                                 // bfloat16 weights, a 32-bit activation as the three bfloat16 values that add up to it
+    using WT = uint16_t;
+    static constexpr int KE = 32, EP = 8, PIECES = 3, RUN = 256;
+    static constexpr bool SCALED = false;
+    __device__ static void convert(const float (&v)[EP], float, uintx4_t (&out)[PIECES]) {
+        uint32_t u[EP];
+#pragma unroll
+        for (int i = 0; i < EP; ++i) u[i] = __float_as_uint(v[i]);
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q) {                  // cut, not rounded: eight bits a piece, nothing overflows; an infinity stays one, a NaN a NaN
+#pragma unroll
+            for (int i = 0; i < EP / 2; ++i) out[q][i] = (u[2 * i] >> 16) | (u[2 * i + 1] & 0xffff0000u);
+#pragma unroll
+            for (int i = 0; i < EP; ++i) {
+                const float x = __uint_as_float(u[i]), a = __uint_as_float(u[i] & 0xffff0000u);
+                u[i] = x == a ? 0u : __float_as_uint(x - a);
+            }
+        }
+    }
+    __device__ static floatx4_t mma(uintx4_t a, uintx4_t b, floatx4_t c) { return TileBf16::mma(a, b, c); }
+};
 struct TileF32 {                                    // everything in 32 bits: v_mfma_f32_16x16x4_f32, component c of both operands' 16 bytes at a time
     using WT = float;
     static constexpr int KE = 16, EP = 4, PIECES = 1, RUN = 256;
+    static constexpr bool SCALED = false;
     __device__ static void convert(const float (&v)[EP], float, uintx4_t (&out)[PIECES]) {
         out[0] = uintx4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
     }
@@ -78,6 +101,7 @@ __device__ __forceinline__ float half_unscale(float largest) { return __uint_as_
 struct TileHalf2 {                                  // IEEE-half weights, a 32-bit activation (times a power of two) as two halves: off by 2^-24 of it at most
     using WT = uint16_t;
     static constexpr int KE = 32, EP = 8, PIECES = 2, RUN = 128;
+    static constexpr bool SCALED = true;                // rows times half_scale(row_max)
     __device__ static void convert(const float (&v)[EP], float scale, uintx4_t (&out)[PIECES]) {
         halfx8_t hi, lo;
 #pragma unroll
@@ -147,7 +171,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
     for (int p = 0; p < PX; ++p) {
         const int r = min(row_base + lr + RP * p, r1 - 1), src = a.rows ? a.rows[r] / a.row_div : r;
         xrow[p] = a.X + (long long)src * a.ldx;
-        scale[p] = PIECES > 1 ? half_scale(a.row_max[src]) : 1.0f;
+        scale[p] = P::SCALED ? half_scale(a.row_max[src]) : 1.0f;
     }
 #pragma unroll
     for (int p = 0; p < PW; ++p) wrow[p] = W + (long long)min(n_base + lr + RP * p, a.N - 1) * a.K;
@@ -266,7 +290,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
     for (int i = 0; i < MI; ++i) {
         const int row = row_base + wm * (TM / WM) + i * 16 + (lane >> 4) * 4;
         float undo[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-        if constexpr (PIECES > 1)
+        if constexpr (P::SCALED)
 #pragma unroll
             for (int r = 0; r < 4; ++r) undo[r] = half_unscale(a.row_max[min(row + r, a.T - 1)]);
         if (a.splits > 1) {

@@ -21,7 +21,7 @@ class DenseDesc(C.Structure):
                 ("accumulate", C.c_int), ("glu_ff", C.c_int), ("glu_limit", C.c_float), ("glu_alpha", C.c_float),
                 ("norm_w", C.c_void_p), ("norm_eps", C.c_float), ("norm_offset", C.c_float), ("glu_up_offset", C.c_float), ("glu_cubic", C.c_float),
                 ("act", C.c_int), ("add_y", C.c_void_p), ("ld_add", C.c_int), ("add_w", C.c_void_p), ("add_eps", C.c_float), ("add_mult", C.c_float),
-                ("x_out", C.c_void_p), ("ldxo", C.c_int), ("scratch", C.c_void_p), ("scratch_bytes", C.c_size_t)]
+                ("x_out", C.c_void_p), ("ldxo", C.c_int), ("scratch", C.c_void_p), ("scratch_bytes", C.c_size_t), ("full_x", C.c_int)]
 
 
 class Rotary(C.Structure):
@@ -181,7 +181,7 @@ def _i(a) -> DeviceBuffer:
 
 def dense(x: np.ndarray, w: np.ndarray, dtype: str = "float32", offsets=None, rows=None, row_div: int = 1, n_rows: Optional[int] = None,
           y0: Optional[np.ndarray] = None, glu_limit: Optional[float] = None, glu_alpha: float = 1.702, norm_w: Optional[np.ndarray] = None,
-          norm_eps: float = 1e-6, norm_offset: float = 0.0, glu_up_offset: float = 1.0, glu_cubic: float = 0.0, act: int = ACT_NONE, add=None, scratch_floats: int = 0):
+          norm_eps: float = 1e-6, norm_offset: float = 0.0, glu_up_offset: float = 1.0, glu_cubic: float = 0.0, act: int = ACT_NONE, add=None, scratch_floats: int = 0, full_x: bool = False):
     """y[r] = x[src(r)] . w[g(r)]^T; w [N, K] or a stack [G, N, K] with `offsets` [G + 1]; rows: source row per output row (divided by row_div);
     y0: start values to accumulate onto; act: an activation on the result; add (few rows) = (add_y, add_w, eps, mult): the rows are first x + mult * rms(add_y) * add_w
     -> (y, those rows)."""
@@ -199,7 +199,7 @@ def dense(x: np.ndarray, w: np.ndarray, dtype: str = "float32", offsets=None, ro
     nb = _f(norm_w) if norm_w is not None else None
     if nb is not None:          # fused RMS norm of the activation rows (few rows)
         d.norm_w, d.norm_eps, d.norm_offset = nb.ptr, norm_eps, norm_offset
-    d.act = act
+    d.act, d.full_x = act, int(full_x)
     sb = DeviceBuffer(scratch_floats * 4) if scratch_floats else None
     if sb is not None:          # room for partial sums: the inputs may be cut into pieces
         d.scratch, d.scratch_bytes = sb.ptr, scratch_floats * 4

@@ -402,6 +402,24 @@ def test_other_sizes_and_degenerate_values(tmp_path, kw):
         e.close()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("kw", [dict(width=512, experts=4, top=4, ff=2048, shared_ff=16), dict(width=500, experts=3, top=3, ff=2051, shared_ff=0), dict(width=64, experts=8, top=2, ff=24, shared_ff=8)])
+def test_a_few_tokens_through_grouped_products_or_two_launches(tmp_path, dtype, kw):
+    """eight tokens at once (large experts that all of them choose: grouped products; small ones: two launches), and one by one (two launches): 32-bit activations either way, so
+    that bfloat16 weights, which hold these values exactly, are as close as 32-bit ones"""
+    cfg = O.small_config(layers=("latent_attention", "latent_attention_2"), **kw)
+    folder, w = make(tmp_path, cfg, seed=21)
+    toks = tokens_for(cfg, 8, seed=22)
+    ref = O.forward(cfg, w, toks).numpy()
+    e = engine_for(folder, dtype)
+    s = e.seq_acquire()
+    whole = e.seq_forward(s, toks)
+    e.seq_release(s)
+    s = e.seq_acquire()
+    one = np.concatenate([e.seq_forward(s, [t]) for t in toks])
+    assert rel(whole, ref) < 1e-5 and rel(one, ref) < 1e-5
+
+
 def test_long_decoding_from_one_token(tmp_path):
     cfg = O.small_config(window=40, **MIXED)
     folder, w = make(tmp_path, cfg, seed=13)

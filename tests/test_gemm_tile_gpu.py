@@ -51,6 +51,26 @@ def test_groups_of_every_size(dtype, sizes):
         assert within_bound(y[s], xr[order[s]], w[g]), g
 
 
+@pytest.mark.parametrize("T,N,K", [(9, 1, 8), (33, 65, 72), (48, 130, 520), (64, 64, 2056), (17, 100, 37), (12, 3, 4104), (70, 33, 515)])
+def test_activations_in_three_pieces(T, N, K):
+    """bfloat16 weights beside 32-bit activations at the edges of the tile, alone and in groups; rows of every magnitude; what is not finite stays in its row"""
+    x, w, _ = values("bfloat16", T, N, K, T + K)
+    x *= np.logspace(-25, 25, T).astype(np.float32)[:, None]
+    x[:, ::16] *= 3000.0
+    assert within_bound(Lr.dense(x, w, "bfloat16", full_x=True), x, w)
+    off = np.array([0, T // 3, T // 3, T], np.int32)
+    ws, order = bf16(np.random.default_rng(8).standard_normal((3, N, K))), np.random.default_rng(9).permutation(T).astype(np.int32)
+    y = Lr.dense(x, ws, "bfloat16", offsets=off, rows=order, row_div=1, full_x=True)
+    for g in range(3):
+        s = slice(off[g], off[g + 1])
+        assert within_bound(y[s], x[order[s]], ws[g]), g
+    x[3, 5], x[6, 2], x[7, 0] = np.inf, np.nan, 3.4028235e38
+    x[7, 1:] = 0.0
+    y = Lr.dense(x, w, "bfloat16", full_x=True)
+    keep = [r for r in range(T) if r not in (3, 6)]
+    assert within_bound(y[keep], x[keep], w) and np.isnan(y[6]).all() and not np.isfinite(y[3]).any()
+
+
 @pytest.mark.parametrize("T,N,K", [(833, 3841, 33), (1025, 3329, 40), (1600, 2049, 67)])
 def test_odd_sizes_in_many_tiles(T, N, K):
     """element by element into the larger tiles (K = 40: rows that do not start on 16 bytes), alone and over rows in groups"""
