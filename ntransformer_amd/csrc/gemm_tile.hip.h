@@ -91,10 +91,9 @@ struct TileF32 {                                    // everything in 32 bits: v_
         return c;
     }
 };
-// the power of two that brings a row's largest |x| into [2^14, 2^15) (1 for a row of zeros or one with an infinity), and its inverse
+// the power of two that brings a row's largest |x| into [2^14, 2^15) (at most 2^125; below 2^15 whatever finite values stand beside an infinity), and its inverse
 __device__ __forceinline__ float half_scale(float largest) {
     const int e = (int)(__float_as_uint(largest) >> 23) & 255;
-    if (e == 0 || e == 255) return 1.0f;
     return __uint_as_float((uint32_t)min(127 + 14 - (e - 127), 252) << 23);
 }
 __device__ __forceinline__ float half_unscale(float largest) { return __uint_as_float((254u << 23) - __float_as_uint(half_scale(largest))); }

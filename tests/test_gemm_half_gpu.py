@@ -62,6 +62,21 @@ def test_infinities_stay_in_their_row():
     assert np.array_equal(y[3], np.where(w[:, 5] == 0, np.nan, np.sign(w[:, 5]) * np.inf).astype(np.float32), equal_nan=True)
 
 
+def test_large_values_beside_an_infinity_and_rows_of_subnormals():
+    """a row with an infinity: its finite values stay finite, whatever their size, so every result has the infinity's sign; a row whose largest value is subnormal is not lost"""
+    x, w = values(9, 64, 128, 6)
+    x[3, 5] = np.inf
+    x[3, 20:28] = np.array([7e4, -7e4, 1e9, -1e9, 3e38, -3e38, 65520.0, -65520.0], np.float32)
+    x[5] *= np.float32(2.0 ** -128)
+    for given_max in (False, True):
+        y = run(x, w, given_max=given_max)
+        assert np.array_equal(y[3], np.where(w[:, 5] == 0, np.nan, np.sign(w[:, 5]) * np.inf).astype(np.float32), equal_nan=True)
+        want = x[5].astype(np.float64) @ w.T.astype(np.float64)
+        assert np.abs(y[5] - want).max() < 1e-3 * np.abs(want).max()
+        rows = [r for r in range(9) if r not in (3, 5)]
+        assert within_bound(y[rows], x[rows], w)
+
+
 def test_what_it_refuses():
     L = _lib.lib()
     b = ops.DeviceBuffer(4096)
