@@ -74,6 +74,21 @@ def test_a_prompt_does_not_depend_on_the_prompts_before_it(formats, boost, tmp_p
     eng.close()
 
 
+@pytest.mark.parametrize("T", [2, 3, 9, 70])
+def test_half_precision_prompts(T, tmp_path, monkeypatch):
+    """every matrix in F16: the tiles with the maxima that norms and activations leave, on their own and summed onto the stream, against the one-token products; a short pass
+    behind a longer one"""
+    path = str(tmp_path / "m.gguf")
+    make(path, WIDE, ("F16",) * 7, monkeypatch)
+    got = []
+    for batched in (1, 0):
+        eng = loaded(path, batched_prefill=batched)
+        eng.forward(PLAIN, 0)
+        got.append(eng.forward(TOWERING[:T], 0))
+        eng.close()
+    assert near(*got)
+
+
 @pytest.mark.parametrize("gate,up", [("Q8_0", "Q4_0"), ("Q4_K", "Q6_K"), ("F16", "F16"), ("F32", "Q8_0")])
 @pytest.mark.parametrize("T", [2, 40, 64, 65])
 def test_gate_and_up_of_two_formats_in_front_of_a_quantised_down(gate, up, T, tmp_path, monkeypatch):
