@@ -373,7 +373,7 @@ __global__ __launch_bounds__(256) void moe_few_down_kernel(const MoeFewArgs a) {
         seg = a.top + 1;
     };
     auto settle = [&]() {                                     // k0 counts on past a segment's last pass into the next one's
-        while (seg <= a.top && k0 >= len) { k0 -= (len + 511) & ~511; next_segment(); if (k0 < 0) k0 = 0; }
+        while (seg <= a.top && k0 >= len) { k0 -= (len + 511) & ~511; next_segment(); }
     };
     float s[RW];
 #pragma unroll
@@ -417,10 +417,36 @@ __global__ __launch_bounds__(256) void moe_few_down_kernel(const MoeFewArgs a) {
             }
         }
     } else {
-        for (; seg <= a.top; next_segment())
-            for (int k = tid; k < len; k += 256)
+        if (a.ff >= 512) {
+            for (; seg <= a.top; next_segment())
+                for (int k = tid; k < len; k += 256)
 #pragma unroll
-                for (int i = 0; i < RW; ++i) s[i] = fmaf(weight_value(mat + (long long)min(i0 + i, a.n - 1) * len + k), mid[(seg < a.top ? seg * a.ff : routed) + k], s[i]);
+                    for (int i = 0; i < RW; ++i) s[i] = fmaf(weight_value(mat + (long long)min(i0 + i, a.n - 1) * len + k), mid[(seg < a.top ? seg * a.ff : routed) + k], s[i]);
+        } else
+        // (short segments: entries of all as one row, four under way -- segment by segment each one's first entries are waited for: 6 choices of 33, width 300: 10.0 us / 7.7; of 1403, width 1001,
+        // 28 / 36)
+        for (int e0 = tid; e0 < K; e0 += 4 * 256) {
+            float x[4], w[4][RW];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int e = e0 + 256 * u, sl = e < routed ? e / a.ff : a.top, id = e < routed ? ids[sl] : 0;
+                const bool in = e < K && (sl == a.top || (id >= 0 && id < a.experts));
+                x[u] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < RW; ++i) w[u][i] = 0.0f;
+                if (in) {
+                    const int k = sl < a.top ? e - sl * a.ff : e - routed, width = sl < a.top ? a.ff : a.shared_ff;
+                    const WT* m = sl < a.top ? (const WT*)a.down + (long long)id * a.n * a.ff : (const WT*)a.shared_down;
+                    x[u] = mid[e];
+#pragma unroll
+                    for (int i = 0; i < RW; ++i) w[u][i] = weight_value(m + (long long)min(i0 + i, a.n - 1) * width + k);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < RW; ++i) s[i] = fmaf(w[u][i], x[u], s[i]);
+        }
     }
 #pragma unroll
     for (int i = 0; i < RW; ++i) {

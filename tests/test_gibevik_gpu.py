@@ -361,6 +361,13 @@ def test_a_few_tokens_gated_experts_into_a_stream(dtype, T, n, E, ff, top, sff):
         assert rel(got, ref) < 1e-5, identity     # (the bound of the ungated form: products of at most 11 264 terms in 32 bits)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,n,E,ff,top,sff", [(2, 65, 6, 300, 5, 101), (8, 9, 3, 511, 3, 0), (1, 3, 4, 1, 4, 1), (3, 33, 5, 515, 2, 11), (2, 17, 3, 513, 3, 700)])
+def test_a_few_tokens_experts_of_odd_sizes(dtype, T, n, E, ff, top, sff):
+    """entry by entry, short segments as one row (more than a round of four under way, a single entry) and longer ones one by one, identity experts among the choices"""
+    test_a_few_tokens_gated_experts_into_a_stream(dtype, T, n, E, ff, top, sff)
+
+
 def test_weighted_sum_with_identity_experts():
     from ntransformer_amd import layers as Lr
     g = np.random.default_rng(6)
