@@ -2,8 +2,9 @@
 // Replaces, for a prompt, the reference's loop of one GEMV per token (attention.cu / ffn.cpp through gemm.cu:32-470): 200 tokens read the weights 200 times, 18 ms a
 // layer of an 8B-shaped F16 model against 0.47 ms as tiles (gemm_tile.hip.h); a 200-token pass of eight such layers 144.5 -> 4.1 ms.  Taken from two tokens on: 16 tokens
 // through a 4096 x 4096 matrix take 15 us, one token's GEMV 12.  Products on v_mfma_f32_16x16x32_f16; a 32-bit activation goes in as two halves after
-// a per-token power of two (largest |x| in [2^14, 2^15)), which leaves 2^-24 of the value: the
-// rounding of the 32-bit products that they replace (error of a 4096-input product against 64 bits: 1.6e-7 of the result both ways).
+// a per-token power of two (largest |x| in [2^14, 2^15)), which is off by at most 2^-23 of the value (a quarter of them by more than 2^-24, where the one-token
+// products take all 24 bits), or by 2^-39 of the row's largest where the second half is subnormal.  Sums in short runs make up for it (error of a 4096-input product against 64 bits: 1.6e-7
+// of the result both ways).
 #include "gemm_tile.hip.h"
 
 namespace ntk {

@@ -97,7 +97,7 @@ __device__ __forceinline__ float half_scale(float largest) {
     return __uint_as_float((uint32_t)min(127 + 14 - (e - 127), 252) << 23);
 }
 __device__ __forceinline__ float half_unscale(float largest) { return __uint_as_float((254u << 23) - __float_as_uint(half_scale(largest))); }
-struct TileHalf2 {                                  // IEEE-half weights, a 32-bit activation (times a power of two) as two halves: off by 2^-24 of it at most
+struct TileHalf2 {                                  // IEEE-half weights, a 32-bit activation (times a power of two) as two halves: off by 2^-23 of it, or 2^-39 of its row's largest, at most
     using WT = uint16_t;
     static constexpr int KE = 32, EP = 8, PIECES = 2, RUN = 128;
     static constexpr bool SCALED = true;                // rows times half_scale(row_max)
@@ -143,7 +143,7 @@ __device__ __forceinline__ bool group_tile(const int* offsets, int G, int t, int
 // LDS is visible to the workgroup; requests to global memory stay in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// grid: (column tiles, row tiles * splits); VEC: every row of X and W starts on 16 bytes and K is a multiple of eight
+// grid: (column tiles, row tiles * splits); VEC: every row of X and W starts on 16 bytes and K is a multiple of EP (no piece crosses the end of a row)
 template <class P, int TM, int TN, int SUB, int WM, int WN, bool VEC>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileArgs a) {
     using WT = typename P::WT;

@@ -1,5 +1,6 @@
-"""ntk_gemm_half (prompt projections over half-precision weights) at the edges of its tiles, chunks and pieces, against float64 sums.  Bound: an activation is off by 2^-24 of its
-value at most, every product and addition rounds to 32 bits once: |error| <= (K + 18) * 2^-24 * sum |x w|."""
+"""ntk_gemm_half (prompt projections over half-precision weights) at the edges of its tiles, chunks and pieces, against float64 sums.  Bound: an activation is off by 2^-23 of its
+value at most (what its row's largest adds, 2^-39, is below that here), the K additions round to 32 bits once each, those of runs and pieces once more:
+|error| <= (K + 18) * 2^-24 * sum |x w|."""
 import ctypes as C
 
 import numpy as np
