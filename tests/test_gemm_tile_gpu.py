@@ -27,7 +27,8 @@ def values(dtype, T, N, K, seed):
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("T,N,K", [(9, 1, 8), (9, 64, 64), (31, 63, 72), (32, 65, 128), (33, 130, 520), (64, 64, 2048), (65, 516, 2056), (128, 128, 32), (129, 257, 96), (200, 640, 1000),
-                                   (300, 2048, 64), (1025, 1028, 40), (12, 3, 4104), (40, 2048, 1536), (17, 100, 37), (70, 33, 515)])
+                                   (300, 2048, 64), (1025, 1028, 40), (12, 3, 4104), (40, 2048, 1536), (17, 100, 37), (70, 33, 515),
+                                   (9, 64, 4), (33, 65, 36), (129, 130, 1004), (40, 516, 2044)])     # (rows of four but not of eight: pieces of four weights, float32 only)
 def test_edges_of_tiles_chunks_and_pieces(dtype, T, N, K):
     x, w, xr = values(dtype, T, N, K, T * 7 + N)
     for room in (0, 2 * T * N, 16 * T * N):
