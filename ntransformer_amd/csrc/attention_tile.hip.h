@@ -63,16 +63,16 @@ __device__ __forceinline__ float attention_score(const TileAttnArgs& a, float s,
 
 // DK, DV: entries of a key and of a value, rounded up (the rest is zero in the operands); VEC: every key / value row is 16-byte aligned and cut in fours
 // BIASED: anything but the scale on the scores (bias by distance, slopes, soft cap)
-constexpr int KW = 2, KT = 16 * KW;                       // waves along the keys, keys of a tile
+constexpr int KT = 32;                                    // keys of a tile: sixteen for each of the two waves along them
 template <int DK, int DV, bool VEC, bool BIASED>
-__global__ __launch_bounds__(128 * KW, 2) void attention_tile_kernel(const TileAttnArgs a) {
+__global__ __launch_bounds__(256, 2) void attention_tile_kernel(const TileAttnArgs a) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int KS = DK + 4, VS = DV + 4, PS = 20, KSTEP = DK / 16, VT = DV / 16;
     constexpr int KU = DK / 32, VU = DV / 32;                 // loader: eight threads on a key's row, 16 bytes each, so many passes
     constexpr int STATE = (8 + 4 * VT) * 64;                  // what a wave leaves for the merge
-    constexpr int TILES = KT * (KS + VS) > (KW - 1) * 2 * STATE ? KT * (KS + VS) : (KW - 1) * 2 * STATE;
+    constexpr int TILES = KT * (KS + VS) > 2 * STATE ? KT * (KS + VS) : 2 * STATE;
     __shared__ __attribute__((aligned(16))) float tiles[TILES];
-    __shared__ __attribute__((aligned(16))) float Ps[2 * KW][16 * PS];
+    __shared__ __attribute__((aligned(16))) float Ps[4][16 * PS];
     float* Ks = tiles;
     float* Vs = tiles + KT * KS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rh = wave & 1, kh = wave >> 1, i16 = lane & 15, g4 = lane >> 4;
@@ -223,12 +223,12 @@ __global__ __launch_bounds__(128 * KW, 2) void attention_tile_kernel(const TileA
             for (int t = 0; t < VT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p4[c], vf[c * VS + 16 * t], acc[t], 0, 0, 0);
         __builtin_amdgcn_wave_barrier();
     }
-    // ---- the waves of a row half meet: all but the first leave (max, sum, vectors), the first adds them to its own in order and stores
+    // ---- the two waves of a row half meet: the second leaves (max, sum, vectors), the first adds them to its own and stores
 #pragma unroll
     for (int r = 0; r < 4; ++r) l[r] = group_sum<16>(l[r]);
     __syncthreads();
+    float* st = tiles + rh * STATE + lane;
     if (kh > 0) {
-        float* st = tiles + ((kh - 1) * 2 + rh) * STATE + lane;
 #pragma unroll
         for (int r = 0; r < 4; ++r) { st[r * 64] = mx[r]; st[(4 + r) * 64] = l[r]; }
 #pragma unroll
@@ -238,21 +238,16 @@ __global__ __launch_bounds__(128 * KW, 2) void attention_tile_kernel(const TileA
     }
     __syncthreads();
     if (kh > 0) return;
-    float w[KW][4];                                           // a part's weight: exp(its maximum - the row's), over the row's sum
+    float w0[4], w1[4];                                       // a part's weight: exp(its maximum - the row's), over the row's sum
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        float m[KW], sum = 0.0f, mm = mx[r];
-        m[0] = mx[r];
-#pragma unroll
-        for (int k = 1; k < KW; ++k) { m[k] = tiles[((k - 1) * 2 + rh) * STATE + r * 64 + lane]; mm = fmaxf(mm, m[k]); }
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-            w[k][r] = m[k] == -INFINITY ? 0.0f : expf(m[k] - mm);
-            sum += w[k][r] * (k ? tiles[((k - 1) * 2 + rh) * STATE + (4 + r) * 64 + lane] : l[r]);
-        }
+        const float m1 = st[r * 64], mm = fmaxf(mx[r], m1);
+        w0[r] = mx[r] == -INFINITY ? 0.0f : expf(mx[r] - mm);
+        w1[r] = m1 == -INFINITY ? 0.0f : expf(m1 - mm);
+        const float sum = fmaf(w1[r], st[(4 + r) * 64], w0[r] * l[r]);
         const float inv = sum > 0.0f ? a.out_scale / sum : 0.0f;
-#pragma unroll
-        for (int k = 0; k < KW; ++k) w[k][r] *= inv;
+        w0[r] *= inv;
+        w1[r] *= inv;
     }
     uint32_t wild = 0;                                        // results that are not finite: bit 4 t + r
 #pragma unroll
@@ -264,9 +259,7 @@ __global__ __launch_bounds__(128 * KW, 2) void attention_tile_kernel(const TileA
 #pragma unroll
         for (int t = 0; t < VT; ++t) {
             if (16 * t + i16 >= a.nV) continue;
-            float y = acc[t][r] * w[0][r];
-#pragma unroll
-            for (int k = 1; k < KW; ++k) y = fmaf(tiles[((k - 1) * 2 + rh) * STATE + (8 + 4 * t + r) * 64 + lane], w[k][r], y);
+            float y = fmaf(st[(8 + 4 * t + r) * 64], w1[r], acc[t][r] * w0[r]);
             if (!(fabsf(y) < INFINITY)) wild |= 1u << (4 * t + r);
             if (gt) y = y / (1.0f + expf(-gt[a.head_gate ? 0 : 16 * t]));
             o[16 * t] = y;
@@ -323,8 +316,8 @@ static void launch_attention_tile(const TileAttnArgs& a, hipStream_t s) {
     const bool biased = a.rel || a.slopes || a.softcap > 0.0f;
 #define NTK_ATTENTION_TILE(DK, DV, VEC)                                                                                          \
     do {                                                                                                                          \
-        if (biased) hipLaunchKernelGGL((attention_tile_kernel<DK, DV, VEC, true>), grid, dim3(128 * KW), 0, s, a);                     \
-        else hipLaunchKernelGGL((attention_tile_kernel<DK, DV, VEC, false>), grid, dim3(128 * KW), 0, s, a);                           \
+        if (biased) hipLaunchKernelGGL((attention_tile_kernel<DK, DV, VEC, true>), grid, dim3(256), 0, s, a);                     \
+        else hipLaunchKernelGGL((attention_tile_kernel<DK, DV, VEC, false>), grid, dim3(256), 0, s, a);                           \
     } while (0)
     if (!vec) {
         if (dk <= 64 && a.nV <= 64) NTK_ATTENTION_TILE(64, 64, false);
