@@ -539,7 +539,7 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
     t.Y = d->Y; t.ldy = d->ldy; t.X = d->X; t.ldx = d->ldx; t.W = d->W; t.wstride = d->wstride; t.offsets = d->offsets; t.G = G; t.rows = d->rows; t.row_div = a.row_div;
     t.T = d->T; t.N = d->N; t.K = d->K; t.accumulate = d->accumulate; t.act = d->act; t.part = d->scratch;
     const int align = bf ? 8 : 4;
-    const bool vec = (d->K % align == 0) && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->W & 15) && (d->wstride % align == 0);
+    const bool vec = (d->K % align == 0) && d->K < 1 << 24 && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->W & 15) && (d->wstride % align == 0);
     if (bf && d->full_x) {                 // (a few tokens' rows: one small tile)
         if (vec) launch_tiles<TileBf16x3, 32, 64, 2, 2, 2, true>(t, 1, s);
         else launch_tiles<TileBf16x3, 32, 64, 2, 2, 2, false>(t, 1, s);

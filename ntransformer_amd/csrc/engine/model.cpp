@@ -697,10 +697,11 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
     auto rp_only = [&](const DevTensor& w) {
         return !w.ptr && w.rp && (w.dtype == NTK_DT_Q4_K || w.dtype == NTK_DT_Q5_K || w.dtype == NTK_DT_Q6_K) && w.out_f % 16 == 0;
     };
-    // half-precision weights: one pass over them for all tokens, too (false: not such a matrix, nothing was launched).  From 4096 inputs on: there the tiles' sums are as close
-    // to 64 bits as the one-token products' (1.6e-7 of the result both, 2.3e-7 against 2.8e-7 at 14336); at 1024 the latter are closer (0.95e-7 against 1.3e-7)
+    // half-precision weights: one pass over them for all tokens, too (false: not such a matrix, nothing was launched).  From 3072 inputs on: there the tiles' results are no further
+    // from 64 bits than the one-token products' (gemm_tile.hip.h: 1.30e-7 against 1.42e-7 of the result at 3072, with channels that tower over the others 1.43 and 1.42; 2.14 and
+    // 2.78 at 14336), at 2560 they are with such channels (1.37 and 1.32), at 1024 in every case (1.07 and 0.99).  Time would draw the line lower: 40 tokens through 2048 x 2048 take 10 us, 130 one by one
     auto project_half = [&](float* Y, const DevTensor& w, const float* X, size_t ystride, size_t xstride, bool accumulate, const float* rm) -> bool {
-        if (!bf16_now || !w.ptr || w.dtype != NTK_DT_F16 || w.in_f < 4096 || ystride != (size_t)w.out_f || xstride != (size_t)w.in_f) return false;
+        if (!bf16_now || !w.ptr || w.dtype != NTK_DT_F16 || w.in_f < 3072 || ystride != (size_t)w.out_f || xstride != (size_t)w.in_f) return false;
         void* ws = cur_ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_;   // (not the one that holds the planes of a quantised matrix's input)
         if (!ws) { ws = cur_ws; planes_of = nullptr; }
         ok(ntk_gemm_half(Y, w.ptr, X, T, (int)w.out_f, (int)w.in_f, accumulate ? 1 : 0, rm, ws, gemm_ws_bytes_, s));

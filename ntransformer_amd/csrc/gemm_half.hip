@@ -3,8 +3,8 @@
 // layer of an 8B-shaped F16 model against 0.47 ms as tiles (gemm_tile.hip.h); a 200-token pass of eight such layers 144.5 -> 4.1 ms.  Taken from two tokens on: 16 tokens
 // through a 4096 x 4096 matrix take 15 us, one token's GEMV 12.  Products on v_mfma_f32_16x16x32_f16; a 32-bit activation goes in as two halves after
 // a per-token power of two (largest |x| in [2^14, 2^15)), which is off by at most 2^-23 of the value (a quarter of them by more than 2^-24, where the one-token
-// products take all 24 bits), or by 2^-39 of the row's largest where the second half is subnormal.  Sums in short runs make up for it (error of a 4096-input product against 64 bits: 1.6e-7
-// of the result both ways).
+// products take all 24 bits), or by 2^-39 of the row's largest where the second half is subnormal.  The sums make up for it (gemm_tile.hip.h): from
+// 3072 inputs on a result is as close to 64 bits as the one-token products' (below, those are closer: 2048 inputs 1.22e-7 of the result against 1.10 .. 1.31e-7, 1024 0.98e-7 against 1.04 .. 1.19e-7).
 #include "gemm_tile.hip.h"
 
 namespace ntk {
@@ -42,7 +42,7 @@ int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out
         t.part = (float*)((char*)workspace + need);
         room = (long long)((workspace_bytes - need) / sizeof(float));
     }
-    const bool vec = in_features % 8 == 0 && !(((uintptr_t)X | (uintptr_t)W) & 15);
+    const bool vec = in_features % 8 == 0 && in_features < 1 << 24 && !(((uintptr_t)X | (uintptr_t)W) & 15);
     if (need) {
         hipLaunchKernelGGL(token_max_kernel, dim3(n_tokens), dim3(256), 0, s, (float*)workspace, X, in_features);
         t.row_max = (const float*)workspace;

@@ -9,6 +9,7 @@
 // 173 -> 122, 1024 x 2048 x 2048 55 -> 26, 40 x 2048 x 7488 102 -> 14; F32 150 x 2048 x 7488 396 -> 60 (77 TF/s), 150 x 14976 x 2048 337 -> 113.
 // The barrier waits for LDS only: a __syncthreads() would also drain the requests that are meant to stay in flight.
 #pragma once
+#include <type_traits>
 #include "common.hip.h"
 
 namespace ntk {
@@ -46,8 +47,11 @@ struct TileArgs {
 };
 
 // ---- the four precisions: WT the stored weight, KE weights per 64 bytes, PIECES how many values stand for one activation.  RUN: the accumulators are added
-// onto a second set and start again from zero every RUN inputs -- as one chain of 32-bit additions a product of 4096 (14336) halves is off by 6e-7 (1.1e-6) of the result, in
-// runs of 128 by 1.6e-7 (2.3e-7), like the sums over 64 lanes of the one-token products (1.6e-7, 2.8e-7); 0: one chain (inputs rounded to eight bits dwarf it)
+// onto a second set and start again from zero every RUN inputs (0: one chain, inputs rounded to eight bits dwarf it).  Products with an activation's pieces behind the first go to
+// a set of their own, which stays small beside the first's, so that they cost it no roundings.  Error of a product of 3072 / 4096 / 14336 halves against 64 bits, in 1e-7 of the result, for normal
+// activations | with channels of 300 times the others: one set, runs of 128 1.52 1.61 2.28 | 1.63 1.75 2.51; so 1.30 1.40 2.14 | 1.43 1.55 2.35; one-token products (sums over 64 lanes)
+// 1.42 1.59 2.78 | 1.42 1.59 2.76.  Three bfloat16 pieces of 512 / 2048 / 4096: one set, runs of 256 1.78 1.84 1.91 | 1.86 1.88 1.99; so 0.76 1.00 1.24 | 0.95 1.17 1.40;
+// one-token products 0.86 1.22 1.59 | 0.85 1.22 1.59.
 struct TileBf16 {                                   // activations rounded to bfloat16
     using WT = uint16_t;
     static constexpr int KE = 32, EP = 8, PIECES = 1, RUN = 0;
@@ -59,7 +63,7 @@ struct TileBf16 {                                   // activations rounded to bf
 };
 struct TileBf16x3 {                                 // bfloat16 weights, a 32-bit activation as the three bfloat16 values that add up to it
     using WT = uint16_t;
-    static constexpr int KE = 32, EP = 8, PIECES = 3, RUN = 256;
+    static constexpr int KE = 32, EP = 8, PIECES = 3, RUN = 128;
     static constexpr bool SCALED = false;
     __device__ static void convert(const float (&v)[EP], float, uintx4_t (&out)[PIECES]) {
         uint32_t u[EP];
@@ -143,9 +147,11 @@ __device__ __forceinline__ bool group_tile(const int* offsets, int G, int t, int
 // LDS is visible to the workgroup; requests to global memory stay in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// grid: (column tiles, row tiles * splits); VEC: every row of X and W starts on 16 bytes and K is a multiple of EP (no piece crosses the end of a row)
+// grid: (column tiles, row tiles * splits); VEC: every row of X and W starts on 16 bytes and K is a multiple of EP (no piece crosses the end of a row), and the rows of a tile lie within 2^32 entries
+// (the forms with pieces: 128 registers, so that two workgroups of eight waves share a CU -- weights at 32-bit offsets from the tile's first row and the odd last chunk behind the loop
+// keep them there without spills; 134 and one workgroup: 200 x 14336 x 4096 halves 103 -> 120 us)
 template <class P, int TM, int TN, int SUB, int WM, int WN, bool VEC>
-__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileArgs a) {
+__global__ __launch_bounds__(64 * WM * WN, P::PIECES > 1 ? 4 : 2) void gemm_tile_kernel(const TileArgs a) {
     using WT = typename P::WT;
     constexpr int BK = P::KE * SUB, EP = P::EP, PIECES = P::PIECES;
     constexpr int THREADS = 64 * WM * WN, PER_ROW = 4 * SUB, RP = THREADS / PER_ROW, PX = TM / RP, PW = TN / RP;      // loader: PER_ROW threads on a row's chunk, RP rows per pass
@@ -164,7 +170,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
     const int lr = tid / PER_ROW, lp = tid % PER_ROW;
     // rows past the end re-read the last one; what they give is not stored
     const float* xrow[PX];
-    const WT* wrow[PW];
+    const WT* wtile = W + (long long)n_base * a.K;
+    typename std::conditional<VEC, uint32_t, size_t>::type wrow[PW];
     float scale[PX];
 #pragma unroll
     for (int p = 0; p < PX; ++p) {
@@ -173,7 +180,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
         scale[p] = P::SCALED ? half_scale(a.row_max[src]) : 1.0f;
     }
 #pragma unroll
-    for (int p = 0; p < PW; ++p) wrow[p] = W + (long long)min(n_base + lr + RP * p, a.N - 1) * a.K;
+    for (int p = 0; p < PW; ++p) wrow[p] = (decltype(wrow[p] + 0))min(lr + RP * p, a.N - 1 - n_base) * a.K;
     struct Chunk { float x[PX][EP]; uintx4_t w[PW]; };
     auto fetch = [&](Chunk& c, int i) {
         const int k = k_begin + i * BK + lp * EP;
@@ -187,7 +194,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
                     c.x[p][4 * q] = v.x; c.x[p][4 * q + 1] = v.y; c.x[p][4 * q + 2] = v.z; c.x[p][4 * q + 3] = v.w;
                 }
 #pragma unroll
-            for (int p = 0; p < PW; ++p) c.w[p] = *reinterpret_cast<const uintx4_t*>(wrow[p] + kc);
+            for (int p = 0; p < PW; ++p) c.w[p] = *reinterpret_cast<const uintx4_t*>(wtile + (wrow[p] + (uint32_t)kc));
         } else {
 #pragma unroll
             for (int p = 0; p < PX; ++p)
@@ -198,11 +205,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
                 if constexpr (sizeof(WT) == 2) {
                     uint32_t v[8];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) v[j] = k + j < k_end ? (uint32_t)wrow[p][k + j] : 0u;
+                    for (int j = 0; j < 8; ++j) v[j] = k + j < k_end ? (uint32_t)wtile[wrow[p] + k + j] : 0u;
                     c.w[p] = uintx4_t{v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16)};
                 } else {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) c.w[p][j] = k + j < k_end ? __float_as_uint((float)wrow[p][k + j]) : 0u;
+                    for (int j = 0; j < 4; ++j) c.w[p][j] = k + j < k_end ? __float_as_uint((float)wtile[wrow[p] + k + j]) : 0u;
                 }
             }
         }
@@ -225,6 +232,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr bool SEP = PIECES > 1;
+    floatx4_t low[SEP ? MI : 1][SEP ? NJ : 1];
+    if constexpr (SEP)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) low[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     constexpr int RUN_CHUNKS = P::RUN / BK;
     static_assert(RUN_CHUNKS % 2 == 0, "a run ends with a pair of chunks");
     floatx4_t total[RUN_CHUNKS ? MI : 1][RUN_CHUNKS ? NJ : 1];
@@ -255,7 +269,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
 #pragma unroll
                 for (int i = 0; i < MI; ++i)
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) acc[i][j] = P::mma(xf[i], wf[j], acc[i][j]);
+                    for (int j = 0; j < NJ; ++j) {
+                        if (SEP && q > 0) low[SEP ? i : 0][SEP ? j : 0] = P::mma(xf[i], wf[j], low[SEP ? i : 0][SEP ? j : 0]);
+                        else acc[i][j] = P::mma(xf[i], wf[j], acc[i][j]);
+                    }
             }
         }
     };
@@ -264,18 +281,23 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tile_kernel(const TileAr
     if (n_chunks > 1) fetch(c1, 1);
     store(c0, 0, 0);
     lds_barrier();
-    for (int i = 0; i < n_chunks; i += 2) {
+    for (int i = 0; i + 1 < n_chunks; i += 2) {
         if (i + 2 < n_chunks) fetch(c0, i + 2);
         multiply(0);
-        if (i + 1 < n_chunks) store(c1, i + 1, 1);
+        store(c1, i + 1, 1);
         lds_barrier();
-        if (i + 1 >= n_chunks) break;
         if (i + 3 < n_chunks) fetch(c1, i + 3);
         multiply(1);
         if (i + 2 < n_chunks) store(c0, i + 2, 0);
         lds_barrier();
         if constexpr (RUN_CHUNKS > 0) { if ((i + 2) % RUN_CHUNKS == 0) end_run(); }
     }
+    if (n_chunks & 1) multiply(0);
+    if constexpr (SEP)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] += low[i][j];
     if constexpr (RUN_CHUNKS > 0) {
         end_run();
 #pragma unroll

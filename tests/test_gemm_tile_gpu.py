@@ -72,6 +72,15 @@ def test_activations_in_three_pieces(T, N, K):
     assert within_bound(y[keep], x[keep], w) and np.isnan(y[6]).all() and not np.isfinite(y[3]).any()
 
 
+@pytest.mark.parametrize("K", [1408, 2048, 4096])
+def test_three_pieces_no_further_from_float64_than_a_few_rows(K):
+    """root mean square over 24576 results; the products of up to eight rows multiply in 32 bits on the vector units"""
+    x, w, _ = values("bfloat16", 48, 512, K, K)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    few = np.concatenate([Lr.dense(x[i:i + 8], w, "bfloat16") for i in range(0, 48, 8)])
+    assert np.linalg.norm(Lr.dense(x, w, "bfloat16", full_x=True) - want) <= np.linalg.norm(few - want)
+
+
 @pytest.mark.parametrize("T,N,K", [(833, 3841, 33), (1025, 3329, 40), (1600, 2049, 67)])
 def test_odd_sizes_in_many_tiles(T, N, K):
     """element by element into the larger tiles (K = 40: rows that do not start on 16 bytes), alone and over rows in groups"""

@@ -8,7 +8,7 @@ from ntransformer_amd import gguf as G
 
 pytestmark = pytest.mark.gpu
 
-WIDE = G.LlamaShape("wide", 4096, 4096, 2, 32, 8, 512, ctx=256, bos=256, eos=257)     # (half-precision matrices go out as tiles from 4096 inputs on)
+WIDE = G.LlamaShape("wide", 4096, 4096, 2, 32, 8, 512, ctx=256, bos=256, eos=257)     # (half-precision matrices go out as tiles from 3072 inputs on)
 NAMES = ("attn_q", "attn_k", "attn_v", "attn_output", "ffn_gate", "ffn_up", "ffn_down")
 
 
