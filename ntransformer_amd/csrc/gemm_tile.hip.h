@@ -380,7 +380,8 @@ __global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const TileArgs a) {
 
 // ---- which tile, and how many pieces of K: the smallest of `chunks x max(alone, workgroups per CU x busy)` + what summing the pieces costs.
 // `alone` is what a chunk takes in a workgroup that has a CU for itself (latency), `busy` what a further workgroup on the CU adds (matrix pipe, LDS), both in us and
-// measured on the shapes of model layers: 12 .. 1024 rows, 2048 .. 28672 outputs, 512 .. 14336 inputs.  The model is within a tenth of the best tile and split there.
+// measured on the shapes of model layers: 12 .. 1024 rows, 2048 .. 28672 outputs, 512 .. 14336 inputs.  Over 70 such shapes it is
+// 2 % behind the best tile and split on average, by more than a tenth in four, by a fifth at most (40 x 28672 x 4096 bf16: 49 us, 41 with 64 x 128 in two pieces).
 struct TileForm { int TM, TN, chunk; float alone, busy; };
 struct TilePlan { int form, splits; };
 static TilePlan plan_tiles(const TileForm* f, int n_forms, int rows, int groups, int N, int K, long long scratch_floats) {
