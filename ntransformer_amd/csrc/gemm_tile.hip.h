@@ -148,10 +148,10 @@ __device__ __forceinline__ bool group_tile(const int* offsets, int G, int t, int
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // grid: (column tiles, row tiles * splits); VEC: every row of X and W starts on 16 bytes and K is a multiple of EP (no piece crosses the end of a row), and the rows of a tile lie within 2^32 entries
-// (the forms with pieces: 128 registers, so that two workgroups of eight waves share a CU -- weights at 32-bit offsets from the tile's first row and the odd last chunk behind the loop
-// keep them there without spills; 134 and one workgroup: 200 x 14336 x 4096 halves 103 -> 120 us)
+// (eight waves and pieces: 128 registers, so that two workgroups share a CU -- weights at 32-bit offsets from the tile's first row and the odd last chunk behind the loop keep them
+// there; with twelve of them spilled 200 x 14336 x 4096 halves took 120 us, so 102)
 template <class P, int TM, int TN, int SUB, int WM, int WN, bool VEC>
-__global__ __launch_bounds__(64 * WM * WN, P::PIECES > 1 ? 4 : 2) void gemm_tile_kernel(const TileArgs a) {
+__global__ __launch_bounds__(64 * WM * WN, WM * WN == 8 && P::PIECES > 1 ? 4 : 2) void gemm_tile_kernel(const TileArgs a) {
     using WT = typename P::WT;
     constexpr int BK = P::KE * SUB, EP = P::EP, PIECES = P::PIECES;
     constexpr int THREADS = 64 * WM * WN, PER_ROW = 4 * SUB, RP = THREADS / PER_ROW, PX = TM / RP, PW = TN / RP;      // loader: PER_ROW threads on a row's chunk, RP rows per pass

@@ -74,12 +74,13 @@ def test_a_prompt_does_not_depend_on_the_prompts_before_it(formats, boost, tmp_p
     eng.close()
 
 
+@pytest.mark.parametrize("width,inter", [(4096, 4096), (3072, 4096), (2048, 3072)])       # (the last: one-token products everywhere but in ffn_down)
 @pytest.mark.parametrize("T", [2, 3, 9, 70])
-def test_half_precision_prompts(T, tmp_path, monkeypatch):
+def test_half_precision_prompts(T, width, inter, tmp_path, monkeypatch):
     """every matrix in F16: the tiles with the maxima that norms and activations leave, on their own and summed onto the stream, against the one-token products; a short pass
     behind a longer one"""
     path = str(tmp_path / "m.gguf")
-    make(path, WIDE, ("F16",) * 7, monkeypatch)
+    make(path, G.LlamaShape("wide", width, inter, 2, width // 128, 8, 512, ctx=256, bos=256, eos=257), ("F16",) * 7, monkeypatch)
     got = []
     for batched in (1, 0):
         eng = loaded(path, batched_prefill=batched)
