@@ -64,6 +64,19 @@ typedef struct ntk_dense_desc {
 #define NTK_ACT_RELU2 1
 int ntk_dense_few_rows(void);   /* up to this many rows a product takes the row-streaming form */
 int ntk_dense(const ntk_dense_desc* d, void* stream);
+/* The same product for more than ntk_dense_few_rows() rows and bfloat16 weights whose activations lie in memory as bfloat16 already (the launch that wrote them rounded them:
+ * the same values as ntk_dense's rounding at the product's input):
+ *   x16 : [x16_rows][ldx16] (16-byte aligned, ldx16 % 8 == 0), in the place of d->X (which may be NULL);
+ *   y16 : NULL: F32 results to d->Y.  Else bfloat16 results, rows ldy16 apart (d->Y unused, no accumulate): d->glu_ff > 0: the gated unit of d (N == 2 * glu_ff), else d->act.
+ * NTK_E_SHAPE where ntk_dense_direct_takes() says 0. */
+typedef struct ntk_direct_desc {
+    const void* x16; int ldx16, x16_rows;
+    void* y16; int ldy16;
+} ntk_direct_desc;
+int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K);
+int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream);
+/* y[t][0..n) = x[t][0..n) rounded to bfloat16 (nearest even), rows ldx floats / ldy values apart */
+int ntk_round_rows(void* y, int ldy, const float* x, int ldx, int T, int n, void* stream);
 /* the plain case: Y[T][N] = X[T][K] . W[N][K]^T */
 int ntk_dense_linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate, void* stream);
 
@@ -74,6 +87,9 @@ int ntk_embed_dense(float* out, const void* table, int tdtype, const int* tokens
  * offset 1: the weight is stored around zero; offset 0: plain.  x rows ldx floats apart, y rows ldy. */
 int ntk_rmsnorm_offset(float* y1, const float* w1, float* y2, const float* w2, int ldy, const float* x, int ldx, int T, int n, float eps, float offset,
                        void* stream);
+/* ... with the results rounded to bfloat16 in the place of (y1 / y2 NULL) or beside the F32 ones: y1_16, y2_16 [T][n], any of the four may be NULL */
+int ntk_rmsnorm_offset_16(float* y1, void* y1_16, const float* w1, float* y2, void* y2_16, const float* w2, int ldy, const float* x, int ldx, int T, int n, float eps,
+                          float offset, void* stream);
 /* out[t] = [a[t] ; b[t]] (two rows of n floats side by side) */
 int ntk_concat_rows(float* out, const float* a, const float* b, int T, int n, void* stream);
 /* y[i] *= 1 / (1 + exp(-g[i])) over T rows of n (y rows ldy apart, g rows ldg) */
@@ -155,6 +171,8 @@ int ntk_gated_seam(const ntk_gated_seam_desc* d, void* stream);
  * Plain weights (nothing is added to them). */
 int ntk_rms_seam(float* h, int ldh, float* x, int ldx, const float* add_y, int ldy, const float* add_w, float mult, const float* w, int T, int n, float eps,
                  void* stream);
+/* ... with the normed rows rounded to bfloat16: h16 [T][n] */
+int ntk_rms_seam_16(void* h16, float* x, int ldx, const float* add_y, int ldy, const float* add_w, float mult, const float* w, int T, int n, float eps, void* stream);
 /* A short causal convolution over time on every channel, then an activation: y[t][c] = act(sum_j w[c][j] * in(t - (taps - 1) + j)[c]), w F32 [n][taps] (tap
  * taps - 1 weighs the present token), in(.) = x rows of this portion, the carried inputs `state` [taps - 1][n] for the rows before it, zeros before the
  * sequence's start (position pos0 + index < 0).  The portion's last taps - 1 inputs are left in `state`.  act 0: none, 1: silu.  y must not overlap x.

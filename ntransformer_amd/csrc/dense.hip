@@ -9,7 +9,7 @@
 // Rows can be grouped (a mixture of experts: sorted rows of group g take matrix g) and gathered (row r reads activation row rows[r] / row_div).
 // Group sizes live on the device, so the grid covers the worst case and workgroups outside their group's range leave at once.
 // A second entry point (ntk_moe_few) runs all of a few tokens' chosen experts, the shared unit and their weighted sum in two row-streaming launches.
-#include "gemm_tile.hip.h"
+#include "gemm_direct.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -498,9 +498,91 @@ static void launch_gemv(const DenseArgs& a, int rows, hipStream_t s) {
     else hipLaunchKernelGGL((dense_gemv_kernel<WT, 1, false, ADD>), grid, dim3(256), lds, s, a);
 }
 
+// x rounded to bfloat16, eight values a thread (V: 16-byte pieces of both; else one by one)
+template <bool V>
+__global__ __launch_bounds__(256) void round_rows_kernel(uint16_t* y, int ldy, const float* x, int ldx, int pieces, int n, long long total) {
+    const long long i = blockIdx.x * 256LL + threadIdx.x;
+    if (i >= total) return;
+    const long long t = i / pieces;
+    const int k = (int)(i - t * pieces) * 8;
+    const float* xr = x + t * ldx + k;
+    uint16_t* yr = y + t * ldy + k;
+    if constexpr (V) {
+        const float4 u = *reinterpret_cast<const float4*>(xr), v = *reinterpret_cast<const float4*>(xr + 4);
+        *reinterpret_cast<uintx4_t*>(yr) = uintx4_t{pack_bf16(u.x, u.y), pack_bf16(u.z, u.w), pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) if (k + j < n) yr[j] = (uint16_t)pack_bf16(xr[j], 0.0f);
+    }
+}
+
+// ---- bf16 products over operands in memory (gemm_direct.hip.h)
+constexpr float kRoundUs = 3.5f, kRoundRate = 4e6f;     // the launch that rounds a product's activations: us, and bytes per us (six an entry)
+static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long room) {
+    static const DirectForm forms[] = {{256, 256, 1, 1.45f, 1.45f, 12.0f}, {256, 128, 1, 0.84f, 0.84f, 9.0f}, {128, 256, 1, 0.85f, 0.85f, 9.0f}, {128, 128, 2, 0.72f, 0.475f, 7.0f},
+                                       {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
+    return plan_direct(forms, 7, 64, rows, groups, N, K, room);
+}
+template <bool GLU>
+static void launch_direct_bf16(const DirectArgs& d, const TilePlan& p, hipStream_t s) {
+    switch (p.form) {
+        case 0: launch_direct<TileBf16, 256, 256, 4, 2, 2, GLU, 2>(d, p.splits, s); break;
+        case 1: launch_direct<TileBf16, 256, 128, 4, 2, 3, GLU, 2>(d, p.splits, s); break;
+        case 2: launch_direct<TileBf16, 128, 256, 2, 4, 3, GLU, 2>(d, p.splits, s); break;
+        case 3: launch_direct<TileBf16, 128, 128, 4, 2, 2, GLU, 4>(d, p.splits, s); break;
+        case 4: launch_direct<TileBf16, 128, 128, 4, 2, 4, GLU, 2>(d, p.splits, s); break;
+        case 5: launch_direct<TileBf16, 64, 128, 2, 2, 3, GLU, 2>(d, p.splits, s); break;
+        default: launch_direct<TileBf16, 64, 64, 2, 2, 3, GLU, 3>(d, p.splits, s); break;
+    }
+}
+
 }  // namespace ntk
 
 using namespace ntk;
+
+int ntk_round_rows(void* y, int ldy, const float* x, int ldx, int T, int n, void* stream) {
+    if (!y || !x) return NTK_E_NULL;
+    if (T < 0 || n <= 0 || ldy < n || ldx < n) return NTK_E_SHAPE;
+    if (T == 0) return NTK_OK;
+    const int pieces = (n + 7) / 8;
+    const long long total = (long long)T * pieces;
+    const bool vec = n % 8 == 0 && ldy % 8 == 0 && ldx % 4 == 0 && !(((uintptr_t)y | (uintptr_t)x) & 15);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    if (vec) hipLaunchKernelGGL(round_rows_kernel<true>, grid, dim3(256), 0, resolve_stream(stream), (uint16_t*)y, ldy, x, ldx, pieces, n, total);
+    else hipLaunchKernelGGL(round_rows_kernel<false>, grid, dim3(256), 0, resolve_stream(stream), (uint16_t*)y, ldy, x, ldx, pieces, n, total);
+    return last_launch_status();
+}
+
+// whole chunks of 64 inputs, and rows that 32-bit offsets reach
+int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K) {
+    return wdtype == NTK_DT_BF16 && T > kGemvRows && N > 0 && K > 0 && K % 64 == 0 && (long long)N * K * 2 < 1LL << 32 && (long long)x16_rows * K * 2 < 1LL << 32;
+}
+
+int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream) {
+    if (!d || !e || !d->W || !e->x16 || (!e->y16 && !d->Y)) return NTK_E_NULL;
+    if (!ntk_dense_direct_takes(d->wdtype, d->T, e->x16_rows, d->N, d->K)) return d->T == 0 ? NTK_OK : NTK_E_SHAPE;
+    const bool glu = d->glu_ff > 0;
+    if (e->ldx16 < d->K || e->ldx16 % 8 || d->wstride % 8 || (long long)e->x16_rows * e->ldx16 * 2 >= 1LL << 32) return NTK_E_SHAPE;
+    if (((uintptr_t)e->x16 | (uintptr_t)d->W) & 15) return NTK_E_ALIGN;
+    if (e->y16 ? (e->ldy16 < (glu ? d->glu_ff : d->N) || d->accumulate) : (glu || d->ldy < d->N)) return NTK_E_SHAPE;
+    if ((glu && (d->N != 2 * d->glu_ff || d->act)) || d->norm_w || d->add_y || d->full_x) return NTK_E_SHAPE;
+    if ((d->offsets && d->G <= 0) || (d->rows && d->row_div <= 0) || (!d->rows && e->x16_rows < d->T)) return NTK_E_SHAPE;
+    if ((d->act != NTK_ACT_NONE && d->act != NTK_ACT_RELU2) || (d->act && d->accumulate)) return NTK_E_SHAPE;
+    const int G = d->offsets ? d->G : 1;
+    DirectArgs a{};
+    TileArgs& t = a.t;
+    t.Y = d->Y; t.ldy = d->ldy; t.W = d->W; t.wstride = d->wstride; t.offsets = d->offsets; t.G = G; t.rows = d->rows; t.row_div = d->rows ? d->row_div : 1;
+    t.T = d->T; t.N = d->N; t.K = d->K; t.accumulate = d->accumulate; t.act = d->act; t.part = d->scratch;
+    a.X16 = e->x16; a.x_row = (uint32_t)e->ldx16 * 2; a.Y16 = (uint16_t*)e->y16; a.ldy16 = e->ldy16;
+    // (no pieces for grouped rows: rows that belong to no group stay untouched)
+    const long long room = d->scratch && !((uintptr_t)d->scratch & 15) && !d->offsets && !e->y16 && d->T <= 65535 ? (long long)(d->scratch_bytes / sizeof(float)) : 0;
+    const TilePlan p = plan_direct_bf16(d->T, G, d->N, d->K, room);
+    if (glu) {
+        a.glu_ff = d->glu_ff; a.limit = d->glu_limit; a.alpha = d->glu_alpha; a.up_offset = d->glu_up_offset; a.cubic = d->glu_cubic;
+        launch_direct_bf16<true>(a, p, resolve_stream(stream));
+    } else launch_direct_bf16<false>(a, p, resolve_stream(stream));
+    return last_launch_status();
+}
 
 int ntk_dense(const ntk_dense_desc* d, void* stream) {
     if (!d || !d->Y || !d->X || !d->W) return NTK_E_NULL;
@@ -558,8 +640,25 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
     // (no pieces for grouped rows: rows that belong to no group stay untouched)
     const long long room = d->scratch && !((uintptr_t)d->scratch & 15) && !d->offsets && d->T <= 65535 ? (long long)(d->scratch_bytes / sizeof(float)) : 0;
     if (bf) {
+        // (a launch that rounds the activations first, where the product over them gains more than that launch takes: rows K 16-bit values apart in the scratch, pieces behind them)
+        const long long image = ((long long)d->T * d->K * 2 + 15) & ~15LL;
+        const bool direct = d->scratch && !((uintptr_t)d->scratch & 15) && !d->rows && (long long)d->scratch_bytes >= image && ntk_dense_direct_takes(d->wdtype, d->T, d->T, d->N, d->K);
         static const TileForm forms[] = {{128, 128, 32, 0.65f, 0.43f}, {64, 128, 64, 0.80f, 0.68f}, {64, 64, 64, 0.70f, 0.35f}, {32, 64, 64, 0.60f, 0.22f}};
         const TilePlan p = plan_tiles(forms, 4, d->T, G, d->N, d->K, room);
+        if (direct) {
+            const long long left = d->offsets || d->T > 65535 ? 0 : ((long long)d->scratch_bytes - image) / (long long)sizeof(float);
+            const TilePlan q = plan_direct_bf16(d->T, G, d->N, d->K, left);
+            if (q.us + kRoundUs + (float)d->T * d->K * 6.0f / kRoundRate < p.us + 4.0f) {       // (p.us is the chunks' time alone)
+                const int st = ntk_round_rows(d->scratch, d->K, d->X, d->ldx, d->T, d->K, stream);
+                if (st != NTK_OK) return st;
+                DirectArgs a16{};
+                a16.t = t;
+                a16.t.part = (float*)((char*)d->scratch + image);
+                a16.X16 = d->scratch; a16.x_row = (uint32_t)d->K * 2;
+                launch_direct_bf16<false>(a16, q, s);
+                return last_launch_status();
+            }
+        }
         if (p.form == 0) launch_tiles<TileBf16, 128, 128, 1, 4, 2, true>(t, p.splits, s);
         else if (p.form == 1) launch_tiles<TileBf16, 64, 128, 2, 2, 4, true>(t, p.splits, s);
         else if (p.form == 2) launch_tiles<TileBf16, 64, 64, 2, 2, 2, true>(t, p.splits, s);

@@ -1004,6 +1004,7 @@ int LayerStackModel::alloc_buffers() {
     // four pieces of a whole pass's rows, and no less than sixteen of a short one's
     pscratch_bytes_ = std::max<size_t>(4 * C * W, (size_t)1 << 22) * sizeof(float);
     ok = ok && fl(&pscratch_, pscratch_bytes_ / sizeof(float));
+    if (wdtype_ == NTK_DT_BF16) ok = ok && (h1_16_ = dev_alloc(C * W * 2)) && (h2_16_ = dev_alloc(C * W * 2));
     if (max_mid_ > 0) ok = ok && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_);
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
     h_stage_ = (int*)nt_hip_malloc_host(2 * C * sizeof(int));
@@ -1049,7 +1050,7 @@ int LayerStackModel::truncate_slot(int slot, int length) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------------ the step
-int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside) {
+int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside, const void* h16) {
     const LatentMixer& m = L.mix;
     const int W = info_.width, H = m.heads, qd = m.qd(), row = m.row(), hv = H * m.vdim, na = (int)m.in.out_f;
     // one product for [query (latent) | latent + key part | gate] of the mixer's input h; norm_inside (few rows): h is the stream, the layer's first norm runs
@@ -1058,7 +1059,7 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
     ntk_dense_desc d{};
     d.Y = a_; d.ldy = na; d.X = h; d.ldx = W; d.W = m.in.ptr; d.wdtype = m.in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = na; d.K = W;
     if (norm_inside) { d.norm_w = L.norm1.w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }
-    LS_TRY(first_product(d));
+    LS_TRY(first_product(d, h16));
     d.add_y = nullptr;
     float* q = a_;
     int ldq = na;
@@ -1083,8 +1084,20 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
     } else {
         const int key0 = m.window > 0 ? std::max(0, pos0 - m.window + 1) : 0;
         const int nkeys = pos0 + T - key0;
-        LS_TRY(linear(kx_, H * m.dim, cache + (size_t)key0 * row, row, m.uk.ptr, m.uk.dtype, nkeys, H * m.dim, m.kv_rank, 0));
-        LS_TRY(linear(vx_, hv, cache + (size_t)key0 * row, row, m.uv.ptr, m.uv.dtype, nkeys, hv, m.kv_rank, 0));
+        const float* lat = cache + (size_t)key0 * row;
+        const size_t image = (size_t)nkeys * m.kv_rank * 2;
+        if (rounded(m.uk, nkeys) && rounded(m.uv, nkeys) && image <= pscratch_bytes_) {       // the latents rounded once for both
+            LS_TRY(ntk_round_rows(pscratch_, m.kv_rank, lat, row, nkeys, m.kv_rank, stream_));
+            const ntk_direct_desc e{pscratch_, m.kv_rank, nkeys, nullptr, 0};
+            ntk_dense_desc u{};
+            u.Y = kx_; u.ldy = H * m.dim; u.W = m.uk.ptr; u.wdtype = m.uk.dtype; u.G = 1; u.T = nkeys; u.N = H * m.dim; u.K = m.kv_rank;
+            LS_TRY(ntk_dense_direct(&u, &e, stream_));
+            u.Y = vx_; u.ldy = hv; u.W = m.uv.ptr; u.wdtype = m.uv.dtype; u.N = hv;
+            LS_TRY(ntk_dense_direct(&u, &e, stream_));
+        } else {
+            LS_TRY(linear(kx_, H * m.dim, lat, row, m.uk.ptr, m.uk.dtype, nkeys, H * m.dim, m.kv_rank, 0));
+            LS_TRY(linear(vx_, hv, lat, row, m.uv.ptr, m.uv.dtype, nkeys, hv, m.kv_rank, 0));
+        }
         LS_TRY(ntk_latent_attention(att_, hv, q, ldq, kx_, H * m.dim, vx_, hv, cache, row, m.kv_rank, m.rot_dim, H, m.dim, m.vdim, 0, pos0, T, key0, m.window, m.scale,
                                     nullptr, stream_));
         if (m.head_gate) LS_TRY(ntk_head_gate(att_, hv, a_ + m.g_off, na, T, H, m.vdim, stream_));
@@ -1094,12 +1107,12 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
 }
 
 // the window mixer: one product for [q | k | v], rotation and cache rows, attention over the window, output projection -> mix_
-int LayerStackModel::run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0) {
+int LayerStackModel::run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, const void* h16) {
     const WindowMixer& m = L.att;
     const int W = info_.width, na = (int)m.in.out_f, hv = m.heads * m.vdim;
     ntk_dense_desc d{};
     d.Y = a_; d.ldy = na; d.X = h; d.ldx = W; d.W = m.in.ptr; d.wdtype = m.in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = na; d.K = W;
-    LS_TRY(first_product(d));
+    LS_TRY(first_product(d, h16));
     LS_TRY(window_heads(m, cache, att_, hv, T, pos0));
     return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
@@ -1169,10 +1182,25 @@ int LayerStackModel::run_lightning(const StackLayer& L, float* state, int T, int
     return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
+// h16: the input rows as bfloat16 too (or alone); then, where both products take such operands, the first leaves the activations as bfloat16 in `act` -- the values that the
+// second would round at its input -- and its two halves never reach memory.
 int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
-                                 int full_x) {
+                                 int full_x, const void* h16) {
     const int W = info_.width;
     ntk_dense_desc d{};
+    if (h16 && !full_x && rounded(ex.gate_up, rows) && rounded(ex.down, rows)) {
+        ntk_direct_desc e{h16, W, rows / top, act, ex.ff};
+        d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype; d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top;
+        d.T = rows; d.N = ex.in_rows(); d.K = W;
+        if (ex.plain) d.act = NTK_ACT_RELU2;
+        else { d.glu_ff = ex.ff; d.glu_limit = ex.limit; d.glu_alpha = glu_alpha; d.glu_up_offset = glu_up_offset; }
+        LS_TRY(ntk_dense_direct(&d, &e, stream_));
+        ntk_dense_desc o{};
+        ntk_direct_desc f{act, ex.ff, rows, nullptr, 0};
+        o.Y = out; o.ldy = W; o.W = ex.down.ptr; o.wstride = ex.down.stride(); o.wdtype = ex.down.dtype; o.offsets = offsets; o.G = ex.gate_up.count; o.T = rows; o.N = W; o.K = ex.ff;
+        o.scratch = pscratch_; o.scratch_bytes = pscratch_bytes_;
+        return ntk_dense_direct(&o, &f, stream_);
+    }
     d.full_x = full_x;
     d.Y = gu; d.ldy = ex.in_rows(); d.X = h; d.ldx = W; d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype;
     d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top; d.T = rows; d.N = ex.in_rows(); d.K = W; d.accumulate = 0;
@@ -1211,7 +1239,7 @@ static bool in_two_launches(const MoeFeedForward& M, int T, int W) {
 
 // router, grouping, the experts' products; then either straight into the stream together with the mixer's output (parallel form) or as a sum of its own
 // in ff_ (sequential form: it is normed before it joins the stream)
-int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool into_stream) {
+int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool into_stream, const void* h16) {
     const MoeFeedForward& M = L.mlp;
     const int W = info_.width, choices = M.experts + M.identity;
     float* sgate = M.has_shared && M.shared_gate ? sg_ : nullptr;
@@ -1249,8 +1277,12 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
         return ntk_moe_few(&d, stream_);
     }
     LS_TRY(ntk_moe_group(offsets_, order_, where_, ids_, T, M.top, choices, stream_));     // (identity experts come last: rows behind offsets_[experts], which no product visits)
-    LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.routed, h, gu_, act_, dn_, T * M.top, offsets_, order_, M.top, few));
-    if (M.has_shared) LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.shared, h, sgu_, sact_, sdn_, T, nullptr, nullptr, 1, 0));
+    if (!h16 && T > ntk_dense_few_rows() && rounded(M.routed.gate_up, T)) {      // (rounded once for the chosen and the shared units)
+        LS_TRY(ntk_round_rows(h2_16_, W, h, W, T, W, stream_));
+        h16 = h2_16_;
+    }
+    LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.routed, h, gu_, act_, dn_, T * M.top, offsets_, order_, M.top, few, h16));
+    if (M.has_shared) LS_TRY(run_experts(M.glu_alpha, M.glu_up_offset, M.shared, h, sgu_, sact_, sdn_, T, nullptr, nullptr, 1, 0, h16));
     if (into_stream) return ntk_moe_combine(x_, mix_, dn_, where_, wts_, M.has_shared ? sdn_ : nullptr, sgate, T, M.top, W, stream_);
     return ntk_moe_sum_ex(ff_, dn_, where_, M.identity ? ids_ : nullptr, M.experts, h, W, wts_, M.has_shared ? sdn_ : nullptr, sgate, T, M.top, W, stream_);
 }
@@ -1265,17 +1297,23 @@ int LayerStackModel::run_dense_ff(const StackLayer& L, int T) {
 }
 
 // the dense gated unit (the experts' unit with one member, clipped or plain): gate and up in one product (decoding: the activation inside its launch), down -> ff_
-int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T) {
-    return run_experts(form_.clipped_glu ? kGluAlpha : 1.0f, form_.clipped_glu ? 1.0f : 0.0f, L.cff, h, gu2_, zf_, ff_, T, nullptr, nullptr, 1, 0);
+int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16) {
+    if (!h16 && rounded(L.cff.gate_up, T)) {
+        LS_TRY(ntk_round_rows(h2_16_, info_.width, h, info_.width, T, info_.width, stream_));
+        h16 = h2_16_;
+    }
+    return run_experts(form_.clipped_glu ? kGluAlpha : 1.0f, form_.clipped_glu ? 1.0f : 0.0f, L.cff, h, gu2_, zf_, ff_, T, nullptr, nullptr, 1, 0, h16);
 }
 
 // the delta rule with per-head gates: one product for [q | k | v | gate | beta | decay], the short convolutions of q, k and v (+ silu) with their carried
 // inputs, the recurrence (unit q and k, decay and write strength formed from their raw projections in its pre-pass), unit norm per head with the shared
 // weight and the silu gate, output projection -> mix_.  state = [S | the convolutions' last inputs]
-int LayerStackModel::run_gated_delta(const StackLayer& L, float* state, int T, int pos0) {
+int LayerStackModel::run_gated_delta(const StackLayer& L, float* state, int T, int pos0, const void* h16) {
     const GatedDeltaMixer& m = L.gdl;
     const int W = info_.width, na = (int)m.in.out_f, nc = m.channels(), hv = m.heads * m.vdim;
-    LS_TRY(linear(a_, na, h1_, W, m.in.ptr, m.in.dtype, T, na, W, 0));
+    ntk_dense_desc in{};
+    in.Y = a_; in.ldy = na; in.X = h1_; in.ldx = W; in.W = m.in.ptr; in.wdtype = m.in.dtype; in.G = 1; in.row_div = 1; in.T = T; in.N = na; in.K = W;
+    LS_TRY(first_product(in, h16));
     ntk_gated_recurrence_desc d{};
     if (T == 1) {   // a decoded token: the convolutions run inside the recurrence's pre-pass
         d.q = a_; d.ldq = na; d.k = a_ + m.k_off; d.ldk = na; d.v = a_ + m.v_off; d.ldv = na;
@@ -1302,18 +1340,37 @@ int LayerStackModel::rms_seam(const NormW& nw, float* out, int T) {
     return st;
 }
 
+// ... for a sublayer whose first matrix is `in`: as bfloat16 alone where that product takes its input so (*h16 = out16, else NULL)
+int LayerStackModel::seam_for(const DenseW& in, const NormW& nw, float* out, void* out16, int T, const void** h16) {
+    const int W = info_.width;
+    *h16 = nullptr;
+    if (rounded(in, T)) {
+        const int st = ntk_rms_seam_16(out16, x_, W, owed_.y, W, owed_.nb.w, residual_mult_, nw.w, T, W, eps_, stream_);
+        if (st == NTK_OK) { owed_.y = nullptr; *h16 = out16; return NTK_OK; }
+        if (st != NTK_E_ALIGN) return st;
+    }
+    return rms_seam(nw, out, T);
+}
+
 int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0) {
-    LS_TRY(rms_seam(L.norm1, h1_, T));
-    if (L.mixer == kMixWindow) LS_TRY(run_window(L, h1_, run.cache + (size_t)slot * opt_.max_context * L.att.row(), T, pos0));
-    else if (L.mixer == kMixLatent) LS_TRY(run_mixer(L, run.cache + (size_t)slot * opt_.max_context * L.mix.row(), T, pos0, h1_));
-    else LS_TRY(run_gated_delta(L, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0));
+    const DenseW& in = L.mixer == kMixWindow ? L.att.in : L.mixer == kMixLatent ? L.mix.in : L.gdl.in;
+    const void* h16 = nullptr;
+    LS_TRY(seam_for(in, L.norm1, h1_, h1_16_, T, &h16));
+    if (L.mixer == kMixWindow) LS_TRY(run_window(L, h1_, run.cache + (size_t)slot * opt_.max_context * L.att.row(), T, pos0, h16));
+    else if (L.mixer == kMixLatent) LS_TRY(run_mixer(L, run.cache + (size_t)slot * opt_.max_context * L.mix.row(), T, pos0, h1_, false, h16));
+    else LS_TRY(run_gated_delta(L, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0, h16));
     owed_ = Owed{mix_, L.norm1b};
     if (!L.has_mlp) return NTK_OK;
-    LS_TRY(rms_seam(L.norm2, h2_, T));
-    LS_TRY(run_unit_ff(L, h2_, T));
+    // (the down product takes the activations as the first one leaves them: both or none)
+    if (rounded(L.cff.down, T)) LS_TRY(seam_for(L.cff.gate_up, L.norm2, h2_, h2_16_, T, &h16));
+    else { h16 = nullptr; LS_TRY(rms_seam(L.norm2, h2_, T)); }
+    LS_TRY(run_unit_ff(L, h2_, T, h16));
     owed_ = Owed{ff_, L.norm2b};
     return NTK_OK;
 }
+
+// T rows of bfloat16 activations go through w as they lie
+bool LayerStackModel::rounded(const DenseW& w, int T) const { return h1_16_ && ntk_dense_direct_takes(w.dtype, T, T, (int)w.out_f, (int)w.in_f) != 0; }
 
 // every product of the model: with room for the partial sums of a product whose inputs are cut into pieces
 int LayerStackModel::product(ntk_dense_desc& d) {
@@ -1328,7 +1385,12 @@ int LayerStackModel::linear(float* Y, int ldy, const float* X, int ldx, const vo
 
 // The first product of a sublayer.  In the post-norm form it reads the stream itself: with few rows, what the stream is still owed joins it inside this launch, which
 // leaves the new stream in the other buffer (its workgroups all read the old one).
-int LayerStackModel::first_product(ntk_dense_desc& d) {
+int LayerStackModel::first_product(ntk_dense_desc& d, const void* x16) {
+    if (x16) {
+        const ntk_direct_desc e{x16, d.K, d.T, nullptr, 0};
+        d.scratch = pscratch_; d.scratch_bytes = pscratch_bytes_;
+        return ntk_dense_direct(&d, &e, stream_);
+    }
     if (!form_.post_norm || !owed_.y || d.X != x_) return product(d);
     const int W = info_.width;
     d.add_y = owed_.y; d.ld_add = W; d.add_w = owed_.nb.w; d.add_eps = eps_; d.add_mult = residual_mult_; d.x_out = x0_; d.ldxo = W;
@@ -1489,15 +1551,22 @@ int LayerStackModel::sequential_layer(const Run& run, const StackLayer& L, int s
 
 int LayerStackModel::parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0) {
     const int W = info_.width;
+    const void *h16 = nullptr, *g16 = nullptr;
     if (T > ntk_dense_few_rows()) {
-        LS_TRY(ntk_rmsnorm_offset(h1_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_));
+        int st = NTK_E_ALIGN;
+        if (rounded(L.mix.in, T)) {        // (the router reads its input as F32)
+            st = ntk_rmsnorm_offset_16(nullptr, h1_16_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? h2_16_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
+            if (st == NTK_OK) { h16 = h1_16_; g16 = L.has_mlp ? h2_16_ : nullptr; }
+        }
+        if (st == NTK_E_ALIGN) st = ntk_rmsnorm_offset(h1_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
+        LS_TRY(st);
     } else if (L.has_mlp) {   // decoding: the mixer's norm runs inside its first product (run_mixer); the feed-forward's input has three readers
         LS_TRY(ntk_rmsnorm_offset(h2_, L.norm2.w, nullptr, nullptr, W, x_, W, T, W, eps_, 1.0f, stream_));
     }
     float* cache = run.cache + (size_t)slot * opt_.max_context * L.mix.row();
     const bool few = T <= ntk_dense_few_rows();
-    LS_TRY(run_mixer(L, cache, T, pos0, few ? x_ : h1_, few));
-    if (L.has_mlp) return run_moe(L, h2_, T, true);
+    LS_TRY(run_mixer(L, cache, T, pos0, few ? x_ : h1_, few, h16));
+    if (L.has_mlp) return run_moe(L, h2_, T, true, g16);
     return ntk_residual_add(x_, mix_, nullptr, T * W, stream_);
 }
 

@@ -311,10 +311,11 @@ private:
     int run_parallel(const StackLayer& L, float* cache, float* state, int T, int pos0);
     int run_gated_ff(const StackLayer& L, int T);
     int parse_gated_delta(const Json& L, GatedDeltaMixer& m);
-    int run_gated_delta(const StackLayer& L, float* state, int T, int pos0);
-    int run_unit_ff(const StackLayer& L, const float* h, int T);
+    int run_gated_delta(const StackLayer& L, float* state, int T, int pos0, const void* h16 = nullptr);
+    int run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16 = nullptr);
     int post_norm_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int rms_seam(const NormW& nw, float* out, int T);
+    int seam_for(const DenseW& in, const NormW& nw, float* out, void* out16, int T, const void** h16);
     int scaled_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int gated_layer(size_t r, const StackLayer& L, int slot, int T, int pos0);
     int parse_mlp(const Json& ml, const std::string& where, StackLayer& S);
@@ -327,18 +328,19 @@ private:
     int alloc_buffers();
     void* dev_alloc(size_t bytes);
     int portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, float* logits_out);
-    int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false);
-    int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0);
+    int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false, const void* h16 = nullptr);
+    int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, const void* h16 = nullptr);
     int window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0);
     int dense_parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int run_lightning(const StackLayer& L, float* state, int T, int pos0);
-    int run_moe(const StackLayer& L, const float* h, int T, bool into_stream);
+    int run_moe(const StackLayer& L, const float* h, int T, bool into_stream, const void* h16 = nullptr);
     int run_dense_ff(const StackLayer& L, int T);
     int run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
-                    int full_x);
+                    int full_x, const void* h16 = nullptr);
     int norm_conv(const NormW& nw, const float* canon, float* conv_state, float* out, int T, int pos0);
     int settle(int T);
-    int first_product(ntk_dense_desc& d);
+    int first_product(ntk_dense_desc& d, const void* x16 = nullptr);
+    bool rounded(const DenseW& w, int T) const;
     int product(ntk_dense_desc& d);
     int linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate);
     int sequential_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
@@ -380,6 +382,7 @@ private:
           *att_ = nullptr, *kx_ = nullptr, *vx_ = nullptr, *mix_ = nullptr, *wts_ = nullptr, *sg_ = nullptr, *gu_ = nullptr, *act_ = nullptr, *dn_ = nullptr,
           *sgu_ = nullptr, *sact_ = nullptr, *sdn_ = nullptr, *scratch_ = nullptr, *xw_ = nullptr, *hn_ = nullptr, *hist_ = nullptr, *ff_ = nullptr, *zf_ = nullptr, *wscratch_ = nullptr, *lscratch_ = nullptr,
           *results_ = nullptr, *zq_ = nullptr, *gu2_ = nullptr, *rscratch_ = nullptr, *cv_ = nullptr, *vfirst_ = nullptr, *mid_ = nullptr, *rz_ = nullptr, *pscratch_ = nullptr;   // gated form: the layer results of the pass [runs + 1][chunk][width], decay pre-activations, [gate | up | residual gate]
+    void *h1_16_ = nullptr, *h2_16_ = nullptr;   // a sublayer's input as bfloat16, in the place of (or beside) h1_ / h2_ where its products take it so
     size_t pscratch_bytes_ = 0;                  // pscratch_: partial sums of products (ntk_dense_desc::scratch)
     size_t max_mid_ = 0;              // (post-norm form: the experts' activations of a token side by side)
     int max_rec_ = 0, max_gu2_ = 0, max_conv_ = 0, max_gv_ = 0;   // (scaled form: convolution channels, key heads x value size of the blending attention layers)

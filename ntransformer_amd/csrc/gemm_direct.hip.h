@@ -1,0 +1,270 @@
+// gemm_direct.hip.h -- tiled products Y[r][n] = sum_k X[r][k] W[n][k] whose operands lie in memory as the matrix cores take them.
+//
+// The form of gemm_tile.hip.h converts activations in every workgroup, on their way through registers into LDS: each of a product's up to 117 column tiles reads 32-bit
+// activations and rounds them again, and with the operands' way through registers a workgroup of eight waves is left with wave tiles of 32 x 64, for which LDS has to
+// deliver 192 bytes a cycle and CU at the matrix cores' full rate, where it has 128.  Here the activations were rounded (or cut into pieces) once, by the launch that wrote them or
+// by one in front of the product; both operands go from memory straight into LDS (global_load_lds, 16 bytes a lane), STAGES chunks of 128 bytes a row deep, and a wave of the large forms owns 64 x 64 or
+// 64 x 128 (96 .. 128 bytes).  What bounds the large ones is the matrix cores: a chunk of a 256 x 256 tile takes 1.45 us of the 1.7 they need at the rate of a large library product
+// (1216 TF/s); below a few tiles a CU it is the latency of the first chunks and the results on their way out (`over` in plan_direct).  Consecutive tiles of an XCD share their weights.
+// Measured (us, weights from memory; the form of gemm_tile.hip.h with its best tile and pieces): bf16 1024 x 14976 x 2048 142 -> 62 (1010 TF/s), 1024 x 2048 x 7488 63 -> 43,
+// 1024 x 6240 x 2048 58 -> 37, 1024 x 2048 x 2048 26 -> 16.5, 40 x 14976 x 2048 22 -> 17, 6144 rows in 32 groups of 2816 x 2048 227 -> 133, of 2048 x 1408 116 -> 62.
+// One chain of matrix instructions over the inputs as there: the same bits where K is not cut.
+#pragma once
+#include "gemm_tile.hip.h"
+
+namespace ntk {
+
+struct DirectArgs {
+    TileArgs t;                                     // X unused
+    const void* X16; uint32_t x_row; long long plane;      // activations as the matrix cores take them, rows of x_row bytes; PIECES planes, `plane` bytes apart
+    uint16_t* Y16; int ldy16; int glu_ff;           // bfloat16 results in the place of t.Y (or NULL); GLU: [r][f] = gated unit of rows f and glu_ff + f of W
+    float limit, alpha, up_offset, cubic;
+};
+
+// N requests of 16 bytes a lane: lane l's land at lds + i * step + 16 l.  The compiler does not count them (M0 is the compiler's: saved and restored)
+template <int STEP>
+__device__ __forceinline__ void direct_load4(uint32_t lds, const void* base, uint32_t o0, uint32_t o1, uint32_t o2, uint32_t o3) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %1\n\t"
+                 "s_add_u32 m0, m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %1\n\t"
+                 "s_add_u32 m0, m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %1\n\t"
+                 "s_add_u32 m0, m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %6, %1\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(o0), "v"(o1), "v"(o2), "v"(o3), "i"(STEP) : "memory", "scc");
+}
+__device__ __forceinline__ void direct_load1(uint32_t lds, const void* base, uint32_t o0) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %1\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(o0) : "memory");
+}
+template <int STEP>
+__device__ __forceinline__ void direct_load2(uint32_t lds, const void* base, uint32_t o0, uint32_t o1) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %1\n\t"
+                 "s_add_u32 m0, m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %1\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(o0), "v"(o1), "i"(STEP) : "memory", "scc");
+}
+template <int N, int STEP>
+__device__ __forceinline__ void direct_load(uint32_t lds, const void* base, const uint32_t (&o)[N]) {
+    constexpr int F = N / 4 * 4;
+#pragma unroll
+    for (int i = 0; i < F; i += 4) direct_load4<STEP>(lds + i * STEP, base, o[i], o[i + 1], o[i + 2], o[i + 3]);
+    if constexpr (N % 4 >= 2) direct_load2<STEP>(lds + F * STEP, base, o[F], o[F + 1]);
+    if constexpr (N % 2) direct_load1(lds + (N - 1) * STEP, base, o[N - 1]);
+}
+template <int V> __device__ __forceinline__ void direct_wait() {   // all but the newest V requests have landed, this wave's LDS reads are done, and so everywhere in the workgroup
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "i"(V) : "memory");
+}
+
+// one-dimensional grid over (row tiles, column tiles, splits), row tiles first; rows of X and W are whole multiples of 128 bytes
+template <class P, int TM, int TN, int WM, int WN, int STAGES, bool GLU, int MINW>
+__global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const DirectArgs d, const int row_tiles, const int col_tiles) {
+    const TileArgs& a = d.t;
+    constexpr int CB = 128, ES = sizeof(typename P::WT), BK = CB / ES, PIECES = P::PIECES, NW = WM * WN, WTM = TM / WM, WTN = TN / WN, MI = WTM / 16, NJ = WTN / 16;
+    constexpr int NX = TM / (8 * NW), NWL = TN / (8 * NW), LPS = NX * PIECES + NWL;      // requests of a wave: X per plane, W; per chunk
+    constexpr int XB = TM * CB, STAGE = (PIECES * TM + TN) * CB;
+    static_assert(TM % (8 * NW) == 0 && TN % (8 * NW) == 0, "whole requests");
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[STAGES * STAGE];
+    // consecutive workgroups go to the eight XCDs in turn: each takes a contiguous range of tiles, so that the row tiles of a column share its weights in one L2
+    const int n_wg = gridDim.x, xcd = blockIdx.x & 7, per = n_wg >> 3, rem = n_wg & 7;
+    int id = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+    const int rt = id % row_tiles;
+    id /= row_tiles;
+    const int ct = id % col_tiles, split = id / col_tiles;
+    int g = 0, row_base = rt * TM, r1 = a.T;
+    if (a.offsets) { if (!group_tile(a.offsets, a.G, rt, TM, g, row_base, r1)) return; }
+    const int n_cols = GLU ? d.glu_ff : a.N, n_base = ct * (GLU ? TN / 2 : TN);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM;
+    const int k_begin = split * a.k_per_split, k_end = min(a.K, k_begin + a.k_per_split), n_chunks = (k_end - k_begin) / BK;
+    // a request brings eight rows of 128 bytes; the 16-byte pieces of row r are stored in the order piece ^ (r & 7)
+    uint32_t xo[NX], wo[NWL];
+    const uint32_t row_bytes = (uint32_t)a.K * ES;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+        const int row = (i * NW + wave) * 8 + (lane >> 3), r = min(row_base + row, r1 - 1), src = a.rows ? a.rows[r] / a.row_div : r;
+        xo[i] = (uint32_t)src * d.x_row + (uint32_t)(((lane & 7) ^ (row & 7)) * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < NWL; ++i) {
+        const int row = (i * NW + wave) * 8 + (lane >> 3);
+        int n;
+        if constexpr (GLU) {                        // a wave's columns: as many gates as the up rows of the same outputs behind them
+            const int c = n_base + (row / WTN) * (WTN / 2) + row % (WTN / 2);
+            n = min(c, n_cols - 1) + (row % WTN >= WTN / 2 ? d.glu_ff : 0);
+        } else n = min(n_base + row, n_cols - 1);
+        wo[i] = (uint32_t)(GLU ? n : n - n_base) * row_bytes + (uint32_t)(((lane & 7) ^ (row & 7)) * 16);
+    }
+    const char* xb = (const char*)d.X16 + (long long)k_begin * ES;
+    const char* wb = (const char*)a.W + ((long long)g * a.wstride + (GLU ? 0 : (long long)n_base * a.K) + k_begin) * ES;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    const uint32_t mine = lds0 + wave * 1024;
+    auto request = [&](int chunk, int slot) {
+        const uint32_t at = mine + slot * STAGE;
+        const long long off = (long long)chunk * CB;
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q) direct_load<NX, NW * 1024>(at + q * XB, xb + q * d.plane + off, xo);
+        direct_load<NWL, NW * 1024>(at + PIECES * XB, wb + off, wo);
+    };
+    floatx4_t acc[MI][NJ];
+    constexpr bool SEP = PIECES > 1;
+    floatx4_t low[SEP ? MI : 1][SEP ? NJ : 1];
+    constexpr int RUN_CHUNKS = P::RUN / BK;
+    floatx4_t total[RUN_CHUNKS ? MI : 1][RUN_CHUNKS ? NJ : 1];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (SEP) low[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (RUN_CHUNKS > 0) total[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    auto end_run = [&]() {
+        if constexpr (RUN_CHUNKS > 0)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) { total[i][j] += acc[i][j]; acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f}; }
+    };
+    const bool idle = row_base + wm * WTM >= r1;    // (uniform) rows past the group's end: nothing to multiply, the matrix cores are a neighbour's
+    auto multiply = [&](int slot) {
+        const uint8_t* s = lds + slot * STAGE;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int piece = (((h * 4 + (lane >> 4)) ^ (lane & 7)) * 16) + (lane & 15) * CB;
+            uintx4_t wf[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) wf[j] = *reinterpret_cast<const uintx4_t*>(s + PIECES * XB + (wn * WTN + j * 16) * CB + piece);
+#pragma unroll
+            for (int q = 0; q < PIECES; ++q) {
+                uintx4_t xf[MI];
+#pragma unroll
+                for (int i = 0; i < MI; ++i) xf[i] = *reinterpret_cast<const uintx4_t*>(s + q * XB + (wm * WTM + i * 16) * CB + piece);
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        if (SEP && q > 0) low[SEP ? i : 0][SEP ? j : 0] = P::mma(xf[i], wf[j], low[SEP ? i : 0][SEP ? j : 0]);
+                        else acc[i][j] = P::mma(xf[i], wf[j], acc[i][j]);
+                    }
+            }
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < STAGES - 1; ++c) if (c < n_chunks) request(c, c);
+    int slot = 0;
+    for (int i = 0; i < n_chunks; ++i) {
+        const int left = n_chunks - 1 - i;          // chunks behind this one
+        if (left >= STAGES - 2) direct_wait<LPS * (STAGES - 2)>();
+        else if (STAGES > 3 && left == 1) direct_wait<LPS>();
+        else direct_wait<0>();
+        if (left >= STAGES - 1) request(i + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);
+        if (!idle) multiply(slot);
+        slot = slot + 1 == STAGES ? 0 : slot + 1;
+        if constexpr (RUN_CHUNKS > 0) { if ((i + 1) % RUN_CHUNKS == 0) end_run(); }
+    }
+    if (idle) return;
+    if constexpr (SEP)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] += low[i][j];
+    if constexpr (RUN_CHUNKS > 0) {
+        end_run();
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = total[i][j];
+    }
+    // accumulator lane map: row 4 * (lane / 16) + r, column lane % 16
+    if constexpr (GLU) {
+        const int col = n_base + wn * (WTN / 2) + (lane & 15), n_left = n_cols - col;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
+            uint16_t* y = d.Y16 + (long long)row * d.ldy16 + col;
+#pragma unroll
+            for (int j = 0; j < NJ / 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (row + r < r1 && j * 16 < n_left) {
+                        const float gg = fminf(acc[i][j][r], d.limit), uu = fminf(fmaxf(acc[i][NJ / 2 + j][r], -d.limit), d.limit);
+                        const float zz = d.cubic != 0.0f ? fmaf(d.cubic * gg * gg, gg, gg) : gg;
+                        const float v = gg * (1.0f / (1.0f + expf(-d.alpha * zz))) * (uu + d.up_offset);
+                        y[(long long)r * d.ldy16 + j * 16] = (uint16_t)pack_bf16(v, 0.0f);
+                    }
+        }
+        return;
+    }
+    const int col = n_base + wn * WTN + (lane & 15), n_left = a.N - col;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
+        float undo[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        if constexpr (P::SCALED)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) undo[r] = half_unscale(a.row_max[min(row + r, a.T - 1)]);
+        if (a.splits > 1) {
+            float* y = a.part + ((long long)split * a.T + row) * a.N + col;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (row + r < r1 && j * 16 < n_left) y[(long long)r * a.N + j * 16] = acc[i][j][r] * undo[r];
+            continue;
+        }
+        float* y = a.Y + (long long)row * a.ldy + col;
+        float old[NJ][4] = {};
+        if (a.accumulate)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) old[j][r] = row + r < r1 && j * 16 < n_left ? y[(long long)r * a.ldy + j * 16] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (row + r < r1 && j * 16 < n_left) {
+                    float v = acc[i][j][r] * undo[r];
+                    if (a.accumulate) v += old[j][r];
+                    else if (a.act == 1) { const float p = fmaxf(v, 0.0f); v = p * p; }          // NTK_ACT_RELU2
+                    if (d.Y16) d.Y16[(long long)(row + r) * d.ldy16 + col + j * 16] = (uint16_t)pack_bf16(v, 0.0f);
+                    else y[(long long)r * a.ldy + j * 16] = v;
+                }
+    }
+}
+
+// ---- which tile, and how many pieces of K.  A tile of a form takes `over` us beside its chunks (first requests, results); n of them on a CU, `resident` at a time, take
+// n * busy a chunk, one alone `alone` (latency).  Constants in us, from layer-like shapes of 16 .. 1024 rows (groups: 600 .. 6144), 2048 .. 14976 outputs, 512 .. 7488 inputs with weights
+// that come from memory; the estimate is within a sixth there, and the choice within a tenth of the best form but for uneven small groups.  Rows of several groups: tiles
+// of a group of the average size, plus half a tile where that is no small part of one.
+struct DirectForm { int TM, TN, resident; float alone, busy, over; };
+static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats) {
+    static const int counts[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    TilePlan best{0, 1, 1e30f};
+    const int chunks = (K + chunk - 1) / chunk;
+    for (int i = 0; i < n_forms; ++i) {
+        const float mean = (float)rows / groups / f[i].TM;
+        const float row_tiles = groups > 1 ? groups * (mean < 0.5f ? 1.0f : mean + 0.5f) : (float)((rows + f[i].TM - 1) / f[i].TM);
+        const float tiles = row_tiles * ((N + f[i].TN - 1) / f[i].TN);
+        for (int s : counts) {
+            if (s > 1 && ((long long)s * rows * N > scratch_floats || chunks < 4 * s)) break;
+            const int n = (int)((tiles * s + 255.0f) / 256.0f);
+            float us = (float)((chunks + s - 1) / s) * (n == 1 ? f[i].alone : n * f[i].busy) + f[i].over * ((n + f[i].resident - 1) / f[i].resident);
+            if (s > 1) us += 3.0f + (float)(s + 1) * rows * N * 4.0f / 7e6f;
+            if (us < best.us) best = TilePlan{i, s, us};
+        }
+    }
+    return best;
+}
+
+template <class P, int TM, int TN, int WM, int WN, int STAGES, bool GLU, int MINW>
+static void launch_direct(DirectArgs d, int splits, hipStream_t s) {
+    constexpr int BK = 128 / (int)sizeof(typename P::WT);
+    const int chunks = d.t.K / BK, per = (chunks + splits - 1) / splits;
+    d.t.k_per_split = per * BK;
+    d.t.splits = (chunks + per - 1) / per;
+    const int row_tiles = d.t.offsets ? d.t.T / TM + d.t.G : (d.t.T + TM - 1) / TM, col_tiles = GLU ? (d.glu_ff + TN / 2 - 1) / (TN / 2) : (d.t.N + TN - 1) / TN;
+    hipLaunchKernelGGL((gemm_direct_kernel<P, TM, TN, WM, WN, STAGES, GLU, MINW>), dim3(row_tiles * col_tiles * d.t.splits), dim3(64 * WM * WN), 0, s, d, row_tiles, col_tiles);
+    if (d.t.splits > 1) launch_tile_sum(d.t, s);
+}
+
+}  // namespace ntk

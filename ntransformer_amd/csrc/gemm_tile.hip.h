@@ -383,11 +383,10 @@ __global__ __launch_bounds__(256) void gemm_tile_sum_kernel(const TileArgs a) {
 // measured on the shapes of model layers: 12 .. 1024 rows, 2048 .. 28672 outputs, 512 .. 14336 inputs.  Over 70 such shapes it is
 // 2 % behind the best tile and split on average, by more than a tenth in four, by a fifth at most (40 x 28672 x 4096 bf16: 49 us, 41 with 64 x 128 in two pieces).
 struct TileForm { int TM, TN, chunk; float alone, busy; };
-struct TilePlan { int form, splits; };
+struct TilePlan { int form, splits; float us; };
 static TilePlan plan_tiles(const TileForm* f, int n_forms, int rows, int groups, int N, int K, long long scratch_floats) {
     static const int counts[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    TilePlan best{0, 1};
-    float best_us = 1e30f;
+    TilePlan best{0, 1, 1e30f};
     for (int i = 0; i < n_forms; ++i) {
         // (rows of several groups: on average half a tile of each is empty)
         const int row_tiles = groups > 1 ? rows / f[i].TM + (groups + 1) / 2 : (rows + f[i].TM - 1) / f[i].TM;
@@ -398,10 +397,16 @@ static TilePlan plan_tiles(const TileForm* f, int n_forms, int rows, int groups,
             const float per_cu = (float)((tiles * s + 255) / 256);
             float us = (float)((chunks + s - 1) / s) * (f[i].alone > per_cu * f[i].busy ? f[i].alone : per_cu * f[i].busy);
             if (s > 1) us += 4.0f + (float)(s + 1) * rows * N * 4.0f / 4e6f;
-            if (us < best_us) { best_us = us; best = TilePlan{i, s}; }
+            if (us < best.us) best = TilePlan{i, s, us};
         }
     }
     return best;
+}
+
+static void launch_tile_sum(const TileArgs& a, hipStream_t s) {
+    const bool four = a.N % 4 == 0 && a.ldy % 4 == 0 && !(((uintptr_t)a.Y | (uintptr_t)a.part) & 15);
+    if (four) hipLaunchKernelGGL((gemm_tile_sum_kernel<4>), dim3((a.N / 4 + 255) / 256, a.T), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((gemm_tile_sum_kernel<1>), dim3((a.N + 255) / 256, a.T), dim3(256), 0, s, a);
 }
 
 template <class P, int TM, int TN, int SUB, int WM, int WN, bool VEC>
@@ -412,10 +417,7 @@ static void launch_tiles(TileArgs a, int splits, hipStream_t s) {
     a.splits = (chunks + per - 1) / per;
     const int row_tiles = a.offsets ? a.T / TM + a.G : (a.T + TM - 1) / TM;
     hipLaunchKernelGGL((gemm_tile_kernel<P, TM, TN, SUB, WM, WN, VEC>), dim3((a.N + TN - 1) / TN, row_tiles * a.splits), dim3(64 * WM * WN), 0, s, a);
-    if (a.splits == 1) return;
-    const bool four = a.N % 4 == 0 && a.ldy % 4 == 0 && !(((uintptr_t)a.Y | (uintptr_t)a.part) & 15);
-    if (four) hipLaunchKernelGGL((gemm_tile_sum_kernel<4>), dim3((a.N / 4 + 255) / 256, a.T), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((gemm_tile_sum_kernel<1>), dim3((a.N + 255) / 256, a.T), dim3(256), 0, s, a);
+    if (a.splits > 1) launch_tile_sum(a, s);
 }
 
 }  // namespace ntk

@@ -24,6 +24,10 @@ class DenseDesc(C.Structure):
                 ("x_out", C.c_void_p), ("ldxo", C.c_int), ("scratch", C.c_void_p), ("scratch_bytes", C.c_size_t), ("full_x", C.c_int)]
 
 
+class DirectDesc(C.Structure):
+    _fields_ = [("x16", C.c_void_p), ("ldx16", C.c_int), ("x16_rows", C.c_int), ("y16", C.c_void_p), ("ldy16", C.c_int)]
+
+
 class Rotary(C.Structure):
     _fields_ = [("freq", C.c_void_p), ("mag", C.c_float), ("dims", C.c_int), ("layout", C.c_int)]
 
@@ -87,6 +91,8 @@ def _bind():
         return L
     vp, i, f, ll = C.c_void_p, C.c_int, C.c_float, C.c_longlong
     L.ntk_dense.argtypes = [C.POINTER(DenseDesc), vp]
+    L.ntk_dense_direct.argtypes = [C.POINTER(DenseDesc), C.POINTER(DirectDesc), vp]
+    L.ntk_round_rows.argtypes = [vp, i, vp, i, i, i, vp]
     L.ntk_embed_sinusoid.argtypes = [vp, vp, i, vp, i, i, i, f, vp, i, vp]
     L.ntk_latent_fold_query_prepare.argtypes = [vp, vp, i, vp, i, i, i, i, i, vp, i, vp, i, vp, f, i, vp]
     L.ntk_moe_pick.argtypes = [vp, vp, vp, vp, i, i, i, i, C.POINTER(RouteDesc), vp]
@@ -94,6 +100,8 @@ def _bind():
     L.ntk_moe_sum_ex.argtypes = [vp, vp, vp, vp, i, vp, i, vp, vp, vp, i, i, i, vp]
     L.ntk_dense_linear.argtypes = [vp, i, vp, i, vp, i, i, i, i, i, vp]
     L.ntk_embed_dense.argtypes = [vp, vp, i, vp, i, i, i, vp]
+    L.ntk_rmsnorm_offset_16.argtypes = [vp, vp, vp, vp, vp, vp, i, vp, i, i, i, f, f, vp]
+    L.ntk_rms_seam_16.argtypes = [vp, vp, i, vp, i, vp, f, vp, i, i, f, vp]
     L.ntk_rmsnorm_offset.argtypes = [vp, vp, vp, vp, i, vp, i, i, i, f, f, vp]
     L.ntk_concat_rows.argtypes = [vp, vp, vp, i, i, vp]
     L.ntk_sigmoid_gate.argtypes = [vp, i, vp, i, i, i, vp]
@@ -214,6 +222,62 @@ def dense(x: np.ndarray, w: np.ndarray, dtype: str = "float32", offsets=None, ro
         check(L.ntk_dense(C.byref(d), None), "ntk_dense")
     y = yb.numpy(np.float32, T * N).reshape(T, N)
     return (y, xo.numpy(np.float32, T * K).reshape(T, K)) if add is not None else y
+
+
+def _bf16(a: np.ndarray) -> np.ndarray:
+    """uint16 bfloat16 -> float32"""
+    return (a.astype(np.uint32) << 16).view(np.float32)
+
+
+def round_rows(x: np.ndarray, n: Optional[int] = None) -> np.ndarray:
+    """the first n columns rounded to bfloat16 (as float32)"""
+    L = _bind()
+    T, n = x.shape[0], n or x.shape[1]
+    xb, yb = _f(x), DeviceBuffer.zeros(T * n * 2)
+    check(L.ntk_round_rows(yb.ptr, n, xb.ptr, x.shape[1], T, n, None), "ntk_round_rows")
+    return _bf16(yb.numpy(np.uint16, T * n).reshape(T, n))
+
+
+def dense_direct(x: np.ndarray, w: np.ndarray, offsets=None, rows=None, row_div: int = 1, n_rows: Optional[int] = None, y0: Optional[np.ndarray] = None, out16: bool = False,
+                 glu_limit: Optional[float] = None, glu_alpha: float = 1.702, glu_up_offset: float = 1.0, glu_cubic: float = 0.0, act: int = ACT_NONE, scratch_floats: int = 0,
+                 fill: float = 0.0):
+    """dense() over activations that are rounded to bfloat16 in a launch of their own; out16 or glu_limit: bfloat16 results (as float32), else float32 ones"""
+    L = _bind()
+    w = np.asarray(w)
+    stacked = w.ndim == 3
+    N, K = w.shape[-2], w.shape[-1]
+    T = int(n_rows if n_rows is not None else (len(rows) if rows is not None else x.shape[0]))
+    glu = glu_limit is not None
+    n_out = N // 2 if glu else N
+    xb, (wb, wdt) = _f(x), weight_buffer(w, "bfloat16")
+    x16 = DeviceBuffer.zeros(x.shape[0] * K * 2)
+    check(L.ntk_round_rows(x16.ptr, K, xb.ptr, x.shape[1], x.shape[0], K, None), "ntk_round_rows")
+    yb = _f(y0) if y0 is not None else _f(np.full((max(T, 1), n_out), fill, np.float32))
+    ob = _i(offsets) if offsets is not None else None
+    rb = _i(rows) if rows is not None else None
+    sb = DeviceBuffer(scratch_floats * 4) if scratch_floats else None
+    d = DenseDesc(yb.ptr, n_out, None, 0, wb.ptr, N * K if stacked else 0, wdt, ob.ptr if ob else None, w.shape[0] if stacked else 1, rb.ptr if rb else None, row_div, T, N, K,
+                  int(y0 is not None))
+    d.act = act
+    if sb is not None:
+        d.scratch, d.scratch_bytes = sb.ptr, scratch_floats * 4
+    if glu:
+        d.glu_ff, d.glu_limit, d.glu_alpha, d.glu_up_offset, d.glu_cubic = n_out, glu_limit, glu_alpha, glu_up_offset, glu_cubic
+    e = DirectDesc(x16.ptr, K, x.shape[0], yb.ptr if glu or out16 else None, n_out)
+    check(L.ntk_dense_direct(C.byref(d), C.byref(e), None), "ntk_dense_direct")
+    if glu or out16:
+        return _bf16(yb.numpy(np.uint16, T * n_out).reshape(T, n_out))
+    return yb.numpy(np.float32, T * n_out).reshape(T, n_out)
+
+
+def rmsnorm_offset_16(x: np.ndarray, w1: np.ndarray, w2: np.ndarray, eps: float, offset: float):
+    """-> the first norm as bfloat16, the second as float32 and as bfloat16 (all as float32)"""
+    L = _bind()
+    T, n = x.shape
+    xb, w1b, w2b = _f(x), _f(w1), _f(w2)
+    a, y, b = DeviceBuffer.zeros(T * n * 2), DeviceBuffer.zeros(T * n * 4), DeviceBuffer.zeros(T * n * 2)
+    check(L.ntk_rmsnorm_offset_16(None, a.ptr, w1b.ptr, y.ptr, b.ptr, w2b.ptr, n, xb.ptr, n, T, n, eps, offset, None), "ntk_rmsnorm_offset_16")
+    return _bf16(a.numpy(np.uint16, T * n).reshape(T, n)), y.numpy(np.float32, T * n).reshape(T, n), _bf16(b.numpy(np.uint16, T * n).reshape(T, n))
 
 
 def rmsnorm_offset(x: np.ndarray, w1: np.ndarray, w2: Optional[np.ndarray], eps: float, offset: float):
@@ -742,6 +806,17 @@ def rms_seam(x: np.ndarray, w: Optional[np.ndarray], eps: float, add_y: Optional
     hb = DeviceBuffer.zeros(T * n * 4) if w is not None else None
     check(L.ntk_rms_seam(hb.ptr if hb else None, n, xb.ptr, n, yb.ptr if yb else None, n, awb.ptr if awb else None, mult, wb.ptr if wb else None, T, n, eps, None), "ntk_rms_seam")
     return xb.numpy(np.float32, T * n).reshape(T, n), (hb.numpy(np.float32, T * n).reshape(T, n) if hb else None)
+
+
+def rms_seam_16(x: np.ndarray, w: np.ndarray, eps: float, add_y: Optional[np.ndarray] = None, add_w: Optional[np.ndarray] = None, mult: float = 1.0):
+    """rms_seam with the normed rows rounded to bfloat16 (as float32)"""
+    L = _bind()
+    T, n = x.shape
+    xb, wb = _f(x), _f(w)
+    yb, awb = (_f(a) if a is not None else None for a in (add_y, add_w))
+    hb = DeviceBuffer.zeros(T * n * 2)
+    check(L.ntk_rms_seam_16(hb.ptr, xb.ptr, n, yb.ptr if yb else None, n, awb.ptr if awb else None, mult, wb.ptr, T, n, eps, None), "ntk_rms_seam_16")
+    return xb.numpy(np.float32, T * n).reshape(T, n), _bf16(hb.numpy(np.uint16, T * n).reshape(T, n))
 
 
 def causal_conv_act(x: np.ndarray, w: np.ndarray, pos0: int, state: Optional[np.ndarray] = None, act: int = 1, n: Optional[int] = None):

@@ -1,0 +1,121 @@
+"""Products whose operands go from memory straight into LDS (csrc/gemm_direct.hip.h) and the launches that leave rounded activations for them, against float64 over the
+rounded inputs.  Bounds: a sum of K products in 32 bits is off by at most (K + 2) 2^-24 of the sum of their sizes; a bfloat16 result by 2^-8 of itself beside that."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -24
+
+
+def _round(x):
+    u = np.ascontiguousarray(x, np.float32).view(np.uint32).astype(np.uint64)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16 << 16).astype(np.uint32).view(np.float32)
+
+
+def _case(rng, T, N, K, G=0):
+    return rng.standard_normal((T, K)).astype(np.float32), _round(rng.standard_normal((G, N, K) if G else (N, K)).astype(np.float32) / np.sqrt(K))
+
+
+def _close(got, x, w, out=None, bf=False, slack=1.0):
+    xd, wd = _round(x).astype(np.float64), w.astype(np.float64)
+    ref = xd @ wd.T
+    bound = (x.shape[1] + 2) * U * (np.abs(xd) @ np.abs(wd).T)
+    if out is not None:
+        ref, bound = out(ref, bound)
+    if bf:
+        bound = bound + 2.0 ** -8 * (np.abs(ref) + bound)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - ref) <= slack * bound + 1e-30).all(), float((np.abs(got - ref) / (bound + 1e-30)).max())
+
+
+# tiles of 64 x 64 .. 256 x 256 and one row, column or chunk less or more; the last three take the large tiles
+@pytest.mark.parametrize("T,N,K", [(9, 16, 64), (9, 1, 64), (63, 65, 128), (64, 64, 192), (65, 130, 64), (129, 257, 320), (255, 512, 448), (257, 63, 1024), (300, 4097, 256),
+                                   (1000, 6200, 64), (1025, 6300, 192), (1000, 16300, 128)])
+def test_direct_products(T, N, K):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(T + N + K)
+    x, w = _case(rng, T, N, K)
+    _close(Lr.dense_direct(x, w), x, w)
+    if T * N < 2e6:
+        y0 = rng.standard_normal((T, N)).astype(np.float32)
+        _close(Lr.dense_direct(x, w, y0=y0), x, w, lambda r, b: (r + y0, b + 2 * U * (np.abs(y0) + np.abs(r))))
+        _close(Lr.dense_direct(x, w, scratch_floats=16 * T * N), x, w, lambda r, b: (r, 2 * b))       # pieces of K
+        _close(Lr.dense_direct(x, w, out16=True, act=1), x, w, lambda r, b: (np.maximum(r, 0) ** 2, 2 * np.abs(r) * b + b * b), bf=True)
+
+
+@pytest.mark.parametrize("T,ff,K", [(9, 8, 64), (65, 33, 128), (200, 129, 256), (257, 448, 64), (1030, 3111, 64), (1024, 8200, 64)])
+@pytest.mark.parametrize("limit,alpha,up,cubic", [(7.0, 1.702, 1.0, 0.0), (float("inf"), 1.0, 0.0, 0.0), (float("inf"), 1.5957691, 0.0, 0.044715)])
+def test_gated_units_inside_the_product(T, ff, K, limit, alpha, up, cubic):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(T + ff)
+    x, w = _case(rng, T, 2 * ff, K)
+
+    def unit(r, b):
+        g, u = np.minimum(r[:, :ff], limit), np.clip(r[:, ff:], -limit, limit)
+        s = 1.0 / (1.0 + np.exp(-alpha * (g + cubic * g ** 3)))
+        # both factors off by their product's bound (the gate's slope is below 1.2), and a few roundings of the unit itself
+        return g * s * (u + up), 1.2 * b[:, :ff] * (np.abs(u + up) + b[:, ff:]) + np.abs(g) * b[:, ff:] + 16 * U * np.abs(g) * (np.abs(u) + 1.0)
+    _close(Lr.dense_direct(x, w, glu_limit=limit, glu_alpha=alpha, glu_up_offset=up, glu_cubic=cubic), x, w, unit, bf=True)
+
+
+@pytest.mark.parametrize("counts", [[0, 1, 64, 65, 0, 130], [300, 0, 0, 3], [255, 256, 257, 1], [17] * 70])
+def test_groups_and_gathered_rows(counts):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(len(counts))
+    T, N, K, G, div = sum(counts), 200, 128, len(counts), 3
+    x, w = _case(rng, (T + div - 1) // div, N, K, G)
+    rows, off = rng.permutation(T), np.concatenate([[0], np.cumsum(counts)])
+    got = Lr.dense_direct(x, w, offsets=off, rows=rows, row_div=div)
+    same = Lr.dense_direct(x[rows // div], w, offsets=off)
+    extra = Lr.dense_direct(x[rows // div], w, offsets=np.minimum(off, T - 5), fill=3.0)                   # rows that belong to no group stay as they are
+    assert np.array_equal(got, same) and (extra[T - 5:] == 3.0).all() and np.array_equal(extra[:T - 5], got[:T - 5])
+    for g in range(G):
+        if counts[g]:
+            _close(got[off[g]:off[g + 1]], x[rows[off[g]:off[g + 1]] // div], w[g])
+
+
+@pytest.mark.parametrize("T,N,K,ld", [(40, 2048, 1024, 1028), (200, 1500, 512, 512), (1000, 2048, 2048, 2112), (300, 700, 1000, 1000)])
+def test_the_product_with_room_for_rounded_activations_equals_the_one_without(T, N, K, ld):
+    """one chain of matrix instructions over the inputs in both: the same bits, unless the inputs are cut into pieces"""
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(N)
+    x = rng.standard_normal((T, ld)).astype(np.float32)
+    w = _round(rng.standard_normal((N, K)).astype(np.float32) / np.sqrt(K))
+    x[3, 5], x[5, 7] = np.inf, np.nan
+    a = Lr.dense(x, w, "bfloat16")
+    b = Lr.dense(x, w, "bfloat16", scratch_floats=T * K // 2 + 4)              # room for the rounded rows alone
+    assert np.array_equal(np.isfinite(a), np.isfinite(b)) and not np.isfinite(b[[3, 5]]).any()
+    assert np.array_equal(np.nan_to_num(a), np.nan_to_num(b))
+    c = Lr.dense(x, w, "bfloat16", scratch_floats=T * K // 2 + 8 * T * N)
+    fin = np.delete(np.arange(T), [3, 5])
+    _close(c[fin], x[fin, :K], w, lambda r, e: (r, 2 * e))
+
+
+def test_rounding_and_what_is_refused():
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(0)
+    for T, ld, n in ((3, 16, 16), (70, 100, 96), (9, 37, 37), (5, 40, 33)):
+        x = rng.standard_normal((T, ld)).astype(np.float32)
+        assert np.array_equal(Lr.round_rows(x, n), _round(x[:, :n]))
+    for T, K in ((8, 64), (20, 96)):           # few rows; no whole chunks of inputs
+        with pytest.raises(Exception):
+            Lr.dense_direct(rng.standard_normal((T, K)).astype(np.float32), np.ones((16, K), np.float32))
+
+
+@pytest.mark.parametrize("T,n", [(1, 4), (9, 64), (33, 1020), (40, 2048), (9, 4096)])
+def test_norms_that_leave_rounded_rows(T, n):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(n)
+    x, y = rng.standard_normal((2, T, n)).astype(np.float32)
+    w, aw = rng.standard_normal((2, n)).astype(np.float32)
+    # (another order of the row's sum: a rounded value may fall to the other side)
+    near = lambda got, want: (np.abs(got - want) <= 2.0 ** -7 * np.abs(want) + 1e-30).all()
+    a, b, c = Lr.rmsnorm_offset_16(x, w, aw, 1e-5, 1.0)
+    p, q = Lr.rmsnorm_offset(x, w, aw, 1e-5, 1.0)
+    assert near(a, p) and np.allclose(b, q, rtol=2e-6, atol=0) and np.array_equal(c, _round(b))
+    for add in (None, y):
+        gx, gh = Lr.rms_seam_16(x, w, 1e-5, add, aw if add is not None else None, 0.7)
+        sx, sh = Lr.rms_seam(x, w, 1e-5, add, aw if add is not None else None, 0.7)
+        assert np.allclose(gx, sx, rtol=2e-6, atol=2e-6) and near(gh, sh)
+    with pytest.raises(Exception):
+        Lr.rms_seam_16(rng.standard_normal((2, 4100)).astype(np.float32), np.ones(4100, np.float32), 1e-5)
