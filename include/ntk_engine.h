@@ -216,6 +216,20 @@ size_t ntk_gemm_half_workspace_bytes(int n_tokens);
 int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
                   size_t workspace_bytes, void* stream);
 
+/* ... for up to three such matrices over the same X (query, key and value; gate and up) in one launch, with the activations' two halves formed once per pass in the workspace
+ * (ntk_gemm_half_many_bytes() of it at least; more is used for partial sums).  Y[i] = W[i] . X; silu != 0 (n == 2, out[0] == out[1]): Y[0] = silu(W[0] . X) * (W[1] . X) alone (ntk_silu_mul).
+ * accumulate only with n == 1.  NTK_E_SHAPE where in_features is no multiple
+ * of 64, the workspace is too small for 16 tokens or, with silu, the two matrices lie 4 GiB apart: nothing has been launched then. */
+typedef struct ntk_half_desc {
+    const void* W[3]; float* Y[3]; int out[3]; int n;
+    const float* X; int n_tokens, in_features, accumulate;
+    const float* row_max;
+    int silu;
+    void* workspace; size_t workspace_bytes;
+} ntk_half_desc;
+size_t ntk_gemm_half_many_bytes(int n_tokens, int in_features);
+int ntk_gemm_half_many(const ntk_half_desc* d, void* stream);
+
 /* Dequantise rows of a (quantised) embedding table on the device: out[t,:] = table[tokens[t],:].
  * Same arithmetic as the host loop in reference src/model/transformer.cpp:419-599; Q5_K is zero-filled
  * exactly as the reference does (:595-598).  tokens is a DEVICE int array. */

@@ -523,7 +523,7 @@ static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long r
                                        {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
     return plan_direct(forms, 7, 64, rows, groups, N, K, room);
 }
-template <bool GLU>
+template <int GLU>
 static void launch_direct_bf16(const DirectArgs& d, const TilePlan& p, hipStream_t s) {
     switch (p.form) {
         case 0: launch_direct<TileBf16, 256, 256, 4, 2, 2, GLU, 2>(d, p.splits, s); break;
@@ -578,9 +578,9 @@ int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* st
     const long long room = d->scratch && !((uintptr_t)d->scratch & 15) && !d->offsets && !e->y16 && d->T <= 65535 ? (long long)(d->scratch_bytes / sizeof(float)) : 0;
     const TilePlan p = plan_direct_bf16(d->T, G, d->N, d->K, room);
     if (glu) {
-        a.glu_ff = d->glu_ff; a.limit = d->glu_limit; a.alpha = d->glu_alpha; a.up_offset = d->glu_up_offset; a.cubic = d->glu_cubic;
-        launch_direct_bf16<true>(a, p, resolve_stream(stream));
-    } else launch_direct_bf16<false>(a, p, resolve_stream(stream));
+        a.glu_ff = d->glu_ff; a.up_at = (uint32_t)d->glu_ff * (uint32_t)d->K * 2; a.limit = d->glu_limit; a.alpha = d->glu_alpha; a.up_offset = d->glu_up_offset; a.cubic = d->glu_cubic;
+        launch_direct_bf16<kGluClipped>(a, p, resolve_stream(stream));
+    } else launch_direct_bf16<kGluNone>(a, p, resolve_stream(stream));
     return last_launch_status();
 }
 
@@ -655,7 +655,7 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
                 a16.t = t;
                 a16.t.part = (float*)((char*)d->scratch + image);
                 a16.X16 = d->scratch; a16.x_row = (uint32_t)d->K * 2;
-                launch_direct_bf16<false>(a16, q, s);
+                launch_direct_bf16<kGluNone>(a16, q, s);
                 return last_launch_status();
             }
         }

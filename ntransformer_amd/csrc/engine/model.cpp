@@ -707,6 +707,23 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         ok(ntk_gemm_half(Y, w.ptr, X, T, (int)w.out_f, (int)w.in_f, accumulate ? 1 : 0, rm, ws, gemm_ws_bytes_, s));
         return true;
     };
+    // several of them over one X in one launch (silu: gate and up, Y[0] = silu(gate) * up); false: not such matrices, nothing was launched
+    auto project_half_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, bool silu) -> bool {
+        ntk_half_desc d{};
+        for (int i = 0; i < n; ++i) {
+            if (!batched || !bf16_now || !Ws[i]->ptr || Ws[i]->dtype != NTK_DT_F16 || Ws[i]->in_f < 3072 || Ws[i]->in_f != Ws[0]->in_f) return false;
+            d.W[i] = Ws[i]->ptr; d.Y[i] = Ys[i]; d.out[i] = (int)Ws[i]->out_f;
+        }
+        void* ws = cur_ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_;   // (as above)
+        const bool own = ws != nullptr;
+        d.n = n; d.X = X; d.n_tokens = T; d.in_features = (int)Ws[0]->in_f; d.row_max = rm; d.silu = silu ? 1 : 0;
+        d.workspace = own ? ws : cur_ws; d.workspace_bytes = gemm_ws_bytes_;
+        const int st = ntk_gemm_half_many(&d, s);
+        if (st == NTK_E_SHAPE || st == NTK_E_ALIGN) return false;
+        if (!own) planes_of = nullptr;
+        ok(st);
+        return true;
+    };
     auto project = [&](float* Y, const DevTensor& w, const float* X, size_t ystride, size_t xstride, const float* rm) {
         if (batched && project_half(Y, w, X, ystride, xstride, false, rm)) return;
         if (batched && bf16_rp && rp_only(w) && ystride == (size_t)w.out_f && xstride == (size_t)w.in_f) {   // straight from the repack
@@ -733,6 +750,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
     // matrices that share X (Q | K | V, gate | up): those of one format go out as ONE launch of the FP16 GEMM, the rest one by one
     auto project_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm) {
         bool done[3] = {false, false, false};
+        if (project_half_many(Ys, Ws, n, X, rm, false)) return;
         if (batched && bf16_now) {
             for (int a = 0; a < n; ++a) {
                 if (done[a]) continue;
@@ -879,6 +897,11 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
                 ok(st);
                 ffn_done = true;
             }
+        }
+        if (!ffn_done && tp_world_ == 1 && (size_t)L.w_gate.out_f == (size_t)I && (size_t)L.w_up.out_f == (size_t)I) {      // half-precision gate and up meet in their product's launch
+            float* const ys[2] = {gate_buf, nullptr};
+            const DevTensor* const ws[2] = {&L.w_gate, &L.w_up};
+            ffn_done = project_half_many(ys, ws, 2, residual_, max_a, true);
         }
         if (!ffn_done) {
             float* const ys[2] = {gate_buf, up_buf};

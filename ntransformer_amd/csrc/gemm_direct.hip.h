@@ -17,9 +17,14 @@ namespace ntk {
 struct DirectArgs {
     TileArgs t;                                     // X unused
     const void* X16; uint32_t x_row; long long plane;      // activations as the matrix cores take them, rows of x_row bytes; PIECES planes, `plane` bytes apart
-    uint16_t* Y16; int ldy16; int glu_ff;           // bfloat16 results in the place of t.Y (or NULL); GLU: [r][f] = gated unit of rows f and glu_ff + f of W
+    uint16_t* Y16; int ldy16; int glu_ff;           // bfloat16 results in the place of t.Y (or NULL); gated units: [r][f] of the weight rows f behind gate_at and up_at bytes of W
+    uint32_t gate_at, up_at;
     float limit, alpha, up_offset, cubic;
+    // several matrices side by side over the same activations (n_seg > 1, no groups, nothing accumulated): the column tiles of one after those of the other, their pieces' columns too
+    int n_seg; const void* segW[3]; float* segY[3]; int seg_out[3], seg_tile[3];
 };
+enum { kGluNone = 0, kGluClipped = 1, kGluSilu = 2 };       // kGluSilu: silu(gate) * up as F32, as a launch of its own forms it
+template <typename T> __device__ __forceinline__ T seg_pick(const T (&v)[3], int i) { return i == 0 ? v[0] : i == 1 ? v[1] : v[2]; }
 
 // N requests of 16 bytes a lane: lane l's land at lds + i * step + 16 l.  The compiler does not count them (M0 is the compiler's: saved and restored)
 template <int STEP>
@@ -56,7 +61,7 @@ template <int V> __device__ __forceinline__ void direct_wait() {   // all but th
 }
 
 // one-dimensional grid over (row tiles, column tiles, splits), row tiles first; rows of X and W are whole multiples of 128 bytes
-template <class P, int TM, int TN, int WM, int WN, int STAGES, bool GLU, int MINW>
+template <class P, int TM, int TN, int WM, int WN, int STAGES, int GLU, int MINW>
 __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const DirectArgs d, const int row_tiles, const int col_tiles) {
     const TileArgs& a = d.t;
     constexpr int CB = 128, ES = sizeof(typename P::WT), BK = CB / ES, PIECES = P::PIECES, NW = WM * WN, WTM = TM / WM, WTN = TN / WN, MI = WTM / 16, NJ = WTN / 16;
@@ -69,10 +74,20 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
     int id = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
     const int rt = id % row_tiles;
     id /= row_tiles;
-    const int ct = id % col_tiles, split = id / col_tiles;
+    int ct = id % col_tiles;
+    const int split = id / col_tiles;
+    const void* Wp = a.W;
+    float* Yp = a.Y;
+    int n_cols = GLU ? d.glu_ff : a.N, ldy = a.ldy, part_col = 0;
+    if (!GLU && d.n_seg > 1) {
+        const int sg = (ct >= d.seg_tile[1] ? 1 : 0) + (d.n_seg > 2 && ct >= d.seg_tile[2] ? 1 : 0);
+        ct -= sg ? seg_pick(d.seg_tile, sg) : 0;
+        Wp = seg_pick(d.segW, sg); Yp = seg_pick(d.segY, sg); n_cols = ldy = seg_pick(d.seg_out, sg);
+        part_col = (sg > 0 ? d.seg_out[0] : 0) + (sg > 1 ? d.seg_out[1] : 0);
+    }
     int g = 0, row_base = rt * TM, r1 = a.T;
     if (a.offsets) { if (!group_tile(a.offsets, a.G, rt, TM, g, row_base, r1)) return; }
-    const int n_cols = GLU ? d.glu_ff : a.N, n_base = ct * (GLU ? TN / 2 : TN);
+    const int n_base = ct * (GLU ? TN / 2 : TN);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM;
     const int k_begin = split * a.k_per_split, k_end = min(a.K, k_begin + a.k_per_split), n_chunks = (k_end - k_begin) / BK;
     // a request brings eight rows of 128 bytes; the 16-byte pieces of row r are stored in the order piece ^ (r & 7)
@@ -86,15 +101,14 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 #pragma unroll
     for (int i = 0; i < NWL; ++i) {
         const int row = (i * NW + wave) * 8 + (lane >> 3);
-        int n;
-        if constexpr (GLU) {                        // a wave's columns: as many gates as the up rows of the same outputs behind them
-            const int c = n_base + (row / WTN) * (WTN / 2) + row % (WTN / 2);
-            n = min(c, n_cols - 1) + (row % WTN >= WTN / 2 ? d.glu_ff : 0);
-        } else n = min(n_base + row, n_cols - 1);
-        wo[i] = (uint32_t)(GLU ? n : n - n_base) * row_bytes + (uint32_t)(((lane & 7) ^ (row & 7)) * 16);
+        if constexpr (GLU != kGluNone) {            // a wave's columns: as many gates as the up rows of the same outputs behind them
+            const int n = min(n_base + (row / WTN) * (WTN / 2) + row % (WTN / 2), n_cols - 1);
+            wo[i] = (uint32_t)n * row_bytes + (row % WTN >= WTN / 2 ? d.up_at : d.gate_at);
+        } else wo[i] = (uint32_t)(min(n_base + row, n_cols - 1) - n_base) * row_bytes;
+        wo[i] += (uint32_t)(((lane & 7) ^ (row & 7)) * 16);
     }
     const char* xb = (const char*)d.X16 + (long long)k_begin * ES;
-    const char* wb = (const char*)a.W + ((long long)g * a.wstride + (GLU ? 0 : (long long)n_base * a.K) + k_begin) * ES;
+    const char* wb = (const char*)Wp + ((long long)g * a.wstride + (GLU ? 0 : (long long)n_base * a.K) + k_begin) * ES;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     const uint32_t mine = lds0 + wave * 1024;
     auto request = [&](int chunk, int slot) {
@@ -139,12 +153,14 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 #pragma unroll
                 for (int i = 0; i < MI; ++i) xf[i] = *reinterpret_cast<const uintx4_t*>(s + q * XB + (wm * WTM + i * 16) * CB + piece);
 #pragma unroll
-                for (int i = 0; i < MI; ++i)
+                for (int c = 0; c < P::STEPS; ++c)          // (neighbouring instructions on different accumulators)
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) {
-                        if (SEP && q > 0) low[SEP ? i : 0][SEP ? j : 0] = P::mma(xf[i], wf[j], low[SEP ? i : 0][SEP ? j : 0]);
-                        else acc[i][j] = P::mma(xf[i], wf[j], acc[i][j]);
-                    }
+                    for (int i = 0; i < MI; ++i)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) {
+                            if (SEP && q > 0) low[SEP ? i : 0][SEP ? j : 0] = P::step(xf[i], wf[j], low[SEP ? i : 0][SEP ? j : 0], c);
+                            else acc[i][j] = P::step(xf[i], wf[j], acc[i][j], c);
+                        }
             }
         }
     };
@@ -175,12 +191,31 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
             for (int j = 0; j < NJ; ++j) acc[i][j] = total[i][j];
     }
     // accumulator lane map: row 4 * (lane / 16) + r, column lane % 16
-    if constexpr (GLU) {
+    if constexpr (GLU == kGluSilu) {
         const int col = n_base + wn * (WTN / 2) + (lane & 15), n_left = n_cols - col;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
             const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
-            uint16_t* y = d.Y16 + (long long)row * d.ldy16 + col;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const bool in = row + r < r1;
+                const float undo = P::SCALED ? half_unscale(a.row_max[min(row + r, a.T - 1)]) : 1.0f;
+                float* y = Yp + (long long)(row + r) * ldy + col;
+#pragma unroll
+                for (int j = 0; j < NJ / 2; ++j)
+                    if (in && j * 16 < n_left) {
+                        const float gg = acc[i][j][r] * undo;
+                        y[j * 16] = gg / (1.0f + expf(-gg)) * (acc[i][NJ / 2 + j][r] * undo);
+                    }
+            }
+        }
+        return;
+    }
+    if constexpr (GLU == kGluClipped) {
+        const int col = n_base + wn * (WTN / 2) + (lane & 15), n_left = n_cols - col;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
 #pragma unroll
             for (int j = 0; j < NJ / 2; ++j)
 #pragma unroll
@@ -189,12 +224,13 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
                         const float gg = fminf(acc[i][j][r], d.limit), uu = fminf(fmaxf(acc[i][NJ / 2 + j][r], -d.limit), d.limit);
                         const float zz = d.cubic != 0.0f ? fmaf(d.cubic * gg * gg, gg, gg) : gg;
                         const float v = gg * (1.0f / (1.0f + expf(-d.alpha * zz))) * (uu + d.up_offset);
-                        y[(long long)r * d.ldy16 + j * 16] = (uint16_t)pack_bf16(v, 0.0f);
+                        if (d.Y16) d.Y16[(long long)(row + r) * d.ldy16 + col + j * 16] = (uint16_t)pack_bf16(v, 0.0f);
+                        else Yp[(long long)(row + r) * ldy + col + j * 16] = v;
                     }
         }
         return;
     }
-    const int col = n_base + wn * WTN + (lane & 15), n_left = a.N - col;
+    const int col = n_base + wn * WTN + (lane & 15), n_left = n_cols - col;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
@@ -203,7 +239,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 #pragma unroll
             for (int r = 0; r < 4; ++r) undo[r] = half_unscale(a.row_max[min(row + r, a.T - 1)]);
         if (a.splits > 1) {
-            float* y = a.part + ((long long)split * a.T + row) * a.N + col;
+            float* y = a.part + ((long long)split * a.T + row) * a.N + part_col + col;
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -211,13 +247,13 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
                     if (row + r < r1 && j * 16 < n_left) y[(long long)r * a.N + j * 16] = acc[i][j][r] * undo[r];
             continue;
         }
-        float* y = a.Y + (long long)row * a.ldy + col;
+        float* y = Yp + (long long)row * ldy + col;
         float old[NJ][4] = {};
         if (a.accumulate)
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) old[j][r] = row + r < r1 && j * 16 < n_left ? y[(long long)r * a.ldy + j * 16] : 0.0f;
+                for (int r = 0; r < 4; ++r) old[j][r] = row + r < r1 && j * 16 < n_left ? y[(long long)r * ldy + j * 16] : 0.0f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -227,7 +263,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
                     if (a.accumulate) v += old[j][r];
                     else if (a.act == 1) { const float p = fmaxf(v, 0.0f); v = p * p; }          // NTK_ACT_RELU2
                     if (d.Y16) d.Y16[(long long)(row + r) * d.ldy16 + col + j * 16] = (uint16_t)pack_bf16(v, 0.0f);
-                    else y[(long long)r * a.ldy + j * 16] = v;
+                    else y[(long long)r * ldy + j * 16] = v;
                 }
     }
 }
@@ -256,15 +292,53 @@ static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int row
     return best;
 }
 
-template <class P, int TM, int TN, int WM, int WN, int STAGES, bool GLU, int MINW>
+// the pieces of several matrices' columns side by side, in order, into each one's own results
+template <int V>
+__global__ __launch_bounds__(256) void gemm_direct_sum_kernel(const DirectArgs d) {
+    const TileArgs& a = d.t;
+    const int n = (blockIdx.x * 256 + threadIdx.x) * V, r = blockIdx.y;
+    if (n >= a.N) return;
+    const int n1 = d.seg_out[0], n2 = n1 + d.seg_out[1], sg = (n >= n1 ? 1 : 0) + (d.n_seg > 2 && n >= n2 ? 1 : 0);
+    float* y = seg_pick(d.segY, sg) + (long long)r * seg_pick(d.seg_out, sg) + n - (sg == 0 ? 0 : sg == 1 ? n1 : n2);
+    const float* p = a.part + (long long)r * a.N + n;
+    float s[V] = {};
+    for (int i = 0; i < a.splits; i += 4) {                 // four requests under way
+        float v[4][V];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float* q = p + (long long)a.T * a.N * min(i + u, a.splits - 1);
+            if constexpr (V == 4) { const float4 t = *reinterpret_cast<const float4*>(q); v[u][0] = t.x; v[u][1] = t.y; v[u][2] = t.z; v[u][3] = t.w; }
+            else v[u][0] = *q;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u < a.splits)
+#pragma unroll
+                for (int j = 0; j < V; ++j) s[j] += v[u][j];
+    }
+    if constexpr (V == 4) *reinterpret_cast<float4*>(y) = float4{s[0], s[1], s[2], s[3]};
+    else y[0] = s[0];
+}
+
+template <class P, int TM, int TN, int WM, int WN, int STAGES, int GLU, int MINW>
 static void launch_direct(DirectArgs d, int splits, hipStream_t s) {
     constexpr int BK = 128 / (int)sizeof(typename P::WT);
     const int chunks = d.t.K / BK, per = (chunks + splits - 1) / splits;
     d.t.k_per_split = per * BK;
     d.t.splits = (chunks + per - 1) / per;
-    const int row_tiles = d.t.offsets ? d.t.T / TM + d.t.G : (d.t.T + TM - 1) / TM, col_tiles = GLU ? (d.glu_ff + TN / 2 - 1) / (TN / 2) : (d.t.N + TN - 1) / TN;
+    const int row_tiles = d.t.offsets ? d.t.T / TM + d.t.G : (d.t.T + TM - 1) / TM;
+    int col_tiles = GLU ? (d.glu_ff + TN / 2 - 1) / (TN / 2) : (d.t.N + TN - 1) / TN;
+    if (d.n_seg > 1) {
+        col_tiles = 0;
+        for (int i = 0; i < d.n_seg; ++i) { d.seg_tile[i] = col_tiles; col_tiles += (d.seg_out[i] + TN - 1) / TN; }
+    }
     hipLaunchKernelGGL((gemm_direct_kernel<P, TM, TN, WM, WN, STAGES, GLU, MINW>), dim3(row_tiles * col_tiles * d.t.splits), dim3(64 * WM * WN), 0, s, d, row_tiles, col_tiles);
-    if (d.t.splits > 1) launch_tile_sum(d.t, s);
+    if (d.t.splits == 1) return;
+    if (d.n_seg <= 1) { launch_tile_sum(d.t, s); return; }
+    bool four = !((uintptr_t)d.t.part & 15);
+    for (int i = 0; i < d.n_seg; ++i) four = four && d.seg_out[i] % 4 == 0 && !((uintptr_t)d.segY[i] & 15);
+    if (four) hipLaunchKernelGGL((gemm_direct_sum_kernel<4>), dim3((d.t.N / 4 + 255) / 256, d.t.T), dim3(256), 0, s, d);
+    else hipLaunchKernelGGL((gemm_direct_sum_kernel<1>), dim3((d.t.N + 255) / 256, d.t.T), dim3(256), 0, s, d);
 }
 
 }  // namespace ntk

@@ -54,12 +54,13 @@ struct TileArgs {
 // one-token products 0.86 1.22 1.59 | 0.85 1.22 1.59.
 struct TileBf16 {                                   // activations rounded to bfloat16
     using WT = uint16_t;
-    static constexpr int KE = 32, EP = 8, PIECES = 1, RUN = 0;
+    static constexpr int KE = 32, EP = 8, PIECES = 1, RUN = 0, STEPS = 1;
     static constexpr bool SCALED = false;
     __device__ static void convert(const float (&v)[EP], float, uintx4_t (&out)[PIECES]) {
         out[0] = uintx4_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
     }
     __device__ static floatx4_t mma(uintx4_t a, uintx4_t b, floatx4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bits_as<bf16x8_t>(a), bits_as<bf16x8_t>(b), c, 0, 0, 0); }
+    __device__ static floatx4_t step(uintx4_t a, uintx4_t b, floatx4_t c, int) { return mma(a, b, c); }
 };
 struct TileBf16x3 {                                 // bfloat16 weights, a 32-bit activation as the three bfloat16 values that add up to it
     using WT = uint16_t;
@@ -89,11 +90,13 @@ struct TileF32 {                                    // everything in 32 bits: v_
     __device__ static void convert(const float (&v)[EP], float, uintx4_t (&out)[PIECES]) {
         out[0] = uintx4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
     }
+    static constexpr int STEPS = 4;                     // (matrix instructions of an operand pair)
     __device__ static floatx4_t mma(uintx4_t a, uintx4_t b, floatx4_t c) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[i]), __uint_as_float(b[i]), c, 0, 0, 0);
+        for (int i = 0; i < 4; ++i) c = step(a, b, c, i);
         return c;
     }
+    __device__ static floatx4_t step(uintx4_t a, uintx4_t b, floatx4_t c, int i) { return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[i]), __uint_as_float(b[i]), c, 0, 0, 0); }
 };
 // the power of two that brings a row's largest |x| into [2^14, 2^15) (at most 2^125; below 2^15 whatever finite values stand beside an infinity), and its inverse
 __device__ __forceinline__ float half_scale(float largest) {
@@ -103,7 +106,7 @@ __device__ __forceinline__ float half_scale(float largest) {
 __device__ __forceinline__ float half_unscale(float largest) { return __uint_as_float((254u << 23) - __float_as_uint(half_scale(largest))); }
 struct TileHalf2 {                                  // IEEE-half weights, a 32-bit activation (times a power of two) as two halves: off by 2^-23 of it, or 2^-39 of its row's largest, at most
     using WT = uint16_t;
-    static constexpr int KE = 32, EP = 8, PIECES = 2, RUN = 128;
+    static constexpr int KE = 32, EP = 8, PIECES = 2, RUN = 128, STEPS = 1;
     static constexpr bool SCALED = true;                // rows times half_scale(row_max)
     __device__ static void convert(const float (&v)[EP], float scale, uintx4_t (&out)[PIECES]) {
         halfx8_t hi, lo;
@@ -118,6 +121,7 @@ struct TileHalf2 {                                  // IEEE-half weights, a 32-b
         __builtin_memcpy(&out[1], &lo, 16);
     }
     __device__ static floatx4_t mma(uintx4_t a, uintx4_t b, floatx4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(bits_as<halfx8_t>(a), bits_as<halfx8_t>(b), c, 0, 0, 0); }
+    __device__ static floatx4_t step(uintx4_t a, uintx4_t b, floatx4_t c, int) { return mma(a, b, c); }
 };
 
 // group and first row of row tile `t` when every group's rows are cut into tiles of TM (all groups together at most T / TM + G of them); false: past the last tile
