@@ -64,10 +64,11 @@ typedef struct ntk_dense_desc {
 #define NTK_ACT_RELU2 1
 int ntk_dense_few_rows(void);   /* up to this many rows a product takes the row-streaming form */
 int ntk_dense(const ntk_dense_desc* d, void* stream);
-/* The same product for more than ntk_dense_few_rows() rows and bfloat16 weights whose activations lie in memory as bfloat16 already (the launch that wrote them rounded them:
- * the same values as ntk_dense's rounding at the product's input):
- *   x16 : [x16_rows][ldx16] (16-byte aligned, ldx16 % 8 == 0), in the place of d->X (which may be NULL);
- *   y16 : NULL: F32 results to d->Y.  Else bfloat16 results, rows ldy16 apart (d->Y unused, no accumulate): d->glu_ff > 0: the gated unit of d (N == 2 * glu_ff), else d->act.
+/* The same product for more than ntk_dense_few_rows() rows over activations that lie in memory as the product takes them: bfloat16 beside bfloat16 weights (the launch that wrote
+ * them rounded them: the same values as ntk_dense's rounding at the product's input), F32 beside F32 ones:
+ *   x16 : [x16_rows][ldx16] (16-byte aligned rows), in the place of d->X (which may be NULL);
+ *   d->glu_ff > 0 : the gated unit of d (N == 2 * glu_ff, no accumulate) in this form, too;
+ *   y16 : NULL: F32 results to d->Y.  Else (bfloat16 weights) bfloat16 results, rows ldy16 apart (d->Y unused, no accumulate).
  * NTK_E_SHAPE where ntk_dense_direct_takes() says 0. */
 typedef struct ntk_direct_desc {
     const void* x16; int ldx16, x16_rows;

@@ -523,6 +523,13 @@ static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long r
                                        {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
     return plan_direct(forms, 7, 64, rows, groups, N, K, room);
 }
+// float32: K in chunks of 32; one form is ahead of larger and smaller tiles and other splits of the tile over waves everywhere (12 .. 200 rows, 900 in 32 groups): us, the form of gemm_tile.hip.h
+// before -> now: 150 x 14976 x 2048 114 -> 91 (101 TF/s of the 153 a large library product reaches), 150 x 2048 x 7488 58 -> 49, 150 x 6240 x 2048 51 -> 39, 12 x 2048 x 2048 11 -> 9
+template <int GLU>
+static void launch_direct_f32(const DirectArgs& d, int groups, long long room, hipStream_t s) {
+    static const DirectForm form[] = {{32, 64, 4, 0.38f, 0.27f, 4.0f}};
+    launch_direct<TileF32, 32, 64, 2, 2, 3, GLU, 4>(d, plan_direct(form, 1, 32, d.t.T, groups, d.t.N, d.t.K, room).splits, s);
+}
 template <int GLU>
 static void launch_direct_bf16(const DirectArgs& d, const TilePlan& p, hipStream_t s) {
     switch (p.form) {
@@ -553,18 +560,20 @@ int ntk_round_rows(void* y, int ldy, const float* x, int ldx, int T, int n, void
     return last_launch_status();
 }
 
-// whole chunks of 64 inputs, and rows that 32-bit offsets reach
+// whole chunks of 128 bytes, and rows that 32-bit offsets reach
 int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K) {
-    return wdtype == NTK_DT_BF16 && T > kGemvRows && N > 0 && K > 0 && K % 64 == 0 && (long long)N * K * 2 < 1LL << 32 && (long long)x16_rows * K * 2 < 1LL << 32;
+    const int es = wdtype == NTK_DT_BF16 ? 2 : 4;
+    return (wdtype == NTK_DT_BF16 || wdtype == NTK_DT_F32) && T > kGemvRows && N > 0 && K > 0 && K % (128 / es) == 0 && (long long)N * K * es < 1LL << 32 && (long long)x16_rows * K * es < 1LL << 32;
 }
 
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream) {
     if (!d || !e || !d->W || !e->x16 || (!e->y16 && !d->Y)) return NTK_E_NULL;
     if (!ntk_dense_direct_takes(d->wdtype, d->T, e->x16_rows, d->N, d->K)) return d->T == 0 ? NTK_OK : NTK_E_SHAPE;
-    const bool glu = d->glu_ff > 0;
-    if (e->ldx16 < d->K || e->ldx16 % 8 || d->wstride % 8 || (long long)e->x16_rows * e->ldx16 * 2 >= 1LL << 32) return NTK_E_SHAPE;
+    const bool glu = d->glu_ff > 0, bf = d->wdtype == NTK_DT_BF16;
+    const int es = bf ? 2 : 4;
+    if (e->ldx16 < d->K || e->ldx16 % (16 / es) || d->wstride % (16 / es) || (long long)e->x16_rows * e->ldx16 * es >= 1LL << 32 || (!bf && e->y16)) return NTK_E_SHAPE;
     if (((uintptr_t)e->x16 | (uintptr_t)d->W) & 15) return NTK_E_ALIGN;
-    if (e->y16 ? (e->ldy16 < (glu ? d->glu_ff : d->N) || d->accumulate) : (glu || d->ldy < d->N)) return NTK_E_SHAPE;
+    if (e->y16 ? (e->ldy16 < (glu ? d->glu_ff : d->N) || d->accumulate) : (d->ldy < (glu ? d->glu_ff : d->N) || (glu && d->accumulate))) return NTK_E_SHAPE;
     if ((glu && (d->N != 2 * d->glu_ff || d->act)) || d->norm_w || d->add_y || d->full_x) return NTK_E_SHAPE;
     if ((d->offsets && d->G <= 0) || (d->rows && d->row_div <= 0) || (!d->rows && e->x16_rows < d->T)) return NTK_E_SHAPE;
     if ((d->act != NTK_ACT_NONE && d->act != NTK_ACT_RELU2) || (d->act && d->accumulate)) return NTK_E_SHAPE;
@@ -573,14 +582,21 @@ int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* st
     TileArgs& t = a.t;
     t.Y = d->Y; t.ldy = d->ldy; t.W = d->W; t.wstride = d->wstride; t.offsets = d->offsets; t.G = G; t.rows = d->rows; t.row_div = d->rows ? d->row_div : 1;
     t.T = d->T; t.N = d->N; t.K = d->K; t.accumulate = d->accumulate; t.act = d->act; t.part = d->scratch;
-    a.X16 = e->x16; a.x_row = (uint32_t)e->ldx16 * 2; a.Y16 = (uint16_t*)e->y16; a.ldy16 = e->ldy16;
+    a.X16 = e->x16; a.x_row = (uint32_t)e->ldx16 * es; a.Y16 = (uint16_t*)e->y16; a.ldy16 = e->ldy16;
     // (no pieces for grouped rows: rows that belong to no group stay untouched)
-    const long long room = d->scratch && !((uintptr_t)d->scratch & 15) && !d->offsets && !e->y16 && d->T <= 65535 ? (long long)(d->scratch_bytes / sizeof(float)) : 0;
-    const TilePlan p = plan_direct_bf16(d->T, G, d->N, d->K, room);
+    const long long room = d->scratch && !((uintptr_t)d->scratch & 15) && !d->offsets && !e->y16 && !glu && d->T <= 65535 ? (long long)(d->scratch_bytes / sizeof(float)) : 0;
+    hipStream_t s = resolve_stream(stream);
     if (glu) {
-        a.glu_ff = d->glu_ff; a.up_at = (uint32_t)d->glu_ff * (uint32_t)d->K * 2; a.limit = d->glu_limit; a.alpha = d->glu_alpha; a.up_offset = d->glu_up_offset; a.cubic = d->glu_cubic;
-        launch_direct_bf16<kGluClipped>(a, p, resolve_stream(stream));
-    } else launch_direct_bf16<kGluNone>(a, p, resolve_stream(stream));
+        a.glu_ff = d->glu_ff; a.up_at = (uint32_t)d->glu_ff * (uint32_t)d->K * es; a.limit = d->glu_limit; a.alpha = d->glu_alpha; a.up_offset = d->glu_up_offset; a.cubic = d->glu_cubic;
+    }
+    if (!bf) {
+        if (glu) launch_direct_f32<kGluClipped>(a, G, room, s);
+        else launch_direct_f32<kGluNone>(a, G, room, s);
+        return last_launch_status();
+    }
+    const TilePlan p = plan_direct_bf16(d->T, G, d->N, d->K, room);
+    if (glu) launch_direct_bf16<kGluClipped>(a, p, s);
+    else launch_direct_bf16<kGluNone>(a, p, s);
     return last_launch_status();
 }
 
@@ -664,10 +680,14 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
         else if (p.form == 2) launch_tiles<TileBf16, 64, 64, 2, 2, 2, true>(t, p.splits, s);
         else launch_tiles<TileBf16, 32, 64, 2, 2, 2, true>(t, p.splits, s);
     } else {
-        static const TileForm forms[] = {{64, 64, 32, 0.78f, 0.70f}, {32, 64, 32, 0.52f, 0.36f}};
-        const TilePlan p = plan_tiles(forms, 2, d->T, G, d->N, d->K, room);
-        if (p.form == 0) launch_tiles<TileF32, 64, 64, 2, 2, 2, true>(t, p.splits, s);
-        else launch_tiles<TileF32, 32, 64, 2, 2, 2, true>(t, p.splits, s);
+        if (!d->rows && d->ldx % 4 == 0 && d->wstride % 4 == 0 && ntk_dense_direct_takes(d->wdtype, d->T, d->T, d->N, d->K) && (long long)d->T * d->ldx * 4 < 1LL << 32) {
+            DirectArgs a32{};
+            a32.t = t; a32.X16 = d->X; a32.x_row = (uint32_t)d->ldx * 4;
+            launch_direct_f32<kGluNone>(a32, G, room, s);
+            return last_launch_status();
+        }
+        static const TileForm form[] = {{32, 64, 32, 0.52f, 0.36f}};
+        launch_tiles<TileF32, 32, 64, 2, 2, 2, true>(t, plan_tiles(form, 1, d->T, G, d->N, d->K, room).splits, s);
     }
     return last_launch_status();
 }

@@ -1202,6 +1202,7 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
         return ntk_dense_direct(&o, &f, stream_);
     }
     d.full_x = full_x;
+    const bool direct = !ex.plain && wdtype_ == NTK_DT_F32 && ntk_dense_direct_takes(NTK_DT_F32, rows, rows / top, ex.in_rows(), W);      // gate and up meet in the first product's launch
     d.Y = gu; d.ldy = ex.in_rows(); d.X = h; d.ldx = W; d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype;
     d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top; d.T = rows; d.N = ex.in_rows(); d.K = W; d.accumulate = 0;
     if (ex.plain) {                       // the activation inside the product, whatever its form
@@ -1211,6 +1212,12 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
     } else if (rows <= ntk_dense_few_rows()) {   // decoding: the activation inside the product's launch
         d.Y = act; d.ldy = ex.ff; d.glu_ff = ex.ff; d.glu_limit = ex.limit; d.glu_alpha = glu_alpha; d.glu_up_offset = glu_up_offset;
         LS_TRY(first_product(d));
+        d.glu_ff = 0;
+    } else if (direct) {
+        const ntk_direct_desc e{h, W, rows / top, nullptr, 0};
+        d.Y = act; d.ldy = ex.ff; d.glu_ff = ex.ff; d.glu_limit = ex.limit; d.glu_alpha = glu_alpha; d.glu_up_offset = glu_up_offset;
+        d.full_x = 0;                     // (32 bits anyway)
+        LS_TRY(ntk_dense_direct(&d, &e, stream_));
         d.glu_ff = 0;
     } else {
         LS_TRY(product(d));
@@ -1370,7 +1377,7 @@ int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot,
 }
 
 // T rows of bfloat16 activations go through w as they lie
-bool LayerStackModel::rounded(const DenseW& w, int T) const { return h1_16_ && ntk_dense_direct_takes(w.dtype, T, T, (int)w.out_f, (int)w.in_f) != 0; }
+bool LayerStackModel::rounded(const DenseW& w, int T) const { return h1_16_ && w.dtype == NTK_DT_BF16 && ntk_dense_direct_takes(w.dtype, T, T, (int)w.out_f, (int)w.in_f) != 0; }
 
 // every product of the model: with room for the partial sums of a product whose inputs are cut into pieces
 int LayerStackModel::product(ntk_dense_desc& d) {

@@ -240,8 +240,8 @@ def round_rows(x: np.ndarray, n: Optional[int] = None) -> np.ndarray:
 
 def dense_direct(x: np.ndarray, w: np.ndarray, offsets=None, rows=None, row_div: int = 1, n_rows: Optional[int] = None, y0: Optional[np.ndarray] = None, out16: bool = False,
                  glu_limit: Optional[float] = None, glu_alpha: float = 1.702, glu_up_offset: float = 1.0, glu_cubic: float = 0.0, act: int = ACT_NONE, scratch_floats: int = 0,
-                 fill: float = 0.0):
-    """dense() over activations that are rounded to bfloat16 in a launch of their own; out16 or glu_limit: bfloat16 results (as float32), else float32 ones"""
+                 fill: float = 0.0, dtype: str = "bfloat16"):
+    """dense() over activations that are rounded to bfloat16 in a launch of their own (float32: taken as they are); out16: bfloat16 results (as float32), else float32 ones"""
     L = _bind()
     w = np.asarray(w)
     stacked = w.ndim == 3
@@ -249,9 +249,11 @@ def dense_direct(x: np.ndarray, w: np.ndarray, offsets=None, rows=None, row_div:
     T = int(n_rows if n_rows is not None else (len(rows) if rows is not None else x.shape[0]))
     glu = glu_limit is not None
     n_out = N // 2 if glu else N
-    xb, (wb, wdt) = _f(x), weight_buffer(w, "bfloat16")
-    x16 = DeviceBuffer.zeros(x.shape[0] * K * 2)
-    check(L.ntk_round_rows(x16.ptr, K, xb.ptr, x.shape[1], x.shape[0], K, None), "ntk_round_rows")
+    xb, (wb, wdt) = _f(x), weight_buffer(w, dtype)
+    bf = dtype == "bfloat16"
+    x16 = DeviceBuffer.zeros(x.shape[0] * K * 2) if bf else xb
+    if bf:
+        check(L.ntk_round_rows(x16.ptr, K, xb.ptr, x.shape[1], x.shape[0], K, None), "ntk_round_rows")
     yb = _f(y0) if y0 is not None else _f(np.full((max(T, 1), n_out), fill, np.float32))
     ob = _i(offsets) if offsets is not None else None
     rb = _i(rows) if rows is not None else None
@@ -263,9 +265,9 @@ def dense_direct(x: np.ndarray, w: np.ndarray, offsets=None, rows=None, row_div:
         d.scratch, d.scratch_bytes = sb.ptr, scratch_floats * 4
     if glu:
         d.glu_ff, d.glu_limit, d.glu_alpha, d.glu_up_offset, d.glu_cubic = n_out, glu_limit, glu_alpha, glu_up_offset, glu_cubic
-    e = DirectDesc(x16.ptr, K, x.shape[0], yb.ptr if glu or out16 else None, n_out)
+    e = DirectDesc(x16.ptr, K if bf else x.shape[1], x.shape[0], yb.ptr if out16 else None, n_out)
     check(L.ntk_dense_direct(C.byref(d), C.byref(e), None), "ntk_dense_direct")
-    if glu or out16:
+    if out16:
         return _bf16(yb.numpy(np.uint16, T * n_out).reshape(T, n_out))
     return yb.numpy(np.float32, T * n_out).reshape(T, n_out)
 

@@ -16,8 +16,8 @@ def _case(rng, T, N, K, G=0):
     return rng.standard_normal((T, K)).astype(np.float32), _round(rng.standard_normal((G, N, K) if G else (N, K)).astype(np.float32) / np.sqrt(K))
 
 
-def _close(got, x, w, out=None, bf=False, slack=1.0):
-    xd, wd = _round(x).astype(np.float64), w.astype(np.float64)
+def _close(got, x, w, out=None, bf=False, slack=1.0, f32=False):
+    xd, wd = (x if f32 else _round(x)).astype(np.float64), w.astype(np.float64)
     ref = xd @ wd.T
     bound = (x.shape[1] + 2) * U * (np.abs(xd) @ np.abs(wd).T)
     if out is not None:
@@ -55,7 +55,30 @@ def test_gated_units_inside_the_product(T, ff, K, limit, alpha, up, cubic):
         s = 1.0 / (1.0 + np.exp(-alpha * (g + cubic * g ** 3)))
         # both factors off by their product's bound (the gate's slope is below 1.2), and a few roundings of the unit itself
         return g * s * (u + up), 1.2 * b[:, :ff] * (np.abs(u + up) + b[:, ff:]) + np.abs(g) * b[:, ff:] + 16 * U * np.abs(g) * (np.abs(u) + 1.0)
-    _close(Lr.dense_direct(x, w, glu_limit=limit, glu_alpha=alpha, glu_up_offset=up, glu_cubic=cubic), x, w, unit, bf=True)
+    kw = dict(glu_limit=limit, glu_alpha=alpha, glu_up_offset=up, glu_cubic=cubic)
+    _close(Lr.dense_direct(x, w, out16=True, **kw), x, w, unit, bf=True)
+    _close(Lr.dense_direct(x, w, **kw), x, w, unit)
+    if T < 1000:
+        w32 = w + rng.standard_normal(w.shape).astype(np.float32) / 1000
+        _close(Lr.dense_direct(x, w32, dtype="float32", **kw), x, w32, unit, f32=True)
+
+
+@pytest.mark.parametrize("T,N,K,ld", [(9, 1, 32, 32), (31, 65, 64, 68), (33, 64, 96, 96), (150, 200, 2048, 2048), (65, 130, 1000, 1000), (200, 700, 416, 1000)])
+def test_float32_products(T, N, K, ld):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(T + N)
+    x, w = rng.standard_normal((T, ld)).astype(np.float32), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32)
+    if K % 32 == 0:
+        _close(Lr.dense_direct(x, w, dtype="float32"), x[:, :K], w, f32=True)
+    y0 = rng.standard_normal((T, N)).astype(np.float32)
+    _close(Lr.dense(x, w, "float32", scratch_floats=16 * T * N), x[:, :K], w, lambda r, b: (r, 2 * b), f32=True)
+    _close(Lr.dense(x, w, "float32", y0=y0), x[:, :K], w, lambda r, b: (r + y0, b + 2 * U * (np.abs(y0) + np.abs(r))), f32=True)
+    off = [0, T // 3, T // 3, T - 2]
+    ws = np.stack([w, w + 1, w * 2]).astype(np.float32)
+    got = Lr.dense(x, ws, "float32", offsets=off)
+    for g in range(3):
+        if off[g + 1] > off[g]:
+            _close(got[off[g]:off[g + 1]], x[off[g]:off[g + 1], :K], ws[g], f32=True)
 
 
 @pytest.mark.parametrize("counts", [[0, 1, 64, 65, 0, 130], [300, 0, 0, 3], [255, 256, 257, 1], [17] * 70])
