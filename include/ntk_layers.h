@@ -211,6 +211,12 @@ size_t ntk_latent_attention_scratch(int T, int H, int vdim_or_rank, int nkeys);
 int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
                          int kv_rank, int rot_dim, int H, int dn, int dv, int shared, int pos0, int T, int key0, int window, float scale, float* scratch,
                          void* stream);
+/* ... with room for the visible keys and values as halves (ntk_prompt_attention_image_bytes() for the positions that a portion sees; 16-byte aligned; NULL: none): the expanded form of a
+ * prompt's portion then multiplies on the half-precision matrix instructions, every 32-bit value as two halves */
+int ntk_latent_attention_ex(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
+                         int kv_rank, int rot_dim, int H, int dn, int dv, int shared, int pos0, int T, int key0, int window, float scale, float* scratch,
+                         void* image, size_t image_bytes, void* stream);
+size_t ntk_prompt_attention_image_bytes(int positions, int kv_heads, int key_entries, int value_entries);     /* 0: sizes without such a form */
 /* fold the unrotated query part through the key up-projection: qf[t][h][0..R) = sum_d q[t][h][d] * W_uk[h*dn + d][0..R), and copy the rotated part behind it
  * (qf [T][H][R+dr]; q rows ldq floats apart); W_uk NTK_DT_BF16 / F32 [H*dn][R] */
 /* ... and, beside it in the same launch, the latents of these tokens into the cache rows: kv [T][ldkv] raw latents -> kv / rms * norm_w (ntk_latent_prepare without a
@@ -296,6 +302,8 @@ typedef struct ntk_window_attention_desc {
 #define NTK_MASK_CHUNKS 1
 size_t ntk_window_attention_scratch(int T, int H, int maps, int dv, int nkeys);
 int ntk_window_attention(const ntk_window_attention_desc* d, void* stream);
+/* ... with room for the visible keys and values as halves (see ntk_latent_attention_ex) */
+int ntk_window_attention_ex(const ntk_window_attention_desc* d, void* image, size_t image_bytes, void* stream);
 
 /* ---- lightning_attention.hip -------------------------------------------------------------------------------------------------------
  * Linear attention with a per-head decay: S_t = decay_h S_(t-1) + k_t v_t^T (S [dn][dv] per head, F32), o_t = S_t^T q_t, with q, k, v = act(raw)

@@ -924,6 +924,11 @@ int LayerStackModel::alloc_buffers() {
     const int W = info_.width;
     chunk_ = std::min(opt_.max_context, 1024);
     size_t sc = 0, wsc = 0, lsc = 0, rsc = 0;
+    // what a portion's attention sees at most, as halves: the portion and a window ahead of it (and the positions that stay visible), or everything
+    auto seen = [&](int window, int keep, int kv_heads, int dk, int dv) {
+        const long long n = window > 0 ? std::min<long long>((long long)window + chunk_ + keep + 64, opt_.max_context) : opt_.max_context;
+        image_bytes_ = std::max(image_bytes_, ntk_prompt_attention_image_bytes((int)n, kv_heads, dk, dv));
+    };
     for (const auto& L : layers_) {
         if (L.mixer == kMixLatent) {
             const LatentMixer& m = L.mix;
@@ -936,6 +941,7 @@ int LayerStackModel::alloc_buffers() {
             max_hr_ = std::max(max_hr_, m.heads * m.kv_rank);
             if (m.kv_rank > 512 || m.vdim > 512) return fail(NTK_E_SHAPE, "kv_rank and vdim up to 512 are supported");
             sc = std::max(sc, ntk_latent_attention_scratch(kSharedRows, m.heads, m.kv_rank, opt_.max_context));
+            seen(m.window, 0, m.heads, m.qd(), m.vdim);
         } else if (L.mixer == kMixGatedDelta) {
             const GatedDeltaMixer& m = L.gdl;
             max_in_ = std::max<int>(max_in_, (int)m.in.out_f);
@@ -952,6 +958,7 @@ int LayerStackModel::alloc_buffers() {
             if (m.vdim > 512) return fail(NTK_E_SHAPE, "vdim up to 512 is supported");
             if (m.v_mix) max_gv_ = std::max(max_gv_, m.kv_heads * m.vdim);
             wsc = std::max(wsc, ntk_window_attention_scratch(chunk_, m.heads, m.maps, m.vdim, opt_.max_context));
+            if (m.maps == 1) seen(m.window, m.keep_first, m.kv_heads, m.dim, m.vdim);
         } else if (L.mixer == kMixLightning) {
             const LightningMixer& m = L.lin;
             max_in_ = std::max<int>(max_in_, (int)m.in.out_f);
@@ -970,6 +977,7 @@ int LayerStackModel::alloc_buffers() {
             max_rec_ = std::max(max_rec_, m.right.heads * m.right.dim);
             rsc = std::max(rsc, ntk_gated_recurrence_scratch(chunk_, m.right.heads, m.right.dim, m.right.dim, 1));
             wsc = std::max(wsc, ntk_window_attention_scratch(chunk_, m.left.heads, 1, m.left.vdim, opt_.max_context));
+            seen(0, 0, m.left.kv_heads, m.left.dim, m.left.vdim);
         }
         if (form_.gated && L.has_mlp) max_gu2_ = std::max<int>(max_gu2_, (int)L.gff.in.out_f), max_ffn_ = std::max(max_ffn_, L.gff.ff);
         if (L.mlp_kind == kMlpMoe) {
@@ -1004,6 +1012,7 @@ int LayerStackModel::alloc_buffers() {
     // four pieces of a whole pass's rows, and no less than sixteen of a short one's
     pscratch_bytes_ = std::max<size_t>(4 * C * W, (size_t)1 << 22) * sizeof(float);
     ok = ok && fl(&pscratch_, pscratch_bytes_ / sizeof(float));
+    if (image_bytes_ && !(image_ = dev_alloc(image_bytes_))) image_bytes_ = 0;      // (a long context may not leave the room: the attention has a form without)
     if (wdtype_ == NTK_DT_BF16) ok = ok && (h1_16_ = dev_alloc(C * W * 2)) && (h2_16_ = dev_alloc(C * W * 2));
     if (max_mid_ > 0) ok = ok && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_);
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
@@ -1098,8 +1107,8 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
             LS_TRY(linear(kx_, H * m.dim, lat, row, m.uk.ptr, m.uk.dtype, nkeys, H * m.dim, m.kv_rank, 0));
             LS_TRY(linear(vx_, hv, lat, row, m.uv.ptr, m.uv.dtype, nkeys, hv, m.kv_rank, 0));
         }
-        LS_TRY(ntk_latent_attention(att_, hv, q, ldq, kx_, H * m.dim, vx_, hv, cache, row, m.kv_rank, m.rot_dim, H, m.dim, m.vdim, 0, pos0, T, key0, m.window, m.scale,
-                                    nullptr, stream_));
+        LS_TRY(ntk_latent_attention_ex(att_, hv, q, ldq, kx_, H * m.dim, vx_, hv, cache, row, m.kv_rank, m.rot_dim, H, m.dim, m.vdim, 0, pos0, T, key0, m.window, m.scale,
+                                       nullptr, image_, image_bytes_, stream_));
         if (m.head_gate) LS_TRY(ntk_head_gate(att_, hv, a_ + m.g_off, na, T, H, m.vdim, stream_));
         else LS_TRY(ntk_sigmoid_gate(att_, hv, a_ + m.g_off, na, T, hv, stream_));
     }
@@ -1140,7 +1149,7 @@ int LayerStackModel::window_heads(const WindowMixer& m, float* cache, float* out
     d.mask_mode = m.mask_mode; d.softcap = m.softcap; d.sink = m.sink ? 1 : 0; d.keep_first = m.keep_first; d.sinks = m.sinks;
     d.slopes = m.slopes;
     if (m.gated) { d.gate = a_ + m.g_off; d.ldg = na; d.head_gate = m.head_gate ? 1 : 0; }     // the gate rides in the launch that writes the heads' results
-    return ntk_window_attention(&d, stream_);
+    return ntk_window_attention_ex(&d, image_, image_bytes_, stream_);
 }
 
 // A layer of the dense parallel form: both sublayers read the stream as it is (decoding: each norm inside its product's launch, the gated unit in the epilogue
@@ -1456,7 +1465,7 @@ int LayerStackModel::run_parallel(const StackLayer& L, float* cache, float* stat
     d.out = att_; d.ldo = no; d.q = a_ + a.q_off; d.ldq = na; d.cache = cache; d.row = a.row(); d.H = a.heads; d.G = a.kv_heads; d.maps = 1; d.dn = a.dim; d.dv = a.vdim;
     d.pos0 = pos0; d.T = T; d.window = 0; d.scale = a.scale; d.out_scale = 1.0f; d.eps = eps_; d.scratch = wscratch_;
     d.rel = a.rel; d.bucket_of = a.bucket_of; d.n_dist = opt_.max_context;
-    LS_TRY(ntk_window_attention(&d, stream_));
+    LS_TRY(ntk_window_attention_ex(&d, image_, image_bytes_, stream_));
     LS_TRY(ntk_sigmoid_gate_scaled(att_, no, a_ + a.g_off, na, nullptr, m.left_scale, T, hv, stream_));
     // ---- right
     LS_TRY(ntk_tanh_rows(a_ + r.w1_off, na, T, r.rank, stream_));

@@ -9,7 +9,7 @@
 // Expanded: a workgroup owns 16 tokens of one head and walks the visible keys in chunks of 64 -- lane = key for the scores (key slabs of 64 entries in
 // LDS), online softmax per row in F32, lane = value column for the weighted sum.  Shared: a workgroup owns 16 (token, head) rows and whole tiles of 32
 // cache rows; the tiles go round up to 128 workgroups and a second launch merges their (max, sum, vector) states.
-#include "attention_tile.hip.h"
+#include "attention_half.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -510,9 +510,19 @@ size_t ntk_latent_attention_scratch(int T, int H, int vdim_or_rank, int nkeys) {
     return (size_t)T * H * shared_splits(nkeys) * (2 + vdim_or_rank);
 }
 
+size_t ntk_prompt_attention_image_bytes(int positions, int kv_heads, int key_entries, int value_entries) {
+    return positions > 0 && kv_heads > 0 && key_entries > 0 && value_entries > 0 ? half_attention_bytes((positions - 1) / 32 + 3, kv_heads, key_entries, value_entries) : 0;
+}
+
 int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
                          int kv_rank, int rot_dim, int H, int dn, int dv, int shared, int pos0, int T, int key0, int window, float scale, float* scratch,
                          void* stream) {
+    return ntk_latent_attention_ex(out, ldo, q, ldq, K, ldk, V, ldv, cache, row, kv_rank, rot_dim, H, dn, dv, shared, pos0, T, key0, window, scale, scratch, nullptr, 0, stream);
+}
+
+int ntk_latent_attention_ex(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
+                            int kv_rank, int rot_dim, int H, int dn, int dv, int shared, int pos0, int T, int key0, int window, float scale, float* scratch,
+                            void* image, size_t image_bytes, void* stream) {
     if (!out || !q || !cache) return NTK_E_NULL;
     if (!shared && (!K || !V)) return NTK_E_NULL;
     if (T < 0 || H <= 0 || kv_rank <= 0 || rot_dim < 0 || pos0 < 0 || key0 < 0 || row < kv_rank + rot_dim) return NTK_E_SHAPE;
@@ -554,7 +564,7 @@ int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const flo
         TileAttnArgs t{};
         t.out = out; t.ldo = ldo; t.q = q; t.ldq = ldq; t.kA = a.kA; t.ldA = a.ldA; t.nA = a.nA; t.hA = a.hA; t.kB = a.kB; t.ldB = a.ldB; t.nB = a.nB;
         t.v = a.v; t.ldV = a.ldV; t.nV = a.nV; t.hV = a.hV; t.key0 = key0; t.H = H; t.G = H; t.pos0 = pos0; t.T = T; t.window = window; t.scale = scale; t.out_scale = 1.0f;
-        launch_attention_tile(t, s);
+        if (!launch_attention_half(t, image, image_bytes, s)) launch_attention_tile(t, s);
         return last_launch_status();
     }
     const int DKP = (a.nA + a.nB + 3) & ~3;

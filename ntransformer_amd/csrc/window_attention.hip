@@ -12,7 +12,7 @@
 // in LDS), online softmax per row and map, lane = value column for the weighted sums (the value slab is loaded once for both maps).  When few rows
 // face many keys (decoding), the chunks go round `splits` workgroups and a second launch merges their (max, sum, vector) states.
 #include <algorithm>
-#include "attention_tile.hip.h"
+#include "attention_half.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -473,7 +473,9 @@ size_t ntk_window_attention_scratch(int T, int H, int maps, int dv, int nkeys) {
     return nkeys > 0 ? states * maps * (2 + dv) : 0;
 }
 
-int ntk_window_attention(const ntk_window_attention_desc* d, void* stream) {
+int ntk_window_attention(const ntk_window_attention_desc* d, void* stream) { return ntk_window_attention_ex(d, nullptr, 0, stream); }
+
+int ntk_window_attention_ex(const ntk_window_attention_desc* d, void* image, size_t image_bytes, void* stream) {
     if (!d || !d->out || !d->q || !d->cache) return NTK_E_NULL;
     if (d->T < 0 || d->H <= 0 || d->G <= 0 || d->H % d->G || d->dn <= 0 || d->dv <= 0 || d->pos0 < 0) return NTK_E_SHAPE;
     if (d->maps != 1 && d->maps != 2) return NTK_E_SHAPE;
@@ -501,7 +503,7 @@ int ntk_window_attention(const ntk_window_attention_desc* d, void* stream) {
         t.v = a.cache + (long long)a.G * a.dn; t.ldV = a.row; t.nV = a.dv; t.hV = a.dv; t.H = a.H; t.G = a.G; t.pos0 = a.pos0; t.T = a.T;
         t.window = a.window; t.chunks = a.chunks; t.keep = a.keep; t.scale = a.scale; t.softcap = a.softcap; t.out_scale = a.out_scale; t.sink = a.sink; t.sinks = a.sinks;
         t.slopes = a.slopes; t.rel = a.rel; t.bucket_of = a.bucket_of; t.n_dist = a.n_dist; t.gate = a.gate; t.ldg = a.ldg; t.head_gate = a.head_gate;
-        launch_attention_tile(t, s);
+        if (!launch_attention_half(t, image, image_bytes, s)) launch_attention_tile(t, s);
         return last_launch_status();
     }
     const int DNP = (d->dn + 3) & ~3;

@@ -111,6 +111,9 @@ def _bind():
     L.ntk_latent_attention_scratch.argtypes = [i, i, i, i]
     L.ntk_latent_attention_scratch.restype = C.c_size_t
     L.ntk_latent_attention.argtypes = [vp, i, vp, i, vp, i, vp, i, vp, i, i, i, i, i, i, i, i, i, i, i, f, vp, vp]
+    L.ntk_latent_attention_ex.argtypes = L.ntk_latent_attention.argtypes[:-1] + [vp, C.c_size_t, vp]
+    L.ntk_prompt_attention_image_bytes.argtypes, L.ntk_prompt_attention_image_bytes.restype = [i] * 4, C.c_size_t
+    L.ntk_window_attention_ex.argtypes = [C.POINTER(WindowAttentionDesc), vp, C.c_size_t, vp]
     L.ntk_latent_fold_query.argtypes = [vp, vp, i, vp, i, i, i, i, i, i, vp]
     L.ntk_latent_unfold_value.argtypes = [vp, i, vp, vp, i, vp, i, i, i, i, i, vp]
     L.ntk_moe_route.argtypes = [vp, vp, vp, vp, i, vp, vp, i, i, i, i, vp]
@@ -311,8 +314,8 @@ def latent_prepare(kv: np.ndarray, norm_w: np.ndarray, eps: float, kv_rank: int,
 
 
 def latent_attention(q: np.ndarray, cache: np.ndarray, kv_rank: int, rot_dim: int, heads: int, pos0: int, window: int, scale: float,
-                     K: Optional[np.ndarray] = None, V: Optional[np.ndarray] = None, key0: int = 0) -> np.ndarray:
-    """expanded form when K [nkeys, H * dn] and V [nkeys, H * dv] are given (q [T, H * (dn + dr)]), else the shared form (q [T, H * (R + dr)])"""
+                     K: Optional[np.ndarray] = None, V: Optional[np.ndarray] = None, key0: int = 0, halves: bool = False) -> np.ndarray:
+    """halves: with room for the keys and values as halves; expanded form when K [nkeys, H * dn] and V [nkeys, H * dv] are given (q [T, H * (dn + dr)]), else the shared form (q [T, H * (R + dr)])"""
     L = _bind()
     T, row = q.shape[0], kv_rank + rot_dim
     qb, cb = _f(q), _f(cache)
@@ -320,8 +323,10 @@ def latent_attention(q: np.ndarray, cache: np.ndarray, kv_rank: int, rot_dim: in
         dn, dv = K.shape[1] // heads, V.shape[1] // heads
         kb, vb = _f(K), _f(V)
         out = DeviceBuffer.zeros(T * heads * dv * 4)
-        check(L.ntk_latent_attention(out.ptr, heads * dv, qb.ptr, q.shape[1], kb.ptr, K.shape[1], vb.ptr, V.shape[1], cb.ptr, row, kv_rank, rot_dim, heads, dn, dv, 0,
-                                     pos0, T, key0, window, scale, None, None), "ntk_latent_attention")
+        room = int(L.ntk_prompt_attention_image_bytes(pos0 + T, heads, dn + rot_dim, dv)) if halves else 0
+        image = DeviceBuffer(room) if room else None
+        check(L.ntk_latent_attention_ex(out.ptr, heads * dv, qb.ptr, q.shape[1], kb.ptr, K.shape[1], vb.ptr, V.shape[1], cb.ptr, row, kv_rank, rot_dim, heads, dn, dv, 0,
+                                        pos0, T, key0, window, scale, None, image.ptr if image else None, room, None), "ntk_latent_attention")
         return out.numpy(np.float32, T * heads * dv).reshape(T, heads * dv)
     nkeys = pos0 + T
     sc = DeviceBuffer.zeros(max(int(L.ntk_latent_attention_scratch(T, heads, kv_rank, nkeys)), 1) * 4)
@@ -486,8 +491,8 @@ def window_prepare_biased(q, k, v, H: int, G: int, dn: int, dv: int, pos0: int, 
 def window_attention(q: np.ndarray, cache: np.ndarray, H: int, G: int, maps: int, dn: int, dv: int, pos0: int, window: int, scale: float, lam: float = 0.0,
                      sub_norm: bool = False, eps: float = 1e-6, out_scale: float = 1.0, split: bool = True, rel: Optional[np.ndarray] = None,
                      bucket_of: Optional[np.ndarray] = None, chunks: bool = False, softcap: float = 0.0, sink: bool = False, gate: Optional[np.ndarray] = None,
-                     keep_first: int = 0, sinks: Optional[np.ndarray] = None, head_gate: bool = False, slopes: Optional[np.ndarray] = None) -> np.ndarray:
-    """q [T, H * maps * dn] (rotated), cache rows [G][maps][dn] keys | [G][dv] values; split: long key ranges of few rows may be cut into merged parts;
+                     keep_first: int = 0, sinks: Optional[np.ndarray] = None, head_gate: bool = False, slopes: Optional[np.ndarray] = None, halves: bool = False) -> np.ndarray:
+    """halves: with room for the keys and values as halves; q [T, H * maps * dn] (rotated), cache rows [G][maps][dn] keys | [G][dv] values; split: long key ranges of few rows may be cut into merged parts;
     rel [buckets, H] with bucket_of [distances]: a bias by distance on the scaled score; keep_first: positions that stay visible beside the window;
     sinks [H]: the sink's score per head; gate [T, H * dv], or [T, H] with head_gate; slopes [H]: slopes[h] * distance comes off the scaled score"""
     L = _bind()
@@ -511,7 +516,9 @@ def window_attention(q: np.ndarray, cache: np.ndarray, H: int, G: int, maps: int
     if gate is not None:        # a sigmoid gate on the result
         gb = _f(gate)
         d.gate, d.ldg, d.head_gate = gb.ptr, gate.shape[1], int(head_gate)
-    check(L.ntk_window_attention(C.byref(d), None), "ntk_window_attention")
+    room = int(L.ntk_prompt_attention_image_bytes(pos0 + T, G, dn, dv)) if halves else 0
+    image = DeviceBuffer(room) if room else None
+    check(L.ntk_window_attention_ex(C.byref(d), image.ptr if image else None, room, None), "ntk_window_attention")
     return out.numpy(np.float32, T * H * dv).reshape(T, H * dv)
 
 
