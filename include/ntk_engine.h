@@ -59,6 +59,8 @@ int ntk_rp_dequant(float* out, const void* rp, int rows, int in_features, int dt
 /* the raw GGUF blocks [rows][in] back from the repacked form, byte for byte (the engine keeps ONE resident copy of a K-quant matrix and unpacks into
  * a scratch in front of the launches that read raw blocks); raw: 4-byte aligned (Q6_K: 2); stream ordered */
 int ntk_rp_unpack(void* raw, const void* rp, int rows, int in_features, int dtype, void* stream);
+/* y[0..rows) = W . x over a repacked matrix with F32 products and sums (in_features <= 32768; x 16-byte aligned): one row of a prompt through its head */
+int ntk_gemv_rp_f32(float* y, const void* rp, const float* x, int rows, int in_features, int dtype, void* stream);
 int ntk_gemv_rp(float* y, const void* rp, const float* x, int out_features, int in_features, int weight_dtype, void* stream);
 int ntk_gemv_rp_fused(const ntk_gemv_seg* segs, int nseg, const float* x, int in_features, const float* norm_w, float eps,
                       const float* resid, int silu_pair, void* stream);

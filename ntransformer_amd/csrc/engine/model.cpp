@@ -609,7 +609,11 @@ float* Model::forward(const int* tokens, int T, int start_pos) {
     auto ok = [&](int st) { if (st != NTK_OK && rc == NTK_OK) rc = st; };
     float* last = hidden_ + (size_t)(T - 1) * H;
     ok(ntk_rmsnorm(last, last, (const float*)output_norm_.ptr, 1, H, cfg_.norm_eps, s));   // in place, :658-659
-    {
+    // (a repacked head is read as it lies, whether its GGUF blocks are resident or not: the same bits either way)
+    int head = NTK_E_DTYPE;
+    if (output_.rp) head = ntk_gemv_rp_f32(logits_, output_.rp, last, (int)output_.out_f, (int)output_.in_f, output_.dtype, s);
+    if (head != NTK_E_DTYPE && head != NTK_E_SHAPE && head != NTK_E_ALIGN) ok(head);
+    else {
         raw_begin();
         const int st = ntk_gemv(logits_, raw_of(output_), last, (int)output_.out_f, (int)output_.in_f, output_.dtype, s);
         if (st == NTK_E_DTYPE) fprintf(stderr, "Unsupported dtype for GEMV: %s\n", dtype_name(output_.dtype));   // gemm.cu:801-803

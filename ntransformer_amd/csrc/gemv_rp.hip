@@ -307,6 +307,106 @@ constexpr int RP_MAXQ = 8;     // super-blocks of x one wave converts in the pro
 #endif
 constexpr int RP_DEPTH = NTK_RP_DEPTH;    // items in flight per wave (tuning builds: -DNTK_RP_DEPTH=n)
 
+// ------------------------------------------------------------------------------------------------------------------
+// One row of F32 activations through a repacked matrix with F32 products (the head behind a prompt): every nibble widened, multiplied in 32 bits and summed
+// in F32, the -32 offset and the minima through sums of x over 16 columns.  The matrix used to be unpacked in front of the raw-block GEMV: a 128256 x 4096 Q6_K
+// head cost 209 us of unpacking and 81 us of product per prompt, 67 us so (6.4 TB/s; the decode GEMV's activations of one exponent per super-block are less precise where channels tower
+// over the others).  A wave owns a tile of 16 rows, lane (kg, i) the columns 16 kg .. of every 64 of row i, with the next super-block's item under way; x lies in LDS.  Bound by
+// the stream of items.
+// ------------------------------------------------------------------------------------------------------------------
+template <int DT> struct RpF32Item {
+    u4 n[2], rec;
+    uint32_t h[2][2], dd;
+    __device__ __forceinline__ void load(const uint8_t* p1, const uint8_t* p2, int kg, int i) {
+        using F = Rp<DT>;
+        const int l = 16 * kg + i;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            n[s] = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p1 + s * F::S1 + 16 * l));
+            if constexpr (DT == NTK_DT_Q5_K) h[s][0] = *reinterpret_cast<const uint32_t*>(p1 + s * F::S1 + 1024 + 4 * l);
+            if constexpr (DT == NTK_DT_Q6_K) {
+                h[s][0] = *reinterpret_cast<const uint32_t*>(p1 + s * F::S1 + 1024 + 8 * l);
+                h[s][1] = *reinterpret_cast<const uint32_t*>(p1 + s * F::S1 + 1024 + 8 * l + 4);
+            }
+        }
+        rec = *reinterpret_cast<const u4*>(p2 + 16 * i);
+        if constexpr (DT == NTK_DT_Q6_K) dd = *reinterpret_cast<const uint16_t*>(p2 + 256 + 2 * i);
+        else dd = *reinterpret_cast<const uint32_t*>(p2 + 256 + 4 * i);
+    }
+};
+template <int DT>
+__global__ __launch_bounds__(512) void rp_gemv_f32_kernel(float* __restrict__ y, const uint8_t* __restrict__ rp, const float* __restrict__ x, int rows, int in, int nsb, int tiles, size_t p2_off) {
+    using F = Rp<DT>;
+    extern __shared__ __attribute__((aligned(16))) float xs[];              // x, then its sums over 16 columns
+    float* sx = xs + in;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 15, kg = lane >> 4;
+    const int first = blockIdx.x * 8 + wave, stride = gridDim.x * 8;
+    RpF32Item<DT> cur, next;
+    auto at = [&](int tile, int sb, RpF32Item<DT>& it) {
+        const size_t item = (size_t)tile * nsb + sb;
+        it.load(rp + item * (2 * F::S1), rp + p2_off + item * F::S2, kg, i);
+    };
+    if (first < tiles) at(first, 0, cur);
+    for (int k = 4 * tid; k < in; k += 4 * 512) *reinterpret_cast<float4*>(xs + k) = *reinterpret_cast<const float4*>(x + k);
+    __syncthreads();
+    for (int k = tid; k < in / 16; k += 512) {
+        float t[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) t[v] = (xs[16 * k + 4 * v] + xs[16 * k + 4 * v + 1]) + (xs[16 * k + 4 * v + 2] + xs[16 * k + 4 * v + 3]);
+        sx[k] = (t[0] + t[1]) + (t[2] + t[3]);
+    }
+    __syncthreads();
+    for (int tile = first; tile < tiles; tile += stride) {
+        float acc = 0.0f, rest = 0.0f;                        // the sum over super-blocks and what its roundings left (with plain sums 2.0e-7 of the result, 1.4e-7 from raw blocks)
+        auto add = [&](float v) {
+            const float t = acc + v, b = t - acc;
+            rest += (acc - (t - b)) + (v - b);
+            acc = t;
+        };
+        for (int sb = 0; sb < nsb; ++sb) {
+            const bool more = sb + 1 < nsb, again = tile + stride < tiles;
+            if (more) at(tile, sb + 1, next);
+            else if (again) at(tile + stride, 0, next);
+            const uint32_t scl[4] = {cur.rec.x, cur.rec.y, cur.rec.z, cur.rec.w};
+            float part[4], low[4];
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int col = 256 * sb + 128 * s + 64 * h + 16 * kg;
+                    const uint32_t w4[4] = {cur.n[s].x, cur.n[s].y, cur.n[s].z, cur.n[s].w};
+                    float four[4];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        uint32_t q = (h ? w4[v] >> 4 : w4[v]) & 0x0F0F0F0Fu;
+                        if constexpr (DT == NTK_DT_Q5_K) q |= ((cur.h[s][0] >> (4 * h + v)) & 0x01010101u) << 4;
+                        if constexpr (DT == NTK_DT_Q6_K) q |= ((cur.h[s][h] >> (2 * v)) & 0x03030303u) << 4;
+                        const float4 xv = *reinterpret_cast<const float4*>(xs + col + 4 * v);
+                        four[v] = fmaf(ub2f(q, 3), xv.w, fmaf(ub2f(q, 2), xv.z, fmaf(ub2f(q, 1), xv.y, ub2f(q, 0) * xv.x)));
+                    }
+                    const float dot = (four[0] + four[1]) + (four[2] + four[3]), sum = sx[col >> 4];
+                    if constexpr (DT == NTK_DT_Q6_K) {
+                        const uint32_t w = scl[2 * s + h] >> (8 * kg);                        // scale (8 s + 4 h + kg)
+                        part[2 * s + h] = (float)(int)(int8_t)(w & 0xFFu) * fmaf(-32.0f, sum, dot);
+                    } else {
+                        const uint32_t sh = 8 * (2 * h + (kg >> 1));                          // sub-block 4 s + 2 h + (kg >> 1)
+                        part[2 * s + h] = (float)((scl[s] >> sh) & 0xFFu) * dot;
+                        low[2 * s + h] = (float)((scl[2 + s] >> sh) & 0xFFu) * sum;
+                    }
+                }
+            const float d = h2f((uint16_t)(cur.dd & 0xFFFFu));
+            float t = d * ((part[0] + part[1]) + (part[2] + part[3]));
+            if constexpr (DT != NTK_DT_Q6_K) t = fmaf(-h2f((uint16_t)(cur.dd >> 16)), (low[0] + low[1]) + (low[2] + low[3]), t);
+            add(t);
+            cur = next;
+        }
+        acc += rest;
+        acc += __shfl_xor(acc, 16, 64);
+        acc += __shfl_xor(acc, 32, 64);
+        if (kg == 0 && 16 * tile + i < rows) y[16 * tile + i] = acc;
+    }
+}
+
 struct RpSeg {
     const uint8_t* rp;   // repacked tensor (P1, then P2 at p2_off)
     float* y;
@@ -883,6 +983,25 @@ int ntk_rp_pack(void* dst, const void* raw, int rows, int in_features, int dtype
     if (dtype == NTK_DT_Q4_K) hipLaunchKernelGGL(ntk::rp_pack_kernel<NTK_DT_Q4_K>, g, b, 0, st, d, r, rows, nsb, p2);
     else if (dtype == NTK_DT_Q5_K) hipLaunchKernelGGL(ntk::rp_pack_kernel<NTK_DT_Q5_K>, g, b, 0, st, d, r, rows, nsb, p2);
     else hipLaunchKernelGGL(ntk::rp_pack_kernel<NTK_DT_Q6_K>, g, b, 0, st, d, r, rows, nsb, p2);
+    return ntk::last_launch_status();
+}
+
+int ntk_gemv_rp_f32(float* y, const void* rp, const float* x, int rows, int in_features, int dtype, void* stream) {
+    if (!y || !rp || !x) return NTK_E_NULL;
+    if (!ntk::rp_supported(dtype)) return NTK_E_DTYPE;
+    if (rows <= 0 || in_features <= 0 || in_features % 256 != 0 || in_features > 32768) return NTK_E_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(rp) | reinterpret_cast<uintptr_t>(x)) & 15) return NTK_E_ALIGN;
+    const int tiles = (rows + 15) / 16, nsb = in_features / 256;
+    const size_t p2 = (size_t)tiles * nsb * 2 * ntk::rp_s1(dtype), lds = (size_t)in_features * 4 + in_features / 4;
+    hipStream_t st = ntk::resolve_stream(stream);
+    // two workgroups a CU where their x fits twice, rounds of whole tiles a wave
+    const int most = lds > 72 * 1024 ? 256 : 512, rounds = (tiles + 8 * most - 1) / (8 * most), grid = (tiles + 8 * rounds - 1) / (8 * rounds);
+    const void* fn = dtype == NTK_DT_Q4_K ? (const void*)ntk::rp_gemv_f32_kernel<NTK_DT_Q4_K> : dtype == NTK_DT_Q5_K ? (const void*)ntk::rp_gemv_f32_kernel<NTK_DT_Q5_K> : (const void*)ntk::rp_gemv_f32_kernel<NTK_DT_Q6_K>;
+    if (lds > 64 * 1024) NTK_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    const uint8_t* r = static_cast<const uint8_t*>(rp);
+    if (dtype == NTK_DT_Q4_K) hipLaunchKernelGGL(ntk::rp_gemv_f32_kernel<NTK_DT_Q4_K>, dim3(grid), dim3(512), lds, st, y, r, x, rows, in_features, nsb, tiles, p2);
+    else if (dtype == NTK_DT_Q5_K) hipLaunchKernelGGL(ntk::rp_gemv_f32_kernel<NTK_DT_Q5_K>, dim3(grid), dim3(512), lds, st, y, r, x, rows, in_features, nsb, tiles, p2);
+    else hipLaunchKernelGGL(ntk::rp_gemv_f32_kernel<NTK_DT_Q6_K>, dim3(grid), dim3(512), lds, st, y, r, x, rows, in_features, nsb, tiles, p2);
     return ntk::last_launch_status();
 }
 
