@@ -23,6 +23,10 @@ extern "C" {
  * place, the rotated k and v converted to F16 (RNE) into the caches at start_pos; k and v are only read.  Identical q and cache rows.  head_dim <= 256. */
 int ntk_rope_kv_store(float* q, const float* k, const float* v, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim,
                       float theta_base, float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream);
+/* ... with q, k and v as the partial sums of their projections (sums[0 .. 2]: [splits[i]][seq_len][row], ntk_gemm_partials; splits 1: the projection itself, sums[0] may be q):
+ * the sums in split order, then the same; the rotated q goes to q, k and v are not stored outside the caches */
+int ntk_reduce_rope_kv_store(float* q, const float* const* sums, const int* splits, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim, float theta_base,
+                             float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream);
 /* ---------------------------------------------------------------------------------------------
  * Engine-level fused operators (no reference counterpart; they compute exactly what the listed
  * sequence of reference launchers computes, in fewer launches, with device-resident positions so a

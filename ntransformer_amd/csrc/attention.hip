@@ -764,6 +764,75 @@ __global__ __launch_bounds__(256) void rope_kv_store_rows_kernel(float* __restri
         for (int e = first; e < per_pos; e += stride) vc[(size_t)cp * per_pos + e] = f2h(v[(size_t)sp * per_pos + e]);
 }
 
+// ... and the same from the projections' partial sums (ntk_gemm_partials): the splits are added here, in order, in the place of a launch that writes their sums
+// for this one to read back.  A short prompt takes a workgroup per 256 pairs of a token, everything requested ahead of the angles; a long one a workgroup per token with one
+// table of them.  16 tokens of the 8B shapes: 4.7 + 4.6 us as two launches, 4.0 as one; 1003 tokens 12.1 + 11.8 us, 14 as one.
+struct RopeSource { const float* p; int n; size_t plane; };
+template <int N>
+__device__ __forceinline__ void rope_sums(const RopeSource& s, const size_t (&at)[N], float (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = s.p[at[i]];
+    for (int sp = 1; sp < s.n; sp += 4) {                    // (four splits' requests under way, the additions in split order)
+        float q[4][N];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < N; ++i) q[j][i] = s.p[(size_t)min(sp + j, s.n - 1) * s.plane + at[i]];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (sp + j < s.n) {
+#pragma unroll
+                for (int i = 0; i < N; ++i) v[i] += q[j][i];
+            }
+    }
+}
+template <bool TABLE>
+__global__ __launch_bounds__(256) void rope_kv_store_parts_kernel(float* __restrict__ q, const RopeSource sq, const RopeSource sk, const RopeSource sv, const int* __restrict__ positions, int n_heads,
+                                                                  int n_kv_heads, int head_dim, float theta, float fscale, int interleaved, uint16_t* __restrict__ kc,
+                                                                  uint16_t* __restrict__ vc, int start_pos, int max_seq) {
+    __shared__ float cs[2][TABLE ? 128 : 1];
+    const int sp = blockIdx.x, half_dim = head_dim / 2, pos = positions[sp];
+    auto angle_of = [&](int i, float& c, float& s) {
+        const float freq = 1.0f / (float)pow((double)theta, (double)((2.0f * i) / head_dim));
+        const float angle = pos * freq * fscale;
+        c = cosf(angle);
+        s = sinf(angle);
+    };
+    if constexpr (TABLE) {
+        for (int i = threadIdx.x; i < half_dim; i += blockDim.x) angle_of(i, cs[0][i], cs[1][i]);
+        __syncthreads();
+    }
+    const int cp = start_pos + sp, per_pos = n_kv_heads * head_dim;
+    const bool store = cp < max_seq;   // reference attention.cu:336
+    const int total = (n_heads + n_kv_heads) * half_dim, first = blockIdx.y * blockDim.x + threadIdx.x, stride = gridDim.y * blockDim.x;
+    for (int idx = first; idx < total; idx += stride) {
+        const int pair = idx % half_dim, head = idx / half_dim;
+        const int i0 = interleaved ? 2 * pair : pair, i1 = interleaved ? 2 * pair + 1 : pair + half_dim;
+        const bool query = head < n_heads;
+        const size_t base = query ? ((size_t)sp * n_heads + head) * head_dim : ((size_t)sp * n_kv_heads + (head - n_heads)) * head_dim;
+        const size_t at[2] = {base + i0, base + i1};
+        float v[2], c, s, ra, rb;
+        if (query) rope_sums(sq, at, v);
+        else rope_sums(sk, at, v);
+        if constexpr (TABLE) { c = cs[0][pair]; s = cs[1][pair]; }
+        else angle_of(pair, c, s);
+        rope_rotate(v[0], v[1], c, s, ra, rb);
+        if (query) { q[at[0]] = ra; q[at[1]] = rb; }
+        else if (store) {
+            uint16_t* row = kc + (size_t)cp * per_pos + (size_t)(head - n_heads) * head_dim;
+            row[i0] = f2h(ra);
+            row[i1] = f2h(rb);
+        }
+    }
+    if (store)
+        for (int e = first; e < per_pos; e += stride) {
+            const size_t at[1] = {(size_t)sp * per_pos + e};
+            float v[1];
+            rope_sums(sv, at, v);
+            vc[(size_t)cp * per_pos + e] = f2h(v[0]);
+        }
+}
+
 __global__ void kv_store_kernel(uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, const float* __restrict__ k,
                                 const float* __restrict__ v, int total, int per_pos, int start_pos, int max_seq) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -859,6 +928,26 @@ int ntk_rope_kv_store(float* q, const float* k, const float* v, const int* posit
     const int parts = seq_len <= 64 ? 4 : 1;
     hipLaunchKernelGGL(ntk::rope_kv_store_rows_kernel, dim3(seq_len, parts), dim3(256), 0, ntk::resolve_stream(stream), q, k, v, positions, n_heads, n_kv_heads,
                        head_dim, theta_base, freq_scale, interleaved, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), start_pos, max_seq);
+    return ntk::last_launch_status();
+}
+
+int ntk_reduce_rope_kv_store(float* q, const float* const* sums, const int* splits, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim, float theta_base,
+                             float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream) {
+    if (!q || !sums || !splits || !sums[0] || !sums[1] || !sums[2] || !positions || !k_cache || !v_cache) return NTK_E_NULL;
+    if (seq_len < 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim <= 0 || (head_dim & 1) || head_dim > 256 || start_pos < 0 || max_seq <= 0) return NTK_E_SHAPE;
+    if (splits[0] < 1 || splits[1] < 1 || splits[2] < 1) return NTK_E_SHAPE;
+    if (seq_len == 0) return NTK_OK;
+    const size_t nq = (size_t)seq_len * n_heads * head_dim, nk = (size_t)seq_len * n_kv_heads * head_dim;
+    const ntk::RopeSource sq{sums[0], splits[0], nq}, sk{sums[1], splits[1], nk}, sv{sums[2], splits[2], nk};
+    hipStream_t s = ntk::resolve_stream(stream);
+    uint16_t *kc = static_cast<uint16_t*>(k_cache), *vc = static_cast<uint16_t*>(v_cache);
+    if (seq_len <= 64) {
+        const int parts = ((n_heads + n_kv_heads) * (head_dim / 2) + 255) / 256;
+        hipLaunchKernelGGL(ntk::rope_kv_store_parts_kernel<false>, dim3(seq_len, parts), dim3(256), 0, s, q, sq, sk, sv, positions, n_heads, n_kv_heads, head_dim, theta_base, freq_scale,
+                           interleaved, kc, vc, start_pos, max_seq);
+    } else
+        hipLaunchKernelGGL(ntk::rope_kv_store_parts_kernel<true>, dim3(seq_len), dim3(256), 0, s, q, sq, sk, sv, positions, n_heads, n_kv_heads, head_dim, theta_base, freq_scale, interleaved,
+                           kc, vc, start_pos, max_seq);
     return ntk::last_launch_status();
 }
 

@@ -751,29 +751,45 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         }
         for (int t = 0; t < T; ++t) gemv(Y + (size_t)t * ystride, w, wp, X + (size_t)t * xstride);
     };
-    // matrices that share X (Q | K | V, gate | up): those of one format go out as ONE launch of the FP16 GEMM, the rest one by one
-    auto project_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm) {
+    // matrices that share X (Q | K | V, gate | up): those of one format go out as ONE launch of the FP16 GEMM, the rest one by one, ahead of them.  sums / splits: the LAST launch may
+    // leave the partial sums of its K splits to the consumer (its matrices' places in the two are then set; a launch behind it would overwrite them)
+    auto project_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, const float** sums = nullptr, int* splits = nullptr) {
         bool done[3] = {false, false, false};
         if (project_half_many(Ys, Ws, n, X, rm, false)) return;
-        if (batched && bf16_now) {
+        struct Group { int idx[3], m; } groups[3];
+        int n_groups = 0;
+        if (batched && bf16_now)
             for (int a = 0; a < n; ++a) {
                 if (done[a]) continue;
-                ntk_gemv_seg segs[3];
-                int idx[3], m = 0;
+                Group& g = groups[n_groups];
+                g.m = 0;
                 for (int b = a; b < n; ++b)
-                    if (!done[b] && Ws[b]->dtype == Ws[a]->dtype && Ws[b]->in_f == Ws[a]->in_f) idx[m++] = b;
-                if (m < 2) continue;
-                bool all_rp = true;
-                for (int k = 0; k < m; ++k) all_rp = all_rp && rp_only(*Ws[idx[k]]);
-                if (!all_rp) raw_begin();   // (the group's tensors side by side in the unpack scratch when their GGUF bytes are not resident)
-                for (int k = 0; k < m; ++k) segs[k] = {all_rp ? Ws[idx[k]]->rp : raw_of(*Ws[idx[k]]), Ys[idx[k]], (int)Ws[idx[k]]->out_f, Ws[idx[k]]->dtype};
-                const int st = gemm_f16(segs, m, X, (int)Ws[a]->in_f, nullptr, X == planes_of ? 1 : 0, rm, nullptr, all_rp);
-                if (st == NTK_OK) { planes_of = X; for (int k = 0; k < m; ++k) done[idx[k]] = true; }
-                else if (st != NTK_E_DTYPE && st != NTK_E_SHAPE && st != NTK_E_ALIGN) { ok(st); return; }
+                    if (!done[b] && Ws[b]->dtype == Ws[a]->dtype && Ws[b]->in_f == Ws[a]->in_f) g.idx[g.m++] = b;
+                if (g.m < 2) continue;
+                for (int k = 0; k < g.m; ++k) done[g.idx[k]] = true;
+                ++n_groups;
             }
-        }
         for (int a = 0; a < n; ++a)
             if (!done[a]) project(Ys[a], *Ws[a], X, (size_t)Ws[a]->out_f, (size_t)Ws[a]->in_f, rm);
+        for (int gi = 0; gi < n_groups; ++gi) {
+            const Group& g = groups[gi];
+            ntk_gemv_seg segs[3];
+            ntk_gemm_partials pt;
+            const bool defer = sums && gi + 1 == n_groups;
+            bool all_rp = true;
+            for (int k = 0; k < g.m; ++k) all_rp = all_rp && rp_only(*Ws[g.idx[k]]);
+            if (!all_rp) raw_begin();   // (the group's tensors side by side in the unpack scratch when their GGUF bytes are not resident)
+            for (int k = 0; k < g.m; ++k) segs[k] = {all_rp ? Ws[g.idx[k]]->rp : raw_of(*Ws[g.idx[k]]), Ys[g.idx[k]], (int)Ws[g.idx[k]]->out_f, Ws[g.idx[k]]->dtype};
+            const int st = gemm_f16(segs, g.m, X, (int)Ws[g.idx[0]]->in_f, nullptr, X == planes_of ? 1 : 0, rm, defer ? &pt : nullptr, all_rp);
+            if (st == NTK_OK) {
+                planes_of = X;
+                if (defer && pt.nsplit > 1)
+                    for (int k = 0; k < g.m; ++k)
+                        if (pt.part[k]) { sums[g.idx[k]] = pt.part[k]; splits[g.idx[k]] = pt.nsplit; }
+            } else if (st != NTK_E_DTYPE && st != NTK_E_SHAPE && st != NTK_E_ALIGN) { ok(st); return; }
+            else
+                for (int k = 0; k < g.m; ++k) project(Ys[g.idx[k]], *Ws[g.idx[k]], X, (size_t)Ws[g.idx[k]]->out_f, (size_t)Ws[g.idx[k]]->in_f, rm);
+        }
     };
     // hidden += W . X (attention.cpp:207 + transformer.cpp:645, ffn.cpp:130 + transformer.cpp:652): the batched
     // projection adds the residual in its epilogue, the reference sequence goes through residual_ and launch_add_inplace
@@ -860,14 +876,20 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
         normed_ahead = false;
         planes_of = planes_ready;   // residual_ has new contents (split already by the launch that wrote them, or not)
         planes_ready = nullptr;
+        const bool one_launch = with_max && T >= 4 && hd <= 256;
+        const float* sums[3] = {q_buf, k_buf, v_buf};     // what the rotation reads: the projections, or the partial sums of the last launch's
+        int splits[3] = {1, 1, 1};
         {
             float* const ys[3] = {q_buf, k_buf, v_buf};
             const DevTensor* const ws[3] = {&L.wq, &L.wk, &L.wv};
-            project_many(ys, ws, 3, residual_, max_a);
+            project_many(ys, ws, 3, residual_, max_a, one_launch ? sums : nullptr, splits);
         }
-        if (with_max && T >= 4 && hd <= 256) {   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
-            ok(ntk_rope_kv_store(q_buf, k_buf, v_buf, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc,
-                                 start_pos, cfg_.max_seq_len, s));
+        if (one_launch) {                            // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
+            if (splits[0] + splits[1] + splits[2] > 3)
+                ok(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
+            else
+                ok(ntk_rope_kv_store(q_buf, k_buf, v_buf, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc,
+                                     start_pos, cfg_.max_seq_len, s));
         } else {
             ok(ntk_rope(q_buf, k_buf, positions_, 1, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, s));
             ok(ntk_copy_to_kv_cache(kc, vc, k_buf, v_buf, T, nkv, hd, start_pos, cfg_.max_seq_len, s));
