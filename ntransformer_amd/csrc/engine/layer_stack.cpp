@@ -1116,11 +1116,12 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
 }
 
 // the window mixer: one product for [q | k | v], rotation and cache rows, attention over the window, output projection -> mix_
-int LayerStackModel::run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, const void* h16) {
+int LayerStackModel::run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, bool norm_inside, const void* h16) {
     const WindowMixer& m = L.att;
     const int W = info_.width, na = (int)m.in.out_f, hv = m.heads * m.vdim;
     ntk_dense_desc d{};
     d.Y = a_; d.ldy = na; d.X = h; d.ldx = W; d.W = m.in.ptr; d.wdtype = m.in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = na; d.K = W;
+    if (norm_inside) { d.norm_w = L.norm1.w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }
     LS_TRY(first_product(d, h16));
     LS_TRY(window_heads(m, cache, att_, hv, T, pos0));
     return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
@@ -1194,7 +1195,7 @@ int LayerStackModel::run_lightning(const StackLayer& L, float* state, int T, int
 // h16: the input rows as bfloat16 too (or alone); then, where both products take such operands, the first leaves the activations as bfloat16 in `act` -- the values that the
 // second would round at its input -- and its two halves never reach memory.
 int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
-                                 int full_x, const void* h16) {
+                                 int full_x, const void* h16, const float* norm_w) {
     const int W = info_.width;
     ntk_dense_desc d{};
     if (h16 && !full_x && rounded(ex.gate_up, rows) && rounded(ex.down, rows)) {
@@ -1214,6 +1215,7 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
     const bool direct = !ex.plain && wdtype_ == NTK_DT_F32 && ntk_dense_direct_takes(NTK_DT_F32, rows, rows / top, ex.in_rows(), W);      // gate and up meet in the first product's launch
     d.Y = gu; d.ldy = ex.in_rows(); d.X = h; d.ldx = W; d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype;
     d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top; d.T = rows; d.N = ex.in_rows(); d.K = W; d.accumulate = 0;
+    if (norm_w) { d.norm_w = norm_w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }
     if (ex.plain) {                       // the activation inside the product, whatever its form
         d.Y = act; d.act = NTK_ACT_RELU2;
         LS_TRY(first_product(d));
@@ -1233,6 +1235,7 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
         LS_TRY(ntk_glu(act, gu, rows, ex.ff, ex.limit, glu_alpha, glu_up_offset, stream_));
     }
     d.add_y = nullptr;
+    d.norm_w = nullptr;
     d.full_x = full_x;
     d.Y = out; d.ldy = W; d.X = act; d.ldx = ex.ff; d.W = ex.down.ptr; d.wstride = ex.down.stride(); d.wdtype = ex.down.dtype;
     d.rows = nullptr; d.row_div = 1; d.N = W; d.K = ex.ff;
@@ -1313,22 +1316,23 @@ int LayerStackModel::run_dense_ff(const StackLayer& L, int T) {
 }
 
 // the dense gated unit (the experts' unit with one member, clipped or plain): gate and up in one product (decoding: the activation inside its launch), down -> ff_
-int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16) {
+int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16, const float* norm_w) {
     if (!h16 && rounded(L.cff.gate_up, T)) {
         LS_TRY(ntk_round_rows(h2_16_, info_.width, h, info_.width, T, info_.width, stream_));
         h16 = h2_16_;
     }
-    return run_experts(form_.clipped_glu ? kGluAlpha : 1.0f, form_.clipped_glu ? 1.0f : 0.0f, L.cff, h, gu2_, zf_, ff_, T, nullptr, nullptr, 1, 0, h16);
+    return run_experts(form_.clipped_glu ? kGluAlpha : 1.0f, form_.clipped_glu ? 1.0f : 0.0f, L.cff, h, gu2_, zf_, ff_, T, nullptr, nullptr, 1, 0, h16, norm_w);
 }
 
 // the delta rule with per-head gates: one product for [q | k | v | gate | beta | decay], the short convolutions of q, k and v (+ silu) with their carried
 // inputs, the recurrence (unit q and k, decay and write strength formed from their raw projections in its pre-pass), unit norm per head with the shared
 // weight and the silu gate, output projection -> mix_.  state = [S | the convolutions' last inputs]
-int LayerStackModel::run_gated_delta(const StackLayer& L, float* state, int T, int pos0, const void* h16) {
+int LayerStackModel::run_gated_delta(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16) {
     const GatedDeltaMixer& m = L.gdl;
     const int W = info_.width, na = (int)m.in.out_f, nc = m.channels(), hv = m.heads * m.vdim;
     ntk_dense_desc in{};
-    in.Y = a_; in.ldy = na; in.X = h1_; in.ldx = W; in.W = m.in.ptr; in.wdtype = m.in.dtype; in.G = 1; in.row_div = 1; in.T = T; in.N = na; in.K = W;
+    in.Y = a_; in.ldy = na; in.X = h; in.ldx = W; in.W = m.in.ptr; in.wdtype = m.in.dtype; in.G = 1; in.row_div = 1; in.T = T; in.N = na; in.K = W;
+    if (norm_inside) { in.norm_w = L.norm1.w; in.norm_eps = eps_; in.norm_offset = norm_offset_; }
     LS_TRY(first_product(in, h16));
     ntk_gated_recurrence_desc d{};
     if (T == 1) {   // a decoded token: the convolutions run inside the recurrence's pre-pass
@@ -1371,12 +1375,20 @@ int LayerStackModel::seam_for(const DenseW& in, const NormW& nw, float* out, voi
 int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0) {
     const DenseW& in = L.mixer == kMixWindow ? L.att.in : L.mixer == kMixLatent ? L.mix.in : L.gdl.in;
     const void* h16 = nullptr;
-    LS_TRY(seam_for(in, L.norm1, h1_, h1_16_, T, &h16));
-    if (L.mixer == kMixWindow) LS_TRY(run_window(L, h1_, run.cache + (size_t)slot * opt_.max_context * L.att.row(), T, pos0, h16));
-    else if (L.mixer == kMixLatent) LS_TRY(run_mixer(L, run.cache + (size_t)slot * opt_.max_context * L.mix.row(), T, pos0, h1_, false, h16));
-    else LS_TRY(run_gated_delta(L, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0, h16));
+    // decoding: what the stream is owed and the norm ride in the sublayer's first product (a launch of 3.9 us and its boundary less, twice a layer)
+    const bool few = T <= ntk_dense_few_rows();
+    if (!few) LS_TRY(seam_for(in, L.norm1, h1_, h1_16_, T, &h16));
+    const float* h = few ? x_ : h1_;
+    if (L.mixer == kMixWindow) LS_TRY(run_window(L, h, run.cache + (size_t)slot * opt_.max_context * L.att.row(), T, pos0, few, h16));
+    else if (L.mixer == kMixLatent) LS_TRY(run_mixer(L, run.cache + (size_t)slot * opt_.max_context * L.mix.row(), T, pos0, h, few, h16));
+    else LS_TRY(run_gated_delta(L, h, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0, few, h16));
     owed_ = Owed{mix_, L.norm1b};
     if (!L.has_mlp) return NTK_OK;
+    if (few) {
+        LS_TRY(run_unit_ff(L, x_, T, nullptr, L.norm2.w));
+        owed_ = Owed{ff_, L.norm2b};
+        return NTK_OK;
+    }
     // (the down product takes the activations as the first one leaves them: both or none)
     if (rounded(L.cff.down, T)) LS_TRY(seam_for(L.cff.gate_up, L.norm2, h2_, h2_16_, T, &h16));
     else { h16 = nullptr; LS_TRY(rms_seam(L.norm2, h2_, T)); }
@@ -1399,15 +1411,15 @@ int LayerStackModel::linear(float* Y, int ldy, const float* X, int ldx, const vo
     return product(d);
 }
 
-// The first product of a sublayer.  In the post-norm form it reads the stream itself: with few rows, what the stream is still owed joins it inside this launch, which
-// leaves the new stream in the other buffer (its workgroups all read the old one).
+// The first product of a sublayer.  In the post-norm form it reads the stream itself, in the scaled form it does with few rows (its norm inside the launch): what the stream is still
+// owed then joins it inside this launch, which leaves the new stream in the other buffer (its workgroups all read the old one).
 int LayerStackModel::first_product(ntk_dense_desc& d, const void* x16) {
     if (x16) {
         const ntk_direct_desc e{x16, d.K, d.T, nullptr, 0};
         d.scratch = pscratch_; d.scratch_bytes = pscratch_bytes_;
         return ntk_dense_direct(&d, &e, stream_);
     }
-    if (!form_.post_norm || !owed_.y || d.X != x_) return product(d);
+    if (!(form_.post_norm || form_.scaled) || !owed_.y || d.X != x_) return product(d);
     const int W = info_.width;
     d.add_y = owed_.y; d.ld_add = W; d.add_w = owed_.nb.w; d.add_eps = eps_; d.add_mult = residual_mult_; d.x_out = x0_; d.ldxo = W;
     LS_TRY(product(d));

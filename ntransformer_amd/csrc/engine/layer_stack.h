@@ -311,8 +311,8 @@ private:
     int run_parallel(const StackLayer& L, float* cache, float* state, int T, int pos0);
     int run_gated_ff(const StackLayer& L, int T);
     int parse_gated_delta(const Json& L, GatedDeltaMixer& m);
-    int run_gated_delta(const StackLayer& L, float* state, int T, int pos0, const void* h16 = nullptr);
-    int run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16 = nullptr);
+    int run_gated_delta(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16);
+    int run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16 = nullptr, const float* norm_w = nullptr);
     int post_norm_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int rms_seam(const NormW& nw, float* out, int T);
     int seam_for(const DenseW& in, const NormW& nw, float* out, void* out16, int T, const void** h16);
@@ -329,14 +329,14 @@ private:
     void* dev_alloc(size_t bytes);
     int portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, float* logits_out);
     int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false, const void* h16 = nullptr);
-    int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, const void* h16 = nullptr);
+    int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, bool norm_inside = false, const void* h16 = nullptr);
     int window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0);
     int dense_parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int run_lightning(const StackLayer& L, float* state, int T, int pos0);
     int run_moe(const StackLayer& L, const float* h, int T, bool into_stream, const void* h16 = nullptr);
     int run_dense_ff(const StackLayer& L, int T);
     int run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
-                    int full_x, const void* h16 = nullptr);
+                    int full_x, const void* h16 = nullptr, const float* norm_w = nullptr);   // norm_w (few rows): the rows are normed inside the first product
     int norm_conv(const NormW& nw, const float* canon, float* conv_state, float* out, int T, int pos0);
     int settle(int T);
     int first_product(ntk_dense_desc& d, const void* x16 = nullptr);
