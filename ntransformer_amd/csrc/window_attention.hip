@@ -365,6 +365,134 @@ __global__ __launch_bounds__(256) void window_attention_kernel(const WinArgs a) 
     }
 }
 
+// ---- a few tokens (decoding): one map, heads of up to 128 + 128 entries on 16 bytes
+// A workgroup owns a token and one key / value head (and every `splits`-th chunk of 64 keys): the keys AND values of a chunk are requested together, ahead of the first product, a wave
+// takes sixteen of them -- sixteen lanes a key for the scores of all the heads that share it, 32 lanes a value row for the sums -- and keeps an online softmax of its own; the
+// four waves meet in LDS.  What bounds it is the one round trip to the cache rows: a decoded token of 16 heads on 4 (128 + 128) behind 40 positions 20.5 us in the form above (a key slab, a
+// value slab and two barriers each, one after the other), 11.4 us here.  Up to four chunks stay in one workgroup (no launch that merges).
+constexpr int kFewTokens = 8, kFewChunk = 64;
+template <int RM>
+__global__ __launch_bounds__(256) void window_attention_few_kernel(const WinArgs a) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ float Ps[4][RM][16];
+    __shared__ __attribute__((aligned(16))) float part[4][RM][132];       // [vector | max | sum]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sub = lane & 15, kq = lane >> 4, half = lane >> 5, col = 4 * (lane & 31);
+    const int g = blockIdx.x, t = blockIdx.y, R = a.H / a.G, pos = a.pos0 + t;
+    const int jlo = first_visible(pos, a.window, a.chunks), kept = min(a.keep, jlo), skip = jlo - kept, n_keys = kept + pos - jlo + 1;
+    auto key_pos = [&](int n) { const int m = min(n, n_keys - 1); return m + (m >= kept ? skip : 0); };
+    const f4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+    f4 q[RM][2];
+#pragma unroll
+    for (int r = 0; r < RM; ++r) {
+        const float* qr = a.q + (long long)t * a.ldq + (long long)(g * R + min(r, R - 1)) * a.dn;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) q[r][e] = 4 * sub + 64 * e < a.dn ? *reinterpret_cast<const f4*>(qr + 4 * sub + 64 * e) : zero;
+    }
+    float mx[RM], l[RM], slope[RM];
+    f4 acc[RM];
+#pragma unroll
+    for (int r = 0; r < RM; ++r) {
+        const int head = g * R + min(r, R - 1);
+        const bool sunk = (a.sink || a.sinks) && blockIdx.z == 0 && wave == 0;       // (one part starts from the sink, a key without a value)
+        mx[r] = sunk ? (a.sinks ? a.sinks[head] : 0.0f) : -INFINITY;
+        l[r] = sunk ? 1.0f : 0.0f;
+        slope[r] = a.slopes ? a.slopes[head] : 0.0f;
+        acc[r] = zero;
+    }
+    const float* kbase = a.cache + g * a.dn;
+    const float* vbase = a.cache + a.G * a.dn + g * a.dv;
+    for (int n0 = blockIdx.z * kFewChunk; n0 < n_keys; n0 += a.splits * kFewChunk) {
+        f4 k[4][2], v[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float* kr = kbase + (long long)key_pos(n0 + 16 * wave + 4 * i + kq) * a.row;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) k[i][e] = 4 * sub + 64 * e < a.dn ? *reinterpret_cast<const f4*>(kr + 4 * sub + 64 * e) : zero;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int n = n0 + 16 * wave + 2 * i + half;
+            const f4 x = col < a.dv ? *reinterpret_cast<const f4*>(vbase + (long long)key_pos(n) * a.row + col) : zero;
+            v[i] = n < n_keys ? x : zero;
+        }
+#pragma unroll
+        for (int r = 0; r < RM; ++r) {
+            float s[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f4 x = q[r][0] * k[i][0], y = q[r][1] * k[i][1];
+                const int n = n0 + 16 * wave + 4 * i + kq, j = key_pos(n), head = g * R + min(r, R - 1);
+                float sv = group_sum<16>(((x[0] + x[1]) + (x[2] + x[3])) + ((y[0] + y[1]) + (y[2] + y[3]))) * a.scale;
+                if (a.rel) sv += a.rel[(long long)a.bucket_of[min(pos - j, a.n_dist - 1)] * a.H + head];
+                if (a.slopes) sv -= slope[r] * (float)(pos - j);
+                if (a.softcap > 0.0f) sv = a.softcap * tanhf(sv / a.softcap);
+                s[i] = n < n_keys ? sv : -INFINITY;
+            }
+            float m = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+            m = fmaxf(m, __shfl_xor(m, 16, 64));
+            m = fmaxf(mx[r], fmaxf(m, __shfl_xor(m, 32, 64)));
+            const float base = m == -INFINITY ? 0.0f : m, corr = mx[r] == -INFINITY ? 0.0f : expf(mx[r] - base);
+            mx[r] = m;
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float p = expf(s[i] - base);             // (0 past the last key)
+                sum += p;
+                if (sub == 0) Ps[wave][r][4 * i + kq] = p;
+            }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            l[r] = fmaf(l[r], corr, sum);
+            acc[r] *= corr;
+        }
+        __builtin_amdgcn_wave_barrier();                       // (a wave's LDS operations run in order)
+#pragma unroll
+        for (int r = 0; r < RM; ++r)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { const float p = Ps[wave][r][2 * i + half]; acc[r] += p * v[i]; }
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int r = 0; r < RM; ++r) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[r][c] += __shfl_xor(acc[r][c], 32, 64);
+        if (half == 0) *reinterpret_cast<f4*>(&part[wave][r][col]) = acc[r];
+        if (lane == 0) { part[wave][r][128] = mx[r]; part[wave][r][129] = l[r]; }
+    }
+    __syncthreads();
+    for (int r = wave; r < R; r += 4) {
+        float m = -INFINITY, w[4], sum = 0.0f, y[WMAXC];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m = fmaxf(m, part[i][r][128]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            w[i] = part[i][r][128] == -INFINITY ? 0.0f : expf(part[i][r][128] - m);
+            sum = fmaf(w[i], part[i][r][129], sum);
+        }
+#pragma unroll
+        for (int c = 0; c < WMAXC; ++c) {
+            y[c] = 0.0f;
+            if (c < 2)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) if (w[i] != 0.0f) y[c] = fmaf(w[i], part[i][r][64 * c + lane], y[c]);
+        }
+        const int h = g * R + r;
+        if (a.splits > 1) {
+            float* st = a.scratch + (((long long)t * a.H + h) * a.splits + blockIdx.z) * (2 + a.dv);
+            if (lane == 0) { st[0] = m; st[1] = sum; }
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                if (64 * c + lane < a.dv) st[2 + 64 * c + lane] = y[c];
+            continue;
+        }
+        const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+        float row[1][WMAXC];
+#pragma unroll
+        for (int c = 0; c < WMAXC; ++c) row[0][c] = y[c] * inv;
+        finish_row<1>(row, lane, a.dv, a.lambda, a.sub_norm, a.eps, a.out_scale, a.out + (long long)t * a.ldo + (long long)h * a.dv, gate_of(a, t, h), a.head_gate ? 0 : 1);
+    }
+}
+
 // merge of the partial states of one (token, head) row, one wave per row: lane = part for the weights exp(max_s - max) and the sum (splits <= 64), then
 // lane = column for the weighted vectors, the parts in order with their loads independent of each other
 template <int M>
@@ -504,6 +632,21 @@ int ntk_window_attention_ex(const ntk_window_attention_desc* d, void* image, siz
         t.window = a.window; t.chunks = a.chunks; t.keep = a.keep; t.scale = a.scale; t.softcap = a.softcap; t.out_scale = a.out_scale; t.sink = a.sink; t.sinks = a.sinks;
         t.slopes = a.slopes; t.rel = a.rel; t.bucket_of = a.bucket_of; t.n_dist = a.n_dist; t.gate = a.gate; t.ldg = a.ldg; t.head_gate = a.head_gate;
         if (!launch_attention_half(t, image, image_bytes, s)) launch_attention_tile(t, s);
+        return last_launch_status();
+    }
+    const int R = d->H / d->G;
+    if (d->maps == 1 && d->T <= kFewTokens && R <= 8 && d->dn <= 128 && d->dv <= 128 && !((d->dn | d->dv | d->row | d->ldq) & 3) && !(((uintptr_t)d->cache | (uintptr_t)d->q) & 15)) {
+        // (the scratch holds 4096 parts)
+        const int chunks = (window_keys(d->pos0, d->T, d->window, a.chunks, a.keep) + kFewChunk - 1) / kFewChunk;
+        a.splits = d->scratch && chunks > 4 ? std::max(1, std::min(std::min(chunks, 64), std::min(4096 / (d->T * d->H), 512 / (d->T * d->G)))) : 1;
+        const dim3 few(d->G, d->T, a.splits);
+        if (R <= 1) hipLaunchKernelGGL(window_attention_few_kernel<1>, few, dim3(256), 0, s, a);
+        else if (R <= 2) hipLaunchKernelGGL(window_attention_few_kernel<2>, few, dim3(256), 0, s, a);
+        else if (R <= 4) hipLaunchKernelGGL(window_attention_few_kernel<4>, few, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(window_attention_few_kernel<8>, few, dim3(256), 0, s, a);
+        const int st = last_launch_status();
+        if (st != NTK_OK || a.splits == 1) return st;
+        hipLaunchKernelGGL(window_attention_merge_kernel<1>, dim3(d->T * d->H), dim3(64), 0, s, a);
         return last_launch_status();
     }
     const int DNP = (d->dn + 3) & ~3;
