@@ -612,7 +612,7 @@ template <> struct DeqI<NTK_DT_Q4_K + GB_RP> {
     using Hdr = RpHdr;
     struct MinOp { uint32_t m0, m1; float ndmin64; };
     template <typename H> __device__ static MinOp min_operand(const H& hd, int g) {   // record bytes 8..15: m_0 .. m_7
-        const uint32_t w = g == 0 ? hd.rec.z : (g == 1 ? hd.rec.w : 0u);
+        const uint32_t w = (hd.rec.z & (g == 0 ? ~0u : 0u)) | (hd.rec.w & (g == 1 ? ~0u : 0u));
         return MinOp{cvt2_u8_f16<0>(w), cvt2_u8_f16<2>(w), -64.0f * h2f((uint16_t)(hd.dd >> 16))};
     }
     struct Raw { uint32_t lo, hi; float s0; };
@@ -643,7 +643,7 @@ template <> struct DeqI<NTK_DT_Q5_K + GB_RP> {
     using Hdr = RpHdr;
     struct MinOp { uint32_t m0, m1; float ndmin64; };
     template <typename H> __device__ static MinOp min_operand(const H& hd, int g) {
-        const uint32_t w = g == 0 ? hd.rec.z : (g == 1 ? hd.rec.w : 0u);
+        const uint32_t w = (hd.rec.z & (g == 0 ? ~0u : 0u)) | (hd.rec.w & (g == 1 ? ~0u : 0u));
         return MinOp{cvt2_u8_f16<0>(w), cvt2_u8_f16<2>(w), -64.0f * h2f((uint16_t)(hd.dd >> 16))};
     }
     struct Raw { uint32_t lo, hi, b5lo, b5hi; float s0; };
@@ -1548,17 +1548,15 @@ __global__ __launch_bounds__(512) void gemm_quant_f16_small_kernel(const GemmSPa
 // time came out at 6.5 - 8 TB/s for every projection, i.e. the L2 -> CU path, with every workgroup of an XCD asking the same channels for the same lines.
 // (A request queue in consumption order -- weights and planes the same distance ahead -- changed nothing: profiles/r06_prompt_kslice.txt.)
 // Here a workgroup owns a K SLICE (blockIdx.y) and NW row tiles: the slice's planes are copied ONCE into LDS by LDS-DMA (<= 64 / NTB steps = 128 KB), every
-// wave then streams ITS tile's weights of the slice (loader, per-wave image and decoders as above, DEPTH units of weights in flight per wave in registers)
+// wave then streams ITS tile's weights of the slice (loader, per-wave image and decoders as above, the next unit of weights in flight per wave in registers)
 // and reads the B operands of a step from LDS.  Planes traffic = slice bytes per workgroup (Wo: 8 MB instead of 67); the slices' partial sums go to the
 // partial-sum area the K splits of the large kernel use ([slice][token][row]; summed in slice order by the launch that consumes the projection or by
 // reduce_splits_kernel), a launch with ONE slice writes Y itself.
-#ifndef NTK_GK_DEPTH4
-#define NTK_GK_DEPTH4 4   // units of 4 steps (Q8_0: 2176 B per 16 rows) in flight per wave
-#endif
-#ifndef NTK_GK_DEPTH8
-#define NTK_GK_DEPTH8 2   // units of 8 steps
-#endif
-template <int SPU> constexpr int gk_depth() { return SPU <= 4 ? NTK_GK_DEPTH4 : (SPU <= 8 ? NTK_GK_DEPTH8 : 1); }   // (16-step units: the next one, 8.7 KB per wave)
+// ONE unit ahead, and a loop of one unit: deeper rings (two units of a K-quant, four of Q8_0, until now) were code before they were bandwidth.  Every launch
+// fetches its instructions anew, a loop of 16 unrolled steps cost each launch about a microsecond more than one of 8 (of 32: 2.5 more), the requests past
+// a slice's end fetched real bytes, and slices had to be whole numbers of groups.  8B at 16 tokens, us per launch, before -> now: Q4_K gate | up 25.9 -> 24.9,
+// Q | K | V 9.8 -> 8.9, Q6_K down 19.1 -> 16.2; eight layers of Q8_0 1220 -> 1095 us.
+// Smaller still loses: the unit's eight steps in a loop of four 846, of two 906 us for 32 layers' gate | up against 814.
 struct GemmKParams {
     GemmBSeg seg[GB_MAX_SEG];
     int nseg;
@@ -1568,7 +1566,7 @@ struct GemmKParams {
     const float* resid;     // (one slice only)
     int T, in, steps;
     unsigned row_bytes;
-    int nsplit, units_per_split;   // blockIdx.y = K slice of units_per_split units (a multiple of the ring depth; nsplit * units_per_split = all units)
+    int nsplit, units_per_split;   // blockIdx.y = K slice of units_per_split units (nsplit * units_per_split = all units)
     int tiles;                     // row tiles (16 RT rows) of all matrices; (blockIdx.x + job * gridDim.x) * NW + wave = this wave's in job `job`
     int jobs;                      // row groups per workgroup
 };
@@ -1593,7 +1591,6 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
     using D = DeqI<DT>;
     constexpr int SPU = D::SPU, NCH = D::NCH, STRIDE = D::STRIDE;
     constexpr int ROWS = 16 * RT, PIECES = D::RP ? RT * D::PPI : ROWS * NCH, NLD = (PIECES + 63) / 64;
-    constexpr int DEPTH = gk_depth<SPU>();
     extern __shared__ __attribute__((aligned(16))) uint8_t gk_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), NW = (int)(blockDim.x >> 6);
@@ -1651,12 +1648,13 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
         }
     }
     auto load_unit = [&](u32x4 (&w)[NLD], int unit) {
+        const uint32_t live = unit < u_hi ? ~0u : 0u;   // (past the slice every lane asks for the matrix's first 16 bytes: straight-line code, exact waits, no traffic)
 #pragma unroll
         for (int n = 0; n < NLD; ++n) {
             uint32_t off;
             if constexpr (D::RP) off = w_row[n] + (uint32_t)unit * (s_pk[n] >> 16);
             else off = min(((w_row[n] + (uint32_t)unit * D::UB) & ~15u) + (s_pk[n] >> 16), seg_w_last);
-            w[n] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(segW + off));
+            w[n] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(segW + (off & live)));
         }
     };
     auto load_sums = [&](uint64_t (&v)[GB_PLANES][NTB], int unit) {   // the step sums of a unit (K-quant minimum term): 8 bytes per lane, piece and token block
@@ -1678,46 +1676,34 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) acc[rt][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // ---- prologue of a row group: its first DEPTH units of weights go out (HBM: the long round trip; for the first group, behind the planes' copy) ----
-    // (scheduling barriers between the requests: the compiler counts its waits from their ORDER -- shuffled, it ends in vmcnt(0) at the head of every group)
-    u32x4 wreg[DEPTH][NLD];
-    uint64_t svr[D::HAS_MIN ? DEPTH : 1][GB_PLANES][NTB];
-    const int u_last = u_hi - 1;
-#pragma unroll
-    for (int k = 0; k < DEPTH; ++k) {   // (requests past the slice repeat its last unit: straight-line code, exact waits)
-        load_unit(wreg[k], min(u_lo + k, u_last));
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (D::HAS_MIN) { load_sums(svr[k], min(u_lo + k, u_last)); __builtin_amdgcn_sched_barrier(0); }
-    }
+    // ---- prologue of a row group: its first unit of weights goes out (HBM: the long round trip; for the first group, behind the planes' copy) ----
+    // (scheduling barriers between the requests: the compiler counts its waits from their ORDER -- shuffled, it ends in vmcnt(0) at the head of every unit)
+    u32x4 wreg[NLD];
+    uint64_t svr[GB_PLANES][NTB];
+    load_unit(wreg, u_lo);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (D::HAS_MIN) { load_sums(svr, u_lo); __builtin_amdgcn_sched_barrier(0); }
     if (it == 0) {   // (uniform) the planes have landed -- and with them this job's first weights; later jobs find the planes there
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the compiler does not count the DMAs)
         __syncthreads();
     }
     const u32x4* planes = reinterpret_cast<const u32x4*>(gk_lds) + lane;   // + ((local step * GB_PLANES + piece) * NTB + token block) * 64
     if (has_tile) {
-        // Groups of DEPTH units, no exit inside (the ring registers never move); every slice is a whole number of groups -- the host plans no other
-        // slices.  (A first build let a short last group run its requests and image writes with the arithmetic skipped: the image writes of such idle
-        // units -- the SAME bytes again -- made whole tiles of other waves come out wrong, differently from launch to launch, with every wait in place
-        // (profiles/r06_prompt_kslice.txt); unexplained, and avoided: nothing is ever written to an image that is not multiplied afterwards.)
-        for (int ug = u_lo; ug < u_hi; ug += DEPTH) {
-#pragma unroll
-        for (int k = 0; k < DEPTH; ++k) {
-            const int u = ug + k;
+        for (int u = u_lo; u < u_hi; ++u) {
             // the unit's bytes into the wave's image (the wave's own reads of the previous unit are complete: DS operations of a wave execute in order)
 #pragma unroll
-            for (int n = 0; n < NLD; ++n) *reinterpret_cast<u32x4*>(stage + (s_pk[n] & 0xFFFFu)) = wreg[k][n];
-            const int u_next = min(u + DEPTH, u_last);
+            for (int n = 0; n < NLD; ++n) *reinterpret_cast<u32x4*>(stage + (s_pk[n] & 0xFFFFu)) = wreg[n];
             __builtin_amdgcn_sched_barrier(0);
-            load_unit(wreg[k], u_next);
+            load_unit(wreg, u + 1);
             __builtin_amdgcn_sched_barrier(0);
             uint64_t sv[GB_PLANES][NTB];
             if constexpr (D::HAS_MIN) {
 #pragma unroll
                 for (int pl = 0; pl < GB_PLANES; ++pl)
 #pragma unroll
-                    for (int tb = 0; tb < NTB; ++tb) sv[pl][tb] = svr[k][pl][tb];
+                    for (int tb = 0; tb < NTB; ++tb) sv[pl][tb] = svr[pl][tb];
                 __builtin_amdgcn_sched_barrier(0);
-                load_sums(svr[k], u_next);   // (same queue, same distance, consumption order: behind the unit's weights)
+                load_sums(svr, min(u + 1, u_hi - 1));   // (same queue, same distance, consumption order: behind the unit's weights)
                 __builtin_amdgcn_sched_barrier(0);
             }
             const uint32_t uoff = (uint32_t)u * D::UB;
@@ -1800,7 +1786,6 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
         }
         // ---- this wave's rows: accumulator element e of lane (i = row of the tile, g) is token tb * 16 + 4 g + e; 1 / s; Y or this slice's partial sums ----
         f32x4 inv_t[NTB];
@@ -2106,7 +2091,7 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
             const int n_min = (units + max_units - 1) / max_units, n_cap = std::min(units, gb_split_rows((int)out_total));
             for (int n = n_min; n <= n_cap; ++n) {
                 const int ups = units / n;
-                if (units % n != 0 || ups % gk_depth<KD::SPU>() != 0 || (force_kn && n != force_kn)) continue;   // (equal slices of whole groups of units)
+                if (units % n != 0 || (force_kn && n != force_kn)) continue;   // (equal slices of whole units)
                 // rounds over the 256 CUs, folded into the workgroups (the planes are copied once): the fewest row groups per workgroup with which
                 // the whole grid -- ceil(wgx / jobs) x n -- is ONE round
                 int jobs = 1;
