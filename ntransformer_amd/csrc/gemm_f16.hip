@@ -1552,11 +1552,10 @@ __global__ __launch_bounds__(512) void gemm_quant_f16_small_kernel(const GemmSPa
 // and reads the B operands of a step from LDS.  Planes traffic = slice bytes per workgroup (Wo: 8 MB instead of 67); the slices' partial sums go to the
 // partial-sum area the K splits of the large kernel use ([slice][token][row]; summed in slice order by the launch that consumes the projection or by
 // reduce_splits_kernel), a launch with ONE slice writes Y itself.
-// ONE unit ahead, and a loop of one unit: deeper rings (two units of a K-quant, four of Q8_0, until now) were code before they were bandwidth.  Every launch
-// fetches its instructions anew, a loop of 16 unrolled steps cost each launch about a microsecond more than one of 8 (of 32: 2.5 more), the requests past
-// a slice's end fetched real bytes, and slices had to be whole numbers of groups.  8B at 16 tokens, us per launch, before -> now: Q4_K gate | up 25.9 -> 24.9,
-// Q | K | V 9.8 -> 8.9, Q6_K down 19.1 -> 16.2; eight layers of Q8_0 1220 -> 1095 us.
-// Smaller still loses: the unit's eight steps in a loop of four 846, of two 906 us for 32 layers' gate | up against 814.
+// ONE unit ahead, and a loop of one unit.  Deeper rings (two units of a K-quant, four of Q8_0, until now) measured slower, a microsecond a launch at the double depth, 2.5 at
+// four times: their requests past a slice's end fetched real bytes, slices had to be whole numbers of rings, and even with both mended two units lost to one (8 layers
+// of 8B Q4_K_M at 16 tokens 996 against 965 us).  8B at 16 tokens, us per launch, before -> now: Q4_K gate | up 25.9 -> 24.9, Q | K | V 9.8 -> 8.9, Q6_K down 19.1 -> 16.2;
+// eight layers of Q8_0 1220 -> 1095 us.  A smaller loop loses too: the unit's eight steps in a loop of four 846, of two 906 us for 32 layers' gate | up against 814.
 struct GemmKParams {
     GemmBSeg seg[GB_MAX_SEG];
     int nseg;
