@@ -118,8 +118,9 @@ __device__ __forceinline__ void direct_load_dword(uint32_t lds, const void* base
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %3, %1\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "s"(base), "s"(lds), "v"(off) : "memory");
 }
 
-// exp(x), x <= 0 and finite: 2^(x log2 e) with the rounding of the product made good
+// exp(x), x <= 0: 2^(x log2 e) with the rounding of the product made good; 0 from -200 on down to -inf, a NaN stays one
 __device__ __forceinline__ float exp_negative(float x) {
+    x = x < -200.0f ? -200.0f : x;
     const float t = x * 1.44269504f;
     const float rest = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t));
     const float r = __builtin_amdgcn_exp2f(t);
@@ -132,7 +133,6 @@ __device__ __forceinline__ float quad_max(float v) {
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-constexpr float kUnseen = -2.3e38f;      // a score below any that counts, and still finite times log2 e
 
 // VEC: query rows, results and gates on 16 bytes, sizes in fours
 template <int DK, int DV, bool VEC, bool BIASED>
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
         }
     }
     const bool sunk = (a.sink || a.sinks) && kh == 0;         // (one of a row's waves starts from the sink)
-    float mx = sunk ? (a.sinks ? fmaxf(a.sinks[head], kUnseen) : 0.0f) : kUnseen, l = sunk && g4 == 0 ? 1.0f : 0.0f;
+    float mx = sunk ? (a.sinks ? a.sinks[head] : 0.0f) : -INFINITY, l = sunk && g4 == 0 ? 1.0f : 0.0f;
     int unit = -100;                                          // acc counts in 2^(unit - 14)
     f4 acc[VT];
 #pragma unroll
@@ -266,14 +266,14 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const int j = j0 + 16 * (e >> 2) + 4 * g4 + (e & 3);
-                    if (!(j <= pos && (j >= lo || j < a.keep))) sv[e] = kUnseen;
+                    if (!(j <= pos && (j >= lo || j < a.keep))) sv[e] = -INFINITY;
                 }
             }
             const float mt = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
-            const float mn = fmaxf(mx, quad_max(mt));
+            const float mn = fmaxf(mx, quad_max(mt)), base = mn == -INFINITY ? 0.0f : mn;
             const int top = max(unit, step);
             if (__any(mn != mx) || top != unit) {             // (a maximum that stays leaves the sums as they are)
-                float corr = exp_negative(mx - mn);
+                float corr = exp_negative(mx - base);
                 l *= corr;
                 corr = ldexpf(corr, unit - top);
                 mx = mn;
@@ -285,8 +285,7 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
             float w[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float p = exp_negative(sv[e] - mn);
-                if (!clear && sv[e] == kUnseen) p = 0.0f;
+                const float p = exp_negative(sv[e] - base);
                 l += p;
                 w[e] = p * c14;
             }
@@ -342,7 +341,7 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
     }
     __syncthreads();
     if (kh > 0 || wrow >= n_rows) return;
-    const float m1 = sm[0], mm = fmaxf(mx, m1);               // a part's weight: exp(its maximum - the row's), over the row's sum
+    const float m1 = sm[0], mm = fmaxf(fmaxf(mx, m1), -3.4028235e38f);   // a part's weight: exp(its maximum - the row's), over the row's sum
     float w0 = exp_negative(mx - mm), w1 = exp_negative(m1 - mm);
     const float sum = fmaf(w1, sm[64], w0 * l), inv = sum > 0.0f ? a.out_scale / sum : 0.0f;
     w0 *= inv;

@@ -89,3 +89,15 @@ def test_keys_that_are_not_finite(what):
     k[40, 0, 3] = what
     got, want = attend(Lr.window_attention, q, k, v, H, 0), attend(window_f32, q, k, v, H, 0)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.nanmax(np.abs(got - want)) < 2e-5 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("low", [-np.inf, np.finfo(np.float32).min, -3e38])
+def test_scores_of_the_types_lowest_value(low):
+    """a bias of the lowest value on the nearest distances: rows that see nothing else weigh all of it alike (-inf: not at all), the others give it no weight"""
+    T, H, dn = 100, 2, 96
+    q, k, v = values(T, 0, H, 1, dn, 64, 8)
+    rel, bucket_of = np.array([[low] * H, [0.25] * H], np.float32), (np.arange(60) > 40).astype(np.int32)
+    got = attend(Lr.window_attention, q, k, v, 1, 0, rel=rel, bucket_of=bucket_of)
+    assert np.abs(got - attend(window_f32, q, k, v, 1, 0, rel=rel, bucket_of=bucket_of)).max() < 2e-5 * np.abs(v).max()
+    mean = np.cumsum(v.astype(np.float64), 0) / np.arange(1, T + 1)[:, None, None]
+    assert np.abs(got[:41] - (0.0 if low == -np.inf else mean[:41])).max() < 2e-5 * np.abs(v).max()
