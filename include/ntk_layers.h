@@ -211,8 +211,8 @@ size_t ntk_latent_attention_scratch(int T, int H, int vdim_or_rank, int nkeys);
 int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
                          int kv_rank, int rot_dim, int H, int dn, int dv, int shared, int pos0, int T, int key0, int window, float scale, float* scratch,
                          void* stream);
-/* ... with room for the visible keys and values as halves (ntk_prompt_attention_image_bytes() for the positions that a portion sees; 16-byte aligned; NULL: none): the expanded form of a
- * prompt's portion then multiplies on the half-precision matrix instructions, every 32-bit value as two halves */
+/* ... with room for the visible keys and values in pieces (ntk_prompt_attention_image_bytes() for the positions that a portion sees; 16-byte aligned; NULL: none): the expanded form of a
+ * prompt's portion then multiplies on the bfloat16 matrix instructions, every 32-bit value as the three bfloat16 values that add up to it; errors no larger than the 32-bit form's */
 int ntk_latent_attention_ex(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
                          int kv_rank, int rot_dim, int H, int dn, int dv, int shared, int pos0, int T, int key0, int window, float scale, float* scratch,
                          void* image, size_t image_bytes, void* stream);
@@ -302,7 +302,7 @@ typedef struct ntk_window_attention_desc {
 #define NTK_MASK_CHUNKS 1
 size_t ntk_window_attention_scratch(int T, int H, int maps, int dv, int nkeys);
 int ntk_window_attention(const ntk_window_attention_desc* d, void* stream);
-/* ... with room for the visible keys and values as halves (see ntk_latent_attention_ex) */
+/* ... with room for the visible keys and values in pieces (see ntk_latent_attention_ex) */
 int ntk_window_attention_ex(const ntk_window_attention_desc* d, void* image, size_t image_bytes, void* stream);
 
 /* ---- lightning_attention.hip -------------------------------------------------------------------------------------------------------

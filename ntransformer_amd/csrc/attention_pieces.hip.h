@@ -1,44 +1,56 @@
-// attention_half.hip.h -- attention of a portion of tokens over F32 keys and values on the half-precision matrix instructions: every 32-bit value goes in as two halves.
+// attention_pieces.hip.h -- attention of a portion of tokens over F32 keys and values on the bfloat16 matrix instructions: every 32-bit value goes in as three bfloat16 pieces.
 //
-// The form of attention_tile.hip.h multiplies in 32 bits, 256 products a cycle and CU; 1024 tokens of 16 heads (keys 192, values 128) took 110 us, three times what the products
-// need there.  A product of two 32-bit values as three of halves (the second halves' own product, 2^-24 of it, is left out) takes 3/8 of the matrix time.  Rows are scaled by
-// powers of two first, the first halves' products have accumulators of their own.  Error of a score of 128 / 192 entries against 64 bits, in 1e-7 of their size: 0.89 / 0.93, as 32-bit
-// products 1.03 / 1.25; of a sum of 1000 weighted values 1.2 and 2.7; of 64 entries 0.86 and 0.74, so keys of up to 64 entries keep the other form.
-// Two launches: attention_image_kernel leaves the visible keys and values of every key / value head as tiles of 32 positions, halves, rows swizzled and values transposed as LDS
-// holds them, once for the up to 32 workgroups that read a tile; attention_half_kernel copies them straight into LDS.
+// The form of attention_tile.hip.h multiplies in 32 bits, 256 products a cycle and CU; 1024 tokens of 16 heads (keys 192, values 128) take 102 us, three times what the products
+// need there.  A 32-bit value is the sum of three bfloat16 pieces (8 + 8 + 8 bits, and bfloat16 has its exponents: nothing is scaled, so no row, position or column loses by the size of
+// another); six products of pieces, all but those below 2^-25 of the value, take 3/8 of the matrix time.  The first pieces' products have accumulators of their own.  Error of a result,
+// 200 tokens behind 300, in 1e-7 of its norm: keys of 72 / 128 / 192 entries 2.5 / 2.6 / 2.7, as 32-bit products 3.9 / 4.6 / 5.3; with channels and positions that tower over the
+// others 5.2 / 4.6 / 3.9, as 32-bit products 10.8 / 9.1 / 7.8.  (Two halves with powers of two per row and tile took half the matrix time, 61 us where this takes 76; a range
+// of 2^15 within a tile cost bits there, 2^39 the results.)
+// Two launches: attention_image_kernel leaves the visible keys and values of every key / value head as tiles of 32 positions, pieces, rows swizzled and values transposed as LDS
+// holds them, once for the up to 32 workgroups that read a tile; attention_pieces_kernel copies them straight into LDS.
 // A workgroup owns 64 rows (a row = a token and one of the heads that share a key / value head): four waves of 16 rows, times two that take the tiles in turn.  Scores are formed
 // transposed (keys x rows), so that a lane's eight weights are the operand of the second product as they stand -- the order of a tile's 32 positions in it is
 // [4 g + r, 16 + 4 g + r] for lane group g, and the values' image has that order -- and maximum, sum and rescaling are one number a lane.
-// Bounds: the three phases of a pair of tiles one after the other -- scores (LDS reads, 24 KB a wave), softmax (vector instructions), weighted values -- 2.6 us a pair, and 8 us around
-// them.  Measured (us, both launches; the 32-bit form): latent, 1024 tokens, 16 heads, keys 192, values 128: 60 (110); 975 tokens behind 1024: 109 (240); window, 1024 tokens, 16
-// heads on 4, 128 + 128, capped scores, a sink, a gate: 68 (113); 150 tokens 25 and 24 (32 and 25).
+// Bounds: the three phases of a pair of tiles one after the other -- scores (matrix instructions, and LDS reads of 36 KB a wave), softmax (vector instructions), weighted values --, 3.9 us
+// a pair, and 8 us around them.  LDS holds one pair's keys: the next pair's are requested when all have formed their scores, and arrive behind softmax and weighted values.
+// Measured (us, both launches; the 32-bit form): latent, 1024 tokens, 16 heads, keys 192, values 128: 76 (102); 975 tokens behind 1024: 133 (225); window, 1024 tokens, 16
+// heads on 4, 128 + 128, capped scores, a sink, a gate: 80 (104); 150 tokens 21 and 21 (24 and 25).
 #pragma once
 #include "attention_tile.hip.h"
 #include "gemm_direct.hip.h"
 
 namespace ntk {
 
-struct HalfAttnArgs {
+struct PieceAttnArgs {
     TileAttnArgs t;
     uint8_t* image;                 // [G][tiles of the image][tile]
     int kept_tiles, first_tile, n_tiles, last_key;      // slot s of the image: tile s below kept_tiles, then first_tile + s - kept_tiles; keys t.key0 (0 for the kept ones) .. last_key
 };
-constexpr int kHalfRows = 64;
-template <int DK, int DV> struct HalfTile { static constexpr int K = 2 * 32 * DK * 2, V = 2 * 32 * DV * 2, BYTES = K + V + 512; };      // [K halves | V halves | factors of 32 keys, of 32 values, the values' step]
+constexpr int kPieceRows = 64;
+template <int DK, int DV> struct PieceTile { static constexpr int K = 3 * 32 * DK * 2, V = 3 * 32 * DV * 2, BYTES = K + V; };      // [a piece of K], three times, [a piece of V], three times
 
-// largest finite |v|, its exponent step: x * 2^-e has its largest in [2^14, 2^15) (e at least -125)
-__device__ __forceinline__ int half_step(float largest) { return max(((int)(__float_as_uint(largest) >> 23) & 255) - 127 - 14, -125); }
-__device__ __forceinline__ float finite_max(float m, float v) { const float a = fabsf(v); return a < INFINITY ? fmaxf(m, a) : m; }
-__device__ __forceinline__ void halves_of(const float (&v)[8], int e, uintx4_t (&out)[2]) { TileHalf2::convert(v, ldexpf(1.0f, -e), out); }
+// x = the sum of its pieces, nearest first (8 + 8 + 8 bits).  What is not finite, or rounds to an infinity, comes out of the products as a NaN, and its rows are formed again
+__device__ __forceinline__ void pieces_of(const float (&x)[8], uintx4_t (&out)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const uint32_t w = pack_bf16(a, b);
+            out[q][i] = w;
+            a -= __uint_as_float(w << 16);
+            b -= __uint_as_float(w & 0xffff0000u);
+        }
+    }
+}
 
 // grid (tiles, G), 256 threads: eight threads on a position's row.  Bound by its bytes.  VEC: rows and their parts on 16 bytes, sizes in fours
 template <int DK, int DV, bool VEC>
-__global__ __launch_bounds__(256) void attention_image_kernel(const HalfAttnArgs h) {
+__global__ __launch_bounds__(256) void attention_image_kernel(const PieceAttnArgs h) {
     const TileAttnArgs& a = h.t;
-    using Tile = HalfTile<DK, DV>;
+    using Tile = PieceTile<DK, DV>;
     constexpr int KP = DK / 64, VP = DV / 64;                 // pieces of eight entries a thread
-    __shared__ __attribute__((aligned(16))) uint16_t vt[2][DV * 32];
-    __shared__ float most[32];
+    __shared__ __attribute__((aligned(16))) uint16_t vt[3][DV * 32];
     const int slot = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, key = tid >> 3, c = tid & 7, dk = a.nA + a.nB;
     const int j = (slot < h.kept_tiles ? slot : h.first_tile + slot - h.kept_tiles) * 32 + key;
     const bool have = j >= a.key0 && j <= h.last_key;
@@ -47,7 +59,7 @@ __global__ __launch_bounds__(256) void attention_image_kernel(const HalfAttnArgs
     const float* pa = a.kA + (jr - a.key0) * a.ldA + (long long)g * a.hA;
     const float* pb = a.kB + jr * a.ldB - a.nA;
     const float* pv = a.v + (jr - a.key0) * a.ldV + (long long)g * a.hV;
-    float kx[KP][8], vx[VP][8], km = 0.0f, vm = 0.0f;
+    float kx[KP][8], vx[VP][8];
     // (no branch around a load: entries past the end re-read the last ones and are cleared)
     auto fetch = [&](float (&v)[8], int d0, int n, const float* first, const float* second, int cut) {
         if constexpr (VEC) {
@@ -62,37 +74,31 @@ __global__ __launch_bounds__(256) void attention_image_kernel(const HalfAttnArgs
             for (int i = 0; i < 8; ++i) { const int e = min(d0 + i, n - 1); v[i] = (e < cut ? first : second)[e]; }
         }
     };
-    auto settle = [&](float (&v)[8], int d0, int n, float& m) {
+    auto settle = [&](float (&v)[8], int d0, int n) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { v[i] = have && d0 + i < n ? v[i] : 0.0f; m = finite_max(m, v[i]); }
+        for (int i = 0; i < 8; ++i) v[i] = have && d0 + i < n ? v[i] : 0.0f;
     };
 #pragma unroll
     for (int p = 0; p < KP; ++p) fetch(kx[p], 8 * (c + 8 * p), dk, pa, pb, a.nA);
 #pragma unroll
     for (int p = 0; p < VP; ++p) fetch(vx[p], 8 * (c + 8 * p), a.nV, pv, pv, a.nV);
 #pragma unroll
-    for (int p = 0; p < KP; ++p) settle(kx[p], 8 * (c + 8 * p), dk, km);
-#pragma unroll
-    for (int p = 0; p < VP; ++p) settle(vx[p], 8 * (c + 8 * p), a.nV, vm);
-#pragma unroll
-    for (int m = 1; m < 8; m <<= 1) { km = fmaxf(km, __shfl_xor(km, m, 64)); vm = fmaxf(vm, __shfl_xor(vm, m, 64)); }
-    const int ke = half_step(km), ve = half_step(vm);
-    if (c == 0) most[key] = vm;
-#pragma unroll
     for (int p = 0; p < KP; ++p) {
-        uintx4_t u[2];
-        halves_of(kx[p], ke, u);
+        uintx4_t u[3];
+        settle(kx[p], 8 * (c + 8 * p), dk);
+        pieces_of(kx[p], u);
         const int at = key * DK * 2 + (((c + 8 * p) & ~7) | ((c ^ key) & 7)) * 16;
-        *reinterpret_cast<uintx4_t*>(img + at) = u[0];
-        *reinterpret_cast<uintx4_t*>(img + 32 * DK * 2 + at) = u[1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<uintx4_t*>(img + q * 32 * DK * 2 + at) = u[q];
     }
     const int grp = (key >> 2) & 3, ent = ((key >> 4) << 2) | (key & 3);
 #pragma unroll
     for (int p = 0; p < VP; ++p) {
-        uintx4_t u[2];
-        halves_of(vx[p], ve, u);
+        uintx4_t u[3];
+        settle(vx[p], 8 * (c + 8 * p), a.nV);
+        pieces_of(vx[p], u);
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < 3; ++q)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int d = 8 * (c + 8 * p) + i;
@@ -103,19 +109,6 @@ __global__ __launch_bounds__(256) void attention_image_kernel(const HalfAttnArgs
     const uintx4_t* s = reinterpret_cast<const uintx4_t*>(&vt[0][0]);
     uintx4_t* o = reinterpret_cast<uintx4_t*>(img + Tile::K);
     for (int i = tid; i < Tile::V / 16; i += 256) o[i] = s[i];
-    if (c == 0) {                                             // factors: 2^step of a key; 2^(step - the tile's largest) of a value
-        float top = 0.0f;
-        for (int i = 0; i < 32; ++i) top = fmaxf(top, most[i]);
-        float* f = reinterpret_cast<float*>(img + Tile::K + Tile::V);
-        f[key] = ldexpf(1.0f, ke);
-        f[32 + key] = ldexpf(1.0f, ve - half_step(top));
-        if (key == 0) reinterpret_cast<int*>(f)[64] = half_step(top);
-    }
-}
-
-__device__ __forceinline__ void direct_load_dword(uint32_t lds, const void* base, uint32_t off) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %3, %1\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "s"(base), "s"(lds), "v"(off) : "memory");
 }
 
 // exp(x), x <= 0: 2^(x log2 e) with the rounding of the product made good; 0 from -200 on down to -inf, a NaN stays one
@@ -126,6 +119,7 @@ __device__ __forceinline__ float exp_negative(float x) {
     const float r = __builtin_amdgcn_exp2f(t);
     return fmaf(r, rest * 0.693147181f, r);
 }
+__device__ __forceinline__ void direct_wait_reads() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }   // this wave's LDS reads are done, and so everywhere in the workgroup; requests stay under way
 // over the four lanes of a row (lane % 16)
 __device__ __forceinline__ float quad_max(float v) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -136,19 +130,17 @@ __device__ __forceinline__ float quad_max(float v) {
 
 // VEC: query rows, results and gates on 16 bytes, sizes in fours
 template <int DK, int DV, bool VEC, bool BIASED>
-__global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnArgs h) {
+__global__ __launch_bounds__(512, 2) void attention_pieces_kernel(const PieceAttnArgs h) {
     typedef float f4 __attribute__((ext_vector_type(4)));
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    using Tile = HalfTile<DK, DV>;
+    using Tile = PieceTile<DK, DV>;
     const TileAttnArgs& a = h.t;
     constexpr int KSTEP = DK / 32, VT = DV / 16, NK = Tile::K / 4096, NV = Tile::V / 4096;      // requests of 1 KB a wave
-    constexpr int AUX = 4 * Tile::K + 2 * Tile::V;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[AUX + 2 * 8 * 512];                   // keys [buffer][tile of a pair], values [tile of a pair], factors [buffer][wave]
-    static_assert(4 * (VT * 256 + 128) * 4 <= AUX, "the merge fits");
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * Tile::K + 2 * Tile::V];             // keys, then values, [tile of a pair]
+    static_assert(4 * (VT * 256 + 128) * 4 <= 2 * Tile::K, "the merge fits");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave & 3, kh = wave >> 2, i16 = lane & 15, g4 = lane >> 4;
-    const int R = a.H / a.G, n_rows = a.T * R, nx = (n_rows + kHalfRows - 1) / kHalfRows, dk = a.nA + a.nB;
+    const int R = a.H / a.G, n_rows = a.T * R, nx = (n_rows + kPieceRows - 1) / kPieceRows, dk = a.nA + a.nB;
     const int g = blockIdx.x % a.G, x = nx - 1 - blockIdx.x / a.G;      // the longest ranges first
-    const int row0 = x * kHalfRows, last = min(row0 + kHalfRows, n_rows) - 1;
+    const int row0 = x * kPieceRows, last = min(row0 + kPieceRows, n_rows) - 1;
     auto first_seen = [&](int p) { return a.window <= 0 ? 0 : a.chunks ? (p / a.window) * a.window : max(0, p - a.window + 1); };
     const int jlo = first_seen(a.pos0 + row0 / R), jhi = a.pos0 + last / R;
     // the tiles walked: 0 .. mine - 1 (positions that stay visible), then from `from` to the last
@@ -160,17 +152,18 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
     uint32_t lin[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) lin[i] = (uint32_t)(rw * 1024 + lane * 16 + i * 4096);
-    auto request = [&](uint32_t at, const uint8_t* from_, int n) {      // n KB for this wave of the four of a tile, 4 KB apart
+    auto request = [&](uint32_t at, const uint8_t* from_, auto n) {      // N KB for this wave of the four of a tile, 4 KB apart
+        constexpr int N = decltype(n)::value;
+        static_assert(N == 6 || N == 9, "tiles of 24 or 36 KB");
         direct_load4<4096>(at + rw * 1024, from_, lin[0], lin[1], lin[2], lin[3]);
-        if (n > 4) direct_load2<4096>(at + rw * 1024 + 16384, from_ + 16384, lin[0], lin[1]);
+        if constexpr (N == 6) direct_load2<4096>(at + rw * 1024 + 16384, from_ + 16384, lin[0], lin[1]);
+        else {
+            direct_load4<4096>(at + rw * 1024 + 16384, from_ + 16384, lin[0], lin[1], lin[2], lin[3]);
+            direct_load1(at + rw * 1024 + 32768, from_ + 32768, lin[0]);
+        }
     };
     auto request_keys = [&](int i) {
-        if (2 * i + kh >= n_walk) return;
-        const uint8_t* im = image_of(2 * i + kh);
-        request(lds0 + ((i & 1) * 2 + kh) * Tile::K, im, NK);
-        const uint32_t f = lds0 + AUX + ((i & 1) * 8 + wave) * 512;     // (every wave its own copy)
-        direct_load_dword(f, im + Tile::K + Tile::V, (uint32_t)lane * 4);
-        direct_load_dword(f + 256, im + Tile::K + Tile::V + 256, 0u);   // (the values' step, in every lane's place)
+        if (2 * i + kh < n_walk) request(lds0 + kh * Tile::K, image_of(2 * i + kh), std::integral_constant<int, NK>{});
     };
     request_keys(0);
     // this wave's rows, and the lane's
@@ -180,11 +173,10 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
     const int wave_lo = first_seen(wave_first), clear_lo = first_seen(max(wave_hi, 0)), clear_hi = wrow + 15 < n_rows ? wave_first : -1;     // tiles inside need no mask
     const float slope = a.slopes ? a.slopes[head] : 0.0f;
     // queries as operands: row i16, entries 32 s + 8 g4 ..
-    halfx8_t qh[KSTEP], ql[KSTEP];
-    float qf;
+    uintx4_t qp[KSTEP][3];
     {
         const float* q = a.q + (long long)tok * a.ldq + (long long)head * dk;
-        float v[KSTEP][8], m = 0.0f;
+        float v[KSTEP][8];
 #pragma unroll
         for (int s = 0; s < KSTEP; ++s) {
             const int d0 = 32 * s + 8 * g4;
@@ -200,22 +192,14 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
             }
         }
 #pragma unroll
-        for (int s = 0; s < KSTEP; ++s)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) { v[s][i] = 32 * s + 8 * g4 + i < dk ? v[s][i] : 0.0f; m = finite_max(m, v[s][i]); }
-        const int qe = half_step(quad_max(m));
-        qf = ldexpf(1.0f, qe);
-#pragma unroll
         for (int s = 0; s < KSTEP; ++s) {
-            uintx4_t u[2];
-            halves_of(v[s], qe, u);
-            qh[s] = bits_as<halfx8_t>(u[0]);
-            ql[s] = bits_as<halfx8_t>(u[1]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[s][i] = 32 * s + 8 * g4 + i < dk ? v[s][i] : 0.0f;
+            pieces_of(v[s], qp[s]);
         }
     }
     const bool sunk = (a.sink || a.sinks) && kh == 0;         // (one of a row's waves starts from the sink)
     float mx = sunk ? (a.sinks ? a.sinks[head] : 0.0f) : -INFINITY, l = sunk && g4 == 0 ? 1.0f : 0.0f;
-    int unit = -100;                                          // acc counts in 2^(unit - 14)
     f4 acc[VT];
 #pragma unroll
     for (int t = 0; t < VT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
@@ -224,45 +208,46 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
         const int n = 2 * i + kh;
         const bool there = n < n_walk, more = n + 2 < n_walk;
         direct_wait<0>();                                     // this pair's keys are there, the previous one's values used up
-        if (there) request(lds0 + 4 * Tile::K + kh * Tile::V, image_of(n) + Tile::K, NV);
-        request_keys(i + 1);
+        if (there) request(lds0 + 2 * Tile::K + kh * Tile::V, image_of(n) + Tile::K, std::integral_constant<int, NV>{});
         const int j0 = tile_of(n) * 32;
         const bool work = there && j0 <= wave_hi && (j0 + 31 >= wave_lo || j0 < a.keep);
-        halfx8_t ph, pl;
-        if (work) {
-            // ---- scores, transposed: 32 keys x 16 rows
-            const uint8_t* ks = lds + ((i & 1) * 2 + kh) * Tile::K;
-            f4 hi[2], lw[2];
+        // ---- scores, transposed: 32 keys x 16 rows.  The first pieces' products have accumulators of their own
+        f4 big[2], low[2][2];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) hi[u] = lw[u] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int u = 0; u < 2; ++u) big[u] = low[0][u] = low[1][u] = f4{0.f, 0.f, 0.f, 0.f};
+        if (work) {
+            const uint8_t* ks = lds + kh * Tile::K;
 #pragma unroll
             for (int s = 0; s < KSTEP; ++s) {
                 const int piece = 4 * s + g4, at = i16 * DK * 2 + ((piece & ~7) | ((piece ^ i16) & 7)) * 16;
-                halfx8_t k0[2], k1[2];
+                uintx4_t k[3][2];
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    k0[u] = *reinterpret_cast<const halfx8_t*>(ks + u * 16 * DK * 2 + at);
-                    k1[u] = *reinterpret_cast<const halfx8_t*>(ks + 32 * DK * 2 + u * 16 * DK * 2 + at);
-                }
+                for (int p = 0; p < 3; ++p)
 #pragma unroll
-                for (int u = 0; u < 2; ++u) hi[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0[u], qh[s], hi[u], 0, 0, 0);
+                    for (int u = 0; u < 2; ++u) k[p][u] = *reinterpret_cast<const uintx4_t*>(ks + p * 32 * DK * 2 + u * 16 * DK * 2 + at);
+                auto mul = [&](f4 (&to)[2], int kp, int qq) {
 #pragma unroll
-                for (int u = 0; u < 2; ++u) lw[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0[u], ql[s], lw[u], 0, 0, 0);
-#pragma unroll
-                for (int u = 0; u < 2; ++u) lw[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1[u], qh[s], lw[u], 0, 0, 0);
+                    for (int u = 0; u < 2; ++u) to[u] = TileBf16::mma(k[kp][u], qp[s][qq], to[u]);
+                };
+                mul(low[0], 0, 2);
+                mul(low[1], 1, 1);
+                mul(big, 0, 0);
+                mul(low[0], 2, 0);
+                mul(low[1], 0, 1);
+                mul(low[0], 1, 0);
             }
+        }
+        direct_wait_reads();                                  // everybody has used this pair's keys
+        request_keys(i + 1);
+        uintx4_t pp[3];
+        if (work) {
             // ---- online softmax: this lane's row, keys j0 + 16 u + 4 g4 + r
-            const float* fac = reinterpret_cast<const float*>(lds + AUX + ((i & 1) * 8 + wave) * 512);
-            const int step = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(fac)[64]);
             float sv[8];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const f4 kf = *reinterpret_cast<const f4*>(fac + 16 * u + 4 * g4);
+            for (int u = 0; u < 2; ++u)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sv[4 * u + r] = attention_score<BIASED>(a, (hi[u][r] + lw[u][r]) * kf[r] * qf, head, pos - (j0 + 16 * u + 4 * g4 + r), slope);
-            }
-            const bool clear = j0 >= clear_lo && j0 + 31 <= clear_hi;
-            if (!clear) {
+                for (int r = 0; r < 4; ++r) sv[4 * u + r] = attention_score<BIASED>(a, big[u][r] + (low[0][u][r] + low[1][u][r]), head, pos - (j0 + 16 * u + 4 * g4 + r), slope);
+            if (!(j0 >= clear_lo && j0 + 31 <= clear_hi)) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const int j = j0 + 16 * (e >> 2) + 4 * g4 + (e & 3);
@@ -271,65 +256,48 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
             }
             const float mt = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
             const float mn = fmaxf(mx, quad_max(mt)), base = mn == -INFINITY ? 0.0f : mn;
-            const int top = max(unit, step);
-            if (__any(mn != mx) || top != unit) {             // (a maximum that stays leaves the sums as they are)
-                float corr = exp_negative(mx - base);
+            if (__any(mn != mx)) {                            // (a maximum that stays leaves the sums as they are)
+                const float corr = exp_negative(mx - base);
                 l *= corr;
-                corr = ldexpf(corr, unit - top);
                 mx = mn;
-                unit = top;
 #pragma unroll
                 for (int t = 0; t < VT; ++t) acc[t] *= corr;
             }
-            const float c14 = ldexpf(1.0f, step - unit + 14);
             float w[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float p = exp_negative(sv[e] - base);
-                l += p;
-                w[e] = p * c14;
+                w[e] = exp_negative(sv[e] - base);
+                l += w[e];
             }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const f4 vf = *reinterpret_cast<const f4*>(fac + 32 + 16 * u + 4 * g4);
-#pragma unroll
-                for (int r = 0; r < 4; r += 2) {
-                    const floatx2_t y{w[4 * u + r] * vf[r], w[4 * u + r + 1] * vf[r + 1]};
-                    const half2_t b = __builtin_convertvector(y, half2_t);
-                    const half2_t c = __builtin_convertvector(y - __builtin_convertvector(b, floatx2_t), half2_t);
-                    ph[4 * u + r] = b[0]; ph[4 * u + r + 1] = b[1];
-                    pl[4 * u + r] = c[0]; pl[4 * u + r + 1] = c[1];
-                }
-            }
+            pieces_of(w, pp);
         }
-        if (more) direct_wait<NK + 2>(); else direct_wait<0>();
+        if (more) direct_wait<NK>(); else direct_wait<0>();   // the values are there
         if (work) {
-            // ---- weighted values, transposed: DV x 16 rows
-            const uint8_t* vs = lds + 4 * Tile::K + kh * Tile::V + i16 * 64 + ((g4 ^ (i16 >> 1)) & 3) * 16;
+            // ---- weighted values, transposed: DV x 16 rows; the smallest products first
+            const uint8_t* vs = lds + 2 * Tile::K + kh * Tile::V + i16 * 64 + ((g4 ^ (i16 >> 1)) & 3) * 16;
 #pragma unroll
             for (int t0 = 0; t0 < VT; t0 += 4) {
-                halfx8_t v0[4], v1[4];
+                uintx4_t v[3][4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    v0[t] = *reinterpret_cast<const halfx8_t*>(vs + (t0 + t) * 16 * 64);
-                    v1[t] = *reinterpret_cast<const halfx8_t*>(vs + DV * 64 + (t0 + t) * 16 * 64);
-                }
+                for (int p = 0; p < 3; ++p)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v1[t], ph, acc[t0 + t], 0, 0, 0);
+                    for (int t = 0; t < 4; ++t) v[p][t] = *reinterpret_cast<const uintx4_t*>(vs + p * DV * 64 + (t0 + t) * 16 * 64);
+                auto mul = [&](int vp, int q) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v0[t], pl, acc[t0 + t], 0, 0, 0);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v0[t], ph, acc[t0 + t], 0, 0, 0);
+                    for (int t = 0; t < 4; ++t) acc[t0 + t] = TileBf16::mma(v[vp][t], pp[q], acc[t0 + t]);
+                };
+                mul(2, 0);
+                mul(0, 2);
+                mul(1, 1);
+                mul(1, 0);
+                mul(0, 1);
+                mul(0, 0);
             }
         }
     }
     // ---- the two waves of sixteen rows meet: the second leaves (max, sum, vectors), the first adds them to its own and stores
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-#pragma unroll
-    for (int t = 0; t < VT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[t][r] = ldexpf(acc[t][r], unit - 14);
     __syncthreads();
     float* st = reinterpret_cast<float*>(lds) + rw * VT * 256 + lane * 4;                       // [wave][vectors], then [wave][max, sum]
     float* sm = reinterpret_cast<float*>(lds) + 4 * VT * 256 + rw * 128 + lane;
@@ -420,7 +388,7 @@ __global__ __launch_bounds__(512, 2) void attention_half_kernel(const HalfAttnAr
 }
 
 // the tiles that a portion's rows see
-static void half_attention_tiles(const TileAttnArgs& a, HalfAttnArgs& h) {
+static void piece_attention_tiles(const TileAttnArgs& a, PieceAttnArgs& h) {
     const int lo = a.window <= 0 ? 0 : a.chunks ? (a.pos0 / a.window) * a.window : std::max(0, a.pos0 - a.window + 1);
     // (a later row's range starts later: positions that stay visible lie ahead of the LAST row's range)
     const int end = a.pos0 + a.T - 1, hi_lo = a.window <= 0 ? 0 : a.chunks ? (end / a.window) * a.window : std::max(0, end - a.window + 1);
@@ -429,33 +397,34 @@ static void half_attention_tiles(const TileAttnArgs& a, HalfAttnArgs& h) {
     h.n_tiles = h.kept_tiles + end / 32 - h.first_tile + 1;
     h.last_key = end;
 }
-static size_t half_attention_bytes(int tiles, int G, int dk, int dv) {
+static size_t piece_attention_bytes(int tiles, int G, int dk, int dv) {
     if (dk <= 64 || dk > 192 || dv > 128) return 0;
-    return (size_t)G * tiles * HalfTile<192, 128>::BYTES;       // (keys of 128 entries on 16 bytes take two thirds)
+    return (size_t)G * tiles * (dk <= 128 ? PieceTile<128, 128>::BYTES : PieceTile<192, 128>::BYTES);
 }
 // false: not a portion for this form, or no room; nothing was launched
-static bool launch_attention_half(const TileAttnArgs& a, void* image, size_t bytes, hipStream_t s) {
+static bool launch_attention_pieces(const TileAttnArgs& a, void* image, size_t bytes, hipStream_t s) {
     const int dk = a.nA + a.nB;
-    HalfAttnArgs h{};
+    PieceAttnArgs h{};
     h.t = a;
-    half_attention_tiles(a, h);
-    const size_t need = half_attention_bytes(h.n_tiles, a.G, dk, a.nV);
+    piece_attention_tiles(a, h);
+    const size_t need = piece_attention_bytes(h.n_tiles, a.G, dk, a.nV);
     if (!need || !image || ((uintptr_t)image & 15) || bytes < need || a.G > 65535) return false;
     h.image = (uint8_t*)image;
     const bool biased = a.rel || a.slopes || a.softcap > 0.0f;
     const uintptr_t bits = (uintptr_t)a.kA | (uintptr_t)a.v | (a.nB ? (uintptr_t)a.kB : 0) | (uintptr_t)a.q | (uintptr_t)a.out | (a.gate && !a.head_gate ? (uintptr_t)a.gate : 0);
     const bool vec = !((a.nA | a.nB | a.nV | a.hA | a.hV | (int)a.ldA | (int)a.ldB | (int)a.ldV | a.ldq | a.ldo | (a.gate && !a.head_gate ? a.ldg : 0)) & 3) && !(bits & 15);
-    const dim3 tiles(h.n_tiles, a.G), grid((a.T * (a.H / a.G) + kHalfRows - 1) / kHalfRows * a.G);
-#define NTK_ATTENTION_HALF(DK, VEC)                                                                                             \
+    const dim3 tiles(h.n_tiles, a.G), grid((a.T * (a.H / a.G) + kPieceRows - 1) / kPieceRows * a.G);
+#define NTK_ATTENTION_PIECES(DK, VEC)                                                                                             \
     do {                                                                                                                          \
         hipLaunchKernelGGL((attention_image_kernel<DK, 128, VEC>), tiles, dim3(256), 0, s, h);                                    \
-        if (biased) hipLaunchKernelGGL((attention_half_kernel<DK, 128, VEC, true>), grid, dim3(512), 0, s, h);                    \
-        else hipLaunchKernelGGL((attention_half_kernel<DK, 128, VEC, false>), grid, dim3(512), 0, s, h);                          \
+        if (biased) hipLaunchKernelGGL((attention_pieces_kernel<DK, 128, VEC, true>), grid, dim3(512), 0, s, h);                    \
+        else hipLaunchKernelGGL((attention_pieces_kernel<DK, 128, VEC, false>), grid, dim3(512), 0, s, h);                          \
     } while (0)
-    if (dk <= 128 && vec) NTK_ATTENTION_HALF(128, true);
-    else if (vec) NTK_ATTENTION_HALF(192, true);
-    else NTK_ATTENTION_HALF(192, false);
-#undef NTK_ATTENTION_HALF
+    if (dk <= 128 && vec) NTK_ATTENTION_PIECES(128, true);
+    else if (dk <= 128) NTK_ATTENTION_PIECES(128, false);
+    else if (vec) NTK_ATTENTION_PIECES(192, true);
+    else NTK_ATTENTION_PIECES(192, false);
+#undef NTK_ATTENTION_PIECES
     return true;
 }
 

@@ -924,7 +924,7 @@ int LayerStackModel::alloc_buffers() {
     const int W = info_.width;
     chunk_ = std::min(opt_.max_context, 1024);
     size_t sc = 0, wsc = 0, lsc = 0, rsc = 0;
-    // what a portion's attention sees at most, as halves: the portion and a window ahead of it (and the positions that stay visible), or everything
+    // what a portion's attention sees at most, in pieces: the portion and a window ahead of it (and the positions that stay visible), or everything
     auto seen = [&](int window, int keep, int kv_heads, int dk, int dv) {
         const long long n = window > 0 ? std::min<long long>((long long)window + chunk_ + keep + 64, opt_.max_context) : opt_.max_context;
         image_bytes_ = std::max(image_bytes_, ntk_prompt_attention_image_bytes((int)n, kv_heads, dk, dv));

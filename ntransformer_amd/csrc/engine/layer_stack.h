@@ -383,7 +383,7 @@ private:
           *sgu_ = nullptr, *sact_ = nullptr, *sdn_ = nullptr, *scratch_ = nullptr, *xw_ = nullptr, *hn_ = nullptr, *hist_ = nullptr, *ff_ = nullptr, *zf_ = nullptr, *wscratch_ = nullptr, *lscratch_ = nullptr,
           *results_ = nullptr, *zq_ = nullptr, *gu2_ = nullptr, *rscratch_ = nullptr, *cv_ = nullptr, *vfirst_ = nullptr, *mid_ = nullptr, *rz_ = nullptr, *pscratch_ = nullptr;   // gated form: the layer results of the pass [runs + 1][chunk][width], decay pre-activations, [gate | up | residual gate]
     void *h1_16_ = nullptr, *h2_16_ = nullptr;   // a sublayer's input as bfloat16, in the place of (or beside) h1_ / h2_ where its products take it so
-    void* image_ = nullptr;                      // a portion's visible keys and values as halves (ntk_latent_attention_ex, ntk_window_attention_ex)
+    void* image_ = nullptr;                      // a portion's visible keys and values in pieces (ntk_latent_attention_ex, ntk_window_attention_ex)
     size_t image_bytes_ = 0;
     size_t pscratch_bytes_ = 0;                  // pscratch_: partial sums of products (ntk_dense_desc::scratch)
     size_t max_mid_ = 0;              // (post-norm form: the experts' activations of a token side by side)

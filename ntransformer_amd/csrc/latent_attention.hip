@@ -9,7 +9,7 @@
 // Expanded: a workgroup owns 16 tokens of one head and walks the visible keys in chunks of 64 -- lane = key for the scores (key slabs of 64 entries in
 // LDS), online softmax per row in F32, lane = value column for the weighted sum.  Shared: a workgroup owns 16 (token, head) rows and whole tiles of 32
 // cache rows; the tiles go round up to 128 workgroups and a second launch merges their (max, sum, vector) states.
-#include "attention_half.hip.h"
+#include "attention_pieces.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -511,7 +511,7 @@ size_t ntk_latent_attention_scratch(int T, int H, int vdim_or_rank, int nkeys) {
 }
 
 size_t ntk_prompt_attention_image_bytes(int positions, int kv_heads, int key_entries, int value_entries) {
-    return positions > 0 && kv_heads > 0 && key_entries > 0 && value_entries > 0 ? half_attention_bytes((positions - 1) / 32 + 3, kv_heads, key_entries, value_entries) : 0;
+    return positions > 0 && kv_heads > 0 && key_entries > 0 && value_entries > 0 ? piece_attention_bytes((positions - 1) / 32 + 3, kv_heads, key_entries, value_entries) : 0;
 }
 
 int ntk_latent_attention(float* out, int ldo, const float* q, int ldq, const float* K, int ldk, const float* V, int ldv, const float* cache, int row,
@@ -564,7 +564,7 @@ int ntk_latent_attention_ex(float* out, int ldo, const float* q, int ldq, const 
         TileAttnArgs t{};
         t.out = out; t.ldo = ldo; t.q = q; t.ldq = ldq; t.kA = a.kA; t.ldA = a.ldA; t.nA = a.nA; t.hA = a.hA; t.kB = a.kB; t.ldB = a.ldB; t.nB = a.nB;
         t.v = a.v; t.ldV = a.ldV; t.nV = a.nV; t.hV = a.hV; t.key0 = key0; t.H = H; t.G = H; t.pos0 = pos0; t.T = T; t.window = window; t.scale = scale; t.out_scale = 1.0f;
-        if (!launch_attention_half(t, image, image_bytes, s)) launch_attention_tile(t, s);
+        if (!launch_attention_pieces(t, image, image_bytes, s)) launch_attention_tile(t, s);
         return last_launch_status();
     }
     const int DKP = (a.nA + a.nB + 3) & ~3;

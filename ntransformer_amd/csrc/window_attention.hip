@@ -12,7 +12,7 @@
 // in LDS), online softmax per row and map, lane = value column for the weighted sums (the value slab is loaded once for both maps).  When few rows
 // face many keys (decoding), the chunks go round `splits` workgroups and a second launch merges their (max, sum, vector) states.
 #include <algorithm>
-#include "attention_half.hip.h"
+#include "attention_pieces.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -631,7 +631,7 @@ int ntk_window_attention_ex(const ntk_window_attention_desc* d, void* image, siz
         t.v = a.cache + (long long)a.G * a.dn; t.ldV = a.row; t.nV = a.dv; t.hV = a.dv; t.H = a.H; t.G = a.G; t.pos0 = a.pos0; t.T = a.T;
         t.window = a.window; t.chunks = a.chunks; t.keep = a.keep; t.scale = a.scale; t.softcap = a.softcap; t.out_scale = a.out_scale; t.sink = a.sink; t.sinks = a.sinks;
         t.slopes = a.slopes; t.rel = a.rel; t.bucket_of = a.bucket_of; t.n_dist = a.n_dist; t.gate = a.gate; t.ldg = a.ldg; t.head_gate = a.head_gate;
-        if (!launch_attention_half(t, image, image_bytes, s)) launch_attention_tile(t, s);
+        if (!launch_attention_pieces(t, image, image_bytes, s)) launch_attention_tile(t, s);
         return last_launch_status();
     }
     const int R = d->H / d->G;

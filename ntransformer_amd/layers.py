@@ -315,7 +315,7 @@ def latent_prepare(kv: np.ndarray, norm_w: np.ndarray, eps: float, kv_rank: int,
 
 def latent_attention(q: np.ndarray, cache: np.ndarray, kv_rank: int, rot_dim: int, heads: int, pos0: int, window: int, scale: float,
                      K: Optional[np.ndarray] = None, V: Optional[np.ndarray] = None, key0: int = 0, halves: bool = False) -> np.ndarray:
-    """halves: with room for the keys and values as halves; expanded form when K [nkeys, H * dn] and V [nkeys, H * dv] are given (q [T, H * (dn + dr)]), else the shared form (q [T, H * (R + dr)])"""
+    """halves: with room for the keys and values in pieces (ntk_*_attention_ex); expanded form when K [nkeys, H * dn] and V [nkeys, H * dv] are given (q [T, H * (dn + dr)]), else the shared form (q [T, H * (R + dr)])"""
     L = _bind()
     T, row = q.shape[0], kv_rank + rot_dim
     qb, cb = _f(q), _f(cache)
@@ -492,7 +492,7 @@ def window_attention(q: np.ndarray, cache: np.ndarray, H: int, G: int, maps: int
                      sub_norm: bool = False, eps: float = 1e-6, out_scale: float = 1.0, split: bool = True, rel: Optional[np.ndarray] = None,
                      bucket_of: Optional[np.ndarray] = None, chunks: bool = False, softcap: float = 0.0, sink: bool = False, gate: Optional[np.ndarray] = None,
                      keep_first: int = 0, sinks: Optional[np.ndarray] = None, head_gate: bool = False, slopes: Optional[np.ndarray] = None, halves: bool = False) -> np.ndarray:
-    """halves: with room for the keys and values as halves; q [T, H * maps * dn] (rotated), cache rows [G][maps][dn] keys | [G][dv] values; split: long key ranges of few rows may be cut into merged parts;
+    """halves: with room for the keys and values in pieces (ntk_*_attention_ex); q [T, H * maps * dn] (rotated), cache rows [G][maps][dn] keys | [G][dv] values; split: long key ranges of few rows may be cut into merged parts;
     rel [buckets, H] with bucket_of [distances]: a bias by distance on the scaled score; keep_first: positions that stay visible beside the window;
     sinks [H]: the sink's score per head; gate [T, H * dv], or [T, H] with head_gate; slopes [H]: slopes[h] * distance comes off the scaled score"""
     L = _bind()

@@ -1,4 +1,4 @@
-"""The prompt attention on half-precision matrix instructions (csrc/attention_half.hip.h): everything that is asked of the 32-bit form, with room for the halves, then the edges of its own tiles
+"""The prompt attention on bfloat16 matrix instructions (csrc/attention_pieces.hip.h): everything that is asked of the 32-bit form, with room for the pieces, then the edges of its own tiles
 (64 rows, pairs of 32 positions, positions that stay visible ahead of a window) and its error beside the 32-bit form's."""
 import functools
 
@@ -51,7 +51,7 @@ def test_no_further_from_float64_than_the_32_bit_form(dn, kind):
     scale = dn ** -0.5 * (0.05 if kind == "towering" else 1.0)
     want = reference(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), pos0, scale)
     err = [np.linalg.norm(attend(f, q, k, v, H, pos0, scale=scale) - want) for f in (Lr.window_attention, window_f32)]
-    print(dn, kind, "error as halves %.3g, in 32 bits %.3g" % tuple(e / np.linalg.norm(want) for e in err))
+    print(dn, kind, "error as pieces %.3g, in 32 bits %.3g" % tuple(e / np.linalg.norm(want) for e in err))
     assert err[0] <= 1.03 * err[1]
 
 
@@ -89,6 +89,46 @@ def test_keys_that_are_not_finite(what):
     k[40, 0, 3] = what
     got, want = attend(Lr.window_attention, q, k, v, H, 0), attend(window_f32, q, k, v, H, 0)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.nanmax(np.abs(got - want)) < 2e-5 * np.abs(v).max()
+
+
+# ... and with two heads a key: from 64 rows on such portions take this form whatever they see
+@pytest.mark.parametrize("T,pos0,H,G,dn,dv", [(32, 0, 2, 1, 65, 1), (33, 95, 4, 2, 100, 128), (130, 1, 6, 3, 72, 33), (96, 160, 32, 16, 191, 64), (9, 40, 8, 1, 128, 100)])
+@pytest.mark.parametrize("window,keep,chunks", [(0, 0, False), (1, 0, False), (33, 0, False), (70, 40, False), (20, 100, False), (64, 0, True), (45, 0, True)])
+def test_edges_with_heads_that_share_keys(T, pos0, H, G, dn, dv, window, keep, chunks):
+    test_edges_of_rows_tiles_and_windows(T, pos0, H, G, dn, dv, window, keep, chunks)
+
+
+@pytest.mark.parametrize("power", [20, 40, 100])
+@pytest.mark.parametrize("kind", ["later", "left of the window", "earlier, without weight", "leading rows", "value columns", "query and key channels"])
+@pytest.mark.parametrize("dn", [128, 192])
+def test_every_row_at_the_error_of_what_it_sees(kind, power, dn):
+    """Sizes that differ by 2^power within a tile: between positions, seen by a row or not, between columns of the values, between channels of queries and keys.  Every row's error over sum(weight |value|)
+    of that row, column by column: the largest is no more than 1.5 of the 32-bit form's largest (two of 30000 numbers of the same distribution)."""
+    T, H, pos0, window = 120, 2, 70, 0
+    q, k, v = values(T, pos0, H, 1, dn, 128, power + dn)
+    big = np.float32(2.0 ** power)
+    if kind == "later":
+        v[pos0 + 40] *= big                     # positions pos0 + 32 .. 39 share its tile, those behind it see it
+        v[pos0 + T - 1] *= big
+    elif kind == "left of the window":
+        window = 50
+        v[[24, 61, 90, 125]] *= big
+    elif kind == "earlier, without weight":     # seen by all, scores of about -150 and lower
+        k[[3, 80]], q[:, :, 0] = 0.0, 1.0
+        k[[3, 80], :, 0] = -150.0 * dn ** 0.5
+        v[[3, 80]] *= big
+    elif kind == "leading rows":
+        v[:100] /= big
+    elif kind == "value columns":
+        v[:, :, ::3] *= big
+    else:
+        s = np.exp2(np.random.default_rng(power).integers(-(power // 2), power // 2, dn)).astype(np.float32)
+        q, k = (q * s).astype(np.float32), (k / s).astype(np.float32)
+    f64 = lambda a: a.astype(np.float64)
+    want, size = (reference(f64(q), f64(k), f64(x), pos0, dn ** -0.5, window) for x in (v, np.abs(v)))
+    err = [(np.abs(attend(f, q, k, v, 1, pos0, window=window) - want) / size).max() for f in (Lr.window_attention, window_f32)]
+    print(kind, power, dn, "as pieces %.3g, in 32 bits %.3g" % tuple(err))
+    assert err[0] <= 1.5 * err[1]
 
 
 @pytest.mark.parametrize("low", [-np.inf, np.finfo(np.float32).min, -3e38])
