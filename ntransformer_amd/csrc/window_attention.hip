@@ -474,7 +474,7 @@ __global__ __launch_bounds__(256) void window_attention_few_kernel(const WinArgs
             y[c] = 0.0f;
             if (c < 2)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) if (w[i] != 0.0f) y[c] = fmaf(w[i], part[i][r][64 * c + lane], y[c]);
+                for (int i = 0; i < 4; ++i) y[c] = fmaf(w[i], part[i][r][64 * c + lane], y[c]);      // (no weight does not make a NaN or an infinity a number: 0 * v, as for a key)
         }
         const int h = g * R + r;
         if (a.splits > 1) {

@@ -56,3 +56,36 @@ def test_only_visible_positions_matter(what):
     bad = np.zeros(got.shape, bool)
     bad[1, :2, 3] = True
     assert np.array_equal(~np.isfinite(got), bad)
+
+
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("pos0", [20, 48, 400, 1500])
+@pytest.mark.parametrize("kind", ["query", "every key", "last key", "key alone in its sixteen", "value without weight"])
+@pytest.mark.parametrize("sink", [None, -1.0])
+def test_what_is_not_a_number_stays_one(kind, pos0, split, sink):
+    """a query or a visible key of NaN makes a head's results NaN (no row of zeros), as an infinite value does whose weight has underflowed (0 * inf)"""
+    H, G, dn, dv = 4, 2, 64, 64
+    q, k, v = values(1, pos0, H, G, dn, dv, 3)
+    bad = np.zeros((1, H, dv), bool)
+    bad[0, :2] = True
+    if kind == "query":
+        q[0, 1, 5] = np.nan
+        bad[0, 0] = False
+    elif kind == "every key":
+        k[:, 0, 5] = np.nan
+    elif kind == "last key":
+        k[pos0, 0, 5] = np.nan
+    elif kind == "key alone in its sixteen":
+        pos0 = pos0 // 16 * 16                  # the token's own key begins a group of sixteen
+        k, v = k[:pos0 + 1], v[:pos0 + 1]
+        k[pos0, 0, 5] = np.nan
+    else:
+        q[:, :, 0], k[3, 0], k[3, 0, 0] = 1.0, 0.0, -8000.0
+        v[3, 0, 7] = np.inf
+        bad[:] = False
+        bad[0, :2, 7] = True
+    cache = np.concatenate([k.reshape(k.shape[0], -1), v.reshape(v.shape[0], -1)], 1)
+    kw = {"sinks": np.full(H, sink, np.float32)} if sink is not None else {}
+    got = Lr.window_attention(q.reshape(1, -1), cache, H, G, 1, dn, dv, pos0, 0, 0.125, split=split, **kw).reshape(1, H, dv)
+    assert np.array_equal(np.isnan(got), bad)
+    assert np.isfinite(got[~bad]).all()
