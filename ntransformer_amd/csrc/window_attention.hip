@@ -368,8 +368,8 @@ __global__ __launch_bounds__(256) void window_attention_kernel(const WinArgs a) 
 // ---- a few tokens (decoding): one map, heads of up to 128 + 128 entries on 16 bytes
 // A workgroup owns a token and one key / value head (and every `splits`-th chunk of 64 keys): the keys AND values of a chunk are requested together, ahead of the first product, a wave
 // takes sixteen of them -- sixteen lanes a key for the scores of all the heads that share it, 32 lanes a value row for the sums -- and keeps an online softmax of its own; the
-// four waves meet in LDS.  What bounds it is the one round trip to the cache rows: a decoded token of 16 heads on 4 (128 + 128) behind 40 positions 20.5 us in the form above (a key slab, a
-// value slab and two barriers each, one after the other), 11.4 us here.  Up to four chunks stay in one workgroup (no launch that merges).
+// four waves meet in LDS.  What bounds it is the one round trip to the cache rows: a decoded token of 16 heads on 4 (128 + 128) behind 40 positions 14.9 us in the form above (a key slab, a
+// value slab and two barriers each, one after the other), 7.3 us here.
 constexpr int kFewTokens = 8, kFewChunk = 64;
 template <int RM>
 __global__ __launch_bounds__(256) void window_attention_few_kernel(const WinArgs a) {
@@ -635,10 +635,16 @@ int ntk_window_attention_ex(const ntk_window_attention_desc* d, void* image, siz
         return last_launch_status();
     }
     const int R = d->H / d->G;
-    if (d->maps == 1 && d->T <= kFewTokens && R <= 8 && d->dn <= 128 && d->dv <= 128 && !((d->dn | d->dv | d->row | d->ldq) & 3) && !(((uintptr_t)d->cache | (uintptr_t)d->q) & 15)) {
-        // (the scratch holds 4096 parts)
-        const int chunks = (window_keys(d->pos0, d->T, d->window, a.chunks, a.keep) + kFewChunk - 1) / kFewChunk;
-        a.splits = d->scratch && chunks > 4 ? std::max(1, std::min(std::min(chunks, 64), std::min(4096 / (d->T * d->H), 512 / (d->T * d->G)))) : 1;
+    // (eight tokens of eight heads a key fill the four tiles of sixteen rows of the form below, which reads a key once for all of them: with 32 / 64 workgroups of a part ahead from 2048 / 256
+    // keys on -- 32 heads on 4 behind 1024 / 4096 keys 22.6 and 22.0 / 61.2 and 63.0 us here, 64 on 8 behind 320 / 4096 20.6 and 21.9 / 104.6 and 114.5)
+    const int chunks = (window_keys(d->pos0, d->T, d->window, a.chunks, a.keep) + kFewChunk - 1) / kFewChunk;
+    const bool full = d->T <= kFewTokens && d->T * R > 48 && chunks > (d->T * d->G >= 64 ? 4 : d->T * d->G >= 32 ? 32 : 1 << 30);
+    if (!full && d->maps == 1 && d->T <= kFewTokens && R <= 8 && d->dn <= 128 && d->dv <= 128 && !((d->dn | d->dv | d->row | d->ldq) & 3) && !(((uintptr_t)d->cache | (uintptr_t)d->q) & 15)) {
+        // Parts (the scratch holds 4096): a chunk after another in one workgroup takes 1.5 us with one head a key, 3.5 with four, 6.3 with eight, the merge 3.  us at 64 / 128 / 256 / 1024
+        // keys, one token, the form below -> in one part up to 256 keys -> so: 16 heads on 4 16.6 / 26.8 / 18.9 / 21.9 -> 7.7 / 11.4 / 19.1 / 12.2 -> 7.3 / 10.4 / 10.5 / 11.8; 8 on 1
+        // 16.5 / 26.6 / 19.1 / 21.9 -> 12.3 / 18.9 / 31.5 / 16.5 -> 11.6 / 14.4 / 14.4 / 15.8; 16 of their own (64 + 64) 9.6 / 15.7 / 12.8 / 13.7 -> 4.5 / 6.1 / 9.3 / 7.4 -> 4.2 / 5.8 /
+        // 7.1 / 7.2.  With eight heads a key one workgroup a CU is enough: 512 parts of 8 tokens of 8 heads behind 4096 keys took 36.5, 256 take 26.4.
+        a.splits = d->scratch && chunks > (R > 2 ? 1 : 2) ? std::max(1, std::min(std::min(chunks, 64), std::min(4096 / (d->T * d->H), (R > 4 ? 256 : 512) / (d->T * d->G)))) : 1;
         const dim3 few(d->G, d->T, a.splits);
         if (R <= 1) hipLaunchKernelGGL(window_attention_few_kernel<1>, few, dim3(256), 0, s, a);
         else if (R <= 2) hipLaunchKernelGGL(window_attention_few_kernel<2>, few, dim3(256), 0, s, a);

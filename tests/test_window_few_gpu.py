@@ -46,6 +46,13 @@ def test_few_tokens(T, pos0, H, G, dn, dv, option):
         assert np.abs(got - want).max() < 2e-5 * max(np.abs(v).max(), np.abs(want).max()), split
 
 
+# two chunks and the first keys of a third, with more and fewer heads a key; eight tokens of eight heads a key on either side of 256 and 2048 keys
+@pytest.mark.parametrize("T,pos0,H,G,dn,dv", [(1, 64, 8, 1, 128, 128), (1, 127, 4, 1, 128, 64), (3, 125, 6, 2, 64, 64), (1, 127, 4, 2, 64, 64), (1, 128, 4, 4, 64, 64), (2, 128, 4, 2, 64, 64),
+                                              (8, 248, 64, 8, 64, 64), (8, 249, 64, 8, 64, 64), (7, 300, 56, 8, 64, 64), (8, 2040, 32, 4, 64, 64), (8, 2041, 32, 4, 64, 64)])
+def test_where_the_keys_are_cut(T, pos0, H, G, dn, dv):
+    test_few_tokens(T, pos0, H, G, dn, dv, "cap_sink")
+
+
 @pytest.mark.parametrize("what", [np.nan, np.inf])
 def test_only_visible_positions_matter(what):
     T, pos0, H, G, dn, dv = 2, 90, 4, 2, 64, 64
