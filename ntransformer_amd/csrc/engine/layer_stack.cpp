@@ -63,6 +63,7 @@ LayerStackModel::~LayerStackModel() {
     for (void* p : allocs_) nt_hip_free(p);
     if (logits_) nt_hip_free(logits_);
     if (capture_buf_) nt_hip_free(capture_buf_);
+    if (image_) nt_hip_free(image_);
     if (h_stage_) nt_hip_free_host(h_stage_);
 }
 
@@ -1012,7 +1013,6 @@ int LayerStackModel::alloc_buffers() {
     // four pieces of a whole pass's rows, and no less than sixteen of a short one's
     pscratch_bytes_ = std::max<size_t>(4 * C * W, (size_t)1 << 22) * sizeof(float);
     ok = ok && fl(&pscratch_, pscratch_bytes_ / sizeof(float));
-    if (image_bytes_ && !(image_ = dev_alloc(image_bytes_))) image_bytes_ = 0;      // (a long context may not leave the room: the attention has a form without)
     if (wdtype_ == NTK_DT_BF16) ok = ok && (h1_16_ = dev_alloc(C * W * 2)) && (h2_16_ = dev_alloc(C * W * 2));
     if (max_mid_ > 0) ok = ok && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_);
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
@@ -1044,7 +1044,22 @@ int LayerStackModel::alloc_buffers() {
             if (!r.conv) return fail(NTK_E_NOMEM, "out of device memory (state)");
         }
     }
+    // behind everything that the model cannot run without, and no more than a quarter of what is left: the attention has a form without
+    size_t left = 0, total = 0;
+    if (image_bytes_ && ntk_device_mem_info(&left, &total) == NTK_OK && image_bytes_ <= left / 4) image_ = nt_hip_malloc(image_bytes_);
+    if (!image_) image_bytes_ = 0;
     return NTK_OK;
+}
+
+// an allocation during a run: it goes ahead of the attention's image
+void* LayerStackModel::late_alloc(size_t bytes) {
+    void* p = nt_hip_malloc(bytes);
+    if (p || !image_) return p;
+    ntk_stream_synchronize(stream_);
+    nt_hip_free(image_);
+    image_ = nullptr;
+    image_bytes_ = 0;
+    return nt_hip_malloc(bytes);
 }
 
 // ------------------------------------------------------------------------------------------------------------------------ slots
@@ -1675,7 +1690,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         if (ntk_stream_synchronize(stream_) != NTK_OK) return nullptr;
         if (logits_) nt_hip_free(logits_);
         logits_rows_ = need;
-        logits_ = (float*)nt_hip_malloc(logits_rows_ * (size_t)info_.vocab * sizeof(float));
+        logits_ = (float*)late_alloc(logits_rows_ * (size_t)info_.vocab * sizeof(float));
         if (!logits_) { logits_rows_ = 0; err_ = "out of device memory (logits)"; return nullptr; }
     }
     if (capture_) {
@@ -1684,7 +1699,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         if (cf > capture_floats_) {
             ntk_stream_synchronize(stream_);
             if (capture_buf_) nt_hip_free(capture_buf_);
-            capture_buf_ = (float*)nt_hip_malloc(cf * sizeof(float));
+            capture_buf_ = (float*)late_alloc(cf * sizeof(float));
             capture_floats_ = capture_buf_ ? cf : 0;
             if (!capture_buf_) { err_ = "out of device memory (capture)"; return nullptr; }
         }

@@ -4,6 +4,7 @@ configuration and random bf16-representable weights, writes them as a model fold
 function, slot cache and kernels); the operator tests call include/ntk_layers.h directly.
 
 Error measure: rms of the difference over rms of the reference.  float32 mode is held to 2e-4 (observed ~1e-6), bfloat16 mode to 4e-2."""
+import ctypes as C
 import json
 import math
 import os
@@ -334,6 +335,45 @@ def test_prefill_against_token_by_token_and_portions(tmp_path, dtype):
     assert np.max(np.sqrt(np.mean((cut - ref) ** 2, axis=1)) / np.sqrt(np.mean(ref ** 2))) < 3 * TOL[dtype]
     if dtype == "float32":
         assert rel(cut, whole) < 1e-5 and rel(one, whole) < 1e-5
+
+
+def test_a_folder_loads_where_all_but_the_attentions_image_fits(tmp_path):
+    """the room for a prompt's keys and values in pieces is optional: it comes behind every buffer that the model cannot run without, caches included"""
+    from ntransformer_amd import _lib
+    L = _lib.lib()
+    L.ntk_debug_malloc_budget.argtypes, L.ntk_debug_malloc_budget.restype = [C.c_longlong], None
+    L.ntk_prompt_attention_image_bytes.argtypes, L.ntk_prompt_attention_image_bytes.restype = [C.c_int] * 4, C.c_size_t
+    cfg = O.small_config(layers=("latent_attention", "latent_attention"), dim=72)
+    folder, w = make(tmp_path, cfg, seed=8)
+    toks = tokens_for(cfg, 200, seed=9)
+    ref = O.forward(cfg, w, toks)
+    image = L.ntk_prompt_attention_image_bytes(512, cfg["layers"][0]["mixer"]["heads"], 72 + 8, 24)
+    assert image > 1 << 20
+    whole = 1 << 28
+    try:
+        L.ntk_debug_malloc_budget(whole)
+        e = engine_for(folder)
+        left, held = 0, []
+        for bit in range(28, -1, -1):          # what the load has left of the budget, to the byte
+            p = L.nt_hip_malloc(1 << bit)
+            if p:
+                left += 1 << bit
+                held.append(p)
+        for p in held:
+            L.nt_hip_free(p)
+        L.ntk_debug_malloc_budget(-1)
+        s = e.seq_acquire()
+        full = e.seq_forward(s, toks)
+        e.close()
+        for budget in (whole - left - image + (1 << 19), whole - left - 1):      # (the logits' buffer is allocated by the first pass)
+            L.ntk_debug_malloc_budget(budget)
+            e = engine_for(folder)
+            s = e.seq_acquire()
+            got = e.seq_forward(s, toks)
+            e.close()
+            assert rel(got, ref) < TOL["float32"] and rel(got, full) < 1e-5
+    finally:
+        L.ntk_debug_malloc_budget(-1)
 
 
 def test_wanted_places_only(tmp_path):
