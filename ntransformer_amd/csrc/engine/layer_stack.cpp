@@ -1213,7 +1213,7 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
                                  int full_x, const void* h16, const float* norm_w) {
     const int W = info_.width;
     ntk_dense_desc d{};
-    if (h16 && !full_x && rounded(ex.gate_up, rows) && rounded(ex.down, rows)) {
+    if (h16 && !full_x && rounded(ex, rows)) {
         ntk_direct_desc e{h16, W, rows / top, act, ex.ff};
         d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype; d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top;
         d.T = rows; d.N = ex.in_rows(); d.K = W;
@@ -1311,7 +1311,7 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
         return ntk_moe_few(&d, stream_);
     }
     LS_TRY(ntk_moe_group(offsets_, order_, where_, ids_, T, M.top, choices, stream_));     // (identity experts come last: rows behind offsets_[experts], which no product visits)
-    if (!h16 && T > ntk_dense_few_rows() && rounded(M.routed.gate_up, T)) {      // (rounded once for the chosen and the shared units)
+    if (!h16 && rounded(M, T)) {      // (rounded once for the chosen and the shared units)
         LS_TRY(ntk_round_rows(h2_16_, W, h, W, T, W, stream_));
         h16 = h2_16_;
     }
@@ -1332,7 +1332,7 @@ int LayerStackModel::run_dense_ff(const StackLayer& L, int T) {
 
 // the dense gated unit (the experts' unit with one member, clipped or plain): gate and up in one product (decoding: the activation inside its launch), down -> ff_
 int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16, const float* norm_w) {
-    if (!h16 && rounded(L.cff.gate_up, T)) {
+    if (!h16 && rounded(L.cff, T)) {
         LS_TRY(ntk_round_rows(h2_16_, info_.width, h, info_.width, T, info_.width, stream_));
         h16 = h2_16_;
     }
@@ -1404,8 +1404,7 @@ int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot,
         owed_ = Owed{ff_, L.norm2b};
         return NTK_OK;
     }
-    // (the down product takes the activations as the first one leaves them: both or none)
-    if (rounded(L.cff.down, T)) LS_TRY(seam_for(L.cff.gate_up, L.norm2, h2_, h2_16_, T, &h16));
+    if (rounded(L.cff, T)) LS_TRY(seam_for(L.cff.gate_up, L.norm2, h2_, h2_16_, T, &h16));
     else { h16 = nullptr; LS_TRY(rms_seam(L.norm2, h2_, T)); }
     LS_TRY(run_unit_ff(L, h2_, T, h16));
     owed_ = Owed{ff_, L.norm2b};
@@ -1414,6 +1413,10 @@ int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot,
 
 // T rows of bfloat16 activations go through w as they lie
 bool LayerStackModel::rounded(const DenseW& w, int T) const { return h1_16_ && w.dtype == NTK_DT_BF16 && ntk_dense_direct_takes(w.dtype, T, T, (int)w.out_f, (int)w.in_f) != 0; }
+// ... and through a unit: its down product takes the activations as the first one leaves them, so both products take such rows or none does
+bool LayerStackModel::rounded(const GatedExperts& ex, int rows) const { return rounded(ex.gate_up, rows) && rounded(ex.down, rows); }
+// ... and through some unit of a mixture
+bool LayerStackModel::rounded(const MoeFeedForward& M, int T) const { return T > ntk_dense_few_rows() && (rounded(M.routed, T * M.top) || (M.has_shared && rounded(M.shared, T))); }
 
 // every product of the model: with room for the partial sums of a product whose inputs are cut into pieces
 int LayerStackModel::product(ntk_dense_desc& d) {
@@ -1598,8 +1601,9 @@ int LayerStackModel::parallel_layer(const Run& run, const StackLayer& L, int slo
     if (T > ntk_dense_few_rows()) {
         int st = NTK_E_ALIGN;
         if (rounded(L.mix.in, T)) {        // (the router reads its input as F32)
-            st = ntk_rmsnorm_offset_16(nullptr, h1_16_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? h2_16_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
-            if (st == NTK_OK) { h16 = h1_16_; g16 = L.has_mlp ? h2_16_ : nullptr; }
+            void* second = L.has_mlp && rounded(L.mlp, T) ? h2_16_ : nullptr;
+            st = ntk_rmsnorm_offset_16(nullptr, h1_16_, L.norm1.w, L.has_mlp ? h2_ : nullptr, second, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
+            if (st == NTK_OK) { h16 = h1_16_; g16 = second; }
         }
         if (st == NTK_E_ALIGN) st = ntk_rmsnorm_offset(h1_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
         LS_TRY(st);

@@ -613,3 +613,39 @@ def test_refused_folders(tmp_path, bad):
     with pytest.raises(Exception):
         e.load_folder(folder, max_context=64, dtype="float32")
     e.close()
+
+
+_COUNT_ROUNDINGS = """
+import sys
+sys.path.insert(0, {root!r}); sys.path.insert(0, {tests!r})
+import torch
+from torch.profiler import profile, ProfilerActivity
+import test_fifotar_gpu as T
+e = T.engine_for({folder!r}, "bfloat16")
+for turn in range(2):
+    s = e.seq_acquire()
+    if turn == 0: e.seq_forward(s, {toks!r})
+    else:
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            e.seq_forward(s, {toks!r})
+            torch.cuda.synchronize()
+    e.seq_release(s)
+names = [ev.name for ev in p.events()]
+print("LAUNCHES", sum("ntk::" in n for n in names), "ROUNDINGS", sum("round_rows_kernel" in n for n in names))
+"""
+
+
+@pytest.mark.parametrize("ff,width", [(96, 64), (112, 64), (128, 64)])
+def test_rows_are_rounded_only_for_units_whose_two_products_take_them(tmp_path, ff, width):
+    """a feed-forward size that is no multiple of 64: its down product reads 32-bit rows, so the unit's input is not rounded in a launch of its own either"""
+    cfg = O.config([O.attention_layer(ff=ff), O.delta_layer(ff=ff), O.latent_layer(ff=ff)], width=width)
+    folder, w = make(tmp_path, cfg)
+    toks = tokens_for(cfg, 40)
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = _COUNT_ROUNDINGS.format(root=os.path.dirname(here), tests=here, folder=folder, toks=toks)
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    launches, roundings = (int(x) for x in out.stdout.split("LAUNCHES")[1].split("ROUNDINGS"))
+    assert launches > 20 and roundings == 0
+    e = engine_for(folder, "bfloat16")
+    assert rel(e.seq_forward(e.seq_acquire(), toks), O.forward(cfg, w, toks)[0]) < TOL["bfloat16"]
