@@ -217,13 +217,15 @@ int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partia
 
 /* Y[t][0..out) (+)= W . X[t] for the tokens of a prompt over IEEE-half weights ([out][in] row-major), one pass over W: the batched form of n_tokens ntk_gemv calls.
  * row_max: the tokens' largest |X| where their producer left it (ntk_rmsnorm_rowmax ...), NULL: taken here.  workspace (16-byte aligned): without row_max at least
- * ntk_gemm_half_workspace_bytes(n_tokens), else NULL is enough; what it holds beyond that is used for partial sums. */
+ * ntk_gemm_half_workspace_bytes(n_tokens), else NULL is enough; what it holds beyond that is used for partial sums or, where that is faster (most shapes, from room for all
+ * rows' halves on: 4 * in_features + 4 bytes a token), for the activations' two halves: all of it may be overwritten. */
 size_t ntk_gemm_half_workspace_bytes(int n_tokens);
 int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
                   size_t workspace_bytes, void* stream);
 
 /* ... for up to three such matrices over the same X (query, key and value; gate and up) in one launch, with the activations' two halves formed once per pass in the workspace
- * (ntk_gemm_half_many_bytes() of it at least; more is used for partial sums).  Y[i] = W[i] . X; silu != 0 (n == 2, out[0] == out[1]): Y[0] = silu(W[0] . X) * (W[1] . X) alone (ntk_silu_mul).
+ * (ntk_gemm_half_many_bytes() of it at least, which is 16 tokens' worth; the tokens go in equal passes of what it holds, 4 * in_features + 4 bytes each, and every pass reads the weights:
+ * give it room for all of them; more is used for partial sums).  Y[i] = W[i] . X; silu != 0 (n == 2, out[0] == out[1]): Y[0] = silu(W[0] . X) * (W[1] . X) alone (ntk_silu_mul).
  * accumulate only with n == 1.  NTK_E_SHAPE where in_features is no multiple
  * of 64, the workspace is too small for 16 tokens or, with silu, the two matrices lie 4 GiB apart: nothing has been launched then. */
 typedef struct ntk_half_desc {

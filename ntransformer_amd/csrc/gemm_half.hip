@@ -23,6 +23,7 @@ __global__ __launch_bounds__(256) void token_max_kernel(float* out, const float*
 // The two halves of every activation, planes [2][T][K] (K a multiple of eight), and the rows' largest |x| where their producer has not left them; one workgroup a row.
 // In the place of forming them again in each of a product's up to 112 column tiles: 200 rows of 4096 or 14336 in 5.1 .. 5.6 us, with or without the rows' maxima given (a gated unit that
 // left them by atomics, four waves a row in each of 112 column tiles, took 192 us in the place of 120).
+constexpr float kSplitUs = 4.0f, kSplitRate = 4e6f, kTileUs = 8.0f;     // that launch: us, and bytes per us (eight an entry); what the tiles over 32-bit activations take beside their chunks
 constexpr int kHalfKeep = 7;      // pieces of eight a thread keeps (rows up to 14336 cross memory once)
 template <bool GIVEN>
 __global__ __launch_bounds__(256) void half_split_kernel(_Float16* out, long long plane, const float* X, int K, float* row_max) {
@@ -85,6 +86,13 @@ static void launch_direct_half(const DirectArgs& d, const TilePlan& p, hipStream
 using namespace ntk;
 
 static size_t half_row_bytes(int K) { return (size_t)K * 4 + 4; }
+// rows of a pass of the direct form: what the workspace and 32-bit offsets hold, in equal passes
+static int half_pass_rows(int T, int K, size_t bytes) {
+    const long long fit = std::min<long long>({T, ((long long)bytes - 32) / (long long)half_row_bytes(K), ((1LL << 32) - 1) / (K * 2LL), 65535LL});
+    const int passes = (T + (int)fit - 1) / (int)fit;
+    return (T + passes - 1) / passes;
+}
+static size_t half_max_bytes(int rows) { return ((size_t)rows * 4 + 15) & ~(size_t)15; }
 size_t ntk_gemm_half_many_bytes(int n_tokens, int in_features) { return n_tokens > 0 && in_features > 0 ? (size_t)std::min(n_tokens, 16) * half_row_bytes(in_features) + 32 : 0; }
 
 int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
@@ -106,9 +114,7 @@ int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
     const long long mat = (long long)d->out[0] * K * 2;
     if (K % 64 || K >= 1 << 22 || N > 1 << 30 || (d->silu && std::abs((long long)(w1 - w0)) + mat >= 1LL << 32)) return NTK_E_SHAPE;
     if (d->workspace_bytes < ntk_gemm_half_many_bytes(T, K)) return NTK_E_SHAPE;
-    // rows of a pass: what the workspace and 32-bit offsets hold
-    const long long fit = std::min<long long>({T, ((long long)d->workspace_bytes - 32) / (long long)half_row_bytes(K), ((1LL << 32) - 1) / (K * 2LL), 65535LL});
-    const int pass = (int)fit, passes = (T + pass - 1) / pass, per = (T + passes - 1) / passes;
+    const int per = half_pass_rows(T, K, d->workspace_bytes);
     hipStream_t s = resolve_stream(stream);
     for (int t0 = 0; t0 < T; t0 += per) {
         const int n = std::min(per, T - t0);
@@ -117,7 +123,7 @@ int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
         _Float16* halves = (_Float16*)d->workspace;
         char* behind = (char*)d->workspace + 4 * plane;                     // (plane is a multiple of 64)
         float* own_max = (float*)behind;
-        behind += ((size_t)n * 4 + 15) & ~(size_t)15;
+        behind += half_max_bytes(n);
         if (d->row_max) hipLaunchKernelGGL(half_split_kernel<true>, dim3(n), dim3(256), 0, s, halves, plane, x, K, const_cast<float*>(d->row_max) + t0);
         else hipLaunchKernelGGL(half_split_kernel<false>, dim3(n), dim3(256), 0, s, halves, plane, x, K, own_max);
         DirectArgs a{};
@@ -152,13 +158,6 @@ int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out
     const size_t need = !row_max ? ntk_gemm_half_workspace_bytes(n_tokens) : 0;
     if (need && (!workspace || ((uintptr_t)workspace & 15))) return workspace ? NTK_E_ALIGN : NTK_E_NULL;
     if (need > workspace_bytes) return NTK_E_SHAPE;
-    if (workspace_bytes >= ntk_gemm_half_many_bytes(n_tokens, in_features) && workspace) {
-        ntk_half_desc d{};
-        d.W[0] = W; d.Y[0] = Y; d.out[0] = out_features; d.n = 1; d.X = X; d.n_tokens = n_tokens; d.in_features = in_features; d.accumulate = accumulate; d.row_max = row_max;
-        d.workspace = workspace; d.workspace_bytes = workspace_bytes;
-        const int st = ntk_gemm_half_many(&d, stream);
-        if (st != NTK_E_SHAPE && st != NTK_E_ALIGN) return st;             // (those two: nothing was launched)
-    }
     hipStream_t s = resolve_stream(stream);
     TileArgs t{};
     t.Y = Y; t.ldy = out_features; t.X = X; t.ldx = in_features; t.W = W; t.row_div = 1; t.G = 1; t.T = n_tokens; t.N = out_features; t.K = in_features; t.accumulate = accumulate;
@@ -169,13 +168,29 @@ int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out
         room = (long long)((workspace_bytes - need) / sizeof(float));
     }
     const bool vec = in_features % 8 == 0 && in_features < 1 << 24 && !(((uintptr_t)X | (uintptr_t)W) & 15);
+    static const TileForm forms[] = {{64, 128, 64, 1.25f, 0.95f}, {32, 64, 64, 0.84f, 0.38f}};
+    const TilePlan p = plan_tiles(forms, 2, n_tokens, 1, out_features, in_features, room);
+    // The halves formed once, in the workspace, where that is estimated to be ahead: every pass of the rows that it holds reads the weights again, and what the halves take is lost to
+    // partial sums.  us over tiles that convert, over halves in a workspace for a third / two thirds / all of the rows / ten times as much: 14336 x 4096, 200 tokens 105, 151 / 89 / 67 / 66;
+    // 1024 x 4096, 100 tokens 21 (20 with room for pieces), 145 / 73 / 39 / 18; 4096 x 14336, 200 tokens 207 (112), 426 / 221 / 116 / 69; 2000 tokens 712, 892 / 630 / 463 / 456.  A twentieth in
+    // hand for the estimates, a tenth with several passes, a third where the halves leave fewer pieces (1024 x 8192, 2000 tokens: 168 in one piece, 126 in three).  Over 99 sizes and nine workspaces none is behind the tiles.
+    if (vec && workspace && !((uintptr_t)workspace & 15) && in_features % 64 == 0 && in_features < 1 << 22 && workspace_bytes >= ntk_gemm_half_many_bytes(n_tokens, in_features)) {
+        const int per = half_pass_rows(n_tokens, in_features, workspace_bytes), passes = (n_tokens + per - 1) / per;
+        const long long left = (long long)workspace_bytes - 4LL * per * in_features - (long long)half_max_bytes(per);
+        const TilePlan q = plan_direct_half(per, out_features, in_features, std::max(left, 0LL) / (long long)sizeof(float));
+        const bool cramped = p.splits > q.splits && left / (long long)sizeof(float) < (long long)p.splits * per * out_features;
+        if ((cramped ? 1.35f : passes > 1 ? 1.12f : 1.05f) * passes * (q.us + kSplitUs + (float)per * in_features * 8.0f / kSplitRate) < p.us + kTileUs) {
+            ntk_half_desc d{};
+            d.W[0] = W; d.Y[0] = Y; d.out[0] = out_features; d.n = 1; d.X = X; d.n_tokens = n_tokens; d.in_features = in_features; d.accumulate = accumulate; d.row_max = row_max;
+            d.workspace = workspace; d.workspace_bytes = workspace_bytes;
+            return ntk_gemm_half_many(&d, stream);
+        }
+    }
     if (need) {
         hipLaunchKernelGGL(token_max_kernel, dim3(n_tokens), dim3(256), 0, s, (float*)workspace, X, in_features);
         t.row_max = (const float*)workspace;
     }
     if (!vec) { launch_tiles<TileHalf2, 64, 64, 2, 2, 2, false>(t, 1, s); return last_launch_status(); }
-    static const TileForm forms[] = {{64, 128, 64, 1.25f, 0.95f}, {32, 64, 64, 0.84f, 0.38f}};
-    const TilePlan p = plan_tiles(forms, 2, n_tokens, 1, out_features, in_features, room);
     if (p.form == 0) launch_tiles<TileHalf2, 64, 128, 2, 2, 4, true>(t, p.splits, s);
     else launch_tiles<TileHalf2, 32, 64, 2, 2, 2, true>(t, p.splits, s);
     return last_launch_status();

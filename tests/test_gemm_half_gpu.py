@@ -12,10 +12,16 @@ from ntransformer_amd import gguf as G
 pytestmark = pytest.mark.gpu
 
 
-def run(x, w, y0=None, room=0, given_max=False):
+def bound():
+    """the library with these entry points' types (an unbound call would cut its pointers to 32 bits)"""
     L = _lib.lib()
     L.ntk_gemm_half_workspace_bytes.restype = C.c_size_t
     L.ntk_gemm_half.argtypes = [C.c_void_p] * 3 + [C.c_int] * 4 + [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
+    return L
+
+
+def run(x, w, y0=None, room=0, given_max=False):
+    L = bound()
     T, K = x.shape
     N = w.shape[0]
     need = int(L.ntk_gemm_half_workspace_bytes(T))
@@ -103,3 +109,24 @@ def test_what_it_refuses():
     assert f(b.ptr, b.ptr, None, 2, 8, 8, 0, None, b.ptr, 4096, None) == -5
     assert f(b.ptr, b.ptr, b.ptr, 2, 8, 8, 0, None, None, 0, None) == -5 and f(b.ptr, b.ptr, b.ptr, 9, 8, 8, 0, None, b.ptr, 32, None) == -2
     assert f(b.ptr, b.ptr, b.ptr, 2, 0, 8, 0, None, b.ptr, 4096, None) == -2 and f(b.ptr, b.ptr, b.ptr, 0, 8, 8, 0, None, b.ptr, 4096, None) == 0
+
+
+def test_a_workspace_for_a_few_rows_is_no_slower_than_the_smallest():
+    """activations go in pieces of what the workspace holds only where that pays: 200 tokens through a workspace for 16 took seven times as long as through none"""
+    import time
+    L = bound()
+    T, N, K = 200, 4096, 4096
+    x, w = ops.DeviceBuffer.zeros(T * K * 4), ops.DeviceBuffer.zeros(N * K * 2)
+    y = ops.DeviceBuffer(T * N * 4)
+    best = {}
+    for rows in (0, 16, 50):
+        size = int(L.ntk_gemm_half_workspace_bytes(T)) + rows * (4 * K + 4)
+        ws = ops.DeviceBuffer(size)
+        for _ in range(6):
+            t0 = time.perf_counter()
+            for _ in range(30):
+                _lib.check(L.ntk_gemm_half(y.ptr, w.ptr, x.ptr, T, N, K, 0, None, ws.ptr, size, None), "ntk_gemm_half")
+            _lib.check(L.ntk_stream_synchronize(None), "synchronize")
+            best[rows] = min(best.get(rows, 1e9), time.perf_counter() - t0)
+    print({r: "%.0f us" % (t / 30 * 1e6) for r, t in best.items()})
+    assert max(best[16], best[50]) < 2.0 * best[0]
