@@ -400,7 +400,7 @@ __global__ __launch_bounds__(512) void rp_gemv_f32_kernel(float* __restrict__ y,
             add(t);
             cur = next;
         }
-        acc += rest;
+        if (fabsf(acc) < INFINITY) acc += rest;               // (what an infinite sum's roundings left is a NaN)
         acc += __shfl_xor(acc, 16, 64);
         acc += __shfl_xor(acc, 32, 64);
         if (kg == 0 && 16 * tile + i < rows) y[16 * tile + i] = acc;

@@ -65,3 +65,32 @@ def test_what_it_refuses():
     for args, code in (((d.ptr, d.ptr, d.ptr, 16, 256, G.GGML_TO_DT[G.GGML_Q8_0]), -1), ((d.ptr, d.ptr, d.ptr, 16, 100, q4), -2), ((d.ptr, d.ptr, d.ptr, 16, 33024, q4), -2),
                        ((d.ptr, d.ptr, None, 16, 256, q4), -5)):
         assert L.ntk_gemv_rp_f32(*args, None) == code
+
+
+@pytest.mark.parametrize("qname", sorted(KQ))
+@pytest.mark.parametrize("kind", ["one sum overflows", "the total overflows", "inf", "nan"])
+def test_what_is_not_finite_is_what_the_raw_blocks_give(qname, kind):
+    """a sum beyond the range is an infinity of its sign, as from raw blocks (which give NaN for an activation that is not finite)"""
+    rows, n, gt = 300, 1024, KQ[qname]
+    raw, w, x = case(gt, rows, n, 5)
+    blocks = raw.copy().reshape(-1, raw.size // (rows * n // 256))
+    at = 208 if qname == "Q6_K" else 0
+    blocks[:, at:at + 2] = np.frombuffer(np.float16(30000.0).tobytes(), np.uint8)
+    if qname != "Q6_K":
+        blocks[:, 2:4] = 0                      # no minima
+    raw = blocks.reshape(-1)
+    if kind.endswith("overflows"):              # every block alike and every product of one sign: the first super-block's sum alone, or the row's from sums that fit
+        raw = np.tile(blocks[:1], (rows * n // 256, 1)).reshape(-1)
+        first = G.dequantize(raw, gt, rows * n)[:256].astype(np.float64)
+        x = -np.tile(np.sign(first) / np.abs(first).sum(), n // 256)
+        x = (np.where(np.arange(n) < 256, 4e39 * x, 0.0) if kind == "one sum overflows" else 2.2e38 * x).astype(np.float32)
+    else:
+        x[700] = {"inf": np.inf, "nan": np.nan}[kind]
+    yb = DB(rows * 4)
+    ops.launch_gemv(yb, DB.from_numpy(raw), DB.from_numpy(x), rows, n, G.GGML_TO_DT[gt])
+    got, want = run(raw, gt, x, rows), yb.numpy(np.float32)[:rows]
+    print(qname, kind, "finite %d inf %d nan %d, raw blocks %d %d %d" % tuple(f(y).sum() for y in (got, want) for f in (np.isfinite, np.isinf, np.isnan)))
+    if kind.endswith("overflows"):
+        assert np.array_equal(want, np.full(rows, -np.inf, np.float32)) and np.array_equal(got, want)
+    else:
+        assert not np.isfinite(got).any()
