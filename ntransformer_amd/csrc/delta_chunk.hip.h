@@ -36,11 +36,12 @@ struct DeltaArgs {
 // accumulators of two waves (rows 4 g + r of 16 each) are then a slot as they stand
 __device__ __forceinline__ int delta_place(int g, int j) { return 4 * g + (j & 3) + 16 * (j >> 2); }
 
-// four values -> three pieces of two dwords each.  (Non-finite: the first piece holds it, the others are zero.)
+// four values -> three pieces of two dwords each.  (Not finite: the first piece holds it, the others are zero.  Above the largest bfloat16: that, not the infinity it would round to.)
 struct DeltaPieces { uint32_t w[3][2]; };
 __device__ __forceinline__ DeltaPieces delta_split(deltax4_t x) {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
     typedef float f2 __attribute__((ext_vector_type(2)));
+    constexpr float top = 3.3895314e38f;
     DeltaPieces p;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -48,7 +49,7 @@ __device__ __forceinline__ DeltaPieces delta_split(deltax4_t x) {
         const bool fa = fabsf(a) < INFINITY, fb = fabsf(b) < INFINITY;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
+            const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(i == 0 ? f2{fa ? __builtin_amdgcn_fmed3f(a, -top, top) : a, fb ? __builtin_amdgcn_fmed3f(b, -top, top) : b} : f2{a, b}, b2));
             p.w[i][h] = w;
             a = fa ? a - __uint_as_float(w << 16) : 0.0f;
             b = fb ? b - __uint_as_float(w & 0xFFFF0000u) : 0.0f;

@@ -23,3 +23,25 @@ def test_sizes_of_values(dn, T, size):
     ref, S = _delta_reference(q, k, v, az, wz, rates, bias, H, G, dn, dv, state.astype(np.float64))
     assert np.linalg.norm((got - ref.reshape(got.shape)) / size) < 1e-6 * np.linalg.norm(ref / size)
     assert np.linalg.norm((st.reshape(S.shape) - S) / size) < 1e-6 * np.linalg.norm(S / size)
+
+
+@pytest.mark.parametrize("what", ["state", "value"])
+def test_values_at_the_end_of_the_range(what):
+    """a value between the largest bfloat16 and the largest 32-bit number stays finite in its pieces"""
+    from ntransformer_amd import layers as Lr
+    T, H, G, dn, dv = 64, 4, 2, 64, 64
+    g = np.random.default_rng(3)
+    q, k, v, az, wz, rates, bias = _delta_inputs(g, T, H, G, dn, dv)
+    state = np.zeros((H, dn, dv))
+    top = np.finfo(np.float32).max
+    if what == "state":
+        state[1, 3, 5] = top * 0.9999
+    else:
+        v = v * 1e-6
+        v.reshape(T, H, dv)[-1, 2, 7] = top * 0.9999
+        az[:] = 30.0
+    kw = dict(decay_form=Lr.DECAY_EXP_SOFTPLUS, wb=bias, decay_rates=rates, G=G, unit_q=True, unit_k=True, head_gates=True, write_gated=True, q_scale=dn ** -0.5)
+    got, st = Lr.gated_recurrence(q, k, v, wz, H, dn, dv, 5, az=az, state=state.astype(np.float32), **kw)
+    ref, S = _delta_reference(q, k, v, az, wz, rates, bias, H, G, dn, dv, state.astype(np.float32).astype(np.float64))
+    assert np.isfinite(got).all() and np.isfinite(st).all()
+    assert np.abs(got - ref.reshape(got.shape)).max() < 1e-5 * max(np.abs(ref).max(), 1e-30)
