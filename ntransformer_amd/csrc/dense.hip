@@ -560,10 +560,11 @@ int ntk_round_rows(void* y, int ldy, const float* x, int ldx, int T, int n, void
     return last_launch_status();
 }
 
-// whole chunks of 128 bytes, and rows that 32-bit offsets reach
+// whole chunks of 128 bytes, rows that 32-bit offsets reach, and a one-dimensional grid of tiles that fits: 2^32 threads, 256 for 32 x 64 results, with room for the groups' tiles
 int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K) {
     const int es = wdtype == NTK_DT_BF16 ? 2 : 4;
-    return (wdtype == NTK_DT_BF16 || wdtype == NTK_DT_F32) && T > kGemvRows && N > 0 && K > 0 && K % (128 / es) == 0 && (long long)N * K * es < 1LL << 32 && (long long)x16_rows * K * es < 1LL << 32;
+    return (wdtype == NTK_DT_BF16 || wdtype == NTK_DT_F32) && T > kGemvRows && N > 0 && K > 0 && K % (128 / es) == 0 && (long long)N * K * es < 1LL << 32 && (long long)x16_rows * K * es < 1LL << 32 &&
+           (T / 32 + 1LL) * (N / 64 + 1LL) < 1LL << 23;
 }
 
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream) {

@@ -215,3 +215,13 @@ def test_bench_launch_model_recovers_fixed_cost_and_rate():
     assert abs(m["fixed_us"] - 3.0) < 0.02 and abs(m["stream_TBs"] - 6.5) < 0.02
     assert m["per_launch"]["wo"][2] == 32 and m["per_launch"]["lm_head"][2] == 1
     assert bench._launch_model(spec, "Q8_0", None) is None
+
+
+@pytest.mark.parametrize("dtype", [0, 9])      # NTK_DT_F32, NTK_DT_BF16
+def test_products_too_large_for_a_one_dimensional_grid_keep_the_form_with_two(dtype):
+    """2^32 threads are a launch's limit: 400000 x 128000 results in tiles of 32 x 64 on 256 threads would be 6.4e9"""
+    f = _lib.lib().ntk_dense_direct_takes
+    f.argtypes, f.restype = [C.c_int] * 5, C.c_int
+    assert f(dtype, 400000, 400000, 128000, 512) == 0
+    assert f(dtype, 100000, 100000, 128000, 512) == 1 and f(dtype, 2000, 2000, 2 ** 20, 128) == 1
+    assert f(dtype, 8, 8, 64, 64) == 0 and f(dtype, 9, 9, 64, 64) == 1 and f(dtype, 9, 9, 64, 72) == 0
