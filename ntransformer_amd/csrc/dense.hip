@@ -687,8 +687,10 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
             launch_direct_f32<kGluNone>(a32, G, room, s);
             return last_launch_status();
         }
-        static const TileForm form[] = {{32, 64, 32, 0.52f, 0.36f}};
-        launch_tiles<TileF32, 32, 64, 2, 2, 2, true>(t, plan_tiles(form, 1, d->T, G, d->N, d->K, room).splits, s);
+        static const TileForm forms[] = {{64, 64, 32, 0.78f, 0.70f}, {32, 64, 32, 0.52f, 0.36f}};
+        const TilePlan p = plan_tiles(forms, 2, d->T, G, d->N, d->K, room);
+        if (p.form == 0) launch_tiles<TileF32, 64, 64, 2, 2, 2, true>(t, p.splits, s);
+        else launch_tiles<TileF32, 32, 64, 2, 2, 2, true>(t, p.splits, s);
     }
     return last_launch_status();
 }
