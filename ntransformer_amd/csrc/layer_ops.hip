@@ -833,7 +833,9 @@ int ntk_causal_conv_act(float* y, int ldy, const float* x, int ldx, const float*
         return last_launch_status();
     }
     const uintptr_t at = (uintptr_t)y | (uintptr_t)x | (uintptr_t)(taps > 1 ? state : nullptr);
-    if (taps <= ntk::kConvRowTaps && !((n | ldx | ldy) & 3) && !(at & 15)) {
+    // (a thread of the rows' form walks eight rows: with less than about a million results there are too few of them.  us, both launches of the other form and this one: 4096 channels, 40
+    // rows 5.1 and 8.0, 200 8.0 and 8.3, 400 11.7 and 9.0; 1024 channels, 400 rows 6.2 and 8.0, 1000 8.9 and 8.3; 12288 channels, 64 rows 7.9 and 8.4, 100 9.8 and 8.6)
+    if (taps <= ntk::kConvRowTaps && (long long)T * n >= 7 << 17 && !((n | ldx | ldy) & 3) && !(at & 15)) {
         hipLaunchKernelGGL(ntk::causal_conv_rows_kernel, dim3((n / 4 + 255) / 256, (T + ntk::kConvRows - 1) / ntk::kConvRows), dim3(256), 0, s, y, ldy, x, ldx, w, state, taps, act, pos0, T, n);
         return last_launch_status();
     }

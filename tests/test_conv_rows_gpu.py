@@ -29,3 +29,22 @@ def test_rows(taps, n):
     plain, _ = Lr.causal_conv_act(x, w, 0, act=0, n=n)
     full = np.concatenate([np.zeros((taps - 1, n)), x[:, :n]])
     assert rel(plain, sum(w[:, j] * full[j:j + T] for j in range(taps))) < 1e-6
+
+
+# as many results as that form is taken for: portions around its tiles, shorter than the history, a last one in the other form
+@pytest.mark.parametrize("taps", [1, 2, 3, 4])
+@pytest.mark.parametrize("n,T,portions", [(131072, 41, ([41], [7, 8, 9, 17], [24, 17], [40, 1])), (458752, 9, ([9], [2, 3, 4], [5, 2, 2])), (4100, 300, ([300], [230, 70]))])
+def test_rows_of_a_million_results(taps, n, T, portions):
+    from ntransformer_amd import layers as Lr
+    g = np.random.default_rng(taps + n)
+    x, w = f32(g.standard_normal((T, n + 4))), f32(g.standard_normal((n, taps)))
+    ref, carried = O.short_conv(x[:, :n].astype(np.float64), w.astype(np.float64))
+    for cuts in portions:
+        parts, st, at = [], None, 0
+        for c in cuts:
+            o, st = Lr.causal_conv_act(x[at:at + c], w, at, state=st if at else None, n=n)
+            parts.append(o)
+            at += c
+        assert at == T and rel(np.concatenate(parts), ref) < 1e-6, cuts
+        if taps > 1:
+            assert np.allclose(st, carried, atol=1e-6)
