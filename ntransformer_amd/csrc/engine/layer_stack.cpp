@@ -1110,7 +1110,10 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
         const int nkeys = pos0 + T - key0;
         const float* lat = cache + (size_t)key0 * row;
         const size_t image = (size_t)nkeys * m.kv_rank * 2;
-        if (rounded(m.uk, nkeys) && rounded(m.uv, nkeys) && image <= pscratch_bytes_) {       // the latents rounded once for both
+        // The latents rounded once for both, where that launch pays: it does not with few positions or a low rank.  us, two products that convert / so: rank 512, 2048 outputs, 100
+        // positions 10.0 / 13.1, 400 13.0 / 14.0, 700 16.4 / 16.3, 1000 19.0 / 17.4; 4096 outputs, 400 18.0 / 16.3; rank 1024, 100 15.5 / 17.1, 200 21.6 / 17.5; rank 256, 4096 outputs, 700 17.1 / 16.6
+        const double work = (double)nkeys * std::min(m.uk.out_f, m.uv.out_f) * m.kv_rank * m.kv_rank;
+        if (work >= 4e11 && rounded(m.uk, nkeys) && rounded(m.uv, nkeys) && image <= pscratch_bytes_) {
             LS_TRY(ntk_round_rows(pscratch_, m.kv_rank, lat, row, nkeys, m.kv_rank, stream_));
             const ntk_direct_desc e{pscratch_, m.kv_rank, nkeys, nullptr, 0};
             ntk_dense_desc u{};

@@ -376,6 +376,19 @@ def test_a_folder_loads_where_all_but_the_attentions_image_fits(tmp_path):
         L.ntk_debug_malloc_budget(-1)
 
 
+@pytest.mark.parametrize("T", [700, 790])
+def test_latents_of_a_high_rank_on_both_sides_of_their_rounding(tmp_path, T):
+    """rank 512, 32 x 64 key entries: from 746 positions on the latents are rounded in a launch of their own, once for keys and values (the same values either way)"""
+    cfg = O.small_config(layers=("latent_attention",), heads=32, dim=64, vdim=64, kv_rank=512, q_rank=64)
+    folder, w = make(tmp_path, cfg, seed=12)
+    toks = tokens_for(cfg, T, seed=13)
+    ref = O.forward(cfg, w, toks).numpy()
+    for dtype in ("bfloat16", "float32"):
+        e = engine_for(folder, dtype, ctx=800)
+        got = e.seq_forward(e.seq_acquire(), toks)
+        assert rel(got, ref) < TOL[dtype] and rel(got[-8:], ref[-8:]) < 2 * TOL[dtype]
+
+
 def test_wanted_places_only(tmp_path):
     cfg = O.small_config(**MIXED)
     folder, w = make(tmp_path, cfg, seed=5)
