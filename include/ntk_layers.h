@@ -76,6 +76,9 @@ typedef struct ntk_direct_desc {
 } ntk_direct_desc;
 int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K);
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream);
+/* whether a unit of `ff` values a row (gate and up, or with `plain` up and an activation; then down) over `rows` rows of `tokens` tokens in `groups` groups is estimated to be faster
+ * with ntk_dense_direct for its first product -- bfloat16: for both, and a launch that rounds the tokens -- than with ntk_dense (`scratch_bytes` for partial sums) and ntk_glu */
+int ntk_dense_unit_direct(int wdtype, int rows, int groups, int tokens, int width, int ff, int plain, size_t scratch_bytes);
 /* y[t][0..n) = x[t][0..n) rounded to bfloat16 (nearest even), rows ldx floats / ldy values apart */
 int ntk_round_rows(void* y, int ldy, const float* x, int ldx, int T, int n, void* stream);
 /* the plain case: Y[T][N] = X[T][K] . W[N][K]^T */

@@ -525,10 +525,17 @@ static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long r
 }
 // float32: K in chunks of 32; one form is ahead of larger and smaller tiles and other splits of the tile over waves everywhere (12 .. 200 rows, 900 in 32 groups): us, the form of gemm_tile.hip.h
 // before -> now: 150 x 14976 x 2048 114 -> 91 (101 TF/s of the 153 a large library product reaches), 150 x 2048 x 7488 58 -> 49, 150 x 6240 x 2048 51 -> 39, 12 x 2048 x 2048 11 -> 9
+static TilePlan plan_direct_f32(int rows, int groups, int N, int K, long long room) {
+    static const DirectForm form[] = {{32, 64, 4, 0.38f, 0.27f, 4.0f}};
+    return plan_direct(form, 1, 32, rows, groups, N, K, room);
+}
 template <int GLU>
 static void launch_direct_f32(const DirectArgs& d, int groups, long long room, hipStream_t s) {
-    static const DirectForm form[] = {{32, 64, 4, 0.38f, 0.27f, 4.0f}};
-    launch_direct<TileF32, 32, 64, 2, 2, 3, GLU, 4>(d, plan_direct(form, 1, 32, d.t.T, groups, d.t.N, d.t.K, room).splits, s);
+    launch_direct<TileF32, 32, 64, 2, 2, 3, GLU, 4>(d, plan_direct_f32(d.t.T, groups, d.t.N, d.t.K, room).splits, s);
+}
+static TilePlan plan_tiles_bf16(int rows, int groups, int N, int K, long long room) {
+    static const TileForm forms[] = {{128, 128, 32, 0.65f, 0.43f}, {64, 128, 64, 0.80f, 0.68f}, {64, 64, 64, 0.70f, 0.35f}, {32, 64, 64, 0.60f, 0.22f}};
+    return plan_tiles(forms, 4, rows, groups, N, K, room);
 }
 template <int GLU>
 static void launch_direct_bf16(const DirectArgs& d, const TilePlan& p, hipStream_t s) {
@@ -565,6 +572,25 @@ int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K) {
     const int es = wdtype == NTK_DT_BF16 ? 2 : 4;
     return (wdtype == NTK_DT_BF16 || wdtype == NTK_DT_F32) && T > kGemvRows && N > 0 && K > 0 && K % (128 / es) == 0 && (long long)N * K * es < 1LL << 32 && (long long)x16_rows * K * es < 1LL << 32 &&
            (T / 32 + 1LL) * (N / 64 + 1LL) < 1LL << 23;
+}
+
+// A unit's first product leaves its activations in its epilogue in the direct form, so its inputs are not cut into pieces: with few tiles and long rows that costs more than the launch
+// that it saves.  us of a unit through ntk_dense, ntk_glu and ntk_dense / directly, 33 rows: 4096 inputs, 512 values bf16 17.7 / 28.4, float32 25.2 / 63.5; 2048, 2816 24.7 / 23.3, 41.4 /
+// 43.3; 2048, 7488 35.7 / 27.1, 84.0 / 64.8.  In groups neither form cuts, and what is left to lose are units of a few values and, without a gate, the launch that the rounding adds.  Over
+// 3076 bf16 units (192 .. 4096 inputs, 128 .. 7488 values, 9 .. 1000 tokens, 1 .. 64 groups) always direct was behind by more than 3 % in 668, by up to 2.4 times, with 0.87 of the time
+// on average; so in 12, by 11 % at most, with 0.86.  Over 270 float32 units of one matrix 113 and up to 3.6 times, 1.09; so none, 0.85.
+int ntk_dense_unit_direct(int wdtype, int rows, int groups, int tokens, int width, int ff, int plain, size_t scratch_bytes) {
+    if (rows <= kGemvRows || groups <= 0 || tokens <= 0 || width <= 0 || ff <= 0) return 0;
+    const int first = plain ? ff : 2 * ff;
+    const long long room = groups > 1 || rows > 65535 ? 0 : (long long)(scratch_bytes / sizeof(float));
+    const float glu = plain ? 0.0f : 3.5f + (float)rows * ff * 12.0f / 4e6f;
+    if (wdtype == NTK_DT_F32)
+        return !plain && (groups > 1 || plan_direct_f32(rows, 1, first, width, 0).us <= plan_direct_f32(rows, 1, first, width, room).us + glu - 2.5f);
+    if (groups > 1 && ff < (plain ? 640 : 256)) return 0;
+    if (groups > 1 && !plain) return 1;
+    const float direct = plan_direct_bf16(rows, groups, first, width, 0).us + plan_direct_bf16(rows, groups, width, ff, room).us + kRoundUs + (float)tokens * width * 6.0f / kRoundRate;
+    const float tiles = plan_tiles_bf16(rows, groups, first, width, room).us + plan_tiles_bf16(rows, groups, width, ff, room).us + 8.0f + glu;
+    return direct < (groups > 1 ? 0.95f : plain ? 0.9f : 0.85f) * tiles;
 }
 
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream) {
@@ -660,8 +686,7 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
         // (a launch that rounds the activations first, where the product over them gains more than that launch takes: rows K 16-bit values apart in the scratch, pieces behind them)
         const long long image = ((long long)d->T * d->K * 2 + 15) & ~15LL;
         const bool direct = d->scratch && !((uintptr_t)d->scratch & 15) && !d->rows && (long long)d->scratch_bytes >= image && ntk_dense_direct_takes(d->wdtype, d->T, d->T, d->N, d->K);
-        static const TileForm forms[] = {{128, 128, 32, 0.65f, 0.43f}, {64, 128, 64, 0.80f, 0.68f}, {64, 64, 64, 0.70f, 0.35f}, {32, 64, 64, 0.60f, 0.22f}};
-        const TilePlan p = plan_tiles(forms, 4, d->T, G, d->N, d->K, room);
+        const TilePlan p = plan_tiles_bf16(d->T, G, d->N, d->K, room);
         if (direct) {
             const long long left = d->offsets || d->T > 65535 ? 0 : ((long long)d->scratch_bytes - image) / (long long)sizeof(float);
             const TilePlan q = plan_direct_bf16(d->T, G, d->N, d->K, left);

@@ -1216,7 +1216,7 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
                                  int full_x, const void* h16, const float* norm_w) {
     const int W = info_.width;
     ntk_dense_desc d{};
-    if (h16 && !full_x && rounded(ex, rows)) {
+    if (h16 && !full_x && rounded(ex, rows, rows / top)) {
         ntk_direct_desc e{h16, W, rows / top, act, ex.ff};
         d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype; d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top;
         d.T = rows; d.N = ex.in_rows(); d.K = W;
@@ -1230,7 +1230,8 @@ int LayerStackModel::run_experts(float glu_alpha, float glu_up_offset, const Gat
         return ntk_dense_direct(&o, &f, stream_);
     }
     d.full_x = full_x;
-    const bool direct = !ex.plain && wdtype_ == NTK_DT_F32 && ntk_dense_direct_takes(NTK_DT_F32, rows, rows / top, ex.in_rows(), W);      // gate and up meet in the first product's launch
+    // (float32: gate and up meet in the first product's launch)
+    const bool direct = wdtype_ == NTK_DT_F32 && ntk_dense_direct_takes(NTK_DT_F32, rows, rows / top, ex.in_rows(), W) && pays(ex, rows, rows / top);
     d.Y = gu; d.ldy = ex.in_rows(); d.X = h; d.ldx = W; d.W = ex.gate_up.ptr; d.wstride = ex.gate_up.stride(); d.wdtype = ex.gate_up.dtype;
     d.offsets = offsets; d.G = ex.gate_up.count; d.rows = order; d.row_div = top; d.T = rows; d.N = ex.in_rows(); d.K = W; d.accumulate = 0;
     if (norm_w) { d.norm_w = norm_w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }
@@ -1335,7 +1336,7 @@ int LayerStackModel::run_dense_ff(const StackLayer& L, int T) {
 
 // the dense gated unit (the experts' unit with one member, clipped or plain): gate and up in one product (decoding: the activation inside its launch), down -> ff_
 int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16, const float* norm_w) {
-    if (!h16 && rounded(L.cff, T)) {
+    if (!h16 && rounded(L.cff, T, T)) {
         LS_TRY(ntk_round_rows(h2_16_, info_.width, h, info_.width, T, info_.width, stream_));
         h16 = h2_16_;
     }
@@ -1407,7 +1408,7 @@ int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot,
         owed_ = Owed{ff_, L.norm2b};
         return NTK_OK;
     }
-    if (rounded(L.cff, T)) LS_TRY(seam_for(L.cff.gate_up, L.norm2, h2_, h2_16_, T, &h16));
+    if (rounded(L.cff, T, T)) LS_TRY(seam_for(L.cff.gate_up, L.norm2, h2_, h2_16_, T, &h16));
     else { h16 = nullptr; LS_TRY(rms_seam(L.norm2, h2_, T)); }
     LS_TRY(run_unit_ff(L, h2_, T, h16));
     owed_ = Owed{ff_, L.norm2b};
@@ -1417,9 +1418,12 @@ int LayerStackModel::scaled_layer(const Run& run, const StackLayer& L, int slot,
 // T rows of bfloat16 activations go through w as they lie
 bool LayerStackModel::rounded(const DenseW& w, int T) const { return h1_16_ && w.dtype == NTK_DT_BF16 && ntk_dense_direct_takes(w.dtype, T, T, (int)w.out_f, (int)w.in_f) != 0; }
 // ... and through a unit: its down product takes the activations as the first one leaves them, so both products take such rows or none does
-bool LayerStackModel::rounded(const GatedExperts& ex, int rows) const { return rounded(ex.gate_up, rows) && rounded(ex.down, rows); }
+bool LayerStackModel::rounded(const GatedExperts& ex, int rows, int tokens) const { return rounded(ex.gate_up, rows) && rounded(ex.down, rows) && pays(ex, rows, tokens); }
+bool LayerStackModel::pays(const GatedExperts& ex, int rows, int tokens) const {
+    return ntk_dense_unit_direct(ex.gate_up.dtype, rows, ex.gate_up.count, tokens, info_.width, ex.ff, ex.plain, pscratch_bytes_) != 0;
+}
 // ... and through some unit of a mixture
-bool LayerStackModel::rounded(const MoeFeedForward& M, int T) const { return T > ntk_dense_few_rows() && (rounded(M.routed, T * M.top) || (M.has_shared && rounded(M.shared, T))); }
+bool LayerStackModel::rounded(const MoeFeedForward& M, int T) const { return T > ntk_dense_few_rows() && (rounded(M.routed, T * M.top, T) || (M.has_shared && rounded(M.shared, T, T))); }
 
 // every product of the model: with room for the partial sums of a product whose inputs are cut into pieces
 int LayerStackModel::product(ntk_dense_desc& d) {

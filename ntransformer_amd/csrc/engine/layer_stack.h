@@ -342,7 +342,8 @@ private:
     int settle(int T);
     int first_product(ntk_dense_desc& d, const void* x16 = nullptr);
     bool rounded(const DenseW& w, int T) const;
-    bool rounded(const GatedExperts& ex, int rows) const;
+    bool rounded(const GatedExperts& ex, int rows, int tokens) const;
+    bool pays(const GatedExperts& ex, int rows, int tokens) const;
     bool rounded(const MoeFeedForward& M, int T) const;
     int product(ntk_dense_desc& d);
     int linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate);

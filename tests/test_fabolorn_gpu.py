@@ -389,6 +389,22 @@ def test_latents_of_a_high_rank_on_both_sides_of_their_rounding(tmp_path, T):
         assert rel(got, ref) < TOL[dtype] and rel(got[-8:], ref[-8:]) < 2 * TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [12, 70, 200])
+def test_wide_experts_leave_their_activations_in_the_first_products_launch(tmp_path, dtype, T):
+    """experts and a shared unit of sizes for which the first product takes the direct form"""
+    from ntransformer_amd import _lib
+    f = _lib.lib().ntk_dense_unit_direct
+    f.argtypes, f.restype = [C.c_int] * 7 + [C.c_size_t], C.c_int
+    kind = 9 if dtype == "bfloat16" else 0
+    assert f(kind, 2 * T, 4, T, 192, 512, 0, 1 << 24) == 1 and f(kind, T, 1, T, 192, 2816, 0, 1 << 24) == 1
+    cfg = O.small_config(width=192, ff=512, shared_ff=2816, **MIXED)
+    folder, w = make(tmp_path, cfg, seed=21)
+    toks = tokens_for(cfg, T, seed=22)
+    e = engine_for(folder, dtype)
+    assert rel(e.seq_forward(e.seq_acquire(), toks), O.forward(cfg, w, toks)) < TOL[dtype]
+
+
 def test_wanted_places_only(tmp_path):
     cfg = O.small_config(**MIXED)
     folder, w = make(tmp_path, cfg, seed=5)

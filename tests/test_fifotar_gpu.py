@@ -649,3 +649,19 @@ def test_rows_are_rounded_only_for_units_whose_two_products_take_them(tmp_path, 
     assert launches > 20 and roundings == 0
     e = engine_for(folder, "bfloat16")
     assert rel(e.seq_forward(e.seq_acquire(), toks), O.forward(cfg, w, toks)[0]) < TOL["bfloat16"]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("ff,width,T", [(2816, 192, 40), (2816, 192, 130), (1408, 192, 300)])
+def test_wide_units_leave_their_activations_in_the_first_products_launch(tmp_path, dtype, ff, width, T):
+    """sizes for which a unit's first product takes the direct form (in bfloat16 its input and its activations are rounded rows): the other tests' units are too narrow for it"""
+    import ctypes as C
+    from ntransformer_amd import _lib
+    f = _lib.lib().ntk_dense_unit_direct
+    f.argtypes, f.restype = [C.c_int] * 7 + [C.c_size_t], C.c_int
+    assert f(9 if dtype == "bfloat16" else 0, T, 1, T, width, ff, 0, 1 << 24) == 1
+    cfg = O.config([O.attention_layer(ff=ff), O.delta_layer(ff=ff), O.latent_layer(ff=ff)], width=width)
+    folder, w = make(tmp_path, cfg, seed=4)
+    toks = tokens_for(cfg, T)
+    e = engine_for(folder, dtype)
+    assert rel(e.seq_forward(e.seq_acquire(), toks), O.forward(cfg, w, toks)[0]) < TOL[dtype]

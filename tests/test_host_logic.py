@@ -225,3 +225,17 @@ def test_products_too_large_for_a_one_dimensional_grid_keep_the_form_with_two(dt
     assert f(dtype, 400000, 400000, 128000, 512) == 0
     assert f(dtype, 100000, 100000, 128000, 512) == 1 and f(dtype, 2000, 2000, 2 ** 20, 128) == 1
     assert f(dtype, 8, 8, 64, 64) == 0 and f(dtype, 9, 9, 64, 64) == 1 and f(dtype, 9, 9, 64, 72) == 0
+
+
+def test_units_that_are_too_narrow_for_one_launch_go_through_two():
+    """ntk_dense_unit_direct: the first product of a direct unit is not cut into pieces, so few tiles over long rows take the other way, whatever the type; wide ones and groups do not"""
+    f = _lib.lib().ntk_dense_unit_direct
+    f.argtypes, f.restype = [C.c_int] * 7 + [C.c_size_t], C.c_int
+    room, F32, BF16 = 1 << 24, 0, 9
+    for dtype in (F32, BF16):
+        assert f(dtype, 33, 1, 33, 4096, 512, 0, room) == 0 and f(dtype, 200, 1, 200, 4096, 128, 0, room) == 0
+        assert f(dtype, 40, 1, 40, 2048, 7488, 0, room) == 1 and f(dtype, 150, 1, 150, 2048, 7488, 0, room) == 1
+        assert f(dtype, 6144, 32, 1024, 2048, 1408, 0, room) == 1
+        assert f(dtype, 8, 1, 8, 2048, 7488, 0, room) == 0 and f(dtype, 40, 0, 40, 2048, 7488, 0, room) == 0
+    assert f(BF16, 1024, 1, 1024, 2048, 2816, 0, room) == 1 and f(BF16, 96, 32, 16, 2048, 128, 0, room) == 0
+    assert f(BF16, 16, 1, 16, 2048, 2816, 1, room) == 0 and f(BF16, 1024, 1, 1024, 2048, 2816, 1, room) == 1 and f(F32, 150, 1, 150, 2048, 7488, 1, room) == 0
