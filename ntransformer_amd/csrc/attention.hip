@@ -766,7 +766,7 @@ __global__ __launch_bounds__(256) void rope_kv_store_rows_kernel(float* __restri
 
 // ... and the same from the projections' partial sums (ntk_gemm_partials): the splits are added here, in order, in the place of a launch that writes their sums
 // for this one to read back.  A short prompt takes a workgroup per 256 pairs of a token, everything requested ahead of the angles; a long one a workgroup per token with one
-// table of them.  16 tokens of the 8B shapes: 4.7 + 4.6 us as two launches, 4.0 as one; 1003 tokens 12.1 + 11.8 us, 14 as one.
+// table of them.  16 tokens of the 8B shapes: 4.7 + 4.6 us as two launches, 4.0 as one; 1003 tokens 12.1 + 11.8 us, 17 - 18 as one.
 struct RopeSource { const float* p; int n; size_t plane; };
 template <int N>
 __device__ __forceinline__ void rope_sums(const RopeSource& s, const size_t (&at)[N], float (&v)[N]) {

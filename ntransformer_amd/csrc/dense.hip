@@ -1,8 +1,11 @@
 // dense.hip -- products with dense weight matrices (bfloat16 or float32, row-major [out][in]) for the layer-list model families.
 //
-// One entry point for a product (ntk_dense) with two kernel forms behind it:
-//   * gemm_tile_kernel    more than kGemvRows rows (gemm_tile.hip.h): bf16 weights on v_mfma_f32_16x16x32_bf16, the F32 activations rounded to bfloat16 (nearest even) on
-//                         their way into LDS; float32 weights on v_mfma_f32_16x16x4_f32 (true 32-bit products and sums);
+// One entry point for a product (ntk_dense) with three kernel forms behind it:
+//   * gemm_direct_kernel  more than kGemvRows rows of whole 128-byte chunks (gemm_direct.hip.h), operands from memory straight into LDS: float32 wherever the rows lie in order and
+//                         aligned; bf16 where a launch that rounds the activations first and the product over them are estimated faster than tiles (ntk_dense_direct takes rows
+//                         that were rounded by whoever wrote them);
+//   * gemm_tile_kernel    the other products of more than kGemvRows rows (gemm_tile.hip.h): bf16 weights on v_mfma_f32_16x16x32_bf16, the F32 activations rounded to bfloat16
+//                         (nearest even) on their way into LDS; float32 weights on v_mfma_f32_16x16x4_f32 (true 32-bit products and sums); gathered and odd-sized rows;
 //   * dense_gemv_kernel   up to kGemvRows rows (decoding): every wave streams a few weight rows at once, 16 bytes per lane and row, the activation
 //                         row sits in LDS; bf16 weights are widened exactly and multiplied in F32.  What runs inside the launch on the way in: what the row is still owed (a
 //                         sublayer's normed output), an RMS norm; on the way out: a gated unit or an activation.
@@ -523,7 +526,8 @@ static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long r
                                        {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
     return plan_direct(forms, 7, 64, rows, groups, N, K, room);
 }
-// float32: K in chunks of 32; one form is ahead of larger and smaller tiles and other splits of the tile over waves everywhere (12 .. 200 rows, 900 in 32 groups): us, the form of gemm_tile.hip.h
+// float32: K in chunks of 32; one form, ahead of larger and smaller tiles and other splits of the tile over waves at the sizes they were tried at (12 .. 200 rows, 900 in 32 groups).  Over 337
+// grouped sizes it takes 0.89 of gemm_tile.hip.h's time on average and is 3 .. 17 % behind it at about eleven (40 rows in 128 groups, 300 in 8 or 16).  us, the form of gemm_tile.hip.h
 // before -> now: 150 x 14976 x 2048 114 -> 91 (101 TF/s of the 153 a large library product reaches), 150 x 2048 x 7488 58 -> 49, 150 x 6240 x 2048 51 -> 39, 12 x 2048 x 2048 11 -> 9
 static TilePlan plan_direct_f32(int rows, int groups, int N, int K, long long room) {
     static const DirectForm form[] = {{32, 64, 4, 0.38f, 0.27f, 4.0f}};

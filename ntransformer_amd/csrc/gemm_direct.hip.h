@@ -4,10 +4,12 @@
 // activations and rounds them again, and with the operands' way through registers a workgroup of eight waves is left with wave tiles of 32 x 64, for which LDS has to
 // deliver 192 bytes a cycle and CU at the matrix cores' full rate, where it has 128.  Here the activations were rounded (or cut into pieces) once, by the launch that wrote them or
 // by one in front of the product; both operands go from memory straight into LDS (global_load_lds, 16 bytes a lane), STAGES chunks of 128 bytes a row deep, and a wave of the large forms owns 64 x 64 or
-// 64 x 128 (96 .. 128 bytes).  What bounds the large ones is the matrix cores: a chunk of a 256 x 256 tile takes 1.45 us of the 1.7 they need at the rate of a large library product
-// (1216 TF/s); below a few tiles a CU it is the latency of the first chunks and the results on their way out (`over` in plan_direct).  Consecutive tiles of an XCD share their weights.
+// 64 x 128 (96 .. 128 bytes).  What bounds the large ones is the matrix cores: a 64-input chunk of 256 x 256
+// tiles on every CU is 2.15 GFLOP, 0.86 us at their dense peak and 1.77 us at the rate of a large library product (1216 TF/s); whole products of 1024 .. 2048 rows run at 930 .. 1010 TF/s.
+// (The 1.45 us a chunk in plan_direct_bf16 is a constant fitted together with `over`, the latency of the first chunks and the results on their way out, which is what bounds products
+// below a few tiles a CU: no measured rate.)  Consecutive tiles of an XCD share their weights.
 // Measured (us, weights from memory; the form of gemm_tile.hip.h with its best tile and pieces): bf16 1024 x 14976 x 2048 142 -> 62 (1010 TF/s), 1024 x 2048 x 7488 63 -> 43,
-// 1024 x 6240 x 2048 58 -> 37, 1024 x 2048 x 2048 26 -> 16.5, 40 x 14976 x 2048 22 -> 17, 6144 rows in 32 groups of 2816 x 2048 227 -> 133, of 2048 x 1408 116 -> 62.
+// 1024 x 6240 x 2048 58 -> 37, 1024 x 2048 x 2048 26 -> 16.5, 40 x 14976 x 2048 22 -> 17, 6144 rows in 32 groups of 2816 x 2048 227 -> 133, of 2048 x 1408 116 -> 72.
 // One chain of matrix instructions over the inputs as there: the same bits where K is not cut.
 #pragma once
 #include "gemm_tile.hip.h"
