@@ -215,6 +215,21 @@ int ntk_reduce_rmsnorm_prepare_x(float* hidden, const ntk_gemm_partials* partial
 int ntk_silu_mul_prepare_x(float* output, const float* gate, const float* up, int n_tokens, int width, void* workspace, void* stream);
 int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials, void* workspace, void* stream);
 
+/* Prompts of at most 32 tokens, whose projections keep a K slice's planes in LDS: their producers scale X per token and 256 columns, so that they need no whole row in one workgroup.
+ *   ntk_gemm_short_takes          1 where ntk_gemm_short takes matrices of these rows and format (raw or repacked) over one X of in_features, else 0
+ *   ntk_short_prepare_x           planes of X as it lies
+ *   ntk_short_norm_prepare_x      hidden += the deferred projection (partials; NULL: hidden as it lies), planes of hidden * weight and the rows' sums of squares: the projection that
+ *                                 reads them is told `normed` and eps and divides its results by the rows' root mean squares (ntk_rmsnorm's definition)
+ *   ntk_short_silu_mul_prepare_x  planes of silu(gate) * up of a deferred gate | up launch
+ *   ntk_gemm_short                ntk_gemm_quant_f16 over such planes (desc->X and reuse_x are not looked at; NTK_E_SHAPE where ntk_gemm_short_takes says 0).  part_at: floats into the
+ *                                 workspace's area of partial sums at which this launch's begin (a multiple of 4), so that several launches may leave theirs to one consumer
+ * n_tokens <= 32, rows a multiple of 32 (NTK_E_SHAPE), 16-byte aligned pointers (NTK_E_ALIGN).  `workspace` must not be the one partials lie in.  Stream ordered, no allocation. */
+int ntk_gemm_short_takes(const int* rows, int nseg, int n_tokens, int in_features, int dtype);
+int ntk_short_prepare_x(const float* X, int n_tokens, int in_features, void* workspace, void* stream);
+int ntk_short_norm_prepare_x(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int hidden_size, void* workspace, void* stream);
+int ntk_short_silu_mul_prepare_x(const ntk_gemm_partials* partials, void* workspace, void* stream);
+int ntk_gemm_short(const ntk_gemm_desc* desc, int normed, float eps, size_t part_at, void* stream);
+
 /* Y[t][0..out) (+)= W . X[t] for the tokens of a prompt over IEEE-half weights ([out][in] row-major), one pass over W: the batched form of n_tokens ntk_gemv calls.
  * row_max: the tokens' largest |X| where their producer left it (ntk_rmsnorm_rowmax ...), NULL: taken here.  workspace (16-byte aligned): without row_max at least
  * ntk_gemm_half_workspace_bytes(n_tokens), else NULL is enough; what it holds beyond that is used for partial sums or, where that is faster (most shapes, from room for all

@@ -547,6 +547,7 @@ int Model::alloc_buffers() {   // transformer.cpp:330-391
         gemm_ws_bytes_ = 0;
         for (const auto& sh : shapes) gemm_ws_bytes_ = std::max(gemm_ws_bytes_, ntk_gemm_quant_workspace_bytes(sh[0], sh[1]));
     }
+    short_known_[0] = short_known_[1] = -1;
     gemm_ws_ = dev(gemm_ws_bytes_, false);
     gemm_ws2_ = dev(gemm_ws_bytes_, false);
     if (tp_world_ > 1) {   // communication buffer: flags + two slots of one prompt's worth of hidden vectors
@@ -629,8 +630,124 @@ float* Model::forward(const int* tokens, int T, int start_pos) {
     return logits_;
 }
 
+// a prompt of T <= 32 tokens whose matrices all take the form that keeps a K slice's planes in LDS (ntk_gemm_short): layers_short
+bool Model::short_prompt(int T) const {
+    if (T < 2 || T > 32 || !batched_prefill_ || !bf16_prefill_ || !gemm_ws_ || !gemm_ws2_ || tp_world_ > 1 || !row_max_ || !prefill_row_max_ || !prefill_fused_split_) return false;
+    const int H = cfg_.hidden_size, I = cfg_.intermediate_size, qd = cfg_.n_heads * cfg_.head_dim;
+    if (H % 32 || I % 32 || qd % 32) return false;
+    // (the plans depend on the matrices and on how many blocks of 16 tokens there are)
+    int& known = short_known_[T <= 16 ? 0 : 1];
+    if (known < 0) known = short_matrices(T) ? 1 : 0;
+    return known == 1;
+}
+bool Model::short_matrices(int T) const {
+    const int H = cfg_.hidden_size, I = cfg_.intermediate_size, qd = cfg_.n_heads * cfg_.head_dim;
+    auto takes = [&](const DevTensor& w, int in) {
+        const int rows = (int)w.out_f;
+        return is_quant(w.dtype) && (w.ptr || w.rp) && (int)w.in_f == in && ntk_gemm_short_takes(&rows, 1, T, in, w.dtype);
+    };
+    for (const LayerWeights& L : layers_) {
+        if (!takes(L.wq, H) || !takes(L.wk, H) || !takes(L.wv, H) || !takes(L.wo, qd) || !takes(L.w_gate, H) || !takes(L.w_up, H) || !takes(L.w_down, I)) return false;
+        if (L.w_gate.dtype != L.w_up.dtype || L.w_gate.out_f != L.w_up.out_f || (int)L.w_gate.out_f != I || (int)L.wo.out_f != H || (int)L.w_down.out_f != H) return false;
+        // (matrices of one format go out together: their plan is the launch's, not each one's)
+        const DevTensor* qkv[3] = {&L.wq, &L.wk, &L.wv};
+        for (int a = 0; a < 3; ++a) {
+            int rows[3], n = 0;
+            for (int b = 0; b < 3; ++b)
+                if (qkv[b]->dtype == qkv[a]->dtype) rows[n++] = (int)qkv[b]->out_f;
+            if (!ntk_gemm_short_takes(rows, n, T, H, qkv[a]->dtype)) return false;
+        }
+        const int gu[2] = {I, I};
+        if (!ntk_gemm_short_takes(gu, 2, T, H, L.w_gate.dtype)) return false;
+    }
+    return true;
+}
+
+// layers_1to1 for such a prompt: every producer of a projection's input leaves its planes in the workspace that the projection before it does not use (no whole row in one workgroup:
+// gemm_f16.hip), every projection leaves its partial sums to the launch behind it.
+int Model::layers_short(int T, int start_pos, int first, int last_layer) {
+    const int H = cfg_.hidden_size, I = cfg_.intermediate_size, hd = cfg_.head_dim, nh = cfg_.n_heads, nkv = cfg_.n_kv_heads;
+    const int qd = nh * hd, kvd = nkv * hd;
+    void* s = stream_;
+    const size_t kv_layer = (size_t)cfg_.max_seq_len * kvd;
+    const float scale = 1.0f / sqrtf((float)hd);
+    float* q_buf = workspace_;
+    float* k_buf = q_buf + (size_t)T * qd;
+    float* v_buf = k_buf + (size_t)T * kvd;
+    float* attn_out = v_buf + (size_t)T * kvd;
+    float* gate_buf = workspace_;
+    float* up_buf = gate_buf + (size_t)T * I;
+    void* ws = gemm_ws_;
+    auto other = [&]() { ws = ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_; return ws; };
+    auto gemm = [&](const DevTensor* const* Ws, float* const* Ys, int n, const float* resid, bool normed, size_t part_at, ntk_gemm_partials* pt) {
+        bool rp = true;
+        for (int i = 0; i < n; ++i) rp = rp && !Ws[i]->ptr && Ws[i]->rp && Ws[i]->dtype != NTK_DT_Q8_0 && Ws[i]->dtype != NTK_DT_Q4_0;
+        if (!rp) raw_begin();
+        ntk_gemv_seg segs[3];
+        for (int i = 0; i < n; ++i) segs[i] = {rp ? Ws[i]->rp : raw_of(*Ws[i]), Ys[i], (int)Ws[i]->out_f, Ws[i]->dtype};
+        ntk_gemm_desc d{};
+        d.segs = segs; d.nseg = n; d.n_tokens = T; d.in_features = (int)Ws[0]->in_f; d.resid = resid;
+        d.workspace = ws; d.workspace_bytes = gemm_ws_bytes_; d.partials = pt; d.weights_repacked = rp ? 1 : 0;
+        return ntk_gemm_short(&d, normed ? 1 : 0, cfg_.norm_eps, part_at, s);
+    };
+    NT_TRY(ntk_short_norm_prepare_x(hidden_, nullptr, (const float*)layers_[first].attn_norm.ptr, T, H, ws, s));
+    for (int i = first; i < last_layer; ++i) {
+        const LayerWeights& L = layers_[i];
+        uint16_t* kc = k_cache_ + (size_t)i * kv_layer;
+        uint16_t* vc = v_cache_ + (size_t)i * kv_layer;
+        const DevTensor* const qkv[3] = {&L.wq, &L.wk, &L.wv};
+        float* const ys[3] = {q_buf, k_buf, v_buf};
+        const float* sums[3] = {q_buf, k_buf, v_buf};
+        int splits[3] = {1, 1, 1};
+        bool done[3] = {false, false, false};
+        size_t at = 0;
+        for (int a = 0; a < 3; ++a) {
+            if (done[a]) continue;
+            const DevTensor* w[3];
+            float* y[3];
+            int idx[3], n = 0;
+            for (int b = a; b < 3; ++b)
+                if (qkv[b]->dtype == qkv[a]->dtype) { w[n] = qkv[b]; y[n] = ys[b]; idx[n++] = b; done[b] = true; }
+            ntk_gemm_partials pt;
+            NT_TRY(gemm(w, y, n, nullptr, true, at, T >= 4 ? &pt : nullptr));
+            if (T >= 4 && pt.nsplit > 1)
+                for (int k = 0; k < n; ++k) {
+                    sums[idx[k]] = pt.part[k];
+                    splits[idx[k]] = pt.nsplit;
+                    at += (size_t)pt.nsplit * T * w[k]->out_f;
+                }
+        }
+        if (T >= 4) {   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
+            NT_TRY(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
+        } else {
+            NT_TRY(ntk_rope(q_buf, k_buf, positions_, 1, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, s));
+            NT_TRY(ntk_copy_to_kv_cache(kc, vc, k_buf, v_buf, T, nkv, hd, start_pos, cfg_.max_seq_len, s));
+        }
+        NT_TRY(ntk_attention_prefill(attn_out, q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
+        ntk_gemm_partials pt;
+        const DevTensor* w[2] = {&L.wo, nullptr};
+        float* y[2] = {hidden_, nullptr};
+        NT_TRY(ntk_short_prepare_x(attn_out, T, qd, other(), s));
+        NT_TRY(gemm(w, y, 1, hidden_, false, 0, &pt));
+        NT_TRY(ntk_short_norm_prepare_x(hidden_, &pt, (const float*)L.ffn_norm.ptr, T, H, other(), s));
+        w[0] = &L.w_gate; w[1] = &L.w_up;
+        y[0] = gate_buf; y[1] = up_buf;
+        NT_TRY(gemm(w, y, 2, nullptr, true, 0, &pt));
+        NT_TRY(ntk_short_silu_mul_prepare_x(&pt, other(), s));
+        w[0] = &L.w_down;
+        y[0] = hidden_;
+        const bool more = i + 1 < last_layer;
+        NT_TRY(gemm(w, y, 1, hidden_, false, 0, more ? &pt : nullptr));
+        if (more) NT_TRY(ntk_short_norm_prepare_x(hidden_, &pt, (const float*)layers_[i + 1].attn_norm.ptr, T, H, other(), s));
+    }
+    int rc = NTK_OK;
+    if (raw_err_ != NTK_OK) { rc = raw_err_; raw_err_ = NTK_OK; }
+    return rc;
+}
+
 // layers [first, last) of the 1:1 path on hidden_[T][H] at positions start_pos.. (positions_ already on the device)
 int Model::layers_1to1(int T, int start_pos, int first, int last_layer) {
+    if (short_prompt(T) && first < last_layer) return layers_short(T, start_pos, first, last_layer);
     const int H = cfg_.hidden_size, I = cfg_.intermediate_size, hd = cfg_.head_dim, nh = cfg_.n_heads, nkv = cfg_.n_kv_heads;
     const int qd = nh * hd, kvd = nkv * hd;
     void* s = stream_;

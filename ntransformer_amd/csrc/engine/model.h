@@ -181,6 +181,10 @@ private:
     int enqueue_token(bool greedy);   // the fused launch sequence for one token
     int enqueue_layers(int first, int last);            // its layer loop
     int layers_1to1(int T, int start_pos, int first, int last);   // the layer loop of forward()
+    bool short_prompt(int T) const;
+    bool short_matrices(int T) const;
+    mutable int short_known_[2] = {-1, -1};   // short_matrices of up to 16 and up to 32 tokens: not asked yet, no, yes
+    int layers_short(int T, int start_pos, int first, int last_layer);
     void prof_mark(int cls, bool begin);
     bool use_persistent_now() const;
     int build_persistent_plan(int kind);   // the same operator sequence as a table for ntk_persistent_launch / ntk_layer_engine_launch (nullptr plan if unsupported)

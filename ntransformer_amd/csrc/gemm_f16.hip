@@ -60,6 +60,8 @@ constexpr int GB_WG_PER_CU = 3, GB_LDS_WG = 53 * 1024, GB_NRING_Q8 = 1;
 constexpr int GB_WG_PER_CU = 2, GB_LDS_WG = 80 * 1024, GB_NRING_Q8 = 2;
 #endif
 constexpr int GB_AUX_BYTES = GB_TOK * 4;                  // per step: one eighth of its unit's record of sums (K-quant minimum term)
+constexpr int GB_SHORT = 32;         // tokens of a short prompt (gemm_quant_f16_kslice_kernel), whose planes are scaled per GB_GROUP columns
+constexpr int GB_GROUP = 256;
 constexpr int GB_MIN_UNIT_BYTES = 8 * GB_AUX_BYTES;       // per unit of 8 steps and 64-token chunk: 2 pieces x 4 token blocks x 2 x 16 tokens x 4 steps x FP16
 
 // bytes k, k + 1 of a dword -> an FP16 pair, one SDWA conversion each (through F32 it is two conversions and a pack per pair: the
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(256) void row_scale_kernel(const float* __restrict_
 // of their scales -- no row_scale_kernel pass over X; the blocks of step 0 leave 1 / s in `inv` for the main kernel
 template <bool FROM_MAX>
 __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ X, int T, int in, u32x4* __restrict__ xb, float* __restrict__ aux,
-                                                      size_t chunk_bytes, const float* __restrict__ scale, float* __restrict__ inv) {
+                                                      size_t chunk_bytes, const float* __restrict__ scale, float* __restrict__ inv, float* __restrict__ group_inv) {
     const int step = blockIdx.x, tb = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int j = lane & 15, g = lane >> 4, t = tb * 16 + j;
     // blockIdx.y = 64-token chunk: its tokens, its planes
@@ -177,6 +179,8 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
         } else {
             sc = scale[t];
         }
+        if (g == 0 && step % (GB_GROUP / 32) == 0 && t < GB_SHORT && blockIdx.y == 0)   // (one scale a token here: every group's; 1 / s of a power of two by its exponent)
+            group_inv[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((254u << 23) - __float_as_uint(sc));
     }
     float p1[8], p2[8];
 #pragma unroll
@@ -265,6 +269,12 @@ __global__ __launch_bounds__(256) void silu_mul_rowmax_kernel(float* __restrict_
 static __host__ __device__ size_t ws_chunk_bytes(int in) {
     return ((size_t)(in / 32 + 1) * GB_STEP_BYTES + (size_t)((in / 32 + 15) / 8) * GB_MIN_UNIT_BYTES + 255) / 256 * 256;
 }
+constexpr size_t GB_SCALE_BYTES = 2 * GB_MAX_CHUNKS * GB_TOK * sizeof(float);   // the launch's 1 / s and s
+// ... and behind those, for the short prompts' form: [GB_GROUP columns][GB_SHORT tokens] 1 / s, then [512 columns][GB_SHORT tokens] sums of squares (short_split below)
+static __host__ __device__ size_t ws_group_floats(int in) { return (size_t)((in + GB_GROUP - 1) / GB_GROUP) * GB_SHORT; }
+static __host__ __device__ size_t ws_group_bytes(int in) { return (ws_group_floats(in) + (size_t)((in + 511) / 512) * GB_SHORT) * sizeof(float); }
+static __host__ __device__ size_t ws_group_offset(int in) { return (size_t)GB_MAX_CHUNKS * ws_chunk_bytes(in) + GB_SCALE_BYTES; }
+static __host__ __device__ size_t ws_part_offset(int in) { return ws_group_offset(in) + (ws_group_bytes(in) + 255) / 256 * 256; }
 // row: the token's `in` floats (global memory; written by THIS workgroup before a __syncthreads()), or null for a padding token (zeros: the records the
 // matrix instructions read beside the prompt's last tokens).  Every thread of the workgroup calls it.
 __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, int t, int in, uint8_t* __restrict__ ws) {
@@ -313,8 +323,129 @@ __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, i
             const int pos = ((tb * 2 + ((step >> 2) & 1)) * 64 + j * 4 + (step & 3));
             rec[pos] = h1;
             rec[4 * 128 + pos] = h2;
+            if (t < GB_SHORT && step % (GB_GROUP / 32) == 0 && step * 32 < in)
+                reinterpret_cast<float*>(ws + ws_group_offset(in))[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((uint32_t)(254 - es) << 23);
         }
     }
+}
+
+// ---- the producers of a SHORT prompt's planes (<= GB_SHORT tokens through gemm_quant_f16_kslice_kernel): a scale per token and GB_GROUP columns -------------------------
+// A scale per token ties a token's row to one workgroup: 16 workgroups for 16 tokens, each of them bound by what one CU reads -- 11.0 us for the unit of 16 x 14336, 6.7 for a norm
+// of 16 x 4096 with eight splits in front.  With a scale per group of columns a WAVE is on its own (no LDS, no barrier): it sums its 512 columns of a token, finds the two groups' largest
+// magnitudes across its lanes and writes their planes, step sums and 1 / s; the GEMM folds a group's products with that 1 / s (a power of two: exact).  The planes are nearer the values
+// than a row's scale leaves them: what a group's own largest value puts into FP16's subnormals is less.  An RMSNorm's 1 / rms belongs to the row: the wave leaves its sum of squares and
+// the GEMM multiplies its sums by 1 / rms.
+// x[8]: lane's values of columns col + {0..3, 16..19}, col = 512 wave + 32 (lane / 4) + 4 (lane % 4); lanes past the row hold zeros.
+__device__ __forceinline__ void short_split(float (&x)[8], int lane, int col512, int t, int in, uint8_t* __restrict__ ws) {
+    const int step = (col512 >> 5) + (lane >> 2), g = lane & 3;
+    uint32_t mb = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mb = max(mb, __float_as_uint(x[e]) & 0x7FFFFFFFu);   // (bit patterns: ordered like the values, and a NaN is not dropped)
+#pragma unroll
+    for (int o = 1; o <= 16; o <<= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
+    const int es = scale_exp_of_max(mb);
+    const float sc = __uint_as_float((uint32_t)es << 23);
+    float p1[8], p2[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        x[e] *= sc;
+        const _Float16 h1 = (_Float16)x[e];
+        p1[e] = (float)h1;
+        p2[e] = x[e] - p1[e];
+    }
+    auto pk = [](float lo, float hi) {
+        const f16x2 h = {(_Float16)lo, (_Float16)hi};
+        return __builtin_bit_cast(uint32_t, h);
+    };
+    float sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    sum += __shfl_xor(sum, 1, 64);
+    sum += __shfl_xor(sum, 2, 64);
+    if (step * 32 >= in) return;
+    const int tb = t >> 4, j = t & 15;
+    u32x4* xb = reinterpret_cast<u32x4*>(ws);
+    const size_t base = ((size_t)step * GB_PLANES * 4 + tb) * 64 + (j + 16 * g);
+    xb[base] = u32x4{pk(p1[0], p1[1]), pk(p1[2], p1[3]), pk(p1[4], p1[5]), pk(p1[6], p1[7])};
+    xb[base + 256] = u32x4{pk(p2[0], p2[1]), pk(p2[2], p2[3]), pk(p2[4], p2[5]), pk(p2[6], p2[7])};
+    if (g == 0) {
+        const float y = sum * 0.015625f;
+        const _Float16 h1 = (_Float16)y, h2 = (_Float16)(y - (float)h1);
+        _Float16* rec = reinterpret_cast<_Float16*>(ws + (size_t)(in / 32 + 1) * GB_STEP_BYTES + (size_t)(step >> 3) * GB_MIN_UNIT_BYTES);
+        const int pos = ((tb * 2 + ((step >> 2) & 1)) * 64 + j * 4 + (step & 3));
+        rec[pos] = h1;
+        rec[4 * 128 + pos] = h2;
+        if ((lane & 31) == 0) reinterpret_cast<float*>(ws + ws_group_offset(in))[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((uint32_t)(254 - es) << 23);
+    }
+}
+// sums of a deferred projection's K splits (in split order), the lane's eight columns at row[0 .. 3], row[16 .. 19]; eight splits' requests under way
+__device__ __forceinline__ void short_sums(const float* __restrict__ row, size_t plane, int nsplit, float (&v)[8]) {
+    auto put = [](float (&d)[8], const float4& a, const float4& b) { d[0] = a.x; d[1] = a.y; d[2] = a.z; d[3] = a.w; d[4] = b.x; d[5] = b.y; d[6] = b.z; d[7] = b.w; };
+    put(v, *reinterpret_cast<const float4*>(row), *reinterpret_cast<const float4*>(row + 16));
+    for (int s0 = 1; s0 < nsplit; s0 += 8) {
+        float q[8][8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float* r = row + (size_t)min(s0 + k, nsplit - 1) * plane;
+            put(q[k], *reinterpret_cast<const float4*>(r), *reinterpret_cast<const float4*>(r + 16));
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (s0 + k < nsplit) {   // (uniform)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += q[k][e];
+            }
+    }
+}
+// grid (ceil(in / 512), T), one wave.  X as it lies
+__global__ __launch_bounds__(64) void short_split_kernel(const float* __restrict__ X, int in, uint8_t* __restrict__ ws) {
+    const int lane = threadIdx.x, t = (int)blockIdx.y, col = (int)blockIdx.x * 512 + 32 * (lane >> 2) + 4 * (lane & 3);
+    float x[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (col < in) short_sums(X + (size_t)t * in + col, 0, 1, x);
+    short_split(x, lane, (int)blockIdx.x * 512, t, in, ws);
+}
+// hidden += the sums of part's splits (nsplit 0: hidden as it lies); planes of hidden * weight, the row's sum of squares by parts of 512 columns
+__global__ __launch_bounds__(64) void short_norm_kernel(float* __restrict__ hidden, const float* __restrict__ part, int nsplit, size_t plane, const float* __restrict__ weight, int H,
+                                                        uint8_t* __restrict__ ws) {
+    const int lane = threadIdx.x, t = (int)blockIdx.y, col = (int)blockIdx.x * 512 + 32 * (lane >> 2) + 4 * (lane & 3);
+    float x[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    float ssq = 0.0f;
+    if (col < H) {
+        float r[8], w[8];
+        float* h = hidden + (size_t)t * H + col;
+        short_sums(h, 0, 1, r);
+        short_sums(weight + col, 0, 1, w);
+        if (nsplit > 0) {
+            short_sums(part + (size_t)t * H + col, plane, nsplit, x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] += r[e];   // (the residual last, as the other forms add it)
+            *reinterpret_cast<float4*>(h) = float4{x[0], x[1], x[2], x[3]};
+            *reinterpret_cast<float4*>(h + 16) = float4{x[4], x[5], x[6], x[7]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = r[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            ssq = fmaf(x[e], x[e], ssq);
+            x[e] *= w[e];
+        }
+    }
+#pragma unroll
+    for (int o = 1; o <= 32; o <<= 1) ssq += __shfl_xor(ssq, o, 64);
+    if (lane == 0) (reinterpret_cast<float*>(ws + ws_group_offset(H)) + ws_group_floats(H))[(int)blockIdx.x * GB_SHORT + t] = ssq;
+    short_split(x, lane, (int)blockIdx.x * 512, t, H, ws);
+}
+// planes of silu(gate) * up, both the sums of their splits
+__global__ __launch_bounds__(64) void short_silu_mul_kernel(const float* __restrict__ pg, const float* __restrict__ pu, int nsplit, size_t plane, int I, uint8_t* __restrict__ ws) {
+    const int lane = threadIdx.x, t = (int)blockIdx.y, col = (int)blockIdx.x * 512 + 32 * (lane >> 2) + 4 * (lane & 3);
+    float x[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (col < I) {
+        float u[8];
+        short_sums(pg + (size_t)t * I + col, plane, nsplit, x);
+        short_sums(pu + (size_t)t * I + col, plane, nsplit, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = x[e] / (1.0f + expf(-x[e])) * u[e];
+    }
+    short_split(x, lane, (int)blockIdx.x * 512, t, I, ws);
 }
 // tokens of the launch rounded up to the token blocks the matrix instructions read (16 per block; the 64-token form reads whole chunks)
 static inline int split_pad_tokens(int T) { return T <= 32 ? (T + 15) / 16 * 16 : (T + GB_TOK - 1) / GB_TOK * GB_TOK; }
@@ -1561,7 +1692,10 @@ struct GemmKParams {
     int nseg;
     const uint8_t* xb;      // operand planes of the (single) chunk
     const uint8_t* aux;     // its step sums (K-quant minimum term)
-    const float* inv;       // [T]: 1 / s
+    const float* group_inv; // [in / GB_GROUP][GB_SHORT]: 1 / s of a group of columns
+    const float* ssq;       // X is to be divided by its rows' root mean squares: [nssq][GB_SHORT] sums of squares, or null
+    int nssq;
+    float eps;
     const float* resid;     // (one slice only)
     int T, in, steps;
     unsigned row_bytes;
@@ -1614,6 +1748,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
 #endif
         }
     }
+    f32x4 inv_t[NTB];   // 1 / rms of the lane's tokens where X wants it, else 1
     for (int it = 0; it < p.jobs; ++it) {
     // this wave's tile (waves past the last tile only help with the copy)
     const int tile_raw = ((int)blockIdx.x + it * (int)gridDim.x) * NW + wave;
@@ -1670,11 +1805,16 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
         img[rt] = D::RP ? stage + rt * D::ITEM + 16 * i : stage + (rt * 16 + i) * STRIDE;
         my_row[rt] = (uint32_t)min(row0 + rt * 16 + i, seg_out - 1) * p.row_bytes;
     }
-    f32x4 acc[RT][NTB];
+    static_assert(SPU * 32 <= GB_GROUP, "a unit lies in one group of columns");
+    auto load_inv = [&](f32x4 (&v)[NTB], int unit) {
+#pragma unroll
+        for (int tb = 0; tb < NTB; ++tb) v[tb] = *reinterpret_cast<const f32x4*>(p.group_inv + (size_t)(unit * (SPU * 32) / GB_GROUP) * GB_SHORT + tb * 16 + 4 * g);
+    };
+    f32x4 sum[RT][NTB];   // the slice's sums; acc: a unit's, in its group's scale
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int tb = 0; tb < NTB; ++tb) acc[rt][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int tb = 0; tb < NTB; ++tb) sum[rt][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // ---- prologue of a row group: its first unit of weights goes out (HBM: the long round trip; for the first group, behind the planes' copy) ----
     // (scheduling barriers between the requests: the compiler counts its waits from their ORDER -- shuffled, it ends in vmcnt(0) at the head of every unit)
     u32x4 wreg[NLD];
@@ -1682,7 +1822,31 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
     load_unit(wreg, u_lo);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (D::HAS_MIN) { load_sums(svr, u_lo); __builtin_amdgcn_sched_barrier(0); }
-    if (it == 0) {   // (uniform) the planes have landed -- and with them this job's first weights; later jobs find the planes there
+    f32x4 ginv[NTB];
+    load_inv(ginv, u_lo);
+    __builtin_amdgcn_sched_barrier(0);
+    if (it == 0) {
+        // (requested behind the first weights and done with before the first row is stored: there, one request behind the other, the parts cost gate | up of 4096 inputs 2.4 us of
+        // 28.7, in front of the first weights Q | K | V 1.3 of 10.9)
+#pragma unroll
+        for (int tb = 0; tb < NTB; ++tb) {
+            inv_t[tb] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+            if (p.ssq) {   // (uniform)
+                const float* src = p.ssq + tb * 16 + 4 * g;
+                f32x4 q = *reinterpret_cast<const f32x4*>(src);
+                for (int k0 = 1; k0 < p.nssq; k0 += 8) {
+                    f32x4 v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const f32x4*>(src + min(k0 + k, p.nssq - 1) * GB_SHORT);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)
+                        if (k0 + k < p.nssq) q += v[k];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) inv_t[tb][e] = 1.0f / sqrtf(q[e] / (float)p.in + p.eps);
+            }
+        }
+        // the planes have landed -- and with them this job's first weights; later jobs find the planes there
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the compiler does not count the DMAs)
         __syncthreads();
     }
@@ -1705,6 +1869,15 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
                 load_sums(svr, min(u + 1, u_hi - 1));   // (same queue, same distance, consumption order: behind the unit's weights)
                 __builtin_amdgcn_sched_barrier(0);
             }
+            f32x4 gi[NTB], acc[RT][NTB];
+#pragma unroll
+            for (int tb = 0; tb < NTB; ++tb) {
+                gi[tb] = ginv[tb];
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            load_inv(ginv, min(u + 1, u_hi - 1));
+            __builtin_amdgcn_sched_barrier(0);
             const uint32_t uoff = (uint32_t)u * D::UB;
             typename D::Hdr hdr[RT];
             typename D::MinOp mop[RT];
@@ -1784,12 +1957,15 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
                         for (int e = 0; e < 4; ++e) acc[rt][tb][e] = fmaf(mop[rt].ndmin64, rr[rt][e], acc[rt][tb][e]);
                 }
             }
+#pragma unroll
+            for (int tb = 0; tb < NTB; ++tb)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[rt][tb][e] = fmaf(acc[rt][tb][e], gi[tb][e], sum[rt][tb][e]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        // ---- this wave's rows: accumulator element e of lane (i = row of the tile, g) is token tb * 16 + 4 g + e; 1 / s; Y or this slice's partial sums ----
-        f32x4 inv_t[NTB];
-#pragma unroll
-        for (int tb = 0; tb < NTB; ++tb) inv_t[tb] = *reinterpret_cast<const f32x4*>(p.inv + tb * 16 + 4 * g);   // (the array is padded to whole chunks)
+        // ---- this wave's rows: accumulator element e of lane (i = row of the tile, g) is token tb * 16 + 4 g + e; 1 / rms where X wants it; Y or this slice's partial sums ----
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const int r = row0 + rt * 16 + i;
@@ -1800,7 +1976,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
                 for (int e = 0; e < 4; ++e) {
                     const int t = tb * 16 + 4 * g + e;
                     if (t >= p.T) continue;
-                    const float y = acc[rt][tb][e] * inv_t[tb][e];
+                    const float y = sum[rt][tb][e] * inv_t[tb][e];
                     if (p.nsplit > 1) p.seg[sidx].part[((size_t)blockIdx.y * p.T + t) * seg_out + r] = y;
                     else { const size_t at = (size_t)t * seg_out + r; p.seg[sidx].Y[at] = p.resid ? y + p.resid[at] : y; }
                 }
@@ -2013,14 +2189,69 @@ __global__ __launch_bounds__(256) void reduce_silu_mul_rowmax_kernel(float* __re
 // one chunk's planes + sums (+ the record of zeros), rounded to 256 B
 // (the sums: whole units of 8 steps covering steps 0 .. in/32 + 7 -- the pre-pass writes a full unit of zeros behind the last step)
 
-constexpr size_t GB_SCALE_BYTES = 2 * GB_MAX_CHUNKS * GB_TOK * sizeof(float);   // the launch's 1 / s and s
+// ---- short prompts (<= 32 tokens): the plan of gemm_quant_f16_kslice_kernel, n == 0 where it does not take the launch ----
+// RT (16 or 32 rows per wave) and the number of K slices, by a two-term model of the launch -- rounds of workgroups over the 256 CUs x (steps of
+// a slice x RT + a fixed part worth `c0` steps: the copy of the planes, the first weights' round trip, the partial sums) -- over the slice counts that
+// keep the planes within LDS (gk_max_steps: 64 / NTB steps beside 16-row images, 48 / NTB beside 32-row ones) and the partial sums within their area.
+// (Four token blocks -- 33 .. 64 tokens -- were built and measured as well: 8B Q8_0 64 tokens 6.38 -> 8.74 ms, Q4_K_M 6.75 -> 9.57: 16-step slices, 8 - 28 of
+// them per matrix, and up to 58 MB of partial sums per launch; the 64-token chunk form keeps those.  profiles/r06_prompt_kslice.txt)
+// (Q8_0: -DNTK_GK_Q8_BLOCKS=8 runs this form in wide units, DeqI<NTK_DT_Q8_0 + GB_WIDE> -- measured slower: see there; the default keeps KDT = DT)
+struct KSlicePlan { int n = 0, rt = 0, ups = 0, jobs = 1; };
+template <int DT> constexpr int kslice_dt() { return (DT == NTK_DT_Q8_0 && NTK_GK_Q8_BLOCKS > 4) ? NTK_DT_Q8_0 + GB_WIDE : DT; }
+template <int DT>
+static KSlicePlan kslice_plan(const int* outs, int nseg, int T, int in) {
+    constexpr int KDT = kslice_dt<DT>();
+    using KD = DeqI<KDT>;
+    KSlicePlan best;
+    static const int kslice_env = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE", -1);   // (tuning builds only: 0 = never, n = up to n tokens)
+    const int kslice_max = kslice_env >= 0 ? kslice_env : GB_SHORT;
+    if (T > kslice_max || T > GB_SHORT || in % (32 * KD::SPU) != 0) return best;
+    const int ntb = T <= 16 ? 1 : 2;
+    const int units = in / (32 * KD::SPU);
+    static const int c0 = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_C0", 32), force_krt = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_RT", 0),
+                     force_kn = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_N", 0);   // (tuning builds only)
+    static const int c1 = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_C1", 8), max_jobs = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_JOBS", 64);   // (tuning builds only; JOBS=1: one row group per workgroup)
+    long out_total = 0;
+    for (int i = 0; i < nseg; ++i) out_total += outs[i];
+    double best_cost = 1e30;
+    for (int krt = 1; krt <= 2; ++krt) {
+        if (force_krt && krt != force_krt) continue;
+        // over the register budget (the build's ISA shows spills): 32 rows x 32 tokens of the K-quant decoders; the raw Q6_K decoder beyond 16 x 16
+        // (Q6_K: the same rule for the raw tensor and its repack -- they must take the same slices to give the same bits)
+        if ((krt == 2 && ntb >= 2 && (KD::SPLIT16 || KD::HAS_MIN)) || (KD::SPLIT16 && (krt == 2 || ntb >= 2))) continue;
+        int kt = 0;
+        for (int i = 0; i < nseg; ++i) kt += (outs[i] + 16 * krt - 1) / (16 * krt);
+        const int max_steps = krt == 1 ? (ntb == 1 ? gk_max_steps<KDT, 1, 1>() : gk_max_steps<KDT, 1, 2>()) : (ntb == 1 ? gk_max_steps<KDT, 2, 1>() : gk_max_steps<KDT, 2, 2>());
+        const int knw = krt == 1 ? (ntb == 1 ? gk_waves<KDT, 1, 1>() : gk_waves<KDT, 1, 2>()) : 8;
+        const int wgx = (kt + knw - 1) / knw, max_units = max_steps / KD::SPU;
+        if (max_units < 1) continue;
+        const int n_min = (units + max_units - 1) / max_units, n_cap = std::min(units, gb_split_rows((int)out_total));
+        for (int n = n_min; n <= n_cap; ++n) {
+            const int ups = units / n;
+            if (units % n != 0 || (force_kn && n != force_kn)) continue;   // (equal slices of whole units)
+            // rounds over the 256 CUs, folded into the workgroups (the planes are copied once): the fewest row groups per workgroup with which
+            // the whole grid -- ceil(wgx / jobs) x n -- is ONE round
+            int jobs = 1;
+            while (jobs < max_jobs && (long)((wgx + jobs - 1) / jobs) * n > 256) ++jobs;
+            const double cost = (double)jobs * (double)(ups * KD::SPU * krt) + c0 + (jobs - 1) * c1;
+            if (cost < best_cost) { best_cost = cost; best.n = n; best.rt = krt; best.ups = ups; best.jobs = jobs; }
+        }
+    }
+    return best;
+}
 
+// a launch whose planes a short prompt's producer has left in the workspace (short_split): nothing but gemm_quant_f16_kslice_kernel reads those
+struct ShortArgs {
+    bool on = false, norm = false;   // norm: X is to be divided by its rows' root mean squares (short_norm_kernel's sums)
+    float eps = 0.0f;
+    size_t part_at = 0, part_cap = 0;   // floats: where the launch's partial sums begin in their area, and the area's size
+};
 struct HostSeg { float* Y; const void* W; int out; };
 
 // T <= GB_MAX_CHUNKS * 64 = 1024 tokens in one launch; nseg matrices [out_s][in] of one format sharing X
 template <int DT>
 static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T, int in, const float* resid, void* ws, int reuse_x,
-                            const float* row_max, ntk_gemm_partials* defer, hipStream_t st) {
+                            const float* row_max, ntk_gemm_partials* defer, const ShortArgs& sh, hipStream_t st) {
     using D = DeqI<DT>;
     constexpr int TRIP = GB_UPT * D::SPU;   // steps per loop trip: K ranges are whole trips
     // whole units only (Q8_0: in a multiple of 128, Q4_0 and the K-quants: of 256): a partial last unit would decode the next row's bytes as
@@ -2048,63 +2279,33 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     p.aux = reinterpret_cast<const float*>(wsb + (size_t)(p.steps + 1) * GB_STEP_BYTES);
     float* scales = reinterpret_cast<float*>(wsb + (size_t)GB_MAX_CHUNKS * p.chunk_bytes);   // [inv: 1024][scale: 1024]
     p.inv = scales;
+    float* group_inv = reinterpret_cast<float*>(wsb + ws_group_offset(in));
     p.resid = resid;
     if (!reuse_x && row_max) {   // the tokens' largest |x| came with X: one pre-pass launch
         hipLaunchKernelGGL(split_x_kernel<true>, dim3(p.steps + 8, p.chunks), dim3(256), 0, st, X, T, in, reinterpret_cast<u32x4*>(wsb),
-                           const_cast<float*>(p.aux), p.chunk_bytes, row_max, scales);
+                           const_cast<float*>(p.aux), p.chunk_bytes, row_max, scales, group_inv);
     } else if (!reuse_x) {
         hipLaunchKernelGGL(row_scale_kernel, dim3((T + 3) / 4), dim3(256), 0, st, X, T, in, scales + GB_MAX_CHUNKS * GB_TOK, scales);
         hipLaunchKernelGGL(split_x_kernel<false>, dim3(p.steps + 8, p.chunks), dim3(256), 0, st, X, T, in, reinterpret_cast<u32x4*>(wsb),
-                           const_cast<float*>(p.aux), p.chunk_bytes, scales + GB_MAX_CHUNKS * GB_TOK, static_cast<float*>(nullptr));
+                           const_cast<float*>(p.aux), p.chunk_bytes, scales + GB_MAX_CHUNKS * GB_TOK, static_cast<float*>(nullptr), group_inv);
     }
     // ---- short prompts (<= 32 tokens), second form: K-slice-stationary (gemm_quant_f16_kslice_kernel) ----
-    // Plan: RT (16 or 32 rows per wave) and the number of K slices, by a two-term model of the launch -- rounds of workgroups over the 256 CUs x (steps of
-    // a slice x RT + a fixed part worth `c0` steps: the copy of the planes, the first weights' round trip, the partial sums) -- over the slice counts that
-    // keep the planes within LDS (gk_max_steps: 64 / NTB steps beside 16-row images, 48 / NTB beside 32-row ones) and the partial sums within their area.
-    static const int kslice_env = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE", -1);   // (tuning builds only: 0 = never, n = up to n tokens)
-    const int kslice_max = kslice_env >= 0 ? kslice_env : 32;
-    // (Four token blocks -- 33 .. 64 tokens -- were built and measured as well: 8B Q8_0 64 tokens 6.38 -> 8.74 ms, Q4_K_M 6.75 -> 9.57: 16-step slices, 8 - 28 of
-    // them per matrix, and up to 58 MB of partial sums per launch; the 64-token chunk form keeps those.  profiles/r06_prompt_kslice.txt)
-    // (Q8_0: -DNTK_GK_Q8_BLOCKS=16 or 8 runs this form in wide units, DeqI<NTK_DT_Q8_0 + GB_WIDE> -- measured slower: see there; the default keeps KDT = DT)
-    constexpr int KDT = (DT == NTK_DT_Q8_0 && NTK_GK_Q8_BLOCKS > 4) ? NTK_DT_Q8_0 + GB_WIDE : DT;
+    constexpr int KDT = kslice_dt<DT>();
     using KD = DeqI<KDT>;
-    if (T <= kslice_max && T <= 32 && in % (32 * KD::SPU) == 0) {
+    int outs[GB_MAX_SEG];
+    for (int i = 0; i < nseg; ++i) outs[i] = segs[i].out;
+    const KSlicePlan plan = kslice_plan<DT>(outs, nseg, T, in);
+    if (sh.on && (plan.n == 0 || sh.part_at + (size_t)plan.n * T * (size_t)out_total > sh.part_cap)) return NTK_E_SHAPE;   // (nothing launched: the planes were there)
+    {
         const int ntb = T <= 16 ? 1 : 2;
-        const int units = in / (32 * KD::SPU);
-        static const int c0 = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_C0", 32), force_krt = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_RT", 0),
-                         force_kn = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_N", 0);   // (tuning builds only)
-        static const int c1 = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_C1", 8), max_jobs = NTK_TUNE_ENV_INT("NTK_GEMM_KSLICE_JOBS", 64);   // (tuning builds only; JOBS=1: one row group per workgroup)
-        int best_n = 0, best_rt = 0, best_ups = 0, best_jobs = 1;
-        double best_cost = 1e30;
-        for (int krt = 1; krt <= 2; ++krt) {
-            if (force_krt && krt != force_krt) continue;
-            // over the register budget (the build's ISA shows spills): 32 rows x 32 tokens of the K-quant decoders; the raw Q6_K decoder beyond 16 x 16
-            // (Q6_K: the same rule for the raw tensor and its repack -- they must take the same slices to give the same bits)
-            if ((krt == 2 && ntb >= 2 && (KD::SPLIT16 || KD::HAS_MIN)) || (KD::SPLIT16 && (krt == 2 || ntb >= 2))) continue;
-            int kt = 0;
-            for (int i = 0; i < nseg; ++i) kt += (segs[i].out + 16 * krt - 1) / (16 * krt);
-            const int max_steps = krt == 1 ? (ntb == 1 ? gk_max_steps<KDT, 1, 1>() : gk_max_steps<KDT, 1, 2>()) : (ntb == 1 ? gk_max_steps<KDT, 2, 1>() : gk_max_steps<KDT, 2, 2>());
-            const int knw = krt == 1 ? (ntb == 1 ? gk_waves<KDT, 1, 1>() : gk_waves<KDT, 1, 2>()) : 8;
-            const int wgx = (kt + knw - 1) / knw, max_units = max_steps / KD::SPU;
-            if (max_units < 1) continue;
-            const int n_min = (units + max_units - 1) / max_units, n_cap = std::min(units, gb_split_rows((int)out_total));
-            for (int n = n_min; n <= n_cap; ++n) {
-                const int ups = units / n;
-                if (units % n != 0 || (force_kn && n != force_kn)) continue;   // (equal slices of whole units)
-                // rounds over the 256 CUs, folded into the workgroups (the planes are copied once): the fewest row groups per workgroup with which
-                // the whole grid -- ceil(wgx / jobs) x n -- is ONE round
-                int jobs = 1;
-                while (jobs < max_jobs && (long)((wgx + jobs - 1) / jobs) * n > 256) ++jobs;
-                const double cost = (double)jobs * (double)(ups * KD::SPU * krt) + c0 + (jobs - 1) * c1;
-                if (cost < best_cost) { best_cost = cost; best_n = n; best_rt = krt; best_ups = ups; best_jobs = jobs; }
-            }
-        }
+        const int best_n = plan.n, best_rt = plan.rt, best_ups = plan.ups, best_jobs = plan.jobs;
         if (best_n > 0) {
             GemmKParams kp{};
             kp.nseg = nseg; kp.T = T; kp.in = in; kp.steps = in / 32; kp.row_bytes = (unsigned)row_bytes;
-            kp.xb = wsb; kp.aux = reinterpret_cast<const uint8_t*>(p.aux); kp.inv = scales; kp.resid = best_n == 1 ? resid : nullptr;
+            kp.xb = wsb; kp.aux = reinterpret_cast<const uint8_t*>(p.aux); kp.group_inv = group_inv; kp.resid = best_n == 1 ? resid : nullptr;
             kp.nsplit = best_n; kp.units_per_split = best_ups;
-            float* kpart = reinterpret_cast<float*>(wsb + (size_t)GB_MAX_CHUNKS * p.chunk_bytes + GB_SCALE_BYTES);
+            if (sh.norm) { kp.ssq = group_inv + ws_group_floats(in); kp.nssq = (in + 511) / 512; kp.eps = sh.eps; }
+            float* kpart = reinterpret_cast<float*>(wsb + ws_part_offset(in)) + sh.part_at;
             int kt = 0;
             for (int i = 0; i < nseg; ++i) {
                 kp.seg[i].W = static_cast<const uint8_t*>(segs[i].W); kp.seg[i].Y = segs[i].Y; kp.seg[i].out = segs[i].out;
@@ -2243,7 +2444,7 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     int rt = out_total >= 2048 ? 2 : 1;
     if (force_rt == 1 || force_rt == 2) rt = force_rt;
     int tiles = 0;
-    float* part = reinterpret_cast<float*>(wsb + (size_t)GB_MAX_CHUNKS * p.chunk_bytes + GB_SCALE_BYTES);
+    float* part = reinterpret_cast<float*>(wsb + ws_part_offset(in));
     for (int i = 0; i < nseg; ++i) {
         p.seg[i].W = static_cast<const uint8_t*>(segs[i].W);
         p.seg[i].Y = segs[i].Y;
@@ -2346,12 +2547,12 @@ __attribute__((visibility("default"))) int ntk_debug_gemm_f16_clock(unsigned lon
 
 size_t ntk_gemm_quant_workspace_bytes(int in_features, int out_features) {
     if (in_features <= 0 || out_features < 0) return 0;
-    return (size_t)ntk::GB_MAX_CHUNKS * ntk::ws_chunk_bytes((in_features + 31) / 32 * 32) + ntk::GB_SCALE_BYTES +
+    return ntk::ws_part_offset((in_features + 31) / 32 * 32) +
            (size_t)ntk::gb_split_rows(out_features) * ntk::GB_TOK * (size_t)out_features * sizeof(float) + 256;
 }
 
 static int gemm_ws_dispatch(const ntk::HostSeg* segs, int nseg, const float* X, int n_tokens, int in_features, int weight_dtype, const float* resid,
-                            void* workspace, int reuse_x, const float* row_max, ntk_gemm_partials* defer, hipStream_t st) {
+                            void* workspace, int reuse_x, const float* row_max, ntk_gemm_partials* defer, const ntk::ShortArgs& sh, hipStream_t st) {
     // (weight_dtype + ntk::GB_RP: the matrices are tensors of the engine's decode repack)
     constexpr int PASS = ntk::GB_MAX_CHUNKS * ntk::GB_TOK;
     if (n_tokens > PASS) reuse_x = 0;   // the planes hold one pass (1024 tokens) at a time
@@ -2369,14 +2570,14 @@ static int gemm_ws_dispatch(const ntk::HostSeg* segs, int nseg, const float* X, 
         const float* rm = row_max ? row_max + t0 : nullptr;
         int rc;
         switch (weight_dtype) {
-            case NTK_DT_Q8_0: rc = ntk::launch_gemm_f16<NTK_DT_Q8_0>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            case NTK_DT_Q4_0: rc = ntk::launch_gemm_f16<NTK_DT_Q4_0>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            case NTK_DT_Q4_K: rc = ntk::launch_gemm_f16<NTK_DT_Q4_K>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            case NTK_DT_Q5_K: rc = ntk::launch_gemm_f16<NTK_DT_Q5_K>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            case NTK_DT_Q4_K + ntk::GB_RP: rc = ntk::launch_gemm_f16<NTK_DT_Q4_K + ntk::GB_RP>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            case NTK_DT_Q5_K + ntk::GB_RP: rc = ntk::launch_gemm_f16<NTK_DT_Q5_K + ntk::GB_RP>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            case NTK_DT_Q6_K + ntk::GB_RP: rc = ntk::launch_gemm_f16<NTK_DT_Q6_K + ntk::GB_RP>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
-            default: rc = ntk::launch_gemm_f16<NTK_DT_Q6_K>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, st); break;
+            case NTK_DT_Q8_0: rc = ntk::launch_gemm_f16<NTK_DT_Q8_0>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            case NTK_DT_Q4_0: rc = ntk::launch_gemm_f16<NTK_DT_Q4_0>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            case NTK_DT_Q4_K: rc = ntk::launch_gemm_f16<NTK_DT_Q4_K>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            case NTK_DT_Q5_K: rc = ntk::launch_gemm_f16<NTK_DT_Q5_K>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            case NTK_DT_Q4_K + ntk::GB_RP: rc = ntk::launch_gemm_f16<NTK_DT_Q4_K + ntk::GB_RP>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            case NTK_DT_Q5_K + ntk::GB_RP: rc = ntk::launch_gemm_f16<NTK_DT_Q5_K + ntk::GB_RP>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            case NTK_DT_Q6_K + ntk::GB_RP: rc = ntk::launch_gemm_f16<NTK_DT_Q6_K + ntk::GB_RP>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
+            default: rc = ntk::launch_gemm_f16<NTK_DT_Q6_K>(sg, nseg, x, T, in_features, rs, workspace, reuse_x, rm, defer, sh, st); break;
         }
         if (rc != NTK_OK) return rc;
     }
@@ -2385,7 +2586,7 @@ static int gemm_ws_dispatch(const ntk::HostSeg* segs, int nseg, const float* X, 
 
 // The FP16 GEMM behind its descriptor (include/ntk_engine.h: ntk_gemm_desc): 1..3 matrices of one format sharing X, optional residual (one matrix),
 // optional token maxima, optional deferral of the split-K sums to the consuming launch.
-int ntk_gemm_quant_f16(const ntk_gemm_desc* d, void* stream) {
+static int gemm_quant_f16_with(const ntk_gemm_desc* d, const ntk::ShortArgs& sh, void* stream) {
     if (!d || !d->segs || !d->X || !d->workspace) return NTK_E_NULL;
     const int nseg = d->nseg, n_tokens = d->n_tokens, in_features = d->in_features;
     if (nseg < 1 || nseg > ntk::GB_MAX_SEG || n_tokens < 0 || in_features <= 0 || (d->resid && nseg != 1)) return NTK_E_SHAPE;
@@ -2411,7 +2612,71 @@ int ntk_gemm_quant_f16(const ntk_gemm_desc* d, void* stream) {
     }
     if (n_tokens == 0 || total == 0) return NTK_OK;
     // (resid with partials: added by the launch's own epilogue when it does not split K -- nothing is deferred then; left to the consumer when it does)
-    return gemm_ws_dispatch(sg, nseg, d->X, n_tokens, in_features, dt, d->resid, d->workspace, d->reuse_x, d->row_max, defer, ntk::resolve_stream(stream));
+    return gemm_ws_dispatch(sg, nseg, d->X, n_tokens, in_features, dt, d->resid, d->workspace, d->reuse_x, d->row_max, defer, sh, ntk::resolve_stream(stream));
+}
+int ntk_gemm_quant_f16(const ntk_gemm_desc* d, void* stream) { return gemm_quant_f16_with(d, ntk::ShortArgs{}, stream); }
+
+// ---- short prompts: planes scaled per 256 columns by their producers (include/ntk_engine.h) ----
+int ntk_gemm_short_takes(const int* rows, int nseg, int n_tokens, int in_features, int dtype) {
+    if (!rows || nseg < 1 || nseg > ntk::GB_MAX_SEG || n_tokens < 2 || in_features <= 0) return 0;
+    for (int i = 0; i < nseg; ++i)
+        if (rows[i] <= 0 || rows[i] % 16 != 0) return 0;
+    switch (dtype) {   // (a tensor and its repack: the same slices)
+        case NTK_DT_Q8_0: return ntk::kslice_plan<NTK_DT_Q8_0>(rows, nseg, n_tokens, in_features).n > 0;
+        case NTK_DT_Q4_0: return ntk::kslice_plan<NTK_DT_Q4_0>(rows, nseg, n_tokens, in_features).n > 0;
+        case NTK_DT_Q4_K: return ntk::kslice_plan<NTK_DT_Q4_K>(rows, nseg, n_tokens, in_features).n > 0;
+        case NTK_DT_Q5_K: return ntk::kslice_plan<NTK_DT_Q5_K>(rows, nseg, n_tokens, in_features).n > 0;
+        case NTK_DT_Q6_K: return ntk::kslice_plan<NTK_DT_Q6_K>(rows, nseg, n_tokens, in_features).n > 0;
+        default: return 0;
+    }
+}
+int ntk_gemm_short(const ntk_gemm_desc* d, int normed, float eps, size_t part_at, void* stream) {
+    if (!d) return NTK_E_NULL;
+    if (d->n_tokens < 1 || d->n_tokens > ntk::GB_SHORT || d->in_features <= 0 || part_at % 4 != 0) return NTK_E_SHAPE;
+    const size_t head = ntk::ws_part_offset((d->in_features + 31) / 32 * 32);
+    if (d->workspace_bytes < head) return NTK_E_SHAPE;
+    ntk::ShortArgs sh;
+    sh.on = true; sh.norm = normed != 0; sh.eps = eps; sh.part_at = part_at; sh.part_cap = (d->workspace_bytes - head) / sizeof(float);
+    ntk_gemm_desc e = *d;
+    e.reuse_x = 1;
+    if (!e.X) e.X = static_cast<const float*>(e.workspace);   // (never read)
+    return gemm_quant_f16_with(&e, sh, stream);
+}
+static int short_check(int T, int in, const void* workspace, uintptr_t ptrs) {
+    if (!workspace) return NTK_E_NULL;
+    if (T < 1 || T > ntk::GB_SHORT || in <= 0 || in % 32 != 0) return NTK_E_SHAPE;
+    return ((ptrs | reinterpret_cast<uintptr_t>(workspace)) & 15) ? NTK_E_ALIGN : NTK_OK;
+}
+int ntk_short_prepare_x(const float* X, int n_tokens, int in_features, void* workspace, void* stream) {
+    if (!X) return NTK_E_NULL;
+    const int rc = short_check(n_tokens, in_features, workspace, reinterpret_cast<uintptr_t>(X));
+    if (rc != NTK_OK) return rc;
+    hipLaunchKernelGGL(ntk::short_split_kernel, dim3((in_features + 511) / 512, n_tokens), dim3(64), 0, ntk::resolve_stream(stream), X, in_features, static_cast<uint8_t*>(workspace));
+    return ntk::last_launch_status();
+}
+int ntk_short_norm_prepare_x(float* hidden, const ntk_gemm_partials* p, const float* weight, int n_tokens, int hidden_size, void* workspace, void* stream) {
+    if (!hidden || !weight) return NTK_E_NULL;
+    const float* part = p ? p->part[0] : nullptr;
+    int nsplit = part ? p->nsplit : 0;
+    if (p && (p->nseg != 1 || p->n_tokens != n_tokens || p->rows[0] != hidden_size || p->nsplit < 1)) return NTK_E_SHAPE;
+    if (p && !part && p->y[0] != hidden) { part = p->y[0]; nsplit = 1; }   // (a launch of one slice wrote Y itself: over hidden with the residual inside, or elsewhere)
+    const int rc = short_check(n_tokens, hidden_size, workspace, reinterpret_cast<uintptr_t>(hidden) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(part));
+    if (rc != NTK_OK) return rc;
+    hipLaunchKernelGGL(ntk::short_norm_kernel, dim3((hidden_size + 511) / 512, n_tokens), dim3(64), 0, ntk::resolve_stream(stream), hidden, part, nsplit,
+                       (size_t)n_tokens * hidden_size, weight, hidden_size, static_cast<uint8_t*>(workspace));
+    return ntk::last_launch_status();
+}
+int ntk_short_silu_mul_prepare_x(const ntk_gemm_partials* p, void* workspace, void* stream) {
+    if (!p) return NTK_E_NULL;
+    if (p->nseg != 2 || p->rows[0] != p->rows[1] || p->nsplit < 1) return NTK_E_SHAPE;
+    const bool sums = p->part[0] && p->part[1];
+    const float *g = sums ? p->part[0] : p->y[0], *u = sums ? p->part[1] : p->y[1];
+    if (!g || !u) return NTK_E_NULL;
+    const int rc = short_check(p->n_tokens, p->rows[0], workspace, reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(u));
+    if (rc != NTK_OK) return rc;
+    hipLaunchKernelGGL(ntk::short_silu_mul_kernel, dim3((p->rows[0] + 511) / 512, p->n_tokens), dim3(64), 0, ntk::resolve_stream(stream), g, u, sums ? p->nsplit : 1,
+                       (size_t)p->n_tokens * p->rows[0], p->rows[0], static_cast<uint8_t*>(workspace));
+    return ntk::last_launch_status();
 }
 
 // hidden[t] += W . X[t] (the projection's splits summed here, residual last) and x_out[t] = rmsnorm(hidden[t]) with its largest |x|

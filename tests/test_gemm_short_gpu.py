@@ -1,0 +1,157 @@
+"""Short prompts' projections over planes that their producers scale per token and 256 columns (ntk_short_*_prepare_x, ntk_gemm_short), against float64 products of the oracle's dequantised
+weights: one block of 16 tokens and two, single tokens and whole blocks, rows that end inside a wave's 512 columns or inside a group, groups of very different size, one slice and several.
+
+Tolerance, of the root of the sum of the products' squares: four times the 1.1e-6 that the oracle's own float32 products show on such matrices (2304 inputs; Q8_0 3.8e-7, Q4_K 6.1e-7, Q6_K
+1.1e-6: sums in any order)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from ntransformer_amd import _lib
+from ntransformer_amd import gguf as G
+from ntransformer_amd.ops import DeviceBuffer as DB
+from oracle import arbiter
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+REL = 4.4e-6
+VP = C.c_void_p
+
+
+def lib():
+    L = _lib.lib()
+    L.ntk_gemm_quant_workspace_bytes.restype = C.c_size_t
+    L.ntk_gemm_quant_workspace_bytes.argtypes = [C.c_int, C.c_int]
+    L.ntk_gemm_short_takes.argtypes = [C.POINTER(C.c_int)] + [C.c_int] * 4
+    L.ntk_short_prepare_x.argtypes = [VP, C.c_int, C.c_int, VP, VP]
+    L.ntk_short_norm_prepare_x.argtypes = [VP, C.POINTER(_lib.GemmPartials), VP, C.c_int, C.c_int, VP, VP]
+    L.ntk_short_silu_mul_prepare_x.argtypes = [C.POINTER(_lib.GemmPartials), VP, VP]
+    L.ntk_gemm_short.argtypes = [C.POINTER(_lib.GemmDesc), C.c_int, C.c_float, C.c_size_t, VP]
+    return L
+
+
+def product(L, ws, nbytes, weights, ys, rows, dt, T, inf, normed=0, eps=0.0, resid=None, partials=None, part_at=0):
+    segs = (_lib.GemvSeg * len(weights))()
+    for i, (w, y) in enumerate(zip(weights, ys)):
+        segs[i].W, segs[i].y, segs[i].rows, segs[i].dtype = w.ptr, y.ptr, rows, dt
+    d = _lib.GemmDesc()
+    d.segs, d.nseg, d.n_tokens, d.in_features, d.resid = segs, len(weights), T, inf, None if resid is None else resid.ptr
+    d.workspace, d.workspace_bytes = ws.ptr, nbytes
+    d.partials = C.pointer(partials) if partials is not None else None
+    _lib.check(L.ntk_gemm_short(C.byref(d), normed, eps, part_at, None), "gemm_short")
+
+
+def weights(r, gt, rows, inf):
+    raw = np.frombuffer(G.synth_tensor(r, gt, rows, inf), np.uint8)
+    dt = G.GGML_TO_DT[gt]
+    return raw, arbiter.dequant(raw, rows, inf, dt).astype(np.float64).reshape(rows, inf), dt
+
+
+def close(got, W, X):
+    """got [T, rows] against W . X, by the products' sizes"""
+    want = X @ W.T
+    size = np.sqrt((X ** 2) @ (W ** 2).T)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - want) <= REL * size + 1e-30).all(), float((np.abs(got - want) / (size + 1e-30)).max())
+
+
+@pytest.mark.parametrize("qname", ["Q8_0", "Q4_0", "Q4_K", "Q5_K", "Q6_K"])
+@pytest.mark.parametrize("T,rows,inf", [(1, 16, 256), (2, 48, 768), (16, 256, 1280), (17, 128, 512), (32, 64, 2304), (5, 2064, 256)])
+def test_products_of_grouped_planes(qname, T, rows, inf):
+    gt = getattr(G, "GGML_" + qname)
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[T, rows + inf]))
+    dims = [(rows, inf)] + ([(rows, inf + 128)] if qname == "Q8_0" else [])      # Q8_0: a last group of half the columns, too
+    for rows, inf in dims:
+        one, two = (C.c_int * 1)(rows), (C.c_int * 2)(rows, rows)
+        raw, W, dt = weights(r, gt, rows, inf)
+        if not (L.ntk_gemm_short_takes(one, 1, max(T, 2), inf, dt) and L.ntk_gemm_short_takes(two, 2, max(T, 2), inf, dt)):
+            assert qname == "Q6_K" and T > 16                                     # (32 tokens of the format that scales per 16 columns)
+            continue
+        Wd = DB.from_numpy(raw)
+        nbytes = L.ntk_gemm_quant_workspace_bytes(inf, 2 * rows)
+        ws, ws2 = DB(nbytes), DB(nbytes)
+        X = r.standard_normal((T, inf)).astype(np.float32)
+        X[:, 64:320] *= np.float32(1e4)                                           # groups of different sizes, zeros, one tiny and one huge row
+        X[T // 2, : inf // 2] = 0.0
+        X[0] *= np.float32(1e12)
+        X[T - 1] *= np.float32(1e-12)
+        y = DB.from_numpy(np.full((T, rows), 7.0, np.float32))
+        _lib.check(L.ntk_short_prepare_x(DB.from_numpy(X).ptr, T, inf, ws.ptr, None), "short_prepare_x")
+        product(L, ws, nbytes, [Wd], [y], rows, dt, T, inf)
+        close(y.numpy(np.float32).reshape(T, rows).astype(np.float64), W, X.astype(np.float64))
+        # RMSNorm in front, a residual behind
+        eps, nw = 1e-5, (1.0 + 0.1 * r.standard_normal(inf)).astype(np.float32)
+        res = r.standard_normal((T, rows)).astype(np.float32)
+        hd = DB.from_numpy(X)
+        _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, None, DB.from_numpy(nw).ptr, T, inf, ws.ptr, None), "short_norm")
+        y = DB.from_numpy(res)
+        product(L, ws, nbytes, [Wd], [y], rows, dt, T, inf, 1, eps, y)
+        assert np.array_equal(hd.numpy(np.float32).reshape(T, inf), X)
+        x64 = X.astype(np.float64)
+        n64 = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + eps) * nw
+        got = y.numpy(np.float32).reshape(T, rows).astype(np.float64)
+        size = np.sqrt((n64 ** 2) @ (W ** 2).T) + np.abs(res)
+        assert (np.abs(got - (res + n64 @ W.T)) <= REL * size).all()
+        # sums of a gate | up launch -> silu * up -> sums of the next product -> its norm
+        if rows % (128 if qname == "Q8_0" else 256) or not L.ntk_gemm_short_takes((C.c_int * 1)(rows), 1, max(T, 2), rows, dt):
+            continue
+        pt = _lib.GemmPartials()
+        small = np.float32(1e-3) * r.standard_normal((T, inf)).astype(np.float32)
+        xd = DB.from_numpy(small)
+        _lib.check(L.ntk_short_prepare_x(xd.ptr, T, inf, ws.ptr, None), "short_prepare_x")
+        g, u = DB.zeros(T * rows * 4), DB.zeros(T * rows * 4)
+        product(L, ws, nbytes, [Wd, Wd], [g, u], rows, dt, T, inf, partials=pt)
+        raw2, W2, _ = weights(r, gt, rows, rows)
+        nb2 = L.ntk_gemm_quant_workspace_bytes(rows, 2 * rows)
+        wa, wb = DB(nb2), DB(nb2)
+        _lib.check(L.ntk_short_silu_mul_prepare_x(C.byref(pt), wa.ptr, None), "short_silu")
+        h0 = r.standard_normal((T, rows)).astype(np.float32)
+        hd = DB.from_numpy(h0)
+        pt2 = _lib.GemmPartials()
+        product(L, wa, nb2, [DB.from_numpy(raw2)], [hd], rows, dt, T, rows, resid=hd, partials=pt2)
+        nw = (1.0 + 0.1 * r.standard_normal(rows)).astype(np.float32)
+        _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, C.byref(pt2), DB.from_numpy(nw).ptr, T, rows, wb.ptr, None), "short_norm")
+        gv = small.astype(np.float64) @ W.T
+        a = gv / (1.0 + np.exp(-gv)) * gv
+        got = hd.numpy(np.float32).reshape(T, rows).astype(np.float64)
+        # (the unit's own rounding beside the product's: gate and up carry REL of their sums' sizes each)
+        ga = np.sqrt((small.astype(np.float64) ** 2) @ (W ** 2).T)
+        ua = np.abs(gv) + ga
+        size = np.sqrt((a ** 2) @ (W2 ** 2).T) + np.sqrt((2 * ga * ua) ** 2 @ (W2 ** 2).T) + np.abs(h0)
+        assert (np.abs(got - (h0 + a @ W2.T)) <= REL * size).all()
+        y = DB.zeros(T * rows * 4)
+        product(L, wb, nb2, [DB.from_numpy(raw2)], [y], rows, dt, T, rows, 1, eps)
+        n64 = got / np.sqrt((got ** 2).mean(1, keepdims=True) + eps) * nw
+        close(y.numpy(np.float32).reshape(T, rows).astype(np.float64), W2, n64)
+
+
+def test_sums_side_by_side_and_what_is_refused():
+    """two launches of different formats leave their sums in one workspace; shapes and sizes that the form does not take launch nothing"""
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[3, 9]))
+    T, rows, inf = 16, 256, 2048
+    raws = [np.frombuffer(G.synth_tensor(r, gt, rows, inf), np.uint8) for gt in (G.GGML_Q4_K, G.GGML_Q6_K)]
+    dts = [G.GGML_TO_DT[gt] for gt in (G.GGML_Q4_K, G.GGML_Q6_K)]
+    X = r.standard_normal((T, inf)).astype(np.float32)
+    nbytes = L.ntk_gemm_quant_workspace_bytes(inf, 2 * rows)
+    ws = DB(nbytes)
+    _lib.check(L.ntk_short_prepare_x(DB.from_numpy(X).ptr, T, inf, ws.ptr, None), "short_prepare_x")
+    bufs, sums, at = [DB.from_numpy(a) for a in raws], [], 0
+    pts = [_lib.GemmPartials(), _lib.GemmPartials()]
+    for w, dt, pt in zip(bufs, dts, pts):
+        y = DB.zeros(T * rows * 4)
+        product(L, ws, nbytes, [w], [y], rows, dt, T, inf, partials=pt, part_at=at)
+        assert pt.nsplit > 1
+        at += pt.nsplit * T * rows
+    assert pts[1].part[0] - pts[0].part[0] == pts[0].nsplit * T * rows * 4
+    for raw, dt, pt in zip(raws, dts, pts):
+        h = DB.zeros(T * rows * 4)
+        _lib.check(L.ntk_short_norm_prepare_x(h.ptr, C.byref(pt), DB.from_numpy(np.ones(rows, np.float32)).ptr, T, rows, DB(nbytes).ptr, None), "short_norm")
+        want = np.stack([O.gemv(raw, x, rows, inf, dt) for x in X]).astype(np.float64)
+        got = h.numpy(np.float32).reshape(T, rows)
+        assert np.abs(got - want).max() <= REL * 8 * np.abs(want).max()
+    one = (C.c_int * 1)(rows)
+    dt = dts[0]
+    assert not L.ntk_gemm_short_takes(one, 1, 33, inf, dt) and not L.ntk_gemm_short_takes(one, 1, 16, inf + 32, dt)
+    assert not L.ntk_gemm_short_takes((C.c_int * 1)(24), 1, 16, inf, dt) and not L.ntk_gemm_short_takes(one, 1, 16, inf, 0)
+    assert L.ntk_short_prepare_x(ws.ptr, 33, inf, ws.ptr, None) != 0 and L.ntk_short_prepare_x(ws.ptr, 4, 40, ws.ptr, None) != 0
