@@ -229,6 +229,12 @@ int ntk_short_prepare_x(const float* X, int n_tokens, int in_features, void* wor
 int ntk_short_norm_prepare_x(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int hidden_size, void* workspace, void* stream);
 int ntk_short_silu_mul_prepare_x(const ntk_gemm_partials* partials, void* workspace, void* stream);
 int ntk_gemm_short(const ntk_gemm_desc* desc, int normed, float eps, size_t part_at, void* stream);
+/* A prompt of at most 32 tokens from position 0 on: ntk_reduce_rope_kv_store, ntk_attention_prefill and ntk_short_prepare_x of its result in one launch.  sums / splits: of q, k and v as in
+ * ntk_reduce_rope_kv_store; angles: ntk_short_angles' table (ntk_short_angles_bytes, 16-byte aligned), formed once a model.  head_dim 128, an even number of heads (NTK_E_SHAPE). */
+size_t ntk_short_angles_bytes(int head_dim);
+int ntk_short_angles(float* table, int head_dim, float theta_base, float freq_scale, void* stream);
+int ntk_short_attention(const float* const* sums, const int* splits, const float* angles, int n_tokens, int n_heads, int n_kv_heads, int head_dim, float scale, int interleaved, void* k_cache,
+                        void* v_cache, int max_seq, void* workspace, void* stream);
 
 /* Y[t][0..out) (+)= W . X[t] for the tokens of a prompt over IEEE-half weights ([out][in] row-major), one pass over W: the batched form of n_tokens ntk_gemv calls.
  * row_max: the tokens' largest |X| where their producer left it (ntk_rmsnorm_rowmax ...), NULL: taken here.  workspace (16-byte aligned): without row_max at least

@@ -26,14 +26,11 @@
 // Bound: MFMA (64 MFMAs = 1024 cycles per 16 queries x 64 keys and SIMD; the softmax adds ~200 VALU instructions per tile).
 #include "common.hip.h"
 #include "attention_merge.hip.h"
+#include "gemm_planes.hip.h"
 
 namespace ntk {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int AM_QT = 64;     // queries per workgroup
 constexpr int AM_KT = 64;     // cache rows per tile
@@ -233,6 +230,204 @@ int launch_attention_prefill_mfma(float* out, const float* Q, const uint16_t* kc
     const dim3 grid(nh, (T + AM_QT - 1) / AM_QT);
     hipLaunchKernelGGL(attention_prefill_mfma_kernel, grid, dim3(256), 0, st, out, Q, kc, vc, T, start_pos, nh, nkv, scale);
     return last_launch_status();
+}
+
+// =================================================================================================================================
+// A short prompt from its first token on (<= 32 tokens, head_dim 128): the sums of the projections' K splits, the rotation, the cache rows, attention over the prompt itself and the planes of
+// its result for the output projection (gemm_planes.hip.h) in ONE launch: 8.7 us for 16 tokens of 32 + 8 heads, 4.6 + 6.7 + 2.8 as three, each a launch's own boundary and a few
+// thousand cycles.  Workgroup = two query heads (one group of 256 columns of the result), 16 waves: they add up and rotate queries, keys and values side by
+// side, then a wave takes 16 of a head's 128 dimensions.  Arithmetic, orders and roundings are rope_kv_store_parts_kernel's and attention_prefill_mfma_kernel's: the caches hold
+// the same bits.  Bound: what a CU reads (the sums of two heads' queries, and of their keys and values once for every four heads: 130 - 260 KB) and the chain of four steps.
+// =================================================================================================================================
+struct ShortSource { const float* p; int n; size_t plane; };
+constexpr int SA_QSTR = AM_HD + 4, SA_KSTR = AM_HD + 8, SA_VSTR = 36;
+template <int TP> constexpr int sa_lds(int slots) { return 2 * TP * SA_QSTR * 4 + slots * (TP * SA_KSTR + AM_HD * SA_VSTR) * 2; }
+
+// the sums, in split order, of two groups of four neighbours (d1: how far the second lies behind the first); nine splits in one round trip
+__device__ __forceinline__ void sa_sums2(const ShortSource& s, size_t at, int d1, f32x4& a, f32x4& b) {
+    a = *reinterpret_cast<const f32x4*>(s.p + at);
+    b = *reinterpret_cast<const f32x4*>(s.p + at + d1);
+    for (int s0 = 1; s0 < s.n; s0 += 8) {
+        f32x4 qa[8], qb[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float* r = s.p + (size_t)min(s0 + k, s.n - 1) * s.plane + at;
+            qa[k] = *reinterpret_cast<const f32x4*>(r);
+            qb[k] = *reinterpret_cast<const f32x4*>(r + d1);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (s0 + k < s.n) { a += qa[k]; b += qb[k]; }   // (uniform)
+    }
+}
+
+// cosines and sines of the first GB_SHORT positions' angles, [2][GB_SHORT][head_dim / 2], by rope_kv_store_parts_kernel's expressions: a model's constant.  (Formed in the launch itself --
+// eight functions a thread -- they were a third of its time: 9.6 us of 16 tokens of 32 + 8 heads against 8.7.)
+__global__ __launch_bounds__(256) void short_angles_kernel(float* __restrict__ table, int half_dim, float theta, float fscale) {
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= GB_SHORT * half_dim) return;
+    const int t = idx / half_dim, i = idx - t * half_dim;
+    const float freq = 1.0f / (float)pow((double)theta, (double)((2.0f * i) / (2 * half_dim)));
+    const float angle = t * freq * fscale;
+    table[idx] = cosf(angle);
+    table[GB_SHORT * half_dim + idx] = sinf(angle);
+}
+
+template <int TP>
+__global__ __launch_bounds__(1024) void short_attention_kernel(const ShortSource sq, const ShortSource sk, const ShortSource sv, const float* __restrict__ table, int interleaved,
+                                                              int T, int n_heads, int n_kv_heads, float scale, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, uint8_t* __restrict__ ws) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t sa_smem[];
+    float* qs = reinterpret_cast<float*>(sa_smem);                                            // [2 heads][TP][SA_QSTR]: rotated queries x scale, later the result
+    uint16_t* kt = reinterpret_cast<uint16_t*>(sa_smem + 2 * TP * SA_QSTR * 4);               // [slots][TP][SA_KSTR]
+    const int h0 = 2 * (int)blockIdx.x, group = n_heads / n_kv_heads;
+    const int kv0 = h0 / group, slots = (h0 + 1) / group == kv0 ? 1 : 2;
+    uint16_t* vt = kt + slots * TP * SA_KSTR;                                                 // [slots][128][SA_VSTR], transposed
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per_pos = n_kv_heads * AM_HD, per_q = n_heads * AM_HD;
+
+    // ---- sums, rotation, cache rows.  Items: (head, token, j): four pairs at columns 4 j and 4 j + 64, or (neighbours rotated) eight neighbours 8 j
+    auto rotate = [&](const f32x4& a, const f32x4& b, int t, int j, f32x4& ra, f32x4& rb) {
+        const f32x4 c = *reinterpret_cast<const f32x4*>(table + t * 64 + 4 * j), sn = *reinterpret_cast<const f32x4*>(table + (GB_SHORT + t) * 64 + 4 * j);
+        if (interleaved) {   // pairs (0, 1) (2, 3) of a, then of b: pair index 4 j + ...
+            float o[8];
+            const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) rope_rotate(v[2 * e], v[2 * e + 1], c[e], sn[e], o[2 * e], o[2 * e + 1]);
+            ra = f32x4{o[0], o[1], o[2], o[3]};
+            rb = f32x4{o[4], o[5], o[6], o[7]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float x, y;
+                rope_rotate(a[e], b[e], c[e], sn[e], x, y);
+                ra[e] = x;
+                rb[e] = y;
+            }
+        }
+    };
+    const int step1 = interleaved ? 4 : 64;
+    auto column = [&](int j) { return interleaved ? 8 * j : 4 * j; };
+    auto halves = [](const f32x4& v) { return u32x2{(uint32_t)f2h(v[0]) | ((uint32_t)f2h(v[1]) << 16), (uint32_t)f2h(v[2]) | ((uint32_t)f2h(v[3]) << 16)}; };
+    // (eight waves queries, four keys, four values: one after the other the three round trips cost 10.7 us a launch of 16 tokens, side by side 9.6)
+    if (tid >= 768)
+    for (int it = tid - 768; it < slots * TP * 16; it += 256) {   // values: eight neighbours an item
+        const int j = it & 15, t = (it >> 4) % TP, sl = it / (16 * TP);
+        f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+        if (t < T) {
+            const size_t at = (size_t)t * per_pos + (size_t)(kv0 + sl) * AM_HD + 8 * j;
+            sa_sums2(sv, at, 4, a, b);
+            if (((kv0 + sl) * group) / 2 == (int)blockIdx.x) {   // (the KV head's first query head's workgroup)
+                const u32x2 lo = halves(a), hi = halves(b);
+                *reinterpret_cast<u32x4*>(vc + at) = u32x4{lo.x, lo.y, hi.x, hi.y};
+            }
+        }
+        uint16_t* col = vt + (sl * AM_HD + 8 * j) * SA_VSTR + t;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            col[e * SA_VSTR] = f2h(a[e]);
+            col[(4 + e) * SA_VSTR] = f2h(b[e]);
+            if constexpr (TP == 16) { col[e * SA_VSTR + 16] = 0; col[(4 + e) * SA_VSTR + 16] = 0; }   // (the matrix instruction takes 32 keys)
+        }
+    }
+    else if (tid >= 512)
+    for (int it = tid - 512; it < slots * TP * 16; it += 256) {   // keys
+        const int j = it & 15, t = (it >> 4) % TP, sl = it / (16 * TP);
+        f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+        if (t < T) {
+            f32x4 x, y;
+            const size_t at = (size_t)t * per_pos + (size_t)(kv0 + sl) * AM_HD + column(j);
+            sa_sums2(sk, at, step1, x, y);
+            rotate(x, y, t, j, a, b);
+            if (((kv0 + sl) * group) / 2 == (int)blockIdx.x) {
+                *reinterpret_cast<u32x2*>(kc + at) = halves(a);
+                *reinterpret_cast<u32x2*>(kc + at + step1) = halves(b);
+            }
+        }
+        uint16_t* row = kt + (sl * TP + t) * SA_KSTR + column(j);
+        *reinterpret_cast<u32x2*>(row) = halves(a);
+        *reinterpret_cast<u32x2*>(row + step1) = halves(b);
+    }
+    else
+    for (int it = tid; it < 2 * TP * 16; it += 512) {       // queries
+        const int j = it & 15, t = (it >> 4) % TP, hd = it / (16 * TP);
+        f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+        if (t < T) {
+            f32x4 x, y;
+            sa_sums2(sq, (size_t)t * per_q + (size_t)(h0 + hd) * AM_HD + column(j), step1, x, y);
+            rotate(x, y, t, j, a, b);
+        }
+        float* row = qs + (hd * TP + t) * SA_QSTR + column(j);
+        *reinterpret_cast<f32x4*>(row) = a * scale;
+        *reinterpret_cast<f32x4*>(row + step1) = b * scale;
+    }
+    __syncthreads();
+
+    // ---- attention: wave = head, 16 dimensions; 16 queries at a time (lane (i, g): query i) ----
+    const int hd = wave >> 3, sl = slots == 2 ? hd : 0, i = lane & 15, g = lane >> 4;
+    f32x4 out[TP / 16];
+#pragma unroll
+    for (int qb = 0; qb < TP / 16; ++qb) {
+        f32x4 s[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float* qp = qs + (hd * TP + 16 * qb + i) * SA_QSTR + 32 * c + 8 * g;
+            const f32x4 a = *reinterpret_cast<const f32x4*>(qp), b = *reinterpret_cast<const f32x4*>(qp + 4);
+            const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+            f16x8 qh, ql;
+            am_split8(x, qh, ql);
+#pragma unroll
+            for (int mt = 0; mt <= qb; ++mt) {
+                const f16x8 ka = *reinterpret_cast<const f16x8*>(kt + (sl * TP + 16 * mt + i) * SA_KSTR + 32 * c + 8 * g);
+                s[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh, s[mt], 0, 0, 0);
+                s[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql, s[mt], 0, 0, 0);
+            }
+        }
+        const int qi = 16 * qb + i;
+        float m = -INFINITY;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s[mt][e] = mt <= qb && 16 * mt + 4 * g + e <= qi ? s[mt][e] : -INFINITY;
+                m = fmaxf(m, s[mt][e]);
+            }
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        const float m_use = m == -INFINITY ? 0.0f : m;   // (scores that are all -inf, or not numbers)
+        float pv[8], l = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            pv[e] = __expf(s[0][e] - m_use);
+            pv[4 + e] = __expf(s[1][e] - m_use);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) l += pv[e];
+        f16x8 ph, pl;
+        am_split8(pv, ph, pl);
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const uint16_t* vrow = vt + (sl * AM_HD + 16 * (wave & 7) + i) * SA_VSTR + 4 * g;
+        const u32x2 v0 = *reinterpret_cast<const u32x2*>(vrow), v1 = *reinterpret_cast<const u32x2*>(vrow + 16);
+        const f16x8 va = __builtin_bit_cast(f16x8, u32x4{v0.x, v0.y, v1.x, v1.y});
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, acc, 0, 0, 0);
+        out[qb] = acc * inv;
+    }
+    __syncthreads();   // (every wave has read its queries: the result takes their place)
+#pragma unroll
+    for (int qb = 0; qb < TP / 16; ++qb) *reinterpret_cast<f32x4*>(qs + (hd * TP + 16 * qb + i) * SA_QSTR + 16 * (wave & 7) + 4 * g) = out[qb];
+    __syncthreads();
+    // ---- half a wave a token: the group's 256 columns ----
+    for (int t0 = 2 * wave; t0 < T; t0 += 32) {   // (uniform)
+        const int t = t0 + (lane >> 5), l = lane & 31, step = l >> 2, gg = l & 3;
+        const float* row = qs + ((step >> 2) * TP + min(t, TP - 1)) * SA_QSTR + 32 * (step & 3) + 4 * gg;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(row), b = *reinterpret_cast<const f32x4*>(row + 16);
+        float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        short_split(x, 8 * (int)blockIdx.x + step, gg, t < T ? t : -1, per_q, ws);
+    }
 }
 
 // =================================================================================================================================
@@ -546,3 +741,37 @@ int launch_attention_decode_kvhead_mfma(float* part, const float* q, const float
 }
 
 }  // namespace ntk
+
+extern "C" size_t ntk_short_angles_bytes(int head_dim) { return head_dim > 0 ? (size_t)2 * ntk::GB_SHORT * (size_t)(head_dim / 2) * sizeof(float) : 0; }
+extern "C" int ntk_short_angles(float* table, int head_dim, float theta_base, float freq_scale, void* stream) {
+    if (!table) return NTK_E_NULL;
+    if (head_dim <= 0 || head_dim % 2 != 0) return NTK_E_SHAPE;
+    hipLaunchKernelGGL(ntk::short_angles_kernel, dim3((ntk::GB_SHORT * (head_dim / 2) + 255) / 256), dim3(256), 0, ntk::resolve_stream(stream), table, head_dim / 2, theta_base, freq_scale);
+    return ntk::last_launch_status();
+}
+extern "C" int ntk_short_attention(const float* const* sums, const int* splits, const float* angles, int n_tokens, int n_heads, int n_kv_heads, int head_dim, float scale,
+                                   int interleaved, void* k_cache, void* v_cache, int max_seq, void* workspace, void* stream) {
+    using namespace ntk;
+    if (!sums || !splits || !sums[0] || !sums[1] || !sums[2] || !angles || !k_cache || !v_cache || !workspace) return NTK_E_NULL;
+    if (head_dim != AM_HD || n_tokens < 1 || n_tokens > GB_SHORT || n_tokens > max_seq || n_heads <= 0 || n_kv_heads <= 0 || n_heads % n_kv_heads != 0 || n_heads % 2 != 0) return NTK_E_SHAPE;
+    uintptr_t bits = reinterpret_cast<uintptr_t>(angles) | reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(workspace);
+    for (int i = 0; i < 3; ++i) {
+        if (splits[i] < 1) return NTK_E_SHAPE;
+        bits |= reinterpret_cast<uintptr_t>(sums[i]);
+    }
+    if (bits & 15) return NTK_E_ALIGN;
+    const size_t nq = (size_t)n_tokens * n_heads * head_dim, nk = (size_t)n_tokens * n_kv_heads * head_dim;
+    const ShortSource sq{sums[0], splits[0], nq}, sk{sums[1], splits[1], nk}, sv{sums[2], splits[2], nk};
+    const int slots = (n_heads / n_kv_heads) % 2 == 0 ? 1 : 2;   // (an odd group: some pairs of heads read two KV heads)
+    static const bool lds_ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&short_attention_kernel<16>), hipFuncAttributeMaxDynamicSharedMemorySize, sa_lds<16>(2)) == hipSuccess &&
+                               hipFuncSetAttribute(reinterpret_cast<const void*>(&short_attention_kernel<32>), hipFuncAttributeMaxDynamicSharedMemorySize, sa_lds<32>(2)) == hipSuccess;
+    if (!lds_ok) return NTK_E_LAUNCH;
+    hipStream_t st = resolve_stream(stream);
+    uint16_t *kc = static_cast<uint16_t*>(k_cache), *vc = static_cast<uint16_t*>(v_cache);
+    uint8_t* ws = static_cast<uint8_t*>(workspace);
+    if (n_tokens <= 16)
+        hipLaunchKernelGGL(short_attention_kernel<16>, dim3(n_heads / 2), dim3(1024), sa_lds<16>(slots), st, sq, sk, sv, angles, interleaved, n_tokens, n_heads, n_kv_heads, scale, kc, vc, ws);
+    else
+        hipLaunchKernelGGL(short_attention_kernel<32>, dim3(n_heads / 2), dim3(1024), sa_lds<32>(slots), st, sq, sk, sv, angles, interleaved, n_tokens, n_heads, n_kv_heads, scale, kc, vc, ws);
+    return last_launch_status();
+}

@@ -533,6 +533,7 @@ int Model::alloc_buffers() {   // transformer.cpp:330-391
     d_token_ = (int*)dev(64, true);
     argmax_scratch_ = (float*)dev(2 * 1024 * 4, false);
     rope_inv_freq_ = (float*)dev((size_t)cfg_.head_dim / 2 * 4 + 64, false);
+    rope_angles_ = (float*)dev(ntk_short_angles_bytes(cfg_.head_dim) + 64, false);
     row_max_ = (float*)dev((size_t)S * 2 * 4, true);
     attn_scratch_ = (float*)dev(ntk_attention_split_scratch_bytes(cfg_.n_heads, cfg_.head_dim, kMaxAttnSplits), true);   // (zeroed: the arrival counters in front)
     h_token_ = (int*)nt_hip_malloc_host(64);
@@ -564,10 +565,11 @@ int Model::alloc_buffers() {   // transformer.cpp:330-391
         return NTK_E_NOMEM;
     }
     *h_token_ = 0;
-    if (rope_inv_freq_) {
+    if (rope_inv_freq_ && rope_angles_) {
         std::vector<float> f((size_t)cfg_.head_dim / 2);
         for (int i = 0; i < cfg_.head_dim / 2; ++i) f[i] = 1.0f / powf(cfg_.rope_theta, (2.0f * i) / cfg_.head_dim);
         nt_hip_memcpy_h2d(rope_inv_freq_, f.data(), f.size() * 4);
+        if (ntk_short_angles(rope_angles_, cfg_.head_dim, cfg_.rope_theta, cfg_.rope_freq_scale, stream_) != NTK_OK || ntk_stream_synchronize(stream_) != NTK_OK) return NTK_E_LAUNCH;
     }
     return NTK_OK;
 }
@@ -701,6 +703,9 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
         int splits[3] = {1, 1, 1};
         bool done[3] = {false, false, false};
         size_t at = 0;
+        // from the prompt's first token on: everything between the projections in one launch
+        const bool whole = start_pos == 0 && hd == 128 && nh % 2 == 0 && rope_angles_ != nullptr;
+        const bool defer = whole || T >= 4;   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
         for (int a = 0; a < 3; ++a) {
             if (done[a]) continue;
             const DevTensor* w[3];
@@ -709,25 +714,29 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
             for (int b = a; b < 3; ++b)
                 if (qkv[b]->dtype == qkv[a]->dtype) { w[n] = qkv[b]; y[n] = ys[b]; idx[n++] = b; done[b] = true; }
             ntk_gemm_partials pt;
-            NT_TRY(gemm(w, y, n, nullptr, true, at, T >= 4 ? &pt : nullptr));
-            if (T >= 4 && pt.nsplit > 1)
+            NT_TRY(gemm(w, y, n, nullptr, true, at, defer ? &pt : nullptr));
+            if (defer && pt.nsplit > 1)
                 for (int k = 0; k < n; ++k) {
                     sums[idx[k]] = pt.part[k];
                     splits[idx[k]] = pt.nsplit;
                     at += (size_t)pt.nsplit * T * w[k]->out_f;
                 }
         }
-        if (T >= 4) {   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
+        if (whole) {
+            NT_TRY(ntk_short_attention(sums, splits, rope_angles_, T, nh, nkv, hd, scale, cfg_.rope_interleaved, kc, vc, cfg_.max_seq_len, other(), s));
+        } else if (T >= 4) {
             NT_TRY(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
         } else {
             NT_TRY(ntk_rope(q_buf, k_buf, positions_, 1, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, s));
             NT_TRY(ntk_copy_to_kv_cache(kc, vc, k_buf, v_buf, T, nkv, hd, start_pos, cfg_.max_seq_len, s));
         }
-        NT_TRY(ntk_attention_prefill(attn_out, q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
+        if (!whole) {
+            NT_TRY(ntk_attention_prefill(attn_out, q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
+            NT_TRY(ntk_short_prepare_x(attn_out, T, qd, other(), s));
+        }
         ntk_gemm_partials pt;
         const DevTensor* w[2] = {&L.wo, nullptr};
         float* y[2] = {hidden_, nullptr};
-        NT_TRY(ntk_short_prepare_x(attn_out, T, qd, other(), s));
         NT_TRY(gemm(w, y, 1, hidden_, false, 0, &pt));
         NT_TRY(ntk_short_norm_prepare_x(hidden_, &pt, (const float*)L.ffn_norm.ptr, T, H, other(), s));
         w[0] = &L.w_gate; w[1] = &L.w_up;

@@ -220,6 +220,7 @@ private:
     int* h_recent_ = nullptr;       // pinned staging of it
     static constexpr int kRecentCap = 4096;
     float* rope_inv_freq_ = nullptr; // [hd/2] 1/powf(theta, 2i/hd), computed once on the host (rotary.cu:47)
+    float* rope_angles_ = nullptr;     // ntk_short_angles of the first 32 positions
     void* stream_ = nullptr;
     bool batched_prefill_ = true;
     struct Timed { int cls; void* a; void* b; int n; bool shared_a; };   // n launches between events a and b

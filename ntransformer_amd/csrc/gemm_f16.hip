@@ -34,35 +34,21 @@
 //     the two 16-column sub-scale groups of Q6_K (which uses two K = 16 MFMAs per step).
 // Bound: instruction issue (MFMA + VALU of two waves per SIMD) under a 1.65-1.7 GHz clock; matrix pipe 41 % busy.
 #include "common.hip.h"
+#include "gemm_planes.hip.h"
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
 namespace ntk {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-constexpr int GB_TOK = 64;           // tokens per pass
 // K splits x 64-token chunks of one launch never exceed this (size of the partial-sum area): 32 for matrices of up to 8192 rows (the narrow
 // ones are the ones that need splits at many chunks), 16 above
 constexpr int gb_split_rows(int out_total) { return out_total <= 8192 ? 32 : 16; }
-constexpr int GB_MAX_CHUNKS = 16;   // 64-token chunks per launch (32 measured no better: 15.1k vs 16.0k tok/s at 2048 tokens)
-constexpr int GB_PIECE = 1024;       // bytes of one (step, plane, token block) operand record
-constexpr int GB_PLANES = 2;         // FP16 pieces of an activation
-constexpr int GB_STEP_BYTES = GB_PLANES * 4 * GB_PIECE;   // 8 KB of activation operands per step
 #ifdef NTK_GEMM_OCC3   // tuning build: three workgroups (12 waves) per CU -- 168 VGPRs, 53 KB of LDS each (Q8_0 without the plane prefetch fits)
 constexpr int GB_WG_PER_CU = 3, GB_LDS_WG = 53 * 1024, GB_NRING_Q8 = 1;
 #else
 constexpr int GB_WG_PER_CU = 2, GB_LDS_WG = 80 * 1024, GB_NRING_Q8 = 2;
 #endif
-constexpr int GB_AUX_BYTES = GB_TOK * 4;                  // per step: one eighth of its unit's record of sums (K-quant minimum term)
-constexpr int GB_SHORT = 32;         // tokens of a short prompt (gemm_quant_f16_kslice_kernel), whose planes are scaled per GB_GROUP columns
-constexpr int GB_GROUP = 256;
-constexpr int GB_MIN_UNIT_BYTES = 8 * GB_AUX_BYTES;       // per unit of 8 steps and 64-token chunk: 2 pieces x 4 token blocks x 2 x 16 tokens x 4 steps x FP16
 
 // bytes k, k + 1 of a dword -> an FP16 pair, one SDWA conversion each (through F32 it is two conversions and a pack per pair: the
 // VALU slots of a step are what the kernel runs out of first); `s_nop 1`: see cvt8_s8_f16 below (these feed the minimum term's matrix instruction)
@@ -123,11 +109,6 @@ typedef uint16_t __attribute__((aligned(2))) u16_a2;
 // s = 2^(14 - floor(log2 m)), m = the token's largest |x|: m s in [2^14, 2^15) -- FP16's largest binade but one.  Exponent fields are
 // kept inside [1, 253] so that both s and 1 / s are normal numbers (an all-zero or subnormal token multiplies to zero either way; a
 // token holding Inf / NaN propagates it through the first piece).  grid = ceil(T / 4), block = 256: one wave per token.
-// exponent field of s from the token's largest |x| (bit pattern; a NaN pattern counts as the largest binade: any scale will do then)
-__device__ __forceinline__ int scale_exp_of_max(uint32_t max_bits) {
-    const int em = (int)((max_bits >> 23) & 0xFFu);
-    return min(253, max(1, 268 - em));
-}
 __global__ __launch_bounds__(256) void row_scale_kernel(const float* __restrict__ X, int T, int in, float* __restrict__ scale, float* __restrict__ inv) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (t >= T) return;
@@ -265,16 +246,7 @@ __global__ __launch_bounds__(256) void silu_mul_rowmax_kernel(float* __restrict_
 // fourteen launches of a layer, a quarter of a short prompt's time.  The kernels below own a whole TOKEN per workgroup, so the workgroup that has written a
 // token's row knows its largest |x| and can split the row itself: planes, step sums and 1 / s go straight into the GEMM workspace and the projection runs
 // with reuse_x = 1.  split_row is split_x_kernel's arithmetic element for element (same scale, same two roundings, the step sums in the same order): the
-// workspace holds the same bits.  Layout of the workspace: [chunk][(in / 32 + 1) step records of 8 KB | sums of the units], then [1 / s][s] of the pass.
-static __host__ __device__ size_t ws_chunk_bytes(int in) {
-    return ((size_t)(in / 32 + 1) * GB_STEP_BYTES + (size_t)((in / 32 + 15) / 8) * GB_MIN_UNIT_BYTES + 255) / 256 * 256;
-}
-constexpr size_t GB_SCALE_BYTES = 2 * GB_MAX_CHUNKS * GB_TOK * sizeof(float);   // the launch's 1 / s and s
-// ... and behind those, for the short prompts' form: [GB_GROUP columns][GB_SHORT tokens] 1 / s, then [512 columns][GB_SHORT tokens] sums of squares (short_split below)
-static __host__ __device__ size_t ws_group_floats(int in) { return (size_t)((in + GB_GROUP - 1) / GB_GROUP) * GB_SHORT; }
-static __host__ __device__ size_t ws_group_bytes(int in) { return (ws_group_floats(in) + (size_t)((in + 511) / 512) * GB_SHORT) * sizeof(float); }
-static __host__ __device__ size_t ws_group_offset(int in) { return (size_t)GB_MAX_CHUNKS * ws_chunk_bytes(in) + GB_SCALE_BYTES; }
-static __host__ __device__ size_t ws_part_offset(int in) { return ws_group_offset(in) + (ws_group_bytes(in) + 255) / 256 * 256; }
+// workspace holds the same bits.
 // row: the token's `in` floats (global memory; written by THIS workgroup before a __syncthreads()), or null for a padding token (zeros: the records the
 // matrix instructions read beside the prompt's last tokens).  Every thread of the workgroup calls it.
 __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, int t, int in, uint8_t* __restrict__ ws) {
@@ -335,47 +307,6 @@ __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, i
 // magnitudes across its lanes and writes their planes, step sums and 1 / s; the GEMM folds a group's products with that 1 / s (a power of two: exact).  The planes are nearer the values
 // than a row's scale leaves them: what a group's own largest value puts into FP16's subnormals is less.  An RMSNorm's 1 / rms belongs to the row: the wave leaves its sum of squares and
 // the GEMM multiplies its sums by 1 / rms.
-// x[8]: lane's values of columns col + {0..3, 16..19}, col = 512 wave + 32 (lane / 4) + 4 (lane % 4); lanes past the row hold zeros.
-__device__ __forceinline__ void short_split(float (&x)[8], int lane, int col512, int t, int in, uint8_t* __restrict__ ws) {
-    const int step = (col512 >> 5) + (lane >> 2), g = lane & 3;
-    uint32_t mb = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) mb = max(mb, __float_as_uint(x[e]) & 0x7FFFFFFFu);   // (bit patterns: ordered like the values, and a NaN is not dropped)
-#pragma unroll
-    for (int o = 1; o <= 16; o <<= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
-    const int es = scale_exp_of_max(mb);
-    const float sc = __uint_as_float((uint32_t)es << 23);
-    float p1[8], p2[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        x[e] *= sc;
-        const _Float16 h1 = (_Float16)x[e];
-        p1[e] = (float)h1;
-        p2[e] = x[e] - p1[e];
-    }
-    auto pk = [](float lo, float hi) {
-        const f16x2 h = {(_Float16)lo, (_Float16)hi};
-        return __builtin_bit_cast(uint32_t, h);
-    };
-    float sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    if (step * 32 >= in) return;
-    const int tb = t >> 4, j = t & 15;
-    u32x4* xb = reinterpret_cast<u32x4*>(ws);
-    const size_t base = ((size_t)step * GB_PLANES * 4 + tb) * 64 + (j + 16 * g);
-    xb[base] = u32x4{pk(p1[0], p1[1]), pk(p1[2], p1[3]), pk(p1[4], p1[5]), pk(p1[6], p1[7])};
-    xb[base + 256] = u32x4{pk(p2[0], p2[1]), pk(p2[2], p2[3]), pk(p2[4], p2[5]), pk(p2[6], p2[7])};
-    if (g == 0) {
-        const float y = sum * 0.015625f;
-        const _Float16 h1 = (_Float16)y, h2 = (_Float16)(y - (float)h1);
-        _Float16* rec = reinterpret_cast<_Float16*>(ws + (size_t)(in / 32 + 1) * GB_STEP_BYTES + (size_t)(step >> 3) * GB_MIN_UNIT_BYTES);
-        const int pos = ((tb * 2 + ((step >> 2) & 1)) * 64 + j * 4 + (step & 3));
-        rec[pos] = h1;
-        rec[4 * 128 + pos] = h2;
-        if ((lane & 31) == 0) reinterpret_cast<float*>(ws + ws_group_offset(in))[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((uint32_t)(254 - es) << 23);
-    }
-}
 // sums of a deferred projection's K splits (in split order), the lane's eight columns at row[0 .. 3], row[16 .. 19]; eight splits' requests under way
 __device__ __forceinline__ void short_sums(const float* __restrict__ row, size_t plane, int nsplit, float (&v)[8]) {
     auto put = [](float (&d)[8], const float4& a, const float4& b) { d[0] = a.x; d[1] = a.y; d[2] = a.z; d[3] = a.w; d[4] = b.x; d[5] = b.y; d[6] = b.z; d[7] = b.w; };
@@ -400,7 +331,7 @@ __global__ __launch_bounds__(64) void short_split_kernel(const float* __restrict
     const int lane = threadIdx.x, t = (int)blockIdx.y, col = (int)blockIdx.x * 512 + 32 * (lane >> 2) + 4 * (lane & 3);
     float x[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (col < in) short_sums(X + (size_t)t * in + col, 0, 1, x);
-    short_split(x, lane, (int)blockIdx.x * 512, t, in, ws);
+    short_split(x, (int)blockIdx.x * 16 + (lane >> 2), lane & 3, t, in, ws);
 }
 // hidden += the sums of part's splits (nsplit 0: hidden as it lies); planes of hidden * weight, the row's sum of squares by parts of 512 columns
 __global__ __launch_bounds__(64) void short_norm_kernel(float* __restrict__ hidden, const float* __restrict__ part, int nsplit, size_t plane, const float* __restrict__ weight, int H,
@@ -432,7 +363,7 @@ __global__ __launch_bounds__(64) void short_norm_kernel(float* __restrict__ hidd
 #pragma unroll
     for (int o = 1; o <= 32; o <<= 1) ssq += __shfl_xor(ssq, o, 64);
     if (lane == 0) (reinterpret_cast<float*>(ws + ws_group_offset(H)) + ws_group_floats(H))[(int)blockIdx.x * GB_SHORT + t] = ssq;
-    short_split(x, lane, (int)blockIdx.x * 512, t, H, ws);
+    short_split(x, (int)blockIdx.x * 16 + (lane >> 2), lane & 3, t, H, ws);
 }
 // planes of silu(gate) * up, both the sums of their splits
 __global__ __launch_bounds__(64) void short_silu_mul_kernel(const float* __restrict__ pg, const float* __restrict__ pu, int nsplit, size_t plane, int I, uint8_t* __restrict__ ws) {
@@ -445,7 +376,7 @@ __global__ __launch_bounds__(64) void short_silu_mul_kernel(const float* __restr
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = x[e] / (1.0f + expf(-x[e])) * u[e];
     }
-    short_split(x, lane, (int)blockIdx.x * 512, t, I, ws);
+    short_split(x, (int)blockIdx.x * 16 + (lane >> 2), lane & 3, t, I, ws);
 }
 // tokens of the launch rounded up to the token blocks the matrix instructions read (16 per block; the 64-token form reads whole chunks)
 static inline int split_pad_tokens(int T) { return T <= 32 ? (T + 15) / 16 * 16 : (T + GB_TOK - 1) / GB_TOK * GB_TOK; }

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from ntransformer_amd import _lib
+from ntransformer_amd import gguf
 from ntransformer_amd import gguf as G
 from ntransformer_amd.ops import DeviceBuffer as DB
 from oracle import arbiter
@@ -155,3 +156,42 @@ def test_sums_side_by_side_and_what_is_refused():
     assert not L.ntk_gemm_short_takes(one, 1, 33, inf, dt) and not L.ntk_gemm_short_takes(one, 1, 16, inf + 32, dt)
     assert not L.ntk_gemm_short_takes((C.c_int * 1)(24), 1, 16, inf, dt) and not L.ntk_gemm_short_takes(one, 1, 16, inf, 0)
     assert L.ntk_short_prepare_x(ws.ptr, 33, inf, ws.ptr, None) != 0 and L.ntk_short_prepare_x(ws.ptr, 4, 40, ws.ptr, None) != 0
+
+
+@pytest.mark.parametrize("T,H,G,splits,interleaved", [(1, 2, 1, (1, 1, 1), 0), (3, 6, 2, (4, 4, 17), 0), (16, 32, 8, (4, 4, 16), 0), (17, 4, 4, (2, 9, 10), 1), (32, 8, 1, (3, 1, 2), 0), (29, 64, 8, (8, 8, 8), 1)])
+def test_attention_and_planes_in_one_launch(T, H, G, splits, interleaved):
+    """against the three launches it replaces: the caches and the products of its planes bit for bit"""
+    L, hd, rows = lib(), 128, 64
+    g = np.random.default_rng(T + H)
+    out = (H * hd, G * hd, G * hd)
+    parts = [g.standard_normal((n, T, r)).astype(np.float32) for n, r in zip(splits, out)]
+    parts[2][:, T // 2] *= np.float32(1e3)
+    raw = np.frombuffer(gguf.synth_tensor(g, gguf.GGML_Q4_K, rows, H * hd), np.uint8)
+    dt = gguf.GGML_TO_DT[gguf.GGML_Q4_K]
+    L.ntk_short_angles.argtypes = [VP, C.c_int, C.c_float, C.c_float, VP]
+    angles = DB.zeros(2 * 32 * hd // 2 * 4)
+    _lib.check(L.ntk_short_angles(angles.ptr, hd, 500000.0, 1.0, None), "short_angles")
+    nbytes = L.ntk_gemm_quant_workspace_bytes(H * hd, rows)
+    L.ntk_reduce_rope_kv_store.argtypes = [VP, C.POINTER(VP), C.POINTER(C.c_int), VP] + [C.c_int] * 4 + [C.c_float, C.c_float, C.c_int, VP, VP, C.c_int, C.c_int, VP]
+    L.ntk_attention_prefill.argtypes = [VP] * 4 + [C.c_int] * 6 + [C.c_float, VP]
+    L.ntk_short_attention.argtypes = [C.POINTER(VP), C.POINTER(C.c_int), VP] + [C.c_int] * 4 + [C.c_float, C.c_int, VP, VP, C.c_int, VP, VP]
+    scale, res = 1.0 / np.sqrt(np.float32(hd)), []
+    for fused in (0, 1):
+        kc, vc = (DB.from_numpy(np.full((T + 2, out[1]), 3.0, np.float16)) for _ in range(2))
+        bufs = [DB.from_numpy(p) for p in parts]
+        arr, ns, ws = (VP * 3)(*[b.ptr for b in bufs]), (C.c_int * 3)(*splits), DB(nbytes)
+        if fused:
+            _lib.check(L.ntk_short_attention(arr, ns, angles.ptr, T, H, G, hd, scale, interleaved, kc.ptr, vc.ptr, T + 2, ws.ptr, None), "short_attention")
+        else:
+            q, o, pos = DB.zeros(T * out[0] * 4), DB.zeros(T * out[0] * 4), DB.from_numpy(np.arange(T, dtype=np.int32))
+            _lib.check(L.ntk_reduce_rope_kv_store(q.ptr, arr, ns, pos.ptr, T, H, G, hd, 500000.0, 1.0, interleaved, kc.ptr, vc.ptr, 0, T + 2, None), "rope")
+            _lib.check(L.ntk_attention_prefill(o.ptr, q.ptr, kc.ptr, vc.ptr, T, 0, H, G, hd, T + 2, scale, None), "attention")
+            _lib.check(L.ntk_short_prepare_x(o.ptr, T, H * hd, ws.ptr, None), "prepare")
+        y = DB.zeros(T * rows * 4)
+        product(L, ws, nbytes, [DB.from_numpy(raw)], [y], rows, dt, T, H * hd)
+        res.append((kc.numpy(np.uint16), vc.numpy(np.uint16), y.numpy(np.float32)))
+    assert np.isfinite(res[0][2]).all()
+    for a, b in zip(*res):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+    assert L.ntk_short_attention(arr, ns, angles.ptr, 33, H, G, hd, scale, 0, kc.ptr, vc.ptr, 64, ws.ptr, None) != 0
+    assert L.ntk_short_attention(arr, ns, angles.ptr, T, H + 1, 1, hd, scale, 0, kc.ptr, vc.ptr, T + 2, ws.ptr, None) != 0
