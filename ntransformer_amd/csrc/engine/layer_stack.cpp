@@ -1145,8 +1145,8 @@ int LayerStackModel::run_window(const StackLayer& L, const float* h, float* cach
     return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
-// what lies between the window mixer's two products: norms, rotation and cache rows, then the attention with its gate -> out [T][heads * vdim]
-int LayerStackModel::window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0) {
+// norms, rotation and cache rows of the window mixer's first product
+int LayerStackModel::window_keys_values(const WindowMixer& m, float* cache, int T, int pos0) {
     const int na = (int)m.in.out_f;
     ntk_rotary rot{m.rot_freq, m.rot_mag, m.rot_dims, form_.rot_halves ? NTK_ROT_HALVES : NTK_ROT_NEIGHBOURS};
     ntk_window_prepare_desc pd{};
@@ -1159,7 +1159,13 @@ int LayerStackModel::window_heads(const WindowMixer& m, float* cache, float* out
     }
     if (m.v_mix && m.v_source) { pd.v_keep = vfirst_; pd.ld_keep = m.kv_heads * m.vdim; }                 // the first blending layer keeps its values of this pass's tokens
     else if (m.v_mix) { pd.v_other = vfirst_; pd.ld_other = m.kv_heads * m.vdim; pd.v_blend = m.v_blend; }    // the later ones blend with them
-    LS_TRY(ntk_window_prepare_ex(&pd, stream_));
+    return ntk_window_prepare_ex(&pd, stream_);
+}
+
+// what lies between the window mixer's two products: the above, then the attention with its gate -> out [T][heads * vdim]
+int LayerStackModel::window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0) {
+    const int na = (int)m.in.out_f;
+    LS_TRY(window_keys_values(m, cache, T, pos0));
     ntk_window_attention_desc d{};
     d.out = out; d.ldo = ldo; d.q = a_; d.ldq = na; d.cache = cache; d.row = m.row(); d.H = m.heads; d.G = m.kv_heads; d.maps = m.maps; d.dn = m.dim; d.dv = m.vdim;
     d.pos0 = pos0; d.T = T; d.window = m.window; d.scale = m.scale; d.lambda = m.lambda;
@@ -1348,6 +1354,15 @@ int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, con
 // weight and the silu gate, output projection -> mix_.  state = [S | the convolutions' last inputs]
 int LayerStackModel::run_gated_delta(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16) {
     const GatedDeltaMixer& m = L.gdl;
+    const int W = info_.width, hv = m.heads * m.vdim;
+    LS_TRY(gated_delta_state(L, h, state, T, pos0, norm_inside, h16));
+    LS_TRY(ntk_head_rmsnorm_gate(att_, hv, att_, hv, m.norm, 0, a_ + m.g_off, (int)m.in.out_f, 2, 1.0f, T, m.heads, m.vdim, eps_, stream_));
+    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
+}
+
+// ... up to the recurrence's results in att_, the state carried on
+int LayerStackModel::gated_delta_state(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16) {
+    const GatedDeltaMixer& m = L.gdl;
     const int W = info_.width, na = (int)m.in.out_f, nc = m.channels(), hv = m.heads * m.vdim;
     ntk_dense_desc in{};
     in.Y = a_; in.ldy = na; in.X = h; in.ldx = W; in.W = m.in.ptr; in.wdtype = m.in.dtype; in.G = 1; in.row_div = 1; in.T = T; in.N = na; in.K = W;
@@ -1366,9 +1381,7 @@ int LayerStackModel::run_gated_delta(const StackLayer& L, const float* h, float*
     d.az = a_ + m.b_off; d.lda = na; d.unit_eps = kUnitKeyEps;
     d.G = m.kv_heads; d.unit_q = 1; d.unit_k = 1; d.head_gates = 1; d.write_gated = 1;
     d.state = state; d.H = m.heads; d.dn = m.dim; d.dv = m.vdim; d.q_scale = 1.0f / std::sqrt((float)m.dim); d.pos0 = pos0; d.T = T; d.scratch = rscratch_;
-    LS_TRY(ntk_gated_recurrence(&d, stream_));
-    LS_TRY(ntk_head_rmsnorm_gate(att_, hv, att_, hv, m.norm, 0, a_ + m.g_off, na, 2, 1.0f, T, m.heads, m.vdim, eps_, stream_));
-    return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
+    return ntk_gated_recurrence(&d, stream_);
 }
 
 // the seam in front of a sublayer of the scaled form: what the stream is still owed joins it (RMS norm, weight, the residual factor), then the norm of the row
@@ -1624,7 +1637,42 @@ int LayerStackModel::parallel_layer(const Run& run, const StackLayer& L, int slo
     return ntk_residual_add(x_, mix_, nullptr, T * W, stream_);
 }
 
-int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, float* logits_out) {
+// What a portion's tokens leave behind in the LAST layer run when none of their results is wanted: their keys and values (or latents), or the recurrence's state.  Nothing reads their
+// results: no later layer, no cache, no logits.
+int LayerStackModel::last_layer_keys(const Run& run, const StackLayer& L, int slot, int T, int pos0) {
+    const int W = info_.width;
+    DenseW in = L.mixer == kMixWindow ? L.att.in : L.mixer == kMixLatent ? L.mix.in : L.gdl.in;
+    int at = 0;
+    if (L.mixer == kMixLatent) {           // its rows for [latent | key part] alone
+        if (L.mix.kv_from >= 0) return NTK_OK;
+        at = L.mix.kv_off;
+        in.ptr = (char*)in.ptr + (size_t)at * W * (in.dtype == NTK_DT_BF16 ? 2 : 4);
+        in.out_f = L.mix.row();
+    }
+    const void* h16 = nullptr;
+    if (form_.scaled) LS_TRY(seam_for(in, L.norm1, h1_, h1_16_, T, &h16));
+    else {
+        int st = NTK_E_ALIGN;
+        if (rounded(in, T)) {
+            st = ntk_rmsnorm_offset_16(nullptr, h1_16_, L.norm1.w, nullptr, nullptr, nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
+            if (st == NTK_OK) h16 = h1_16_;
+        }
+        if (st == NTK_E_ALIGN) st = ntk_rmsnorm_offset(h1_, L.norm1.w, nullptr, nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
+        LS_TRY(st);
+    }
+    if (L.mixer == kMixGatedDelta) return gated_delta_state(L, h1_, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0, false, h16);
+    const int na = L.mixer == kMixWindow ? (int)L.att.in.out_f : (int)L.mix.in.out_f;
+    ntk_dense_desc d{};
+    d.Y = a_ + at; d.ldy = na; d.X = h1_; d.ldx = W; d.W = in.ptr; d.wdtype = in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = (int)in.out_f; d.K = W;
+    LS_TRY(first_product(d, h16));
+    if (L.mixer == kMixWindow) return window_keys_values(L.att, run.cache + (size_t)slot * opt_.max_context * L.att.row(), T, pos0);
+    const LatentMixer& m = L.mix;
+    ntk_rotary rot{m.rot_freq, m.rot_mag, m.rot_dims, m.rot_layout};
+    return ntk_latent_prepare(run.cache + (size_t)slot * opt_.max_context * m.row(), m.row(), a_ + m.kv_off, na, m.kv_norm, eps_, m.kv_rank, m.rot_dim, nullptr, 0, 0, 0, &rot, pos0, T, stream_);
+}
+
+// want_last: the portion's last token is wanted and no other
+int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out) {
     const int W = info_.width;
     // (the embedding is kept beside the stream only where a repeated span is entered through a projection of both)
     const bool keep_embedding = has_loop_ && form_.loop_projection;
@@ -1642,6 +1690,11 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, in
     LS_TRY(ntk_embed_dense_scaled(keep_embedding ? x0_ : x_, embed_.ptr, embed_.dtype, tokens_dev, T, info_.vocab, W, embed_scale_, stream_));
     bool x_is_x0 = keep_embedding;   // until the first layer run writes x_
     owed_.y = nullptr;
+    // The last layer's results are read where they are wanted and nowhere else: of the other tokens it needs what later tokens attend to (last_layer_keys), and a last token alone takes the
+    // layer as a decoded token does.  A layer's worth of a prompt's time less: 1 / 2 of it with two layers, 1 / 32 with 32.  (ten tokens on: fewer go through the one-token products anyway)
+    const bool tail = (form_.scaled || !(form_.gated || form_.sequential || form_.post_norm || form_.dense_parallel)) && T > ntk_dense_few_rows() + 1 && (n_want == 0 || want_last) && !(capture_ && capture_buf_);
+    struct Streams { float *&x, *&x0, *&v, *const kx, *const kx0, *const kv; ~Streams() { x = kx; x0 = kx0; v = kv; } };
+    Streams whole{x_, x0_, vfirst_, x_, x0_, vfirst_};
     for (size_t r = 0; r < runs_.size(); ++r) {
         const Run& run = runs_[r];
         const StackLayer& L = layers_[(size_t)run.layer];
@@ -1650,6 +1703,18 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, in
             LS_TRY(ntk_concat_rows(cat_, x_is_x0 ? x0_ : x_, x0_, T, W, stream_));
             LS_TRY(linear(x_, W, cat_, 2 * W, loop_in_.ptr, loop_in_.dtype, T, W, 2 * W, 0));
             x_is_x0 = false;
+        }
+        if (tail && r + 1 == runs_.size()) {
+            const Owed owed = owed_;
+            LS_TRY(last_layer_keys(run, L, slot, want_last ? T - 1 : T, pos0));
+            if (!want_last) return NTK_OK;
+            // the last token's row of the stream (what it is owed included) and of the first layer's values
+            owed_ = owed;
+            if (owed_.y) owed_.y += (size_t)(T - 1) * W;
+            x_ += (size_t)(T - 1) * W;
+            if (vfirst_ && L.mixer == kMixWindow) vfirst_ += (size_t)(T - 1) * L.att.kv_heads * L.att.vdim;
+            pos0 += T - 1;
+            T = 1;
         }
         if (form_.gated) {
             LS_TRY(gated_layer(r, L, slot, T, pos0));
@@ -1731,7 +1796,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         if (nw > 0) memcpy(h_stage_ + chunk_, rel.data(), (size_t)nw * sizeof(int));
         if (ntk_memcpy_h2d_async(tokens_dev_, h_stage_, (size_t)(nw > 0 ? chunk_ + nw : T) * sizeof(int), stream_) != NTK_OK) { err_ = "forward: the copy of the tokens failed"; return nullptr; }
         const int prev_token = at > 0 ? tokens[at - 1] : pos0 > 0 ? slots_.token(slot, pos0 - 1) : 0;
-        const int st = portion(slot, tokens_dev_, prev_token, T, pos0 + at, want_dev_, w1 - done_want, logits_ + (size_t)done_want * info_.vocab);
+        const int st = portion(slot, tokens_dev_, prev_token, T, pos0 + at, want_dev_, w1 - done_want, w1 - done_want == 1 && rel[0] == T - 1, logits_ + (size_t)done_want * info_.vocab);
         if (st != NTK_OK) { if (err_.empty()) err_ = std::string("forward: ") + ntk_status_string(st); return nullptr; }
         done_want = w1;
     }

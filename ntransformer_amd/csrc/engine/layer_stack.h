@@ -312,6 +312,7 @@ private:
     int run_gated_ff(const StackLayer& L, int T);
     int parse_gated_delta(const Json& L, GatedDeltaMixer& m);
     int run_gated_delta(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16);
+    int gated_delta_state(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16);
     int run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16 = nullptr, const float* norm_w = nullptr);
     int post_norm_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int rms_seam(const NormW& nw, float* out, int T);
@@ -328,10 +329,12 @@ private:
     int alloc_buffers();
     void* dev_alloc(size_t bytes);
     void* late_alloc(size_t bytes);
-    int portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, float* logits_out);
+    int portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out);
+    int last_layer_keys(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false, const void* h16 = nullptr);
     int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, bool norm_inside = false, const void* h16 = nullptr);
     int window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0);
+    int window_keys_values(const WindowMixer& m, float* cache, int T, int pos0);
     int dense_parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int run_lightning(const StackLayer& L, float* state, int T, int pos0);
     int run_moe(const StackLayer& L, const float* h, int T, bool into_stream, const void* h16 = nullptr);
