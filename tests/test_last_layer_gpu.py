@@ -70,3 +70,23 @@ def test_scaled_form(tmp_path, dtype, T, last):
 @pytest.mark.parametrize("kw", [dict(), dict(layers=("latent_attention_2",)), dict(layers=("latent_attention", "latent_attention_2"), loop=(0, 2, 2)), dict(mlp_on=(True, False))])
 def test_parallel_form(tmp_path, dtype, T, kw):
     check(FO, FO.small_config(**kw), tmp_path, dtype, T)
+
+
+@pytest.mark.parametrize("mix", ["Q8_0", "Q4_K_M", "F16"])
+@pytest.mark.parametrize("T", [32, 33, 70])
+def test_gguf_prompts(mix, T):
+    """against the per-token sequence, which runs every layer for every token: the prompt's logits, and those of tokens decoded behind it (which read the last layer's cache rows).  Caches of
+    halves: a value at a rounding boundary falls to either side, 1e-3 (2e-4 seen)"""
+    from ntransformer_amd import engine as E
+    spec = E.synth_spec("small", mix, seed=3, layers=2)
+    toks = [int(t) for t in np.random.default_rng(T).integers(0, 2048, T + 3)]
+    out = []
+    for batched in (1, 0):
+        e = E.Engine()
+        e.load_synthetic(spec, 128)
+        e.set_option("batched_prefill", batched)
+        lg = [e.forward(toks[:T], 0)]
+        lg += [e.decode_fused(t, T + i, False) for i, t in enumerate(toks[T:])]
+        e.close()
+        out.append(np.stack(lg))
+    assert np.isfinite(out[0]).all() and rel(out[0], out[1]) < 1e-3
