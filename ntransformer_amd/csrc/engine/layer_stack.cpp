@@ -65,6 +65,7 @@ LayerStackModel::~LayerStackModel() {
     if (capture_buf_) nt_hip_free(capture_buf_);
     if (image_) nt_hip_free(image_);
     if (h_stage_) nt_hip_free_host(h_stage_);
+    if (h_logits_) nt_hip_free_host(h_logits_);
 }
 
 void* LayerStackModel::dev_alloc(size_t bytes) {
@@ -1018,6 +1019,7 @@ int LayerStackModel::alloc_buffers() {
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
     h_stage_ = (int*)nt_hip_malloc_host(2 * C * sizeof(int));
     ok = ok && h_stage_ != nullptr;
+    h_logits_ = (float*)nt_hip_malloc_host((size_t)info_.vocab * sizeof(float));   // (none: a copy of the runtime's)
     if (max_top_ > 0) {
         const size_t P = C * max_top_;
         ok = ok && in(&ids_, P) && fl(&wts_, P) && fl(&sg_, C) && in(&offsets_, (size_t)max_e_ + 1) && in(&order_, P) && in(&where_, P) && fl(&gu_, P * max_ff2_) &&
@@ -1790,11 +1792,17 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         for (int i = done_want; i < w1; ++i) rel[(size_t)(i - done_want)] = want[i] - at;
         // the pinned staging area is free once the previous pass's copy has run: wait for the stream (idle already after a copy_logits), then one
         // stream-ordered copy brings the tokens and the wanted places
+        const int nw = w1 - done_want;
+        if (T + nw <= 32) {   // (a few of them as arguments of a launch: no staging area, nothing to wait for)
+            std::vector<int> words(tokens + at, tokens + at + T);
+            words.insert(words.end(), rel.begin(), rel.begin() + nw);
+            if (ntk_store_words(tokens_dev_, T, want_dev_, nw, words.data(), stream_) != NTK_OK) { err_ = "forward: the launch that brings the tokens failed"; return nullptr; }
+        } else {
         if (ntk_stream_synchronize(stream_) != NTK_OK) { err_ = "forward: the stream failed"; return nullptr; }
         memcpy(h_stage_, tokens + at, (size_t)T * sizeof(int));
-        const int nw = w1 - done_want;
         if (nw > 0) memcpy(h_stage_ + chunk_, rel.data(), (size_t)nw * sizeof(int));
         if (ntk_memcpy_h2d_async(tokens_dev_, h_stage_, (size_t)(nw > 0 ? chunk_ + nw : T) * sizeof(int), stream_) != NTK_OK) { err_ = "forward: the copy of the tokens failed"; return nullptr; }
+        }
         const int prev_token = at > 0 ? tokens[at - 1] : pos0 > 0 ? slots_.token(slot, pos0 - 1) : 0;
         const int st = portion(slot, tokens_dev_, prev_token, T, pos0 + at, want_dev_, w1 - done_want, w1 - done_want == 1 && rel[0] == T - 1, logits_ + (size_t)done_want * info_.vocab);
         if (st != NTK_OK) { if (err_.empty()) err_ = std::string("forward: ") + ntk_status_string(st); return nullptr; }
@@ -1808,6 +1816,12 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
 
 int LayerStackModel::copy_logits(float* host, int rows) {
     if (!host || rows < 0 || rows > last_rows_) return NTK_E_SHAPE;
+    if (rows == 1 && h_logits_) {
+        LS_TRY(ntk_copy_out(h_logits_, logits_, (size_t)info_.vocab * sizeof(float), stream_));
+        LS_TRY(ntk_stream_synchronize(stream_));
+        memcpy(host, h_logits_, (size_t)info_.vocab * sizeof(float));
+        return NTK_OK;
+    }
     LS_TRY(ntk_stream_synchronize(stream_));
     if (rows) nt_hip_memcpy_d2h(host, logits_, (size_t)rows * info_.vocab * sizeof(float));
     return NTK_OK;

@@ -58,6 +58,8 @@ void Model::free_all() {
     h_ring_ = nullptr;
     if (h_recent_) nt_hip_free_host(h_recent_);
     h_recent_ = nullptr;
+    if (h_logits_) nt_hip_free_host(h_logits_);
+    h_logits_ = nullptr;
     sample_scratch_ = nullptr;
     d_recent_ = nullptr;
     attn_sync_ = nullptr;
@@ -538,6 +540,7 @@ int Model::alloc_buffers() {   // transformer.cpp:330-391
     attn_scratch_ = (float*)dev(ntk_attention_split_scratch_bytes(cfg_.n_heads, cfg_.head_dim, kMaxAttnSplits), true);   // (zeroed: the arrival counters in front)
     h_token_ = (int*)nt_hip_malloc_host(64);
     h_ring_ = (unsigned long long*)nt_hip_malloc_host(64);
+    h_logits_ = (float*)nt_hip_malloc_host((size_t)cfg_.vocab_size * 4);   // (none: a copy of the runtime's)
     if (h_ring_) memset(h_ring_, 0, 64);
     sample_scratch_ = dev(ntk_sample_scratch_bytes(cfg_.vocab_size), false);
     attn_sync_ = (unsigned*)dev(4096, true);
@@ -599,14 +602,19 @@ float* Model::forward(const int* tokens, int T, int start_pos) {
     void* s = stream_;
     tp_call_ = 0;
     // embedding rows are dequantised on the device (the reference does it on the host and uploads, :419-599)
-    if (ntk_memcpy_h2d_async(tokens_dev_, tokens, (size_t)T * 4, s) != NTK_OK) return nullptr;
+    std::vector<int> pos(T);
+    for (int i = 0; i < T; ++i) pos[i] = start_pos + i;
+    const bool words = T <= 16;   // (tokens and positions as arguments of one launch)
+    if (words) {
+        std::vector<int> both(tokens, tokens + T);
+        both.insert(both.end(), pos.begin(), pos.end());
+        if (ntk_store_words(tokens_dev_, T, positions_, T, both.data(), s) != NTK_OK) return nullptr;
+    } else if (ntk_memcpy_h2d_async(tokens_dev_, tokens, (size_t)T * 4, s) != NTK_OK) return nullptr;
     const int est = ntk_embed_rows(hidden_, token_embd_.ptr, tokens_dev_, T, H, token_embd_.dtype, s);
     if (est == NTK_E_DTYPE) fprintf(stderr, "Error: Unsupported embedding dtype: %s\n", dtype_name(token_embd_.dtype));
     else if (est != NTK_OK) return nullptr;
-    std::vector<int> pos(T);
-    for (int i = 0; i < T; ++i) pos[i] = start_pos + i;
-    if (ntk_memcpy_h2d_async(positions_, pos.data(), (size_t)T * 4, s) != NTK_OK) return nullptr;
-    if (ntk_stream_synchronize(s) != NTK_OK) return nullptr;   // `pos` / `tokens` are host temporaries
+    if (!words && ntk_memcpy_h2d_async(positions_, pos.data(), (size_t)T * 4, s) != NTK_OK) return nullptr;
+    if (!words && ntk_stream_synchronize(s) != NTK_OK) return nullptr;   // `pos` / `tokens` are host temporaries
 
     // The last layer's results are read at the last token only: of the others it needs their cache rows, and the last token takes it as a decoded token does.  One layer of the pass's time
     // less (1 / 32 of 32 layers); prompts of up to 32 tokens spend a layer on its launches, not on its tokens, and keep the whole layer.
@@ -1119,7 +1127,20 @@ int Model::set_device_pos(int pos) {
 }
 int Model::sync() { return ntk_stream_synchronize(stream_); }
 int Model::host_token() const { return *h_token_; }
+int Model::set_device_step(int pos, int token) {
+    if (token < 0 || token >= cfg_.vocab_size) { err_ = "token id out of range"; return NTK_E_SHAPE; }
+    *h_token_ = token;
+    host_pos_ = pos;
+    const int words[2] = {token, pos};
+    return ntk_store_words(d_token_, 1, d_pos_, 1, words, stream_);
+}
 int Model::copy_logits(float* host) {
+    if (h_logits_) {
+        NT_TRY(ntk_copy_out(h_logits_, logits_, (size_t)cfg_.vocab_size * 4, stream_));
+        NT_TRY(ntk_stream_synchronize(stream_));
+        memcpy(host, h_logits_, (size_t)cfg_.vocab_size * 4);
+        return NTK_OK;
+    }
     NT_TRY(ntk_memcpy_d2h_async(host, logits_, (size_t)cfg_.vocab_size * 4, stream_));
     return ntk_stream_synchronize(stream_);
 }

@@ -56,6 +56,7 @@ public:
     int decode_step_fused(bool greedy, bool use_graph);
     int set_device_token(int token);
     int set_device_pos(int pos);
+    int set_device_step(int pos, int token);   // both for ONE step, as arguments of a launch: in the stream's order, nothing waited for
     // attention regime by context length (each regime is its own captured graph: the grid of the attention launch is fixed in it).
     // 0: the single-pass kernel, one workgroup per query head, walks the head's cache serially (4.2 us per layer at 16 positions, 7.5 at
     //    512, 30.7 at 4095).  Beyond 544 positions: ntk_attention_decode_split = partial states of `splits` workgroups + a combine launch:
@@ -214,6 +215,7 @@ private:
     int* d_token_ = nullptr;        // device scalar: id of the token being decoded
     int* h_token_ = nullptr;        // pinned mirror of the argmax result
     unsigned long long* h_ring_ = nullptr;   // pinned ring of 4 x {token, position + 1}: ntk_argmax_advance / wait_token
+    float* h_logits_ = nullptr;       // pinned: the logits on their way to the caller
     std::chrono::steady_clock::time_point wait_t0_;
     float* argmax_scratch_ = nullptr;
     void* sample_scratch_ = nullptr;

@@ -314,9 +314,47 @@ __global__ __launch_bounds__(1024) void gated_rmsnorm_kernel(float* y, int ldy, 
 
 constexpr int kFewRows = 32;   // up to this many rows a row kernel runs workgroups of 1024 threads
 
+// ---- what a pass takes from the host and leaves there: words as arguments of a launch, results by a launch's own stores into pinned memory.  A decoded token of 32000 logits spent 5 + 5 us
+// on two copies of the runtime and waited for the stream twice (a copy into pageable memory is one more round trip of the host); so 2 + 4 and once.
+struct Words { int v[32]; };
+__global__ __launch_bounds__(64) void store_words_kernel(int* __restrict__ a, int na, int* __restrict__ b, int n, const Words w) {
+    const int i = threadIdx.x;
+    if (i >= n) return;
+    if (i < na) a[i] = w.v[i];
+    else b[i - na] = w.v[i];
+}
+__global__ __launch_bounds__(256) void copy_out_kernel(uint32_t* __restrict__ out, const uint32_t* __restrict__ src, size_t words, int wide) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (wide) {
+        if (4 * i + 3 < words) *reinterpret_cast<uint4*>(out + 4 * i) = *reinterpret_cast<const uint4*>(src + 4 * i);
+        else
+            for (size_t k = 4 * i; k < words; ++k) out[k] = src[k];
+    } else if (i < words) out[i] = src[i];
+}
 }  // namespace ntk
 
 using namespace ntk;
+
+int ntk_store_words(int* a, int na, int* b, int nb, const int* values, void* stream) {
+    if ((!a && na > 0) || (!b && nb > 0) || !values) return NTK_E_NULL;
+    if (na < 0 || nb < 0 || na + nb > 32) return NTK_E_SHAPE;
+    if (na + nb == 0) return NTK_OK;
+    Words w{};
+    for (int i = 0; i < na + nb; ++i) w.v[i] = values[i];
+    hipLaunchKernelGGL(store_words_kernel, dim3(1), dim3(64), 0, resolve_stream(stream), a, na, b, na + nb, w);
+    return last_launch_status();
+}
+int ntk_copy_out(void* pinned, const void* src, size_t size, void* stream) {
+    if (!pinned || !src) return NTK_E_NULL;
+    const uintptr_t at = (uintptr_t)pinned | (uintptr_t)src;
+    if (size % 4 || size / 4 > (size_t)0x7FFFFFFF * 256) return NTK_E_SHAPE;
+    if (at & 3) return NTK_E_ALIGN;
+    if (size == 0) return NTK_OK;
+    const int wide = (at & 15) == 0;
+    const size_t words = size / 4, threads = wide ? (words + 3) / 4 : words;
+    hipLaunchKernelGGL(copy_out_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, resolve_stream(stream), static_cast<uint32_t*>(pinned), static_cast<const uint32_t*>(src), words, wide);
+    return last_launch_status();
+}
 
 int ntk_embed_dense(float* out, const void* table, int tdtype, const int* tokens, int T, int vocab, int width, void* stream) {
     return ntk_embed_dense_scaled(out, table, tdtype, tokens, T, vocab, width, 1.0f, stream);
