@@ -366,6 +366,9 @@ typedef struct ntk_gated_recurrence_desc {
 size_t ntk_gated_recurrence_scratch(int T, int H, int dn, int dv, int removal);
 size_t ntk_gated_recurrence_scratch_ex(const ntk_gated_recurrence_desc* d);   /* from d's T, H, dn, dv, az and the per-head options */
 int ntk_gated_recurrence(const ntk_gated_recurrence_desc* d, void* stream);
+/* ONE token of the delta rule with a gate per head and its convolutions (T == 1, head_gates, write_gated, conv_w; d->scratch is not used) together with ntk_head_rmsnorm_gate(act silu, one
+ * weight of dv entries for all heads) of its result, gate [H * dv]: two launches.  NTK_E_SHAPE (nothing launched) beyond dn 128, dv 128 or four taps. */
+int ntk_gated_delta_step(const ntk_gated_recurrence_desc* d, const float* norm_w, const float* gate, float eps, void* stream);
 
 /* ---- moe.hip ---------------------------------------------------------------------------------------------------------------------- */
 /* Router of a mixture of experts, one launch: z = W_r h (F32 weights [E][n]), s = softmax(z); the `top` largest (ties: the lower index), weights

@@ -1357,13 +1357,14 @@ int LayerStackModel::run_unit_ff(const StackLayer& L, const float* h, int T, con
 int LayerStackModel::run_gated_delta(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16) {
     const GatedDeltaMixer& m = L.gdl;
     const int W = info_.width, hv = m.heads * m.vdim;
-    LS_TRY(gated_delta_state(L, h, state, T, pos0, norm_inside, h16));
-    LS_TRY(ntk_head_rmsnorm_gate(att_, hv, att_, hv, m.norm, 0, a_ + m.g_off, (int)m.in.out_f, 2, 1.0f, T, m.heads, m.vdim, eps_, stream_));
+    bool normed = false;
+    LS_TRY(gated_delta_state(L, h, state, T, pos0, norm_inside, h16, &normed));
+    if (!normed) LS_TRY(ntk_head_rmsnorm_gate(att_, hv, att_, hv, m.norm, 0, a_ + m.g_off, (int)m.in.out_f, 2, 1.0f, T, m.heads, m.vdim, eps_, stream_));
     return linear(mix_, W, att_, hv, m.o.ptr, m.o.dtype, T, W, hv, 0);
 }
 
-// ... up to the recurrence's results in att_, the state carried on
-int LayerStackModel::gated_delta_state(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16) {
+// ... up to the recurrence's results in att_, the state carried on; normed: a decoded token's heads may pass their norm and gate in the same launch (then *normed is set)
+int LayerStackModel::gated_delta_state(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16, bool* normed) {
     const GatedDeltaMixer& m = L.gdl;
     const int W = info_.width, na = (int)m.in.out_f, nc = m.channels(), hv = m.heads * m.vdim;
     ntk_dense_desc in{};
@@ -1383,6 +1384,10 @@ int LayerStackModel::gated_delta_state(const StackLayer& L, const float* h, floa
     d.az = a_ + m.b_off; d.lda = na; d.unit_eps = kUnitKeyEps;
     d.G = m.kv_heads; d.unit_q = 1; d.unit_k = 1; d.head_gates = 1; d.write_gated = 1;
     d.state = state; d.H = m.heads; d.dn = m.dim; d.dv = m.vdim; d.q_scale = 1.0f / std::sqrt((float)m.dim); d.pos0 = pos0; d.T = T; d.scratch = rscratch_;
+    if (T == 1 && normed) {
+        const int st = ntk_gated_delta_step(&d, m.norm, a_ + m.g_off, eps_, stream_);
+        if (st != NTK_E_SHAPE) { *normed = true; return st; }
+    }
     return ntk_gated_recurrence(&d, stream_);
 }
 
@@ -1662,7 +1667,7 @@ int LayerStackModel::last_layer_keys(const Run& run, const StackLayer& L, int sl
         if (st == NTK_E_ALIGN) st = ntk_rmsnorm_offset(h1_, L.norm1.w, nullptr, nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
         LS_TRY(st);
     }
-    if (L.mixer == kMixGatedDelta) return gated_delta_state(L, h1_, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0, false, h16);
+    if (L.mixer == kMixGatedDelta) return gated_delta_state(L, h1_, run.state + (size_t)slot * L.gdl.state_floats(), T, pos0, false, h16, nullptr);
     const int na = L.mixer == kMixWindow ? (int)L.att.in.out_f : (int)L.mix.in.out_f;
     ntk_dense_desc d{};
     d.Y = a_ + at; d.ldy = na; d.X = h1_; d.ldx = W; d.W = in.ptr; d.wdtype = in.dtype; d.G = 1; d.row_div = 1; d.T = T; d.N = (int)in.out_f; d.K = W;

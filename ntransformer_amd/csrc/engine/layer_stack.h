@@ -312,7 +312,7 @@ private:
     int run_gated_ff(const StackLayer& L, int T);
     int parse_gated_delta(const Json& L, GatedDeltaMixer& m);
     int run_gated_delta(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16);
-    int gated_delta_state(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16);
+    int gated_delta_state(const StackLayer& L, const float* h, float* state, int T, int pos0, bool norm_inside, const void* h16, bool* normed);
     int run_unit_ff(const StackLayer& L, const float* h, int T, const void* h16 = nullptr, const float* norm_w = nullptr);
     int post_norm_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int rms_seam(const NormW& nw, float* out, int T);

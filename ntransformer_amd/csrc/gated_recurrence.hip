@@ -121,31 +121,37 @@ __global__ __launch_bounds__(64) void gated_recurrence_prepare_kernel(const RecA
 // value channels of the state heads that share them (each channel's carried inputs are read, used and shifted by the one thread that owns the channel), then
 // forms the same vectors as the kernel above, with the same sums in the same lane order.
 constexpr int kStepConvTaps = 16;
-struct ConvTaps {                                        // one channel's carried inputs, taps and present input, all requested before anything is stored
-    float hist[kStepConvTaps - 1], w[kStepConvTaps], x;
+template <int TAPS>
+struct ConvTapsOf {                                        // one channel's carried inputs, taps and present input, all requested before anything is stored
+    float hist[TAPS - 1], w[TAPS], x;
     __device__ __forceinline__ void load(const float* cw, const float* state, int taps, int n, int c, float xin, int pos0) {
 #pragma unroll
-        for (int j = 0; j < kStepConvTaps - 1; ++j) hist[j] = (j < taps - 1 && pos0 - (taps - 1) + j >= 0) ? state[(long long)j * n + c] : 0.0f;
+        for (int j = 0; j < TAPS - 1; ++j) hist[j] = (j < taps - 1 && pos0 - (taps - 1) + j >= 0) ? state[(long long)j * n + c] : 0.0f;
 #pragma unroll
-        for (int j = 0; j < kStepConvTaps; ++j) w[j] = j < taps ? cw[(long long)c * taps + j] : 0.0f;
+        for (int j = 0; j < TAPS; ++j) w[j] = j < taps ? cw[(long long)c * taps + j] : 0.0f;
         x = xin;
     }
-    // the convolution and silu; the carried rows shift in place
-    __device__ __forceinline__ float finish(float* state, int taps, int n, int c) const {
+    // the convolution and silu
+    __device__ __forceinline__ float value(int taps) const {
         float s = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kStepConvTaps - 1; ++j)
+        for (int j = 0; j < TAPS - 1; ++j)
             if (j < taps - 1) s = fmaf(w[j], hist[j], s);
 #pragma unroll
-        for (int j = 0; j < kStepConvTaps; ++j)
+        for (int j = 0; j < TAPS; ++j)
             if (j == taps - 1) s = fmaf(w[j], x, s);
-#pragma unroll
-        for (int j = 1; j < kStepConvTaps - 1; ++j)
-            if (j < taps - 1) state[(long long)(j - 1) * n + c] = hist[j];
-        if (taps > 1) state[(long long)(taps - 2) * n + c] = x;
         return s / (1.0f + expf(-s));
     }
+    // ... and the carried rows shift in place
+    __device__ __forceinline__ float finish(float* state, int taps, int n, int c) const {
+#pragma unroll
+        for (int j = 1; j < TAPS - 1; ++j)
+            if (j < taps - 1) state[(long long)(j - 1) * n + c] = hist[j];
+        if (taps > 1) state[(long long)(taps - 2) * n + c] = x;
+        return value(taps);
+    }
 };
+using ConvTaps = ConvTapsOf<kStepConvTaps>;
 
 template <bool DELTA>
 __global__ __launch_bounds__(256) void gated_recurrence_prepare_step_kernel(const RecArgs a) {
@@ -212,6 +218,115 @@ __global__ __launch_bounds__(256) void gated_recurrence_prepare_step_kernel(cons
                 dst[4 * a.dn + d] = uu * aa;
             }
         }
+    }
+}
+
+// ---- a decoded token of the delta rule with one gate a head: the short convolutions of q, k and v and the state's step in one launch, every head's norm and silu gate and the convolutions'
+// carried inputs in a second.  Three launches before (the pre-pass above 7.9 us, the walk of one token 8.0, the norm 3.4, with 16 heads of 128 x 128 on 8), each little more than its own
+// boundary and its first requests.  A wave takes 16 columns of a head's state, a lane dn / 4 rows of one: u^T S and S^T q meet in two lane exchanges, the only barrier stands behind the
+// convolutions, which every workgroup forms for itself -- so nothing may shift their carried inputs before all have read them: the second launch does.  (All of a q / k head's columns in one
+// workgroup, norm and shift inside: 13.7 us, three launches 15.9, so 9.5; a CU takes 8 us for the 128 KB of state in and out that 64 share here.)
+constexpr int kStepTaps = 4;                             // (of the convolutions; more take the three launches)
+template <int RPL>
+__global__ __launch_bounds__(128) void gated_delta_step_kernel(const RecArgs a) {
+    constexpr int DP = 4 * RPL;
+    __shared__ float qs[DP], ks[DP], vs[32];
+    const int G = a.G > 0 ? a.G : a.H, h = blockIdx.x, g = h / (a.H / G), c0 = blockIdx.y * 32;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cl = wave * 16 + (lane & 15), c = c0 + cl, rg = lane >> 4;
+    const int nch = 2 * G * a.dn + a.H * a.dv;
+    const bool live = c < a.dv;
+    // requests: the channels' inputs and taps (q and k of one index a thread; then the workgroup's values), the head's gates, the state
+    ConvTapsOf<kStepTaps> Q, K, V;
+    const int d = threadIdx.x, cv = c0 + d;
+    const bool hv = d < 32 && cv < a.dv;
+    if (d < a.dn) {
+        Q.load(a.conv_w, a.conv_state, a.conv_taps, nch, g * a.dn + d, a.q[(long long)g * a.dn + d], a.pos0);
+        K.load(a.conv_w, a.conv_state, a.conv_taps, nch, (G + g) * a.dn + d, a.k[(long long)g * a.dn + d], a.pos0);
+    }
+    if (hv) V.load(a.conv_w, a.conv_state, a.conv_taps, nch, 2 * G * a.dn + h * a.dv + cv, a.v[(long long)h * a.dv + cv], a.pos0);
+    const float wz = a.wz[h] + (a.wb ? a.wb[h] : 0.0f), az = a.az[h] + (a.ab ? a.ab[h] : 0.0f), rate = a.decay_rates ? a.decay_rates[h] : a.decay_param;
+    __builtin_amdgcn_sched_barrier(0);
+    float S[RPL];
+    const unsigned at = (unsigned)((h * a.dn + rg * RPL) * a.dv + c), dv = (unsigned)a.dv;   // (32-bit offsets: 64-bit row addresses kept from the loads to the stores are 64 registers)
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) S[j] = a.pos0 > 0 && live && rg * RPL + j < a.dn ? a.state[at + (unsigned)j * dv] : 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
+    if (d < DP) {
+        qs[d] = d < a.dn ? Q.value(a.conv_taps) : 0.0f;
+        ks[d] = d < a.dn ? K.value(a.conv_taps) : 0.0f;
+    }
+    if (d < 32) vs[d] = hv ? V.value(a.conv_taps) : 0.0f;
+    __syncthreads();
+    float ss = 0.0f, sq = 0.0f;
+    for (int e = lane; e < a.dn; e += 64) { ss = fmaf(ks[e], ks[e], ss); sq = fmaf(qs[e], qs[e], sq); }   // (every wave for itself, in the pre-pass's lane order)
+    const float inv_k = 1.0f / sqrtf(wave_sum(ss) + a.unit_eps);
+    const float qmul = a.unit_q ? a.q_scale / sqrtf(wave_sum(sq) + a.unit_eps) : a.q_scale;
+    const float kmul = a.unit_k ? inv_k : 1.0f;
+    const float w = decay_of(wz, a.decay_form, rate), ah = 1.0f / (1.0f + expf(-az));
+    const float v = vs[cl] * ah;
+    // (what is one factor for a column stays outside its sums: u^T S = w / |k| sum k S, the step's two k terms are one, o = q_scale / |q| sum S q)
+    float p0 = 0.0f, p1 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < RPL; j += 4) {
+        const float4 k4 = *reinterpret_cast<const float4*>(ks + rg * RPL + j);
+        p0 = fmaf(k4.x, S[j], p0);
+        p1 = fmaf(k4.y, S[j + 1], p1);
+        p0 = fmaf(k4.z, S[j + 2], p0);
+        p1 = fmaf(k4.w, S[j + 3], p1);
+    }
+    float us = p0 + p1;
+    us += __shfl_xor(us, 16, 64);
+    us += __shfl_xor(us, 32, 64);
+    const float coef = fmaf(-(inv_k * ah), us * (inv_k * w), kmul * v);
+    float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < RPL; j += 4) {
+        const float4 k4 = *reinterpret_cast<const float4*>(ks + rg * RPL + j), q4 = *reinterpret_cast<const float4*>(qs + rg * RPL + j);
+        S[j] = fmaf(w, S[j], k4.x * coef);
+        S[j + 1] = fmaf(w, S[j + 1], k4.y * coef);
+        S[j + 2] = fmaf(w, S[j + 2], k4.z * coef);
+        S[j + 3] = fmaf(w, S[j + 3], k4.w * coef);
+        o0 = fmaf(S[j], q4.x, o0);
+        o1 = fmaf(S[j + 1], q4.y, o1);
+        o0 = fmaf(S[j + 2], q4.z, o0);
+        o1 = fmaf(S[j + 3], q4.w, o1);
+    }
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+        if (live && rg * RPL + j < a.dn) a.state[at + (unsigned)j * dv] = S[j];
+    float o = o0 + o1;
+    o += __shfl_xor(o, 16, 64);
+    o += __shfl_xor(o, 32, 64);
+    if (live && rg == 0) a.out[(long long)h * a.dv + c] = o * qmul;
+}
+// a workgroup a head: its norm and gate (first wave, two columns a lane), and a share of all channels' carried inputs
+__global__ __launch_bounds__(256) void gated_delta_finish_kernel(const RecArgs a, const float* __restrict__ norm, const float* __restrict__ gate, float eps) {
+    const int h = blockIdx.x, lane = threadIdx.x;
+    const int G = a.G > 0 ? a.G : a.H, nqk = 2 * G * a.dn, nch = nqk + a.H * a.dv;
+    if (lane < 64) {
+        float x[2], ss = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            x[u] = lane + 64 * u < a.dv ? a.out[(long long)h * a.dv + lane + 64 * u] : 0.0f;
+            ss = fmaf(x[u], x[u], ss);
+        }
+        const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)a.dv + eps);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int c = lane + 64 * u;
+            if (c >= a.dv) continue;
+            const float gg = gate[(long long)h * a.dv + c];
+            a.out[(long long)h * a.dv + c] = x[u] * inv * norm[c] * (gg * (1.0f / (1.0f + expf(-gg))));
+        }
+    }
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < nch; c += gridDim.x * 256) {   // (a channel's history belongs to one thread)
+        const float x = c < G * a.dn ? a.q[c] : c < nqk ? a.k[c - G * a.dn] : a.v[c - nqk];
+        float keep[kStepTaps - 1];
+#pragma unroll
+        for (int j = 1; j < kStepTaps - 1; ++j) keep[j] = j < a.conv_taps - 1 && a.pos0 - (a.conv_taps - 1) + j >= 0 ? a.conv_state[(long long)j * nch + c] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < kStepTaps - 1; ++j)
+            if (j < a.conv_taps - 1) a.conv_state[(long long)j * nch + c] = j + 1 < a.conv_taps - 1 ? keep[j + 1 < kStepTaps - 1 ? j + 1 : j] : x;
     }
 }
 
@@ -667,4 +782,28 @@ int ntk_gated_recurrence(const ntk_gated_recurrence_desc* d, void* stream) {
     if (d->dn <= 16 * 16) return launch_rec<16, 16>(a, s);
     if (d->dn <= 16 * 32) return launch_rec<16, 32>(a, s);
     return launch_rec<32, 32>(a, s);
+}
+
+int ntk_gated_delta_step(const ntk_gated_recurrence_desc* d, const float* norm_w, const float* gate, float eps, void* stream) {
+    if (!d || !d->out || !d->q || !d->k || !d->v || !d->wz || !d->az || !d->state || !d->conv_w || !norm_w || !gate) return NTK_E_NULL;
+    if (d->T != 1 || !d->head_gates || !d->write_gated || d->H <= 0 || d->dn <= 0 || d->dn > 128 || d->dv <= 0 || d->pos0 < 0) return NTK_E_SHAPE;
+    if (d->decay_form != NTK_DECAY_GIVEN && d->decay_form != NTK_DECAY_SIGMOID_ROOT && d->decay_form != NTK_DECAY_EXP_SIGMOID && d->decay_form != NTK_DECAY_EXP_SOFTPLUS) return NTK_E_SHAPE;
+    if (d->decay_form == NTK_DECAY_SIGMOID_ROOT && !(d->decay_param > 0.0f)) return NTK_E_SHAPE;
+    if (d->G < 0 || (d->G > 0 && d->H % d->G)) return NTK_E_SHAPE;
+    if (d->conv_taps < 1 || d->conv_taps > kStepConvTaps || (d->conv_taps > 1 && !d->conv_state)) return NTK_E_SHAPE;
+    const int G = d->G > 0 ? d->G : d->H;
+    if (d->dv > 128 || d->conv_taps > kStepTaps || (long long)d->H * d->dn * d->dv >= 1LL << 30 || d->ldq < G * d->dn || d->ldk < G * d->dn || d->ldv < d->H * d->dv ||
+        d->ldo < d->H * d->dv || d->ldw < d->H || d->lda < d->H) return NTK_E_SHAPE;
+    const RecArgs a{d->out, d->ldo, d->q, d->ldq, d->k, d->ldk, d->v, d->ldv, d->wz, d->ldw, d->wb, d->decay_form, d->decay_param, d->az, d->lda, d->ab, d->unit_eps,
+                    d->state, d->H, d->dn, d->dv, d->q_scale, d->pos0, 1, 0, nullptr, 1, 1, nullptr, nullptr, nullptr, nullptr,
+                    d->G, d->unit_q, d->unit_k, 1, 1, d->decay_rates, nullptr, d->conv_w, d->conv_state, d->conv_taps};
+    hipStream_t s = resolve_stream(stream);
+    const dim3 grid(d->H, (d->dv + 31) / 32);
+    if (d->dn <= 32) hipLaunchKernelGGL(gated_delta_step_kernel<8>, grid, dim3(128), 0, s, a);
+    else if (d->dn <= 64) hipLaunchKernelGGL(gated_delta_step_kernel<16>, grid, dim3(128), 0, s, a);
+    else hipLaunchKernelGGL(gated_delta_step_kernel<32>, grid, dim3(128), 0, s, a);
+    const int st = last_launch_status();
+    if (st != NTK_OK) return st;
+    hipLaunchKernelGGL(gated_delta_finish_kernel, dim3(d->H), dim3(256), 0, s, a, norm_w, gate, eps);
+    return last_launch_status();
 }
