@@ -64,6 +64,8 @@ typedef struct ntk_dense_desc {
 #define NTK_ACT_RELU2 1
 int ntk_dense_few_rows(void);   /* up to this many rows a product takes the row-streaming form */
 int ntk_dense(const ntk_dense_desc* d, void* stream);
+/* ... with its results capped: Y = cap * tanh(y / cap) (ntk_softcap_rows behind it, inside its launch where the rows are few).  cap > 0; no activation, no accumulate, no glu_ff. */
+int ntk_dense_capped(const ntk_dense_desc* d, float cap, void* stream);
 /* The same product for more than ntk_dense_few_rows() rows over activations that lie in memory as the product takes them: bfloat16 beside bfloat16 weights (the launch that wrote
  * them rounded them: the same values as ntk_dense's rounding at the product's input), F32 beside F32 ones:
  *   x16 : [x16_rows][ldx16] (16-byte aligned rows), in the place of d->X (which may be NULL);
@@ -105,6 +107,8 @@ int ntk_residual_add(float* x, const float* a, const float* b, int n, void* stre
 
 /* out[t][:] = table[tokens[t]][:] * scale */
 int ntk_embed_dense_scaled(float* out, const void* table, int tdtype, const int* tokens, int T, int vocab, int width, float scale, void* stream);
+/* ... of one token that is given with the launch (ntk_embed_dense_scaled's rows of 16-byte aligned tables, width a multiple of 4; NTK_E_ALIGN else) */
+int ntk_embed_token(float* out, const void* table, int tdtype, int token, int vocab, int width, float scale, void* stream);
 /* ... and a row of a second table picked by the token and the one before it: out[t][:] = table[tokens[t]][:] * scale + bigram[r][:] with
  * r = (tokens[t-1] * mul_prev + tokens[t] * mul_cur) mod buckets (64-bit), and r = buckets for a sequence's first token (pos0 + t == 0); bigram [buckets + 1][width]
  * in the table's dtype.  prev is the token before tokens[0] (unused when pos0 == 0). */
@@ -226,6 +230,13 @@ size_t ntk_prompt_attention_image_bytes(int positions, int kv_heads, int key_ent
  * rotated part, dr == 0 only: then the fold reads nothing that it writes) */
 int ntk_latent_fold_query_prepare(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int R, float* cache, int row, const float* kv,
                                   int ldkv, const float* norm_w, float eps, int pos0, void* stream);
+/* ... and with rotated parts: ntk_latent_prepare (the cache rows; q itself is only read) and ntk_latent_fold_query in one launch */
+int ntk_latent_fold_query_rotate(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int dr, int R, const ntk_rotary* rot, float* cache, int row,
+                                 const float* kv, int ldkv, const float* norm_w, float eps, int pos0, void* stream);
+/* ntk_latent_attention's shared form and ntk_latent_unfold_value_ex of its result: the states of the parts meet in the launch that unfolds them where they are few enough for that to be the
+ * faster (lat, the joined states, is written and read in between elsewhere).  scratch as in ntk_latent_attention. */
+int ntk_latent_attention_unfold(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,
+                                int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale, float* scratch, void* stream);
 int ntk_latent_fold_query(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int dr, int R, void* stream);
 /* out[t][h*dv + v] = sum_r W_uv[h*dv + v][r] * lat[t][h][r]  (the value up-projection applied after the weighted sum), times sigmoid(gate[t][h*dv+v]) if gate */
 int ntk_latent_unfold_value(float* out, int ldo, const float* lat, const void* w_uv, int wdtype, const float* gate, int ldg, int T, int H, int dv, int R,

@@ -38,7 +38,9 @@ struct DenseArgs {
     const float* add_y; int ld_add; const float* add_w; float add_eps, add_mult; float* x_out; int ldxo;   // few-row form only: see ntk_dense_desc
 };
 
-__device__ __forceinline__ float activate(float v, int act) {
+constexpr int kActCap = -1;                             // cap * tanh(v / cap), cap in glu_limit: of ntk_dense_capped alone
+__device__ __forceinline__ float activate(float v, int act, float cap) {
+    if (act == kActCap) return cap * tanhf(v / cap);
     if (act == NTK_ACT_RELU2) { const float p = fmaxf(v, 0.0f); return p * p; }
     return v;
 }
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(const DenseArgs a) {
                 t = gg * (1.0f / (1.0f + expf(-a.glu_alpha * zz))) * (uu + a.glu_up_offset);
             }
             float* y = a.Y + (long long)r * a.ldy + n0 + i;
-            *y = a.accumulate ? *y + t : activate(t, a.act);
+            *y = a.accumulate ? *y + t : activate(t, a.act, a.glu_limit);
         }
     }
 }
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(256) void moe_few_up_kernel(const MoeFewArgs a) {
             if constexpr (GLU) {
                 const float limit = chosen ? a.limit : a.shared_limit, g = fminf(s[i], limit), u = fminf(fmaxf(s[RW + i], -limit), limit);
                 v = g * (1.0f / (1.0f + expf(-a.alpha * g))) * (u + a.up_offset);
-            } else v = activate(s[i], a.act);
+            } else v = activate(s[i], a.act, 0.0f);
             a.mid[(long long)t * rows + m0 + i] = v * wt;
         }
     }
@@ -631,7 +633,16 @@ int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* st
     return last_launch_status();
 }
 
-int ntk_dense(const ntk_dense_desc* d, void* stream) {
+static int dense_with(const ntk_dense_desc* d, float cap, void* stream);
+int ntk_dense(const ntk_dense_desc* d, void* stream) { return dense_with(d, 0.0f, stream); }
+int ntk_dense_capped(const ntk_dense_desc* d, float cap, void* stream) {
+    if (!d) return NTK_E_NULL;
+    if (!(cap > 0.0f) || d->act || d->accumulate || d->glu_ff > 0) return NTK_E_SHAPE;
+    const bool inside = d->T <= kGemvRows;              // (a launch of 4.6 us less behind the head of a decoded token)
+    const int st = dense_with(d, inside ? cap : 0.0f, stream);
+    return st != NTK_OK || inside ? st : ntk_softcap_rows(d->Y, d->ldy, cap, d->T, d->N, stream);
+}
+static int dense_with(const ntk_dense_desc* d, float cap, void* stream) {
     if (!d || !d->Y || !d->X || !d->W) return NTK_E_NULL;
     if (d->wdtype != NTK_DT_BF16 && d->wdtype != NTK_DT_F32) return NTK_E_DTYPE;
     if (d->T < 0 || d->N <= 0 || d->K <= 0 || d->ldx < d->K || d->ldy < (d->glu_ff > 0 ? d->glu_ff : d->N)) return NTK_E_SHAPE;
@@ -650,6 +661,7 @@ int ntk_dense(const ntk_dense_desc* d, void* stream) {
         if ((size_t)d->K * 4 > 160 * 1024 - 1024) return NTK_E_SHAPE;
         a.glu_ff = d->glu_ff; a.glu_limit = d->glu_limit; a.glu_alpha = d->glu_alpha; a.glu_up_offset = d->glu_up_offset; a.glu_cubic = d->glu_cubic;
         a.norm_w = d->norm_w; a.norm_eps = d->norm_eps; a.norm_offset = d->norm_offset;
+        if (cap > 0.0f) { a.act = kActCap; a.glu_limit = cap; }
         a.vec = (d->K % 8 == 0) && !((uintptr_t)d->W & 15) && !((d->wstride * (d->wdtype == NTK_DT_BF16 ? 2 : 4)) & 15);
         a.xvec = (d->K % 4 == 0) && (d->ldx % 4 == 0) && !((uintptr_t)d->X & 15) && !((uintptr_t)d->norm_w & 15);
         if (d->add_y) {

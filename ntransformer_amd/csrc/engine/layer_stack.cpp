@@ -1099,14 +1099,13 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
     }
     ntk_rotary rot{m.rot_freq, m.rot_mag, m.rot_dims, m.rot_layout};
     const bool own = m.kv_from < 0;                       // (else: the rows another layer wrote for these tokens earlier in the pass)
-    const bool beside = own && m.rot_dim == 0 && T <= kSharedRows;      // nothing rotated, few tokens: the cache rows are written beside the queries' fold
+    const bool beside = own && T <= kSharedRows;      // few tokens: the cache rows are written beside the queries' fold
     if (own && !beside) LS_TRY(ntk_latent_prepare(cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, m.kv_rank, m.rot_dim, q, ldq, H, qd, &rot, pos0, T, stream_));
     if (T <= kSharedRows) {
-        if (beside) LS_TRY(ntk_latent_fold_query_prepare(qf_, q, ldq, m.uk.ptr, m.uk.dtype, T, H, m.dim, m.kv_rank, cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, pos0, stream_));
+        if (beside) LS_TRY(ntk_latent_fold_query_rotate(qf_, q, ldq, m.uk.ptr, m.uk.dtype, T, H, m.dim, m.rot_dim, m.kv_rank, &rot, cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, pos0, stream_));
         else LS_TRY(ntk_latent_fold_query(qf_, q, ldq, m.uk.ptr, m.uk.dtype, T, H, m.dim, m.rot_dim, m.kv_rank, stream_));
-        LS_TRY(ntk_latent_attention(lat_, H * m.kv_rank, qf_, H * row, nullptr, 0, nullptr, 0, cache, row, m.kv_rank, m.rot_dim, H, m.dim, m.vdim, 1, pos0, T, 0,
-                                    m.window, m.scale, scratch_, stream_));
-        LS_TRY(ntk_latent_unfold_value_ex(att_, hv, lat_, m.uv.ptr, m.uv.dtype, a_ + m.g_off, na, m.head_gate ? 1 : 0, T, H, m.vdim, m.kv_rank, stream_));
+        LS_TRY(ntk_latent_attention_unfold(att_, hv, m.uv.ptr, m.uv.dtype, a_ + m.g_off, na, m.head_gate ? 1 : 0, m.vdim, lat_, qf_, cache, row, m.kv_rank, m.rot_dim, H, pos0, T, m.window,
+                                           m.scale, scratch_, stream_));
     } else {
         const int key0 = m.window > 0 ? std::max(0, pos0 - m.window + 1) : 0;
         const int nkeys = pos0 + T - key0;
@@ -1678,8 +1677,8 @@ int LayerStackModel::last_layer_keys(const Run& run, const StackLayer& L, int sl
     return ntk_latent_prepare(run.cache + (size_t)slot * opt_.max_context * m.row(), m.row(), a_ + m.kv_off, na, m.kv_norm, eps_, m.kv_rank, m.rot_dim, nullptr, 0, 0, 0, &rot, pos0, T, stream_);
 }
 
-// want_last: the portion's last token is wanted and no other
-int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out) {
+// want_last: the portion's last token is wanted and no other; token >= 0: the portion's only token, not in tokens_dev
+int LayerStackModel::portion(int slot, const int* tokens_dev, int token, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out) {
     const int W = info_.width;
     // (the embedding is kept beside the stream only where a repeated span is entered through a projection of both)
     const bool keep_embedding = has_loop_ && form_.loop_projection;
@@ -1693,6 +1692,8 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, in
         LS_TRY(ntk_embed_sinusoid(x_, embed_.ptr, embed_.dtype, tokens_dev, T, info_.vocab, W, embed_scale_, sin_freq_, pos0, stream_));
     } else if (buckets_ > 0) {
         LS_TRY(ntk_embed_bigram(x_, embed_.ptr, bigram_.ptr, embed_.dtype, tokens_dev, prev_token, pos0, T, info_.vocab, W, embed_scale_, buckets_, mul_prev_, mul_cur_, stream_));
+    } else if (token >= 0) {
+        LS_TRY(ntk_embed_token(keep_embedding ? x0_ : x_, embed_.ptr, embed_.dtype, token, info_.vocab, W, embed_scale_, stream_));
     } else
     LS_TRY(ntk_embed_dense_scaled(keep_embedding ? x0_ : x_, embed_.ptr, embed_.dtype, tokens_dev, T, info_.vocab, W, embed_scale_, stream_));
     bool x_is_x0 = keep_embedding;   // until the first layer run writes x_
@@ -1754,8 +1755,10 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int prev_token, in
         else if (final_norm_.b) { LS_TRY(ntk_layernorm(hn_, W, rows, W, final_norm_.w, final_norm_.b, n_want, W, eps_, 0, stream_)); d.X = hn_; }
         else if (n_want <= ntk_dense_few_rows()) { d.norm_w = final_norm_.w; d.norm_eps = eps_; d.norm_offset = norm_offset_; }   // the output norm inside the head's launch
         else { LS_TRY(ntk_rmsnorm_offset(hn_, final_norm_.w, nullptr, nullptr, W, rows, W, n_want, W, eps_, norm_offset_, stream_)); d.X = hn_; }
-        LS_TRY(product(d));
-        if (logit_softcap_ > 0.0f) LS_TRY(ntk_softcap_rows(logits_out, info_.vocab, logit_softcap_, n_want, info_.vocab, stream_));
+        if (logit_softcap_ > 0.0f) {
+            d.scratch = pscratch_; d.scratch_bytes = pscratch_bytes_;
+            LS_TRY(ntk_dense_capped(&d, logit_softcap_, stream_));
+        } else LS_TRY(product(d));
         if (logit_scale_ != 1.0f) LS_TRY(ntk_scale(logits_out, (long long)n_want * info_.vocab, logit_scale_, stream_));
     }
     return NTK_OK;
@@ -1798,7 +1801,10 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         // the pinned staging area is free once the previous pass's copy has run: wait for the stream (idle already after a copy_logits), then one
         // stream-ordered copy brings the tokens and the wanted places
         const int nw = w1 - done_want;
-        if (T + nw <= 32) {   // (a few of them as arguments of a launch: no staging area, nothing to wait for)
+        // (a decoded token goes with the launch of its embedding, where that is the plain table's)
+        const bool alone = T == 1 && nw <= 1 && tokens[at] >= 0 && info_.width % 4 == 0 && !((uintptr_t)embed_.ptr & 15) && !(form_.gated || form_.post_norm || buckets_ > 0);
+        if (alone) {
+        } else if (T + nw <= 32) {   // (a few of them as arguments of a launch: no staging area, nothing to wait for)
             std::vector<int> words(tokens + at, tokens + at + T);
             words.insert(words.end(), rel.begin(), rel.begin() + nw);
             if (ntk_store_words(tokens_dev_, T, want_dev_, nw, words.data(), stream_) != NTK_OK) { err_ = "forward: the launch that brings the tokens failed"; return nullptr; }
@@ -1809,7 +1815,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         if (ntk_memcpy_h2d_async(tokens_dev_, h_stage_, (size_t)(nw > 0 ? chunk_ + nw : T) * sizeof(int), stream_) != NTK_OK) { err_ = "forward: the copy of the tokens failed"; return nullptr; }
         }
         const int prev_token = at > 0 ? tokens[at - 1] : pos0 > 0 ? slots_.token(slot, pos0 - 1) : 0;
-        const int st = portion(slot, tokens_dev_, prev_token, T, pos0 + at, want_dev_, w1 - done_want, w1 - done_want == 1 && rel[0] == T - 1, logits_ + (size_t)done_want * info_.vocab);
+        const int st = portion(slot, tokens_dev_, alone ? tokens[at] : -1, prev_token, T, pos0 + at, want_dev_, w1 - done_want, w1 - done_want == 1 && rel[0] == T - 1, logits_ + (size_t)done_want * info_.vocab);
         if (st != NTK_OK) { if (err_.empty()) err_ = std::string("forward: ") + ntk_status_string(st); return nullptr; }
         done_want = w1;
     }

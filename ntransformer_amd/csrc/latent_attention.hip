@@ -407,8 +407,9 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(float* out,
 // ------------------------------------------------------------------------------------------------------------------- fold / unfold
 // qf[t][h][r] = sum_d q[t][h][d] W_uk[h * dn + d][r]; rotated part copied behind.  grid (R / 64, H, T): 64 columns per workgroup, the d range in
 // four parts (one per wave), added through LDS in wave order
-// kv != NULL (dr == 0): the workgroups (0, H, T) write the tokens' normed latents into the cache rows beside that
-struct FoldPrepare { float* cache; int row; const float* kv; int ldkv; const float* norm_w; float eps; int pos0; };
+// kv != NULL: the workgroups (0, H, T) write the tokens' cache rows beside that -- normed latents, rotated key parts -- and the queries' rotated parts turn on their way (dr == 0: neither has
+// one), by latent_prepare_kernel's expressions.  A decoded token's two launches of 5.0 and 4.2 us are one of 4.6 - 4.9 (16 heads of 128 + 64, rank 512).
+struct FoldPrepare { float* cache; int row; const float* kv; int ldkv; const float* norm_w; float eps; int pos0; const double* freq; float mag; int dims, halves; };
 template <typename WT>
 __global__ __launch_bounds__(256) void latent_fold_query_kernel(float* qf, const float* q, int ldq, const WT* w, int H, int dn, int dr, int R, const FoldPrepare p) {
     extern __shared__ float qs[];      // [dn + dr] then [4][64] partial sums
@@ -420,6 +421,15 @@ __global__ __launch_bounds__(256) void latent_fold_query_kernel(float* qf, const
         for (int i = threadIdx.x; i < R; i += 256) ss = fmaf(src[i], src[i], ss);
         const float inv = 1.0f / sqrtf(block_sum(ss, qs) / (float)R + p.eps);
         for (int i = threadIdx.x; i < R; i += 256) dst[i] = src[i] * inv * p.norm_w[i];
+        const int half = p.dims / 2, pair = p.halves ? half : 1, step = p.halves ? 1 : 2;
+        for (int i = threadIdx.x; i < half; i += 256) {
+            const double ang = (double)(p.pos0 + (int)blockIdx.z) * p.freq[i];
+            float ra, rb;
+            rope_rotate(src[R + step * i], src[R + step * i + pair], (float)(cos(ang) * (double)p.mag), (float)(sin(ang) * (double)p.mag), ra, rb);
+            dst[R + step * i] = ra;
+            dst[R + step * i + pair] = rb;
+        }
+        for (int i = p.dims + threadIdx.x; i < dr; i += 256) dst[R + i] = src[R + i];
         return;
     }
     float* part = qs + dn + dr;
@@ -443,8 +453,17 @@ __global__ __launch_bounds__(256) void latent_fold_query_kernel(float* qf, const
     part[wave * 64 + lane] = s;
     __syncthreads();
     if (wave == 0 && r < R) o[r] = ((part[lane] + part[64 + lane]) + part[128 + lane]) + part[192 + lane];
-    if (blockIdx.x == 0)
-        for (int d = threadIdx.x; d < dr; d += 256) o[R + d] = qs[dn + d];
+    if (blockIdx.x == 0) {
+        const int half = p.dims / 2, pair = p.halves ? half : 1, step = p.halves ? 1 : 2;
+        for (int i = threadIdx.x; i < half; i += 256) {
+            const double ang = (double)(p.pos0 + t) * p.freq[i];
+            float ra, rb;
+            rope_rotate(qs[dn + step * i], qs[dn + step * i + pair], (float)(cos(ang) * (double)p.mag), (float)(sin(ang) * (double)p.mag), ra, rb);
+            o[R + step * i] = ra;
+            o[R + step * i + pair] = rb;
+        }
+        for (int d = p.dims + threadIdx.x; d < dr; d += 256) o[R + d] = qs[dn + d];
+    }
 }
 
 // out[t][h * dv + v] = W_uv[h * dv + v][:] . lat[t][h][:] (* sigmoid(gate));  grid (dv / 16, H, T): a wave owns 4 outputs and walks their rows together
@@ -483,9 +502,100 @@ __global__ __launch_bounds__(256) void latent_unfold_value_kernel(float* out, in
     }
 }
 
+// ... with the parts' states (latent_attention_shared_kernel) joined in front, for ranks of whole pieces of eight up to 512: every workgroup of a head joins them for itself, two columns a thread.
+// us of the merge above and the unfolding / so, 16 heads of 128, rank 512, one token: 2 states 3.6 + 6.0 / 5.1, 36 states 4.1 + 6.4 / 8.3
+constexpr int kJoinStates = 48;                          // (states of all tokens: beyond, what the workgroups of a head read again costs more than the launch)
+template <typename WT>
+__global__ __launch_bounds__(256) void latent_join_unfold_kernel(float* out, int ldo, const float* scratch, int splits, const WT* w, const float* gate, int ldg, int H, int dv, int R, int head_gate) {
+    __shared__ float wt[256], red[16];
+    __shared__ __attribute__((aligned(16))) float ls[512];
+    const int h = blockIdx.y, t = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int v0 = blockIdx.x * 16 + wave * 4, r0 = lane * 8, c = 2 * tid;
+    float wv[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const WT* row = w + ((long long)h * dv + min(v0 + i, dv - 1)) * R + r0;
+        if constexpr (sizeof(WT) == 2) {
+            uint4 b{0u, 0u, 0u, 0u};
+            if (r0 < R) b = *reinterpret_cast<const uint4*>(row);
+            const uint32_t u[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { wv[i][2 * k] = __uint_as_float(u[k] << 16); wv[i][2 * k + 1] = __uint_as_float(u[k] & 0xFFFF0000u); }
+        } else {
+            float4 a{0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+            if (r0 < R) { a = *reinterpret_cast<const float4*>(row); b = *reinterpret_cast<const float4*>(row + 4); }
+            wv[i][0] = a.x; wv[i][1] = a.y; wv[i][2] = a.z; wv[i][3] = a.w; wv[i][4] = b.x; wv[i][5] = b.y; wv[i][6] = b.z; wv[i][7] = b.w;
+        }
+    }
+    const float* st = scratch + ((long long)t * H + h) * splits * (2 + R);
+    const long long step = 2 + R;
+    float2 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = u < splits && c < R ? *reinterpret_cast<const float2*>(st + u * step + 2 + c) : float2{0.0f, 0.0f};
+    const float m = tid < splits ? st[tid * step] : -INFINITY, l = tid < splits ? st[tid * step + 1] : 0.0f;
+    const float mx = block_max(m, red);
+    const float we = m == -INFINITY ? 0.0f : expf(m - mx);
+    wt[tid] = we;
+    const float den = block_sum(we * l, red);            // (its barriers publish wt)
+    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+    float2 sum{0.0f, 0.0f};
+    for (int s = 0; s < splits; s += 8) {                // states in order, eight requested ahead
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (s + u < splits) { sum.x = fmaf(x[u].x, wt[s + u], sum.x); sum.y = fmaf(x[u].y, wt[s + u], sum.y); }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (s + 8 + u < splits && c < R) x[u] = *reinterpret_cast<const float2*>(st + (s + 8 + u) * step + 2 + c);
+    }
+    if (c < R) *reinterpret_cast<float2*>(ls + c) = float2{sum.x * inv, sum.y * inv};
+    __syncthreads();
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (r0 < R) {
+        const float4 a = *reinterpret_cast<const float4*>(ls + r0), b = *reinterpret_cast<const float4*>(ls + r0 + 4);
+        const float xx[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) s[i] = fmaf(wv[i][k], xx[k], s[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float tsum = wave_sum_lane63(s[i]);
+        if (lane == 63 && v0 + i < dv) {
+            if (gate) tsum *= 1.0f / (1.0f + expf(-gate[(long long)t * ldg + (head_gate ? h : h * dv + v0 + i)]));
+            out[(long long)t * ldo + h * dv + v0 + i] = tsum;
+        }
+    }
+}
+
 static int shared_splits(int nkeys) {       // workgroups per row tile: one per tile of KB keys, at most 128
     const int tiles = (nkeys + KB - 1) / KB + 1;     // (+ 1: a tile's first key is the window's, not a multiple of KB)
     return tiles < 1 ? 1 : tiles > 128 ? 128 : tiles;
+}
+
+static int shared_keys(int pos0, int T, int window) { return window > 0 ? (window + T - 1 < pos0 + T ? window + T - 1 : pos0 + T) : pos0 + T; }
+// the shared form: every part's states into the scratch; merge: joined in `out`
+static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, int ldq, const float* cache, int row, int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale,
+                         float* scratch, bool merge, void* stream) {
+    if (!scratch) return NTK_E_NULL;
+    if (kv_rank > 512) return NTK_E_SHAPE;
+    hipStream_t s = resolve_stream(stream);
+    sa.q = q; sa.ldq = ldq; sa.cache = cache; sa.row = row; sa.R = kv_rank; sa.dr = rot_dim; sa.H = H; sa.pos0 = pos0; sa.T = T; sa.window = window;
+    sa.scale = scale; sa.scratch = scratch;
+    sa.splits = shared_splits(shared_keys(pos0, T, window));
+    const int rows = T * H, DK = kv_rank + rot_dim;
+    if (((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) > 156 * 1024) return NTK_E_SHAPE;     // (keys of up to 812 entries)
+    const size_t lds = ((size_t)KB * (((DK + 15) & ~15) + 4) + 5 * SROWS * (KB + 4) + 3 * SROWS) * sizeof(float);
+    static bool raised_s = false;   // (idempotent: a race sets the same attribute twice)
+    if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel<13, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
+    const dim3 grid((rows + SROWS - 1) / SROWS, sa.splits);
+    if (DK <= 128) hipLaunchKernelGGL((latent_attention_shared_kernel<2, 2>), grid, dim3(256), lds, s, sa);
+    else if (DK <= 320) hipLaunchKernelGGL((latent_attention_shared_kernel<5, 5>), grid, dim3(256), lds, s, sa);
+    else hipLaunchKernelGGL((latent_attention_shared_kernel<13, 8>), grid, dim3(256), lds, s, sa);
+    const int st = last_launch_status();
+    if (st != NTK_OK || !merge) return st;
+    hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(rows, (kv_rank + 63) / 64), dim3(256), 0, s, out, ldo, (const float*)scratch, sa.splits, kv_rank, H);
+    return last_launch_status();
 }
 
 }  // namespace ntk
@@ -529,26 +639,8 @@ int ntk_latent_attention_ex(float* out, int ldo, const float* q, int ldq, const 
     if (T == 0) return NTK_OK;
     hipStream_t s = resolve_stream(stream);
     if (shared) {
-        if (!scratch) return NTK_E_NULL;
-        if (kv_rank > 512) return NTK_E_SHAPE;
         SharedArgs sa{};
-        sa.q = q; sa.ldq = ldq; sa.cache = cache; sa.row = row; sa.R = kv_rank; sa.dr = rot_dim; sa.H = H; sa.pos0 = pos0; sa.T = T; sa.window = window;
-        sa.scale = scale; sa.scratch = scratch;
-        const int nkeys = window > 0 ? (window + T - 1 < pos0 + T ? window + T - 1 : pos0 + T) : pos0 + T;
-        sa.splits = shared_splits(nkeys);
-        const int rows = T * H, DK = kv_rank + rot_dim;
-        if (((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) > 156 * 1024) return NTK_E_SHAPE;     // (keys of up to 812 entries)
-        const size_t lds = ((size_t)KB * (((DK + 15) & ~15) + 4) + 5 * SROWS * (KB + 4) + 3 * SROWS) * sizeof(float);
-        static bool raised_s = false;   // (idempotent: a race sets the same attribute twice)
-        if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel<13, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
-        const dim3 grid((rows + SROWS - 1) / SROWS, sa.splits);
-        if (DK <= 128) hipLaunchKernelGGL((latent_attention_shared_kernel<2, 2>), grid, dim3(256), lds, s, sa);
-        else if (DK <= 320) hipLaunchKernelGGL((latent_attention_shared_kernel<5, 5>), grid, dim3(256), lds, s, sa);
-        else hipLaunchKernelGGL((latent_attention_shared_kernel<13, 8>), grid, dim3(256), lds, s, sa);
-        int st = last_launch_status();
-        if (st != NTK_OK) return st;
-        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(rows, (kv_rank + 63) / 64), dim3(256), 0, s, out, ldo, (const float*)scratch, sa.splits, kv_rank, H);
-        return last_launch_status();
+        return launch_shared(sa, out, ldo, q, ldq, cache, row, kv_rank, rot_dim, H, pos0, T, window, scale, scratch, true, stream);
     }
     if (dn <= 0 || dv <= 0) return NTK_E_SHAPE;
     AttnArgs a{};
@@ -599,7 +691,35 @@ int ntk_latent_fold_query_prepare(float* qf, const float* q, int ldq, const void
                                   int ldkv, const float* norm_w, float eps, int pos0, void* stream) {
     if (!cache || !kv || !norm_w) return NTK_E_NULL;
     if (row < R || ldkv < R || pos0 < 0) return NTK_E_SHAPE;
-    return fold_query(qf, q, ldq, w_uk, wdtype, T, H, dn, 0, R, FoldPrepare{cache, row, kv, ldkv, norm_w, eps, pos0}, stream);
+    return fold_query(qf, q, ldq, w_uk, wdtype, T, H, dn, 0, R, FoldPrepare{cache, row, kv, ldkv, norm_w, eps, pos0, nullptr, 1.0f, 0, 0}, stream);
+}
+
+int ntk_latent_fold_query_rotate(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int dr, int R, const ntk_rotary* rot, float* cache, int row,
+                                 const float* kv, int ldkv, const float* norm_w, float eps, int pos0, void* stream) {
+    if (!cache || !kv || !norm_w || !rot || (rot->dims > 0 && !rot->freq)) return NTK_E_NULL;
+    if (dr < 0 || rot->dims < 0 || (rot->dims & 1) || rot->dims > dr || row < R + dr || ldkv < R + dr || pos0 < 0) return NTK_E_SHAPE;
+    if (rot->layout != NTK_ROT_NEIGHBOURS && rot->layout != NTK_ROT_HALVES) return NTK_E_SHAPE;
+    return fold_query(qf, q, ldq, w_uk, wdtype, T, H, dn, dr, R, FoldPrepare{cache, row, kv, ldkv, norm_w, eps, pos0, rot->freq, rot->mag, rot->dims, rot->layout == NTK_ROT_HALVES ? 1 : 0}, stream);
+}
+
+int ntk_latent_attention_unfold(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,
+                                int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale, float* scratch, void* stream) {
+    if (!out || !w_uv || !lat || !qf || !cache || !scratch) return NTK_E_NULL;
+    if (wdtype != NTK_DT_BF16 && wdtype != NTK_DT_F32) return NTK_E_DTYPE;
+    if (T < 0 || H <= 0 || dv <= 0 || kv_rank <= 0 || rot_dim < 0 || pos0 < 0 || row < kv_rank + rot_dim) return NTK_E_SHAPE;
+    if (T == 0) return NTK_OK;
+    SharedArgs sa{};
+    const int ldq = H * (kv_rank + rot_dim);
+    const bool join = kv_rank % 8 == 0 && kv_rank <= 512 && T * shared_splits(shared_keys(pos0, T, window)) <= kJoinStates && !(((uintptr_t)w_uv | (uintptr_t)scratch) & 15);
+    const int st = launch_shared(sa, lat, H * kv_rank, qf, ldq, cache, row, kv_rank, rot_dim, H, pos0, T, window, scale, scratch, !join, stream);
+    if (st != NTK_OK) return st;
+    if (!join) return ntk_latent_unfold_value_ex(out, ldo, lat, w_uv, wdtype, gate, ldg, head_gate, T, H, dv, kv_rank, stream);
+    const dim3 grid((dv + 15) / 16, H, T);
+    if (wdtype == NTK_DT_BF16)
+        hipLaunchKernelGGL(latent_join_unfold_kernel<uint16_t>, grid, dim3(256), 0, resolve_stream(stream), out, ldo, (const float*)scratch, sa.splits, (const uint16_t*)w_uv, gate, ldg, H, dv, kv_rank, head_gate);
+    else
+        hipLaunchKernelGGL(latent_join_unfold_kernel<float>, grid, dim3(256), 0, resolve_stream(stream), out, ldo, (const float*)scratch, sa.splits, (const float*)w_uv, gate, ldg, H, dv, kv_rank, head_gate);
+    return last_launch_status();
 }
 
 int ntk_latent_unfold_value(float* out, int ldo, const float* lat, const void* w_uv, int wdtype, const float* gate, int ldg, int T, int H, int dv, int R,

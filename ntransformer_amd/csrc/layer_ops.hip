@@ -23,6 +23,22 @@ __global__ __launch_bounds__(256) void embed_dense_kernel(float* out, const TT* 
     }
 }
 
+// ... four entries a thread (width % 4 == 0, aligned); tokens NULL: one token, given with the launch.  us, one row of 2048 / 1024 rows: 5.7 / 8.1 a workgroup a row above, 2.5 / 3.9 so
+template <typename TT>
+__global__ __launch_bounds__(256) void embed_dense_wide_kernel(float* out, const TT* table, const int* tokens, int token, int vocab, int width, float scale) {
+    const int t = blockIdx.y, i = 4 * ((int)blockIdx.x * 256 + (int)threadIdx.x), tok = tokens ? tokens[t] : token;
+    if (i >= width) return;
+    float4 v{0.0f, 0.0f, 0.0f, 0.0f};
+    if (tok >= 0 && tok < vocab) {
+        const TT* row = table + (long long)tok * width + i;
+        if constexpr (sizeof(TT) == 2) {
+            const uint2 b = *reinterpret_cast<const uint2*>(row);
+            v = float4{__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xFFFF0000u), __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xFFFF0000u)};
+        } else v = *reinterpret_cast<const float4*>(row);
+    }
+    *reinterpret_cast<float4*>(out + (long long)t * width + i) = float4{v.x * scale, v.y * scale, v.z * scale, v.w * scale};
+}
+
 template <typename TT> __device__ __forceinline__ float table_value(const TT* row, int i) {
     if constexpr (sizeof(TT) == 2) return __uint_as_float((uint32_t)row[i] << 16); else return row[i];
 }
@@ -360,10 +376,25 @@ int ntk_embed_dense(float* out, const void* table, int tdtype, const int* tokens
     return ntk_embed_dense_scaled(out, table, tdtype, tokens, T, vocab, width, 1.0f, stream);
 }
 
+static bool embed_wide(float* out, const void* table, int tdtype, const int* tokens, int token, int T, int vocab, int width, float scale, void* stream) {
+    if (width % 4 || (((uintptr_t)out | (uintptr_t)table) & 15) || T > 65535) return false;
+    const dim3 grid((width / 4 + 255) / 256, T);
+    if (tdtype == NTK_DT_BF16) hipLaunchKernelGGL(embed_dense_wide_kernel<uint16_t>, grid, dim3(256), 0, resolve_stream(stream), out, (const uint16_t*)table, tokens, token, vocab, width, scale);
+    else hipLaunchKernelGGL(embed_dense_wide_kernel<float>, grid, dim3(256), 0, resolve_stream(stream), out, (const float*)table, tokens, token, vocab, width, scale);
+    return true;
+}
+int ntk_embed_token(float* out, const void* table, int tdtype, int token, int vocab, int width, float scale, void* stream) {
+    if (!out || !table) return NTK_E_NULL;
+    if (tdtype != NTK_DT_BF16 && tdtype != NTK_DT_F32) return NTK_E_DTYPE;
+    if (vocab <= 0 || width <= 0) return NTK_E_SHAPE;
+    return embed_wide(out, table, tdtype, nullptr, token, 1, vocab, width, scale, stream) ? last_launch_status() : NTK_E_ALIGN;
+}
+
 int ntk_embed_dense_scaled(float* out, const void* table, int tdtype, const int* tokens, int T, int vocab, int width, float scale, void* stream) {
     if (!out || !table || !tokens) return NTK_E_NULL;
     if (T < 0 || vocab <= 0 || width <= 0) return NTK_E_SHAPE;
     if (T == 0) return NTK_OK;
+    if ((tdtype == NTK_DT_BF16 || tdtype == NTK_DT_F32) && embed_wide(out, table, tdtype, tokens, 0, T, vocab, width, scale, stream)) return last_launch_status();
     if (tdtype == NTK_DT_BF16) hipLaunchKernelGGL(embed_dense_kernel<uint16_t>, dim3(T), dim3(256), 0, resolve_stream(stream), out, (const uint16_t*)table, tokens, vocab, width, scale);
     else if (tdtype == NTK_DT_F32) hipLaunchKernelGGL(embed_dense_kernel<float>, dim3(T), dim3(256), 0, resolve_stream(stream), out, (const float*)table, tokens, vocab, width, scale);
     else return NTK_E_DTYPE;
