@@ -1284,7 +1284,8 @@ static bool in_two_launches(const MoeFeedForward& M, int T, int W) {
 
 // router, grouping, the experts' products; then either straight into the stream together with the mixer's output (parallel form) or as a sum of its own
 // in ff_ (sequential form: it is normed before it joins the stream)
-int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool into_stream, const void* h16) {
+// (norm_w: h is the norm of the stream by this weight, to be formed in the router's launch)
+int LayerStackModel::run_moe(const StackLayer& L, float* h, int T, bool into_stream, const void* h16, const float* norm_w) {
     const MoeFeedForward& M = L.mlp;
     const int W = info_.width, choices = M.experts + M.identity;
     float* sgate = M.has_shared && M.shared_gate ? sg_ : nullptr;
@@ -1309,7 +1310,8 @@ int LayerStackModel::run_moe(const StackLayer& L, const float* h, int T, bool in
         route.add_y = owed_.y; route.ld_add = W; route.add_w = owed_.nb.w; route.add_eps = eps_;
         owed_.y = nullptr;
     }
-    LS_TRY(ntk_moe_route_ex(ids_, wts_, sgate, h, W, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
+    if (norm_w) LS_TRY(ntk_moe_norm_route(ids_, wts_, sgate, h, W, x_, W, norm_w, eps_, 1.0f, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
+    else LS_TRY(ntk_moe_route_ex(ids_, wts_, sgate, h, W, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
     const bool few = !M.routed.plain && T <= ntk_dense_few_rows() && mid <= NTK_MOE_FEW_MID && W <= NTK_MOE_FEW_MID && !(into_stream && M.identity);
     if (few && in_two_launches(M, T, W)) {
         ntk_moe_few_desc d{};
@@ -1633,13 +1635,11 @@ int LayerStackModel::parallel_layer(const Run& run, const StackLayer& L, int slo
         }
         if (st == NTK_E_ALIGN) st = ntk_rmsnorm_offset(h1_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
         LS_TRY(st);
-    } else if (L.has_mlp) {   // decoding: the mixer's norm runs inside its first product (run_mixer); the feed-forward's input has three readers
-        LS_TRY(ntk_rmsnorm_offset(h2_, L.norm2.w, nullptr, nullptr, W, x_, W, T, W, eps_, 1.0f, stream_));
-    }
+    }   // (decoding: the mixer's norm runs inside its first product (run_mixer), the feed-forward's in its router's launch)
     float* cache = run.cache + (size_t)slot * opt_.max_context * L.mix.row();
     const bool few = T <= ntk_dense_few_rows();
     LS_TRY(run_mixer(L, cache, T, pos0, few ? x_ : h1_, few, h16));
-    if (L.has_mlp) return run_moe(L, h2_, T, true, g16);
+    if (L.has_mlp) return run_moe(L, h2_, T, true, g16, few ? L.norm2.w : nullptr);
     return ntk_residual_add(x_, mix_, nullptr, T * W, stream_);
 }
 

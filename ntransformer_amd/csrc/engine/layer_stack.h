@@ -337,7 +337,7 @@ private:
     int window_keys_values(const WindowMixer& m, float* cache, int T, int pos0);
     int dense_parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int run_lightning(const StackLayer& L, float* state, int T, int pos0);
-    int run_moe(const StackLayer& L, const float* h, int T, bool into_stream, const void* h16 = nullptr);
+    int run_moe(const StackLayer& L, float* h, int T, bool into_stream, const void* h16 = nullptr, const float* norm_w = nullptr);
     int run_dense_ff(const StackLayer& L, int T);
     int run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
                     int full_x, const void* h16 = nullptr, const float* norm_w = nullptr);   // norm_w (few rows): the rows are normed inside the first product

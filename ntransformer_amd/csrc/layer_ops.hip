@@ -23,7 +23,7 @@ __global__ __launch_bounds__(256) void embed_dense_kernel(float* out, const TT* 
     }
 }
 
-// ... four entries a thread (width % 4 == 0, aligned); tokens NULL: one token, given with the launch.  us, one row of 2048 / 1024 rows: 5.7 / 8.1 a workgroup a row above, 2.5 / 3.9 so
+// ... four entries a thread (width % 4 == 0, aligned); tokens NULL: one token, given with the launch.  us, one row of 2048 / 1024 rows: 5.7 / 8.1 a workgroup a row above, 2.5 / 4.5 so
 template <typename TT>
 __global__ __launch_bounds__(256) void embed_dense_wide_kernel(float* out, const TT* table, const int* tokens, int token, int vocab, int width, float scale) {
     const int t = blockIdx.y, i = 4 * ((int)blockIdx.x * 256 + (int)threadIdx.x), tok = tokens ? tokens[t] : token;

@@ -15,7 +15,9 @@ constexpr int kMaxExperts = 256;
 // one workgroup per token: its 16 waves share the experts (wave w: experts w, w + 16, ...), a lane requests its whole part of the router row before
 // it uses any of it; thread 0 then does the softmax and the `top` picks over the scores in LDS
 constexpr int kRouteThreads = 1024;
-struct RouteForm { int score, groups, keep, group_top, renorm; float scale; const float* correction; const float* add_y; int ld_add; const float* add_w; float add_eps; };
+struct RouteForm { int score, groups, keep, group_top, renorm; float scale; const float* correction; const float* add_y; int ld_add; const float* add_w; float add_eps;
+    const float* src; int ldsrc; const float* norm_w; float norm_eps, norm_offset;     // (norm_w: the token's row is the RMS norm of a row of src, formed in the launch and left in h; NULL: h holds it)
+};
 
 // the largest of a wave's 4 x 64 values (lane l holds entries l, l + 64, l + 128, l + 192); equal values: the lower index
 __device__ __forceinline__ void wave_argmax4(const float (&v)[4], int lane, float& bv, int& bi) {
@@ -119,7 +121,18 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(int* ids, floa
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = kRouteThreads / 64;
     const long long t = blockIdx.x;
     float* x = h + t * ldh;
-    if (f.add_y) {     // (uniform) what the row is still owed joins it: y / rms(y) * w; a thread re-reads its own entries
+    if (f.norm_w) {    // (uniform).  us, one token of 2048 among 32 experts: 6.4 the norm in a launch of its own and 7.5 the choice, 9.1 so (weights requested ahead of the row: 10.9)
+        __shared__ float red[16];
+        const float* y = f.src + t * f.ldsrc;
+        float ss = 0.0f;
+        for (int k = threadIdx.x; k < n; k += kRouteThreads) { const float v = y[k]; xs[k] = v; ss = fmaf(v, v, ss); }
+        const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)n + f.norm_eps);
+        for (int k = threadIdx.x; k < n; k += kRouteThreads) {
+            const float v = xs[k] * inv * (f.norm_offset + f.norm_w[k]);
+            xs[k] = v;
+            x[k] = v;
+        }
+    } else if (f.add_y) {     // (uniform) what the row is still owed joins it: y / rms(y) * w; a thread re-reads its own entries
         __shared__ float red[16];
         const float* y = f.add_y + t * f.ld_add;
         float ss = 0.0f;
@@ -322,7 +335,7 @@ static int route_form(const ntk_route_desc* r, int E, int top, RouteForm* f) {
     if (r->score != 0 && r->score != 1) return NTK_E_SHAPE;
     const int groups = r->groups > 1 ? r->groups : 1;
     if (groups > 1 && (E % groups || r->keep < 1 || r->keep > groups || r->group_top < 1 || r->group_top > 8 || (long long)r->keep * (E / groups) < top)) return NTK_E_SHAPE;
-    *f = RouteForm{r->score, groups, r->keep, r->group_top, r->renorm, r->scale, r->correction, r->add_y, r->ld_add, r->add_w, r->add_eps};
+    *f = RouteForm{r->score, groups, r->keep, r->group_top, r->renorm, r->scale, r->correction, r->add_y, r->ld_add, r->add_w, r->add_eps, nullptr, 0, nullptr, 0.0f, 0.0f};
     return NTK_OK;
 }
 
@@ -336,6 +349,19 @@ int ntk_moe_route_ex(int* ids, float* wts, float* sgate, const float* h, int ldh
     const int st = route_form(r, E, top, &f);
     if (st != NTK_OK || T == 0) return st;
     hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(kRouteThreads), (size_t)n * 4, resolve_stream(stream), ids, wts, sgate, (float*)h, ldh, w_router, shared_gate_w, n, E, top, f);
+    return last_launch_status();
+}
+
+int ntk_moe_norm_route(int* ids, float* wts, float* sgate, float* h, int ldh, const float* x, int ldx, const float* norm_w, float norm_eps, float norm_offset, const float* w_router,
+                       const float* shared_gate_w, int T, int n, int E, int top, const ntk_route_desc* r, void* stream) {
+    if (!ids || !wts || !h || !x || !norm_w || !w_router || !r) return NTK_E_NULL;
+    if (T < 0 || n <= 0 || E <= 0 || E > kMaxExperts || top <= 0 || top > E || ldh < n || ldx < n || r->add_y || h == x) return NTK_E_SHAPE;
+    if ((size_t)n * 4 > 128 * 1024) return NTK_E_SHAPE;
+    RouteForm f;
+    const int st = route_form(r, E, top, &f);
+    if (st != NTK_OK || T == 0) return st;
+    f.src = x; f.ldsrc = ldx; f.norm_w = norm_w; f.norm_eps = norm_eps; f.norm_offset = norm_offset;
+    hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(kRouteThreads), (size_t)n * 4, resolve_stream(stream), ids, wts, sgate, h, ldh, w_router, shared_gate_w, n, E, top, f);
     return last_launch_status();
 }
 

@@ -113,3 +113,25 @@ def test_capped_products(dtype, T, N, K):
     assert np.array_equal(*out) and np.abs(out[0]).max() <= 1.5
     d.act = 1
     assert L.ntk_dense_capped(C.byref(d), 1.5, None) != 0
+
+
+@pytest.mark.parametrize("T,n,E,top", [(1, 2048, 32, 6), (8, 192, 6, 2), (3, 2052, 33, 4), (2, 70, 5, 5), (1, 5000, 200, 8)])
+def test_router_of_a_row_normed_in_its_launch(T, n, E, top):
+    L, g = Lr._bind(), np.random.default_rng(n)
+    L.ntk_moe_norm_route.argtypes = [VP, VP, VP, VP, I, VP, I, VP, F, F, VP, VP] + [I] * 4 + [C.POINTER(Lr.RouteDesc), VP]
+    x = DB.from_numpy((3 * g.standard_normal((T, n))).astype(np.float32))
+    nw, wr, ws = (DB.from_numpy((0.2 * g.standard_normal(s)).astype(np.float32)) for s in (n, (E, n), n))
+    r = Lr.RouteDesc()
+    r.score, r.groups, r.renorm, r.scale = 0, 1, 1, 1.0
+    out = []
+    for one in (0, 1):
+        h, ids, wts, sg = DB.zeros(T * n * 4), DB.zeros(T * top * 4), DB.zeros(T * top * 4), DB.zeros(T * 4)
+        if one:
+            Lr.check(L.ntk_moe_norm_route(ids.ptr, wts.ptr, sg.ptr, h.ptr, n, x.ptr, n, nw.ptr, 1e-5, 1.0, wr.ptr, ws.ptr, T, n, E, top, C.byref(r), None), "norm_route")
+        else:
+            Lr.check(L.ntk_rmsnorm_offset(h.ptr, nw.ptr, None, None, n, x.ptr, n, T, n, 1e-5, 1.0, None), "norm")
+            Lr.check(L.ntk_moe_route_ex(ids.ptr, wts.ptr, sg.ptr, h.ptr, n, wr.ptr, ws.ptr, T, n, E, top, C.byref(r), None), "route")
+        out.append((ids.numpy(np.int32)[:T * top], h.numpy(np.float32)[:T * n], wts.numpy(np.float32)[:T * top], sg.numpy(np.float32)[:T]))
+    assert np.array_equal(out[0][0], out[1][0])
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert np.isfinite(b).all() and np.abs(a - b).max() <= 2e-5 * np.abs(a).max()      # (logits of up to 5000 products behind a norm whose sum has another order)
