@@ -86,11 +86,6 @@ void*  nt_hip_malloc_host(size_t size);              /* pinned */
 void   nt_hip_free_host(void* p);
 int    ntk_memcpy_h2d_async(void* dst, const void* src, size_t size, void* stream);   /* device.cu:136-144 */
 int    ntk_memcpy_d2h_async(void* dst, const void* src, size_t size, void* stream);
-/* Words of the host into device memory as arguments of a launch (a copy of a few bytes is a launch that fetches them over the bus, and its source has to outlive it): values[0 .. na) to a, the
- * nb behind them to b (NULL with nb 0).  na + nb <= 32 (NTK_E_SHAPE). */
-int    ntk_store_words(int* a, int na, int* b, int nb, const int* values, void* stream);
-/* size bytes (a multiple of 4, both pointers 4-byte aligned) into pinned host memory (nt_hip_malloc_host) by a launch in the stream's order: there once the stream has been waited for */
-int    ntk_copy_out(void* pinned, const void* src, size_t size, void* stream);
 /* the reference's names, kept as aliases so its host code / tests link unchanged (device.h:79-88) */
 void*  nt_cuda_malloc(size_t size);
 void   nt_cuda_free(void* p);

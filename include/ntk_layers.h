@@ -452,6 +452,12 @@ int ntk_moe_sum_ex(float* out, const float* d, const int* where, const int* ids,
 int ntk_moe_combine(float* x, const float* mix, const float* d, const int* where, const float* wts, const float* shared, const float* sgate, int T, int top,
                     int n, void* stream);
 
+/* Words of the host into device memory as arguments of a launch (a copy of a few bytes is a launch that fetches them over the bus, and its source has to outlive it): values[0 .. na) to a, the
+ * nb behind them to b (NULL with nb 0).  na + nb <= 32 (NTK_E_SHAPE). */
+int    ntk_store_words(int* a, int na, int* b, int nb, const int* values, void* stream);
+/* size bytes (a multiple of 4, both pointers 4-byte aligned) into pinned host memory (nt_hip_malloc_host) by a launch in the stream's order: there once the stream has been waited for */
+int    ntk_copy_out(void* pinned, const void* src, size_t size, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,6 +1,7 @@
 // engine/model.cpp -- see model.h
 #include "model.h"
 #include "../../../include/ntk_engine.h"
+#include "../../../include/ntk_layers.h"
 #ifdef NTK_EXPERIMENTS
 #include "ntk_experiments.h"
 #endif

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
         } else {
             sc = scale[t];
         }
-        if (g == 0 && step % (GB_GROUP / 32) == 0 && t < GB_SHORT && blockIdx.y == 0)   // (one scale a token here: every group's; 1 / s of a power of two by its exponent)
+        if (g == 0 && step % (GB_GROUP / 32) == 0 && T <= GB_SHORT && blockIdx.y == 0)   // (a short prompt; one scale a token here: every group's; 1 / s of a power of two by its exponent)
             group_inv[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((254u << 23) - __float_as_uint(sc));
     }
     float p1[8], p2[8];
@@ -295,7 +295,7 @@ __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, i
             const int pos = ((tb * 2 + ((step >> 2) & 1)) * 64 + j * 4 + (step & 3));
             rec[pos] = h1;
             rec[4 * 128 + pos] = h2;
-            if (t < GB_SHORT && step % (GB_GROUP / 32) == 0 && step * 32 < in)
+            if (gridDim.x <= GB_SHORT && step % (GB_GROUP / 32) == 0 && step * 32 < in)   // (a short prompt; a workgroup a token)
                 reinterpret_cast<float*>(ws + ws_group_offset(in))[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((uint32_t)(254 - es) << 23);
         }
     }

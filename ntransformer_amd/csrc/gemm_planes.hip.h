@@ -31,11 +31,10 @@ static __host__ __device__ size_t ws_chunk_bytes(int in) {
     return ((size_t)(in / 32 + 1) * GB_STEP_BYTES + (size_t)((in / 32 + 15) / 8) * GB_MIN_UNIT_BYTES + 255) / 256 * 256;
 }
 constexpr size_t GB_SCALE_BYTES = 2 * GB_MAX_CHUNKS * GB_TOK * sizeof(float);   // the launch's 1 / s and s
-// ... and behind those, for the short prompts' form: [GB_GROUP columns][GB_SHORT tokens] 1 / s, then [512 columns][GB_SHORT tokens] sums of squares (short_split below)
+// ... and, in the second chunk's area (a short prompt has one chunk), for the short prompts' form: [GB_GROUP columns][GB_SHORT tokens] 1 / s, then [512 columns][GB_SHORT tokens] sums of squares (short_split below)
 static __host__ __device__ size_t ws_group_floats(int in) { return (size_t)((in + GB_GROUP - 1) / GB_GROUP) * GB_SHORT; }
-static __host__ __device__ size_t ws_group_bytes(int in) { return (ws_group_floats(in) + (size_t)((in + 511) / 512) * GB_SHORT) * sizeof(float); }
-static __host__ __device__ size_t ws_group_offset(int in) { return (size_t)GB_MAX_CHUNKS * ws_chunk_bytes(in) + GB_SCALE_BYTES; }
-static __host__ __device__ size_t ws_part_offset(int in) { return ws_group_offset(in) + (ws_group_bytes(in) + 255) / 256 * 256; }
+static __host__ __device__ size_t ws_group_offset(int in) { return ws_chunk_bytes(in); }   // (fits: a 128th of the chunk's records at most)
+static __host__ __device__ size_t ws_part_offset(int in) { return (size_t)GB_MAX_CHUNKS * ws_chunk_bytes(in) + GB_SCALE_BYTES; }
 // Half a wave splits a token's group of columns: lane l of its 32 holds in x[8] the values of columns 32 step + 4 g + {0 .. 3, 16 .. 19}, step = the group's first + l / 4, g = l % 4; steps
 // past the row hold zeros.  t: the token, < 0: nothing is written.
 __device__ __forceinline__ void short_split(float (&x)[8], int step, int g, int t, int in, uint8_t* __restrict__ ws) {
