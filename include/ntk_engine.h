@@ -215,6 +215,16 @@ int ntk_reduce_rmsnorm_prepare_x(float* hidden, const ntk_gemm_partials* partial
 int ntk_silu_mul_prepare_x(float* output, const float* gate, const float* up, int n_tokens, int width, void* workspace, void* stream);
 int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials, void* workspace, void* stream);
 
+/* ... and of a prompt of more than 64 tokens (up to 1024, one pass): the planes from four tokens a workgroup.  ntk_rows_prepare_takes: 1 where the three take such a prompt (norm: the second), else 0
+ *   ntk_rows_prepare_x            X as it lies
+ *   ntk_rows_norm_prepare_x       hidden += the deferred projection (partials; NULL: hidden as it lies), planes of its RMSNorm; x_out (may be NULL): the normalised rows themselves
+ *   ntk_rows_silu_mul_prepare_x   planes of silu(gate) * up of a gate | up launch, deferred or not; output (may be NULL, may be the gate's y): the rows themselves
+ * Workspace and alignments as above; results as the launches above give them, up to the order of a norm's sum. */
+int ntk_rows_prepare_takes(int n_tokens, int width, int norm);
+int ntk_rows_prepare_x(const float* X, int n_tokens, int width, void* workspace, void* stream);
+int ntk_rows_norm_prepare_x(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int width, float eps, float* x_out, void* workspace, void* stream);
+int ntk_rows_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials, void* workspace, void* stream);
+
 /* Prompts of at most 32 tokens, whose projections keep a K slice's planes in LDS: their producers scale X per token and 256 columns, so that they need no whole row in one workgroup.
  *   ntk_gemm_short_takes          1 where ntk_gemm_short takes matrices of these rows and format (raw or repacked) over one X of in_features, else 0
  *   ntk_short_prepare_x           planes of X as it lies

@@ -7,6 +7,7 @@
 #endif
 
 #include <hip/hip_runtime.h>
+#include <initializer_list>
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -839,13 +840,24 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
     // (up to 64 tokens: a producer that owns a whole token per workgroup writes its planes in 16-byte pieces a kilobyte apart -- at 1024 tokens the pass
     // measured 5 % SLOWER than with the GEMM's own pre-pass, 8B Q8_0 28 010 -> 26 460 tok/s; at 16 - 64 tokens it is 2 - 5 % faster)
     const bool fuse_split = with_max && prefill_fused_split_ && gemm_ws2_ != nullptr && T <= 64;
+    // (... beyond: four tokens a workgroup, rows_split_kernel, where its registers hold the row; wider rows leave their maxima)
+    const bool rows_split = with_max && prefill_fused_split_ && gemm_ws2_ != nullptr && T > 64;
+    auto splits_rows = [&](size_t width, bool norm) { return fuse_split || (rows_split && ntk_rows_prepare_takes(T, (int)width, norm ? 1 : 0)); };
     auto f16_ok = [&](const DevTensor& w) {   // the formats and shapes ntk_gemm_quant_f16 takes
         const bool kq = w.dtype == NTK_DT_Q4_0 || w.dtype == NTK_DT_Q4_K || w.dtype == NTK_DT_Q5_K || w.dtype == NTK_DT_Q6_K;
         return (w.dtype == NTK_DT_Q8_0 || kq) && w.in_f % (kq ? 256 : 128) == 0 && w.out_f % 16 == 0 && (w.ptr || w.rp);
     };
+    // nothing but planes is read of X where every matrix that reads it goes through that GEMM, whatever it would refuse looked at ahead: such rows are not written at all
+    auto planes_only = [&](std::initializer_list<const DevTensor*> ws, size_t width) {
+        if (!rows_split) return false;
+        for (const DevTensor* w : ws)
+            if (!f16_ok(*w) || (size_t)w->in_f != width || w->nbytes > 0xE0000000u || (reinterpret_cast<uintptr_t>(w->ptr ? w->ptr : w->rp) & 15)) return false;
+        return true;
+    };
     auto prepare_x = [&](const float* X, const DevTensor& w) {   // X as it lies (the attention output): row maximum + split in one launch
-        if (!fuse_split || !f16_ok(w) || X == planes_of) return;
-        if (ntk_gemm_prepare_x(X, T, (int)w.in_f, flip_ws(), s) == NTK_OK) planes_of = X;
+        if (!splits_rows(w.in_f, false) || !f16_ok(w) || X == planes_of) return;
+        void* ws = flip_ws();
+        if ((fuse_split ? ntk_gemm_prepare_x(X, T, (int)w.in_f, ws, s) : ntk_rows_prepare_x(X, T, (int)w.in_f, ws, s)) == NTK_OK) planes_of = X;
         else planes_of = nullptr;
     };
     // One resident copy (round 6): a K-quant matrix whose GGUF bytes were freed after the load-time repack is read by the FP16 GEMM FROM THE REPACK
@@ -979,9 +991,11 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         max_a = written ? rm_a : nullptr;
         if (zero_b) b_clear = written && rm_b;
     };
-    auto norm = [&](const DevTensor& nw, bool zero_b, const DevTensor& next_w) {
-        if (fuse_split && f16_ok(next_w) && (int)next_w.in_f == H) {
-            ok(ntk_rmsnorm_prepare_x(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, flip_ws(), s));
+    auto norm = [&](const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only) {     // only: planes_only of the matrices that read it
+        if (splits_rows(H, true) && f16_ok(next_w) && (int)next_w.in_f == H) {
+            void* ws = flip_ws();
+            ok(fuse_split ? ntk_rmsnorm_prepare_x(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, ws, s)
+                          : ntk_rows_norm_prepare_x(hidden_, nullptr, (const float*)nw.ptr, T, H, cfg_.norm_eps, only ? nullptr : residual_, ws, s));
             planes_ready = residual_;
             left_max(false, zero_b);
             return;
@@ -992,7 +1006,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
     };
     // hidden += W . X followed by the NEXT RMSNorm (nw; into residual_, with the token maxima) as one consumer launch of the projection's K splits
     // (ntk_gemm_quant_f16 with `partials` + ntk_reduce_rmsnorm_rowmax); false = not this shape / format: the caller runs project_add + norm
-    auto project_add_norm = [&](const DevTensor& w, const float* X, const float* rm, const DevTensor& nw, bool zero_b, const DevTensor& next_w) -> bool {
+    auto project_add_norm = [&](const DevTensor& w, const float* X, const float* rm, const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only) -> bool {
         if (!with_max || tp_world_ > 1 || !is_quant(w.dtype) || (size_t)w.out_f != (size_t)H) return false;
         ntk_gemm_partials pt;
         int st = NTK_E_DTYPE;
@@ -1010,8 +1024,10 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         }
         if (st == NTK_E_DTYPE || st == NTK_E_SHAPE || st == NTK_E_ALIGN) return false;   // (nothing was launched)
         planes_of = nullptr;
-        if (st == NTK_OK && fuse_split && f16_ok(next_w) && (int)next_w.in_f == H) {   // (the partial sums lie in cur_ws: the planes go to the other one)
-            st = ntk_reduce_rmsnorm_prepare_x(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, flip_ws(), s);
+        if (st == NTK_OK && splits_rows(H, true) && f16_ok(next_w) && (int)next_w.in_f == H) {   // (the partial sums lie in cur_ws: the planes go to the other one)
+            void* ws = flip_ws();
+            st = fuse_split ? ntk_reduce_rmsnorm_prepare_x(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, ws, s)
+                            : ntk_rows_norm_prepare_x(hidden_, &pt, (const float*)nw.ptr, T, H, cfg_.norm_eps, only ? nullptr : residual_, ws, s);
             planes_ready = residual_;
             left_max(false, zero_b);
         } else
@@ -1024,7 +1040,8 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         const LayerWeights& L = layers_[i];
         uint16_t* kc = k_cache_ + (size_t)i * kv_layer;
         uint16_t* vc = v_cache_ + (size_t)i * kv_layer;
-        if (!normed_ahead) norm(L.attn_norm, true, L.wq);
+        auto only_qkv = [&](const LayerWeights& l) { return planes_only({&l.wq, &l.wk, &l.wv}, H); };
+        if (!normed_ahead) norm(L.attn_norm, true, L.wq, only_qkv(L));
         normed_ahead = false;
         planes_of = planes_ready;   // residual_ has new contents (split already by the launch that wrote them, or not)
         planes_ready = nullptr;
@@ -1049,9 +1066,10 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         if (keys_last && i + 1 == last_layer) break;
         if (T == 1) ok(ntk_attention_decode(attn_out, q_buf, kc, vc, start_pos + T, nh, nkv, hd, cfg_.max_seq_len, scale, s));
         else ok(ntk_attention_prefill(attn_out, q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
-        if (!project_add_norm(L.wo, attn_out, nullptr, L.ffn_norm, false, L.w_gate)) {
+        const bool only_unit = planes_only({&L.w_gate, &L.w_up}, H);
+        if (!project_add_norm(L.wo, attn_out, nullptr, L.ffn_norm, false, L.w_gate, only_unit)) {
             project_add(L.wo, attn_out, qd, nullptr);
-            norm(L.ffn_norm, false, L.w_gate);
+            norm(L.ffn_norm, false, L.w_gate, only_unit);
         }
         planes_of = planes_ready;
         planes_ready = nullptr;
@@ -1068,8 +1086,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             ntk_gemm_partials pt;
             int st = gemm_f16(segs, 2, residual_, (int)L.w_gate.in_f, nullptr, residual_ == planes_of ? 1 : 0, max_a, &pt, both_rp);
             if (st != NTK_E_DTYPE && st != NTK_E_SHAPE && st != NTK_E_ALIGN) {   // (those three: nothing was launched)
-                if (st == NTK_OK && fuse_split && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I) {
-                    st = ntk_reduce_silu_mul_prepare_x(gate_buf, &pt, flip_ws(), s);
+                if (st == NTK_OK && splits_rows(I, false) && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I) {
+                    void* ws = flip_ws();
+                    st = fuse_split ? ntk_reduce_silu_mul_prepare_x(gate_buf, &pt, ws, s) : ntk_rows_silu_mul_prepare_x(planes_only({&L.w_down}, I) ? nullptr : gate_buf, &pt, ws, s);
                     planes_ready = gate_buf;
                 } else
                 if (st == NTK_OK) st = ntk_reduce_silu_mul_rowmax(gate_buf, &pt, rm_b, s), max_b = b_clear ? rm_b : nullptr;
@@ -1087,8 +1106,11 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             const DevTensor* const ws[2] = {&L.w_gate, &L.w_up};
             project_many(ys, ws, 2, residual_, max_a);
             int st_silu = NTK_E_SHAPE;   // (in place: exactly one of these launches runs)
-            if (fuse_split && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I && tp_world_ == 1) {
-                st_silu = ntk_silu_mul_prepare_x(gate_buf, gate_buf, up_buf, T, I, flip_ws(), s);
+            if (splits_rows(I, false) && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I && tp_world_ == 1) {
+                ntk_gemm_partials pt{};
+                pt.nseg = 2; pt.n_tokens = T; pt.nsplit = 1; pt.y[0] = gate_buf; pt.y[1] = up_buf; pt.rows[0] = pt.rows[1] = I;
+                void* ws = flip_ws();
+                st_silu = fuse_split ? ntk_silu_mul_prepare_x(gate_buf, gate_buf, up_buf, T, I, ws, s) : ntk_rows_silu_mul_prepare_x(planes_only({&L.w_down}, I) ? nullptr : gate_buf, &pt, ws, s);
                 if (st_silu == NTK_OK) planes_ready = gate_buf;
             } else if (with_max && rm_b) {
                 st_silu = ntk_silu_mul_rowmax(gate_buf, gate_buf, up_buf, T, I, rm_b, s);
@@ -1100,7 +1122,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         planes_of = planes_ready;
         planes_ready = nullptr;
         // down projection + residual, and the NEXT layer's first RMSNorm in the same consumer launch when there is a next layer in this pass
-        if (i + 1 < last_layer && project_add_norm(L.w_down, gate_buf, max_b, layers_[i + 1].attn_norm, true, layers_[i + 1].wq)) normed_ahead = true;
+        if (i + 1 < last_layer && project_add_norm(L.w_down, gate_buf, max_b, layers_[i + 1].attn_norm, true, layers_[i + 1].wq, only_qkv(layers_[i + 1]))) normed_ahead = true;
         else project_add(L.w_down, gate_buf, I, max_b);
         if (rc != NTK_OK) break;
     }

@@ -37,6 +37,7 @@
 #include "gemm_planes.hip.h"
 #include <algorithm>
 #include <cstdlib>
+#include <initializer_list>
 #include <type_traits>
 
 namespace ntk {
@@ -417,6 +418,190 @@ __global__ __launch_bounds__(1024) void rmsnorm_split_kernel(float* __restrict__
     const float m = block_max(__uint_as_float(mb <= 0x7F800000u ? mb : 0x7F800000u), red);
     __syncthreads();   // (workgroup-scope: every thread's stores to `out` are visible to the threads that split them)
     split_row(out, __float_as_uint(m), t, hidden, ws);
+}
+
+// ---- the producers of a LONG prompt's planes: four tokens a workgroup, planes only -------------------------------------------------------------------------------------
+// What bounds them is memory: a row passes through HBM or the Infinity Cache as often as launches touch it.  A launch that leaves the row and its largest |x| and a second that splits
+// it write and read the row once more; a workgroup a token (above) writes its planes in 16-byte pieces, of which four tokens share every 64 bytes.  Four tokens a workgroup of 16 waves
+// write whole 64 bytes, the row stays in registers between its sums, its norm and its split, and the 16 tokens of an operand record go to one XCD (the map of blockIdx below), whose L2
+// joins their halves of a line.  Lane j + 4 g + 16 s of wave w: token j, columns 32 step + 4 g + {0 .. 3, 16 .. 19} of step 4 (16 it + w) + s -- a float4 of the row is a quarter of
+// 64 contiguous bytes, a 16-byte piece of the planes likewise.
+// us, 1003 tokens (a launch for the rows and their maxima + one for the split -> this one): 4096 columns as they lie 7.1 + 6.9 -> 9.4; a norm of 4096 behind two splits 17.9 + 7.6 ->
+// 17.5 (82 MB, 4.7 TB/s); silu(gate) * up of 14336 30.5 + 20.4 -> 30.9 (172 MB, 5.6 TB/s; 42.5 with the rows written beside their planes)
+constexpr int RS_TOK = 4, RS_STEPS = 64;   // tokens of a workgroup; steps of 32 columns of one turn of its 16 waves
+struct RowsSplitParams {
+    const float* a;        // LIES: X.  NORM: the projection's partial sums [nsplit][T][W] (nsplit 0: hidden as it lies).  SILU: the gate's
+    const float* b;        // SILU: the up projection's
+    float* hidden;         // NORM: += the sums
+    const float* weight;
+    float* out;            // the rows themselves, if anything but the planes is read (may be NULL)
+    int nsplit, T, W;
+    float eps;
+    uint8_t* ws;
+};
+enum { RS_LIES, RS_NORM, RS_SILU };
+template <int MODE, int NI>
+__global__ __launch_bounds__(1024) void rows_split_kernel(const RowsSplitParams p) {
+    __shared__ float sums[16][RS_TOK];
+    __shared__ uint32_t tops[16][RS_TOK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = lane & 3, g = (lane >> 2) & 3, s4 = lane >> 4;
+    const int bid = (int)blockIdx.x, grp = (bid >> 5) * 32 + (bid & 7) * 4 + ((bid >> 3) & 3);   // (blocks go to the eight XCDs in turn: four in a row of one XCD are one record's tokens)
+    const int t = grp * RS_TOK + j, tc = min(t, p.T - 1), W = p.W;
+    if (grp * RS_TOK >= (p.T + GB_TOK - 1) / GB_TOK * GB_TOK) return;
+    const size_t plane = (size_t)p.T * W, row = (size_t)tc * W;
+    float v[NI][8];
+    auto in_row = [&](int it) { return ((it * 16 + wave) * 4 + s4) * 32 < W; };
+    auto col = [&](int it) { return in_row(it) ? ((it * 16 + wave) * 4 + s4) * 32 + 4 * g : 0; };   // (a step past the row: column 0 again, dropped below)
+    auto get = [](float (&d)[8], const float* src) {
+        const float4 x = *reinterpret_cast<const float4*>(src), y = *reinterpret_cast<const float4*>(src + 16);
+        d[0] = x.x; d[1] = x.y; d[2] = x.z; d[3] = x.w; d[4] = y.x; d[5] = y.y; d[6] = y.z; d[7] = y.w;
+    };
+    auto put = [](float* dst, const float (&d)[8]) {
+        *reinterpret_cast<float4*>(dst) = float4{d[0], d[1], d[2], d[3]};
+        *reinterpret_cast<float4*>(dst + 16) = float4{d[4], d[5], d[6], d[7]};
+    };
+    if constexpr (MODE == RS_NORM) {
+        if (p.nsplit == 0) {
+#pragma unroll
+            for (int it = 0; it < NI; ++it) get(v[it], p.hidden + row + col(it));
+        } else {
+#pragma unroll
+            for (int it = 0; it < NI; ++it) get(v[it], p.a + row + col(it));
+            for (int sp = 1; sp < p.nsplit; ++sp) {
+                float q[NI][8];
+#pragma unroll
+                for (int it = 0; it < NI; ++it) get(q[it], p.a + (size_t)sp * plane + row + col(it));
+#pragma unroll
+                for (int it = 0; it < NI; ++it)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[it][e] += q[it][e];
+            }
+#pragma unroll
+            for (int it = 0; it < NI; ++it) {
+                float r[8];
+                get(r, p.hidden + row + col(it));
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[it][e] += r[e];
+                if (in_row(it) && t < p.T) put(p.hidden + row + col(it), v[it]);
+            }
+        }
+        float ssq = 0.0f;
+#pragma unroll
+        for (int it = 0; it < NI; ++it)
+            if (in_row(it))
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ssq = fmaf(v[it][e], v[it][e], ssq);
+#pragma unroll
+        for (int o = 4; o <= 32; o <<= 1) ssq += __shfl_xor(ssq, o, 64);
+        if (lane < RS_TOK) sums[wave][lane] = ssq;
+        __syncthreads();
+        float tot = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) tot += sums[w][j];
+        const float rms_inv = 1.0f / sqrtf(tot / (float)W + p.eps);
+#pragma unroll
+        for (int it = 0; it < NI; ++it) {
+            float w[8];
+            get(w, p.weight + col(it));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[it][e] = v[it][e] * rms_inv * w[e];
+        }
+    } else {
+#pragma unroll
+        for (int it = 0; it < NI; ++it) {
+            get(v[it], p.a + row + col(it));
+            if constexpr (MODE == RS_SILU) {
+                float u[8];
+                get(u, p.b + row + col(it));
+                for (int sp = 1; sp < p.nsplit; ++sp) {
+                    float q[8], r[8];
+                    get(q, p.a + (size_t)sp * plane + row + col(it));
+                    get(r, p.b + (size_t)sp * plane + row + col(it));
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) { v[it][e] += q[e]; u[e] += r[e]; }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    v[it][e] = v[it][e] / (1.0f + expf(-v[it][e])) * u[e];
+                    asm volatile("" : "+v"(v[it][e]));   // (here: sunk into what asks for it, both operands of all turns are in registers, 51 more than there are)
+                }
+            }
+        }
+    }
+    uint32_t mb = 0;   // (bit patterns: ordered like the values, and a NaN is not dropped)
+#pragma unroll
+    for (int it = 0; it < NI; ++it)
+        if (in_row(it) && t < p.T) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mb = max(mb, __float_as_uint(v[it][e]) & 0x7FFFFFFFu);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[it][e] = 0.0f;   // (a padding token: the zeros that the matrix instructions read beside the last tokens)
+        }
+#pragma unroll
+    for (int o = 4; o <= 32; o <<= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
+    if (lane < RS_TOK) tops[wave][lane] = mb;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; ++w) mb = max(mb, tops[w][j]);
+    const int es = scale_exp_of_max(mb);
+    const float sc = __uint_as_float((uint32_t)es << 23);
+    const size_t chunk_bytes = ws_chunk_bytes(W);
+    if (tid < RS_TOK) reinterpret_cast<float*>(p.ws + (size_t)GB_MAX_CHUNKS * chunk_bytes)[t] = __uint_as_float((uint32_t)(254 - es) << 23);   // 1 / s
+    const int tl = t & (GB_TOK - 1), tb = tl >> 4, j16 = tl & 15;
+    uint8_t* chunk = p.ws + (size_t)(t / GB_TOK) * chunk_bytes;
+    u32x4* xb = reinterpret_cast<u32x4*>(chunk) + tb * 64 + (j16 + 16 * g);
+    _Float16* aux = reinterpret_cast<_Float16*>(chunk + (size_t)(W / 32 + 1) * GB_STEP_BYTES) + tb * 128 + j16 * 4;
+    auto sums_at = [&](int step) { return aux + (size_t)(step >> 3) * (GB_MIN_UNIT_BYTES / 2) + ((step >> 2) & 1) * 64 + (step & 3); };
+    auto pk = [](float lo, float hi) {
+        const f16x2 h = {(_Float16)lo, (_Float16)hi};
+        return __builtin_bit_cast(uint32_t, h);
+    };
+#pragma unroll
+    for (int it = 0; it < NI; ++it) {
+        const int step = (it * 16 + wave) * 4 + s4;
+        if (p.out && in_row(it) && t < p.T) put(p.out + row + col(it), v[it]);
+        float p1[8], p2[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[it][e] *= sc;
+            const _Float16 h1 = (_Float16)v[it][e];
+            p1[e] = (float)h1;
+            p2[e] = v[it][e] - p1[e];
+        }
+        float sum = ((v[it][0] + v[it][1]) + (v[it][2] + v[it][3])) + ((v[it][4] + v[it][5]) + (v[it][6] + v[it][7]));
+        sum += __shfl_xor(sum, 4, 64);   // (split_x_kernel: + column group g ^ 1, then + the other pair)
+        sum += __shfl_xor(sum, 8, 64);
+        if (in_row(it)) {
+            xb[(size_t)step * (GB_PLANES * 4 * 64)] = u32x4{pk(p1[0], p1[1]), pk(p1[2], p1[3]), pk(p1[4], p1[5]), pk(p1[6], p1[7])};
+            xb[(size_t)step * (GB_PLANES * 4 * 64) + 256] = u32x4{pk(p2[0], p2[1]), pk(p2[2], p2[3]), pk(p2[4], p2[5]), pk(p2[6], p2[7])};
+            if (g == 0) {
+                const float y = sum * 0.015625f;
+                const _Float16 h1 = (_Float16)y;
+                sums_at(step)[0] = h1;
+                sums_at(step)[4 * 128] = (_Float16)(y - (float)h1);
+            }
+        }
+    }
+    if (wave < 2) {   // the record of zeros behind the row, and a whole unit of zero sums
+        const int step = W / 32 + wave * 4 + s4;
+        if (step == W / 32)
+#pragma unroll
+            for (int pl = 0; pl < GB_PLANES; ++pl) xb[(size_t)step * (GB_PLANES * 4 * 64) + pl * 256] = u32x4{0u, 0u, 0u, 0u};
+        if (g == 0) { sums_at(step)[0] = (_Float16)0.0f; sums_at(step)[4 * 128] = (_Float16)0.0f; }
+    }
+}
+// turns of 2048 columns that the waves' registers hold: 128 a lane, the row's eighth part among them
+static inline int rows_split_turns(int width, bool one_operand) { return (width + 2047) / 2048 <= (one_operand ? 7 : 4) ? (width + 2047) / 2048 : 0; }
+template <int MODE>
+static int rows_split(const RowsSplitParams& p, hipStream_t st) {
+    const int n = rows_split_turns(p.W, MODE != RS_NORM);
+    const dim3 grid((unsigned)(((p.T + GB_TOK - 1) / GB_TOK * (GB_TOK / RS_TOK) + 31) / 32 * 32)), block(1024);
+    if (n == 0) return NTK_E_SHAPE;
+    if (n <= 2) hipLaunchKernelGGL((rows_split_kernel<MODE, 2>), grid, block, 0, st, p);
+    else if (n <= 4) hipLaunchKernelGGL((rows_split_kernel<MODE, 4>), grid, block, 0, st, p);
+    else if constexpr (MODE != RS_NORM) hipLaunchKernelGGL((rows_split_kernel<MODE, 7>), grid, block, 0, st, p);
+    return last_launch_status();
 }
 
 // ---- per-format weight operand ---------------------------------------------------------------------------------------------
@@ -2714,6 +2899,49 @@ int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* p, voi
     hipLaunchKernelGGL(ntk::silu_mul_split_kernel, dim3(ntk::split_pad_tokens(T)), dim3(1024), 0, ntk::resolve_stream(stream), output, p->part[0], p->part[1], p->nsplit, T, I,
                        static_cast<uint8_t*>(workspace));
     return ntk::last_launch_status();
+}
+
+// ---- a long prompt's producers (include/ntk_engine.h): rows_split_kernel -------------------------------------------------------------------------------------------------
+int ntk_rows_prepare_takes(int n_tokens, int width, int norm) {
+    return n_tokens > ntk::GB_TOK && n_tokens <= ntk::GB_MAX_CHUNKS * ntk::GB_TOK && width > 0 && width % 32 == 0 && ntk::rows_split_turns(width, !norm) > 0;
+}
+static bool rows_aligned(std::initializer_list<const void*> ps) {
+    for (const void* q : ps)
+        if (reinterpret_cast<uintptr_t>(q) & 15) return false;
+    return true;
+}
+int ntk_rows_prepare_x(const float* X, int n_tokens, int width, void* workspace, void* stream) {
+    if (!X || !workspace) return NTK_E_NULL;
+    if (!ntk_rows_prepare_takes(n_tokens, width, 0)) return NTK_E_SHAPE;
+    if (!rows_aligned({X, workspace})) return NTK_E_ALIGN;
+    ntk::RowsSplitParams p{};
+    p.a = X; p.T = n_tokens; p.W = width; p.ws = static_cast<uint8_t*>(workspace);
+    return ntk::rows_split<ntk::RS_LIES>(p, ntk::resolve_stream(stream));
+}
+int ntk_rows_norm_prepare_x(float* hidden, const ntk_gemm_partials* q, const float* weight, int n_tokens, int width, float eps, float* x_out, void* workspace, void* stream) {
+    if (!hidden || !weight || !workspace) return NTK_E_NULL;
+    if (!ntk_rows_prepare_takes(n_tokens, width, 1)) return NTK_E_SHAPE;
+    ntk::RowsSplitParams p{};
+    if (q) {
+        if (q->nseg != 1 || q->n_tokens != n_tokens || q->rows[0] != width || q->nsplit < 1) return NTK_E_SHAPE;
+        const bool sums = q->nsplit > 1 && q->part[0];
+        p.a = sums ? q->part[0] : q->y[0];
+        p.nsplit = sums ? q->nsplit : q->y[0] != hidden ? 1 : 0;   // (a projection that did not split wrote y, hidden's own rows with the residual if that is where y lies)
+    }
+    if (!rows_aligned({hidden, weight, x_out, workspace, p.a})) return NTK_E_ALIGN;
+    p.hidden = hidden; p.weight = weight; p.eps = eps; p.out = x_out; p.T = n_tokens; p.W = width; p.ws = static_cast<uint8_t*>(workspace);
+    return ntk::rows_split<ntk::RS_NORM>(p, ntk::resolve_stream(stream));
+}
+int ntk_rows_silu_mul_prepare_x(float* output, const ntk_gemm_partials* q, void* workspace, void* stream) {
+    if (!q || !workspace) return NTK_E_NULL;
+    if (q->nseg != 2 || q->rows[0] != q->rows[1] || q->nsplit < 1 || !ntk_rows_prepare_takes(q->n_tokens, q->rows[0], 0)) return NTK_E_SHAPE;
+    const bool sums = q->nsplit > 1 && q->part[0] && q->part[1];
+    ntk::RowsSplitParams p{};
+    p.a = sums ? q->part[0] : q->y[0]; p.b = sums ? q->part[1] : q->y[1]; p.nsplit = sums ? q->nsplit : 1;
+    if (!p.a || !p.b) return NTK_E_NULL;
+    if (!rows_aligned({p.a, p.b, output, workspace})) return NTK_E_ALIGN;
+    p.out = output; p.T = q->n_tokens; p.W = q->rows[0]; p.ws = static_cast<uint8_t*>(workspace);
+    return ntk::rows_split<ntk::RS_SILU>(p, ntk::resolve_stream(stream));
 }
 
 int ntk_rmsnorm_rowmax(float* output, const float* input, const float* weight, int n_tokens, int hidden_size, float eps, float* row_max,
