@@ -875,6 +875,14 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         ok(ntk_gemm_half(Y, w.ptr, X, T, (int)w.out_f, (int)w.in_f, accumulate ? 1 : 0, rm, ws, gemm_ws_bytes_, s));
         return true;
     };
+    // halves_of: the input whose halves ntk_half_norm_split has left in cur_ws (no rows are written: half_only of what reads it)
+    const float* halves_of = nullptr;
+    auto half_only = [&](std::initializer_list<const DevTensor*> ws) {
+        if (!with_max || !prefill_fused_split_ || tp_world_ > 1 || !gemm_ws2_ || !ntk_half_norm_takes(T, H, gemm_ws_bytes_)) return false;
+        for (const DevTensor* w : ws)
+            if (!w->ptr || w->dtype != NTK_DT_F16 || w->in_f < 3072 || (int)w->in_f != H || (reinterpret_cast<uintptr_t>(w->ptr) & 15)) return false;
+        return true;
+    };
     // several of them over one X in one launch (silu: gate and up, Y[0] = silu(gate) * up); false: not such matrices, nothing was launched
     auto project_half_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, bool silu) -> bool {
         ntk_half_desc d{};
@@ -882,11 +890,12 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             if (!batched || !bf16_now || !Ws[i]->ptr || Ws[i]->dtype != NTK_DT_F16 || Ws[i]->in_f < 3072 || Ws[i]->in_f != Ws[0]->in_f) return false;
             d.W[i] = Ws[i]->ptr; d.Y[i] = Ys[i]; d.out[i] = (int)Ws[i]->out_f;
         }
-        void* ws = cur_ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_;   // (as above)
+        const bool ready = X == halves_of;
+        void* ws = ready ? cur_ws : cur_ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_;   // (as above)
         const bool own = ws != nullptr;
         d.n = n; d.X = X; d.n_tokens = T; d.in_features = (int)Ws[0]->in_f; d.row_max = rm; d.silu = silu ? 1 : 0;
         d.workspace = own ? ws : cur_ws; d.workspace_bytes = gemm_ws_bytes_;
-        const int st = ntk_gemm_half_many(&d, s);
+        const int st = ready ? ntk_gemm_half_normed(&d, s) : ntk_gemm_half_many(&d, s);
         if (st == NTK_E_SHAPE || st == NTK_E_ALIGN) return false;
         if (!own) planes_of = nullptr;
         ok(st);
@@ -991,7 +1000,15 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         max_a = written ? rm_a : nullptr;
         if (zero_b) b_clear = written && rm_b;
     };
-    auto norm = [&](const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only) {     // only: planes_only of the matrices that read it
+    auto norm = [&](const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only, bool half) {     // only, half: planes_only, half_only of the matrices that read it
+        halves_of = nullptr;
+        if (half) {
+            planes_of = planes_ready = nullptr;
+            ok(ntk_half_norm_split(hidden_, nullptr, (const float*)nw.ptr, T, H, cfg_.norm_eps, cur_ws, gemm_ws_bytes_, s));
+            halves_of = residual_;
+            left_max(false, zero_b);
+            return;
+        }
         if (splits_rows(H, true) && f16_ok(next_w) && (int)next_w.in_f == H) {
             void* ws = flip_ws();
             ok(fuse_split ? ntk_rmsnorm_prepare_x(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, ws, s)
@@ -1006,7 +1023,18 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
     };
     // hidden += W . X followed by the NEXT RMSNorm (nw; into residual_, with the token maxima) as one consumer launch of the projection's K splits
     // (ntk_gemm_quant_f16 with `partials` + ntk_reduce_rmsnorm_rowmax); false = not this shape / format: the caller runs project_add + norm
-    auto project_add_norm = [&](const DevTensor& w, const float* X, const float* rm, const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only) -> bool {
+    auto project_add_norm = [&](const DevTensor& w, const float* X, const float* rm, const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only, bool half) -> bool {
+        if (half && w.ptr && w.dtype == NTK_DT_F16 && w.in_f >= 3072 && (size_t)w.out_f == (size_t)H) {   // (the pieces lie in the other workspace: the halves go to this one)
+            ntk_gemm_partials pt;
+            void* ws = cur_ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_;
+            int st = ntk_gemm_half_defer(hidden_, w.ptr, X, T, H, (int)w.in_f, rm, ws, gemm_ws_bytes_, &pt, s);
+            planes_of = planes_ready = nullptr;
+            if (st == NTK_OK) st = ntk_half_norm_split(hidden_, &pt, (const float*)nw.ptr, T, H, cfg_.norm_eps, cur_ws, gemm_ws_bytes_, s);
+            halves_of = residual_;
+            left_max(false, zero_b);
+            ok(st);
+            return true;
+        }
         if (!with_max || tp_world_ > 1 || !is_quant(w.dtype) || (size_t)w.out_f != (size_t)H) return false;
         ntk_gemm_partials pt;
         int st = NTK_E_DTYPE;
@@ -1023,6 +1051,15 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             st = gemm_f16(&sg, 1, X, (int)w.in_f, hidden_, X == planes_of ? 1 : 0, rm, &pt, false);
         }
         if (st == NTK_E_DTYPE || st == NTK_E_SHAPE || st == NTK_E_ALIGN) return false;   // (nothing was launched)
+        if (half) {   // (an unquantised group behind a quantised projection)
+            if (st == NTK_OK) st = ntk_half_norm_split(hidden_, &pt, (const float*)nw.ptr, T, H, cfg_.norm_eps, flip_ws(), gemm_ws_bytes_, s);
+            planes_of = planes_ready = nullptr;
+            halves_of = residual_;
+            left_max(false, zero_b);
+            ok(st);
+            return true;
+        }
+        halves_of = nullptr;
         planes_of = nullptr;
         if (st == NTK_OK && splits_rows(H, true) && f16_ok(next_w) && (int)next_w.in_f == H) {   // (the partial sums lie in cur_ws: the planes go to the other one)
             void* ws = flip_ws();
@@ -1041,7 +1078,8 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         uint16_t* kc = k_cache_ + (size_t)i * kv_layer;
         uint16_t* vc = v_cache_ + (size_t)i * kv_layer;
         auto only_qkv = [&](const LayerWeights& l) { return planes_only({&l.wq, &l.wk, &l.wv}, H); };
-        if (!normed_ahead) norm(L.attn_norm, true, L.wq, only_qkv(L));
+        auto half_qkv = [&](const LayerWeights& l) { return half_only({&l.wq, &l.wk, &l.wv}); };
+        if (!normed_ahead) norm(L.attn_norm, true, L.wq, only_qkv(L), half_qkv(L));
         normed_ahead = false;
         planes_of = planes_ready;   // residual_ has new contents (split already by the launch that wrote them, or not)
         planes_ready = nullptr;
@@ -1067,9 +1105,11 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         if (T == 1) ok(ntk_attention_decode(attn_out, q_buf, kc, vc, start_pos + T, nh, nkv, hd, cfg_.max_seq_len, scale, s));
         else ok(ntk_attention_prefill(attn_out, q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
         const bool only_unit = planes_only({&L.w_gate, &L.w_up}, H);
-        if (!project_add_norm(L.wo, attn_out, nullptr, L.ffn_norm, false, L.w_gate, only_unit)) {
+        const intptr_t apart = (intptr_t)L.w_gate.ptr - (intptr_t)L.w_up.ptr;
+        const bool half_unit = half_only({&L.w_gate, &L.w_up}) && std::abs(apart) < (1LL << 32) - (intptr_t)L.w_gate.out_f * H * 2;   // (what ntk_gemm_half_many takes as a gated pair)
+        if (!project_add_norm(L.wo, attn_out, nullptr, L.ffn_norm, false, L.w_gate, only_unit, half_unit)) {
             project_add(L.wo, attn_out, qd, nullptr);
-            norm(L.ffn_norm, false, L.w_gate, only_unit);
+            norm(L.ffn_norm, false, L.w_gate, only_unit, half_unit);
         }
         planes_of = planes_ready;
         planes_ready = nullptr;
@@ -1122,7 +1162,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         planes_of = planes_ready;
         planes_ready = nullptr;
         // down projection + residual, and the NEXT layer's first RMSNorm in the same consumer launch when there is a next layer in this pass
-        if (i + 1 < last_layer && project_add_norm(L.w_down, gate_buf, max_b, layers_[i + 1].attn_norm, true, layers_[i + 1].wq, only_qkv(layers_[i + 1]))) normed_ahead = true;
+        if (i + 1 < last_layer && project_add_norm(L.w_down, gate_buf, max_b, layers_[i + 1].attn_norm, true, layers_[i + 1].wq, only_qkv(layers_[i + 1]), half_qkv(layers_[i + 1]))) normed_ahead = true;
         else project_add(L.w_down, gate_buf, I, max_b);
         if (rc != NTK_OK) break;
     }

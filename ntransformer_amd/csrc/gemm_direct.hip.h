@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256) void gemm_direct_sum_kernel(const DirectArgs d
 }
 
 template <class P, int TM, int TN, int WM, int WN, int STAGES, int GLU, int MINW>
-static void launch_direct(DirectArgs d, int splits, hipStream_t s) {
+static int launch_direct(DirectArgs d, int splits, hipStream_t s, bool sum = true) {      // (as launch_tiles; sum false: one matrix)
     constexpr int BK = 128 / (int)sizeof(typename P::WT);
     const int chunks = d.t.K / BK, per = (chunks + splits - 1) / splits;
     d.t.k_per_split = per * BK;
@@ -335,12 +335,13 @@ static void launch_direct(DirectArgs d, int splits, hipStream_t s) {
         for (int i = 0; i < d.n_seg; ++i) { d.seg_tile[i] = col_tiles; col_tiles += (d.seg_out[i] + TN - 1) / TN; }
     }
     hipLaunchKernelGGL((gemm_direct_kernel<P, TM, TN, WM, WN, STAGES, GLU, MINW>), dim3(row_tiles * col_tiles * d.t.splits), dim3(64 * WM * WN), 0, s, d, row_tiles, col_tiles);
-    if (d.t.splits == 1) return;
-    if (d.n_seg <= 1) { launch_tile_sum(d.t, s); return; }
+    if (d.t.splits == 1 || !sum) return d.t.splits;
+    if (d.n_seg <= 1) { launch_tile_sum(d.t, s); return d.t.splits; }
     bool four = !((uintptr_t)d.t.part & 15);
     for (int i = 0; i < d.n_seg; ++i) four = four && d.seg_out[i] % 4 == 0 && !((uintptr_t)d.segY[i] & 15);
     if (four) hipLaunchKernelGGL((gemm_direct_sum_kernel<4>), dim3((d.t.N / 4 + 255) / 256, d.t.T), dim3(256), 0, s, d);
     else hipLaunchKernelGGL((gemm_direct_sum_kernel<1>), dim3((d.t.N + 255) / 256, d.t.T), dim3(256), 0, s, d);
+    return d.t.splits;
 }
 
 }  // namespace ntk

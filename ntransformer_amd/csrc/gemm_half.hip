@@ -67,17 +67,87 @@ __global__ __launch_bounds__(256) void half_split_kernel(_Float16* out, long lon
     for (int k = 8 * (threadIdx.x + 256 * kHalfKeep); k < K; k += 8 * 256) put(k, *reinterpret_cast<const float4*>(x + k), *reinterpret_cast<const float4*>(x + k + 4));
 }
 
+// hidden += the pieces of a projection (nsplit 0: hidden as it lies), and of its RMSNorm the two halves and the rows' largest |x|, as half_split_kernel leaves them; a workgroup a row, which
+// stays in registers.  In the place of three launches that each take the row through memory (the sum, the norm, the split): us, 200 rows of 4096 behind eight pieces 6.2 + 8.0 + 5.2,
+// 7.2 so.
+struct HalfNormArgs { float* hidden; const float* part; int nsplit, H; long long pieces; const float* weight; float eps; _Float16* out; long long plane; float* row_max; };
+template <int KEEP>
+__global__ __launch_bounds__(1024) void half_norm_split_kernel(const HalfNormArgs a) {
+    __shared__ float red[16], top[16];
+    float* h = a.hidden + (long long)blockIdx.x * a.H;
+    const float* p = a.part + (long long)blockIdx.x * a.H;
+    const int bd = (int)blockDim.x;
+    float v[KEEP][8];
+    float ssq = 0.0f;
+    auto get = [](float (&d)[8], const float* src) {
+        const float4 x = *reinterpret_cast<const float4*>(src), y = *reinterpret_cast<const float4*>(src + 4);
+        d[0] = x.x; d[1] = x.y; d[2] = x.z; d[3] = x.w; d[4] = y.x; d[5] = y.y; d[6] = y.z; d[7] = y.w;
+    };
+    float w[KEEP][8];
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) {
+        const int k = 8 * ((int)threadIdx.x + bd * u), at = k < a.H ? k : 0;     // (past the row: column 0 again, dropped)
+        float old[8];
+        get(old, h + at);
+        get(w[u], a.weight + at);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] = 0.0f;
+        for (int i = 0; i < a.nsplit; i += 4) {                 // four pieces under way, added in order
+            float q[4][8];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) get(q[c], p + a.pieces * min(i + c, a.nsplit - 1) + at);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (i + c < a.nsplit)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[u][e] += q[c][e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] += old[e];
+        if (k < a.H) {
+            if (a.nsplit) {
+                *reinterpret_cast<float4*>(h + k) = float4{v[u][0], v[u][1], v[u][2], v[u][3]};
+                *reinterpret_cast<float4*>(h + k + 4) = float4{v[u][4], v[u][5], v[u][6], v[u][7]};
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ssq = fmaf(v[u][e], v[u][e], ssq);
+        }
+    }
+    const float inv = 1.0f / sqrtf(block_sum(ssq, red) / (float)a.H + a.eps);
+    uint32_t mb = 0;   // (bit patterns: ordered like the values, and a NaN is not dropped)
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[u][e] = v[u][e] * inv * w[u][e];
+            if (8 * ((int)threadIdx.x + bd * u) < a.H) mb = max(mb, __float_as_uint(v[u][e]) & 0x7FFFFFFFu);
+        }
+    const float largest = block_max(__uint_as_float(mb <= 0x7F800000u ? mb : 0x7F800000u), top);
+    if (threadIdx.x == 0) a.row_max[blockIdx.x] = largest;
+    const float scale = half_scale(largest);
+    uint16_t* o = reinterpret_cast<uint16_t*>(a.out) + (long long)blockIdx.x * a.H;
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) {
+        const int k = 8 * ((int)threadIdx.x + bd * u);
+        if (k >= a.H) continue;
+        uintx4_t b[2];
+        TileHalf2::convert(v[u], scale, b);
+        *reinterpret_cast<uintx4_t*>(o + k) = b[0];
+        *reinterpret_cast<uintx4_t*>(o + a.plane + k) = b[1];
+    }
+}
+
 // two matrix instructions a product: constants as for bf16 (plan_direct), from 16 .. 200 rows, 1024 .. 28672 outputs, 4096 .. 14336 inputs
 static TilePlan plan_direct_half(int rows, int N, int K, long long room) {
     static const DirectForm forms[] = {{128, 256, 1, 1.65f, 1.65f, 12.0f}, {64, 128, 2, 0.82f, 0.495f, 5.0f}, {64, 64, 2, 0.47f, 0.315f, 4.0f}};
     return plan_direct(forms, 3, 64, rows, 1, N, K, room);
 }
 template <int GLU>
-static void launch_direct_half(const DirectArgs& d, const TilePlan& p, hipStream_t s) {
+static int launch_direct_half(const DirectArgs& d, const TilePlan& p, hipStream_t s, bool sum = true) {
     switch (p.form) {
-        case 0: launch_direct<TileHalf2, 128, 256, 2, 4, 2, GLU, 2>(d, p.splits, s); break;
-        case 1: launch_direct<TileHalf2, 64, 128, 2, 2, 2, GLU, 2>(d, p.splits, s); break;
-        default: launch_direct<TileHalf2, 64, 64, 2, 2, 3, GLU, 2>(d, p.splits, s); break;
+        case 0: return launch_direct<TileHalf2, 128, 256, 2, 4, 2, GLU, 2>(d, p.splits, s, sum);
+        case 1: return launch_direct<TileHalf2, 64, 128, 2, 2, 2, GLU, 2>(d, p.splits, s, sum);
+        default: return launch_direct<TileHalf2, 64, 64, 2, 2, 3, GLU, 2>(d, p.splits, s, sum);
     }
 }
 
@@ -95,7 +165,12 @@ static int half_pass_rows(int T, int K, size_t bytes) {
 static size_t half_max_bytes(int rows) { return ((size_t)rows * 4 + 15) & ~(size_t)15; }
 size_t ntk_gemm_half_many_bytes(int n_tokens, int in_features) { return n_tokens > 0 && in_features > 0 ? (size_t)std::min(n_tokens, 16) * half_row_bytes(in_features) + 32 : 0; }
 
-int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
+// a product whose sums are left to its consumer: where they are, or that there are none
+static void leave(ntk_gemm_partials* q, float* Y, int rows, int T, int splits, const float* part) {
+    *q = ntk_gemm_partials{};
+    q->nseg = 1; q->n_tokens = T; q->nsplit = splits; q->part[0] = splits > 1 ? part : nullptr; q->y[0] = Y; q->rows[0] = rows;
+}
+static int half_many(const ntk_half_desc* d, bool ready, ntk_gemm_partials* defer, void* stream) {
     if (!d || !d->X || d->n < 1 || d->n > 3) return NTK_E_NULL;
     long long N = 0;
     uintptr_t bits = (uintptr_t)d->X | (uintptr_t)d->workspace;
@@ -115,6 +190,7 @@ int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
     if (K % 64 || K >= 1 << 22 || N > 1 << 30 || (d->silu && std::abs((long long)(w1 - w0)) + mat >= 1LL << 32)) return NTK_E_SHAPE;
     if (d->workspace_bytes < ntk_gemm_half_many_bytes(T, K)) return NTK_E_SHAPE;
     const int per = half_pass_rows(T, K, d->workspace_bytes);
+    if ((ready || defer) && per < T) return NTK_E_SHAPE;
     hipStream_t s = resolve_stream(stream);
     for (int t0 = 0; t0 < T; t0 += per) {
         const int n = std::min(per, T - t0);
@@ -124,12 +200,13 @@ int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
         char* behind = (char*)d->workspace + 4 * plane;                     // (plane is a multiple of 64)
         float* own_max = (float*)behind;
         behind += half_max_bytes(n);
-        if (d->row_max) hipLaunchKernelGGL(half_split_kernel<true>, dim3(n), dim3(256), 0, s, halves, plane, x, K, const_cast<float*>(d->row_max) + t0);
+        if (ready) ;                                                        // (ntk_half_norm_split has left them)
+        else if (d->row_max) hipLaunchKernelGGL(half_split_kernel<true>, dim3(n), dim3(256), 0, s, halves, plane, x, K, const_cast<float*>(d->row_max) + t0);
         else hipLaunchKernelGGL(half_split_kernel<false>, dim3(n), dim3(256), 0, s, halves, plane, x, K, own_max);
         DirectArgs a{};
         TileArgs& t = a.t;
         t.W = d->W[0]; t.Y = d->Y[0] + (long long)t0 * d->out[0]; t.ldy = d->out[0]; t.G = 1; t.row_div = 1; t.T = n; t.N = (int)N; t.K = K; t.accumulate = d->accumulate;
-        t.row_max = d->row_max ? d->row_max + t0 : own_max;
+        t.row_max = d->row_max && !ready ? d->row_max + t0 : own_max;
         t.part = (float*)behind;
         a.X16 = halves; a.x_row = (uint32_t)K * 2; a.plane = plane * 2;
         const long long left = (char*)d->workspace + d->workspace_bytes - behind;
@@ -143,15 +220,43 @@ int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) {
         }
         a.n_seg = d->n;
         for (int i = 0; i < d->n; ++i) { a.segW[i] = d->W[i]; a.segY[i] = d->Y[i] + (long long)t0 * d->out[i]; a.seg_out[i] = d->out[i]; }
-        launch_direct_half<kGluNone>(a, p, s);
+        const int splits = launch_direct_half<kGluNone>(a, p, s, !defer);
+        if (defer) leave(defer, d->Y[0], d->out[0], T, splits, t.part);
     }
     return last_launch_status();
 }
+int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) { return half_many(d, false, nullptr, stream); }
+
+// ---- a norm's halves from the launch that sums the projection in front of it (include/ntk_engine.h) ----
+int ntk_half_norm_takes(int n_tokens, int width, size_t workspace_bytes) {
+    return n_tokens > 0 && n_tokens <= 65535 && width > 0 && width % 64 == 0 && width <= 16384 && workspace_bytes >= ntk_gemm_half_many_bytes(n_tokens, width) &&
+           half_pass_rows(n_tokens, width, workspace_bytes) == n_tokens;
+}
+int ntk_half_norm_split(float* hidden, const ntk_gemm_partials* q, const float* weight, int n_tokens, int width, float eps, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!hidden || !weight || !workspace) return NTK_E_NULL;
+    if (!ntk_half_norm_takes(n_tokens, width, workspace_bytes)) return NTK_E_SHAPE;
+    HalfNormArgs a{};
+    a.part = hidden;                            // (never read with nsplit 0)
+    if (q) {
+        if (q->nseg != 1 || q->n_tokens != n_tokens || q->rows[0] != width || q->nsplit < 1) return NTK_E_SHAPE;
+        const bool sums = q->nsplit > 1 && q->part[0];
+        if (sums || q->y[0] != hidden) { a.part = sums ? q->part[0] : q->y[0]; a.nsplit = sums ? q->nsplit : 1; }
+    }
+    if (!a.part) return NTK_E_NULL;
+    if (((uintptr_t)hidden | (uintptr_t)weight | (uintptr_t)workspace | (uintptr_t)a.part) & 15) return NTK_E_ALIGN;
+    a.hidden = hidden; a.H = width; a.pieces = (long long)n_tokens * width; a.weight = weight; a.eps = eps;
+    a.out = (_Float16*)workspace; a.plane = a.pieces; a.row_max = (float*)((char*)workspace + 4 * a.plane);
+    const int threads = width <= 2048 ? 256 : width <= 4096 ? 512 : 1024;
+    if (width <= 8 * threads) hipLaunchKernelGGL(half_norm_split_kernel<1>, dim3(n_tokens), dim3(threads), 0, resolve_stream(stream), a);
+    else hipLaunchKernelGGL(half_norm_split_kernel<2>, dim3(n_tokens), dim3(threads), 0, resolve_stream(stream), a);
+    return last_launch_status();
+}
+int ntk_gemm_half_normed(const ntk_half_desc* d, void* stream) { return half_many(d, true, nullptr, stream); }
 
 size_t ntk_gemm_half_workspace_bytes(int n_tokens) { return ((size_t)(n_tokens > 0 ? n_tokens : 0) * sizeof(float) + 15) & ~(size_t)15; }
 
-int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
-                   size_t workspace_bytes, void* stream) {
+static int gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
+                     size_t workspace_bytes, ntk_gemm_partials* defer, void* stream) {
     if (!Y || !W || !X) return NTK_E_NULL;
     if (n_tokens < 0 || out_features <= 0 || in_features <= 0) return NTK_E_SHAPE;
     if (n_tokens == 0) return NTK_OK;
@@ -183,7 +288,7 @@ int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out
             ntk_half_desc d{};
             d.W[0] = W; d.Y[0] = Y; d.out[0] = out_features; d.n = 1; d.X = X; d.n_tokens = n_tokens; d.in_features = in_features; d.accumulate = accumulate; d.row_max = row_max;
             d.workspace = workspace; d.workspace_bytes = workspace_bytes;
-            return ntk_gemm_half_many(&d, stream);
+            return half_many(&d, false, passes == 1 ? defer : nullptr, stream);
         }
     }
     if (need) {
@@ -191,7 +296,17 @@ int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out
         t.row_max = (const float*)workspace;
     }
     if (!vec) { launch_tiles<TileHalf2, 64, 64, 2, 2, 2, false>(t, 1, s); return last_launch_status(); }
-    if (p.form == 0) launch_tiles<TileHalf2, 64, 128, 2, 2, 4, true>(t, p.splits, s);
-    else launch_tiles<TileHalf2, 32, 64, 2, 2, 2, true>(t, p.splits, s);
+    const int splits = p.form == 0 ? launch_tiles<TileHalf2, 64, 128, 2, 2, 4, true>(t, p.splits, s, !defer) : launch_tiles<TileHalf2, 32, 64, 2, 2, 2, true>(t, p.splits, s, !defer);
+    if (defer) leave(defer, Y, out_features, n_tokens, splits, t.part);
     return last_launch_status();
+}
+int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
+                   size_t workspace_bytes, void* stream) {
+    return gemm_half(Y, W, X, n_tokens, out_features, in_features, accumulate, row_max, workspace, workspace_bytes, nullptr, stream);
+}
+int ntk_gemm_half_defer(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, const float* row_max, void* workspace, size_t workspace_bytes,
+                        ntk_gemm_partials* partials, void* stream) {
+    if (!partials) return NTK_E_NULL;
+    leave(partials, Y, out_features, n_tokens, 1, nullptr);
+    return gemm_half(Y, W, X, n_tokens, out_features, in_features, 1, row_max, workspace, workspace_bytes, partials, stream);
 }

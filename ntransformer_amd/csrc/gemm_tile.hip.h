@@ -414,14 +414,15 @@ static void launch_tile_sum(const TileArgs& a, hipStream_t s) {
 }
 
 template <class P, int TM, int TN, int SUB, int WM, int WN, bool VEC>
-static void launch_tiles(TileArgs a, int splits, hipStream_t s) {
+static int launch_tiles(TileArgs a, int splits, hipStream_t s, bool sum = true) {      // the pieces of K that a.part holds (sum: added up by a launch of their own)
     constexpr int BK = P::KE * SUB;
     const int chunks = (a.K + BK - 1) / BK, per = (chunks + splits - 1) / splits;
     a.k_per_split = per * BK;
     a.splits = (chunks + per - 1) / per;
     const int row_tiles = a.offsets ? a.T / TM + a.G : (a.T + TM - 1) / TM;
     hipLaunchKernelGGL((gemm_tile_kernel<P, TM, TN, SUB, WM, WN, VEC>), dim3((a.N + TN - 1) / TN, row_tiles * a.splits), dim3(64 * WM * WN), 0, s, a);
-    if (a.splits > 1) launch_tile_sum(a, s);
+    if (a.splits > 1 && sum) launch_tile_sum(a, s);
+    return a.splits;
 }
 
 }  // namespace ntk
