@@ -254,6 +254,9 @@ size_t ntk_gemm_half_workspace_bytes(int n_tokens);
 int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
                   size_t workspace_bytes, void* stream);
 
+/* Y[t] = W . X[t] of F16 or F32 rows in one launch, each product with ntk_gemv's bits.  in_features a multiple of 8, 16-byte aligned W and X (NTK_E_ALIGN: nothing was launched). */
+int ntk_gemv_tokens(float* y, const void* W, const float* x, int n_tokens, int out_features, int in_features, int weight_dtype, void* stream);
+
 /* ... for up to three such matrices over the same X (query, key and value; gate and up) in one launch, with the activations' two halves formed once per pass in the workspace
  * (ntk_gemm_half_many_bytes() of it at least, which is 16 tokens' worth; the tokens go in equal passes of what it holds, 4 * in_features + 4 bytes each, and every pass reads the weights:
  * give it room for all of them; more is used for partial sums).  Y[i] = W[i] . X; silu != 0 (n == 2, out[0] == out[1]): Y[0] = silu(W[0] . X) * (W[1] . X) alone (ntk_silu_mul).

@@ -922,6 +922,10 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
                 st = ntk_gemm_quant(Y, wp, X, T, (int)w.out_f, (int)w.in_f, w.dtype, nullptr, s);
             if (st != NTK_E_ALIGN && st != NTK_E_SHAPE) { ok(st); return; }   // those two: shapes only the per-token loop takes
         }
+        if (batched && wp && (w.dtype == NTK_DT_F16 || w.dtype == NTK_DT_F32) && ystride == (size_t)w.out_f && xstride == (size_t)w.in_f) {
+            const int st = ntk_gemv_tokens(Y, wp, X, T, (int)w.out_f, (int)w.in_f, w.dtype, s);
+            if (st != NTK_E_ALIGN && st != NTK_E_SHAPE) { ok(st); return; }
+        }
         for (int t = 0; t < T; ++t) gemv(Y + (size_t)t * ystride, w, wp, X + (size_t)t * xstride);
     };
     // matrices that share X (Q | K | V, gate | up): those of one format go out as ONE launch of the FP16 GEMM, the rest one by one, ahead of them.  sums / splits: the LAST launch may

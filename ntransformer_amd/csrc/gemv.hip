@@ -629,6 +629,51 @@ __global__ __launch_bounds__(256) void gemv_dense_kernel(float* __restrict__ y, 
     }
 }
 
+// ... and of a prompt's tokens, for the matrices that are too narrow for the tiles over halves (model.cpp: their results would be further from 64 bits): ROWS rows and TOK tokens a wave,
+// a weight read once for its tokens and an activation once for its rows.  A product adds up in gemv_dense_kernel's order: identical bits.  us, 2 / 16 / 200 tokens of 1024
+// through 1024 rows: 9.1 / 57 / 669 with a launch a token, 3.3 / 4.3 / 21 so (20 TF/s on the vector units)
+template <typename T, int ROWS, int TOK>
+__global__ __launch_bounds__(256) void gemv_dense_tokens_kernel(float* __restrict__ y, const T* __restrict__ W, const float* __restrict__ x, int n_tokens, int out, int in) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int lane = threadIdx.x & 63, r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * ROWS, t0 = blockIdx.y * TOK;
+    if (r0 >= out) return;
+    float acc[ROWS][TOK] = {};
+    for (int i = lane; i < in / V; i += 64) {
+        u32x4 raw[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) raw[r] = *(reinterpret_cast<const u32x4*>(W + (size_t)min(r0 + r, out - 1) * in) + i);
+#pragma unroll
+        for (int t = 0; t < TOK; ++t) {
+            const float* xt = x + (size_t)min(t0 + t, n_tokens - 1) * in + V * i;
+            float xv[V];
+#pragma unroll
+            for (int q = 0; q < V; q += 4) {
+                const float4 f = *reinterpret_cast<const float4*>(xt + q);
+                xv[q] = f.x; xv[q + 1] = f.y; xv[q + 2] = f.z; xv[q + 3] = f.w;
+            }
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const uint32_t w[4] = {raw[r].x, raw[r].y, raw[r].z, raw[r].w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if constexpr (sizeof(T) == 4) acc[r][t] = fmaf(__uint_as_float(w[q]), xv[q], acc[r][t]);
+                    else {
+                        acc[r][t] = fmaf(h2f((uint16_t)(w[q] & 0xFFFF)), xv[2 * q], acc[r][t]);
+                        acc[r][t] = fmaf(h2f((uint16_t)(w[q] >> 16)), xv[2 * q + 1], acc[r][t]);
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int t = 0; t < TOK; ++t) {
+            const float s = wave_sum(acc[r][t]);
+            if (lane == 0 && r0 + r < out && t0 + t < n_tokens) y[(size_t)(t0 + t) * out + r0 + r] = s;
+        }
+}
+
 // ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
@@ -892,6 +937,25 @@ int ntk_gemv(float* y, const void* W, const float* x, int out_features, int in_f
     if (!ntk::is_quant(weight_dtype)) return NTK_E_DTYPE;
     ntk_gemv_seg seg{W, y, out_features, weight_dtype};
     return ntk::dispatch_quant(weight_dtype, &seg, 1, x, in_features, nullptr, 0.0f, nullptr, 0, st);
+}
+
+int ntk_gemv_tokens(float* y, const void* W, const float* x, int n_tokens, int out_features, int in_features, int weight_dtype, void* stream) {
+    if (!y || !W || !x) return NTK_E_NULL;
+    if (n_tokens < 0 || out_features < 0 || in_features <= 0 || n_tokens > 65535 * 4) return NTK_E_SHAPE;
+    if (weight_dtype != NTK_DT_F32 && weight_dtype != NTK_DT_F16) return NTK_E_DTYPE;
+    if (in_features % 8 || ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(x)) & 15)) return NTK_E_ALIGN;   // (rows and tokens all on 16 bytes, where gemv_dense_kernel takes pieces)
+    if (n_tokens == 0 || out_features == 0) return NTK_OK;
+    auto go = [&](auto kernel, auto w, int tok) {
+        hipLaunchKernelGGL(kernel, dim3((out_features + 7) / 8, (n_tokens + tok - 1) / tok), dim3(256), 0, ntk::resolve_stream(stream), y, w, x, n_tokens, out_features, in_features);
+    };
+    if (weight_dtype == NTK_DT_F32) {
+        if (n_tokens <= 4) go(ntk::gemv_dense_tokens_kernel<float, 2, 4>, static_cast<const float*>(W), 4);
+        else go(ntk::gemv_dense_tokens_kernel<float, 2, 8>, static_cast<const float*>(W), 8);
+    } else {
+        if (n_tokens <= 4) go(ntk::gemv_dense_tokens_kernel<uint16_t, 2, 4>, static_cast<const uint16_t*>(W), 4);
+        else go(ntk::gemv_dense_tokens_kernel<uint16_t, 2, 8>, static_cast<const uint16_t*>(W), 8);
+    }
+    return ntk::last_launch_status();
 }
 
 int ntk_gemv_add(float* y, const void* W, const float* x, int out_features, int in_features, int weight_dtype, void* stream) {
