@@ -45,6 +45,24 @@ __device__ __forceinline__ float activate(float v, int act, float cap) {
     return v;
 }
 
+// what a product of the few-row forms leaves: s = the wave's sums (lane 63's count), outputs n0 .. of activation row r
+template <int RW, bool GLU>
+__device__ __forceinline__ void leave_outputs(const DenseArgs& a, const float (&s)[RW], int r, int n0, int n_out) {
+    constexpr int OUT = GLU ? RW / 2 : RW;
+#pragma unroll
+    for (int i = 0; i < OUT; ++i) {
+        if (n0 + i >= n_out) continue;
+        float t = s[i];
+        if constexpr (GLU) {
+            const float gg = fminf(s[i], a.glu_limit), uu = fminf(fmaxf(s[i + OUT], -a.glu_limit), a.glu_limit);
+            const float zz = a.glu_cubic != 0.0f ? fmaf(a.glu_cubic * gg * gg, gg, gg) : gg;
+            t = gg * (1.0f / (1.0f + expf(-a.glu_alpha * zz))) * (uu + a.glu_up_offset);
+        }
+        float* y = a.Y + (long long)r * a.ldy + n0 + i;
+        *y = a.accumulate ? *y + t : activate(t, a.act, a.glu_limit);
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------- few rows: waves stream weight rows
 // One workgroup per (group of 4 * RW outputs, activation row): the activation row sits in LDS, each wave owns RW consecutive weight rows and walks
 // them together -- per step a lane requests the NEXT 16 bytes of each of its RW rows, then reads its 8 activations once and feeds RW sums from the bytes that
@@ -219,18 +237,149 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(const DenseArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < RW; ++i) s[i] = wave_sum_lane63(s[i]);
+    if (lane == 63) leave_outputs<RW, GLU>(a, s, r, n0, n_out);
+}
+
+// ... with the weights read once for R activation rows (a workgroup a row reads them R times, mostly out of the Infinity Cache): the rows' next 1024 columns sit in LDS, a
+// lane feeds RW x R sums from a piece of weights.  A row's norm is summed by one wave in the order of the workgroup above, and a sum over k in that kernel's: identical bits.
+// Rows on 16 bytes, one group.
+constexpr int kRowsStage = 1024;                        // two pieces
+template <typename WT, int RW, bool GLU, bool ADD, int R>
+__global__ __launch_bounds__(256) void dense_gemv_rows_kernel(const DenseArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float xs[];   // [R][columns of a stage]
+    __shared__ float scale[2][R];                                // 1 / rms of the rows, and of what they are still owed
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r0 = blockIdx.y * R, live = min(R, a.T - r0);
+    constexpr int OUT = GLU ? RW / 2 : RW, NV = sizeof(WT) == 2 ? 1 : 2;
+    const int n_out = GLU ? a.glu_ff : a.N, n0 = (blockIdx.x * 4 + wave) * OUT;
+    const WT* w[RW];
 #pragma unroll
-    for (int i = 0; i < OUT; ++i) {
-        if (lane == 63 && n0 + i < n_out) {
-            float t = s[i];
-            if constexpr (GLU) {
-                const float gg = fminf(s[i], a.glu_limit), uu = fminf(fmaxf(s[i + OUT], -a.glu_limit), a.glu_limit);
-                const float zz = a.glu_cubic != 0.0f ? fmaf(a.glu_cubic * gg * gg, gg, gg) : gg;
-                t = gg * (1.0f / (1.0f + expf(-a.glu_alpha * zz))) * (uu + a.glu_up_offset);
+    for (int i = 0; i < RW; ++i) {                          // rows past the end re-read the last one and are not stored
+        const int row = GLU ? (i < OUT ? min(n0 + i, n_out - 1) : a.glu_ff + min(n0 + i - OUT, n_out - 1)) : min(n0 + i, n_out - 1);
+        w[i] = (const WT*)a.W + (long long)row * a.K;
+    }
+    auto weights = [&](uintx4_t (&u)[RW][NV], int k) {
+#pragma unroll
+        for (int i = 0; i < RW; ++i)
+#pragma unroll
+            for (int p = 0; p < NV; ++p) u[i][p] = __builtin_nontemporal_load(reinterpret_cast<const uintx4_t*>(w[i] + k) + p);
+    };
+    // a ring of pieces of 512 columns of the wave's weights: with the rows in one workgroup there are few waves, and what hides the memory's latency is what each has under way
+    constexpr int D = RW >= 4 ? 4 : 8 / RW;
+    uintx4_t ring[D][RW][NV];
+    auto request = [&](int d, int piece) {
+        const int k = piece * 512 + lane * 8;
+        if (k < a.K) weights(ring[d], k);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) request(d, d);
+    auto x_of = [&](int r) { return a.X + (long long)(a.rows ? a.rows[r] / a.row_div : r) * a.ldx; };
+    auto owed = [&](float4 v, int r, int k, float iy) {     // what the row is still owed joins it
+        const float4 y = *reinterpret_cast<const float4*>(a.add_y + (long long)r * a.ld_add + k), aw = *reinterpret_cast<const float4*>(a.add_w + k);
+        v.x = fmaf(y.x * iy, aw.x, v.x); v.y = fmaf(y.y * iy, aw.y, v.y); v.z = fmaf(y.z * iy, aw.z, v.z); v.w = fmaf(y.w * iy, aw.w, v.w);
+        return v;
+    };
+    // (threads tid, tid + 64, ... of that workgroup are this wave's lanes one after the other; their waves' sums join as block_sum joins them)
+    auto sum_of = [&](auto&& at) {
+        float part[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float s = 0.0f;
+            for (int k = 4 * (lane + 64 * q); k < a.K; k += 1024) {
+                const float4 v = at(k);
+                s = fmaf(v.x, v.x, s); s = fmaf(v.y, v.y, s); s = fmaf(v.z, v.z, s); s = fmaf(v.w, v.w, s);
             }
-            float* y = a.Y + (long long)r * a.ldy + n0 + i;
-            *y = a.accumulate ? *y + t : activate(t, a.act, a.glu_limit);
+            part[q] = wave_sum(s);
         }
+        return ((part[0] + part[1]) + part[2]) + part[3];
+    };
+    if (ADD || a.norm_w)
+        for (int j = wave; j < live; j += 4) {
+            const int r = r0 + j;
+            const float* x = x_of(r);
+            float iy = 0.0f, inv = 1.0f;
+            if constexpr (ADD) iy = a.add_mult / sqrtf(sum_of([&](int k) { return *reinterpret_cast<const float4*>(a.add_y + (long long)r * a.ld_add + k); }) / (float)a.K + a.add_eps);
+            if (a.norm_w)
+                inv = 1.0f / sqrtf(sum_of([&](int k) {
+                          const float4 v = *reinterpret_cast<const float4*>(x + k);
+                          return ADD ? owed(v, r, k, iy) : v;
+                      }) / (float)a.K + a.norm_eps);
+            if (lane == 0) { scale[0][j] = inv; scale[1][j] = iy; }
+        }
+    float s[R][RW] = {};
+    float4 ahead[R];                                        // the next stage's columns of the rows, four a thread
+    auto fetch = [&](int k0) {
+        const int k = k0 + 4 * tid;
+        if (k < a.K)
+#pragma unroll
+            for (int j = 0; j < R; ++j) ahead[j] = *reinterpret_cast<const float4*>(x_of(r0 + min(j, live - 1)) + k);
+    };
+    auto stage = [&](int k0) {                              // `ahead` into LDS, finished; the stage behind it requested
+        __syncthreads();
+        const int k = k0 + 4 * tid;
+        if (k < a.K) {
+            const float4 nw = a.norm_w ? *reinterpret_cast<const float4*>(a.norm_w + k) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const int r = r0 + min(j, live - 1);
+                float4 v = ahead[j];
+                if constexpr (ADD) {
+                    v = owed(v, r, k, scale[1][min(j, live - 1)]);
+                    if (blockIdx.x == 0 && j < live) *reinterpret_cast<float4*>(a.x_out + (long long)r * a.ldxo + k) = v;
+                }
+                if (a.norm_w) {
+                    const float inv = scale[0][min(j, live - 1)];
+                    v.x = v.x * inv * (a.norm_offset + nw.x); v.y = v.y * inv * (a.norm_offset + nw.y); v.z = v.z * inv * (a.norm_offset + nw.z); v.w = v.w * inv * (a.norm_offset + nw.w);
+                }
+                *reinterpret_cast<float4*>(xs + j * kRowsStage + 4 * tid) = v;
+            }
+        }
+        __syncthreads();
+        fetch(k0 + kRowsStage);
+    };
+    fetch(0);
+    __syncthreads();
+    const int pieces = (a.K + 511) / 512;
+    for (int p0 = 0; p0 < pieces; p0 += D)
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const int p = p0 + d, k = p * 512 + lane * 8;
+            if (p >= pieces) break;                         // (uniform)
+            if (d % 2 == 0) stage(p * 512);
+            if (k < a.K) {
+                float wv[RW][8];
+#pragma unroll
+                for (int i = 0; i < RW; ++i) {
+                    if constexpr (sizeof(WT) == 2) {
+                        const uint32_t uu[4] = {ring[d][i][0].x, ring[d][i][0].y, ring[d][i][0].z, ring[d][i][0].w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) { wv[i][2 * e] = __uint_as_float(uu[e] << 16); wv[i][2 * e + 1] = __uint_as_float(uu[e] & 0xffff0000u); }
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            wv[i][4 * q] = __uint_as_float(ring[d][i][q].x); wv[i][4 * q + 1] = __uint_as_float(ring[d][i][q].y);
+                            wv[i][4 * q + 2] = __uint_as_float(ring[d][i][q].z); wv[i][4 * q + 3] = __uint_as_float(ring[d][i][q].w);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    const float* xj = xs + j * kRowsStage + (d & 1) * 512 + lane * 8;
+                    const float4 x0 = *reinterpret_cast<const float4*>(xj), x1 = *reinterpret_cast<const float4*>(xj + 4);
+                    const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+                    for (int i = 0; i < RW; ++i)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) s[j][i] = fmaf(wv[i][e], xv[e], s[j][i]);
+                }
+            }
+            request(d, p + D);
+        }
+    if (n0 >= n_out) return;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+#pragma unroll
+        for (int i = 0; i < RW; ++i) s[j][i] = wave_sum_lane63(s[j][i]);
+        if (lane == 63 && j < live) leave_outputs<RW, GLU>(a, s[j], r0 + j, n0, n_out);
     }
 }
 
@@ -479,12 +628,52 @@ static void launch_moe_few(const MoeFewArgs& a, int T, bool glu, hipStream_t s) 
     hipLaunchKernelGGL((moe_few_down_kernel<WT, 3>), dim3((a.n + kDownRows - 1) / kDownRows, T), dim3(256), 0, s, a);
 }
 
+// Which launches of 2 .. 8 rows read their weights once.  The other form's rows run side by side while a few workgroups a CU hold them all (2048 outputs of bf16 up to five rows), and a norm is
+// formed there by a workgroup, here by a wave; what is saved are the weights' further passes, of which bf16 has half.  us, a workgroup a row / this, rows 2, 4, 8: bf16 2048 x 2048 5.3 / 4.6,
+// 5.5 / 5.6, 9.0 / 7.7; 6144 x 2048 8.0 / 7.4, 14.6 / 9.2, 25 / 12; behind a norm 9.2 / 9.0, 15.7 / 10.9, 28 / 15; 2048 x 2048 behind one 5.8 / 6.3, 6.4 / 7.6, 10.3 / 11.0; float32 2048 x 2048 8.1 / 6.2,
+// 13.2 / 7.3, 23 / 9.6, behind a norm and a sum 9.8 / 10.2, 14.1 / 12.0, 24 / 18; gated units with both, bf16 1408 x 2048 7.5 / 9.7, 8.8 / 11.7, 12 / 19, 7488 x 2048 27 / 24, 44 / 29, 81 / 46;
+// float32 10.8 / 12.5, 18 / 15, 31 / 22 and 48 / 36, 91 / 42, 171 / 57.
+template <typename WT, bool ADD>
+static bool rows_share_weights(const DenseArgs& a, int rows) {
+    if (rows < 2 || !a.vec || !a.xvec || a.offsets) return false;
+    const long long n = a.glu_ff > 0 ? a.glu_ff : a.N, size = n * a.K;
+    if constexpr (sizeof(WT) == 2) {
+        if (a.glu_ff > 0) return n >= 4096 && size >= 8LL << 20;
+        return size >= 4LL << 20 && n * rows >= (size >= 8LL << 20 ? 12288 : 16384) && (n >= 4096 || !(ADD || a.norm_w));
+    }
+    if (a.glu_ff > 0) return size >= 2800000 && (rows >= 3 || n >= 4096);
+    if constexpr (ADD) return size >= 4LL << 20 && (rows >= 4 || n >= 4096);
+    return size >= (a.norm_w ? 2LL << 20 : 1LL << 20);
+}
+
 template <typename WT, bool ADD>
 static void launch_gemv(const DenseArgs& a, int rows, hipStream_t s) {
     const size_t lds = ((size_t)a.K * 4 + 15) & ~(size_t)15;
     // Rows per wave, measured over layer-like shapes (2048 .. 64000 outputs of 768 .. 4096 inputs, 1 .. 6 activation rows): two rows per wave are
     // the best or within noise everywhere from 4096 outputs x rows on (a 64000 x 4096 head: 84 us against 98 with one or eight), one below; launches
     // under ~20 MB sit at 4 - 6 us whatever the choice.  The GLU form keeps pairs: 4 pairs per wave for the large expert launches.
+    if (rows_share_weights<WT, ADD>(a, rows)) {
+        auto go = [&](auto rw, auto glu, auto r) {
+            constexpr int RW = decltype(rw)::value, R = decltype(r)::value;
+            constexpr bool GLU = decltype(glu)::value;
+            const int n = GLU ? a.glu_ff : a.N, out = 4 * (GLU ? RW / 2 : RW);
+            hipLaunchKernelGGL((dense_gemv_rows_kernel<WT, RW, GLU, ADD, R>), dim3((n + out - 1) / out, (rows + R - 1) / R), dim3(256), (size_t)R * kRowsStage * 4, s, a);
+        };
+        using Yes = std::true_type; using No = std::false_type;
+        using C1 = std::integral_constant<int, 1>; using C2 = std::integral_constant<int, 2>; using C4 = std::integral_constant<int, 4>;
+        auto pick = [&](auto r) {
+            if (a.glu_ff >= 4096) go(C4{}, Yes{}, r);
+            else if (a.glu_ff > 0) go(C2{}, Yes{}, r);
+            else if (a.N >= 4096) go(C2{}, No{}, r);
+            else go(C1{}, No{}, r);
+        };
+        if (rows == 2) pick(C2{});
+        else if (rows == 3) pick(std::integral_constant<int, 3>{});
+        else if (rows == 4) pick(C4{});
+        else if (rows <= 6) pick(std::integral_constant<int, 6>{});
+        else pick(std::integral_constant<int, 8>{});
+        return;
+    }
     const long long work = (long long)a.N * rows;
     int rw = work >= 4096 ? 2 : 1;
     if (const int force = NTK_TUNE_ENV_INT("NTK_DENSE_GEMV_RW", 0)) rw = force;   // (tuning builds only)

@@ -1,0 +1,51 @@
+"""A few activation rows over weights read once (dense_gemv_rows_kernel): every row holds the bits that it has alone."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from ntransformer_amd import layers as Lr
+from ntransformer_amd.ops import DeviceBuffer as DB
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(g, dtype, shape):
+    w = (g.standard_normal(shape) / np.sqrt(shape[-1])).astype(np.float32)
+    return (w.view(np.uint32) >> 16).astype(np.uint16) if dtype == "bf16" else w
+
+
+# rows of each of the three forms and their remainders; columns of less than a piece a lane, of a stage and of several with a remainder; outputs past the waves' rows
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("T,N,K,kind", [(2, 6148, 2048, "plain"), (3, 4100, 1032, "plain"), (4, 4100, 1040, "norm"), (5, 4099, 1032, "add"), (8, 1601, 7488, "plain"), (7, 4097, 5128, "add"), (8, 6000, 1544, "norm"),
+                                        (2, 4099, 2056, "glu"), (6, 4200, 2048, "glu"), (8, 700, 4608, "glu"), (3, 4164, 2048, "accumulate"), (5, 2500, 2048, "rows"), (8, 40, 512, "norm")])
+def test_rows_hold_the_bits_of_one(dtype, T, N, K, kind):
+    L, g = Lr._bind(), np.random.default_rng(T + N + K)
+    n = 2 * N if kind == "glu" else N
+    W, nw, aw = DB.from_numpy(_weights(g, dtype, (n, K))), DB.from_numpy((0.1 * g.standard_normal(K)).astype(np.float32)), DB.from_numpy(g.standard_normal(K).astype(np.float32))
+    x, y = g.standard_normal((T, K)).astype(np.float32), g.standard_normal((T, K)).astype(np.float32)
+    xb, yb, y0 = DB.from_numpy(x), DB.from_numpy(y), g.standard_normal((T, N)).astype(np.float32)
+    pick = DB.from_numpy(np.arange(T, dtype=np.int32)[::-1].copy() * 2)
+
+    def run(first, count, out, keep):
+        d = Lr.DenseDesc()
+        d.Y, d.ldy, d.X, d.ldx, d.W, d.wdtype, d.T, d.N, d.K = out.ptr + 4 * first * N, N, xb.ptr + (0 if kind == "rows" else 4 * first * K), K, W.ptr, Lr.DT_BF16 if dtype == "bf16" else Lr.DT_F32, count, n, K
+        if kind in ("norm", "add", "glu"):
+            d.norm_w, d.norm_eps, d.norm_offset = nw.ptr, 1e-5, 1.0
+        if kind == "add":
+            d.add_y, d.ld_add, d.add_w, d.add_eps, d.add_mult, d.x_out, d.ldxo = yb.ptr + 4 * first * K, K, aw.ptr, 1e-5, 0.7, keep.ptr + 4 * first * K, K
+        if kind == "glu":
+            d.glu_ff, d.glu_limit, d.glu_alpha, d.glu_up_offset = N, 3e38, 1.0, 0.0
+        if kind == "accumulate":
+            d.accumulate = 1
+        if kind == "rows":
+            d.rows, d.row_div = pick.ptr + 4 * first, 2
+        Lr.check(L.ntk_dense(C.byref(d), None), "dense")
+
+    all_, one, k0, k1 = DB.from_numpy(y0), DB.from_numpy(y0), DB.zeros(T * K * 4), DB.zeros(T * K * 4)
+    run(0, T, all_, k0)
+    for t in range(T):
+        run(t, 1, one, k1)
+    a, b = all_.numpy(np.float32), one.numpy(np.float32)
+    assert np.isfinite(a).all() and np.array_equal(a, b)
+    assert np.array_equal(k0.numpy(np.float32), k1.numpy(np.float32))
