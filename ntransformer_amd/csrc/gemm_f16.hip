@@ -2588,12 +2588,15 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
         return n;
     };
     // two chunks (128 tokens) per workgroup when that still gives every CU two workgroups -- directly, or (narrow matrices: the 8B down /
-    // o / Q|K|V projections at 1024 tokens) with K split in two
+    // o / Q|K|V projections at 1024 tokens) with K split in two.  From six chunks on three workgroups for two CUs are enough, and K may go in four: us, six layers of the 8B shape, one chunk a
+    // workgroup there / two, 330 tokens Q8_0 3200 / 3085, Q4_K_M 3190 / 3130; 400 3650 / 3452, 3710 / 3580; 600 4771 / 4690, 4890 / 4830; 800 5930 / 5655, 6150 / 5970; two layers of the 70B shape,
+    // 700 tokens Q8_0 3980 / 3850.  With two chunks the same cost 8B Q4_K_M 1.5 %, with five 0.5 %.
     int nsplit = splits_for(chunks64);
     bool cw2 = false;
     if (CW2_OK && al && rt == 2 && chunks64 >= 2 && force_cw != 1) {
         const int pairs = (chunks64 + 1) / 2, n2 = splits_for(pairs);
-        if ((n2 <= 2 && (long)p.row_wgs * pairs * n2 >= 512) || force_cw == 2) { cw2 = true; nsplit = n2; p.chunks = pairs; }
+        const bool wide = chunks64 > 5;
+        if ((n2 <= (wide ? 4 : 2) && (long)p.row_wgs * pairs * n2 >= (wide ? 384 : 512)) || force_cw == 2) { cw2 = true; nsplit = n2; p.chunks = pairs; }
     }
     const int tps = (trips + nsplit - 1) / nsplit;   // trips per split
     nsplit = (trips + tps - 1) / tps;                // no empty split
