@@ -90,3 +90,10 @@ def test_gguf_prompts(mix, T):
         e.close()
         out.append(np.stack(lg))
     assert np.isfinite(out[0]).all() and rel(out[0], out[1]) < 1e-3
+
+
+@pytest.mark.parametrize("mix", ["Q6_K", "Q4_K_M", "Q8_0"])
+@pytest.mark.parametrize("T", [16, 17])
+def test_gguf_prompts_beside_the_short_form(mix, T):
+    """(formats that layers_short takes up to 16 tokens only; 1e-3 as above)"""
+    test_gguf_prompts(mix, T)
