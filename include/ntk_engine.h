@@ -27,6 +27,9 @@ int ntk_rope_kv_store(float* q, const float* k, const float* v, const int* posit
  * the sums in split order, then the same; the rotated q goes to q, k and v are not stored outside the caches */
 int ntk_reduce_rope_kv_store(float* q, const float* const* sums, const int* splits, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim, float theta_base,
                              float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream);
+/* ... from pieces of query, key and value side by side: [splits][seq_len][n_heads + 2 n_kv_heads][head_dim] */
+int ntk_reduce_rope_kv_store_joined(float* q, const float* sums, int splits, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim, float theta_base, float freq_scale,
+                                    int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream);
 /* ---------------------------------------------------------------------------------------------
  * Engine-level fused operators (no reference counterpart; they compute exactly what the listed
  * sequence of reference launchers computes, in fewer launches, with device-resident positions so a
@@ -273,12 +276,12 @@ size_t ntk_gemm_half_many_bytes(int n_tokens, int in_features);
 int ntk_gemm_half_many(const ntk_half_desc* d, void* stream);
 /* ... with a norm between two of them and no row in between.  ntk_gemm_half_defer: ntk_gemm_half with accumulate that may leave its pieces of K to the launch behind it (partials: as those of
  * ntk_gemm_quant_f16; they lie in the workspace).  ntk_half_norm_split: hidden += that projection (partials; NULL: hidden as it lies), and the halves of its RMSNorm into `workspace` (another one), from
- * which ntk_gemm_half_normed is ntk_gemm_half_many (X, row_max not looked at).  ntk_half_norm_takes: 1 where the workspace holds all tokens (width a multiple of 64, up to 16384), else 0. */
+ * which ntk_gemm_half_normed is ntk_gemm_half_many (X, row_max not looked at; no unit's sums are left).  ntk_half_norm_takes: 1 where the workspace holds all tokens (width a multiple of 64, up to 16384), else 0. */
 int ntk_gemm_half_defer(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, const float* row_max, void* workspace, size_t workspace_bytes,
                         ntk_gemm_partials* partials, void* stream);
 int ntk_half_norm_takes(int n_tokens, int width, size_t workspace_bytes);
 int ntk_half_norm_split(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int width, float eps, void* workspace, size_t workspace_bytes, void* stream);
-int ntk_gemm_half_normed(const ntk_half_desc* d, void* stream);
+int ntk_gemm_half_normed(const ntk_half_desc* d, ntk_gemm_partials* partials, void* stream);      /* partials (or NULL): several matrices' pieces left as those of one of all their rows */
 
 /* Dequantise rows of a (quantised) embedding table on the device: out[t,:] = table[tokens[t],:].
  * Same arithmetic as the host loop in reference src/model/transformer.cpp:419-599; Q5_K is zero-filled

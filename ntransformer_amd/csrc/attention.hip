@@ -765,9 +765,10 @@ __global__ __launch_bounds__(256) void rope_kv_store_rows_kernel(float* __restri
 }
 
 // ... and the same from the projections' partial sums (ntk_gemm_partials): the splits are added here, in order, in the place of a launch that writes their sums
-// for this one to read back.  A short prompt takes a workgroup per 256 pairs of a token, everything requested ahead of the angles; a long one a workgroup per token with one
+// for this one to read back.  A short prompt takes a workgroup per 256 pairs of a token, everything requested ahead of the angles; a long one four workgroups per token, each with a
 // table of them.  16 tokens of the 8B shapes: 4.7 + 4.6 us as two launches, 4.0 as one; 1003 tokens 12.1 + 11.8 us, 17 - 18 as one.
-struct RopeSource { const float* p; int n; size_t plane; };
+// (A long prompt's token in four workgroups, each with the table, instead of one: a pass of 65 tokens through six layers 1746 -> 1690 us, 200 tokens 2450 -> 2400, 1000 the same.)
+struct RopeSource { const float* p; int n; size_t plane; int ld; };     // pieces `plane` apart, a token's values ld apart
 template <int N>
 __device__ __forceinline__ void rope_sums(const RopeSource& s, const size_t (&at)[N], float (&v)[N]) {
 #pragma unroll
@@ -809,7 +810,7 @@ __global__ __launch_bounds__(256) void rope_kv_store_parts_kernel(float* __restr
         const int pair = idx % half_dim, head = idx / half_dim;
         const int i0 = interleaved ? 2 * pair : pair, i1 = interleaved ? 2 * pair + 1 : pair + half_dim;
         const bool query = head < n_heads;
-        const size_t base = query ? ((size_t)sp * n_heads + head) * head_dim : ((size_t)sp * n_kv_heads + (head - n_heads)) * head_dim;
+        const size_t base = query ? (size_t)sp * sq.ld + head * head_dim : (size_t)sp * sk.ld + (head - n_heads) * head_dim;
         const size_t at[2] = {base + i0, base + i1};
         float v[2], c, s, ra, rb;
         if (query) rope_sums(sq, at, v);
@@ -817,7 +818,7 @@ __global__ __launch_bounds__(256) void rope_kv_store_parts_kernel(float* __restr
         if constexpr (TABLE) { c = cs[0][pair]; s = cs[1][pair]; }
         else angle_of(pair, c, s);
         rope_rotate(v[0], v[1], c, s, ra, rb);
-        if (query) { q[at[0]] = ra; q[at[1]] = rb; }
+        if (query) { float* out = q + ((size_t)sp * n_heads + head) * head_dim; out[i0] = ra; out[i1] = rb; }
         else if (store) {
             uint16_t* row = kc + (size_t)cp * per_pos + (size_t)(head - n_heads) * head_dim;
             row[i0] = f2h(ra);
@@ -826,7 +827,7 @@ __global__ __launch_bounds__(256) void rope_kv_store_parts_kernel(float* __restr
     }
     if (store)
         for (int e = first; e < per_pos; e += stride) {
-            const size_t at[1] = {(size_t)sp * per_pos + e};
+            const size_t at[1] = {(size_t)sp * sv.ld + e};
             float v[1];
             rope_sums(sv, at, v);
             vc[(size_t)cp * per_pos + e] = f2h(v[0]);
@@ -931,14 +932,29 @@ int ntk_rope_kv_store(float* q, const float* k, const float* v, const int* posit
     return ntk::last_launch_status();
 }
 
+static int reduce_rope(float* q, const ntk::RopeSource& sq, const ntk::RopeSource& sk, const ntk::RopeSource& sv, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim,
+                       float theta_base, float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream);
 int ntk_reduce_rope_kv_store(float* q, const float* const* sums, const int* splits, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim, float theta_base,
                              float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream) {
     if (!q || !sums || !splits || !sums[0] || !sums[1] || !sums[2] || !positions || !k_cache || !v_cache) return NTK_E_NULL;
     if (seq_len < 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim <= 0 || (head_dim & 1) || head_dim > 256 || start_pos < 0 || max_seq <= 0) return NTK_E_SHAPE;
     if (splits[0] < 1 || splits[1] < 1 || splits[2] < 1) return NTK_E_SHAPE;
     if (seq_len == 0) return NTK_OK;
-    const size_t nq = (size_t)seq_len * n_heads * head_dim, nk = (size_t)seq_len * n_kv_heads * head_dim;
-    const ntk::RopeSource sq{sums[0], splits[0], nq}, sk{sums[1], splits[1], nk}, sv{sums[2], splits[2], nk};
+    const int nq = n_heads * head_dim, nk = n_kv_heads * head_dim;
+    const ntk::RopeSource sq{sums[0], splits[0], (size_t)seq_len * nq, nq}, sk{sums[1], splits[1], (size_t)seq_len * nk, nk}, sv{sums[2], splits[2], (size_t)seq_len * nk, nk};
+    return reduce_rope(q, sq, sk, sv, positions, seq_len, n_heads, n_kv_heads, head_dim, theta_base, freq_scale, interleaved, k_cache, v_cache, start_pos, max_seq, stream);
+}
+int ntk_reduce_rope_kv_store_joined(float* q, const float* sums, int splits, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim, float theta_base, float freq_scale,
+                                    int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream) {
+    if (!q || !sums || !positions || !k_cache || !v_cache) return NTK_E_NULL;
+    if (seq_len < 0 || n_heads <= 0 || n_kv_heads <= 0 || head_dim <= 0 || (head_dim & 1) || head_dim > 256 || start_pos < 0 || max_seq <= 0 || splits < 1) return NTK_E_SHAPE;
+    if (seq_len == 0) return NTK_OK;
+    const int nq = n_heads * head_dim, nk = n_kv_heads * head_dim, all = nq + 2 * nk;
+    auto at = [&](int col) { return ntk::RopeSource{sums + col, splits, (size_t)seq_len * all, all}; };
+    return reduce_rope(q, at(0), at(nq), at(nq + nk), positions, seq_len, n_heads, n_kv_heads, head_dim, theta_base, freq_scale, interleaved, k_cache, v_cache, start_pos, max_seq, stream);
+}
+static int reduce_rope(float* q, const ntk::RopeSource& sq, const ntk::RopeSource& sk, const ntk::RopeSource& sv, const int* positions, int seq_len, int n_heads, int n_kv_heads, int head_dim,
+                       float theta_base, float freq_scale, int interleaved, void* k_cache, void* v_cache, int start_pos, int max_seq, void* stream) {
     hipStream_t s = ntk::resolve_stream(stream);
     uint16_t *kc = static_cast<uint16_t*>(k_cache), *vc = static_cast<uint16_t*>(v_cache);
     if (seq_len <= 64) {
@@ -946,7 +962,7 @@ int ntk_reduce_rope_kv_store(float* q, const float* const* sums, const int* spli
         hipLaunchKernelGGL(ntk::rope_kv_store_parts_kernel<false>, dim3(seq_len, parts), dim3(256), 0, s, q, sq, sk, sv, positions, n_heads, n_kv_heads, head_dim, theta_base, freq_scale,
                            interleaved, kc, vc, start_pos, max_seq);
     } else
-        hipLaunchKernelGGL(ntk::rope_kv_store_parts_kernel<true>, dim3(seq_len), dim3(256), 0, s, q, sq, sk, sv, positions, n_heads, n_kv_heads, head_dim, theta_base, freq_scale, interleaved,
+        hipLaunchKernelGGL(ntk::rope_kv_store_parts_kernel<true>, dim3(seq_len, 4), dim3(256), 0, s, q, sq, sk, sv, positions, n_heads, n_kv_heads, head_dim, theta_base, freq_scale, interleaved,
                            kc, vc, start_pos, max_seq);
     return ntk::last_launch_status();
 }

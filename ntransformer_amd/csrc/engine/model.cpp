@@ -885,7 +885,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         return true;
     };
     // several of them over one X in one launch (silu: gate and up, Y[0] = silu(gate) * up); false: not such matrices, nothing was launched
-    auto project_half_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, bool silu) -> bool {
+    auto project_half_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, bool silu, ntk_gemm_partials* joined = nullptr) -> bool {     // joined: the pieces of a product over ready halves may be left there
         ntk_half_desc d{};
         for (int i = 0; i < n; ++i) {
             if (!batched || !bf16_now || !Ws[i]->ptr || Ws[i]->dtype != NTK_DT_F16 || Ws[i]->in_f < 3072 || Ws[i]->in_f != Ws[0]->in_f) return false;
@@ -896,7 +896,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         const bool own = ws != nullptr;
         d.n = n; d.X = X; d.n_tokens = T; d.in_features = (int)Ws[0]->in_f; d.row_max = rm; d.silu = silu ? 1 : 0;
         d.workspace = own ? ws : cur_ws; d.workspace_bytes = gemm_ws_bytes_;
-        const int st = ready ? ntk_gemm_half_normed(&d, s) : ntk_gemm_half_many(&d, s);
+        const int st = ready ? ntk_gemm_half_normed(&d, joined, s) : ntk_gemm_half_many(&d, s);
         if (st == NTK_E_SHAPE || st == NTK_E_ALIGN) return false;
         if (!own) planes_of = nullptr;
         ok(st);
@@ -931,9 +931,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
     };
     // matrices that share X (Q | K | V, gate | up): those of one format go out as ONE launch of the FP16 GEMM, the rest one by one, ahead of them.  sums / splits: the LAST launch may
     // leave the partial sums of its K splits to the consumer (its matrices' places in the two are then set; a launch behind it would overwrite them)
-    auto project_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, const float** sums = nullptr, int* splits = nullptr) {
+    auto project_many = [&](float* const* Ys, const DevTensor* const* Ws, int n, const float* X, const float* rm, const float** sums = nullptr, int* splits = nullptr, ntk_gemm_partials* joined = nullptr) {
         bool done[3] = {false, false, false};
-        if (project_half_many(Ys, Ws, n, X, rm, false)) return;
+        if (project_half_many(Ys, Ws, n, X, rm, false, joined)) return;
         struct Group { int idx[3], m; } groups[3];
         int n_groups = 0;
         if (batched && bf16_now)
@@ -1091,13 +1091,17 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         const bool one_launch = with_max && T >= 4 && hd <= 256;
         const float* sums[3] = {q_buf, k_buf, v_buf};     // what the rotation reads: the projections, or the partial sums of the last launch's
         int splits[3] = {1, 1, 1};
+        ntk_gemm_partials joined{};                       // (or of all three side by side)
         {
             float* const ys[3] = {q_buf, k_buf, v_buf};
             const DevTensor* const ws[3] = {&L.wq, &L.wk, &L.wv};
-            project_many(ys, ws, 3, residual_, max_a, one_launch ? sums : nullptr, splits);
+            project_many(ys, ws, 3, residual_, max_a, one_launch ? sums : nullptr, splits, one_launch ? &joined : nullptr);
         }
         if (one_launch) {                            // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
-            if (splits[0] + splits[1] + splits[2] > 3)
+            if (joined.part[0])
+                ok(ntk_reduce_rope_kv_store_joined(q_buf, joined.part[0], joined.nsplit, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos,
+                                                   cfg_.max_seq_len, s));
+            else if (splits[0] + splits[1] + splits[2] > 3)
                 ok(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
             else
                 ok(ntk_rope_kv_store(q_buf, k_buf, v_buf, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc,

@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256) void gemm_direct_sum_kernel(const DirectArgs d
 }
 
 template <class P, int TM, int TN, int WM, int WN, int STAGES, int GLU, int MINW>
-static int launch_direct(DirectArgs d, int splits, hipStream_t s, bool sum = true) {      // (as launch_tiles; sum false: one matrix)
+static int launch_direct(DirectArgs d, int splits, hipStream_t s, bool sum = true) {      // (as launch_tiles; without the sum several matrices' pieces lie as those of one of all their rows)
     constexpr int BK = 128 / (int)sizeof(typename P::WT);
     const int chunks = d.t.K / BK, per = (chunks + splits - 1) / splits;
     d.t.k_per_split = per * BK;

@@ -221,7 +221,7 @@ static int half_many(const ntk_half_desc* d, bool ready, ntk_gemm_partials* defe
         a.n_seg = d->n;
         for (int i = 0; i < d->n; ++i) { a.segW[i] = d->W[i]; a.segY[i] = d->Y[i] + (long long)t0 * d->out[i]; a.seg_out[i] = d->out[i]; }
         const int splits = launch_direct_half<kGluNone>(a, p, s, !defer);
-        if (defer) leave(defer, d->Y[0], d->out[0], T, splits, t.part);
+        if (defer) leave(defer, d->Y[0], (int)N, T, splits, t.part);
     }
     return last_launch_status();
 }
@@ -251,7 +251,10 @@ int ntk_half_norm_split(float* hidden, const ntk_gemm_partials* q, const float* 
     else hipLaunchKernelGGL(half_norm_split_kernel<2>, dim3(n_tokens), dim3(threads), 0, resolve_stream(stream), a);
     return last_launch_status();
 }
-int ntk_gemm_half_normed(const ntk_half_desc* d, void* stream) { return half_many(d, true, nullptr, stream); }
+int ntk_gemm_half_normed(const ntk_half_desc* d, ntk_gemm_partials* partials, void* stream) {
+    if (d && d->silu && partials) return NTK_E_SHAPE;
+    return half_many(d, true, partials, stream);
+}
 
 size_t ntk_gemm_half_workspace_bytes(int n_tokens) { return ((size_t)(n_tokens > 0 ? n_tokens : 0) * sizeof(float) + 15) & ~(size_t)15; }
 

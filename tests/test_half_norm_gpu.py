@@ -24,7 +24,7 @@ def _bind():
     L.ntk_half_norm_takes.argtypes = [I, I, Z]
     L.ntk_half_norm_split.argtypes = [VP, P, VP, I, I, F, VP, Z, VP]
     L.ntk_rmsnorm.argtypes = [VP, VP, VP, I, I, F, VP]
-    L.ntk_gemm_half_many.argtypes = L.ntk_gemm_half_normed.argtypes = [C.POINTER(HalfDesc), VP]
+    L.ntk_gemm_half_many.argtypes, L.ntk_gemm_half_normed.argtypes = [C.POINTER(HalfDesc), VP], [C.POINTER(HalfDesc), P, VP]
     return L
 
 
@@ -40,12 +40,12 @@ def test_norm_over_deferred_pieces(T, H, K):
     xb, n = DB.from_numpy(x), 4 * T * (max(H, K) + 1) + 64 + 16 * T * H * 4
     a, b = DB.zeros(n), DB.zeros(n)
 
-    def product(call, X):
+    def product(call, X, *left):
         d, ys = HalfDesc(), [DB.zeros(T * o * 4) for o in outs]
         for i, o in enumerate(outs):
             d.W[i], d.Y[i], d.out[i] = U[i].ptr, ys[i].ptr, o
         d.n, d.X, d.n_tokens, d.in_features, d.workspace, d.workspace_bytes = 2, X.ptr, T, H, b.ptr, n
-        _lib.check(call(C.byref(d), None), "product")
+        _lib.check(call(C.byref(d), *left, None), "product")
         return [y.numpy(np.float32) for y in ys]
 
     one, norm = DB.from_numpy(h0), DB.zeros(T * H * 4)
@@ -57,10 +57,19 @@ def test_norm_over_deferred_pieces(T, H, K):
     _lib.check(L.ntk_gemm_half_defer(hid.ptr, W.ptr, xb.ptr, T, H, K, None, a.ptr, n, C.byref(p), None), "defer")
     assert p.n_tokens == T and p.rows[0] == H and p.y[0] == hid.ptr and (p.nsplit > 1) == bool(p.part[0])
     _lib.check(L.ntk_half_norm_split(hid.ptr, C.byref(p), nw.ptr, T, H, 1e-5, b.ptr, n, None), "norm_split")
-    got = product(L.ntk_gemm_half_normed, xb)
+    got = product(L.ntk_gemm_half_normed, xb, None)
     assert np.array_equal(hid.numpy(np.float32), one.numpy(np.float32))
     _lib.check(L.ntk_half_norm_split(hid.ptr, None, nw.ptr, T, H, 1e-5, b.ptr, n, None), "norm_split")
-    again = product(L.ntk_gemm_half_normed, xb)
+    again = product(L.ntk_gemm_half_normed, xb, None)
+    left = _lib.GemmPartials()
+    product(L.ntk_gemm_half_normed, xb, C.byref(left))
+    if left.nsplit > 1:                                                     # the matrices' pieces side by side, in the order that their sums take
+        at = left.part[0] - b.ptr
+        pieces = b.numpy(np.uint8)[at:at + 4 * left.nsplit * T * sum(outs)].view(np.float32).reshape(left.nsplit, T, sum(outs))
+        tot = pieces[0]
+        for u in range(1, left.nsplit):
+            tot = tot + pieces[u]
+        assert np.array_equal(tot[:, :outs[0]].reshape(-1), got[0]) and np.array_equal(tot[:, outs[0]:].reshape(-1), got[1])
     for w, q, r in zip(want, got, again):
         # the rows' norms differ by their sums' order alone: at most 2^-24 sqrt(H) / 2 of a value and the halves' 2^-23, near 1e-6 of the results' size
         assert np.isfinite(q).all() and np.abs(q - w).max() <= 4e-6 * max(np.abs(w).max(), 1e-3)
