@@ -257,6 +257,8 @@ size_t ntk_gemm_half_workspace_bytes(int n_tokens);
 int ntk_gemm_half(float* Y, const void* W, const float* X, int n_tokens, int out_features, int in_features, int accumulate, const float* row_max, void* workspace,
                   size_t workspace_bytes, void* stream);
 
+/* y_i (+)= W_i . x of one to three matrices of F16 or of F32 rows in one launch, each product with ntk_gemv's bits */
+int ntk_gemv_dense(const ntk_gemv_seg* segs, int nseg, const float* x, int in_features, int add, void* stream);
 /* Y[t] = W . X[t] of F16 or F32 rows in one launch, each product with ntk_gemv's bits.  in_features a multiple of 8, 16-byte aligned W and X (NTK_E_ALIGN: nothing was launched). */
 int ntk_gemv_tokens(float* y, const void* W, const float* x, int n_tokens, int out_features, int in_features, int weight_dtype, void* stream);
 

@@ -1396,14 +1396,26 @@ int Model::enqueue_layers(int first, int last_layer) {
                 if (st != NTK_E_DTYPE && st != NTK_E_ALIGN && st != NTK_E_SHAPE) return st;
             }
         }
+        const float* normed = nullptr;   // norm(x) for the matrices that do not form it themselves
         for (int a = 0; a < n; ++a) {
             if (done[a]) continue;
             const DevTensor& w = *ws[a];
             if (!is_quant(w.dtype)) {
                 const float* xin = x;
                 if (nw) {
-                    NT_TRY(ntk_rmsnorm(residual_ + H, x, nw, 1, (int)w.in_f, cfg_.norm_eps, s));
-                    xin = residual_ + H;
+                    if (!normed) NT_TRY(ntk_rmsnorm(residual_ + H, x, nw, 1, (int)w.in_f, cfg_.norm_eps, s));
+                    xin = normed = residual_ + H;
+                }
+                if ((w.dtype == NTK_DT_F16 || w.dtype == NTK_DT_F32) && w.ptr && (!resid || resid == ys[a])) {   // those of its type in one launch, a residual added where it lies
+                    ntk_gemv_seg segs[3];
+                    int m = 0;
+                    for (int b = a; b < n; ++b) {
+                        if (done[b] || ws[b]->dtype != w.dtype || ws[b]->in_f != w.in_f || !ws[b]->ptr || (resid && b != a)) continue;
+                        segs[m++] = {ws[b]->ptr, ys[b], (int)ws[b]->out_f, w.dtype};
+                        done[b] = true;
+                    }
+                    NT_TRY(ntk_gemv_dense(segs, m, xin, (int)w.in_f, resid ? 1 : 0, s));
+                    continue;
                 }
                 float* y = resid ? residual_ : ys[a];
                 raw_begin();

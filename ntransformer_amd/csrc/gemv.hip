@@ -589,15 +589,19 @@ __global__ __launch_bounds__(512, 4) void gemv_quant_pair_kernel(const GemvParam
 // Dense F16 / F32 rows (reference gemm.cu:476-671): one wave per row, 16-byte lane loads when the row
 // is aligned, scalar otherwise (the reference's own F32 test uses in = 3).  Not on any target config.
 // ------------------------------------------------------------------------------------------------
+// (up to three matrices over the same x side by side: decoding a model of such rows is a chain of launches, us a layer of the 8B shape 142 with a launch a matrix, its own norm and a launch for the residual, 111 so)
+template <typename T> struct DenseSegs { const T* W[3]; float* y[3]; int end[3]; };   // end: rows up to and with each matrix
 template <typename T, bool ADD>
-__global__ __launch_bounds__(256) void gemv_dense_kernel(float* __restrict__ y, const T* __restrict__ W,
-                                                         const float* __restrict__ x, int out, int in) {
+__global__ __launch_bounds__(256) void gemv_dense_kernel(const DenseSegs<T> d, const float* __restrict__ x, int in) {
     const int lane = threadIdx.x & 63;
     const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int nwaves = gridDim.x * (blockDim.x >> 6);
     constexpr int V = 16 / (int)sizeof(T);
+    const int out = d.end[2];
     for (int r = wave; r < out; r += nwaves) {
-        const T* w = W + (size_t)r * in;
+        const int sg = (r >= d.end[0]) + (r >= d.end[1]), row = r - (sg == 0 ? 0 : d.end[sg - 1]);     // (uniform)
+        const T* w = (sg == 0 ? d.W[0] : sg == 1 ? d.W[1] : d.W[2]) + (size_t)row * in;
+        float* y = (sg == 0 ? d.y[0] : sg == 1 ? d.y[1] : d.y[2]) + row;
         float acc = 0.0f;
         int done = 0;
         if ((reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
@@ -625,7 +629,7 @@ __global__ __launch_bounds__(256) void gemv_dense_kernel(float* __restrict__ y, 
             acc = fmaf(wv, x[i], acc);
         }
         acc = wave_sum(acc);
-        if (lane == 0) y[r] = ADD ? y[r] + acc : acc;
+        if (lane == 0) *y = ADD ? *y + acc : acc;
     }
 }
 
@@ -907,15 +911,22 @@ static int dispatch_quant(int dt, const ntk_gemv_seg* segs, int nseg, const floa
     }
 }
 
-template <bool ADD>
-static int launch_dense(float* y, const void* W, const float* x, int out, int in, int dt, hipStream_t st) {
+template <bool ADD, typename T>
+static int launch_dense_as(const ntk_gemv_seg* segs, int n, const float* x, int in, hipStream_t st) {
+    DenseSegs<T> d{};
+    long long out = 0;
+    for (int i = 0; i < 3; ++i) {
+        if (i < n) { d.W[i] = static_cast<const T*>(segs[i].W); d.y[i] = segs[i].y; out += segs[i].rows; }
+        if (out > 0x7FFFFFFFll) return NTK_E_SHAPE;
+        d.end[i] = (int)out;
+    }
     if (out == 0) return NTK_OK;
-    const int grid = std::min((out + 3) / 4, 2048);
-    if (dt == NTK_DT_F32)
-        hipLaunchKernelGGL((gemv_dense_kernel<float, ADD>), dim3(grid), dim3(256), 0, st, y, (const float*)W, x, out, in);
-    else
-        hipLaunchKernelGGL((gemv_dense_kernel<uint16_t, ADD>), dim3(grid), dim3(256), 0, st, y, (const uint16_t*)W, x, out, in);
+    hipLaunchKernelGGL((gemv_dense_kernel<T, ADD>), dim3((unsigned)std::min<long long>((out + 3) / 4, 2048)), dim3(256), 0, st, d, x, in);
     return last_launch_status();
+}
+template <bool ADD>
+static int launch_dense(const ntk_gemv_seg* segs, int n, const float* x, int in, hipStream_t st) {
+    return segs[0].dtype == NTK_DT_F32 ? launch_dense_as<ADD, float>(segs, n, x, in, st) : launch_dense_as<ADD, uint16_t>(segs, n, x, in, st);
 }
 
 }  // namespace ntk
@@ -933,7 +944,10 @@ int ntk_gemv(float* y, const void* W, const float* x, int out_features, int in_f
     if (out_features < 0 || in_features <= 0) return NTK_E_SHAPE;
     hipStream_t st = ntk::resolve_stream(stream);
     if (weight_dtype == NTK_DT_F32 || weight_dtype == NTK_DT_F16)
-        return ntk::launch_dense<false>(y, W, x, out_features, in_features, weight_dtype, st);
+    {
+        const ntk_gemv_seg one{W, y, out_features, weight_dtype};
+        return ntk::launch_dense<false>(&one, 1, x, in_features, st);
+    }
     if (!ntk::is_quant(weight_dtype)) return NTK_E_DTYPE;
     ntk_gemv_seg seg{W, y, out_features, weight_dtype};
     return ntk::dispatch_quant(weight_dtype, &seg, 1, x, in_features, nullptr, 0.0f, nullptr, 0, st);
@@ -962,7 +976,20 @@ int ntk_gemv_add(float* y, const void* W, const float* x, int out_features, int 
     if (!y || !W || !x) return NTK_E_NULL;
     if (out_features < 0 || in_features <= 0) return NTK_E_SHAPE;
     if (weight_dtype != NTK_DT_F16) return NTK_E_DTYPE;   // reference gemm.cu:861-869
-    return ntk::launch_dense<true>(y, W, x, out_features, in_features, weight_dtype, ntk::resolve_stream(stream));
+    const ntk_gemv_seg one{W, y, out_features, weight_dtype};
+    return ntk::launch_dense<true>(&one, 1, x, in_features, ntk::resolve_stream(stream));
+}
+
+int ntk_gemv_dense(const ntk_gemv_seg* segs, int nseg, const float* x, int in_features, int add, void* stream) {
+    if (!segs || !x) return NTK_E_NULL;
+    if (nseg < 1 || nseg > 3 || in_features <= 0) return NTK_E_SHAPE;
+    for (int i = 0; i < nseg; ++i) {
+        if (!segs[i].W || !segs[i].y) return NTK_E_NULL;
+        if (segs[i].rows < 0) return NTK_E_SHAPE;
+        if (segs[i].dtype != segs[0].dtype || (segs[i].dtype != NTK_DT_F32 && segs[i].dtype != NTK_DT_F16)) return NTK_E_DTYPE;
+    }
+    hipStream_t st = ntk::resolve_stream(stream);
+    return add ? ntk::launch_dense<true>(segs, nseg, x, in_features, st) : ntk::launch_dense<false>(segs, nseg, x, in_features, st);
 }
 
 #ifdef NTK_EXPERIMENTS
