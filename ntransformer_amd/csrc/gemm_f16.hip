@@ -1809,6 +1809,7 @@ struct GemmKParams {
     const uint8_t* xb;      // operand planes of the (single) chunk
     const uint8_t* aux;     // its step sums (K-quant minimum term)
     const float* group_inv; // [in / GB_GROUP][GB_SHORT]: 1 / s of a group of columns
+    int whole;              // one scale a token (planes by split_x_kernel or split_row): a slice's sums run on over its units, 1 / s at their end
     const float* ssq;       // X is to be divided by its rows' root mean squares: [nssq][GB_SHORT] sums of squares, or null
     int nssq;
     float eps;
@@ -1864,7 +1865,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
 #endif
         }
     }
-    f32x4 inv_t[NTB];   // 1 / rms of the lane's tokens where X wants it, else 1
+    f32x4 inv_t[NTB];   // 1 / rms of the lane's tokens where X wants it, 1 / s where it is the whole token's, else 1
     for (int it = 0; it < p.jobs; ++it) {
     // this wave's tile (waves past the last tile only help with the copy)
     const int tile_raw = ((int)blockIdx.x + it * (int)gridDim.x) * NW + wave;
@@ -1946,7 +1947,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
         // 28.7, in front of the first weights Q | K | V 1.3 of 10.9)
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) {
-            inv_t[tb] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+            inv_t[tb] = p.whole ? *reinterpret_cast<const f32x4*>(p.group_inv + tb * 16 + 4 * g) : f32x4{1.0f, 1.0f, 1.0f, 1.0f};
             if (p.ssq) {   // (uniform)
                 const float* src = p.ssq + tb * 16 + 4 * g;
                 f32x4 q = *reinterpret_cast<const f32x4*>(src);
@@ -1990,7 +1991,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
             for (int tb = 0; tb < NTB; ++tb) {
                 gi[tb] = ginv[tb];
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) acc[rt][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int rt = 0; rt < RT; ++rt) acc[rt][tb] = p.whole ? sum[rt][tb] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             }
             load_inv(ginv, min(u + 1, u_hi - 1));
             __builtin_amdgcn_sched_barrier(0);
@@ -2078,7 +2079,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) sum[rt][tb][e] = fmaf(acc[rt][tb][e], gi[tb][e], sum[rt][tb][e]);
+                    for (int e = 0; e < 4; ++e) sum[rt][tb][e] = p.whole ? acc[rt][tb][e] : fmaf(acc[rt][tb][e], gi[tb][e], sum[rt][tb][e]);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- this wave's rows: accumulator element e of lane (i = row of the tile, g) is token tb * 16 + 4 g + e; 1 / rms where X wants it; Y or this slice's partial sums ----
@@ -2418,7 +2419,7 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
         if (best_n > 0) {
             GemmKParams kp{};
             kp.nseg = nseg; kp.T = T; kp.in = in; kp.steps = in / 32; kp.row_bytes = (unsigned)row_bytes;
-            kp.xb = wsb; kp.aux = reinterpret_cast<const uint8_t*>(p.aux); kp.group_inv = group_inv; kp.resid = best_n == 1 ? resid : nullptr;
+            kp.xb = wsb; kp.aux = reinterpret_cast<const uint8_t*>(p.aux); kp.group_inv = group_inv; kp.whole = sh.on ? 0 : 1; kp.resid = best_n == 1 ? resid : nullptr;
             kp.nsplit = best_n; kp.units_per_split = best_ups;
             if (sh.norm) { kp.ssq = group_inv + ws_group_floats(in); kp.nssq = (in + 511) / 512; kp.eps = sh.eps; }
             float* kpart = reinterpret_cast<float*>(wsb + ws_part_offset(in)) + sh.part_at;
