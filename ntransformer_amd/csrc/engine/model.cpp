@@ -731,7 +731,7 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
         size_t at = 0;
         // from the prompt's first token on: everything between the projections in one launch
         const bool whole = start_pos == 0 && hd == 128 && nh % 2 == 0 && rope_angles_ != nullptr;
-        const bool defer = whole || T >= 4;   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
+        const bool defer = whole || (T >= 4 && hd <= 256);   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too; wider heads are turned in place)
         for (int a = 0; a < 3; ++a) {
             if (done[a]) continue;
             const DevTensor* w[3];
@@ -750,7 +750,7 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
         }
         if (whole) {
             NT_TRY(ntk_short_attention(sums, splits, rope_angles_, T, nh, nkv, hd, scale, cfg_.rope_interleaved, kc, vc, cfg_.max_seq_len, other(), s));
-        } else if (T >= 4) {
+        } else if (defer) {
             NT_TRY(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
         } else {
             NT_TRY(ntk_rope(q_buf, k_buf, positions_, 1, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, s));
