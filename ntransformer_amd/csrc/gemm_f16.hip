@@ -2365,6 +2365,22 @@ struct ShortArgs {
 };
 struct HostSeg { float* Y; const void* W; int out; };
 
+// a matrix's pieces are addressed with 32-bit offsets
+template <class D>
+static bool offsets_fit(int out, int in) {
+    if ((size_t)out * ((size_t)in / D::BW * D::BB) > 0xFFFFFF00ull) return false;
+    if constexpr (D::RP) return (size_t)(out / 16) * (size_t)(in / 256) * (size_t)D::ITEM <= 0xFFFFFFF0ull;
+    return true;
+}
+
+// (a tensor and its repack LARGER: the same slices, and the larger of the two has to fit)
+template <int DT, int LARGER>
+static int short_takes(const int* rows, int nseg, int T, int in) {
+    for (int i = 0; i < nseg; ++i)
+        if (!offsets_fit<DeqI<LARGER>>(rows[i], in)) return 0;
+    return kslice_plan<DT>(rows, nseg, T, in).n > 0;
+}
+
 // T <= GB_MAX_CHUNKS * 64 = 1024 tokens in one launch; nseg matrices [out_s][in] of one format sharing X
 template <int DT>
 static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T, int in, const float* resid, void* ws, int reuse_x,
@@ -2377,10 +2393,7 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     const size_t row_bytes = (size_t)in / D::BW * D::BB;
     long out_total = 0;
     for (int i = 0; i < nseg; ++i) {
-        if (segs[i].out <= 0 || segs[i].out % 16 != 0 || (size_t)segs[i].out * row_bytes > 0xFFFFFF00ull) return NTK_E_SHAPE;   // 32-bit piece offsets
-        if constexpr (D::RP) {
-            if ((size_t)(segs[i].out / 16) * (size_t)(in / 256) * (size_t)D::ITEM > 0xFFFFFFF0ull) return NTK_E_SHAPE;
-        }
+        if (segs[i].out <= 0 || segs[i].out % 16 != 0 || !offsets_fit<D>(segs[i].out, in)) return NTK_E_SHAPE;
         if ((reinterpret_cast<uintptr_t>(segs[i].W) & 15) || (reinterpret_cast<uintptr_t>(segs[i].Y) & 15)) return NTK_E_ALIGN;
         out_total += segs[i].out;
     }
@@ -2741,12 +2754,12 @@ int ntk_gemm_short_takes(const int* rows, int nseg, int n_tokens, int in_feature
     if (!rows || nseg < 1 || nseg > ntk::GB_MAX_SEG || n_tokens < 2 || in_features <= 0) return 0;
     for (int i = 0; i < nseg; ++i)
         if (rows[i] <= 0 || rows[i] % 16 != 0) return 0;
-    switch (dtype) {   // (a tensor and its repack: the same slices)
-        case NTK_DT_Q8_0: return ntk::kslice_plan<NTK_DT_Q8_0>(rows, nseg, n_tokens, in_features).n > 0;
-        case NTK_DT_Q4_0: return ntk::kslice_plan<NTK_DT_Q4_0>(rows, nseg, n_tokens, in_features).n > 0;
-        case NTK_DT_Q4_K: return ntk::kslice_plan<NTK_DT_Q4_K>(rows, nseg, n_tokens, in_features).n > 0;
-        case NTK_DT_Q5_K: return ntk::kslice_plan<NTK_DT_Q5_K>(rows, nseg, n_tokens, in_features).n > 0;
-        case NTK_DT_Q6_K: return ntk::kslice_plan<NTK_DT_Q6_K>(rows, nseg, n_tokens, in_features).n > 0;
+    switch (dtype) {
+        case NTK_DT_Q8_0: return ntk::short_takes<NTK_DT_Q8_0, NTK_DT_Q8_0>(rows, nseg, n_tokens, in_features);
+        case NTK_DT_Q4_0: return ntk::short_takes<NTK_DT_Q4_0, NTK_DT_Q4_0>(rows, nseg, n_tokens, in_features);
+        case NTK_DT_Q4_K: return ntk::short_takes<NTK_DT_Q4_K, NTK_DT_Q4_K + ntk::GB_RP>(rows, nseg, n_tokens, in_features);
+        case NTK_DT_Q5_K: return ntk::short_takes<NTK_DT_Q5_K, NTK_DT_Q5_K + ntk::GB_RP>(rows, nseg, n_tokens, in_features);
+        case NTK_DT_Q6_K: return ntk::short_takes<NTK_DT_Q6_K, NTK_DT_Q6_K + ntk::GB_RP>(rows, nseg, n_tokens, in_features);
         default: return 0;
     }
 }
