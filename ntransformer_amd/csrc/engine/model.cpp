@@ -618,22 +618,19 @@ float* Model::forward(const int* tokens, int T, int start_pos) {
     if (!words && ntk_memcpy_h2d_async(positions_, pos.data(), (size_t)T * 4, s) != NTK_OK) return nullptr;
     if (!words && ntk_stream_synchronize(s) != NTK_OK) return nullptr;   // `pos` / `tokens` are host temporaries
 
-    // The last layer's results are read at the last token only: of the others it needs their cache rows, and the last token takes it as a decoded token does.  One layer of the pass's time
-    // less (1 / 32 of 32 layers); prompts of up to 32 tokens that layers_short takes, and the half-precision ones, spend a layer on its weights, not on its tokens, and keep the whole layer; so do
-    // those of up to 16.  us, 17 tokens, whole / so: two layers of the 70B shape in Q6_K 1190 / 899, in Q4_K_M 862 / 687, eight of the 8B shape 1562 / 1478, 1155 / 1103; in Q8_0 (layers_short) 926 / 1085.
+    // The last layer's results are read at the last token only: of the others it needs their cache rows, and from its attention on the pass goes on with the last few tokens -- from a row on 16 bytes,
+    // two at least, by a prompt's own launches.  (As a decoded token the last one would have a K-quant's inputs rounded to 22 bits of their block's largest: 3.1e-7 of a product of normal
+    // values, 1.6e-6 beside outliers, 1.6e-7 here in both; and those launches take fewer head sizes, contexts and widths.)  us, whole / so: four layers of the 8B shape in Q8_0, 33 tokens
+    // 764 / 723, 1000 4643 / 3803; in Q4_K_M, 17 tokens 623 / 587; in F16, 33 tokens 661 / 642; two of the 70B shape in Q6_K, 17 tokens 1085 / 881.  Prompts of up to 16 tokens, and those of up to
+    // 32 that layers_short takes or that are half-precision, spend a layer on its weights, not on its tokens.
     const bool tail = batched_prefill_ && tp_world_ == 1 && cfg_.n_layers > 0 && (T > 32 || (T > 16 && is_quant(layers_.back().w_down.dtype) && !short_prompt(T)));
     int rc = layers_1to1(T, start_pos, 0, cfg_.n_layers, tail);
     if (rc == NTK_OK && tail) {
         float* const rows = hidden_;
-        int* const pos_word = d_pos_;
-        const int regime = attn_regime_;
-        hidden_ += (size_t)(T - 1) * H;
-        d_pos_ = positions_ + (T - 1);
-        attn_regime_ = regime_at(start_pos + T - 1);
-        rc = enqueue_layers(cfg_.n_layers - 1, cfg_.n_layers);
+        const int few = 4 + T % 4;
+        hidden_ += (size_t)(T - few) * H;
+        rc = layers_1to1(few, start_pos + T - few, cfg_.n_layers - 1, cfg_.n_layers, false, workspace_ + (size_t)(T - few) * qd);
         hidden_ = rows;
-        d_pos_ = pos_word;
-        attn_regime_ = regime;
     }
     auto ok = [&](int st) { if (st != NTK_OK && rc == NTK_OK) rc = st; };
     float* last = hidden_ + (size_t)(T - 1) * H;
@@ -780,9 +777,10 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
     return rc;
 }
 
-// layers [first, last) of the 1:1 path on hidden_[T][H] at positions start_pos.. (positions_ already on the device); keys_last: of the last one only the cache rows
-int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool keys_last) {
-    if (short_prompt(T) && first < last_layer) return layers_short(T, start_pos, first, last_layer);
+// layers [first, last) of the 1:1 path on hidden_[T][H] at positions start_pos.. (positions_ already on the device).  keys_last: of the last one only the cache rows, the rotated queries left at the
+// front of workspace_; queries: those of the first one's T tokens, whose cache rows are written, with room for as many behind them
+int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool keys_last, float* queries) {
+    if (!queries && short_prompt(T) && first < last_layer) return layers_short(T, start_pos, first, last_layer);
     const int H = cfg_.hidden_size, I = cfg_.intermediate_size, hd = cfg_.head_dim, nh = cfg_.n_heads, nkv = cfg_.n_kv_heads;
     const int qd = nh * hd, kvd = nkv * hd;
     void* s = stream_;
@@ -791,7 +789,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
     float* q_buf = workspace_;
     float* k_buf = q_buf + (size_t)T * qd;
     float* v_buf = k_buf + (size_t)T * kvd;
-    float* attn_out = v_buf + (size_t)T * kvd;
+    float* attn_out = queries ? queries + (size_t)T * qd : v_buf + (size_t)T * kvd;
     float* gate_buf = workspace_;
     float* up_buf = gate_buf + (size_t)T * I;
     int rc = NTK_OK;
@@ -1084,35 +1082,38 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         uint16_t* vc = v_cache_ + (size_t)i * kv_layer;
         auto only_qkv = [&](const LayerWeights& l) { return planes_only({&l.wq, &l.wk, &l.wv}, H); };
         auto half_qkv = [&](const LayerWeights& l) { return half_only({&l.wq, &l.wk, &l.wv}); };
-        if (!normed_ahead) norm(L.attn_norm, true, L.wq, only_qkv(L), half_qkv(L));
-        normed_ahead = false;
-        planes_of = planes_ready;   // residual_ has new contents (split already by the launch that wrote them, or not)
-        planes_ready = nullptr;
-        const bool one_launch = with_max && T >= 4 && hd <= 256;
-        const float* sums[3] = {q_buf, k_buf, v_buf};     // what the rotation reads: the projections, or the partial sums of the last launch's
-        int splits[3] = {1, 1, 1};
-        ntk_gemm_partials joined{};                       // (or of all three side by side)
-        {
-            float* const ys[3] = {q_buf, k_buf, v_buf};
-            const DevTensor* const ws[3] = {&L.wq, &L.wk, &L.wv};
-            project_many(ys, ws, 3, residual_, max_a, one_launch ? sums : nullptr, splits, one_launch ? &joined : nullptr);
-        }
-        if (one_launch) {                            // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
-            if (joined.part[0])
-                ok(ntk_reduce_rope_kv_store_joined(q_buf, joined.part[0], joined.nsplit, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos,
-                                                   cfg_.max_seq_len, s));
-            else if (splits[0] + splits[1] + splits[2] > 3)
-                ok(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
-            else
-                ok(ntk_rope_kv_store(q_buf, k_buf, v_buf, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc,
-                                     start_pos, cfg_.max_seq_len, s));
-        } else {
-            ok(ntk_rope(q_buf, k_buf, positions_, 1, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, s));
-            ok(ntk_copy_to_kv_cache(kc, vc, k_buf, v_buf, T, nkv, hd, start_pos, cfg_.max_seq_len, s));
+        const bool given = queries && i == first;
+        if (!given) {
+            if (!normed_ahead) norm(L.attn_norm, true, L.wq, only_qkv(L), half_qkv(L));
+            normed_ahead = false;
+            planes_of = planes_ready;   // residual_ has new contents (split already by the launch that wrote them, or not)
+            planes_ready = nullptr;
+            const bool one_launch = with_max && T >= 4 && hd <= 256;
+            const float* sums[3] = {q_buf, k_buf, v_buf};     // what the rotation reads: the projections, or the partial sums of the last launch's
+            int splits[3] = {1, 1, 1};
+            ntk_gemm_partials joined{};                       // (or of all three side by side)
+            {
+                float* const ys[3] = {q_buf, k_buf, v_buf};
+                const DevTensor* const ws[3] = {&L.wq, &L.wk, &L.wv};
+                project_many(ys, ws, 3, residual_, max_a, one_launch ? sums : nullptr, splits, one_launch ? &joined : nullptr);
+            }
+            if (one_launch) {                            // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too)
+                if (joined.part[0])
+                    ok(ntk_reduce_rope_kv_store_joined(q_buf, joined.part[0], joined.nsplit, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos,
+                                                       cfg_.max_seq_len, s));
+                else if (splits[0] + splits[1] + splits[2] > 3)
+                    ok(ntk_reduce_rope_kv_store(q_buf, sums, splits, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc, start_pos, cfg_.max_seq_len, s));
+                else
+                    ok(ntk_rope_kv_store(q_buf, k_buf, v_buf, positions_, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, kc, vc,
+                                         start_pos, cfg_.max_seq_len, s));
+            } else {
+                ok(ntk_rope(q_buf, k_buf, positions_, 1, T, nh, nkv, hd, cfg_.rope_theta, cfg_.rope_freq_scale, cfg_.rope_interleaved, s));
+                ok(ntk_copy_to_kv_cache(kc, vc, k_buf, v_buf, T, nkv, hd, start_pos, cfg_.max_seq_len, s));
+            }
         }
         if (keys_last && i + 1 == last_layer) break;
         if (T == 1) ok(ntk_attention_decode(attn_out, q_buf, kc, vc, start_pos + T, nh, nkv, hd, cfg_.max_seq_len, scale, s));
-        else ok(ntk_attention_prefill(attn_out, q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
+        else ok(ntk_attention_prefill(attn_out, given ? queries : q_buf, kc, vc, T, start_pos, nh, nkv, hd, cfg_.max_seq_len, scale, s));
         const bool only_unit = planes_only({&L.w_gate, &L.w_up}, H);
         const intptr_t apart = (intptr_t)L.w_gate.ptr - (intptr_t)L.w_up.ptr;
         const bool half_unit = half_only({&L.w_gate, &L.w_up}) && std::abs(apart) < (1LL << 32) - (intptr_t)L.w_gate.out_f * H * 2;   // (what ntk_gemm_half_many takes as a gated pair)
@@ -1765,11 +1766,9 @@ int Model::build_persistent_plan(int kind) {
 int Model::build_persistent_plan(int) { return NTK_E_SHAPE; }
 #endif
 
-int Model::regime_at(int pos) const {
-    return (attn_scratch_ && (cfg_.head_dim == 64 || cfg_.head_dim == 128 || cfg_.head_dim == 256)) ? attention_regime(pos, cfg_.head_dim) : 0;
-}
 void Model::pick_attention_regime() {
-    attn_regime_ = regime_at(host_pos_);
+    attn_regime_ = (attn_scratch_ && (cfg_.head_dim == 64 || cfg_.head_dim == 128 || cfg_.head_dim == 256))
+                       ? attention_regime(host_pos_, cfg_.head_dim) : 0;
     ++host_pos_;   // every fused token ends with ntk_advance_pos on the device; set_device_pos() re-bases both
 }
 

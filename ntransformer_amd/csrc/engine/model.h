@@ -181,8 +181,7 @@ private:
     void free_all();
     int enqueue_token(bool greedy);   // the fused launch sequence for one token
     int enqueue_layers(int first, int last);            // its layer loop
-    int layers_1to1(int T, int start_pos, int first, int last, bool keys_last = false);   // the layer loop of forward()
-    int regime_at(int pos) const;
+    int layers_1to1(int T, int start_pos, int first, int last, bool keys_last = false, float* queries = nullptr);   // the layer loop of forward()
     bool short_prompt(int T) const;
     bool short_matrices(int T) const;
     mutable int short_known_[2] = {-1, -1};   // short_matrices of up to 16 and up to 32 tokens: not asked yet, no, yes
