@@ -83,8 +83,8 @@ def test_rows_of_the_table(dtype, width):
     wd = 9 if dtype == "bf16" else 0
     want = ((bf16(x).astype(np.uint32) << 16).view(np.float32) if dtype == "bf16" else x) * np.float32(1.7)
     toks = [3, 6, 0, 7, 2]                                     # (one past the table: zeros)
-    o = DB.from_numpy(np.full((5, width), 9.0, np.float32))
-    Lr.check(L.ntk_embed_dense_scaled(o.ptr, tab.ptr, wd, DB.from_numpy(np.array(toks, np.int32)).ptr, 5, 7, width, 1.7, None), "embed")
+    o, at = DB.from_numpy(np.full((5, width), 9.0, np.float32)), DB.from_numpy(np.array(toks, np.int32))
+    Lr.check(L.ntk_embed_dense_scaled(o.ptr, tab.ptr, wd, at.ptr, 5, 7, width, 1.7, None), "embed")
     got = o.numpy(np.float32).reshape(5, width)
     for t, k in enumerate(toks):
         assert np.array_equal(got[t], want[k] if k < 7 else np.zeros(width, np.float32))

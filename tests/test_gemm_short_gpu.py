@@ -77,15 +77,15 @@ def test_products_of_grouped_planes(qname, T, rows, inf):
         X[T // 2, : inf // 2] = 0.0
         X[0] *= np.float32(1e12)
         X[T - 1] *= np.float32(1e-12)
-        y = DB.from_numpy(np.full((T, rows), 7.0, np.float32))
-        _lib.check(L.ntk_short_prepare_x(DB.from_numpy(X).ptr, T, inf, ws.ptr, None), "short_prepare_x")
+        y, Xd = DB.from_numpy(np.full((T, rows), 7.0, np.float32)), DB.from_numpy(X)
+        _lib.check(L.ntk_short_prepare_x(Xd.ptr, T, inf, ws.ptr, None), "short_prepare_x")
         product(L, ws, nbytes, [Wd], [y], rows, dt, T, inf)
         close(y.numpy(np.float32).reshape(T, rows).astype(np.float64), W, X.astype(np.float64))
         # RMSNorm in front, a residual behind
         eps, nw = 1e-5, (1.0 + 0.1 * r.standard_normal(inf)).astype(np.float32)
         res = r.standard_normal((T, rows)).astype(np.float32)
-        hd = DB.from_numpy(X)
-        _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, None, DB.from_numpy(nw).ptr, T, inf, ws.ptr, None), "short_norm")
+        hd, nd = DB.from_numpy(X), DB.from_numpy(nw)
+        _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, None, nd.ptr, T, inf, ws.ptr, None), "short_norm")
         y = DB.from_numpy(res)
         product(L, ws, nbytes, [Wd], [y], rows, dt, T, inf, 1, eps, y)
         assert np.array_equal(hd.numpy(np.float32).reshape(T, inf), X)
@@ -105,14 +105,15 @@ def test_products_of_grouped_planes(qname, T, rows, inf):
         product(L, ws, nbytes, [Wd, Wd], [g, u], rows, dt, T, inf, partials=pt)
         raw2, W2, _ = weights(r, gt, rows, rows)
         nb2 = L.ntk_gemm_quant_workspace_bytes(rows, 2 * rows)
-        wa, wb = DB(nb2), DB(nb2)
+        wa, wb, Wd2 = DB(nb2), DB(nb2), DB.from_numpy(raw2)
         _lib.check(L.ntk_short_silu_mul_prepare_x(C.byref(pt), wa.ptr, None), "short_silu")
         h0 = r.standard_normal((T, rows)).astype(np.float32)
         hd = DB.from_numpy(h0)
         pt2 = _lib.GemmPartials()
-        product(L, wa, nb2, [DB.from_numpy(raw2)], [hd], rows, dt, T, rows, resid=hd, partials=pt2)
+        product(L, wa, nb2, [Wd2], [hd], rows, dt, T, rows, resid=hd, partials=pt2)
         nw = (1.0 + 0.1 * r.standard_normal(rows)).astype(np.float32)
-        _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, C.byref(pt2), DB.from_numpy(nw).ptr, T, rows, wb.ptr, None), "short_norm")
+        nd = DB.from_numpy(nw)
+        _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, C.byref(pt2), nd.ptr, T, rows, wb.ptr, None), "short_norm")
         gv = small.astype(np.float64) @ W.T
         a = gv / (1.0 + np.exp(-gv)) * gv
         got = hd.numpy(np.float32).reshape(T, rows).astype(np.float64)
@@ -122,7 +123,7 @@ def test_products_of_grouped_planes(qname, T, rows, inf):
         size = np.sqrt((a ** 2) @ (W2 ** 2).T) + np.sqrt((2 * ga * ua) ** 2 @ (W2 ** 2).T) + np.abs(h0)
         assert (np.abs(got - (h0 + a @ W2.T)) <= REL * size).all()
         y = DB.zeros(T * rows * 4)
-        product(L, wb, nb2, [DB.from_numpy(raw2)], [y], rows, dt, T, rows, 1, eps)
+        product(L, wb, nb2, [Wd2], [y], rows, dt, T, rows, 1, eps)
         n64 = got / np.sqrt((got ** 2).mean(1, keepdims=True) + eps) * nw
         close(y.numpy(np.float32).reshape(T, rows).astype(np.float64), W2, n64)
 
@@ -135,19 +136,19 @@ def test_sums_side_by_side_and_what_is_refused():
     dts = [G.GGML_TO_DT[gt] for gt in (G.GGML_Q4_K, G.GGML_Q6_K)]
     X = r.standard_normal((T, inf)).astype(np.float32)
     nbytes = L.ntk_gemm_quant_workspace_bytes(inf, 2 * rows)
-    ws = DB(nbytes)
-    _lib.check(L.ntk_short_prepare_x(DB.from_numpy(X).ptr, T, inf, ws.ptr, None), "short_prepare_x")
+    ws, Xd = DB(nbytes), DB.from_numpy(X)
+    _lib.check(L.ntk_short_prepare_x(Xd.ptr, T, inf, ws.ptr, None), "short_prepare_x")
     bufs, sums, at = [DB.from_numpy(a) for a in raws], [], 0
-    pts = [_lib.GemmPartials(), _lib.GemmPartials()]
-    for w, dt, pt in zip(bufs, dts, pts):
-        y = DB.zeros(T * rows * 4)
+    pts, ys = [_lib.GemmPartials(), _lib.GemmPartials()], [DB.zeros(T * rows * 4) for _ in dts]
+    for w, y, dt, pt in zip(bufs, ys, dts, pts):
         product(L, ws, nbytes, [w], [y], rows, dt, T, inf, partials=pt, part_at=at)
         assert pt.nsplit > 1
         at += pt.nsplit * T * rows
     assert pts[1].part[0] - pts[0].part[0] == pts[0].nsplit * T * rows * 4
+    ones, ws2 = DB.from_numpy(np.ones(rows, np.float32)), DB(nbytes)
     for raw, dt, pt in zip(raws, dts, pts):
         h = DB.zeros(T * rows * 4)
-        _lib.check(L.ntk_short_norm_prepare_x(h.ptr, C.byref(pt), DB.from_numpy(np.ones(rows, np.float32)).ptr, T, rows, DB(nbytes).ptr, None), "short_norm")
+        _lib.check(L.ntk_short_norm_prepare_x(h.ptr, C.byref(pt), ones.ptr, T, rows, ws2.ptr, None), "short_norm")
         want = np.stack([O.gemv(raw, x, rows, inf, dt) for x in X]).astype(np.float64)
         got = h.numpy(np.float32).reshape(T, rows)
         assert np.abs(got - want).max() <= REL * 8 * np.abs(want).max()
@@ -178,7 +179,7 @@ def test_attention_and_planes_in_one_launch(T, H, G, splits, interleaved):
     scale, res = 1.0 / np.sqrt(np.float32(hd)), []
     for fused in (0, 1):
         kc, vc = (DB.from_numpy(np.full((T + 2, out[1]), 3.0, np.float16)) for _ in range(2))
-        bufs = [DB.from_numpy(p) for p in parts]
+        bufs, Wd = [DB.from_numpy(p) for p in parts], DB.from_numpy(raw)
         arr, ns, ws = (VP * 3)(*[b.ptr for b in bufs]), (C.c_int * 3)(*splits), DB(nbytes)
         if fused:
             _lib.check(L.ntk_short_attention(arr, ns, angles.ptr, T, H, G, hd, scale, interleaved, kc.ptr, vc.ptr, T + 2, ws.ptr, None), "short_attention")
@@ -188,7 +189,7 @@ def test_attention_and_planes_in_one_launch(T, H, G, splits, interleaved):
             _lib.check(L.ntk_attention_prefill(o.ptr, q.ptr, kc.ptr, vc.ptr, T, 0, H, G, hd, T + 2, scale, None), "attention")
             _lib.check(L.ntk_short_prepare_x(o.ptr, T, H * hd, ws.ptr, None), "prepare")
         y = DB.zeros(T * rows * 4)
-        product(L, ws, nbytes, [DB.from_numpy(raw)], [y], rows, dt, T, H * hd)
+        product(L, ws, nbytes, [Wd], [y], rows, dt, T, H * hd)
         res.append((kc.numpy(np.uint16), vc.numpy(np.uint16), y.numpy(np.float32)))
     assert np.isfinite(res[0][2]).all()
     for a, b in zip(*res):
