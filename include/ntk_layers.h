@@ -63,6 +63,7 @@ typedef struct ntk_dense_desc {
 #define NTK_ACT_NONE 0
 #define NTK_ACT_RELU2 1
 int ntk_dense_few_rows(void);   /* up to this many rows a product takes the row-streaming form */
+int ntk_dense_few_inputs(void); /* ... which takes up to this many inputs (NTK_E_SHAPE beyond; more rows have no such limit) */
 int ntk_dense(const ntk_dense_desc* d, void* stream);
 /* ... with its results capped: Y = cap * tanh(y / cap) (ntk_softcap_rows behind it, inside its launch where the rows are few).  cap > 0; no activation, no accumulate, no glu_ff. */
 int ntk_dense_capped(const ntk_dense_desc* d, float cap, void* stream);
@@ -233,6 +234,7 @@ int ntk_latent_fold_query_prepare(float* qf, const float* q, int ldq, const void
 /* ... and with rotated parts: ntk_latent_prepare (the cache rows; q itself is only read) and ntk_latent_fold_query in one launch */
 int ntk_latent_fold_query_rotate(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int dr, int R, const ntk_rotary* rot, float* cache, int row,
                                  const float* kv, int ldkv, const float* norm_w, float eps, int pos0, void* stream);
+int ntk_latent_shared_takes(int kv_rank, int rot_dim);   /* 1 where ntk_latent_attention's shared form takes such keys (NTK_E_SHAPE of it elsewhere), else 0 */
 /* ntk_latent_attention's shared form and ntk_latent_unfold_value_ex of its result: the states of the parts meet in the launch that unfolds them where they are few enough for that to be the
  * faster (lat, the joined states, is written and read in between elsewhere).  scratch as in ntk_latent_attention. */
 int ntk_latent_attention_unfold(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,

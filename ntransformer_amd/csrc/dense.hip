@@ -69,6 +69,7 @@ __device__ __forceinline__ void leave_outputs(const DenseArgs& a, const float (&
 // have arrived; one DPP reduction per row at the end.  The first weights are requested together with the activation row and the weights of its norm, so they
 // travel behind the norm's sum over the workgroup.  RW is picked so that the launch still has a few workgroups per CU.
 constexpr int kGemvRows = 8;       // up to this many rows take this form
+constexpr int kGemvInputs = (160 * 1024 - 1024) / 4;   // ... of up to this many inputs (a row sits in LDS)
 template <typename WT, int RW, bool GLU, bool ADD>
 __global__ __launch_bounds__(256) void dense_gemv_kernel(const DenseArgs a) {
     extern __shared__ __attribute__((aligned(16))) float xs[];   // the activation row
@@ -847,7 +848,7 @@ static int dense_with(const ntk_dense_desc* d, float cap, void* stream) {
     DenseArgs a{d->Y, d->ldy, d->X, d->ldx, d->W, d->wstride, d->offsets, d->rows, d->rows ? d->row_div : 1, d->T, d->N, d->K, d->accumulate, G, 0, 0, 0, 0.0f, 0.0f, 0.0f, 0.0f, nullptr, 0.0f, 0.0f, d->act, nullptr, 0, nullptr, 0.0f, 0.0f, nullptr, 0};
     hipStream_t s = resolve_stream(stream);
     if (d->T <= kGemvRows) {
-        if ((size_t)d->K * 4 > 160 * 1024 - 1024) return NTK_E_SHAPE;
+        if (d->K > kGemvInputs) return NTK_E_SHAPE;
         a.glu_ff = d->glu_ff; a.glu_limit = d->glu_limit; a.glu_alpha = d->glu_alpha; a.glu_up_offset = d->glu_up_offset; a.glu_cubic = d->glu_cubic;
         a.norm_w = d->norm_w; a.norm_eps = d->norm_eps; a.norm_offset = d->norm_offset;
         if (cap > 0.0f) { a.act = kActCap; a.glu_limit = cap; }
@@ -952,6 +953,7 @@ int ntk_moe_few(const ntk_moe_few_desc* d, void* stream) {
 }
 
 int ntk_dense_few_rows(void) { return kGemvRows; }
+int ntk_dense_few_inputs(void) { return ntk::kGemvInputs; }
 
 int ntk_dense_linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate, void* stream) {
     ntk_dense_desc d{};

@@ -1677,6 +1677,18 @@ int LayerStackModel::last_layer_keys(const Run& run, const StackLayer& L, int sl
     return ntk_latent_prepare(run.cache + (size_t)slot * opt_.max_context * m.row(), m.row(), a_ + m.kv_off, na, m.kv_norm, eps_, m.kv_rank, m.rot_dim, nullptr, 0, 0, 0, &rot, pos0, T, stream_);
 }
 
+// A prompt's launches take more than a decoded token's: products of any number of inputs, latent keys of any size.
+bool LayerStackModel::takes_one_token(const StackLayer& L) const {
+    const DenseW& o = L.mixer == kMixWindow ? L.att.o : L.mixer == kMixLatent ? L.mix.o : L.gdl.o;
+    int64_t most = std::max<int64_t>(info_.width, o.in_f);
+    if (L.mixer == kMixLatent) {
+        if (!ntk_latent_shared_takes(L.mix.kv_rank, L.mix.rot_dim)) return false;
+        most = std::max<int64_t>(most, L.mix.q_rank);
+    }
+    if (L.has_mlp) most = std::max(most, form_.scaled ? L.cff.down.in_f : std::max(L.mlp.routed.down.in_f, L.mlp.has_shared ? L.mlp.shared.down.in_f : 0));
+    return most <= ntk_dense_few_inputs();
+}
+
 // want_last: the portion's last token is wanted and no other; token >= 0: the portion's only token, not in tokens_dev
 int LayerStackModel::portion(int slot, const int* tokens_dev, int token, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out) {
     const int W = info_.width;
@@ -1699,8 +1711,10 @@ int LayerStackModel::portion(int slot, const int* tokens_dev, int token, int pre
     bool x_is_x0 = keep_embedding;   // until the first layer run writes x_
     owed_.y = nullptr;
     // The last layer's results are read where they are wanted and nowhere else: of the other tokens it needs what later tokens attend to (last_layer_keys), and a last token alone takes the
-    // layer as a decoded token does.  A layer's worth of a prompt's time less: 1 / 2 of it with two layers, 1 / 32 with 32.  (ten tokens on: fewer go through the one-token products anyway)
-    const bool tail = (form_.scaled || !(form_.gated || form_.sequential || form_.post_norm || form_.dense_parallel)) && T > ntk_dense_few_rows() + 1 && (n_want == 0 || want_last) && !(capture_ && capture_buf_);
+    // layer as a decoded token does, where the launches of one take it.  A layer's worth of a prompt's time less: 1 / 2 of it with two layers, 1 / 32 with 32.  (ten tokens on: fewer go
+    // through the one-token products anyway)
+    const bool tail = !runs_.empty() && (form_.scaled || !(form_.gated || form_.sequential || form_.post_norm || form_.dense_parallel)) && T > ntk_dense_few_rows() + 1 &&
+                      (n_want == 0 || (want_last && takes_one_token(layers_[(size_t)runs_.back().layer]))) && !(capture_ && capture_buf_);
     struct Streams { float *&x, *&x0, *&v, *const kx, *const kx0, *const kv; ~Streams() { x = kx; x0 = kx0; v = kv; } };
     Streams whole{x_, x0_, vfirst_, x_, x0_, vfirst_};
     for (size_t r = 0; r < runs_.size(); ++r) {

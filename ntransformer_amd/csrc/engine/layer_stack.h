@@ -331,6 +331,7 @@ private:
     void* late_alloc(size_t bytes);
     int portion(int slot, const int* tokens_dev, int token, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out);
     int last_layer_keys(const Run& run, const StackLayer& L, int slot, int T, int pos0);
+    bool takes_one_token(const StackLayer& L) const;
     int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false, const void* h16 = nullptr);
     int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, bool norm_inside = false, const void* h16 = nullptr);
     int window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0);

@@ -578,13 +578,12 @@ static int shared_keys(int pos0, int T, int window) { return window > 0 ? (windo
 static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, int ldq, const float* cache, int row, int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale,
                          float* scratch, bool merge, void* stream) {
     if (!scratch) return NTK_E_NULL;
-    if (kv_rank > 512) return NTK_E_SHAPE;
+    if (!ntk_latent_shared_takes(kv_rank, rot_dim)) return NTK_E_SHAPE;
     hipStream_t s = resolve_stream(stream);
     sa.q = q; sa.ldq = ldq; sa.cache = cache; sa.row = row; sa.R = kv_rank; sa.dr = rot_dim; sa.H = H; sa.pos0 = pos0; sa.T = T; sa.window = window;
     sa.scale = scale; sa.scratch = scratch;
     sa.splits = shared_splits(shared_keys(pos0, T, window));
     const int rows = T * H, DK = kv_rank + rot_dim;
-    if (((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) > 156 * 1024) return NTK_E_SHAPE;     // (keys of up to 812 entries)
     const size_t lds = ((size_t)KB * (((DK + 15) & ~15) + 4) + 5 * SROWS * (KB + 4) + 3 * SROWS) * sizeof(float);
     static bool raised_s = false;   // (idempotent: a race sets the same attribute twice)
     if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel<13, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
@@ -601,6 +600,11 @@ static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, in
 }  // namespace ntk
 
 using namespace ntk;
+
+int ntk_latent_shared_takes(int kv_rank, int rot_dim) {
+    const int DK = kv_rank + rot_dim;
+    return kv_rank > 0 && kv_rank <= 512 && rot_dim >= 0 && ((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) <= 156 * 1024;     // (keys of up to 816 entries)
+}
 
 int ntk_latent_prepare(float* cache, int row, const float* kv, int ldkv, const float* norm_w, float eps, int kv_rank, int rot_dim, float* q, int ldq, int H, int qd,
                        const ntk_rotary* rot, int pos0, int T, void* stream) {

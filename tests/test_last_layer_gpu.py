@@ -72,6 +72,21 @@ def test_parallel_form(tmp_path, dtype, T, kw):
     check(FO, FO.small_config(**kw), tmp_path, dtype, T)
 
 
+@pytest.mark.parametrize("last", ["20480", "40960", "latent"])
+def test_last_layers_beyond_a_decoded_tokens_launches(tmp_path, last):
+    """a unit of 40960 values, keys of 820 entries: what the products and the attention of a few tokens refuse, a prompt's take, its last layer whole (of 20480 values they take)"""
+    layers = {"20480": [O.attention_layer(size=24), O.attention_layer(size=24, ff=20480)], "40960": [O.attention_layer(size=24), O.attention_layer(size=24, ff=40960)], "latent": [O.latent_layer(heads=2, dim=8, rot_dim=308, kv_rank=512)]}[last]
+    cfg = O.config(layers, width=64)
+    w = O.random_weights(cfg, 5)
+    O.save_model(str(tmp_path / "m"), cfg, w)
+    toks = [int(t) for t in np.random.default_rng(3).integers(0, cfg["vocab"], 16)]
+    e = Engine()
+    e.load_folder(str(tmp_path / "m"), max_context=32, dtype="float32", slots=1)
+    got = e.seq_forward(e.seq_acquire(), toks, want=[15])
+    e.close()
+    assert rel(got, O.forward(cfg, w, toks)[0][15:]) < TOL["float32"]
+
+
 @pytest.mark.parametrize("mix", ["Q8_0", "Q4_K_M", "F16"])
 @pytest.mark.parametrize("T", [32, 33, 70])
 def test_gguf_prompts(mix, T):
