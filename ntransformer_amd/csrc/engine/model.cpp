@@ -79,7 +79,7 @@ void Model::free_all() {
     host_pos_ = 0;
     attn_regime_ = 0;
     k_cache_ = v_cache_ = nullptr;
-    hidden_ = residual_ = workspace_ = logits_ = argmax_scratch_ = rope_inv_freq_ = attn_scratch_ = row_max_ = nullptr;
+    hidden_ = residual_ = workspace_ = logits_ = argmax_scratch_ = rope_inv_freq_ = rope_angles_ = attn_scratch_ = row_max_ = nullptr;
     positions_ = tokens_dev_ = d_pos_ = d_token_ = nullptr;
 }
 
@@ -570,10 +570,12 @@ int Model::alloc_buffers() {   // transformer.cpp:330-391
         return NTK_E_NOMEM;
     }
     *h_token_ = 0;
-    if (rope_inv_freq_ && rope_angles_) {
+    if (rope_inv_freq_) {
         std::vector<float> f((size_t)cfg_.head_dim / 2);
         for (int i = 0; i < cfg_.head_dim / 2; ++i) f[i] = 1.0f / powf(cfg_.rope_theta, (2.0f * i) / cfg_.head_dim);
         nt_hip_memcpy_h2d(rope_inv_freq_, f.data(), f.size() * 4);
+    }
+    if (rope_angles_) {   // (none: short prompts rotate in a launch of their own)
         if (ntk_short_angles(rope_angles_, cfg_.head_dim, cfg_.rope_theta, cfg_.rope_freq_scale, stream_) != NTK_OK || ntk_stream_synchronize(stream_) != NTK_OK) return NTK_E_LAUNCH;
     }
     return NTK_OK;
