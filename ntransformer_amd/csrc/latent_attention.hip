@@ -691,19 +691,18 @@ int ntk_latent_fold_query(float* qf, const float* q, int ldq, const void* w_uk, 
     return fold_query(qf, q, ldq, w_uk, wdtype, T, H, dn, dr, R, FoldPrepare{}, stream);
 }
 
-int ntk_latent_fold_query_prepare(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int R, float* cache, int row, const float* kv,
-                                  int ldkv, const float* norm_w, float eps, int pos0, void* stream) {
-    if (!cache || !kv || !norm_w) return NTK_E_NULL;
-    if (row < R || ldkv < R || pos0 < 0) return NTK_E_SHAPE;
-    return fold_query(qf, q, ldq, w_uk, wdtype, T, H, dn, 0, R, FoldPrepare{cache, row, kv, ldkv, norm_w, eps, pos0, nullptr, 1.0f, 0, 0}, stream);
-}
-
 int ntk_latent_fold_query_rotate(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int dr, int R, const ntk_rotary* rot, float* cache, int row,
                                  const float* kv, int ldkv, const float* norm_w, float eps, int pos0, void* stream) {
     if (!cache || !kv || !norm_w || !rot || (rot->dims > 0 && !rot->freq)) return NTK_E_NULL;
     if (dr < 0 || rot->dims < 0 || (rot->dims & 1) || rot->dims > dr || row < R + dr || ldkv < R + dr || pos0 < 0) return NTK_E_SHAPE;
     if (rot->layout != NTK_ROT_NEIGHBOURS && rot->layout != NTK_ROT_HALVES) return NTK_E_SHAPE;
     return fold_query(qf, q, ldq, w_uk, wdtype, T, H, dn, dr, R, FoldPrepare{cache, row, kv, ldkv, norm_w, eps, pos0, rot->freq, rot->mag, rot->dims, rot->layout == NTK_ROT_HALVES ? 1 : 0}, stream);
+}
+
+int ntk_latent_fold_query_prepare(float* qf, const float* q, int ldq, const void* w_uk, int wdtype, int T, int H, int dn, int R, float* cache, int row, const float* kv,
+                                  int ldkv, const float* norm_w, float eps, int pos0, void* stream) {
+    const ntk_rotary none{nullptr, 1.0f, 0, NTK_ROT_NEIGHBOURS};
+    return ntk_latent_fold_query_rotate(qf, q, ldq, w_uk, wdtype, T, H, dn, 0, R, &none, cache, row, kv, ldkv, norm_w, eps, pos0, stream);
 }
 
 int ntk_latent_attention_unfold(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,
