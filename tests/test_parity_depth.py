@@ -470,3 +470,14 @@ def test_depth_8b_q4_k_m_massive_activations():
     # itself sits 5.0e-4 from the arbiter forced to its own roundings and 2.1e-2 from the free one.  abs_scale = 66: the forced-arbiter bar as 1e-4 OF THE
     # LOGIT RMS; flip_scale 40.
     _depth_parity("8b_q4_k_m_massive_activations_6_layers", "8b", "Q4_K_M", 6, 20, 3, patch=patch, flip_scale=40.0, abs_scale=66.0, e2e_kv_from_oracle=True)
+
+
+def test_depth_8b_q4_k_m_massive_activations_16_tokens():
+    """the model above in two layers, a prompt of 16 tokens: every projection over planes that are scaled per token and 256 columns (20 tokens of a mix with Q6_K in it take one scale a token).  Layer by
+    layer at the seeded models' bars.  (End to end the prompt's logits are 1.5e-4 from the arbiter forced to its cache, the per-token sequence's 1.6e-4, the oracle's 5.7e-4; the tokens decoded behind
+    it are fused launches' either way.)"""
+    factors = {5: 1000.0, 1033: 1000.0, 2500: 1000.0, 4000: 1000.0, 3333: 4000.0}
+
+    def patch(path):
+        assert _scale_norm_channels(path, factors) >= 5
+    _depth_parity("8b_q4_k_m_massive_activations_2_layers", "8b", "Q4_K_M", 2, 16, 2, patch=patch, flip_scale=40.0, end_to_end=False)
