@@ -88,3 +88,19 @@ def test_the_last_tokens_products_are_a_prompts(tmp_path, T):
             sq.append(rel(got, arbiter.ArbiterModel(om).forward(toks, 0, (K, V))) ** 2)
         return np.sqrt(np.mean(sq))
     assert error(T) < 1.5 * error(16)
+
+
+@pytest.mark.parametrize("mix", ["Q8_0", "Q4_K_M"])
+@pytest.mark.parametrize("start", [5, 600])
+@pytest.mark.parametrize("T", [2, 3, 4, 16, 17, 32, 33, 70])
+def test_prompts_behind_a_context(mix, start, T):
+    """a prompt that begins behind others: the short form's own rotation and attention (2 and 3 tokens: of whole projections), several formats' sums side by side, the last layer cut short; few and more
+    positions in front than the single-pass attention of a decoded token walks"""
+    check(spec(1024, 2048, 8, 2, mix), 1024, [start, T])
+
+
+@pytest.mark.parametrize("T", [2, 5, 33, 70, 200])
+@pytest.mark.parametrize("start", [0, 7])
+def test_half_precision_chain(T, start):
+    """from 3072 inputs on: the norm's halves from the launch that sums the projection in front of it, query, key and value rotated from their joined pieces, the last layer cut short from 33 tokens on"""
+    check(spec(3072, 3200, 24, 8, "F16"), 256, [start, T] if start else [T])
