@@ -1,6 +1,7 @@
 """ntk_gated_delta_step -- a decoded token of the delta rule: convolutions and step in one launch, head norm, silu gate and carried inputs in a second -- against the launches it replaces (ntk_gated_recurrence with the
-convolutions inside, ntk_head_rmsnorm_gate) token by token: results, state and carried inputs within 1e-6 (sums of up to 128 products in float32, in another order), from an empty state whose
-memory holds NaN.  Sizes below, at and between the rows a lane holds, columns that end inside a wave, one head a group and several."""
+convolutions inside, ntk_head_rmsnorm_gate) token by token, from an empty state whose memory holds NaN: the state within 1e-6 of its largest value (sums of up to 128 products in float32, in another
+order: 16 of the largest one's half ulps), the results within 4e-6 (such a sum over the state, and the head's norm and gate: the difference of a value goes through the norm's factor, up to 3 here), the
+carried inputs the same bits.  Sizes below, at and between the rows a lane holds, columns that end inside a wave, one head a group and several."""
 import ctypes as C
 
 import numpy as np

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 VP, I, F = C.c_void_p, C.c_int, C.c_float
 
 
-@pytest.mark.parametrize("T", [1, 64, 65, 256, 257])      # (a workgroup per 256 pairs, four a token, one a token)
+@pytest.mark.parametrize("T", [1, 64, 65, 256, 257])      # (up to 64 tokens a workgroup per 256 pairs, beyond four a token)
 @pytest.mark.parametrize("H,G,hd,splits,interleaved", [(4, 2, 64, 2, 0), (8, 2, 128, 3, 1), (3, 3, 34, 1, 0)])
 def test_pieces_side_by_side(T, H, G, hd, splits, interleaved):
     L, g = _lib.lib(), np.random.default_rng(T + H)
