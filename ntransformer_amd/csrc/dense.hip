@@ -633,18 +633,26 @@ static void launch_moe_few(const MoeFewArgs& a, int T, bool glu, hipStream_t s) 
 // formed there by a workgroup, here by a wave; what is saved are the weights' further passes, of which bf16 has half.  us, a workgroup a row / this, rows 2, 4, 8: bf16 2048 x 2048 5.3 / 4.6,
 // 5.5 / 5.6, 9.0 / 7.7; 6144 x 2048 8.0 / 7.4, 14.6 / 9.2, 25 / 12; behind a norm 9.2 / 9.0, 15.7 / 10.9, 28 / 15; 2048 x 2048 behind one 5.8 / 6.3, 6.4 / 7.6, 10.3 / 11.0; float32 2048 x 2048 8.1 / 6.2,
 // 13.2 / 7.3, 23 / 9.6, behind a norm and a sum 9.8 / 10.2, 14.1 / 12.0, 24 / 18; gated units with both, bf16 1408 x 2048 7.5 / 9.7, 8.8 / 11.7, 12 / 19, 7488 x 2048 27 / 24, 44 / 29, 81 / 46;
-// float32 10.8 / 12.5, 18 / 15, 31 / 22 and 48 / 36, 91 / 42, 171 / 57.
+// float32 10.8 / 12.5, 18 / 15, 31 / 22 and 48 / 36, 91 / 42, 171 / 57.  With few outputs the other form's rows fill CUs that this one leaves idle, and a norm's waves walk all its inputs: float32, 8
+// rows, 256 x 4096 6.5 / 10.8, 512 x 8192 17 / 20, behind a norm 256 x 14336 21 / 52, 704 x 4096 14 / 17, and 1024 x 4096, 2 rows, 8.6 / 10.0; with a sum 1024 x 4096, 4 rows, 13 / 17; units of
+// 704 x 4096, 4 rows, 18 / 20.  bf16 units, rows 2, 5, 8: 4096 x 3072 16 / 18, 34 / 27, 53 / 32; 4608 x 2560 17 / 18, 33 / 42, 52 / 50; 6144 x 2560 20 / 19, 46 / 43, 70 / 51.
+// Of 5194 launches of 512 .. 14336 inputs, 1024 .. 32000 outputs and 2 .. 8 rows that this takes four are behind the other form by more than 2 %, by 5 % at most.
 template <typename WT, bool ADD>
 static bool rows_share_weights(const DenseArgs& a, int rows) {
     if (rows < 2 || !a.vec || !a.xvec || a.offsets) return false;
     const long long n = a.glu_ff > 0 ? a.glu_ff : a.N, size = n * a.K;
     if constexpr (sizeof(WT) == 2) {
-        if (a.glu_ff > 0) return n >= 4096 && size >= 8LL << 20;
-        return size >= 4LL << 20 && n * rows >= (size >= 8LL << 20 ? 12288 : 16384) && (n >= 4096 || !(ADD || a.norm_w));
+        const bool normed = ADD || a.norm_w;
+        if (a.glu_ff == 0) return size >= 4LL << 20 && n * rows >= (size >= 8LL << 20 && !normed ? 12288 : 16384) && (n >= 4096 || !normed);
+        if (rows == 2) return n >= 6144 && a.K >= 2048;
+        const long long groups = (n + 15) / 16;      // (from five rows on one a CU at a time: two rounds are worth it from three quarters of their places on)
+        if (rows > 4 && rows < 8 && (size < 10000000 || 4 * groups < 3 * ((groups + 255) / 256 * 256))) return false;
+        return n >= 4096 && size >= 8LL << 20;
     }
-    if (a.glu_ff > 0) return size >= 2800000 && (rows >= 3 || n >= 4096);
-    if constexpr (ADD) return size >= 4LL << 20 && (rows >= 4 || n >= 4096);
-    return size >= (a.norm_w ? 2LL << 20 : 1LL << 20);
+    if (a.glu_ff > 0) return size >= 2800000 && n >= 1024 && (rows >= 3 || n >= 4096);
+    if constexpr (ADD) return size >= 4LL << 20 && n >= 2048 && (rows >= 4 || n >= 4096);
+    if (a.norm_w) return size >= 2LL << 20 && (n >= 2048 || (n >= 1024 && n * rows >= 8192));
+    return size >= 1LL << 20 && n >= 1024;
 }
 
 template <typename WT, bool ADD>
