@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void row_scale_kernel(const float* __restrict_
 // of their scales -- no row_scale_kernel pass over X; the blocks of step 0 leave 1 / s in `inv` for the main kernel
 template <bool FROM_MAX>
 __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ X, int T, int in, u32x4* __restrict__ xb, float* __restrict__ aux,
-                                                      size_t chunk_bytes, const float* __restrict__ scale, float* __restrict__ inv, float* __restrict__ group_inv) {
+                                                      size_t chunk_bytes, const float* __restrict__ scale, float* __restrict__ inv) {
     const int step = blockIdx.x, tb = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int j = lane & 15, g = lane >> 4, t = tb * 16 + j;
     // blockIdx.y = 64-token chunk: its tokens, its planes
@@ -161,8 +161,6 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
         } else {
             sc = scale[t];
         }
-        if (g == 0 && step % (GB_GROUP / 32) == 0 && T <= GB_SHORT && blockIdx.y == 0)   // (a short prompt; one scale a token here: every group's; 1 / s of a power of two by its exponent)
-            group_inv[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((254u << 23) - __float_as_uint(sc));
     }
     float p1[8], p2[8];
 #pragma unroll
@@ -296,8 +294,6 @@ __device__ __forceinline__ void split_row(const float* row, uint32_t max_bits, i
             const int pos = ((tb * 2 + ((step >> 2) & 1)) * 64 + j * 4 + (step & 3));
             rec[pos] = h1;
             rec[4 * 128 + pos] = h2;
-            if (gridDim.x <= GB_SHORT && step % (GB_GROUP / 32) == 0 && step * 32 < in)   // (a short prompt; a workgroup a token)
-                reinterpret_cast<float*>(ws + ws_group_offset(in))[step / (GB_GROUP / 32) * GB_SHORT + t] = __uint_as_float((uint32_t)(254 - es) << 23);
         }
     }
 }
@@ -1810,8 +1806,8 @@ struct GemmKParams {
     int nseg;
     const uint8_t* xb;      // operand planes of the (single) chunk
     const uint8_t* aux;     // its step sums (K-quant minimum term)
+    const float* inv;       // [T]: 1 / s (WHOLE)
     const float* group_inv; // [in / GB_GROUP][GB_SHORT]: 1 / s of a group of columns
-    int whole;              // one scale a token (planes by split_x_kernel or split_row): a slice's sums run on over its units, 1 / s at their end -- the bits that such launches have always given
     const float* ssq;       // X is to be divided by its rows' root mean squares: [nssq][GB_SHORT] sums of squares, or null
     int nssq;
     float eps;
@@ -1838,7 +1834,9 @@ template <int DT, int RT, int NTB> constexpr int gk_max_steps() {
     return (160 * 1024 - gk_waves<DT, RT, NTB>() * (16 * RT * row)) / (GB_PLANES * NTB * GB_PIECE) / DeqI<DT>::SPU * DeqI<DT>::SPU;
 }
 
-template <int DT, int RT, int NTB, bool AL>
+// WHOLE: one scale a token (planes by split_x_kernel or split_row): a slice's sums run on over its units, 1 / s at their end -- the bits that such launches have always given.  (As a question put to
+// the launch it cost them the registers and instructions of the other form: Q4_K of 32 tokens 21.4 us a launch, 20.0 so.)
+template <int DT, int RT, int NTB, bool AL, bool WHOLE>
 __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16_kslice_kernel(const GemmKParams p) {
     using D = DeqI<DT>;
     constexpr int SPU = D::SPU, NCH = D::NCH, STRIDE = D::STRIDE;
@@ -1867,7 +1865,7 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
 #endif
         }
     }
-    f32x4 inv_t[NTB];   // 1 / rms of the lane's tokens where X wants it, 1 / s where it is the whole token's, else 1
+    f32x4 inv_t[NTB];   // 1 / rms of the lane's tokens where X wants it, else 1 (WHOLE: 1 / s, at the end)
     for (int it = 0; it < p.jobs; ++it) {
     // this wave's tile (waves past the last tile only help with the copy)
     const int tile_raw = ((int)blockIdx.x + it * (int)gridDim.x) * NW + wave;
@@ -1929,7 +1927,8 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) v[tb] = *reinterpret_cast<const f32x4*>(p.group_inv + (size_t)(unit * (SPU * 32) / GB_GROUP) * GB_SHORT + tb * 16 + 4 * g);
     };
-    f32x4 sum[RT][NTB];   // the slice's sums; acc: a unit's, in its group's scale
+    f32x4 sum[RT][NTB], of_unit[RT][NTB];   // the slice's sums; a unit's, in its group's scale
+    f32x4 (&acc)[RT][NTB] = WHOLE ? sum : of_unit;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -1942,14 +1941,14 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (D::HAS_MIN) { load_sums(svr, u_lo); __builtin_amdgcn_sched_barrier(0); }
     f32x4 ginv[NTB];
-    load_inv(ginv, u_lo);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!WHOLE) { load_inv(ginv, u_lo); __builtin_amdgcn_sched_barrier(0); }
     if (it == 0) {
         // (requested behind the first weights and done with before the first row is stored: there, one request behind the other, the parts cost gate | up of 4096 inputs 2.4 us of
         // 28.7, in front of the first weights Q | K | V 1.3 of 10.9)
+        if constexpr (!WHOLE)
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) {
-            inv_t[tb] = p.whole ? *reinterpret_cast<const f32x4*>(p.group_inv + tb * 16 + 4 * g) : f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+            inv_t[tb] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
             if (p.ssq) {   // (uniform)
                 const float* src = p.ssq + tb * 16 + 4 * g;
                 f32x4 q = *reinterpret_cast<const f32x4*>(src);
@@ -1988,15 +1987,17 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
                 load_sums(svr, min(u + 1, u_hi - 1));   // (same queue, same distance, consumption order: behind the unit's weights)
                 __builtin_amdgcn_sched_barrier(0);
             }
-            f32x4 gi[NTB], acc[RT][NTB];
+            f32x4 gi[NTB];
+            if constexpr (!WHOLE) {
 #pragma unroll
-            for (int tb = 0; tb < NTB; ++tb) {
-                gi[tb] = ginv[tb];
+                for (int tb = 0; tb < NTB; ++tb) {
+                    gi[tb] = ginv[tb];
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) acc[rt][tb] = p.whole ? sum[rt][tb] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int rt = 0; rt < RT; ++rt) acc[rt][tb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+                load_inv(ginv, min(u + 1, u_hi - 1));
+                __builtin_amdgcn_sched_barrier(0);
             }
-            load_inv(ginv, min(u + 1, u_hi - 1));
-            __builtin_amdgcn_sched_barrier(0);
             const uint32_t uoff = (uint32_t)u * D::UB;
             typename D::Hdr hdr[RT];
             typename D::MinOp mop[RT];
@@ -2076,15 +2077,19 @@ __global__ __launch_bounds__((64 * gk_waves<DT, RT, NTB>())) void gemm_quant_f16
                         for (int e = 0; e < 4; ++e) acc[rt][tb][e] = fmaf(mop[rt].ndmin64, rr[rt][e], acc[rt][tb][e]);
                 }
             }
+            if constexpr (!WHOLE)
 #pragma unroll
             for (int tb = 0; tb < NTB; ++tb)
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) sum[rt][tb][e] = p.whole ? acc[rt][tb][e] : fmaf(acc[rt][tb][e], gi[tb][e], sum[rt][tb][e]);
+                    for (int e = 0; e < 4; ++e) sum[rt][tb][e] = fmaf(acc[rt][tb][e], gi[tb][e], sum[rt][tb][e]);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- this wave's rows: accumulator element e of lane (i = row of the tile, g) is token tb * 16 + 4 g + e; 1 / rms where X wants it; Y or this slice's partial sums ----
+        if constexpr (WHOLE)
+#pragma unroll
+            for (int tb = 0; tb < NTB; ++tb) inv_t[tb] = *reinterpret_cast<const f32x4*>(p.inv + tb * 16 + 4 * g);   // (the array is padded to whole chunks)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const int r = row0 + rt * 16 + i;
@@ -2415,11 +2420,11 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     p.resid = resid;
     if (!reuse_x && row_max) {   // the tokens' largest |x| came with X: one pre-pass launch
         hipLaunchKernelGGL(split_x_kernel<true>, dim3(p.steps + 8, p.chunks), dim3(256), 0, st, X, T, in, reinterpret_cast<u32x4*>(wsb),
-                           const_cast<float*>(p.aux), p.chunk_bytes, row_max, scales, group_inv);
+                           const_cast<float*>(p.aux), p.chunk_bytes, row_max, scales);
     } else if (!reuse_x) {
         hipLaunchKernelGGL(row_scale_kernel, dim3((T + 3) / 4), dim3(256), 0, st, X, T, in, scales + GB_MAX_CHUNKS * GB_TOK, scales);
         hipLaunchKernelGGL(split_x_kernel<false>, dim3(p.steps + 8, p.chunks), dim3(256), 0, st, X, T, in, reinterpret_cast<u32x4*>(wsb),
-                           const_cast<float*>(p.aux), p.chunk_bytes, scales + GB_MAX_CHUNKS * GB_TOK, static_cast<float*>(nullptr), group_inv);
+                           const_cast<float*>(p.aux), p.chunk_bytes, scales + GB_MAX_CHUNKS * GB_TOK, static_cast<float*>(nullptr));
     }
     // ---- short prompts (<= 32 tokens), second form: K-slice-stationary (gemm_quant_f16_kslice_kernel) ----
     constexpr int KDT = kslice_dt<DT>();
@@ -2434,7 +2439,7 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
         if (best_n > 0) {
             GemmKParams kp{};
             kp.nseg = nseg; kp.T = T; kp.in = in; kp.steps = in / 32; kp.row_bytes = (unsigned)row_bytes;
-            kp.xb = wsb; kp.aux = reinterpret_cast<const uint8_t*>(p.aux); kp.group_inv = group_inv; kp.whole = sh.on ? 0 : 1; kp.resid = best_n == 1 ? resid : nullptr;
+            kp.xb = wsb; kp.aux = reinterpret_cast<const uint8_t*>(p.aux); kp.inv = scales; kp.group_inv = group_inv; kp.resid = best_n == 1 ? resid : nullptr;
             kp.nsplit = best_n; kp.units_per_split = best_ups;
             if (sh.norm) { kp.ssq = group_inv + ws_group_floats(in); kp.nssq = (in + 511) / 512; kp.eps = sh.eps; }
             float* kpart = reinterpret_cast<float*>(wsb + ws_part_offset(in)) + sh.part_at;
@@ -2459,27 +2464,29 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
             static const bool kslice_lds_ok = [] {   // up to 160 KB of dynamic LDS: opt in once per kernel
                 bool ok = true;
                 auto set = [&](const void* f, size_t n) { ok &= hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) == hipSuccess; };
-                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 1, true>), gk_lds_bytes<KDT, 1, 1>(gk_waves<KDT, 1, 1>(), gk_max_steps<KDT, 1, 1>()));
-                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 1, false>), gk_lds_bytes<KDT, 1, 1>(gk_waves<KDT, 1, 1>(), gk_max_steps<KDT, 1, 1>()));
-                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 1, true>), gk_lds_bytes<KDT, 2, 1>(gk_waves<KDT, 2, 1>(), gk_max_steps<KDT, 2, 1>()));
-                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 1, false>), gk_lds_bytes<KDT, 2, 1>(gk_waves<KDT, 2, 1>(), gk_max_steps<KDT, 2, 1>()));
-                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 2, true>), gk_lds_bytes<KDT, 1, 2>(gk_waves<KDT, 1, 2>(), gk_max_steps<KDT, 1, 2>()));
-                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 2, false>), gk_lds_bytes<KDT, 1, 2>(gk_waves<KDT, 1, 2>(), gk_max_steps<KDT, 1, 2>()));
+                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 1, true, true>), gk_lds_bytes<KDT, 1, 1>(gk_waves<KDT, 1, 1>(), gk_max_steps<KDT, 1, 1>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 1, true, false>), gk_lds_bytes<KDT, 1, 1>(gk_waves<KDT, 1, 1>(), gk_max_steps<KDT, 1, 1>()));
+                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 1, false, true>), gk_lds_bytes<KDT, 1, 1>(gk_waves<KDT, 1, 1>(), gk_max_steps<KDT, 1, 1>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 1, false, false>), gk_lds_bytes<KDT, 1, 1>(gk_waves<KDT, 1, 1>(), gk_max_steps<KDT, 1, 1>()));
+                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 1, true, true>), gk_lds_bytes<KDT, 2, 1>(gk_waves<KDT, 2, 1>(), gk_max_steps<KDT, 2, 1>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 1, true, false>), gk_lds_bytes<KDT, 2, 1>(gk_waves<KDT, 2, 1>(), gk_max_steps<KDT, 2, 1>()));
+                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 1, false, true>), gk_lds_bytes<KDT, 2, 1>(gk_waves<KDT, 2, 1>(), gk_max_steps<KDT, 2, 1>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 1, false, false>), gk_lds_bytes<KDT, 2, 1>(gk_waves<KDT, 2, 1>(), gk_max_steps<KDT, 2, 1>()));
+                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 2, true, true>), gk_lds_bytes<KDT, 1, 2>(gk_waves<KDT, 1, 2>(), gk_max_steps<KDT, 1, 2>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 2, true, false>), gk_lds_bytes<KDT, 1, 2>(gk_waves<KDT, 1, 2>(), gk_max_steps<KDT, 1, 2>()));
+                set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 2, false, true>), gk_lds_bytes<KDT, 1, 2>(gk_waves<KDT, 1, 2>(), gk_max_steps<KDT, 1, 2>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 1, 2, false, false>), gk_lds_bytes<KDT, 1, 2>(gk_waves<KDT, 1, 2>(), gk_max_steps<KDT, 1, 2>()));
                 if constexpr (!KD::SPLIT16) {
-                    set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 2, true>), gk_lds_bytes<KDT, 2, 2>(gk_waves<KDT, 2, 2>(), gk_max_steps<KDT, 2, 2>()));
-                    set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 2, false>), gk_lds_bytes<KDT, 2, 2>(gk_waves<KDT, 2, 2>(), gk_max_steps<KDT, 2, 2>()));
+                    set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 2, true, true>), gk_lds_bytes<KDT, 2, 2>(gk_waves<KDT, 2, 2>(), gk_max_steps<KDT, 2, 2>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 2, true, false>), gk_lds_bytes<KDT, 2, 2>(gk_waves<KDT, 2, 2>(), gk_max_steps<KDT, 2, 2>()));
+                    set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 2, false, true>), gk_lds_bytes<KDT, 2, 2>(gk_waves<KDT, 2, 2>(), gk_max_steps<KDT, 2, 2>())); set(reinterpret_cast<const void*>(&gemm_quant_f16_kslice_kernel<KDT, 2, 2, false, false>), gk_lds_bytes<KDT, 2, 2>(gk_waves<KDT, 2, 2>(), gk_max_steps<KDT, 2, 2>()));
                 }
                 return ok;
             }();
             if (!kslice_lds_ok) return NTK_E_LAUNCH;
-            // (one launch site per instantiation: RT x NTB x AL)
+            // (one launch site per instantiation: RT x NTB x AL x WHOLE)
             auto go = [&](auto rt_c, auto ntb_c) {
                 constexpr int R = decltype(rt_c)::value, N = decltype(ntb_c)::value;
                 if constexpr (R == 2 && N >= 2 && KD::SPLIT16) return;
                 else {
                     const size_t klds = gk_lds_bytes<KDT, R, N>(gk_waves<KDT, R, N>(), slice_steps);
-                    if (kal) hipLaunchKernelGGL((gemm_quant_f16_kslice_kernel<KDT, R, N, true>), kgrid, kblock, klds, st, kp);
-                    else hipLaunchKernelGGL((gemm_quant_f16_kslice_kernel<KDT, R, N, false>), kgrid, kblock, klds, st, kp);
+                    if (kal && sh.on) hipLaunchKernelGGL((gemm_quant_f16_kslice_kernel<KDT, R, N, true, false>), kgrid, kblock, klds, st, kp);
+                    else if (kal) hipLaunchKernelGGL((gemm_quant_f16_kslice_kernel<KDT, R, N, true, true>), kgrid, kblock, klds, st, kp);
+                    else if (sh.on) hipLaunchKernelGGL((gemm_quant_f16_kslice_kernel<KDT, R, N, false, false>), kgrid, kblock, klds, st, kp);
+                    else hipLaunchKernelGGL((gemm_quant_f16_kslice_kernel<KDT, R, N, false, true>), kgrid, kblock, klds, st, kp);
                 }
             };
             using I1 = std::integral_constant<int, 1>; using I2 = std::integral_constant<int, 2>;
