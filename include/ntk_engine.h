@@ -224,8 +224,11 @@ int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partia
  *   ntk_rows_silu_mul_prepare_x   planes of silu(gate) * up of a gate | up launch, deferred or not; output (may be NULL, may be the gate's y): the rows themselves
  * Workspace and alignments as above; results as the launches above give them, up to the order of a norm's sum. */
 int ntk_rows_prepare_takes(int n_tokens, int width, int norm);
+int ntk_rows_prepare_pays(int n_tokens, int width, int norm, int nsplit);   /* ... and is ahead of the launches that it replaces (nsplit: pieces to add up; 0: rows as they lie; the third has 1 at least) */
 int ntk_rows_prepare_x(const float* X, int n_tokens, int width, void* workspace, void* stream);
 int ntk_rows_norm_prepare_x(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int width, float eps, float* x_out, void* workspace, void* stream);
+int ntk_rows_norm_prepare_zero(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int width, float eps, float* x_out, float* zero_tokens, void* workspace,
+                               void* stream);   /* ... that clears zero_tokens (n_tokens floats, may be NULL) as ntk_rmsnorm_rowmax does */
 int ntk_rows_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials, void* workspace, void* stream);
 
 /* Prompts of at most 32 tokens, whose projections keep a K slice's planes in LDS: their producers scale X per token and 256 columns, so that they need no whole row in one workgroup.

@@ -841,9 +841,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
     // (up to 64 tokens: a producer that owns a whole token per workgroup writes its planes in 16-byte pieces a kilobyte apart -- at 1024 tokens the pass
     // measured 5 % SLOWER than with the GEMM's own pre-pass, 8B Q8_0 28 010 -> 26 460 tok/s; at 16 - 64 tokens it is 2 - 5 % faster)
     const bool fuse_split = with_max && prefill_fused_split_ && gemm_ws2_ != nullptr && T <= 64;
-    // (... beyond: four tokens a workgroup, rows_split_kernel, where its registers hold the row; wider rows leave their maxima)
+    // (... beyond: four tokens a workgroup, rows_split_kernel, where its registers hold the row and few pieces are added up; other rows leave their maxima)
     const bool rows_split = with_max && prefill_fused_split_ && gemm_ws2_ != nullptr && T > 64;
-    auto splits_rows = [&](size_t width, bool norm) { return fuse_split || (rows_split && ntk_rows_prepare_takes(T, (int)width, norm ? 1 : 0)); };
+    auto splits_rows = [&](size_t width, bool norm, int nsplit) { return fuse_split || (rows_split && ntk_rows_prepare_pays(T, (int)width, norm ? 1 : 0, nsplit)); };
     auto f16_ok = [&](const DevTensor& w) {   // the formats and shapes ntk_gemm_quant_f16 takes
         const bool kq = w.dtype == NTK_DT_Q4_0 || w.dtype == NTK_DT_Q4_K || w.dtype == NTK_DT_Q5_K || w.dtype == NTK_DT_Q6_K;
         return (w.dtype == NTK_DT_Q8_0 || kq) && w.in_f % (kq ? 256 : 128) == 0 && w.out_f % 16 == 0 && (w.ptr || w.rp);
@@ -856,7 +856,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         return true;
     };
     auto prepare_x = [&](const float* X, const DevTensor& w) {   // X as it lies (the attention output): row maximum + split in one launch
-        if (!splits_rows(w.in_f, false) || !f16_ok(w) || X == planes_of) return;
+        if (!splits_rows(w.in_f, false, 0) || !f16_ok(w) || X == planes_of) return;
         void* ws = flip_ws();
         if ((fuse_split ? ntk_gemm_prepare_x(X, T, (int)w.in_f, ws, s) : ntk_rows_prepare_x(X, T, (int)w.in_f, ws, s)) == NTK_OK) planes_of = X;
         else planes_of = nullptr;
@@ -1001,9 +1001,9 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         project(residual_, w, X, H, xstride, rm);
         ok(ntk_add_inplace(hidden_, residual_, T * H, s));
     };
-    auto left_max = [&](bool written, bool zero_b) {   // a norm has written residual_ (zero_b: the layer's first, which clears rm_b if it leaves maxima at all)
+    auto left_max = [&](bool written, bool zero_b, bool cleared = false) {   // a norm has written residual_ (zero_b: the layer's first, which clears rm_b if it leaves maxima at all, or cleared)
         max_a = written ? rm_a : nullptr;
-        if (zero_b) b_clear = written && rm_b;
+        if (zero_b) b_clear = (written || cleared) && rm_b;
     };
     auto norm = [&](const DevTensor& nw, bool zero_b, const DevTensor& next_w, bool only, bool half) {     // only, half: planes_only, half_only of the matrices that read it
         halves_of = nullptr;
@@ -1014,12 +1014,12 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             left_max(false, zero_b);
             return;
         }
-        if (splits_rows(H, true) && f16_ok(next_w) && (int)next_w.in_f == H) {
+        if (splits_rows(H, true, 0) && f16_ok(next_w) && (int)next_w.in_f == H) {
             void* ws = flip_ws();
             ok(fuse_split ? ntk_rmsnorm_prepare_x(residual_, hidden_, (const float*)nw.ptr, T, H, cfg_.norm_eps, ws, s)
-                          : ntk_rows_norm_prepare_x(hidden_, nullptr, (const float*)nw.ptr, T, H, cfg_.norm_eps, only ? nullptr : residual_, ws, s));
+                          : ntk_rows_norm_prepare_zero(hidden_, nullptr, (const float*)nw.ptr, T, H, cfg_.norm_eps, only ? nullptr : residual_, zero_b ? rm_b : nullptr, ws, s));
             planes_ready = residual_;
-            left_max(false, zero_b);
+            left_max(false, zero_b, !fuse_split);
             return;
         }
         left_max(with_max, zero_b);
@@ -1043,7 +1043,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         if (!with_max || tp_world_ > 1 || !is_quant(w.dtype) || (size_t)w.out_f != (size_t)H) return false;
         ntk_gemm_partials pt;
         int st = NTK_E_DTYPE;
-        prepare_x(X, w);
+        if (fuse_split || !rm) prepare_x(X, w);   // (where its maxima are there, the GEMM's own split is the faster)
         if (rp_only(w)) {   // straight from the repack
             const ntk_gemv_seg sg{w.rp, hidden_, (int)w.out_f, w.dtype};
             st = gemm_f16(&sg, 1, X, (int)w.in_f, hidden_, X == planes_of ? 1 : 0, rm, &pt, true);
@@ -1066,12 +1066,13 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
         }
         halves_of = nullptr;
         planes_of = nullptr;
-        if (st == NTK_OK && splits_rows(H, true) && f16_ok(next_w) && (int)next_w.in_f == H) {   // (the partial sums lie in cur_ws: the planes go to the other one)
+        const int pieces = pt.nsplit > 1 ? pt.nsplit : pt.y[0] != hidden_ ? 1 : 0;
+        if (st == NTK_OK && splits_rows(H, true, pieces) && f16_ok(next_w) && (int)next_w.in_f == H) {   // (the partial sums lie in cur_ws: the planes go to the other one)
             void* ws = flip_ws();
             st = fuse_split ? ntk_reduce_rmsnorm_prepare_x(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, ws, s)
-                            : ntk_rows_norm_prepare_x(hidden_, &pt, (const float*)nw.ptr, T, H, cfg_.norm_eps, only ? nullptr : residual_, ws, s);
+                            : ntk_rows_norm_prepare_zero(hidden_, &pt, (const float*)nw.ptr, T, H, cfg_.norm_eps, only ? nullptr : residual_, zero_b ? rm_b : nullptr, ws, s);
             planes_ready = residual_;
-            left_max(false, zero_b);
+            left_max(false, zero_b, !fuse_split);
         } else
         if (st == NTK_OK) left_max(true, zero_b), st = ntk_reduce_rmsnorm_rowmax(hidden_, &pt, (const float*)nw.ptr, cfg_.norm_eps, residual_, rm_a, zero_b ? rm_b : nullptr, s);
         ok(st);
@@ -1138,7 +1139,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             ntk_gemm_partials pt;
             int st = gemm_f16(segs, 2, residual_, (int)L.w_gate.in_f, nullptr, residual_ == planes_of ? 1 : 0, max_a, &pt, both_rp);
             if (st != NTK_E_DTYPE && st != NTK_E_SHAPE && st != NTK_E_ALIGN) {   // (those three: nothing was launched)
-                if (st == NTK_OK && splits_rows(I, false) && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I) {
+                if (st == NTK_OK && splits_rows(I, false, pt.nsplit) && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I) {
                     void* ws = flip_ws();
                     st = fuse_split ? ntk_reduce_silu_mul_prepare_x(gate_buf, &pt, ws, s) : ntk_rows_silu_mul_prepare_x(planes_only({&L.w_down}, I) ? nullptr : gate_buf, &pt, ws, s);
                     planes_ready = gate_buf;
@@ -1158,7 +1159,7 @@ int Model::layers_1to1(int T, int start_pos, int first, int last_layer, bool key
             const DevTensor* const ws[2] = {&L.w_gate, &L.w_up};
             project_many(ys, ws, 2, residual_, max_a);
             int st_silu = NTK_E_SHAPE;   // (in place: exactly one of these launches runs)
-            if (splits_rows(I, false) && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I && tp_world_ == 1) {
+            if (splits_rows(I, false, 1) && f16_ok(L.w_down) && (size_t)L.w_down.in_f == (size_t)I && tp_world_ == 1) {
                 ntk_gemm_partials pt{};
                 pt.nseg = 2; pt.n_tokens = T; pt.nsplit = 1; pt.y[0] = gate_buf; pt.y[1] = up_buf; pt.rows[0] = pt.rows[1] = I;
                 void* ws = flip_ws();

@@ -433,6 +433,7 @@ struct RowsSplitParams {
     float* hidden;         // NORM: += the sums
     const float* weight;
     float* out;            // the rows themselves, if anything but the planes is read (may be NULL)
+    float* zero;           // NORM: a float a token to clear (may be NULL)
     int nsplit, T, W;
     float eps;
     uint8_t* ws;
@@ -546,6 +547,8 @@ __global__ __launch_bounds__(1024) void rows_split_kernel(const RowsSplitParams 
     const float sc = __uint_as_float((uint32_t)es << 23);
     const size_t chunk_bytes = ws_chunk_bytes(W);
     if (tid < RS_TOK) reinterpret_cast<float*>(p.ws + (size_t)GB_MAX_CHUNKS * chunk_bytes)[t] = __uint_as_float((uint32_t)(254 - es) << 23);   // 1 / s
+    if constexpr (MODE == RS_NORM)
+        if (p.zero && tid < RS_TOK && t < p.T) p.zero[t] = 0.0f;
     const int tl = t & (GB_TOK - 1), tb = tl >> 4, j16 = tl & 15;
     uint8_t* chunk = p.ws + (size_t)(t / GB_TOK) * chunk_bytes;
     u32x4* xb = reinterpret_cast<u32x4*>(chunk) + tb * 64 + (j16 + 16 * g);
@@ -2931,6 +2934,20 @@ int ntk_reduce_silu_mul_prepare_x(float* output, const ntk_gemm_partials* p, voi
 int ntk_rows_prepare_takes(int n_tokens, int width, int norm) {
     return n_tokens > ntk::GB_TOK && n_tokens <= ntk::GB_MAX_CHUNKS * ntk::GB_TOK && width > 0 && width % 32 == 0 && ntk::rows_split_turns(width, !norm) > 0;
 }
+// Where that launch is ahead of the two that leave the rows with their maxima and split them.  Four tokens a workgroup are a quarter of the workgroups, each of which walks its pieces one after the
+// other: with few tokens the launches of a token a workgroup are ahead as soon as there are pieces.  us by which a pass of several layers grew for one of them (width, tokens): a norm over eight pieces
+// 2048, 200 + 11, over four 4096, 100 + 5, 4096, 330 + 2.3, 3072, 512 + 2.5, over two 768, 200 + 1.3, 1024, 330 + 0.8, 1024, 850 - 2, 2048, 600 - 3.7, 4096, 1000 - 7, 5120, 700 - 7, 8192, 256 + 8,
+// 8192, 400 + 4, 8192, 512 - 11; a whole unit 5632, 150 + 4, 5632, 600 - 0.4, 5632, 850 - 4.6, 8192, 100 + 3, 8192, 512 - 2, 8192, 1000 - 7, 14336, 100 + 9, 14336, 330 - 1.5, 14336, 600 - 7, 14336,
+// 1000 - 16, of two pieces 2816, 200 + 1.2, 2816, 850 - 3, 14336, 200 + 14 (in front of a product alone, 700 tokens, 5120 17.4 / 20.2, 8192 24.4 / 21.4), of four 2816, 512 + 7; rows as they lie 768,
+// 65 - 1.4, 1024, 330 - 3, 4096, 100 - 4, 4096, 850 - 9: always.  A norm of whole rows (one a pass): 4096, 100 / 330 / 1024 in front of a product alone 10.9 / 13.2 / 18.0, so 8.7 / 9.5 / 9.5.
+int ntk_rows_prepare_pays(int n_tokens, int width, int norm, int nsplit) {
+    if (!ntk_rows_prepare_takes(n_tokens, width, norm) || nsplit < 0 || nsplit > 2) return 0;
+    const long long size = (long long)n_tokens * width;
+    if (norm) return nsplit == 0 || (nsplit == 1 ? width <= 4096 || n_tokens >= 330 : n_tokens >= 600 || (width > 5120 && n_tokens >= 512));
+    if (nsplit == 0) return 1;
+    if (nsplit == 1) return n_tokens >= 512 && size >= 3900000;
+    return n_tokens >= 700 && width >= 2560 && (width <= 4096 || size >= 5200000);
+}
 static bool rows_aligned(std::initializer_list<const void*> ps) {
     for (const void* q : ps)
         if (reinterpret_cast<uintptr_t>(q) & 15) return false;
@@ -2945,6 +2962,9 @@ int ntk_rows_prepare_x(const float* X, int n_tokens, int width, void* workspace,
     return ntk::rows_split<ntk::RS_LIES>(p, ntk::resolve_stream(stream));
 }
 int ntk_rows_norm_prepare_x(float* hidden, const ntk_gemm_partials* q, const float* weight, int n_tokens, int width, float eps, float* x_out, void* workspace, void* stream) {
+    return ntk_rows_norm_prepare_zero(hidden, q, weight, n_tokens, width, eps, x_out, nullptr, workspace, stream);
+}
+int ntk_rows_norm_prepare_zero(float* hidden, const ntk_gemm_partials* q, const float* weight, int n_tokens, int width, float eps, float* x_out, float* zero_tokens, void* workspace, void* stream) {
     if (!hidden || !weight || !workspace) return NTK_E_NULL;
     if (!ntk_rows_prepare_takes(n_tokens, width, 1)) return NTK_E_SHAPE;
     ntk::RowsSplitParams p{};
@@ -2955,7 +2975,7 @@ int ntk_rows_norm_prepare_x(float* hidden, const ntk_gemm_partials* q, const flo
         p.nsplit = sums ? q->nsplit : q->y[0] != hidden ? 1 : 0;   // (a projection that did not split wrote y, hidden's own rows with the residual if that is where y lies)
     }
     if (!rows_aligned({hidden, weight, x_out, workspace, p.a})) return NTK_E_ALIGN;
-    p.hidden = hidden; p.weight = weight; p.eps = eps; p.out = x_out; p.T = n_tokens; p.W = width; p.ws = static_cast<uint8_t*>(workspace);
+    p.hidden = hidden; p.weight = weight; p.eps = eps; p.out = x_out; p.zero = zero_tokens; p.T = n_tokens; p.W = width; p.ws = static_cast<uint8_t*>(workspace);
     return ntk::rows_split<ntk::RS_NORM>(p, ntk::resolve_stream(stream));
 }
 int ntk_rows_silu_mul_prepare_x(float* output, const ntk_gemm_partials* q, void* workspace, void* stream) {
