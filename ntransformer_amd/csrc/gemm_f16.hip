@@ -2616,7 +2616,8 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     // two chunks (128 tokens) per workgroup when that still gives every CU two workgroups -- directly, or (narrow matrices: the 8B down /
     // o / Q|K|V projections at 1024 tokens) with K split in two.  From six chunks on three workgroups for two CUs are enough, and K may go in four: us, six layers of the 8B shape, one chunk a
     // workgroup there / two, 330 tokens Q8_0 3200 / 3085, Q4_K_M 3190 / 3130; 400 3650 / 3452, 3710 / 3580; 600 4771 / 4690, 4890 / 4830; 800 5930 / 5655, 6150 / 5970; two layers of the 70B shape,
-    // 700 tokens Q8_0 3980 / 3850.  With two chunks the same cost 8B Q4_K_M 1.5 %, with five 0.5 %.
+    // 700 tokens Q8_0 3980 / 3850.  With two chunks the same cost 8B Q4_K_M 1.5 %, with five 0.5 %.  Two layers of the 70B shape, one chunk a workgroup at any length / so, 330, 500, 800, 1024 tokens:
+    // Q8_0 2589, 3247, 5163, 5860 / 2328, 2843, 4687, 5160, Q4_K_M 2496, 3132, 4847, 5621 / 2307, 2843, 4473, 5207; four of the 8B shape Q8_0 2163, 2459, 3884, 4286 / 1992, 2336, 3538, 3828.
     int nsplit = splits_for(chunks64);
     bool cw2 = false;
     if (CW2_OK && al && rt == 2 && chunks64 >= 2 && force_cw != 1) {
