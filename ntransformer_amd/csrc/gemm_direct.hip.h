@@ -22,6 +22,7 @@ struct DirectArgs {
     uint16_t* Y16; int ldy16; int glu_ff;           // bfloat16 results in the place of t.Y (or NULL); gated units: [r][f] of the weight rows f behind gate_at and up_at bytes of W
     uint32_t gate_at, up_at;
     float limit, alpha, up_offset, cubic;
+    int tile_rows;                                  // EVEN forms: rows of a tile, whole pieces of sixteen
     // several matrices side by side over the same activations (n_seg > 1, no groups, nothing accumulated): the column tiles of one after those of the other, their pieces' columns too
     int n_seg; const void* segW[3]; float* segY[3]; int seg_out[3], seg_tile[3];
 };
@@ -69,6 +70,10 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
     constexpr int CB = 128, ES = sizeof(typename P::WT), BK = CB / ES, PIECES = P::PIECES, NW = WM * WN, WTM = TM / WM, WTN = TN / WN, MI = WTM / 16, NJ = WTN / 16;
     constexpr int NX = TM / (8 * NW), NWL = TN / (8 * NW), LPS = NX * PIECES + NWL;      // requests of a wave: X per plane, W; per chunk
     constexpr int XB = TM * CB, STAGE = (PIECES * TM + TN) * CB;
+    // the rows go evenly over the tiles (never in groups): two pieces an activation leave the matrix cores and LDS both full, so that rows a tile does not have count.  200 rows 112 -> 107 us, 130 111 -> 92
+    // (28672 x 4096), 130 of 4096 x 14336 in eight pieces 54 -> 47.  Not smaller tiles (64 x 128: 51 -> 54, what a step asks each time) and not bfloat16, which waits for its weights then (even tiles of
+    // 1024 rows in 32 groups of 2816 x 2048: no gain)
+    constexpr bool EVEN = PIECES > 1 && TM >= 128;
     static_assert(TM % (8 * NW) == 0 && TN % (8 * NW) == 0, "whole requests");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[STAGES * STAGE];
     // consecutive workgroups go to the eight XCDs in turn: each takes a contiguous range of tiles, so that the row tiles of a column share its weights in one L2
@@ -87,10 +92,10 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
         Wp = seg_pick(d.segW, sg); Yp = seg_pick(d.segY, sg); n_cols = ldy = seg_pick(d.seg_out, sg);
         part_col = (sg > 0 ? d.seg_out[0] : 0) + (sg > 1 ? d.seg_out[1] : 0);
     }
-    int g = 0, row_base = rt * TM, r1 = a.T;
+    int g = 0, row_base = rt * (EVEN ? d.tile_rows : TM), r1 = EVEN ? min(a.T, row_base + d.tile_rows) : a.T;
     if (a.offsets) { if (!group_tile(a.offsets, a.G, rt, TM, g, row_base, r1)) return; }
     const int n_base = ct * (GLU ? TN / 2 : TN);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = EVEN ? wave / WN : wave % WM, wn = EVEN ? wave % WN : wave / WM;
     const int k_begin = split * a.k_per_split, k_end = min(a.K, k_begin + a.k_per_split), n_chunks = (k_end - k_begin) / BK;
     // a request brings eight rows of 128 bytes; the 16-byte pieces of row r are stored in the order piece ^ (r & 7)
     uint32_t xo[NX], wo[NWL];
@@ -140,7 +145,10 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) { total[i][j] += acc[i][j]; acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f}; }
     };
-    const bool idle = row_base + wm * WTM >= r1;    // (uniform) rows past the group's end: nothing to multiply, the matrix cores are a neighbour's
+    // (uniform) EVEN: the tile's pieces of sixteen rows, shared among the waves of a column (wm differs between the two waves of a SIMD, so that each SIMD has its share of those left out)
+    const int pieces16 = (r1 - row_base + 15) / 16, n16 = EVEN ? pieces16 / WM + (wm < pieces16 % WM ? 1 : 0) : MI;
+    const int first_row = EVEN ? 16 * (wm * (pieces16 / WM) + min(wm, pieces16 % WM)) : wm * WTM, row_end = EVEN ? min(r1, row_base + first_row + 16 * n16) : r1;
+    const bool idle = row_base + first_row >= row_end;    // (uniform) rows past the group's end: nothing to multiply, the matrix cores are a neighbour's
     auto multiply = [&](int slot) {
         const uint8_t* s = lds + slot * STAGE;
 #pragma unroll
@@ -153,16 +161,21 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
             for (int q = 0; q < PIECES; ++q) {
                 uintx4_t xf[MI];
 #pragma unroll
-                for (int i = 0; i < MI; ++i) xf[i] = *reinterpret_cast<const uintx4_t*>(s + q * XB + (wm * WTM + i * 16) * CB + piece);
+                for (int i = 0; i < MI; ++i) {
+                    if (EVEN && i && i >= n16) break;
+                    xf[i] = *reinterpret_cast<const uintx4_t*>(s + q * XB + (first_row + i * 16) * CB + piece);
+                }
 #pragma unroll
                 for (int c = 0; c < P::STEPS; ++c)          // (neighbouring instructions on different accumulators)
 #pragma unroll
-                    for (int i = 0; i < MI; ++i)
+                    for (int i = 0; i < MI; ++i) {
+                        if (EVEN && i && i >= n16) break;
 #pragma unroll
                         for (int j = 0; j < NJ; ++j) {
                             if (SEP && q > 0) low[SEP ? i : 0][SEP ? j : 0] = P::step(xf[i], wf[j], low[SEP ? i : 0][SEP ? j : 0], c);
                             else acc[i][j] = P::step(xf[i], wf[j], acc[i][j], c);
                         }
+                    }
             }
         }
     };
@@ -197,10 +210,10 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
         const int col = n_base + wn * (WTN / 2) + (lane & 15), n_left = n_cols - col;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-            const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
+            const int row = row_base + first_row + i * 16 + (lane >> 4) * 4;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const bool in = row + r < r1;
+                const bool in = row + r < row_end;
                 const float undo = P::SCALED ? half_unscale(a.row_max[min(row + r, a.T - 1)]) : 1.0f;
                 float* y = Yp + (long long)(row + r) * ldy + col;
 #pragma unroll
@@ -217,12 +230,12 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
         const int col = n_base + wn * (WTN / 2) + (lane & 15), n_left = n_cols - col;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-            const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
+            const int row = row_base + first_row + i * 16 + (lane >> 4) * 4;
 #pragma unroll
             for (int j = 0; j < NJ / 2; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (row + r < r1 && j * 16 < n_left) {
+                    if (row + r < row_end && j * 16 < n_left) {
                         const float gg = fminf(acc[i][j][r], d.limit), uu = fminf(fmaxf(acc[i][NJ / 2 + j][r], -d.limit), d.limit);
                         const float zz = d.cubic != 0.0f ? fmaf(d.cubic * gg * gg, gg, gg) : gg;
                         const float v = gg * (1.0f / (1.0f + expf(-d.alpha * zz))) * (uu + d.up_offset);
@@ -235,7 +248,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
     const int col = n_base + wn * WTN + (lane & 15), n_left = n_cols - col;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-        const int row = row_base + wm * WTM + i * 16 + (lane >> 4) * 4;
+        const int row = row_base + first_row + i * 16 + (lane >> 4) * 4;
         float undo[4] = {1.0f, 1.0f, 1.0f, 1.0f};
         if constexpr (P::SCALED)
 #pragma unroll
@@ -246,7 +259,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (row + r < r1 && j * 16 < n_left) y[(long long)r * a.N + j * 16] = acc[i][j][r] * undo[r];
+                    if (row + r < row_end && j * 16 < n_left) y[(long long)r * a.N + j * 16] = acc[i][j][r] * undo[r];
             continue;
         }
         float* y = Yp + (long long)row * ldy + col;
@@ -255,12 +268,12 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) old[j][r] = row + r < r1 && j * 16 < n_left ? y[(long long)r * ldy + j * 16] : 0.0f;
+                for (int r = 0; r < 4; ++r) old[j][r] = row + r < row_end && j * 16 < n_left ? y[(long long)r * ldy + j * 16] : 0.0f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (row + r < r1 && j * 16 < n_left) {
+                if (row + r < row_end && j * 16 < n_left) {
                     float v = acc[i][j][r] * undo[r];
                     if (a.accumulate) v += old[j][r];
                     else if (a.act == 1) { const float p = fmaxf(v, 0.0f); v = p * p; }          // NTK_ACT_RELU2
@@ -274,7 +287,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 // n * busy a chunk, one alone `alone` (latency).  Constants in us, from layer-like shapes of 16 .. 1024 rows (groups: 600 .. 6144), 2048 .. 14976 outputs, 512 .. 7488 inputs with weights
 // that come from memory; the estimate is within a sixth there, and the choice within a tenth of the best form but for uneven small groups.  Rows of several groups: tiles
 // of a group of the average size, plus half a tile where that is no small part of one.
-struct DirectForm { int TM, TN, resident; float alone, busy, over; };
+struct DirectForm { int TM, TN, resident; float alone, busy, over, even; };       // even: the part of a chunk's time that goes with the rows a tile has (rows evenly over the tiles)
 static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats) {
     static const int counts[] = {1, 2, 3, 4, 6, 8, 12, 16};
     TilePlan best{0, 1, 1e30f};
@@ -286,7 +299,8 @@ static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int row
         for (int s : counts) {
             if (s > 1 && ((long long)s * rows * N > scratch_floats || chunks < 4 * s)) break;
             const int n = (int)((tiles * s + 255.0f) / 256.0f);
-            float us = (float)((chunks + s - 1) / s) * (n == 1 ? f[i].alone : n * f[i].busy) + f[i].over * ((n + f[i].resident - 1) / f[i].resident);
+            const float full = 1.0f - f[i].even * (1.0f - std::min(1.0f, mean / row_tiles));
+            float us = (float)((chunks + s - 1) / s) * full * (n == 1 ? f[i].alone : n * f[i].busy) + f[i].over * ((n + f[i].resident - 1) / f[i].resident);
             if (s > 1) us += 3.0f + (float)(s + 1) * rows * N * 4.0f / 7e6f;
             if (us < best.us) best = TilePlan{i, s, us};
         }
@@ -329,6 +343,7 @@ static int launch_direct(DirectArgs d, int splits, hipStream_t s, bool sum = tru
     d.t.k_per_split = per * BK;
     d.t.splits = (chunks + per - 1) / per;
     const int row_tiles = d.t.offsets ? d.t.T / TM + d.t.G : (d.t.T + TM - 1) / TM;
+    d.tile_rows = ((d.t.T + 15) / 16 + row_tiles - 1) / row_tiles * 16;
     int col_tiles = GLU ? (d.glu_ff + TN / 2 - 1) / (TN / 2) : (d.t.N + TN - 1) / TN;
     if (d.n_seg > 1) {
         col_tiles = 0;

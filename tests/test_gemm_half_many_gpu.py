@@ -77,6 +77,16 @@ def test_gated_unit_in_the_launch(T, K, ff):
         assert (np.abs(y - g * s * u) <= bound).all()
 
 
+@pytest.mark.parametrize("T", [129, 144, 145, 161, 200, 257, 300])
+def test_rows_shared_evenly_over_tiles(T):
+    """the 128 x 256 form (28672 columns: it is the estimate's choice) where its row tiles are not full: 5 and 4 sixteens of 128 rows, odd counts, a last row of its own, three tiles"""
+    x, ws = values(T, 1024, (14336, 14336), T)
+    y = run(x, ws, silu=True)
+    (g, bg), (u, bu) = product(x, ws[0]), product(x, ws[1])
+    s = 1.0 / (1.0 + np.exp(-g))
+    assert (np.abs(y - g * s * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(g * s) * bu + 16 * U * np.abs(g * s * u) + 1e-37).all()
+
+
 def test_a_row_that_is_not_finite_and_what_is_refused():
     x, ws = values(20, 128, (70, 70), 3)
     x[4, 9], x[6, 1] = np.nan, np.inf
