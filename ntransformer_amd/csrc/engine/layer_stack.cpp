@@ -924,7 +924,14 @@ int LayerStackModel::load(const std::string& dir, const SeqLoadOptions& opt) {
 
 int LayerStackModel::alloc_buffers() {
     const int W = info_.width;
-    chunk_ = std::min(opt_.max_context, 1024);
+    // Tokens of an internal pass: every launch of a layer runs once a pass, so a prompt cut in two pays its launches, its weights' way to the matrix cores and each launch's last wave twice.
+    // us a prompt, passes of 1024 / 2048 / 4096 tokens: attention, recurrence and latents in bfloat16 (2048 wide, four layers), 1100 tokens 1698 / 1382 / 1376, 1999 2345 / 1972 / 1972, 2500
+    // 3194 / 2763 / 2508, 8000 10578 / 8640 / 8261; in float32, 1999 tokens 7535 / 7180 / 7172; two layers of 32 experts, 1100 tokens 1127 / 823 / 823, 2500 2021 / 1700 / 1463, 8000 7014 /
+    // 5476 / 5070.  (The workspaces go with it: about a gigabyte at these widths.)  A token's choices of experts are rows of their own, and rows a grid's second dimension.
+    chunk_ = 4096;
+    for (const auto& L : layers_)
+        if (L.mlp_kind == kMlpMoe) while (chunk_ > 1024 && (long long)chunk_ * L.mlp.top > 32768) chunk_ /= 2;
+    chunk_ = std::min(opt_.max_context, chunk_);
     size_t sc = 0, wsc = 0, lsc = 0, rsc = 0;
     // what a portion's attention sees at most, in pieces: the portion and a window ahead of it (and the positions that stay visible), or everything
     auto seen = [&](int window, int keep, int kv_heads, int dk, int dv) {
@@ -1795,7 +1802,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
     }
     if (capture_) {
         const size_t cf = runs_.size() * (size_t)n * info_.width;
-        if (n > chunk_) { err_ = "capture: the portion must fit one internal pass"; return nullptr; }
+        if (n > std::min(chunk_, 1024)) { err_ = "capture: the portion must fit one internal pass"; return nullptr; }
         if (cf > capture_floats_) {
             ntk_stream_synchronize(stream_);
             if (capture_buf_) nt_hip_free(capture_buf_);
