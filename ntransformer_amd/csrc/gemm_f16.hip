@@ -35,6 +35,7 @@
 // Bound: instruction issue (MFMA + VALU of two waves per SIMD) under a 1.65-1.7 GHz clock; matrix pipe 41 % busy.
 #include "common.hip.h"
 #include "gemm_planes.hip.h"
+#include "gemm_short.hip.h"
 #include <algorithm>
 #include <cstdlib>
 #include <initializer_list>
@@ -2375,6 +2376,24 @@ struct ShortArgs {
 };
 struct HostSeg { float* Y; const void* W; int out; };
 
+// sums of n slices (1: Y is written) to the caller's next launch, which adds them up (and the residual) itself, or into Y
+static int leave_slices(const HostSeg* segs, int nseg, const float* const* parts, int n, int T, const float* resid, ntk_gemm_partials* defer, hipStream_t st) {
+    if (defer) {
+        defer->nseg = nseg; defer->n_tokens = T; defer->nsplit = n;
+        for (int i = 0; i < nseg; ++i) { defer->part[i] = n > 1 ? const_cast<float*>(parts[i]) : nullptr; defer->y[i] = segs[i].Y; defer->rows[i] = segs[i].out; }
+    } else if (n > 1) {
+        ReduceArgs ra{};
+        ra.nseg = nseg; ra.T = T; ra.nsplit = n; ra.resid = resid;
+        size_t biggest = 0;
+        for (int i = 0; i < nseg; ++i) {
+            ra.Y[i] = segs[i].Y; ra.part[i] = parts[i]; ra.out[i] = segs[i].out;
+            biggest = std::max(biggest, ((size_t)T * segs[i].out + 3) / 4);
+        }
+        hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((biggest + 255) / 256), nseg), dim3(256), 0, st, ra);
+    }
+    return last_launch_status();
+}
+
 // a matrix's pieces are addressed with 32-bit offsets
 template <class D>
 static bool offsets_fit(int out, int in) {
@@ -2436,6 +2455,29 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     for (int i = 0; i < nseg; ++i) outs[i] = segs[i].out;
     const KSlicePlan plan = kslice_plan<DT>(outs, nseg, T, in);
     if (sh.on && (plan.n == 0 || sh.part_at + (size_t)plan.n * T * (size_t)out_total > sh.part_cap)) return NTK_E_SHAPE;   // (nothing launched: the planes were there)
+    if constexpr (D::RP) {
+        // 2 .. 16 tokens, many rows: the planes in registers (gemm_short.hip); never in more slices than the form below, so that its sums fit where that one's do
+        const ShortStreamPlan sp = sh.on && T <= SS_TOKENS ? short_stream_plan(DT - GB_RP, in / 256, (int)(out_total / 16), plan.n, plan.jobs * plan.ups * KD::SPU * plan.rt) : ShortStreamPlan{};
+        if (sp.n > 0) {
+            ShortStreamParams q{};
+            q.nseg = nseg; q.T = T; q.in = in; q.units = in / 256; q.tiles = (int)(out_total / 16);
+            q.xb = wsb; q.aux = reinterpret_cast<const uint8_t*>(p.aux); q.group_inv = group_inv;
+            if (sh.norm) { q.ssq = group_inv + ws_group_floats(in); q.nssq = (in + 511) / 512; q.eps = sh.eps; }
+            q.ups = sp.ups; q.groups = sp.groups; q.resid = sp.n == 1 ? resid : nullptr;
+            float* part = reinterpret_cast<float*>(wsb + ws_part_offset(in)) + sh.part_at;
+            const float* parts[GB_MAX_SEG] = {};
+            int tile = 0;
+            for (int i = 0; i < nseg; ++i) {
+                q.seg[i] = ShortStreamSeg{static_cast<const uint8_t*>(segs[i].W), segs[i].Y, part, segs[i].out, tile,
+                                          (uint32_t)((size_t)(segs[i].out / 16) * (size_t)q.units * (size_t)(2 * D::S1))};
+                parts[i] = part;
+                tile += segs[i].out / 16;
+                part += (size_t)sp.n * T * segs[i].out;
+            }
+            const int rc = short_stream_launch(DT - GB_RP, q, sp, st);
+            return rc == NTK_OK ? leave_slices(segs, nseg, parts, sp.n, T, resid, defer, st) : rc;
+        }
+    }
     {
         const int ntb = T <= 16 ? 1 : 2;
         const int best_n = plan.n, best_rt = plan.rt, best_ups = plan.ups, best_jobs = plan.jobs;
@@ -2495,22 +2537,9 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
             using I1 = std::integral_constant<int, 1>; using I2 = std::integral_constant<int, 2>;
             if (best_rt == 1) { if (ntb == 1) go(I1{}, I1{}); else go(I1{}, I2{}); }
             else { if (ntb == 1) go(I2{}, I1{}); else go(I2{}, I2{}); }
-            if (defer) {   // the caller's next launch sums the slices (and adds the residual) itself
-                defer->nseg = nseg; defer->n_tokens = T; defer->nsplit = best_n;
-                for (int i = 0; i < nseg; ++i) { defer->part[i] = best_n > 1 ? kp.seg[i].part : nullptr; defer->y[i] = segs[i].Y; defer->rows[i] = segs[i].out; }
-                if (best_n > 1) return last_launch_status();
-            }
-            if (best_n > 1) {
-                ReduceArgs ra{};
-                ra.nseg = nseg; ra.T = T; ra.nsplit = best_n; ra.resid = resid;
-                size_t biggest = 0;
-                for (int i = 0; i < nseg; ++i) {
-                    ra.Y[i] = segs[i].Y; ra.part[i] = kp.seg[i].part; ra.out[i] = segs[i].out;
-                    biggest = std::max(biggest, ((size_t)T * segs[i].out + 3) / 4);
-                }
-                hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((biggest + 255) / 256), nseg), dim3(256), 0, st, ra);
-            }
-            return last_launch_status();
+            const float* parts[GB_MAX_SEG] = {};
+            for (int i = 0; i < nseg; ++i) parts[i] = kp.seg[i].part;
+            return leave_slices(segs, nseg, parts, best_n, T, resid, defer, st);
         }
     }
     // ---- short prompts (<= 32 tokens): the weight-streaming form (gemm_quant_f16_small_kernel) ----

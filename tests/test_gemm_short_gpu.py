@@ -230,3 +230,56 @@ def test_a_scale_per_group_is_no_further_from_64_bits_than_one_per_token(qname, 
         errs.append(float(np.sqrt(np.mean(((y.numpy(np.float32).reshape(T, rows) - want) / size) ** 2))))
     print("rms error over size, a scale per group / per token:", errs)
     assert errs[0] <= 1.1 * errs[1]
+
+
+@pytest.mark.parametrize("qname", ["Q4_K", "Q5_K", "Q6_K"])
+@pytest.mark.parametrize("T,rows,inf", [(2, (16,), 256), (7, (16, 16, 16), 28672), (16, (4096, 80), 1280), (16, (65536,), 256), (9, (43008, 16), 768), (2, (33024,), 1024), (16, (20480, 48, 6000), 1280),
+                                        (5, (16400,), 2304), (16, (9216, 4096), 2816), (3, (6160,), 6144)])
+def test_products_through_the_decode_repack(qname, T, rows, inf):
+    """the repack through either form: with its planes in LDS (few rows) and in registers (gemm_short.hip: many) -- one unit of 256 columns, three, four, five, nine, eleven, 24 over its waves and
+    slices, tiles that end inside a batch, several matrices, the norm's 1 / rms, a residual.  Values and bound as above."""
+    gt = getattr(G, "GGML_" + qname)
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[T, sum(rows) + inf]))
+    from ntransformer_amd import ops
+    mats, dt = [], None
+    for n in rows:
+        raw, W, dt = weights(r, gt, n, inf)
+        mats.append((ops.rp_pack(DB.from_numpy(raw), n, inf, dt), W))
+    assert L.ntk_gemm_short_takes((C.c_int * len(rows))(*rows), len(rows), T, inf, dt)
+    nbytes = L.ntk_gemm_quant_workspace_bytes(inf, sum(rows))
+    ws = DB.zeros(nbytes)
+    X = r.standard_normal((T, inf)).astype(np.float32)
+    X[:, 64:320] *= np.float32(1e4)
+    X[T // 2, : inf // 2] = 0.0
+    X[0] *= np.float32(1e12)
+    X[T - 1] *= np.float32(1e-12)
+
+    def go(normed, eps=0.0, resid=None, partials=None):
+        ys = [DB.from_numpy(np.full((T, n), 7.0, np.float32)) for n in rows] if resid is None else [resid]
+        segs = (_lib.GemvSeg * len(rows))()
+        for s, (w, _), y, n in zip(segs, mats, ys, rows):
+            s.W, s.y, s.rows, s.dtype = w.ptr, y.ptr, n, dt
+        d = _lib.GemmDesc()
+        d.segs, d.nseg, d.n_tokens, d.in_features, d.resid, d.weights_repacked = segs, len(rows), T, inf, None if resid is None else resid.ptr, 1
+        d.workspace, d.workspace_bytes = ws.ptr, nbytes
+        d.partials = C.pointer(partials) if partials is not None else None
+        _lib.check(L.ntk_gemm_short(C.byref(d), normed, eps, 0, None), "gemm_short")
+        return [y.numpy(np.float32).reshape(T, n).astype(np.float64) for y, n in zip(ys, rows)]
+    Xd = DB.from_numpy(X)
+    _lib.check(L.ntk_short_prepare_x(Xd.ptr, T, inf, ws.ptr, None), "short_prepare_x")
+    x64 = X.astype(np.float64)
+    first = go(0)
+    for (_, W), y in zip(mats, first):
+        close(y, W, x64)
+    assert all(np.array_equal(a, b) for a, b in zip(first, go(0)))
+    eps, nw = 1e-5, (1.0 + 0.1 * r.standard_normal(inf)).astype(np.float32)
+    hd, nd = DB.from_numpy(X), DB.from_numpy(nw)
+    _lib.check(L.ntk_short_norm_prepare_x(hd.ptr, None, nd.ptr, T, inf, ws.ptr, None), "short_norm")
+    n64 = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + eps) * nw
+    for (_, W), y in zip(mats, go(1, eps)):
+        close(y, W, n64)
+    if len(rows) > 1 or rows[0] % 256:
+        return
+    W, res, pt = mats[0][1], r.standard_normal((T, rows[0])).astype(np.float32), _lib.GemmPartials()
+    got = go(1, eps, DB.from_numpy(res))[0]
+    assert (np.abs(got - (res + n64 @ W.T)) <= REL * (np.sqrt((n64 ** 2) @ (W ** 2).T) + np.abs(res))).all()
