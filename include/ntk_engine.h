@@ -334,6 +334,8 @@ void ntk_debug_malloc_budget(long long bytes);
 
 /* *d_pos += 1 (one thread); keeps positions on the device across graph replays */
 int ntk_advance_pos(int* d_pos, void* stream);
+/* ONE token's row (as ntk_embed_rows; formats without a branch: zeros), the token and its position as arguments: they go into *d_token and *d_pos for the launches behind */
+int ntk_embed_token_row(float* out, const void* table, int token, int pos, int* d_token, int* d_pos, int hidden, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -459,6 +459,11 @@ int ntk_moe_combine(float* x, const float* mix, const float* d, const int* where
 int    ntk_store_words(int* a, int na, int* b, int nb, const int* values, void* stream);
 /* size bytes (a multiple of 4, both pointers 4-byte aligned) into pinned host memory (nt_hip_malloc_host) by a launch in the stream's order: there once the stream has been waited for */
 int    ntk_copy_out(void* pinned, const void* src, size_t size, void* stream);
+/* ... of `words` words in pieces of NTK_COPY_OUT_PIECE, each followed by `turn` in its word of there[ntk_copy_out_words(words)] (pinned, too): a host that reads `turn` there may read the piece, whether or
+ * not the launch has ended.  bump (or NULL): a device word that the launch adds one to */
+#define NTK_COPY_OUT_PIECE 4096
+size_t ntk_copy_out_words(size_t words);
+int    ntk_copy_out_pieces(void* pinned, const void* src, size_t words, unsigned* there, unsigned turn, int* bump, void* stream);
 
 #ifdef __cplusplus
 }

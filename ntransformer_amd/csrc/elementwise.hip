@@ -134,6 +134,13 @@ __global__ void embed_rows_kernel(float* __restrict__ out, const uint8_t* __rest
     if (e < hidden) out[(size_t)blockIdx.x * hidden + e] = embed_elem(table, tok, hidden, dt, e);
 }
 
+// one token given as an argument, and its words (token id, position) for the launches behind: a launch less than storing them first
+__global__ void embed_token_kernel(float* __restrict__ out, const uint8_t* __restrict__ table, int token, int pos, int* __restrict__ d_token, int* __restrict__ d_pos, int hidden, int dt) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e == 0) { *d_token = token; *d_pos = pos; }
+    if (e < hidden) out[e] = embed_elem(table, token, hidden, dt, e);
+}
+
 // ---- greedy argmax, first maximum wins (sampler.cpp:18-28: strict '>' scanning upwards) ----------------
 __device__ __forceinline__ void amax_merge(float& v, int& i, float ov, int oi) {
     if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
@@ -315,6 +322,12 @@ int ntk_embed_rows(float* out, const void* table, const int* tokens, int n_token
         case NTK_DT_F32: case NTK_DT_F16: case NTK_DT_Q8_0: case NTK_DT_Q4_0: case NTK_DT_Q4_K: case NTK_DT_Q6_K: return NTK_OK;
         default: return NTK_E_DTYPE;
     }
+}
+int ntk_embed_token_row(float* out, const void* table, int token, int pos, int* d_token, int* d_pos, int hidden, int dtype, void* stream) {
+    if (!out || !table || !d_token || !d_pos) return NTK_E_NULL;
+    if (token < 0 || hidden <= 0) return NTK_E_SHAPE;
+    hipLaunchKernelGGL(embed_token_kernel, dim3((hidden + 255) / 256), dim3(256), 0, resolve_stream(stream), out, (const uint8_t*)table, token, pos, d_token, d_pos, hidden, dtype);
+    return last_launch_status();
 }
 int ntk_argmax(const float* logits, int n, int* d_out_token, int* h_mirror, float* scratch, void* stream) {
     if (!logits || !d_out_token || !scratch) return NTK_E_NULL;

@@ -174,11 +174,7 @@ int nt_engine_decode_fused(nt_engine_t e, int token, int pos, int use_graph, flo
     if (!e || !logits_out || !GGUF(e)) return NTK_E_NULL;
     nt::Model& m = E(e)->model();
     if (pos < 0 || pos >= m.config().max_seq_len) return NTK_E_SHAPE;
-    int rc = m.set_device_step(pos, token);
-    if (rc != NTK_OK) return rc;
-    rc = m.decode_step_fused(false, use_graph != 0);
-    if (rc != NTK_OK) return rc;
-    rc = m.copy_logits(logits_out);
+    const int rc = m.decode_token(token, pos, use_graph != 0, logits_out);
     if (rc != NTK_OK) return rc;
     return m.check_persistent();
 }

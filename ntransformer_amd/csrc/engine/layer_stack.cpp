@@ -65,7 +65,7 @@ LayerStackModel::~LayerStackModel() {
     if (capture_buf_) nt_hip_free(capture_buf_);
     if (image_) nt_hip_free(image_);
     if (h_stage_) nt_hip_free_host(h_stage_);
-    if (h_logits_) nt_hip_free_host(h_logits_);
+    out_row_.clear();
 }
 
 void* LayerStackModel::dev_alloc(size_t bytes) {
@@ -1026,7 +1026,7 @@ int LayerStackModel::alloc_buffers() {
     want_dev_ = tokens_dev_ ? tokens_dev_ + C : nullptr;   // one staging area: [tokens of a pass | wanted places], filled by ONE stream-ordered copy from pinned memory
     h_stage_ = (int*)nt_hip_malloc_host(2 * C * sizeof(int));
     ok = ok && h_stage_ != nullptr;
-    h_logits_ = (float*)nt_hip_malloc_host((size_t)info_.vocab * sizeof(float));   // (none: a copy of the runtime's)
+    out_row_.alloc((size_t)info_.vocab);                     // (none: a copy of the runtime's)
     if (max_top_ > 0) {
         const size_t P = C * max_top_;
         ok = ok && in(&ids_, P) && fl(&wts_, P) && fl(&sg_, C) && in(&offsets_, (size_t)max_e_ + 1) && in(&order_, P) && in(&where_, P) && fl(&gu_, P * max_ff2_) &&
@@ -1848,12 +1848,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
 
 int LayerStackModel::copy_logits(float* host, int rows) {
     if (!host || rows < 0 || rows > last_rows_) return NTK_E_SHAPE;
-    if (rows == 1 && h_logits_) {
-        LS_TRY(ntk_copy_out(h_logits_, logits_, (size_t)info_.vocab * sizeof(float), stream_));
-        LS_TRY(ntk_stream_synchronize(stream_));
-        memcpy(host, h_logits_, (size_t)info_.vocab * sizeof(float));
-        return NTK_OK;
-    }
+    if (rows == 1 && out_row_) return out_row_.fetch(host, logits_, nullptr, stream_);
     LS_TRY(ntk_stream_synchronize(stream_));
     if (rows) nt_hip_memcpy_d2h(host, logits_, (size_t)rows * info_.vocab * sizeof(float));
     return NTK_OK;

@@ -49,6 +49,7 @@
 #pragma once
 #include <string>
 #include <vector>
+#include "host_rows.h"
 #include "safetensors.h"
 #include "sequence_model.h"
 #include "../../../include/ntk_layers.h"
@@ -397,7 +398,7 @@ private:
     size_t max_mid_ = 0;              // (post-norm form: the experts' activations of a token side by side)
     int max_rec_ = 0, max_gu2_ = 0, max_conv_ = 0, max_gv_ = 0;   // (scaled form: convolution channels, key heads x value size of the blending attention layers)
     int *ids_ = nullptr, *offsets_ = nullptr, *order_ = nullptr, *where_ = nullptr, *tokens_dev_ = nullptr, *want_dev_ = nullptr;
-    float* h_logits_ = nullptr;       // pinned: one row of logits on its way to the caller
+    HostRows out_row_;                // one row of logits on its way to the caller
     int* h_stage_ = nullptr;          // pinned: tokens and wanted places of the pass being launched
     float* logits_ = nullptr;
     size_t logits_rows_ = 0;

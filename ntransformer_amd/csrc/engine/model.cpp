@@ -60,8 +60,7 @@ void Model::free_all() {
     h_ring_ = nullptr;
     if (h_recent_) nt_hip_free_host(h_recent_);
     h_recent_ = nullptr;
-    if (h_logits_) nt_hip_free_host(h_logits_);
-    h_logits_ = nullptr;
+    out_row_.clear();
     sample_scratch_ = nullptr;
     d_recent_ = nullptr;
     attn_sync_ = nullptr;
@@ -542,7 +541,7 @@ int Model::alloc_buffers() {   // transformer.cpp:330-391
     attn_scratch_ = (float*)dev(ntk_attention_split_scratch_bytes(cfg_.n_heads, cfg_.head_dim, kMaxAttnSplits), true);   // (zeroed: the arrival counters in front)
     h_token_ = (int*)nt_hip_malloc_host(64);
     h_ring_ = (unsigned long long*)nt_hip_malloc_host(64);
-    h_logits_ = (float*)nt_hip_malloc_host((size_t)cfg_.vocab_size * 4);   // (none: a copy of the runtime's)
+    out_row_.alloc((size_t)cfg_.vocab_size);   // (none: a copy of the runtime's)
     if (h_ring_) memset(h_ring_, 0, 64);
     sample_scratch_ = dev(ntk_sample_scratch_bytes(cfg_.vocab_size), false);
     attn_sync_ = (unsigned*)dev(4096, true);
@@ -1211,12 +1210,7 @@ int Model::set_device_step(int pos, int token) {
     return ntk_store_words(d_token_, 1, d_pos_, 1, words, stream_);
 }
 int Model::copy_logits(float* host) {
-    if (h_logits_) {
-        NT_TRY(ntk_copy_out(h_logits_, logits_, (size_t)cfg_.vocab_size * 4, stream_));
-        NT_TRY(ntk_stream_synchronize(stream_));
-        memcpy(host, h_logits_, (size_t)cfg_.vocab_size * 4);
-        return NTK_OK;
-    }
+    if (out_row_) return out_row_.fetch(host, logits_, nullptr, stream_);
     NT_TRY(ntk_memcpy_d2h_async(host, logits_, (size_t)cfg_.vocab_size * 4, stream_));
     return ntk_stream_synchronize(stream_);
 }
@@ -1271,14 +1265,17 @@ static int rp_mask() {
 #endif
 }
 
-int Model::enqueue_token(bool greedy) {
+int Model::enqueue_token(TokenKind kind) {
     const int H = cfg_.hidden_size;
+    const bool greedy = kind == kGreedy;
     void* s = stream_;
     tp_call_ = 0;
-    prof_mark(2, true);
-    const int est = ntk_embed_rows(hidden_, token_embd_.ptr, d_token_, 1, H, token_embd_.dtype, s);
-    prof_mark(2, false);
-    if (est != NTK_OK && est != NTK_E_DTYPE) return est;
+    if (kind != kBare) {
+        prof_mark(2, true);
+        const int est = ntk_embed_rows(hidden_, token_embd_.ptr, d_token_, 1, H, token_embd_.dtype, s);
+        prof_mark(2, false);
+        if (est != NTK_OK && est != NTK_E_DTYPE) return est;
+    }
 #ifdef NTK_EXPERIMENTS
     if (use_persistent_now()) {   // every layer and the LM head in one launch
         NT_TRY(persistent_kind_ == 2 ? ntk_layer_engine_launch(persistent_plan_, d_pos_, s) : ntk_persistent_launch(persistent_plan_, d_pos_, s));
@@ -1310,6 +1307,7 @@ int Model::enqueue_token(bool greedy) {
             NT_TRY(ntk_gemv(logits_, w.ptr, residual_ + H, (int)w.out_f, (int)w.in_f, w.dtype, s));
         }
     }
+    if (kind == kBare) return NTK_OK;
     prof_mark(2, true);
     // greedy: arg-max, token -> device word + pinned ring, position + 1 in ONE tail (ntk_argmax_advance); otherwise only the position
     if (greedy) NT_TRY(ntk_argmax_advance(logits_, cfg_.vocab_size, d_token_, h_token_, h_ring_, d_pos_, argmax_scratch_, s));
@@ -1775,16 +1773,34 @@ void Model::pick_attention_regime() {
     ++host_pos_;   // every fused token ends with ntk_advance_pos on the device; set_device_pos() re-bases both
 }
 
-int Model::decode_step_fused(bool greedy, bool use_graph) {
+int Model::decode_step_fused(bool greedy, bool use_graph) { return run_token(greedy ? kGreedy : kSampled, use_graph); }
+
+// A given token at a given position: its words go with the launch of its embedding row, in front of the captured layers, and the launch that takes the logits out advances the position -- a token is
+// two launches shorter than set_device_step, decode_step_fused and copy_logits one after the other.
+int Model::decode_token(int token, int pos, bool use_graph, float* host) {
+    if (tp_world_ > 1 || !out_row_ || use_persistent_now()) {
+        NT_TRY(set_device_step(pos, token));
+        NT_TRY(decode_step_fused(false, use_graph));
+        return copy_logits(host);
+    }
+    if (token < 0 || token >= cfg_.vocab_size) { err_ = "token id out of range"; return NTK_E_SHAPE; }
+    *h_token_ = token;
+    host_pos_ = pos;
+    NT_TRY(ntk_embed_token_row(hidden_, token_embd_.ptr, token, pos, d_token_, d_pos_, cfg_.hidden_size, token_embd_.dtype, stream_));
+    NT_TRY(run_token(kBare, use_graph));
+    return out_row_.fetch(host, logits_, d_pos_, stream_);
+}
+
+int Model::run_token(TokenKind kind, bool use_graph) {
     pick_attention_regime();
-    if (!use_graph) return enqueue_token(greedy);
-    ihipGraphExec_t*& slot = graphs_[greedy ? 1 : 0][use_persistent_now() ? kPersistentSlot : attn_regime_];
+    if (!use_graph) return enqueue_token(kind);
+    ihipGraphExec_t*& slot = graphs_[kind][use_persistent_now() ? kPersistentSlot : attn_regime_];
     hipStream_t st = static_cast<hipStream_t>(stream_);
     if (!slot) {   // capture once: every per-token quantity (token id, position) lives in device memory
         hipGraph_t g = nullptr;
         // (relaxed under tensor parallelism: ranks sharing a process run their own runtime calls on other threads meanwhile)
         if (hipStreamBeginCapture(st, tp_world_ > 1 ? hipStreamCaptureModeRelaxed : hipStreamCaptureModeThreadLocal) != hipSuccess) return NTK_E_LAUNCH;
-        const int rc = enqueue_token(greedy);
+        const int rc = enqueue_token(kind);
         const hipError_t e = hipStreamEndCapture(st, &g);
         if (rc != NTK_OK || e != hipSuccess || !g) { if (g) (void)hipGraphDestroy(g); return rc != NTK_OK ? rc : NTK_E_LAUNCH; }
         hipGraphExec_t ex = nullptr;
@@ -1802,7 +1818,7 @@ int Model::profile_token(float ms[4], int calls[4], bool coarse) {
     prof_ = &rec;
     prof_coarse_ = coarse;
     pick_attention_regime();
-    int rc = enqueue_token(true);
+    int rc = enqueue_token(kGreedy);
     if (coarse && !rec.empty()) {   // close the last run
         void* e = ntk_event_create();
         ntk_event_record(e, stream_);

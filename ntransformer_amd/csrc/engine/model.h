@@ -9,6 +9,7 @@
 #include <string>
 #include <vector>
 #include "gguf.h"
+#include "host_rows.h"
 #include "synth.h"
 
 struct ihipGraphExec_t;   // hipGraphExec_t
@@ -54,6 +55,7 @@ public:
     // token is one hipGraph replay.  Token comes from d_token_ (set_device_token / previous argmax).
     // If greedy: also runs the device argmax and advances the position.
     int decode_step_fused(bool greedy, bool use_graph);
+    int decode_token(int token, int pos, bool use_graph, float* host);   // a given token's logits: set_device_step, a step and copy_logits with two launches less
     int set_device_token(int token);
     int set_device_pos(int pos);
     int set_device_step(int pos, int token);   // both for ONE step, as arguments of a launch: in the stream's order, nothing waited for
@@ -179,7 +181,9 @@ private:
     int tp_allreduce(float* hidden, int n);   // hidden += sum over ranks of the partial vectors in the current slot
     float* tp_slot() const;           // where the next partial vector goes
     void free_all();
-    int enqueue_token(bool greedy);   // the fused launch sequence for one token
+    enum TokenKind { kSampled = 0, kGreedy = 1, kBare = 2 };    // bare: the embedded row is there, and the caller's launch behind the logits advances the position
+    int enqueue_token(TokenKind kind);   // the fused launch sequence for one token
+    int run_token(TokenKind kind, bool use_graph);
     int enqueue_layers(int first, int last);            // its layer loop
     int layers_1to1(int T, int start_pos, int first, int last, bool keys_last = false, float* queries = nullptr);   // the layer loop of forward()
     bool short_prompt(int T) const;
@@ -214,7 +218,7 @@ private:
     int* d_token_ = nullptr;        // device scalar: id of the token being decoded
     int* h_token_ = nullptr;        // pinned mirror of the argmax result
     unsigned long long* h_ring_ = nullptr;   // pinned ring of 4 x {token, position + 1}: ntk_argmax_advance / wait_token
-    float* h_logits_ = nullptr;       // pinned: the logits on their way to the caller
+    HostRows out_row_;                // the logits on their way to the caller
     std::chrono::steady_clock::time_point wait_t0_;
     float* argmax_scratch_ = nullptr;
     void* sample_scratch_ = nullptr;
@@ -230,7 +234,7 @@ private:
     std::vector<Timed>* prof_ = nullptr;   // non-null while profile_token() runs
     // one captured token per (greedy?, attention regime)
     static constexpr int kPersistentSlot = kAttnRegimes;   // the persistent forms of regime 0 have their own slot
-    ihipGraphExec_t* graphs_[2][kAttnRegimes + 1] = {};   // [greedy][attention regime 0..2, 3 = persistent]
+    ihipGraphExec_t* graphs_[3][kAttnRegimes + 1] = {};   // [sampled, greedy, layers and head alone][attention regime 0..2, 3 = persistent]
     int host_pos_ = 0;               // host mirror of *d_pos_ (set_device_pos + one per fused step): picks the regime
     int attn_regime_ = 0;            // regime enqueue_token() emits
     float* attn_scratch_ = nullptr;  // partial softmax states of the split-KV attention

@@ -347,6 +347,22 @@ __global__ __launch_bounds__(256) void copy_out_kernel(uint32_t* __restrict__ ou
             for (size_t k = 4 * i; k < words; ++k) out[k] = src[k];
     } else if (i < words) out[i] = src[i];
 }
+// a piece a workgroup: its stores are out (system scope) in front of its word
+__global__ __launch_bounds__(256) void copy_out_pieces_kernel(uint32_t* __restrict__ out, const uint32_t* __restrict__ src, size_t words, int wide, unsigned* __restrict__ there, unsigned turn, int* __restrict__ bump) {
+    const size_t at = (size_t)blockIdx.x * NTK_COPY_OUT_PIECE, end = min(words, at + NTK_COPY_OUT_PIECE);
+    if (bump && blockIdx.x == 0 && threadIdx.x == 0) *bump += 1;
+    if (wide && at + NTK_COPY_OUT_PIECE <= words) {
+#pragma unroll
+        for (int k = 0; k < NTK_COPY_OUT_PIECE / 1024; ++k) {
+            const size_t i = at + 4 * (size_t)(threadIdx.x + 256 * k);
+            *reinterpret_cast<uint4*>(out + i) = *reinterpret_cast<const uint4*>(src + i);
+        }
+    } else
+        for (size_t i = at + threadIdx.x; i < end; i += 256) out[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(there + blockIdx.x, turn, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 }  // namespace ntk
 
 using namespace ntk;
@@ -369,6 +385,17 @@ int ntk_copy_out(void* pinned, const void* src, size_t size, void* stream) {
     const int wide = (at & 15) == 0;
     const size_t words = size / 4, threads = wide ? (words + 3) / 4 : words;
     hipLaunchKernelGGL(copy_out_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, resolve_stream(stream), static_cast<uint32_t*>(pinned), static_cast<const uint32_t*>(src), words, wide);
+    return last_launch_status();
+}
+
+size_t ntk_copy_out_words(size_t words) { return (words + NTK_COPY_OUT_PIECE - 1) / NTK_COPY_OUT_PIECE; }
+int ntk_copy_out_pieces(void* pinned, const void* src, size_t words, unsigned* there, unsigned turn, int* bump, void* stream) {
+    if (!pinned || !src || !there) return NTK_E_NULL;
+    const uintptr_t at = (uintptr_t)pinned | (uintptr_t)src;
+    if (words == 0 || words > (size_t)0x7FFFFFFF) return NTK_E_SHAPE;
+    if ((at | (uintptr_t)there | (uintptr_t)bump) & 3) return NTK_E_ALIGN;
+    hipLaunchKernelGGL(copy_out_pieces_kernel, dim3((unsigned)ntk_copy_out_words(words)), dim3(256), 0, resolve_stream(stream), static_cast<uint32_t*>(pinned), static_cast<const uint32_t*>(src),
+                       words, (int)((at & 15) == 0), there, turn, bump);
     return last_launch_status();
 }
 
