@@ -158,6 +158,11 @@ int ntk_tanh_rows(float* x, int ldx, int T, int n, void* stream);
  * w_head_stride 0: one weight vector [dv] shared by the heads; dv: a weight per head and column.  act 0: no gate (g unused), 1: sigmoid, 2: silu. */
 int ntk_head_rmsnorm_gate(float* y, int ldy, const float* x, int ldx, const float* w, int w_head_stride, const float* g, int ldg, int act, float scale, int T, int H,
                           int dv, float eps, void* stream);
+/* ... with the results rounded to bfloat16, rows H * dv apart.  Entries in fours on 16 bytes (y16: 8) and up to 256 a head, else NTK_E_ALIGN (nothing launched). */
+int ntk_head_rmsnorm_gate_16(void* y16, const float* x, int ldx, const float* w, int w_head_stride, const float* g, int ldg, int act, float scale, int T, int H, int dv,
+                             float eps, void* stream);
+/* y16[t][i] = x[t][i] * sigmoid(g[t][per_head ? i / per_head : i]) rounded to bfloat16, rows n apart: as above in fours, T up to 65535. */
+int ntk_gate_rows_16(void* y16, const float* x, int ldx, const float* g, int ldg, int per_head, int T, int n, void* stream);
 /* The seam of a layer whose sublayer results join the stream through a gate and whose layer results are averaged over depth, in one launch:
  *   r[t]  = x[t] + (y[t] + yb) * sigmoid(g[t] + gb)                (yb, gb: bias vectors [n], may be NULL)
  *   n_hist == 0:  x[t] = r[t]

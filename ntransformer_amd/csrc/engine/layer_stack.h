@@ -351,6 +351,8 @@ private:
     bool pays(const GatedExperts& ex, int rows, int tokens) const;
     bool rounded(const MoeFeedForward& M, int T) const;
     int product(ntk_dense_desc& d);
+    void* rounded_rows(const DenseW& w, int T) const;
+    int rounded_product(float* Y, const DenseW& w, int T);
     int linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate);
     int sequential_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);

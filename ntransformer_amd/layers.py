@@ -101,6 +101,8 @@ def _bind():
     L.ntk_dense_linear.argtypes = [vp, i, vp, i, vp, i, i, i, i, i, vp]
     L.ntk_embed_dense.argtypes = [vp, vp, i, vp, i, i, i, vp]
     L.ntk_rmsnorm_offset_16.argtypes = [vp, vp, vp, vp, vp, vp, i, vp, i, i, i, f, f, vp]
+    L.ntk_head_rmsnorm_gate_16.argtypes = [vp, vp, i, vp, i, vp, i, i, f, i, i, i, f, vp]
+    L.ntk_gate_rows_16.argtypes = [vp, vp, i, vp, i, i, i, i, vp]
     L.ntk_rms_seam_16.argtypes = [vp, vp, i, vp, i, vp, f, vp, i, i, f, vp]
     L.ntk_rmsnorm_offset.argtypes = [vp, vp, vp, vp, i, vp, i, i, i, f, f, vp]
     L.ntk_concat_rows.argtypes = [vp, vp, vp, i, i, vp]
@@ -283,6 +285,25 @@ def rmsnorm_offset_16(x: np.ndarray, w1: np.ndarray, w2: np.ndarray, eps: float,
     a, y, b = DeviceBuffer.zeros(T * n * 2), DeviceBuffer.zeros(T * n * 4), DeviceBuffer.zeros(T * n * 2)
     check(L.ntk_rmsnorm_offset_16(None, a.ptr, w1b.ptr, y.ptr, b.ptr, w2b.ptr, n, xb.ptr, n, T, n, eps, offset, None), "ntk_rmsnorm_offset_16")
     return _bf16(a.numpy(np.uint16, T * n).reshape(T, n)), y.numpy(np.float32, T * n).reshape(T, n), _bf16(b.numpy(np.uint16, T * n).reshape(T, n))
+
+
+def head_rmsnorm_gate_16(x: np.ndarray, w: np.ndarray, g: Optional[np.ndarray], act: int, scale: float, heads: int, dim: int, eps: float) -> np.ndarray:
+    """x [T, >= heads * dim], w [dim] or [heads, dim] -> [T, heads * dim] (bfloat16 as float32)"""
+    L = _bind()
+    T, n = len(x), heads * dim
+    xb, wb, gb, y = _f(x), _f(w), _f(g) if g is not None else None, DeviceBuffer.zeros(T * n * 2)
+    check(L.ntk_head_rmsnorm_gate_16(y.ptr, xb.ptr, x.shape[1], wb.ptr, dim if w.ndim > 1 else 0, gb.ptr if gb else None, g.shape[1] if gb else 0, act, scale, T, heads, dim, eps, None),
+          "ntk_head_rmsnorm_gate_16")
+    return _bf16(y.numpy(np.uint16, T * n).reshape(T, n))
+
+
+def gate_rows_16(x: np.ndarray, g: np.ndarray, n: int, per_head: int = 0) -> np.ndarray:
+    """x [T, >= n], g [T, >= n, or n / per_head] -> [T, n] (bfloat16 as float32)"""
+    L = _bind()
+    T = len(x)
+    xb, gb, y = _f(x), _f(g), DeviceBuffer.zeros(T * n * 2)
+    check(L.ntk_gate_rows_16(y.ptr, xb.ptr, x.shape[1], gb.ptr, g.shape[1], per_head, T, n, None), "ntk_gate_rows_16")
+    return _bf16(y.numpy(np.uint16, T * n).reshape(T, n))
 
 
 def rmsnorm_offset(x: np.ndarray, w1: np.ndarray, w2: Optional[np.ndarray], eps: float, offset: float):

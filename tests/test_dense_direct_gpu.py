@@ -142,3 +142,39 @@ def test_norms_that_leave_rounded_rows(T, n):
         assert np.allclose(gx, sx, rtol=2e-6, atol=2e-6) and near(gh, sh)
     with pytest.raises(Exception):
         Lr.rms_seam_16(rng.standard_normal((2, 4100)).astype(np.float32), np.ones(4100, np.float32), 1e-5)
+
+
+# bfloat16 keeps eight bits: half a step is 2^-8 of a value; the float32 before it (a mean of up to 256 squares, an exponential) is a few steps of 2^-24 off
+def _rounded_near(got, want):
+    return (np.abs(got - want) <= (2.0 ** -8 + 64 * 2.0 ** -24) * np.abs(want) + 1e-30).all()
+
+
+@pytest.mark.parametrize("T,heads,dim,act,shared", [(1, 1, 4, 2, True), (33, 3, 60, 1, False), (40, 5, 64, 2, True), (9, 7, 68, 0, True), (70, 16, 128, 2, True), (5, 3, 132, 1, False), (33, 2, 256, 2, False)])
+def test_head_norms_that_leave_rounded_rows(T, heads, dim, act, shared):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(dim)
+    n = heads * dim
+    x, g = rng.standard_normal((2, T, n + 8)).astype(np.float32)
+    w = rng.standard_normal(dim if shared else (heads, dim)).astype(np.float32)
+    v = x[:, :n].astype(np.float64).reshape(T, heads, dim)
+    c = g[:, :n].astype(np.float64).reshape(T, heads, dim)
+    s = 1 / (1 + np.exp(-c))
+    want = v / np.sqrt((v * v).mean(-1, keepdims=True) + 1e-5) * w * (s * c if act == 2 else s if act else 1.0) * 0.7
+    assert _rounded_near(Lr.head_rmsnorm_gate_16(x, w, g if act else None, act, 0.7, heads, dim, 1e-5), want.reshape(T, n))
+    with pytest.raises(Exception):                   # no fours; a head of more than a wave
+        Lr.head_rmsnorm_gate_16(x[:, :6].copy(), w.reshape(-1)[:2].copy(), None, 0, 1.0, 1, 2, 1e-5)
+    with pytest.raises(Exception):
+        Lr.head_rmsnorm_gate_16(rng.standard_normal((2, 260)).astype(np.float32), np.ones(260, np.float32), None, 0, 1.0, 1, 260, 1e-5)
+
+
+@pytest.mark.parametrize("T,n,per_head", [(1, 4, 0), (33, 1020, 0), (9, 1028, 0), (40, 2048, 128), (5, 24, 4), (70, 2112, 192)])
+def test_gates_that_leave_rounded_rows(T, n, per_head):
+    from ntransformer_amd import layers as Lr
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((T, n + 4)).astype(np.float32)
+    g = rng.standard_normal((T, n // per_head + 3 if per_head else n + 8)).astype(np.float32) * 4
+    s = 1 / (1 + np.exp(-g.astype(np.float64)))
+    s = np.repeat(s[:, :n // per_head], per_head, axis=1) if per_head else s[:, :n]
+    assert _rounded_near(Lr.gate_rows_16(x, g, n, per_head), x[:, :n] * s)
+    with pytest.raises(Exception):
+        Lr.gate_rows_16(x, g, 3, 0)
