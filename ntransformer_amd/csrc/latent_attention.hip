@@ -204,135 +204,132 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const AttnArgs a)
 }
 
 // ------------------------------------------------------------------------------------------------------------------- the shared form (decoding)
-// Keys and values are the cache rows themselves, so a workgroup loads a tile of KB = 32 rows [latent | rotated] ONCE (a thread's requests in flight together) and uses it for
-// every (token, head) row of its tile of 16, on the F32 matrix instructions: wave w forms the scores of 16 rows x 32 keys over every fourth step of 16 entries (queries as
-// operands in registers, straight from memory), the four parts meet in LDS, sixteen threads run the online softmax of their row, then wave w sums the weighted latents
-// of a quarter of the columns.  The tiles of 32 keys go round `splits` workgroups; each leaves one (max, sum, vector) state per row and latent_attention_merge_kernel adds
-// them.  Latency bounds it: launch, one round trip for tile and queries, ~70 matrix instructions, softmax, ~64 more, the states out.  With the products on the vector
-// units (one LDS read per two FMAs) and the tile in three round trips 1100 positions took 21.4 us, now 12.2.
+// Keys and values are the cache rows themselves.  A workgroup takes 32 of them (KB) for a tile of 16 (token, head) rows on the F32 matrix instructions, and the operands go from memory
+// into registers as they are needed: wave w forms the scores over every NWth step of 16 entries (a lane's four entries of a key, as of its query), the parts meet in LDS,
+// NW * 4 threads run the online softmax of a row, then wave w sums columns 64 w ..: a lane's four columns of a key are one request and belong to four tiles of results, so
+// its results are four neighbours too.  The tiles of 32 keys go round `splits` workgroups; each leaves one (max, sum) and one vector per row, joined in the launch behind.
+// Latency bounds it with few positions: launch, ONE round trip for queries, keys and values together, 40 matrix instructions a wave, softmax, 32 more, the states out.  us, 16 heads,
+// 512 + 64, a token at 44 / 1100 positions: four waves with the tile in LDS 11.4 / 13.0, so 8.6 / 9.4; the matrix instructions bound it with many: with the merge, 8000 31.9 -> 19.2, 32000
+// 92.7 -> 44.4 (the next tile's rows are on their way under this one's work, and two workgroups fit on a CU).
 constexpr int KB = 32, SROWS = 16;
 struct SharedArgs {
     const float* q; int ldq;          // [T][H][R + dr], ldq floats between tokens
     const float* cache; int row;      // cache rows
     int R, dr, H, pos0, T, window, splits;
     float scale;
-    float* scratch;                   // [rows][splits][2 + R]
+    float* scratch;                   // [rows][splits][R] vectors, then [rows][splits][2] maxima and sums
 };
 
-// SSTEPS: keys of (latent + rotated) up to 64 * SSTEPS entries; CT: ranks up to 64 * CT.  Three sizes of it: registers for 832 entries leave a SIMD one wave, which is enough for
-// the few workgroups of a decoded token but not where many rows walk a long context.  8 tokens of 64 heads at 8000 positions, latents of 32 + 8: 293 us in the largest
-// size, 121 in the smallest (vector form 158); 256 + 32: 338 -> 156 (262); one token of 16 heads of 64 + 16: 25.7 -> 22.2 (30.5).
-template <int SSTEPS, int CT>
-__global__ __launch_bounds__(256) void latent_attention_shared_kernel(const SharedArgs a) {
-    constexpr int LOADS = 2 * SSTEPS < 20 ? 2 * SSTEPS : 20;       // quads of a row that a thread requests together
+// NW waves: ranks up to 64 * NW; KS: keys of (latent + rotated) up to 16 * NW * KS entries; V: rows of whole fours on 16 bytes.  The smaller sizes need fewer registers, which
+// counts where many rows walk a long context.  us with the merge, 8 tokens of 64 heads at 8000 positions, tile in LDS / so: 32 + 8 121 / 43, 256 + 32 157 / 95, 512 + 64 400 / 193.
+template <int KS, int NW, bool V>
+__global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const SharedArgs a) {
     typedef float f4 __attribute__((ext_vector_type(4)));
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    constexpr int PP = KB + 4;
-    const int DK = a.R + a.dr, D16 = (DK + 15) & ~15, DKP = D16 + 4;      // rows 16-byte aligned, 4 banks apart; zero behind DK
-    float* Ks = lds;                               // [KB][DKP]
-    float* Sp = Ks + KB * DKP;                     // [4][SROWS][PP] parts of the scores
-    float* Ps = Sp + 4 * SROWS * PP;               // [SROWS][PP]
-    float* ms = Ps + SROWS * PP;                   // [SROWS] running max
-    float* ls = ms + SROWS;                        // [SROWS] running sum
-    float* cr = ls + SROWS;                        // [SROWS] correction of this tile
+    typedef f4 f4_anywhere __attribute__((aligned(4)));
+    constexpr int PP = KB + 4, TPR = 4 * NW, KPT = KB / TPR;       // softmax: threads a row, keys a thread
+    __shared__ float Sp[NW * SROWS * PP];          // parts of the scores
+    __shared__ __attribute__((aligned(16))) float Ps[SROWS * PP];
+    __shared__ float ms[SROWS], ls[SROWS], cr[SROWS];      // running max and sum, correction of this tile
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, g4 = lane >> 4;
+    const int DK = a.R + a.dr, steps = (DK + 15) / 16, col = 64 * wave + 4 * i16;
     const int n_rows = a.T * a.H, row0 = blockIdx.x * SROWS;
     const int last_row = min(row0 + SROWS, n_rows) - 1;
     const int pmin = a.pos0 + row0 / a.H, pmax = a.pos0 + last_row / a.H;
     const int jlo = a.window > 0 ? max(0, pmin - a.window + 1) : 0, jhi = pmax;
-    const bool vec4 = (DK % 4 == 0) && (a.row % 4 == 0) && !((uintptr_t)a.cache & 15);
-    // the wave's part of the queries: row i16, entries 16 s + 4 g4 .. of the steps s = wave, wave + 4, ...
-    f4 qf[SSTEPS];
+    auto four = [](const float* p, int at, int end) -> f4 {         // entries at .. at + 3 of a row of `end`, zero behind it
+        f4 v{0.f, 0.f, 0.f, 0.f};
+        if constexpr (V) { if (at < end) v = *reinterpret_cast<const f4*>(p + at); }
+        else if (at + 4 <= end) v = *reinterpret_cast<const f4_anywhere*>(p + at);
+        else if (at < end)
+            for (int c = 0; c < 4; ++c) if (at + c < end) v[c] = p[at + c];
+        return v;
+    };
+    // (keys past the last re-read it; their weight is zero)
+    f4 qf[KS], kf[KS][2], vf[2][4];
+    auto load_keys = [&](int j0) {
+        const float* k0 = a.cache + (long long)min(j0 + i16, jhi) * a.row, *k1 = a.cache + (long long)min(j0 + 16 + i16, jhi) * a.row;
+#pragma unroll
+        for (int u = 0; u < KS; ++u) {
+            const int st = wave + NW * u;
+            if (st < steps) { kf[u][0] = four(k0, 16 * st + 4 * g4, DK); kf[u][1] = four(k1, 16 * st + 4 * g4, DK); }
+        }
+    };
+    const bool sums = 64 * wave < a.R;             // (uniform over the wave)
+    auto load_values = [&](int j0) {
+        if (!sums) return;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) vf[e][c] = four(a.cache + (long long)min(j0 + 16 * e + 4 * g4 + c, jhi) * a.row, col, a.R);
+    };
+    int j0 = jlo + KB * (int)blockIdx.y;
+    const int hop = KB * a.splits;
     {
         const int r = min(row0 + i16, n_rows - 1);
         const float* q = a.q + (long long)(r / a.H) * a.ldq + (long long)(r % a.H) * DK;
-        const bool qv = (DK % 4 == 0) && (a.ldq % 4 == 0) && !((uintptr_t)a.q & 15);
 #pragma unroll
-        for (int u = 0; u < SSTEPS; ++u) {
-            const int d = 16 * (wave + 4 * u) + 4 * g4;
-            qf[u] = f4{0.f, 0.f, 0.f, 0.f};
-            if (d < DK) {
-                if (qv) qf[u] = *reinterpret_cast<const f4*>(q + d);
-                else
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) qf[u][c] = d + c < DK ? q[d + c] : 0.0f;
-            }
-        }
+        for (int u = 0; u < KS; ++u)
+            if (wave + NW * u < steps) qf[u] = four(q, 16 * (wave + NW * u) + 4 * g4, DK);
     }
+    if (j0 <= jhi) { load_keys(j0); load_values(j0); }
     if (tid < SROWS) { ms[tid] = -INFINITY; ls[tid] = 0.0f; }
-    const int srow = tid >> 4, sub = tid & 15;     // softmax: sixteen threads per row, two keys each
+    const int srow = tid / TPR, sub = tid % TPR;
     const int rpos = row0 + srow < n_rows ? a.pos0 + (row0 + srow) / a.H : -1;
-    f4 acc[CT];                                    // tiles of 16 columns per wave
+    f4 acc[4];                                     // column 64 wave + 4 i16 + t of rows 4 g4 ..
 #pragma unroll
-    for (int t = 0; t < CT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-    const int col0 = wave * ((((a.R + 15) / 16 + 3) / 4) * 16);           // the wave's columns
-    const int n_ct = min(max(((a.R + 15) / 16) - col0 / 16, 0), ((a.R + 15) / 16 + 3) / 4);
-    int tile = 0;
-    for (int j0 = jlo; j0 <= jhi; j0 += KB, ++tile) {
-        if (tile % a.splits != (int)blockIdx.y) continue;
+    for (int t = 0; t < 4; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+    for (; j0 <= jhi; j0 += hop) {
         const int nk = min(KB, jhi + 1 - j0);
-        const int lk = tid >> 3, lc = tid & 7;     // thread -> (key, every eighth quad)
-        __syncthreads();                           // the previous tile is used up (and ms is written)
-        const float* src = a.cache + (long long)(j0 + min(lk, nk - 1)) * a.row;     // (keys past the last re-read it; their weight is zero)
-        if (vec4) {
-            for (int c0 = lc; 4 * c0 < D16; c0 += 8 * LOADS) {
-                f4 v[LOADS];
-#pragma unroll
-                for (int u = 0; u < LOADS; ++u) {
-                    const int d = 4 * (c0 + 8 * u);
-                    v[u] = f4{0.f, 0.f, 0.f, 0.f};
-                    if (d < DK) v[u] = *reinterpret_cast<const f4*>(src + d);
-                }
-#pragma unroll
-                for (int u = 0; u < LOADS; ++u)
-                    if (4 * (c0 + 8 * u) < D16) *reinterpret_cast<f4*>(&Ks[lk * DKP + 4 * (c0 + 8 * u)]) = v[u];
-            }
-        } else {
-            for (int d = lc; d < D16; d += 8) Ks[lk * DKP + d] = d < DK ? src[d] : 0.0f;
-        }
-        __syncthreads();
+        const bool more = j0 + hop <= jhi;
         // ---- scores: this wave's steps
         f4 s0{0.f, 0.f, 0.f, 0.f}, s1{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int u = 0; u < SSTEPS; ++u) {
-            const int st = wave + 4 * u;
-            if (16 * st >= D16) continue;          // (uniform over the wave)
-            const f4 k0 = *reinterpret_cast<const f4*>(&Ks[i16 * DKP + 16 * st + 4 * g4]), k1 = *reinterpret_cast<const f4*>(&Ks[(16 + i16) * DKP + 16 * st + 4 * g4]);
+        for (int u = 0; u < KS; ++u) {
+            if (wave + NW * u >= steps) continue;  // (uniform over the wave)
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], k0[c], s0, 0, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], k1[c], s1, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], kf[u][0][c], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], kf[u][1][c], s1, 0, 0, 0);
             }
         }
+        if (more) load_keys(j0 + hop);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             Sp[(wave * SROWS + 4 * g4 + r) * PP + i16] = s0[r];
             Sp[(wave * SROWS + 4 * g4 + r) * PP + 16 + i16] = s1[r];
         }
-        __syncthreads();
+        __syncthreads();                           // (also: every wave has read the previous tile's weights)
         // ---- online softmax
         {
-            float sv[2];
+            float sv[KPT], mc = -INFINITY;
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int key = sub + 16 * e, j = j0 + key;
-                const float* sp = Sp + srow * PP + key;
-                const float sum = (sp[0] + sp[SROWS * PP]) + (sp[2 * SROWS * PP] + sp[3 * SROWS * PP]);
+            for (int e = 0; e < KPT; ++e) {
+                const int key = sub + TPR * e, j = j0 + key;
+                float part[NW];
+#pragma unroll
+                for (int w = 0; w < NW; ++w) part[w] = Sp[(w * SROWS + srow) * PP + key];
+#pragma unroll
+                for (int n = NW / 2; n; n >>= 1)
+#pragma unroll
+                    for (int w = 0; w < n; ++w) part[w] += part[w + n];
                 const bool vis = key < nk && rpos >= 0 && j <= rpos && (a.window <= 0 || rpos - j < a.window);
-                sv[e] = vis ? sum * a.scale : -INFINITY;
+                sv[e] = vis ? part[0] * a.scale : -INFINITY;
+                mc = fmaxf(mc, sv[e]);
             }
-            float mc = fmaxf(sv[0], sv[1]);
 #pragma unroll
-            for (int o = 8; o >= 1; o >>= 1) mc = fmaxf(mc, __shfl_xor(mc, o, 16));
+            for (int o = TPR / 2; o >= 1; o >>= 1) mc = fmaxf(mc, __shfl_xor(mc, o, TPR));
             const float mo = ms[srow];
             const float mn = fmaxf(mo, mc), msafe = mn == -INFINITY ? 0.0f : mn;
-            const float e0 = sv[0] == -INFINITY ? 0.0f : expf(sv[0] - msafe), e1 = sv[1] == -INFINITY ? 0.0f : expf(sv[1] - msafe);
-            float sum = e0 + e1;
+            float sum = 0.0f;
 #pragma unroll
-            for (int o = 8; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 16);
-            Ps[srow * PP + sub] = e0;
-            Ps[srow * PP + 16 + sub] = e1;
-            if (sub == 0) {                        // (the row's sixteen lanes are of one wave: all have read ms)
+            for (int e = 0; e < KPT; ++e) {
+                const float p = sv[e] == -INFINITY ? 0.0f : expf(sv[e] - msafe);
+                Ps[srow * PP + sub + TPR * e] = p;
+                sum += p;
+            }
+#pragma unroll
+            for (int o = TPR / 2; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, TPR);
+            if (sub == 0) {                        // (the row's lanes are of one wave: all have read ms)
                 const float corr = mo == -INFINITY ? 0.0f : expf(mo - msafe);
                 ls[srow] = ls[srow] * corr + sum;
                 ms[srow] = mn;
@@ -341,33 +338,38 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(const Shar
         }
         __syncthreads();
         // ---- weighted latents: this wave's columns
-        float corr[4];
+        if (sums) {
+            const f4 p0 = *reinterpret_cast<const f4*>(&Ps[i16 * PP + 4 * g4]), p1 = *reinterpret_cast<const f4*>(&Ps[i16 * PP + 16 + 4 * g4]);
+            float corr[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) corr[r] = cr[4 * g4 + r];
-        const f4 p0 = *reinterpret_cast<const f4*>(&Ps[i16 * PP + 4 * g4]), p1 = *reinterpret_cast<const f4*>(&Ps[i16 * PP + 16 + 4 * g4]);
+            for (int r = 0; r < 4; ++r) corr[r] = cr[4 * g4 + r];
 #pragma unroll
-        for (int t = 0; t < CT; ++t) {
-            if (t >= n_ct) continue;               // (uniform over the wave)
-            const float* vf = &Ks[(4 * g4) * DKP + col0 + 16 * t + i16];
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][r] *= corr[r];
+                for (int r = 0; r < 4; ++r) acc[t][r] *= corr[r];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {          // component c of the weights belongs to key 4 g4 + c
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[c], vf[c * DKP], acc[t], 0, 0, 0);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[c], vf[(16 + c) * DKP], acc[t], 0, 0, 0);
-            }
+            for (int c = 0; c < 4; ++c)            // component c of the weights belongs to key 4 g4 + c
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[c], vf[0][c][t], acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[c], vf[1][c][t], acc[t], 0, 0, 0);
+                }
+            if (more) load_values(j0 + hop);
         }
     }
-    __syncthreads();
+    __syncthreads();                               // (a workgroup without a tile: ms is written)
+    const long long states = (long long)n_rows * a.splits;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int i = 4 * g4 + r;
         if (row0 + i >= n_rows) continue;
-        float* st = a.scratch + ((long long)(row0 + i) * a.splits + blockIdx.y) * (2 + a.R);
-        if (wave == 0 && i16 == 0) { st[0] = ms[i]; st[1] = ls[i]; }
+        const long long at = (long long)(row0 + i) * a.splits + blockIdx.y;
+        if (wave == 0 && i16 == 0) { a.scratch[states * a.R + 2 * at] = ms[i]; a.scratch[states * a.R + 2 * at + 1] = ls[i]; }
+        float* st = a.scratch + at * a.R;
+        if constexpr (V) { if (col < a.R) *reinterpret_cast<f4*>(st + col) = f4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]}; }
+        else
 #pragma unroll
-        for (int t = 0; t < CT; ++t)
-            if (t < n_ct && col0 + 16 * t + i16 < a.R) st[2 + col0 + 16 * t + i16] = acc[t][r];
+            for (int t = 0; t < 4; ++t) if (col + t < a.R) st[col + t] = acc[t][r];
     }
 }
 
@@ -378,14 +380,14 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(float* out,
     __shared__ float red[16];
     __shared__ float part[4][64];
     const int r = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;   // r = t * H + h
-    const float* st = scratch + (long long)r * splits * (2 + nV);
-    const long long step = 2 + nV;
+    const float* st = scratch + (long long)r * splits * nV, *ml = scratch + ((long long)gridDim.x * nV + 2LL * r) * splits;
+    const long long step = nV;
     const int v = blockIdx.y * 64 + lane, each = (splits + 3) / 4, s0 = wave * each, s1 = min(s0 + each, splits);
     float x[8];                                    // the wave's first eight states requested together with the maxima
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = s0 + u < s1 && v < nV ? st[(s0 + u) * step + 2 + v] : 0.0f;
+    for (int u = 0; u < 8; ++u) x[u] = s0 + u < s1 && v < nV ? st[(s0 + u) * step + v] : 0.0f;
     const int mine = threadIdx.x;                  // (at most 128 states)
-    const float m = mine < splits ? st[mine * step] : -INFINITY, l = mine < splits ? st[mine * step + 1] : 0.0f;
+    const float m = mine < splits ? ml[2 * mine] : -INFINITY, l = mine < splits ? ml[2 * mine + 1] : 0.0f;
     const float mx = block_max(m, red);
     const float w = m == -INFINITY ? 0.0f : expf(m - mx);
     wt[threadIdx.x] = w;
@@ -397,7 +399,7 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(float* out,
         for (int u = 0; u < 8; ++u)
             if (s + u < s1) sum = fmaf(x[u], wt[s + u], sum);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = s + 8 + u < s1 && v < nV ? st[(s + 8 + u) * step + 2 + v] : 0.0f;
+        for (int u = 0; u < 8; ++u) x[u] = s + 8 + u < s1 && v < nV ? st[(s + 8 + u) * step + v] : 0.0f;
     }
     part[wave][lane] = sum;
     __syncthreads();
@@ -502,15 +504,29 @@ __global__ __launch_bounds__(256) void latent_unfold_value_kernel(float* out, in
     }
 }
 
-// ... with the parts' states (latent_attention_shared_kernel) joined in front, for ranks of whole pieces of eight up to 512: every workgroup of a head joins them for itself, two columns a thread.
-// us of the merge above and the unfolding / so, 16 heads of 128, rank 512, one token: 2 states 3.6 + 6.0 / 5.1, 36 states 4.1 + 6.4 / 8.3
+// ... with the parts' states (latent_attention_shared_kernel) joined in front, for ranks of whole pieces of eight up to 512: every workgroup of a head joins them for itself.  All
+// states are requested at once with the matrix rows: a thread takes four columns of every fourth state, the four parts of a column meet in LDS; a wave then owns four outputs.
+// us of the merge above and the unfolding / with the states eight after eight and 16 outputs a workgroup / so, 16 heads of 128, rank 512, one token: 2 states 3.6 + 6.0 / 5.1 / 4.9, 36 states
+// 4.1 + 6.4 / 8.3 / 5.2
 constexpr int kJoinStates = 48;                          // (states of all tokens: beyond, what the workgroups of a head read again costs more than the launch)
 template <typename WT>
-__global__ __launch_bounds__(256) void latent_join_unfold_kernel(float* out, int ldo, const float* scratch, int splits, const WT* w, const float* gate, int ldg, int H, int dv, int R, int head_gate) {
-    __shared__ float wt[256], red[16];
-    __shared__ __attribute__((aligned(16))) float ls[512];
+__global__ __launch_bounds__(512) void latent_join_unfold_kernel(float* out, int ldo, const float* scratch, int splits, const WT* w, const float* gate, int ldg, int H, int dv, int R, int head_gate) {
+    constexpr int EACH = kJoinStates / 4;
+    __shared__ float wt[kJoinStates], red;
+    __shared__ __attribute__((aligned(16))) float part[4][512];
+    typedef float f4 __attribute__((ext_vector_type(4)));
     const int h = blockIdx.y, t = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int v0 = blockIdx.x * 16 + wave * 4, r0 = lane * 8, c = 2 * tid;
+    const int v0 = blockIdx.x * 32 + wave * 4, r0 = lane * 8, c = 4 * (tid & 127), mine = tid >> 7;
+    const long long at = ((long long)t * H + h) * splits, states = (long long)gridDim.z * H * splits;
+    const float* st = scratch + at * R, *ml = scratch + states * R + 2 * at;
+    float m = -INFINITY, l = 0.0f;
+    if (wave == 0 && lane < splits) { m = ml[2 * lane]; l = ml[2 * lane + 1]; }
+    f4 x[EACH];
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) {
+        x[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (4 * u + mine < splits && c < R) x[u] = *reinterpret_cast<const f4*>(st + (long long)(4 * u + mine) * R + c);
+    }
     float wv[4][8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -527,32 +543,35 @@ __global__ __launch_bounds__(256) void latent_join_unfold_kernel(float* out, int
             wv[i][0] = a.x; wv[i][1] = a.y; wv[i][2] = a.z; wv[i][3] = a.w; wv[i][4] = b.x; wv[i][5] = b.y; wv[i][6] = b.z; wv[i][7] = b.w;
         }
     }
-    const float* st = scratch + ((long long)t * H + h) * splits * (2 + R);
-    const long long step = 2 + R;
-    float2 x[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = u < splits && c < R ? *reinterpret_cast<const float2*>(st + u * step + 2 + c) : float2{0.0f, 0.0f};
-    const float m = tid < splits ? st[tid * step] : -INFINITY, l = tid < splits ? st[tid * step + 1] : 0.0f;
-    const float mx = block_max(m, red);
-    const float we = m == -INFINITY ? 0.0f : expf(m - mx);
-    wt[tid] = we;
-    const float den = block_sum(we * l, red);            // (its barriers publish wt)
-    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-    float2 sum{0.0f, 0.0f};
-    for (int s = 0; s < splits; s += 8) {                // states in order, eight requested ahead
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (s + u < splits) { sum.x = fmaf(x[u].x, wt[s + u], sum.x); sum.y = fmaf(x[u].y, wt[s + u], sum.y); }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (s + 8 + u < splits && c < R) x[u] = *reinterpret_cast<const float2*>(st + (s + 8 + u) * step + 2 + c);
+    if (wave == 0) {                                     // (at most 48 states: one wave has them)
+        const float mx = wave_max(m);
+        const float we = m == -INFINITY ? 0.0f : expf(m - mx);
+        if (lane < kJoinStates) wt[lane] = we;           // (zero behind the last)
+        const float den = wave_sum(we * l);
+        if (lane == 0) red = den > 0.0f ? 1.0f / den : 0.0f;
     }
-    if (c < R) *reinterpret_cast<float2*>(ls + c) = float2{sum.x * inv, sum.y * inv};
     __syncthreads();
+    f4 sum{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < EACH; ++u) {
+        const float we = wt[4 * u + mine];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum[k] = fmaf(x[u][k], we, sum[k]);
+    }
+    *reinterpret_cast<f4*>(&part[mine][c]) = sum;
+    __syncthreads();
+    if (v0 >= dv) return;
+    const float inv = red;
     float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (r0 < R) {
-        const float4 a = *reinterpret_cast<const float4*>(ls + r0), b = *reinterpret_cast<const float4*>(ls + r0 + 4);
-        const float xx[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        float xx[8];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const f4 p0 = *reinterpret_cast<const f4*>(&part[0][r0 + 4 * k]), p1 = *reinterpret_cast<const f4*>(&part[1][r0 + 4 * k]), p2 = *reinterpret_cast<const f4*>(&part[2][r0 + 4 * k]),
+                     p3 = *reinterpret_cast<const f4*>(&part[3][r0 + 4 * k]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xx[4 * k + j] = ((p0[j] + p1[j]) + (p2[j] + p3[j])) * inv;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -584,13 +603,16 @@ static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, in
     sa.scale = scale; sa.scratch = scratch;
     sa.splits = shared_splits(shared_keys(pos0, T, window));
     const int rows = T * H, DK = kv_rank + rot_dim;
-    const size_t lds = ((size_t)KB * (((DK + 15) & ~15) + 4) + 5 * SROWS * (KB + 4) + 3 * SROWS) * sizeof(float);
-    static bool raised_s = false;   // (idempotent: a race sets the same attribute twice)
-    if (!raised_s) { NTK_HIP_TRY(hipFuncSetAttribute((const void*)latent_attention_shared_kernel<13, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024)); raised_s = true; }
     const dim3 grid((rows + SROWS - 1) / SROWS, sa.splits);
-    if (DK <= 128) hipLaunchKernelGGL((latent_attention_shared_kernel<2, 2>), grid, dim3(256), lds, s, sa);
-    else if (DK <= 320) hipLaunchKernelGGL((latent_attention_shared_kernel<5, 5>), grid, dim3(256), lds, s, sa);
-    else hipLaunchKernelGGL((latent_attention_shared_kernel<13, 8>), grid, dim3(256), lds, s, sa);
+    const bool whole = !((kv_rank | rot_dim | row | ldq) & 3) && !(((uintptr_t)cache | (uintptr_t)q | (uintptr_t)scratch) & 15);
+    auto launch = [&](auto kernel, auto narrow, int waves) {
+        if (whole) hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, s, sa);
+        else hipLaunchKernelGGL(narrow, grid, dim3(64 * waves), 0, s, sa);
+    };
+    if (DK <= 128) launch(latent_attention_shared_kernel<2, 4, true>, latent_attention_shared_kernel<2, 4, false>, 4);
+    else if (DK <= 320 && kv_rank <= 256) launch(latent_attention_shared_kernel<5, 4, true>, latent_attention_shared_kernel<5, 4, false>, 4);
+    else if (DK <= 640) launch(latent_attention_shared_kernel<5, 8, true>, latent_attention_shared_kernel<5, 8, false>, 8);
+    else launch(latent_attention_shared_kernel<7, 8, true>, latent_attention_shared_kernel<7, 8, false>, 8);
     const int st = last_launch_status();
     if (st != NTK_OK || !merge) return st;
     hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(rows, (kv_rank + 63) / 64), dim3(256), 0, s, out, ldo, (const float*)scratch, sa.splits, kv_rank, H);
@@ -602,8 +624,7 @@ static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, in
 using namespace ntk;
 
 int ntk_latent_shared_takes(int kv_rank, int rot_dim) {
-    const int DK = kv_rank + rot_dim;
-    return kv_rank > 0 && kv_rank <= 512 && rot_dim >= 0 && ((size_t)(KB + SROWS) * (((DK + 3) & ~3) + 4) + SROWS * KB + 3 * SROWS) * sizeof(float) <= 156 * 1024;     // (keys of up to 816 entries)
+    return kv_rank > 0 && kv_rank <= 512 && rot_dim >= 0 && kv_rank + rot_dim <= 816;
 }
 
 int ntk_latent_prepare(float* cache, int row, const float* kv, int ldkv, const float* norm_w, float eps, int kv_rank, int rot_dim, float* q, int ldq, int H, int qd,
@@ -717,11 +738,11 @@ int ntk_latent_attention_unfold(float* out, int ldo, const void* w_uv, int wdtyp
     const int st = launch_shared(sa, lat, H * kv_rank, qf, ldq, cache, row, kv_rank, rot_dim, H, pos0, T, window, scale, scratch, !join, stream);
     if (st != NTK_OK) return st;
     if (!join) return ntk_latent_unfold_value_ex(out, ldo, lat, w_uv, wdtype, gate, ldg, head_gate, T, H, dv, kv_rank, stream);
-    const dim3 grid((dv + 15) / 16, H, T);
+    const dim3 grid((dv + 31) / 32, H, T);
     if (wdtype == NTK_DT_BF16)
-        hipLaunchKernelGGL(latent_join_unfold_kernel<uint16_t>, grid, dim3(256), 0, resolve_stream(stream), out, ldo, (const float*)scratch, sa.splits, (const uint16_t*)w_uv, gate, ldg, H, dv, kv_rank, head_gate);
+        hipLaunchKernelGGL(latent_join_unfold_kernel<uint16_t>, grid, dim3(512), 0, resolve_stream(stream), out, ldo, (const float*)scratch, sa.splits, (const uint16_t*)w_uv, gate, ldg, H, dv, kv_rank, head_gate);
     else
-        hipLaunchKernelGGL(latent_join_unfold_kernel<float>, grid, dim3(256), 0, resolve_stream(stream), out, ldo, (const float*)scratch, sa.splits, (const float*)w_uv, gate, ldg, H, dv, kv_rank, head_gate);
+        hipLaunchKernelGGL(latent_join_unfold_kernel<float>, grid, dim3(512), 0, resolve_stream(stream), out, ldo, (const float*)scratch, sa.splits, (const float*)w_uv, gate, ldg, H, dv, kv_rank, head_gate);
     return last_launch_status();
 }
 

@@ -100,6 +100,13 @@ def test_shared_latents_at_the_limits_of_the_operand_sizes(R, dr, H, T, pos0, wi
     test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, window)
 
 
+@pytest.mark.parametrize("R,dr", [(256, 60), (260, 60), (252, 68), (512, 128), (509, 131), (512, 132), (512, 304), (64, 752)])
+@pytest.mark.parametrize("T,H,pos0,window", [(1, 17, 31, 0), (4, 8, 32, 0), (2, 16, 4500, 0)])
+def test_shared_latents_by_rank_and_by_key(R, dr, H, T, pos0, window):
+    """four and eight waves (a rank of 256 and one past it, keys of 320), keys of 640, the longest ones; the last position of a tile, the first of the next, several tiles a workgroup"""
+    test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, window)
+
+
 @pytest.mark.parametrize("what", [np.nan, np.inf, -np.inf])
 @pytest.mark.parametrize("H,G,dn,dv,window,keep,option", [(2, 2, 64, 64, 0, 0, ""), (4, 1, 33, 17, 0, 0, "gate"), (2, 1, 128, 128, 20, 3, "cap_sink"), (3, 3, 192, 100, 33, 0, "slopes"),
                                                           (4, 2, 40, 64, 48, 0, "chunks"), (2, 1, 16, 33, 0, 0, "rel"), (3, 1, 128, 36, 37, 0, "head_gate")])
