@@ -412,6 +412,20 @@ int ntk_moe_route_ex(int* ids, float* wts, float* sgate, const float* h, int ldh
 /* ... of h = x / rms(x) * (norm_offset + norm_w), formed in the same launch and left in h (r->add_y NULL) */
 int ntk_moe_norm_route(int* ids, float* wts, float* sgate, float* h, int ldh, const float* x, int ldx, const float* norm_w, float norm_eps, float norm_offset, const float* w_router,
                        const float* shared_gate_w, int T, int n, int E, int top, const ntk_route_desc* r, void* stream);
+/* ... as one argument */
+typedef struct ntk_norm_route {
+    int* ids; float* wts; float* sgate;
+    float* h; int ldh;
+    const float* x; int ldx;
+    const float* norm_w; float norm_eps, norm_offset;
+    const float* w_router; const float* shared_gate_w;
+    int T, n, E, top;
+    const ntk_route_desc* form;
+} ntk_norm_route;
+/* ntk_latent_attention_unfold, and ntk_moe_norm_route of a router that waits for nothing the attention leaves (neither may read what the other writes): in the attention's launch where it
+ * has room for it, else behind it */
+int ntk_latent_attention_unfold_route(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,
+                                      int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale, float* scratch, const ntk_norm_route* route, void* stream);
 /* The choice alone, from router outputs that a product left: z [T][ldz] = [E outputs | the shared unit's gate ahead of its sigmoid (if sgate)] (r->add_y must be NULL) */
 int ntk_moe_pick(int* ids, float* wts, float* sgate, const float* z, int ldz, int T, int E, int top, const ntk_route_desc* r, void* stream);
 /* The experts of a few tokens (T <= ntk_dense_few_rows(), decoding) in two launches, without grouping: plain units U_e then D_e with the activation `act` between them,

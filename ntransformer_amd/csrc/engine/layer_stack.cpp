@@ -1083,7 +1083,7 @@ int LayerStackModel::truncate_slot(int slot, int length) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------------ the step
-int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside, const void* h16) {
+int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside, const void* h16, const ntk_norm_route* beside) {
     const LatentMixer& m = L.mix;
     const int W = info_.width, H = m.heads, qd = m.qd(), row = m.row(), hv = H * m.vdim, na = (int)m.in.out_f;
     // one product for [query (latent) | latent + key part | gate] of the mixer's input h; norm_inside (few rows): h is the stream, the layer's first norm runs
@@ -1116,13 +1116,13 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
     }
     ntk_rotary rot{m.rot_freq, m.rot_mag, m.rot_dims, m.rot_layout};
     const bool own = m.kv_from < 0;                       // (else: the rows another layer wrote for these tokens earlier in the pass)
-    const bool beside = own && T <= kSharedRows;      // few tokens: the cache rows are written beside the queries' fold
-    if (own && !beside) LS_TRY(ntk_latent_prepare(cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, m.kv_rank, m.rot_dim, q, ldq, H, qd, &rot, pos0, T, stream_));
+    const bool with_fold = own && T <= kSharedRows;      // few tokens: the cache rows are written beside the queries' fold
+    if (own && !with_fold) LS_TRY(ntk_latent_prepare(cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, m.kv_rank, m.rot_dim, q, ldq, H, qd, &rot, pos0, T, stream_));
     if (T <= kSharedRows) {
-        if (beside) LS_TRY(ntk_latent_fold_query_rotate(qf_, q, ldq, m.uk.ptr, m.uk.dtype, T, H, m.dim, m.rot_dim, m.kv_rank, &rot, cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, pos0, stream_));
+        if (with_fold) LS_TRY(ntk_latent_fold_query_rotate(qf_, q, ldq, m.uk.ptr, m.uk.dtype, T, H, m.dim, m.rot_dim, m.kv_rank, &rot, cache, row, a_ + m.kv_off, na, m.kv_norm, eps_, pos0, stream_));
         else LS_TRY(ntk_latent_fold_query(qf_, q, ldq, m.uk.ptr, m.uk.dtype, T, H, m.dim, m.rot_dim, m.kv_rank, stream_));
-        LS_TRY(ntk_latent_attention_unfold(att_, hv, m.uv.ptr, m.uv.dtype, a_ + m.g_off, na, m.head_gate ? 1 : 0, m.vdim, lat_, qf_, cache, row, m.kv_rank, m.rot_dim, H, pos0, T, m.window,
-                                           m.scale, scratch_, stream_));
+        LS_TRY(ntk_latent_attention_unfold_route(att_, hv, m.uv.ptr, m.uv.dtype, a_ + m.g_off, na, m.head_gate ? 1 : 0, m.vdim, lat_, qf_, cache, row, m.kv_rank, m.rot_dim, H, pos0, T, m.window,
+                                                 m.scale, scratch_, beside, stream_));
     } else {
         const int key0 = m.window > 0 ? std::max(0, pos0 - m.window + 1) : 0;
         const int nkeys = pos0 + T - key0;
@@ -1304,10 +1304,18 @@ static bool in_two_launches(const MoeFeedForward& M, int T, int W) {
     return two <= six;
 }
 
+// the parallel form's router of a few tokens: its rows are the norm of the stream as the layer finds it, left in h2_
+ntk_norm_route LayerStackModel::norm_route(const StackLayer& L, int T) const {
+    const MoeFeedForward& M = L.mlp;
+    const int W = info_.width;
+    float* sgate = M.has_shared && M.shared_gate ? sg_ : nullptr;
+    return ntk_norm_route{ids_, wts_, sgate, h2_, W, x_, W, L.norm2.w, eps_, 1.0f, M.router, sgate ? M.shared_gate : nullptr, T, W, M.experts + M.identity, M.top, &M.route};
+}
+
 // router, grouping, the experts' products; then either straight into the stream together with the mixer's output (parallel form) or as a sum of its own
 // in ff_ (sequential form: it is normed before it joins the stream)
-// (norm_w: h is the norm of the stream by this weight, to be formed in the router's launch)
-int LayerStackModel::run_moe(const StackLayer& L, float* h, int T, bool into_stream, const void* h16, const float* norm_w) {
+// (routed: the choice and h are there already, from norm_route)
+int LayerStackModel::run_moe(const StackLayer& L, float* h, int T, bool into_stream, const void* h16, bool routed) {
     const MoeFeedForward& M = L.mlp;
     const int W = info_.width, choices = M.experts + M.identity;
     float* sgate = M.has_shared && M.shared_gate ? sg_ : nullptr;
@@ -1332,8 +1340,7 @@ int LayerStackModel::run_moe(const StackLayer& L, float* h, int T, bool into_str
         route.add_y = owed_.y; route.ld_add = W; route.add_w = owed_.nb.w; route.add_eps = eps_;
         owed_.y = nullptr;
     }
-    if (norm_w) LS_TRY(ntk_moe_norm_route(ids_, wts_, sgate, h, W, x_, W, norm_w, eps_, 1.0f, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
-    else LS_TRY(ntk_moe_route_ex(ids_, wts_, sgate, h, W, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
+    if (!routed) LS_TRY(ntk_moe_route_ex(ids_, wts_, sgate, h, W, M.router, sgate ? M.shared_gate : nullptr, T, W, choices, M.top, &route, stream_));
     const bool few = !M.routed.plain && T <= ntk_dense_few_rows() && mid <= NTK_MOE_FEW_MID && W <= NTK_MOE_FEW_MID && !(into_stream && M.identity);
     if (few && in_two_launches(M, T, W)) {
         ntk_moe_few_desc d{};
@@ -1678,11 +1685,13 @@ int LayerStackModel::parallel_layer(const Run& run, const StackLayer& L, int slo
         }
         if (st == NTK_E_ALIGN) st = ntk_rmsnorm_offset(h1_, L.norm1.w, L.has_mlp ? h2_ : nullptr, L.has_mlp ? L.norm2.w : nullptr, W, x_, W, T, W, eps_, 1.0f, stream_);
         LS_TRY(st);
-    }   // (decoding: the mixer's norm runs inside its first product (run_mixer), the feed-forward's in its router's launch)
+    }   // (decoding: the mixer's norm runs inside its first product (run_mixer), the feed-forward's with its router, which waits for nothing of the mixer: beside attention)
     float* cache = run.cache + (size_t)slot * opt_.max_context * L.mix.row();
     const bool few = T <= ntk_dense_few_rows();
-    LS_TRY(run_mixer(L, cache, T, pos0, few ? x_ : h1_, few, h16));
-    if (L.has_mlp) return run_moe(L, h2_, T, true, g16, few ? L.norm2.w : nullptr);
+    const bool routed = few && L.has_mlp;
+    const ntk_norm_route route = routed ? norm_route(L, T) : ntk_norm_route{};
+    LS_TRY(run_mixer(L, cache, T, pos0, few ? x_ : h1_, few, h16, routed ? &route : nullptr));
+    if (L.has_mlp) return run_moe(L, h2_, T, true, g16, routed);
     return ntk_residual_add(x_, mix_, nullptr, T * W, stream_);
 }
 

@@ -333,13 +333,14 @@ private:
     int portion(int slot, const int* tokens_dev, int token, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out);
     int last_layer_keys(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     bool takes_one_token(const StackLayer& L) const;
-    int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false, const void* h16 = nullptr);
+    int run_mixer(const StackLayer& L, float* cache, int T, int pos0, const float* h, bool norm_inside = false, const void* h16 = nullptr, const ntk_norm_route* beside = nullptr);
     int run_window(const StackLayer& L, const float* h, float* cache, int T, int pos0, bool norm_inside = false, const void* h16 = nullptr);
     int window_heads(const WindowMixer& m, float* cache, float* out, int ldo, int T, int pos0);
     int window_keys_values(const WindowMixer& m, float* cache, int T, int pos0);
     int dense_parallel_layer(const Run& run, const StackLayer& L, int slot, int T, int pos0);
     int run_lightning(const StackLayer& L, float* state, int T, int pos0);
-    int run_moe(const StackLayer& L, float* h, int T, bool into_stream, const void* h16 = nullptr, const float* norm_w = nullptr);
+    int run_moe(const StackLayer& L, float* h, int T, bool into_stream, const void* h16 = nullptr, bool routed = false);
+    ntk_norm_route norm_route(const StackLayer& L, int T) const;
     int run_dense_ff(const StackLayer& L, int T);
     int run_experts(float glu_alpha, float glu_up_offset, const GatedExperts& ex, const float* h, float* gu, float* act, float* out, int rows, const int* offsets, const int* order, int top,
                     int full_x, const void* h16 = nullptr, const float* norm_w = nullptr);   // norm_w (few rows): the rows are normed inside the first product

@@ -10,6 +10,7 @@
 // LDS), online softmax per row in F32, lane = value column for the weighted sum.  Shared: a workgroup owns 16 (token, head) rows and whole tiles of 32
 // cache rows; the tiles go round up to 128 workgroups and a second launch merges their (max, sum, vector) states.
 #include "attention_pieces.hip.h"
+#include "moe_route.hip.h"
 #include "../../include/ntk_layers.h"
 
 namespace ntk {
@@ -222,8 +223,24 @@ struct SharedArgs {
 
 // NW waves: ranks up to 64 * NW; KS: keys of (latent + rotated) up to 16 * NW * KS entries; V: rows of whole fours on 16 bytes.  The smaller sizes need fewer registers, which
 // counts where many rows walk a long context.  us with the merge, 8 tokens of 64 heads at 8000 positions, tile in LDS / so: 32 + 8 121 / 43, 256 + 32 157 / 95, 512 + 64 400 / 193.
-template <int KS, int NW, bool V>
-__global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const SharedArgs a) {
+// ROUTE: the first `beside` rows of the grid's workgroups choose a token's experts each (route_token), which waits for nothing that attention leaves.  Attention of one token leaves most
+// CUs idle and takes about as long: us, 16 heads, 512 + 64, 1100 positions, and a router of 32 experts of 2048 inputs: 9.6 + 8.7 in two launches, 10.8 so (12.5 with four rows
+// of the router a wave, requested behind the norm).
+struct NoRoute {};
+struct RouteBeside { RouteJob job; int T, rows; };
+constexpr int kRouteBesideInputs = 4096;
+template <int KS, int NW, bool V, bool ROUTE = false>
+__global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const SharedArgs a, const std::conditional_t<ROUTE, RouteBeside, NoRoute> route) {
+    int part = blockIdx.y;
+    if constexpr (ROUTE) {
+        __shared__ __attribute__((aligned(16))) float xs[kRouteBesideInputs];
+        if (part < route.rows) {
+            const int t = part * (int)gridDim.x + (int)blockIdx.x;
+            if (t < route.T) route_token<NW, 5>(route.job, t, xs);
+            return;
+        }
+        part -= route.rows;
+    }
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef f4 f4_anywhere __attribute__((aligned(4)));
     constexpr int PP = KB + 4, TPR = 4 * NW, KPT = KB / TPR;       // softmax: threads a row, keys a thread
@@ -262,7 +279,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
 #pragma unroll
             for (int c = 0; c < 4; ++c) vf[e][c] = four(a.cache + (long long)min(j0 + 16 * e + 4 * g4 + c, jhi) * a.row, col, a.R);
     };
-    int j0 = jlo + KB * (int)blockIdx.y;
+    int j0 = jlo + KB * part;
     const int hop = KB * a.splits;
     {
         const int r = min(row0 + i16, n_rows - 1);
@@ -305,15 +322,15 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
 #pragma unroll
             for (int e = 0; e < KPT; ++e) {
                 const int key = sub + TPR * e, j = j0 + key;
-                float part[NW];
+                float sc[NW];
 #pragma unroll
-                for (int w = 0; w < NW; ++w) part[w] = Sp[(w * SROWS + srow) * PP + key];
+                for (int w = 0; w < NW; ++w) sc[w] = Sp[(w * SROWS + srow) * PP + key];
 #pragma unroll
                 for (int n = NW / 2; n; n >>= 1)
 #pragma unroll
-                    for (int w = 0; w < n; ++w) part[w] += part[w + n];
+                    for (int w = 0; w < n; ++w) sc[w] += sc[w + n];
                 const bool vis = key < nk && rpos >= 0 && j <= rpos && (a.window <= 0 || rpos - j < a.window);
-                sv[e] = vis ? part[0] * a.scale : -INFINITY;
+                sv[e] = vis ? sc[0] * a.scale : -INFINITY;
                 mc = fmaxf(mc, sv[e]);
             }
 #pragma unroll
@@ -363,7 +380,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
     for (int r = 0; r < 4; ++r) {
         const int i = 4 * g4 + r;
         if (row0 + i >= n_rows) continue;
-        const long long at = (long long)(row0 + i) * a.splits + blockIdx.y;
+        const long long at = (long long)(row0 + i) * a.splits + part;
         if (wave == 0 && i16 == 0) { a.scratch[states * a.R + 2 * at] = ms[i]; a.scratch[states * a.R + 2 * at + 1] = ls[i]; }
         float* st = a.scratch + at * a.R;
         if constexpr (V) { if (col < a.R) *reinterpret_cast<f4*>(st + col) = f4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]}; }
@@ -593,9 +610,16 @@ static int shared_splits(int nkeys) {       // workgroups per row tile: one per 
 }
 
 static int shared_keys(int pos0, int T, int window) { return window > 0 ? (window + T - 1 < pos0 + T ? window + T - 1 : pos0 + T) : pos0 + T; }
+static bool shared_whole(const float* q, int ldq, const float* cache, int row, int kv_rank, int rot_dim, const float* scratch) {
+    return !((kv_rank | rot_dim | row | ldq) & 3) && !(((uintptr_t)cache | (uintptr_t)q | (uintptr_t)scratch) & 15);
+}
+// A router beside attention: where the workgroups are of eight waves (four walk the router's rows alone for longer than such attention takes) and a row fits beside a tile.
+static bool shared_takes_route(bool whole, int kv_rank, int rot_dim, int n) {
+    return whole && kv_rank + rot_dim > 128 && (kv_rank + rot_dim > 320 || kv_rank > 256) && ntk_latent_shared_takes(kv_rank, rot_dim) && n <= kRouteBesideInputs;
+}
 // the shared form: every part's states into the scratch; merge: joined in `out`
 static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, int ldq, const float* cache, int row, int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale,
-                         float* scratch, bool merge, void* stream) {
+                         float* scratch, bool merge, void* stream, const RouteBeside* route = nullptr) {
     if (!scratch) return NTK_E_NULL;
     if (!ntk_latent_shared_takes(kv_rank, rot_dim)) return NTK_E_SHAPE;
     hipStream_t s = resolve_stream(stream);
@@ -603,12 +627,19 @@ static int launch_shared(SharedArgs& sa, float* out, int ldo, const float* q, in
     sa.scale = scale; sa.scratch = scratch;
     sa.splits = shared_splits(shared_keys(pos0, T, window));
     const int rows = T * H, DK = kv_rank + rot_dim;
-    const dim3 grid((rows + SROWS - 1) / SROWS, sa.splits);
-    const bool whole = !((kv_rank | rot_dim | row | ldq) & 3) && !(((uintptr_t)cache | (uintptr_t)q | (uintptr_t)scratch) & 15);
+    dim3 grid((rows + SROWS - 1) / SROWS, sa.splits);
+    const bool whole = shared_whole(q, ldq, cache, row, kv_rank, rot_dim, scratch);
     auto launch = [&](auto kernel, auto narrow, int waves) {
-        if (whole) hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, s, sa);
-        else hipLaunchKernelGGL(narrow, grid, dim3(64 * waves), 0, s, sa);
+        if (whole) hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, s, sa, NoRoute{});
+        else hipLaunchKernelGGL(narrow, grid, dim3(64 * waves), 0, s, sa, NoRoute{});
     };
+    if (route) {                                   // (shared_takes_route)
+        RouteBeside r = *route;
+        r.rows = (r.T + (int)grid.x - 1) / (int)grid.x;
+        grid.y += r.rows;
+        if (DK <= 640) hipLaunchKernelGGL((latent_attention_shared_kernel<5, 8, true, true>), grid, dim3(512), 0, s, sa, r);
+        else hipLaunchKernelGGL((latent_attention_shared_kernel<7, 8, true, true>), grid, dim3(512), 0, s, sa, r);
+    } else
     if (DK <= 128) launch(latent_attention_shared_kernel<2, 4, true>, latent_attention_shared_kernel<2, 4, false>, 4);
     else if (DK <= 320 && kv_rank <= 256) launch(latent_attention_shared_kernel<5, 4, true>, latent_attention_shared_kernel<5, 4, false>, 4);
     else if (DK <= 640) launch(latent_attention_shared_kernel<5, 8, true>, latent_attention_shared_kernel<5, 8, false>, 8);
@@ -728,14 +759,31 @@ int ntk_latent_fold_query_prepare(float* qf, const float* q, int ldq, const void
 
 int ntk_latent_attention_unfold(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,
                                 int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale, float* scratch, void* stream) {
+    return ntk_latent_attention_unfold_route(out, ldo, w_uv, wdtype, gate, ldg, head_gate, dv, lat, qf, cache, row, kv_rank, rot_dim, H, pos0, T, window, scale, scratch, nullptr, stream);
+}
+
+int ntk_latent_attention_unfold_route(float* out, int ldo, const void* w_uv, int wdtype, const float* gate, int ldg, int head_gate, int dv, float* lat, const float* qf, const float* cache, int row,
+                                      int kv_rank, int rot_dim, int H, int pos0, int T, int window, float scale, float* scratch, const ntk_norm_route* route, void* stream) {
     if (!out || !w_uv || !lat || !qf || !cache || !scratch) return NTK_E_NULL;
     if (wdtype != NTK_DT_BF16 && wdtype != NTK_DT_F32) return NTK_E_DTYPE;
     if (T < 0 || H <= 0 || dv <= 0 || kv_rank <= 0 || rot_dim < 0 || pos0 < 0 || row < kv_rank + rot_dim) return NTK_E_SHAPE;
+    RouteBeside rb{};
+    if (route) {
+        const int st = norm_route_job(route, &rb.job);
+        if (st != NTK_OK) return st;
+        rb.T = route->T;
+    }
+    const int ldq = H * (kv_rank + rot_dim);
+    const bool beside = route && T > 0 && shared_takes_route(shared_whole(qf, ldq, cache, row, kv_rank, rot_dim, scratch), kv_rank, rot_dim, route->n);
+    if (route && !beside) {
+        const int st = ntk_moe_norm_route(route->ids, route->wts, route->sgate, route->h, route->ldh, route->x, route->ldx, route->norm_w, route->norm_eps, route->norm_offset, route->w_router,
+                                          route->shared_gate_w, route->T, route->n, route->E, route->top, route->form, stream);
+        if (st != NTK_OK) return st;
+    }
     if (T == 0) return NTK_OK;
     SharedArgs sa{};
-    const int ldq = H * (kv_rank + rot_dim);
     const bool join = kv_rank % 8 == 0 && kv_rank <= 512 && T * shared_splits(shared_keys(pos0, T, window)) <= kJoinStates && !(((uintptr_t)w_uv | (uintptr_t)scratch) & 15);
-    const int st = launch_shared(sa, lat, H * kv_rank, qf, ldq, cache, row, kv_rank, rot_dim, H, pos0, T, window, scale, scratch, !join, stream);
+    const int st = launch_shared(sa, lat, H * kv_rank, qf, ldq, cache, row, kv_rank, rot_dim, H, pos0, T, window, scale, scratch, !join, stream, beside ? &rb : nullptr);
     if (st != NTK_OK) return st;
     if (!join) return ntk_latent_unfold_value_ex(out, ldo, lat, w_uv, wdtype, gate, ldg, head_gate, T, H, dv, kv_rank, stream);
     const dim3 grid((dv + 31) / 32, H, T);

@@ -5,170 +5,15 @@
 //
 // A token's result never depends on the other tokens of the launch: the grouping only decides WHERE a pair's row sits, each row is computed on its
 // own, and the sum over a token's slots runs in slot order.
-#include "common.hip.h"
-#include "../../include/ntk_layers.h"
+#include "moe_route.hip.h"
 
 namespace ntk {
 
-constexpr int kMaxExperts = 256;
-
-// one workgroup per token: its 16 waves share the experts (wave w: experts w, w + 16, ...), a lane requests its whole part of the router row before
-// it uses any of it; thread 0 then does the softmax and the `top` picks over the scores in LDS
-constexpr int kRouteThreads = 1024;
-struct RouteForm { int score, groups, keep, group_top, renorm; float scale; const float* correction; const float* add_y; int ld_add; const float* add_w; float add_eps;
-    const float* src; int ldsrc; const float* norm_w; float norm_eps, norm_offset;     // (norm_w: the token's row is the RMS norm of a row of src, formed in the launch and left in h; NULL: h holds it)
-};
-
-// the largest of a wave's 4 x 64 values (lane l holds entries l, l + 64, l + 128, l + 192); equal values: the lower index
-__device__ __forceinline__ void wave_argmax4(const float (&v)[4], int lane, float& bv, int& bi) {
-    bv = wave_max(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
-    bi = 0;
-#pragma unroll
-    for (int c = 3; c >= 0; --c) {                            // (the lowest index is the first lane of the first quarter that holds the value)
-        const unsigned long long m = __ballot(v[c] == bv);
-        if (m) bi = 64 * c + __ffsll((unsigned long long)m) - 1;
-    }
-}
-
-// scores and the picks by one wave: lane l holds experts l, l + 64, l + 128, l + 192; z [E] in LDS
-__device__ __forceinline__ void pick_experts(float* z, int lane, long long t, int E, int top, const RouteForm& f, int* ids, float* wts) {
-    float v[4];
-    float den = 1.0f;
-    if (f.score == 0) {
-        float m = -INFINITY;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) { v[c] = lane + 64 * c < E ? z[lane + 64 * c] : -INFINITY; m = fmaxf(m, v[c]); }
-        m = wave_max(m);
-        den = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) { v[c] = lane + 64 * c < E ? expf(v[c] - m) : -INFINITY; den += fmaxf(v[c], 0.0f); }
-        den = wave_sum(den);
-    } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) v[c] = lane + 64 * c < E ? 1.0f / (1.0f + expf(-z[lane + 64 * c])) : -INFINITY;
-    }
-    if (f.correction) {     // (uniform) what is chosen by is no longer what is weighted with: the scores stay in LDS, v becomes the choice scores
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (lane + 64 * c < E) { const float s = v[c] / den; z[lane + 64 * c] = s; v[c] = s + f.correction[lane + 64 * c]; }
-        __builtin_amdgcn_wave_barrier();
-    }
-    __shared__ int pick_id[kMaxExperts];
-    __shared__ float pick_sc[kMaxExperts];
-    if (f.groups > 1) {
-        // group scores: lane l owns groups l, l + 64, ...: the sum of the group's `group_top` largest scores
-        __shared__ float sc[kMaxExperts];
-        __shared__ unsigned char open_group[kMaxExperts];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (lane + 64 * c < E) sc[lane + 64 * c] = v[c];
-        __builtin_amdgcn_wave_barrier();
-        const int per = E / f.groups;
-        float gs[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int g = lane + 64 * c;
-            gs[c] = -INFINITY;
-            if (g < f.groups) {
-                float sum = 0.0f;
-                const int nt = min(f.group_top, per);
-                float last = INFINITY;
-                int last_e = -1;
-                for (int k = 0; k < nt; ++k) {                // the largest behind the one before it (equal values: by index)
-                    float best = -INFINITY;
-                    int bi = -1;
-                    for (int e = g * per; e < (g + 1) * per; ++e)
-                        if ((sc[e] < last || (sc[e] == last && e > last_e)) && sc[e] > best) { best = sc[e]; bi = e; }
-                    last = best;
-                    last_e = bi;
-                    sum += best;
-                }
-                gs[c] = sum;
-            }
-            if (g < kMaxExperts) open_group[g] = 0;
-        }
-        __builtin_amdgcn_wave_barrier();
-        for (int k = 0; k < f.keep; ++k) {                    // (taken ones are marked -inf)
-            float bv;
-            int bi;
-            wave_argmax4(gs, lane, bv, bi);
-            if (lane == 0) open_group[bi] = 1;
-            if ((bi & 63) == lane) gs[bi >> 6] = -INFINITY;
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (lane + 64 * c < E && !open_group[(lane + 64 * c) / per]) v[c] = -INFINITY;
-    }
-    float chosen = 0.0f;
-    for (int s = 0; s < top; ++s) {
-        float bv;
-        int bi;
-        wave_argmax4(v, lane, bv, bi);
-        const float sc1 = f.correction ? z[bi] : bv / den;
-        chosen += sc1;
-        if (lane == 0) { pick_id[s] = bi; pick_sc[s] = sc1; }
-        if ((bi & 63) == lane) v[bi >> 6] = -INFINITY;
-    }
-    const float mul = (f.renorm ? 1.0f / (chosen + 1e-20f) : 1.0f) * f.scale;
-    for (int s = lane; s < top; s += 64) { ids[t * top + s] = pick_id[s]; wts[t * top + s] = pick_sc[s] * mul; }   // (same wave wrote them: in order)
-}
-
-__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(int* ids, float* wts, float* sgate, float* h, int ldh, const float* wr, const float* wsg,
-                                                                 int n, int E, int top, const RouteForm f) {
-    __shared__ float z[kMaxExperts];
+// one workgroup per token
+constexpr int kRouteWaves = 16;
+__global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(const RouteJob j) {
     extern __shared__ __attribute__((aligned(16))) float xs[];   // the token's row
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = kRouteThreads / 64;
-    const long long t = blockIdx.x;
-    float* x = h + t * ldh;
-    if (f.norm_w) {    // (uniform).  us, one token of 2048 among 32 experts: 6.4 the norm in a launch of its own and 7.5 the choice, 9.1 so (weights requested ahead of the row: 10.9)
-        __shared__ float red[16];
-        const float* y = f.src + t * f.ldsrc;
-        float ss = 0.0f;
-        for (int k = threadIdx.x; k < n; k += kRouteThreads) { const float v = y[k]; xs[k] = v; ss = fmaf(v, v, ss); }
-        const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)n + f.norm_eps);
-        for (int k = threadIdx.x; k < n; k += kRouteThreads) {
-            const float v = xs[k] * inv * (f.norm_offset + f.norm_w[k]);
-            xs[k] = v;
-            x[k] = v;
-        }
-    } else if (f.add_y) {     // (uniform) what the row is still owed joins it: y / rms(y) * w; a thread re-reads its own entries
-        __shared__ float red[16];
-        const float* y = f.add_y + t * f.ld_add;
-        float ss = 0.0f;
-        for (int k = threadIdx.x; k < n; k += kRouteThreads) { xs[k] = x[k]; ss = fmaf(y[k], y[k], ss); }
-        const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)n + f.add_eps);
-        for (int k = threadIdx.x; k < n; k += kRouteThreads) {
-            const float v = fmaf(y[k] * inv, f.add_w[k], xs[k]);
-            xs[k] = v;
-            x[k] = v;
-        }
-    } else {
-        for (int k = threadIdx.x; k < n; k += kRouteThreads) xs[k] = x[k];
-    }
-    __syncthreads();
-    const bool vec = (n % 4 == 0) && !((uintptr_t)wr & 15) && !(wsg && ((uintptr_t)wsg & 15));
-    for (int e = wave; e < E + (wsg ? 1 : 0); e += nw) {
-        const float* w = e < E ? wr + (long long)e * n : wsg;
-        float s = 0.0f;
-        if (vec) {
-#pragma unroll 4
-            for (int k = lane * 4; k < n; k += 256) {
-                const float4 a4 = *reinterpret_cast<const float4*>(w + k), x4 = *reinterpret_cast<const float4*>(xs + k);
-                s = fmaf(a4.x, x4.x, s); s = fmaf(a4.y, x4.y, s); s = fmaf(a4.z, x4.z, s); s = fmaf(a4.w, x4.w, s);
-            }
-        } else {
-            for (int k = lane; k < n; k += 64) s = fmaf(w[k], xs[k], s);
-        }
-        s = wave_sum(s);
-        if (lane == 0) {
-            if (e < E) z[e] = s;
-            else if (sgate) sgate[t] = 1.0f / (1.0f + expf(-s));
-        }
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    pick_experts(z, lane, t, E, top, f, ids, wts);
+    route_token<kRouteWaves, 1>(j, blockIdx.x, xs);
 }
 
 // the same picks from logits that a product left: z [T][ldz] = [E router outputs | the shared unit's gate (if sgate)], one wave per token
@@ -348,20 +193,30 @@ int ntk_moe_route_ex(int* ids, float* wts, float* sgate, const float* h, int ldh
     RouteForm f;
     const int st = route_form(r, E, top, &f);
     if (st != NTK_OK || T == 0) return st;
-    hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(kRouteThreads), (size_t)n * 4, resolve_stream(stream), ids, wts, sgate, (float*)h, ldh, w_router, shared_gate_w, n, E, top, f);
+    const RouteJob j{ids, wts, sgate, (float*)h, ldh, w_router, shared_gate_w, n, E, top, f};
+    hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(64 * kRouteWaves), (size_t)n * 4, resolve_stream(stream), j);
     return last_launch_status();
+}
+
+int ntk::norm_route_job(const ntk_norm_route* d, RouteJob* job) {
+    if (!d || !d->ids || !d->wts || !d->h || !d->x || !d->norm_w || !d->w_router || !d->form) return NTK_E_NULL;
+    if (d->T < 0 || d->n <= 0 || d->E <= 0 || d->E > kMaxExperts || d->top <= 0 || d->top > d->E || d->ldh < d->n || d->ldx < d->n || d->form->add_y || d->h == d->x) return NTK_E_SHAPE;
+    if ((size_t)d->n * 4 > 128 * 1024) return NTK_E_SHAPE;
+    RouteForm f;
+    const int st = route_form(d->form, d->E, d->top, &f);
+    if (st != NTK_OK) return st;
+    f.src = d->x; f.ldsrc = d->ldx; f.norm_w = d->norm_w; f.norm_eps = d->norm_eps; f.norm_offset = d->norm_offset;
+    *job = RouteJob{d->ids, d->wts, d->sgate, d->h, d->ldh, d->w_router, d->shared_gate_w, d->n, d->E, d->top, f};
+    return NTK_OK;
 }
 
 int ntk_moe_norm_route(int* ids, float* wts, float* sgate, float* h, int ldh, const float* x, int ldx, const float* norm_w, float norm_eps, float norm_offset, const float* w_router,
                        const float* shared_gate_w, int T, int n, int E, int top, const ntk_route_desc* r, void* stream) {
-    if (!ids || !wts || !h || !x || !norm_w || !w_router || !r) return NTK_E_NULL;
-    if (T < 0 || n <= 0 || E <= 0 || E > kMaxExperts || top <= 0 || top > E || ldh < n || ldx < n || r->add_y || h == x) return NTK_E_SHAPE;
-    if ((size_t)n * 4 > 128 * 1024) return NTK_E_SHAPE;
-    RouteForm f;
-    const int st = route_form(r, E, top, &f);
+    const ntk_norm_route d{ids, wts, sgate, h, ldh, x, ldx, norm_w, norm_eps, norm_offset, w_router, shared_gate_w, T, n, E, top, r};
+    RouteJob j;
+    const int st = norm_route_job(&d, &j);
     if (st != NTK_OK || T == 0) return st;
-    f.src = x; f.ldsrc = ldx; f.norm_w = norm_w; f.norm_eps = norm_eps; f.norm_offset = norm_offset;
-    hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(kRouteThreads), (size_t)n * 4, resolve_stream(stream), ids, wts, sgate, h, ldh, w_router, shared_gate_w, n, E, top, f);
+    hipLaunchKernelGGL(moe_route_kernel, dim3(T), dim3(64 * kRouteWaves), (size_t)n * 4, resolve_stream(stream), j);
     return last_launch_status();
 }
 

@@ -75,6 +75,13 @@ class RouteDesc(C.Structure):
                 ("add_y", C.c_void_p), ("ld_add", C.c_int), ("add_w", C.c_void_p), ("add_eps", C.c_float)]
 
 
+class NormRoute(C.Structure):
+    """ntk_norm_route"""
+    _fields_ = [("ids", C.c_void_p), ("wts", C.c_void_p), ("sgate", C.c_void_p), ("h", C.c_void_p), ("ldh", C.c_int), ("x", C.c_void_p), ("ldx", C.c_int), ("norm_w", C.c_void_p),
+                ("norm_eps", C.c_float), ("norm_offset", C.c_float), ("w_router", C.c_void_p), ("shared_gate_w", C.c_void_p), ("T", C.c_int), ("n", C.c_int), ("E", C.c_int), ("top", C.c_int),
+                ("form", C.POINTER(RouteDesc))]
+
+
 class MoeFewDesc(C.Structure):
     _fields_ = [("out", C.c_void_p), ("ldo", C.c_int), ("h", C.c_void_p), ("ldh", C.c_int), ("ids", C.c_void_p), ("wts", C.c_void_p), ("top", C.c_int), ("experts", C.c_int),
                 ("up", C.c_void_p), ("down", C.c_void_p), ("ff", C.c_int), ("shared_up", C.c_void_p), ("shared_down", C.c_void_p), ("shared_ff", C.c_int), ("sgate", C.c_void_p),

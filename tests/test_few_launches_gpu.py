@@ -135,3 +135,40 @@ def test_router_of_a_row_normed_in_its_launch(T, n, E, top):
     assert np.array_equal(out[0][0], out[1][0])
     for a, b in zip(out[0][1:], out[1][1:]):
         assert np.isfinite(b).all() and np.abs(a - b).max() <= 2e-5 * np.abs(a).max()      # (logits of up to 5000 products behind a norm whose sum has another order)
+
+
+@pytest.mark.parametrize("T,H,R,dr,pos0,n,E,top", [(1, 16, 512, 64, 1100, 2048, 32, 6), (8, 1, 512, 64, 300, 2052, 33, 4), (3, 16, 512, 304, 20, 4096, 256, 8), (2, 5, 328, 8, 9, 70, 5, 5),
+                                                 (1, 16, 512, 64, 40, 5000, 32, 6), (2, 4, 256, 32, 90, 512, 12, 3), (1, 4, 330, 6, 90, 512, 12, 3)])
+def test_router_beside_attention(T, H, R, dr, pos0, n, E, top):
+    """the last three: rows too long for that launch, attention of four waves, keys off 16 bytes -- the router's own launch"""
+    L, g = Lr._bind(), np.random.default_rng(n + R)
+    L.ntk_latent_attention_unfold.argtypes = [VP, I, VP, I, VP] + [I] * 3 + [VP, VP, VP] + [I] * 7 + [F, VP, VP]
+    L.ntk_latent_attention_unfold_route.argtypes = [VP, I, VP, I, VP] + [I] * 3 + [VP, VP, VP] + [I] * 7 + [F, VP, VP, VP]
+    L.ntk_moe_norm_route.argtypes = [VP, VP, VP, VP, I, VP, I, VP, F, F, VP, VP] + [I] * 4 + [C.POINTER(Lr.RouteDesc), VP]
+    row, dv = R + dr, 24
+    qf, cache = (DB.from_numpy(g.standard_normal(s).astype(np.float32)) for s in ((T, H * row), (pos0 + T, row)))
+    w, wd = weights(g, (H * dv, R), "bf16")
+    L.ntk_latent_attention_scratch.restype = C.c_size_t
+    scr = DB.zeros(int(L.ntk_latent_attention_scratch(T, H, R, pos0 + T)) * 4)
+    lat = DB.zeros(T * H * R * 4)
+    x = DB.from_numpy((3 * g.standard_normal((T, n))).astype(np.float32))
+    nw, wr, ws = (DB.from_numpy((0.2 * g.standard_normal(s)).astype(np.float32)) for s in (n, (E, n), n))
+    form = Lr.RouteDesc()
+    form.score, form.groups, form.renorm, form.scale = 0, 1, 1, 1.0
+    out = []
+    for one in (0, 1):
+        o, h, ids, wts, sg = DB.zeros(T * H * dv * 4), DB.zeros(T * n * 4), DB.zeros(T * top * 4), DB.zeros(T * top * 4), DB.zeros(T * 4)
+        att = (o.ptr, H * dv, w.ptr, wd, None, 0, 0, dv, lat.ptr, qf.ptr, cache.ptr, row, R, dr, H, pos0, T, 0, 0.05, scr.ptr)
+        if one:
+            r = Lr.NormRoute(ids.ptr, wts.ptr, sg.ptr, h.ptr, n, x.ptr, n, nw.ptr, 1e-5, 1.0, wr.ptr, ws.ptr, T, n, E, top, C.pointer(form))
+            Lr.check(L.ntk_latent_attention_unfold_route(*att, C.byref(r), None), "beside")
+        else:
+            Lr.check(L.ntk_latent_attention_unfold(*att, None), "unfold")
+            Lr.check(L.ntk_moe_norm_route(ids.ptr, wts.ptr, sg.ptr, h.ptr, n, x.ptr, n, nw.ptr, 1e-5, 1.0, wr.ptr, ws.ptr, T, n, E, top, C.byref(form), None), "route")
+        out.append((o.numpy(np.float32), ids.numpy(np.int32)[:T * top], h.numpy(np.float32)[:T * n], wts.numpy(np.float32)[:T * top], sg.numpy(np.float32)[:T]))
+    for a, b in zip(out[0][:2], out[1][:2]):
+        assert np.array_equal(a, b)
+    for a, b in zip(out[0][2:], out[1][2:]):
+        assert np.isfinite(b).all() and np.abs(a - b).max() <= 2e-5 * np.abs(a).max()      # (a norm whose sum is of eight waves' parts instead of sixteen in front of up to 4096 products)
+    r.top = E + 1
+    assert L.ntk_latent_attention_unfold_route(*att, C.byref(r), None) != 0
