@@ -140,7 +140,7 @@ __global__ __launch_bounds__(1024) void half_norm_split_kernel(const HalfNormArg
 // two matrix instructions a product: constants as for bf16 (plan_direct), from 16 .. 200 rows, 1024 .. 28672 outputs, 4096 .. 14336 inputs
 static TilePlan plan_direct_half(int rows, int N, int K, long long room) {
     static const DirectForm forms[] = {{128, 256, 1, 1.65f, 1.65f, 12.0f, 0.6f}, {64, 128, 2, 0.82f, 0.495f, 5.0f, 0.0f}, {64, 64, 2, 0.47f, 0.315f, 4.0f, 0.0f}};
-    return plan_direct(forms, 3, 64, rows, 1, N, K, room);
+    return plan_direct(forms, 3, 64, rows, 1, N, K, room, true);
 }
 template <int GLU>
 static int launch_direct_half(const DirectArgs& d, const TilePlan& p, hipStream_t s, bool sum = true) {

@@ -87,6 +87,15 @@ def test_rows_shared_evenly_over_tiles(T):
     assert (np.abs(y - g * s * u) <= 1.1 * bg * (np.abs(u) + bu) + np.abs(g * s) * bu + 16 * U * np.abs(g * s * u) + 1e-37).all()
 
 
+@pytest.mark.parametrize("T,K,outs", [(256, 4096, (4096, 1024, 1024)), (150, 2048, (2048,)), (70, 4160, (6100, 33, 10))])
+def test_five_pieces_of_k(T, K, outs):
+    """128 x 256, 64 x 64 and 64 x 128 tiles in five pieces, the last of them shorter (64, 32 and 65 chunks)"""
+    x, ws = values(T, K, outs, T + K)
+    for y, w in zip(run(x, ws, room=16 * T * sum(outs)), ws):
+        want, bound = product(x, w)
+        assert (np.abs(y - want) <= bound).all()
+
+
 def test_a_row_that_is_not_finite_and_what_is_refused():
     x, ws = values(20, 128, (70, 70), 3)
     x[4, 9], x[6, 1] = np.nan, np.inf
