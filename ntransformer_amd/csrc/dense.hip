@@ -724,7 +724,15 @@ constexpr float kRoundUs = 3.5f, kRoundRate = 4e6f;     // the launch that round
 static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long room) {
     static const DirectForm forms[] = {{256, 256, 1, 1.45f, 1.45f, 12.0f}, {256, 128, 1, 0.84f, 0.84f, 9.0f}, {128, 256, 1, 0.85f, 0.85f, 9.0f}, {128, 128, 2, 0.72f, 0.475f, 7.0f},
                                        {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
-    return plan_direct(forms, 7, 64, rows, groups, N, K, room);
+    TilePlan p = plan_direct(forms, 7, 64, rows, groups, N, K, room);
+    // One matrix: which tile and how many pieces with the last round of tiles on a CU at its own pace (p.us stays the estimate that the lines between this and the other forms were drawn with).
+    // us: 150 x 2048 x 2048 13.6 -> 11.6, 700 x 4096 x 14336 97 -> 88, 1500 x 4096 x 14336 229 -> 179, 65 x 6240 x 2048 15.5 -> 14.7; of 380 sizes of 9 .. 2200 rows 1.00
+    // on average (most plans stay), none of those whose plan changes behind by more than 2 %.
+    if (groups == 1) {
+        const TilePlan q = plan_direct(forms, 7, 64, rows, 1, N, K, room, true);
+        p.form = q.form; p.splits = q.splits;
+    }
+    return p;
 }
 // float32: K in chunks of 32; one form, ahead of larger and smaller tiles and other splits of the tile over waves at the sizes they were tried at (12 .. 200 rows, 900 in 32 groups).  Over 337
 // grouped sizes it takes 0.89 of gemm_tile.hip.h's time on average and is 3 .. 17 % behind it at about eleven (40 rows in 128 groups, 300 in 8 or 16).  us, the form of gemm_tile.hip.h

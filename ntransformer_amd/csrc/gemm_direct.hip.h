@@ -288,8 +288,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 // that come from memory; the estimate is within a sixth there, and the choice within a tenth of the best form but for uneven small groups.  Rows of several groups: tiles
 // of a group of the average size, plus half a tile where that is no small part of one.
 struct DirectForm { int TM, TN, resident; float alone, busy, over, even; };       // even: the part of a chunk's time that goes with the rows a tile has (rows evenly over the tiles)
-// rounds: a CU whose tiles are no whole number of `resident` ones has the rest at the pace of a tile alone, and five pieces are looked at too.  The two-piece products' constants were
-// fitted so; those of one piece stand without.  us before / so (halves of 32-bit activations, with their split and the sum): 200 x 6144 x 4096 46.8 / 39.8 (768 tiles of 64 x 128 on 512 places
+// rounds: a CU whose tiles are no whole number of `resident` ones has the rest at the pace of a tile alone, and five pieces are looked at too where six put a second tile on a CU (126 x 512 x
+// 2048 in bf16: 8.3 in six, 8.9 in five).  us before / so (halves of 32-bit activations, with their split and the sum): 200 x 6144 x 4096 46.8 / 39.8 (768 tiles of 64 x 128 on 512 places
 // / 240 of 128 x 256 in five pieces), 256 52.9 / 43.2, 160 x 4096 x 4096 28.7 / 27.4; of 152 sizes the 12 whose plan changes are 0.8 .. 1.02 of the time before.
 static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats, bool rounds = false) {
     static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
@@ -301,7 +301,7 @@ static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int row
         const float tiles = row_tiles * ((N + f[i].TN - 1) / f[i].TN);
         for (int s : counts) {
             if (s > 1 && ((long long)s * rows * N > scratch_floats || chunks < 4 * s)) break;
-            if (s == 5 && !rounds) continue;
+            if (s == 5 && (!rounds || tiles * 6.0f <= 256.0f)) continue;
             const int n = (int)((tiles * s + 255.0f) / 256.0f);
             const float full = 1.0f - f[i].even * (1.0f - std::min(1.0f, mean / row_tiles));
             const int rest = rounds ? n % f[i].resident : n == 1 ? 1 : 0;

@@ -43,6 +43,14 @@ def test_direct_products(T, N, K):
         _close(Lr.dense_direct(x, w, out16=True, act=1), x, w, lambda r, b: (np.maximum(r, 0) ** 2, 2 * np.abs(r) * b + b * b), bf=True)
 
 
+@pytest.mark.parametrize("T,N,K", [(212, 1536, 2048), (150, 4096, 4096), (500, 3072, 4096)])
+def test_five_pieces_of_k(T, N, K):
+    """plans of five pieces (64 x 64, 64 x 128 and 128 x 128 tiles): chunks of 64 that they do not share evenly (32 and 64)"""
+    from ntransformer_amd import layers as Lr
+    x, w = _case(np.random.default_rng(T), T, N, K)
+    _close(Lr.dense_direct(x, w, scratch_floats=16 * T * N), x, w, lambda r, b: (r, 2 * b))
+
+
 @pytest.mark.parametrize("T,ff,K", [(9, 8, 64), (65, 33, 128), (200, 129, 256), (257, 448, 64), (1030, 3111, 64), (1024, 8200, 64)])
 @pytest.mark.parametrize("limit,alpha,up,cubic", [(7.0, 1.702, 1.0, 0.0), (float("inf"), 1.0, 0.0, 0.0), (float("inf"), 1.5957691, 0.0, 0.044715)])
 def test_gated_units_inside_the_product(T, ff, K, limit, alpha, up, cubic):
