@@ -705,15 +705,23 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
     float* up_buf = gate_buf + (size_t)T * I;
     void* ws = gemm_ws_;
     auto other = [&]() { ws = ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_; return ws; };
-    auto gemm = [&](const DevTensor* const* Ws, float* const* Ys, int n, const float* resid, bool normed, size_t part_at, ntk_gemm_partials* pt) {
+    auto repacked = [&](const DevTensor* const* Ws, int n) {
         bool rp = true;
         for (int i = 0; i < n; ++i) rp = rp && !Ws[i]->ptr && Ws[i]->rp && Ws[i]->dtype != NTK_DT_Q8_0 && Ws[i]->dtype != NTK_DT_Q4_0;
-        if (!rp) raw_begin();
-        ntk_gemv_seg segs[3];
+        return rp;
+    };
+    auto describe = [&](const DevTensor* const* Ws, float* const* Ys, int n, const float* resid, ntk_gemm_partials* pt, bool rp, ntk_gemv_seg (&segs)[3]) {
         for (int i = 0; i < n; ++i) segs[i] = {rp ? Ws[i]->rp : raw_of(*Ws[i]), Ys[i], (int)Ws[i]->out_f, Ws[i]->dtype};
         ntk_gemm_desc d{};
         d.segs = segs; d.nseg = n; d.n_tokens = T; d.in_features = (int)Ws[0]->in_f; d.resid = resid;
         d.workspace = ws; d.workspace_bytes = gemm_ws_bytes_; d.partials = pt; d.weights_repacked = rp ? 1 : 0;
+        return d;
+    };
+    auto gemm = [&](const DevTensor* const* Ws, float* const* Ys, int n, const float* resid, bool normed, size_t part_at, ntk_gemm_partials* pt) {
+        const bool rp = repacked(Ws, n);
+        if (!rp) raw_begin();
+        ntk_gemv_seg segs[3];
+        const ntk_gemm_desc d = describe(Ws, Ys, n, resid, pt, rp, segs);
         return ntk_gemm_short(&d, normed ? 1 : 0, cfg_.norm_eps, part_at, s);
     };
     NT_TRY(ntk_short_norm_prepare_x(hidden_, nullptr, (const float*)layers_[first].attn_norm.ptr, T, H, ws, s));
@@ -730,22 +738,34 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
         // from the prompt's first token on: everything between the projections in one launch
         const bool whole = start_pos == 0 && hd == 128 && nh % 2 == 0 && rope_angles_ != nullptr;
         const bool defer = whole || (T >= 4 && hd <= 256);   // (the prompt form of the rotation: ntk_rope takes it from 4 tokens on, too; wider heads are turned in place)
+        // (one launch a format; two formats together)
+        struct Of { const DevTensor* w[3]; float* y[3]; int idx[3], n = 0; ntk_gemm_partials pt; } of[3];
+        int kinds = 0;
         for (int a = 0; a < 3; ++a) {
             if (done[a]) continue;
-            const DevTensor* w[3];
-            float* y[3];
-            int idx[3], n = 0;
+            Of& o = of[kinds++];
             for (int b = a; b < 3; ++b)
-                if (qkv[b]->dtype == qkv[a]->dtype) { w[n] = qkv[b]; y[n] = ys[b]; idx[n++] = b; done[b] = true; }
-            ntk_gemm_partials pt;
-            NT_TRY(gemm(w, y, n, nullptr, true, at, defer ? &pt : nullptr));
-            if (defer && pt.nsplit > 1)
-                for (int k = 0; k < n; ++k) {
-                    sums[idx[k]] = pt.part[k];
-                    splits[idx[k]] = pt.nsplit;
-                    at += (size_t)pt.nsplit * T * w[k]->out_f;
-                }
+                if (qkv[b]->dtype == qkv[a]->dtype) { o.w[o.n] = qkv[b]; o.y[o.n] = ys[b]; o.idx[o.n++] = b; done[b] = true; }
         }
+        auto leaves = [&](const Of& o) {
+            if (!defer || o.pt.nsplit <= 1) return;
+            for (int k = 0; k < o.n; ++k) {
+                sums[o.idx[k]] = o.pt.part[k];
+                splits[o.idx[k]] = o.pt.nsplit;
+                at += (size_t)o.pt.nsplit * T * o.w[k]->out_f;
+            }
+        };
+        if (kinds == 2 && defer && repacked(of[0].w, of[0].n) && repacked(of[1].w, of[1].n)) {
+            ntk_gemv_seg sa[3], sb[3];
+            const ntk_gemm_desc da = describe(of[0].w, of[0].y, of[0].n, nullptr, &of[0].pt, true, sa), db = describe(of[1].w, of[1].y, of[1].n, nullptr, &of[1].pt, true, sb);
+            NT_TRY(ntk_gemm_short_two(&da, &db, 1, cfg_.norm_eps, 0, s));
+            leaves(of[0]);
+            leaves(of[1]);
+        } else
+            for (int a = 0; a < kinds; ++a) {
+                NT_TRY(gemm(of[a].w, of[a].y, of[a].n, nullptr, true, at, defer ? &of[a].pt : nullptr));
+                leaves(of[a]);
+            }
         if (whole) {
             NT_TRY(ntk_short_attention(sums, splits, rope_angles_, T, nh, nkv, hd, scale, cfg_.rope_interleaved, kc, vc, cfg_.max_seq_len, other(), s));
         } else if (defer) {

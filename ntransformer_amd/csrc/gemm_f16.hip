@@ -2410,6 +2410,26 @@ static int short_takes(const int* rows, int nseg, int T, int in) {
     return kslice_plan<DT>(rows, nseg, T, in).n > 0;
 }
 
+// gemm_short.hip's launch over the planes of workspace wsb; parts: where each matrix's sums of slices lie
+template <int DT>
+static void stream_params(ShortStreamParams* q, const HostSeg* segs, int nseg, int T, int in, const ShortStreamPlan& sp, uint8_t* wsb, const ShortArgs& sh, const float* resid, const float** parts) {
+    float* group_inv = reinterpret_cast<float*>(wsb + ws_group_offset(in));
+    q->nseg = nseg; q->T = T; q->in = in; q->units = in / 256;
+    q->xb = wsb; q->aux = wsb + (size_t)(in / 32 + 1) * GB_STEP_BYTES; q->group_inv = group_inv;
+    if (sh.norm) { q->ssq = group_inv + ws_group_floats(in); q->nssq = (in + 511) / 512; q->eps = sh.eps; }
+    q->ups = sp.ups; q->groups = sp.groups; q->resid = sp.n == 1 ? resid : nullptr;
+    float* part = reinterpret_cast<float*>(wsb + ws_part_offset(in)) + sh.part_at;
+    int tile = 0;
+    for (int i = 0; i < nseg; ++i) {
+        q->seg[i] = ShortStreamSeg{static_cast<const uint8_t*>(segs[i].W), segs[i].Y, part, segs[i].out, tile,
+                                   (uint32_t)((size_t)(segs[i].out / 16) * (size_t)q->units * (size_t)(2 * DeqI<DT>::S1))};
+        parts[i] = part;
+        tile += segs[i].out / 16;
+        part += (size_t)sp.n * T * segs[i].out;
+    }
+    q->tiles = tile;
+}
+
 // T <= GB_MAX_CHUNKS * 64 = 1024 tokens in one launch; nseg matrices [out_s][in] of one format sharing X
 template <int DT>
 static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T, int in, const float* resid, void* ws, int reuse_x,
@@ -2460,20 +2480,8 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
         const ShortStreamPlan sp = sh.on && T <= SS_TOKENS ? short_stream_plan(DT - GB_RP, in / 256, (int)(out_total / 16), plan.n, plan.jobs * plan.ups * KD::SPU * plan.rt) : ShortStreamPlan{};
         if (sp.n > 0) {
             ShortStreamParams q{};
-            q.nseg = nseg; q.T = T; q.in = in; q.units = in / 256; q.tiles = (int)(out_total / 16);
-            q.xb = wsb; q.aux = reinterpret_cast<const uint8_t*>(p.aux); q.group_inv = group_inv;
-            if (sh.norm) { q.ssq = group_inv + ws_group_floats(in); q.nssq = (in + 511) / 512; q.eps = sh.eps; }
-            q.ups = sp.ups; q.groups = sp.groups; q.resid = sp.n == 1 ? resid : nullptr;
-            float* part = reinterpret_cast<float*>(wsb + ws_part_offset(in)) + sh.part_at;
             const float* parts[GB_MAX_SEG] = {};
-            int tile = 0;
-            for (int i = 0; i < nseg; ++i) {
-                q.seg[i] = ShortStreamSeg{static_cast<const uint8_t*>(segs[i].W), segs[i].Y, part, segs[i].out, tile,
-                                          (uint32_t)((size_t)(segs[i].out / 16) * (size_t)q.units * (size_t)(2 * D::S1))};
-                parts[i] = part;
-                tile += segs[i].out / 16;
-                part += (size_t)sp.n * T * segs[i].out;
-            }
+            stream_params<DT>(&q, segs, nseg, T, in, sp, wsb, sh, resid, parts);
             const int rc = short_stream_launch(DT - GB_RP, q, sp, st);
             return rc == NTK_OK ? leave_slices(segs, nseg, parts, sp.n, T, resid, defer, st) : rc;
         }
@@ -2816,6 +2824,82 @@ int ntk_gemm_short(const ntk_gemm_desc* d, int normed, float eps, size_t part_at
     e.reuse_x = 1;
     if (!e.X) e.X = static_cast<const float*>(e.workspace);   // (never read)
     return gemm_quant_f16_with(&e, sh, stream);
+}
+// ---- matrices of two formats over the same planes ----
+extern "C++" { namespace {
+// one side of such a launch: what launch_gemm_f16 asks of it, and what it would take by itself
+struct PairSide { ntk::HostSeg segs[ntk::GB_MAX_SEG]; int nseg, dt, rows; ntk::KSlicePlan lds; float us; };
+template <int DT>
+bool pair_side(const ntk_gemm_desc* d, PairSide* o) {
+    int outs[ntk::GB_MAX_SEG];
+    o->rows = 0;
+    for (int i = 0; i < d->nseg; ++i) {
+        const ntk_gemv_seg& g = d->segs[i];
+        if (!g.W || !g.y || g.dtype != DT || g.rows <= 0 || g.rows % 16 || ((reinterpret_cast<uintptr_t>(g.W) | reinterpret_cast<uintptr_t>(g.y)) & 15)) return false;
+        if (!ntk::offsets_fit<ntk::DeqI<DT + ntk::GB_RP>>(g.rows, d->in_features)) return false;
+        o->segs[i] = ntk::HostSeg{g.y, g.W, g.rows};
+        outs[i] = g.rows;
+        o->rows += g.rows;
+    }
+    o->nseg = d->nseg; o->dt = DT;
+    o->lds = ntk::kslice_plan<DT + ntk::GB_RP>(outs, d->nseg, d->n_tokens, d->in_features);
+    if (o->lds.n == 0) return false;
+    o->us = ntk::short_stream_plan(DT, d->in_features / 256, o->rows / 16, o->lds.n, o->lds.jobs * o->lds.ups * ntk::DeqI<DT + ntk::GB_RP>::SPU * o->lds.rt).us;
+    return true;
+}
+bool pair_side(const ntk_gemm_desc* d, PairSide* o) {
+    switch (d->segs[0].dtype) {
+        case NTK_DT_Q4_K: return pair_side<NTK_DT_Q4_K>(d, o);
+        case NTK_DT_Q5_K: return pair_side<NTK_DT_Q5_K>(d, o);
+        case NTK_DT_Q6_K: return pair_side<NTK_DT_Q6_K>(d, o);
+        default: return false;
+    }
+}
+void pair_params(const PairSide& o, ntk::ShortStreamParams* q, int T, int in, const ntk::ShortStreamPlan& sp, uint8_t* ws, const ntk::ShortArgs& sh, const float** parts) {
+    if (o.dt == NTK_DT_Q4_K) ntk::stream_params<NTK_DT_Q4_K + ntk::GB_RP>(q, o.segs, o.nseg, T, in, sp, ws, sh, nullptr, parts);
+    else if (o.dt == NTK_DT_Q5_K) ntk::stream_params<NTK_DT_Q5_K + ntk::GB_RP>(q, o.segs, o.nseg, T, in, sp, ws, sh, nullptr, parts);
+    else ntk::stream_params<NTK_DT_Q6_K + ntk::GB_RP>(q, o.segs, o.nseg, T, in, sp, ws, sh, nullptr, parts);
+}
+} }  // namespace
+// floats of partial sums that a launch has left
+static size_t left_behind(const ntk_gemm_partials* p) {
+    size_t n = 0;
+    if (p && p->nsplit > 1)
+        for (int i = 0; i < p->nseg; ++i) n += (size_t)p->nsplit * p->n_tokens * p->rows[i];
+    return n;
+}
+int ntk_gemm_short_two(const ntk_gemm_desc* a, const ntk_gemm_desc* b, int normed, float eps, size_t part_at, void* stream) {
+    if (!a || !b) return NTK_E_NULL;
+    const int T = a->n_tokens, in = a->in_features;
+    const bool like = a->segs && b->segs && a->nseg >= 1 && b->nseg >= 1 && a->nseg <= ntk::GB_MAX_SEG && b->nseg <= ntk::GB_MAX_SEG && a->weights_repacked && b->weights_repacked && a->partials &&
+                      b->partials && !a->resid && !b->resid && a->workspace && a->workspace == b->workspace && a->workspace_bytes == b->workspace_bytes && b->n_tokens == T && b->in_features == in &&
+                      T >= 2 && T <= ntk::SS_TOKENS && in > 0 && in % 256 == 0 && part_at % 4 == 0 && !(reinterpret_cast<uintptr_t>(a->workspace) & 15);
+    PairSide sa, sb;
+    if (like && pair_side(a, &sa) && pair_side(b, &sb) && sa.dt != sb.dt) {
+        const bool turned = sa.dt > sb.dt;
+        PairSide &lo = turned ? sb : sa, &hi = turned ? sa : sb;
+        ntk::ShortStreamPlan plo, phi;
+        const size_t head = ntk::ws_part_offset((in + 31) / 32 * 32), cap = a->workspace_bytes > head ? (a->workspace_bytes - head) / sizeof(float) : 0;
+        if (a->workspace_bytes >= ntk_gemm_quant_workspace_bytes(in, sa.rows + sb.rows) &&
+            ntk::short_stream_plan_two(lo.dt, hi.dt, in / 256, lo.rows / 16, hi.rows / 16, std::min(lo.lds.n, hi.lds.n), lo.us + hi.us, &plo, &phi) &&
+            part_at + (size_t)plo.n * T * (size_t)(sa.rows + sb.rows) <= cap) {
+            ntk::ShortArgs sh;
+            sh.on = true; sh.norm = normed != 0; sh.eps = eps; sh.part_at = part_at; sh.part_cap = cap;
+            ntk::ShortStreamParams q[2] = {};
+            const float* parts[2][ntk::GB_MAX_SEG] = {};
+            uint8_t* ws = static_cast<uint8_t*>(a->workspace);
+            pair_params(lo, &q[0], T, in, plo, ws, sh, parts[0]);
+            if (plo.n > 1) sh.part_at += (size_t)plo.n * T * (size_t)lo.rows;
+            pair_params(hi, &q[1], T, in, phi, ws, sh, parts[1]);
+            hipStream_t st = ntk::resolve_stream(stream);
+            const int rc = ntk::short_stream_launch_two(lo.dt, hi.dt, q[0], q[1], plo, phi, st);
+            if (rc != NTK_OK) return rc;
+            ntk::leave_slices(lo.segs, lo.nseg, parts[0], plo.n, T, nullptr, (turned ? b : a)->partials, st);
+            return ntk::leave_slices(hi.segs, hi.nseg, parts[1], phi.n, T, nullptr, (turned ? a : b)->partials, st);
+        }
+    }
+    const int rc = ntk_gemm_short(a, normed, eps, part_at, stream);
+    return rc != NTK_OK ? rc : ntk_gemm_short(b, normed, eps, part_at + left_behind(a->partials), stream);
 }
 static int short_check(int T, int in, const void* workspace, uintptr_t ptrs) {
     if (!workspace) return NTK_E_NULL;

@@ -38,18 +38,18 @@ __device__ __forceinline__ void ss_turn(uint32_t (&r)[4]) {
     r[0] = c[0]; r[1] = c[1]; r[2] = d[0]; r[3] = d[1];
 }
 
-// Workgroup (x, slice): eight waves, wave = (row group wave / ups, unit slice * ups + wave % ups of 256 columns), tiles (x + k gridDim.x) * groups + row group for k = 0, 1, ...
+// Workgroup (x, slice): eight waves, wave = (row group wave / ups, unit slice * ups + wave % ups of 256 columns), tiles (x + k wgx) * groups + row group for k = 0, 1, ...
+typedef f32x4 SsSums[SS_AHEAD * SS_WAVES][64];
 template <int DT>
-__global__ __launch_bounds__(64 * SS_WAVES, 2) void short_stream_kernel(const ShortStreamParams p) {
+__device__ __forceinline__ void short_stream(const ShortStreamParams& p, const int bx, const int slice, const int wgx, const int slices, SsSums (&sums)[2]) {
     using R = Sp<DT>;
     constexpr bool FOLD = DT != NTK_DT_Q6_K;
     constexpr int ITEM1 = 2 * R::S1;
-    __shared__ __attribute__((aligned(16))) f32x4 sums[2][SS_AHEAD * SS_WAVES][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), i = lane & 15, g = lane >> 4;
-    const int grp = wave / p.ups, first = (int)blockIdx.y * p.ups, here = min(p.ups, p.units - first);         // the slice's units
+    const int grp = wave / p.ups, first = slice * p.ups, here = min(p.ups, p.units - first);         // the slice's units
     const int u = min(first + wave % p.ups, p.units - 1);
     const bool works = grp < p.groups && wave % p.ups < here;
-    const int stride = (int)gridDim.x * p.groups, turns = (p.tiles + stride - 1) / stride, tile0 = (int)blockIdx.x * p.groups + grp;
+    const int stride = wgx * p.groups, turns = (p.tiles + stride - 1) / stride, tile0 = bx * p.groups + grp;
 
     // 1 / rms of the lane's tokens (4 g + e): the parts of the rows' sums of squares are asked for first, added up behind the other requests
     f32x4 part[8];
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(64 * SS_WAVES, 2) void short_stream_kernel(const Sh
         return y * ginv;
     };
     for (int k0 = 0; k0 < turns; k0 += SS_AHEAD) {
-        f32x4 (&buf)[SS_AHEAD * SS_WAVES][64] = sums[(k0 / SS_AHEAD) & 1];
+        SsSums& buf = sums[(k0 / SS_AHEAD) & 1];
         if (works)
 #pragma unroll
             for (int a = 0; a < SS_AHEAD; ++a) {
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * SS_WAVES, 2) void short_stream_kernel(const Sh
             }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");       // (the requests stay under way; the other buffer's sums were read in front of this)
         for (int l = wave; l < SS_AHEAD * p.groups; l += SS_WAVES) {
-            const int a = l / p.groups, gr = l - a * p.groups, tile = ((int)blockIdx.x + (k0 + a) * (int)gridDim.x) * p.groups + gr;
+            const int a = l / p.groups, gr = l - a * p.groups, tile = (bx + (k0 + a) * wgx) * p.groups + gr;
             if (k0 + a >= turns || tile >= p.tiles) continue;
             f32x4 y = buf[a * SS_WAVES + gr * p.ups][lane];
             for (int w = 1; w < here; ++w) y += buf[a * SS_WAVES + gr * p.ups + w][lane];
@@ -247,20 +247,35 @@ __global__ __launch_bounds__(64 * SS_WAVES, 2) void short_stream_kernel(const Sh
                 const int t = 4 * g + e;
                 if (t >= p.T) continue;
                 const float v = y[e] * rms[e];
-                if (gridDim.y > 1) p.seg[sg].part[((size_t)blockIdx.y * p.T + t) * out + r] = v;
+                if (slices > 1) p.seg[sg].part[((size_t)slice * p.T + t) * out + r] = v;
                 else { const size_t at = (size_t)t * out + r; p.seg[sg].Y[at] = p.resid ? v + p.resid[at] : v; }
             }
         }
     }
 }
 
+template <int DT>
+__global__ __launch_bounds__(64 * SS_WAVES, 2) void short_stream_kernel(const ShortStreamParams p) {
+    __shared__ __attribute__((aligned(16))) SsSums sums[2];
+    short_stream<DT>(p, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, sums);
+}
+
+// matrices of two formats over the same planes (a K-quant mix keeps more bits of some): a.wgx columns of workgroups have the first format's, the others the second's
+template <int DA, int DB>
+__global__ __launch_bounds__(64 * SS_WAVES, 2) void short_stream_two_kernel(const ShortStreamParams a, const ShortStreamParams b, const int wgx) {
+    __shared__ __attribute__((aligned(16))) SsSums sums[2];
+    if ((int)blockIdx.x < wgx) short_stream<DA>(a, blockIdx.x, blockIdx.y, wgx, gridDim.y, sums);
+    else short_stream<DB>(b, (int)blockIdx.x - wgx, blockIdx.y, (int)gridDim.x - wgx, gridDim.y, sums);
+}
+
 // Turns (tiles a wave takes) decide: the chip's 256 workgroups are there at once.  us of a launch, this form / the one with its planes in LDS, 16 tokens: gate | up of 28672 x 4096 (14 turns, two slices) Q4_K
 // 21.0 / 26.4, Q5_K 25.0 / 29.5, Q6_K 28.0 / 34.8; 57344 x 8192 (56 turns) 60 / 83, 93 / 97, 95 / 117; 8192 x 28672 (29) 36 / 42, 50 / 50, 53 / 60; Q | K | V of 4096 columns (3) 9.6 / 10.6, 10.8 / 11.9, 11.6 / 12.3;
 // behind it: 4096 x 4096 (2) 8.5 / 7.2, 9.3 / 8.3, 9.8 / 8.5, 4096 x 14336 (8) 14.6 / 13.2, 17.3 / 14.8, 18.7 / 17.0, 1024 x 4096 (1) 9 / 6.9 -- a wave reads 16 KB of planes before its first
 // product.  `other`: steps of 32 columns a wave of that form takes one after the other.
+static float turn_us(int dt) { return dt == NTK_DT_Q4_K ? 1.03f : dt == NTK_DT_Q5_K ? 1.3f : 1.54f; }
 ShortStreamPlan short_stream_plan(int dt, int units, int tiles, int most, int other) {
     ShortStreamPlan b;
-    const float turn = dt == NTK_DT_Q4_K ? 1.03f : dt == NTK_DT_Q5_K ? 1.3f : 1.54f, step = dt == NTK_DT_Q4_K ? 0.15f : dt == NTK_DT_Q5_K ? 0.17f : 0.22f;
+    const float turn = turn_us(dt), step = dt == NTK_DT_Q4_K ? 0.15f : dt == NTK_DT_Q5_K ? 0.17f : 0.22f;
     float best = 5.0f + step * (float)other;
     for (int ups = 1; ups <= std::min(units, SS_WAVES); ++ups) {
         const int n = (units + ups - 1) / ups, groups = SS_WAVES / ups;
@@ -269,7 +284,31 @@ ShortStreamPlan short_stream_plan(int dt, int units, int tiles, int most, int ot
         const float us = 6.3f + turn * (float)turns + 0.1f * (float)n;
         if (us < best) { best = us; b.n = n; b.ups = ups; b.groups = groups; b.wgx = wgx; }
     }
+    b.us = best;
     return b;
+}
+
+// Two formats in one launch: the chip's workgroups shared so that the one that ends last ends as early as can be.  Against two launches (apart: their estimates) what is saved is mostly the second
+// one's way to its first product: us, 16 tokens, 5120 rows in Q4_K and 1024 in Q6_K, 4096 columns: 10.4 + 6.8 -> 12.0; short prompts through eight 8B-shaped layers in Q4_K_M 673 -> 645 (2 tokens),
+// 735 -> 709 (16), eight 70B-shaped ones (Q4_K and Q5_K or Q6_K) 1389 -> 1347, 1534 -> 1469, four of 1024 columns 236 -> 233.
+bool short_stream_plan_two(int da, int db, int units, int tiles_a, int tiles_b, int most, float apart, ShortStreamPlan* a, ShortStreamPlan* b) {
+    float best = apart;
+    bool found = false;
+    for (int ups = 1; ups <= std::min(units, SS_WAVES); ++ups) {
+        const int n = (units + ups - 1) / ups, groups = SS_WAVES / ups;
+        if (n > most || n > 128 || (units + n - 1) / n != ups) continue;
+        const int room = 256 / n;
+        for (int wa = 1; wa < room; ++wa) {
+            const int wb = room - wa, ta = (tiles_a + wa * groups - 1) / (wa * groups), tb = (tiles_b + wb * groups - 1) / (wb * groups);
+            const float us = 6.8f + std::max(turn_us(da) * (float)ta, turn_us(db) * (float)tb) + 0.1f * (float)n;
+            if (us >= best) continue;
+            best = us;
+            found = true;
+            *a = *b = ShortStreamPlan{n, ups, groups, std::min(wa, (tiles_a + groups - 1) / groups), us};
+            b->wgx = std::min(wb, (tiles_b + groups - 1) / groups);
+        }
+    }
+    return found;
 }
 
 int short_stream_launch(int dt, const ShortStreamParams& p, const ShortStreamPlan& plan, hipStream_t st) {
@@ -280,6 +319,15 @@ int short_stream_launch(int dt, const ShortStreamParams& p, const ShortStreamPla
         case NTK_DT_Q6_K: hipLaunchKernelGGL(short_stream_kernel<NTK_DT_Q6_K>, grid, block, 0, st, p); break;
         default: return NTK_E_DTYPE;
     }
+    return last_launch_status();
+}
+
+int short_stream_launch_two(int da, int db, const ShortStreamParams& a, const ShortStreamParams& b, const ShortStreamPlan& pa, const ShortStreamPlan& pb, hipStream_t st) {
+    const dim3 grid(pa.wgx + pb.wgx, pa.n), block(64 * SS_WAVES);
+    if (da == NTK_DT_Q4_K && db == NTK_DT_Q5_K) hipLaunchKernelGGL((short_stream_two_kernel<NTK_DT_Q4_K, NTK_DT_Q5_K>), grid, block, 0, st, a, b, pa.wgx);
+    else if (da == NTK_DT_Q4_K && db == NTK_DT_Q6_K) hipLaunchKernelGGL((short_stream_two_kernel<NTK_DT_Q4_K, NTK_DT_Q6_K>), grid, block, 0, st, a, b, pa.wgx);
+    else if (da == NTK_DT_Q6_K && db == NTK_DT_Q5_K) hipLaunchKernelGGL((short_stream_two_kernel<NTK_DT_Q6_K, NTK_DT_Q5_K>), grid, block, 0, st, a, b, pa.wgx);
+    else return NTK_E_DTYPE;
     return last_launch_status();
 }
 

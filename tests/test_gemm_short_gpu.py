@@ -283,3 +283,47 @@ def test_products_through_the_decode_repack(qname, T, rows, inf):
     W, res, pt = mats[0][1], r.standard_normal((T, rows[0])).astype(np.float32), _lib.GemmPartials()
     got = go(1, eps, DB.from_numpy(res))[0]
     assert (np.abs(got - (res + n64 @ W.T)) <= REL * (np.sqrt((n64 ** 2) @ (W ** 2).T) + np.abs(res))).all()
+
+
+@pytest.mark.parametrize("qa,qb", [("Q4_K", "Q6_K"), ("Q5_K", "Q4_K"), ("Q6_K", "Q5_K"), ("Q8_0", "Q4_K")])
+@pytest.mark.parametrize("T,ra,rb,inf", [(16, (4096, 1024), (1024,), 4096), (2, (16,), (16,), 256), (7, (80,), (4096, 48), 1280), (11, (6160, 1040), (1040,), 2304), (17, (1024,), (512,), 1024)])
+def test_two_formats_over_one_workspace(qa, qb, T, ra, rb, inf):
+    """one launch for both (K-quants of up to 16 tokens), or one after the other: results as each one's own, the second's sums behind the first's; the bound as above"""
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[T, sum(ra) + inf]))
+    L.ntk_gemm_short_two.argtypes = [C.POINTER(_lib.GemmDesc)] * 2 + [C.c_int, C.c_float, C.c_size_t, VP]
+    from ntransformer_amd import ops
+    nbytes = L.ntk_gemm_quant_workspace_bytes(inf, 4 * (sum(ra) + sum(rb)))       # (two launches' sums side by side)
+    ws, eps = DB.zeros(nbytes), 1e-5
+    X, nw = r.standard_normal((T, inf)).astype(np.float32), (1.0 + 0.1 * r.standard_normal(inf)).astype(np.float32)
+    X[:, 64:200] *= np.float32(1e3)
+    xd, nd = DB.from_numpy(X), DB.from_numpy(nw)
+    _lib.check(L.ntk_short_norm_prepare_x(xd.ptr, None, nd.ptr, T, inf, ws.ptr, None), "short_norm")
+    x64 = X.astype(np.float64)
+    n64 = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + eps) * nw
+    sides, keep = [], []
+    for q, rows in ((qa, ra), (qb, rb)):
+        mats, pt = [], _lib.GemmPartials()
+        segs = (_lib.GemvSeg * len(rows))()
+        for s, n in zip(segs, rows):
+            raw, W, dt = weights(r, getattr(G, "GGML_" + q), n, inf)
+            w = DB.from_numpy(raw) if q == "Q8_0" else ops.rp_pack(DB.from_numpy(raw), n, inf, dt)
+            y = DB.from_numpy(np.full((T, n), 7.0, np.float32))
+            s.W, s.y, s.rows, s.dtype = w.ptr, y.ptr, n, dt
+            mats.append((W, y, n))
+            keep.append(w)
+        if not L.ntk_gemm_short_takes((C.c_int * len(rows))(*rows), len(rows), T, inf, dt):
+            pytest.skip("not a size of this form")
+        d = _lib.GemmDesc()
+        d.segs, d.nseg, d.n_tokens, d.in_features, d.weights_repacked = segs, len(rows), T, inf, int(q != "Q8_0")
+        d.workspace, d.workspace_bytes, d.partials = ws.ptr, nbytes, C.pointer(pt)
+        sides.append((d, pt, mats, segs))
+    _lib.check(L.ntk_gemm_short_two(C.byref(sides[0][0]), C.byref(sides[1][0]), 1, eps, 0, None), "gemm_short_two")
+    whole = ws.numpy(np.float32)
+    for d, pt, mats, _ in sides:
+        for k, (W, y, n) in enumerate(mats):
+            if pt.nsplit > 1:
+                at = (pt.part[k] - ws.ptr) // 4
+                got = whole[at:at + pt.nsplit * T * n].reshape(pt.nsplit, T, n).astype(np.float64).sum(0)
+            else:
+                got = y.numpy(np.float32).reshape(T, n).astype(np.float64)
+            close(got, W, n64)
