@@ -245,7 +245,8 @@ int ntk_short_prepare_x(const float* X, int n_tokens, int in_features, void* wor
 int ntk_short_norm_prepare_x(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int hidden_size, void* workspace, void* stream);
 int ntk_short_silu_mul_prepare_x(const ntk_gemm_partials* partials, void* workspace, void* stream);
 int ntk_gemm_short(const ntk_gemm_desc* desc, int normed, float eps, size_t part_at, void* stream);
-/* ntk_gemm_short of a, then of b with its partial sums behind a's: matrices of two formats over the same planes, in one launch where that is estimated to be ahead (repacked K-quants, sums left) */
+/* ntk_gemm_short of a, then of b with its partial sums behind a's: matrices of two formats over the same planes, in one launch where one of them has many rows and that is estimated to be ahead
+ * (repacked K-quants, sums left) */
 int ntk_gemm_short_two(const ntk_gemm_desc* a, const ntk_gemm_desc* b, int normed, float eps, size_t part_at, void* stream);
 /* A prompt of at most 32 tokens from position 0 on: ntk_reduce_rope_kv_store, ntk_attention_prefill and ntk_short_prepare_x of its result in one launch.  sums / splits: of q, k and v as in
  * ntk_reduce_rope_kv_store; angles: ntk_short_angles' table (ntk_short_angles_bytes, 16-byte aligned), formed once a model.  head_dim 128, an even number of heads (NTK_E_SHAPE). */

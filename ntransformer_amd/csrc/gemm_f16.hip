@@ -2828,7 +2828,7 @@ int ntk_gemm_short(const ntk_gemm_desc* d, int normed, float eps, size_t part_at
 // ---- matrices of two formats over the same planes ----
 extern "C++" { namespace {
 // one side of such a launch: what launch_gemm_f16 asks of it, and what it would take by itself
-struct PairSide { ntk::HostSeg segs[ntk::GB_MAX_SEG]; int nseg, dt, rows; ntk::KSlicePlan lds; float us; };
+struct PairSide { ntk::HostSeg segs[ntk::GB_MAX_SEG]; int nseg, dt, rows; ntk::KSlicePlan lds; ntk::ShortStreamPlan own; };
 template <int DT>
 bool pair_side(const ntk_gemm_desc* d, PairSide* o) {
     int outs[ntk::GB_MAX_SEG];
@@ -2844,7 +2844,7 @@ bool pair_side(const ntk_gemm_desc* d, PairSide* o) {
     o->nseg = d->nseg; o->dt = DT;
     o->lds = ntk::kslice_plan<DT + ntk::GB_RP>(outs, d->nseg, d->n_tokens, d->in_features);
     if (o->lds.n == 0) return false;
-    o->us = ntk::short_stream_plan(DT, d->in_features / 256, o->rows / 16, o->lds.n, o->lds.jobs * o->lds.ups * ntk::DeqI<DT + ntk::GB_RP>::SPU * o->lds.rt).us;
+    o->own = ntk::short_stream_plan(DT, d->in_features / 256, o->rows / 16, o->lds.n, o->lds.jobs * o->lds.ups * ntk::DeqI<DT + ntk::GB_RP>::SPU * o->lds.rt);
     return true;
 }
 bool pair_side(const ntk_gemm_desc* d, PairSide* o) {
@@ -2875,13 +2875,14 @@ int ntk_gemm_short_two(const ntk_gemm_desc* a, const ntk_gemm_desc* b, int norme
                       b->partials && !a->resid && !b->resid && a->workspace && a->workspace == b->workspace && a->workspace_bytes == b->workspace_bytes && b->n_tokens == T && b->in_features == in &&
                       T >= 2 && T <= ntk::SS_TOKENS && in > 0 && in % 256 == 0 && part_at % 4 == 0 && !(reinterpret_cast<uintptr_t>(a->workspace) & 15);
     PairSide sa, sb;
-    if (like && pair_side(a, &sa) && pair_side(b, &sb) && sa.dt != sb.dt) {
+    // (where one of them takes gemm_short.hip's form by itself: matrices too small for that keep the other form, whose sums are the same from a tensor and from its repack)
+    if (like && pair_side(a, &sa) && pair_side(b, &sb) && sa.dt != sb.dt && (sa.own.n > 0 || sb.own.n > 0)) {
         const bool turned = sa.dt > sb.dt;
         PairSide &lo = turned ? sb : sa, &hi = turned ? sa : sb;
         ntk::ShortStreamPlan plo, phi;
         const size_t head = ntk::ws_part_offset((in + 31) / 32 * 32), cap = a->workspace_bytes > head ? (a->workspace_bytes - head) / sizeof(float) : 0;
         if (a->workspace_bytes >= ntk_gemm_quant_workspace_bytes(in, sa.rows + sb.rows) &&
-            ntk::short_stream_plan_two(lo.dt, hi.dt, in / 256, lo.rows / 16, hi.rows / 16, std::min(lo.lds.n, hi.lds.n), lo.us + hi.us, &plo, &phi) &&
+            ntk::short_stream_plan_two(lo.dt, hi.dt, in / 256, lo.rows / 16, hi.rows / 16, std::min(lo.lds.n, hi.lds.n), lo.own.us + hi.own.us, &plo, &phi) &&
             part_at + (size_t)plo.n * T * (size_t)(sa.rows + sb.rows) <= cap) {
             ntk::ShortArgs sh;
             sh.on = true; sh.norm = normed != 0; sh.eps = eps; sh.part_at = part_at; sh.part_cap = cap;

@@ -290,7 +290,7 @@ ShortStreamPlan short_stream_plan(int dt, int units, int tiles, int most, int ot
 
 // Two formats in one launch: the chip's workgroups shared so that the one that ends last ends as early as can be.  Against two launches (apart: their estimates) what is saved is mostly the second
 // one's way to its first product: us, 16 tokens, 5120 rows in Q4_K and 1024 in Q6_K, 4096 columns: 10.4 + 6.8 -> 12.0; short prompts through eight 8B-shaped layers in Q4_K_M 673 -> 645 (2 tokens),
-// 735 -> 709 (16), eight 70B-shaped ones (Q4_K and Q5_K or Q6_K) 1389 -> 1347, 1534 -> 1469, four of 1024 columns 236 -> 233.
+// 735 -> 709 (16), eight 70B-shaped ones (Q4_K and Q5_K or Q6_K) 1389 -> 1347, 1534 -> 1469.
 bool short_stream_plan_two(int da, int db, int units, int tiles_a, int tiles_b, int most, float apart, ShortStreamPlan* a, ShortStreamPlan* b) {
     float best = apart;
     bool found = false;
