@@ -334,6 +334,8 @@ int ntk_debug_sclk_end(unsigned* d_flag, void* other_stream);
 /* test instrumentation: after this call nt_hip_malloc hands out at most `bytes` more device bytes and then fails like an exhausted device
  * (NULL + the reference's message); bytes < 0 removes the budget.  Process-wide; tests only (the load-time repack's "does not fit" path). */
 void ntk_debug_malloc_budget(long long bytes);
+/* test instrumentation: how often the process has waited for a stream (ntk_stream_synchronize) */
+long long ntk_debug_stream_waits(void);
 
 /* *d_pos += 1 (one thread); keeps positions on the device across graph replays */
 int ntk_advance_pos(int* d_pos, void* stream);

@@ -352,6 +352,7 @@ private:
     bool pays(const GatedExperts& ex, int rows, int tokens) const;
     bool rounded(const MoeFeedForward& M, int T) const;
     int product(ntk_dense_desc& d);
+    int wait_for_stream();
     void* rounded_rows(const DenseW& w, int T) const;
     int rounded_product(float* Y, const DenseW& w, int T);
     int linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate);
@@ -400,9 +401,11 @@ private:
     size_t pscratch_bytes_ = 0;                  // pscratch_: partial sums of products (ntk_dense_desc::scratch)
     size_t max_mid_ = 0;              // (post-norm form: the experts' activations of a token side by side)
     int max_rec_ = 0, max_gu2_ = 0, max_conv_ = 0, max_gv_ = 0;   // (scaled form: convolution channels, key heads x value size of the blending attention layers)
-    int *ids_ = nullptr, *offsets_ = nullptr, *order_ = nullptr, *where_ = nullptr, *tokens_dev_ = nullptr, *want_dev_ = nullptr;
+    int *ids_ = nullptr, *offsets_ = nullptr, *order_ = nullptr, *where_ = nullptr, *tokens_dev_ = nullptr;
     HostRows out_row_;                // one row of logits on its way to the caller
-    int* h_stage_ = nullptr;          // pinned: tokens and wanted places of the pass being launched
+    int* h_stage_ = nullptr;          // pinned: tokens and wanted places of the pass being launched, in two halves
+    int stage_ = 0;                   // the half that is next
+    bool stage_busy_[2] = {false, false};   // its copy may still be on its way
     float* logits_ = nullptr;
     size_t logits_rows_ = 0;
     int last_rows_ = 0;

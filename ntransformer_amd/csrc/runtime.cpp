@@ -125,7 +125,11 @@ void* ntk_stream(int which) {
     if (which < 0 || which > 2 || ensure_ready() != NTK_OK) return nullptr;
     return rt().streams[which];
 }
+// test instrumentation: waits for a stream so far
+static std::atomic<long long> g_stream_waits{0};
+long long ntk_debug_stream_waits(void) { return g_stream_waits.load(); }
 int ntk_stream_synchronize(void* stream) {
+    g_stream_waits.fetch_add(1, std::memory_order_relaxed);
     hipStream_t s = resolve_stream(stream);
     return hipStreamSynchronize(s) == hipSuccess ? NTK_OK : NTK_E_LAUNCH;
 }
