@@ -78,6 +78,8 @@ typedef struct ntk_direct_desc {
     void* y16; int ldy16;
 } ntk_direct_desc;
 int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K);
+/* how ntk_dense_direct does a bfloat16 product of `rows` rows in `groups` groups with room floats of scratch (0: gated or grouped): plan = {rows, columns of a tile, tiles a CU holds at once, pieces of K} */
+int ntk_dense_direct_plan(int rows, int groups, int N, int K, long long room, int* plan);
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream);
 /* whether a unit of `ff` values a row (gate and up, or with `plain` up and an activation; then down) over `rows` rows of `tokens` tokens in `groups` groups is estimated to be faster
  * with ntk_dense_direct for its first product -- bfloat16: for both, and a launch that rounds the tokens -- than with ntk_dense (`scratch_bytes` for partial sums) and ntk_glu */

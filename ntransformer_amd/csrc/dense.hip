@@ -721,18 +721,10 @@ __global__ __launch_bounds__(256) void round_rows_kernel(uint16_t* y, int ldy, c
 
 // ---- bf16 products over operands in memory (gemm_direct.hip.h)
 constexpr float kRoundUs = 3.5f, kRoundRate = 4e6f;     // the launch that rounds a product's activations: us, and bytes per us (six an entry)
+static const DirectForm kFormsBf16[] = {{256, 256, 1, 1.45f, 1.45f, 12.0f}, {256, 128, 1, 0.84f, 0.84f, 9.0f}, {128, 256, 1, 0.85f, 0.85f, 9.0f}, {128, 128, 2, 0.72f, 0.475f, 7.0f},
+                                        {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
 static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long room) {
-    static const DirectForm forms[] = {{256, 256, 1, 1.45f, 1.45f, 12.0f}, {256, 128, 1, 0.84f, 0.84f, 9.0f}, {128, 256, 1, 0.85f, 0.85f, 9.0f}, {128, 128, 2, 0.72f, 0.475f, 7.0f},
-                                       {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
-    TilePlan p = plan_direct(forms, 7, 64, rows, groups, N, K, room);
-    // One matrix: which tile and how many pieces with the last round of tiles on a CU at its own pace (p.us stays the estimate that the lines between this and the other forms were drawn with).
-    // us: 150 x 2048 x 2048 13.6 -> 11.6, 700 x 4096 x 14336 97 -> 88, 1500 x 4096 x 14336 229 -> 179, 65 x 6240 x 2048 15.5 -> 14.7; of 380 sizes of 9 .. 2200 rows 1.00
-    // on average (most plans stay), none of those whose plan changes behind by more than 2 %.
-    if (groups == 1) {
-        const TilePlan q = plan_direct(forms, 7, 64, rows, 1, N, K, room, true);
-        p.form = q.form; p.splits = q.splits;
-    }
-    return p;
+    return plan_direct(kFormsBf16, 7, 64, rows, groups, N, K, room, groups == 1 ? 1.05f : 0.0f);
 }
 // float32: K in chunks of 32; one form, ahead of larger and smaller tiles and other splits of the tile over waves at the sizes they were tried at (12 .. 200 rows, 900 in 32 groups).  Over 337
 // grouped sizes it takes 0.89 of gemm_tile.hip.h's time on average and is 3 .. 17 % behind it at about eleven (40 rows in 128 groups, 300 in 8 or 16).  us, the form of gemm_tile.hip.h
@@ -805,6 +797,13 @@ int ntk_dense_unit_direct(int wdtype, int rows, int groups, int tokens, int widt
     return direct < (groups > 1 ? 0.95f : plain ? 0.9f : 0.85f) * tiles;
 }
 
+int ntk_dense_direct_plan(int rows, int groups, int N, int K, long long room, int* plan) {
+    if (!plan) return NTK_E_NULL;
+    if (rows <= 0 || groups <= 0 || N <= 0 || K <= 0) return NTK_E_SHAPE;
+    const TilePlan p = plan_direct_bf16(rows, groups, N, K, room);
+    tell_plan(kFormsBf16[p.form], p, plan);
+    return NTK_OK;
+}
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream) {
     if (!d || !e || !d->W || !e->x16 || (!e->y16 && !d->Y)) return NTK_E_NULL;
     if (!ntk_dense_direct_takes(d->wdtype, d->T, e->x16_rows, d->N, d->K)) return d->T == 0 ? NTK_OK : NTK_E_SHAPE;

@@ -1875,7 +1875,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         } else {
             // one stream-ordered copy of [tokens | wanted places] from pinned memory, its two halves in turn: one is free again once anything queued behind its copy is known to have run (a row of logits
             // fetched, or a wait), so that a prompt behind a fetched row waits for nothing (its marker would be queued once the stream has run dry).  us, a prompt of 64 tokens with such a wait / without:
-            // one layer of attention 2048 wide 155 / 129, one mixture of 16 experts 145 / 126; 512 wide 95 / 63, 106 / 81.
+            // one layer of attention 2048 wide 155 / 129, one mixture of 16 experts 145 / 126; 192 wide 95 / 63, 106 / 81.
             if (stage_busy_[stage_]) {
                 if (wait_for_stream() != NTK_OK) { err_ = "forward: the stream failed"; return nullptr; }
             }

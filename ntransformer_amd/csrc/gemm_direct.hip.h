@@ -288,12 +288,16 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 // that come from memory; the estimate is within a sixth there, and the choice within a tenth of the best form but for uneven small groups.  Rows of several groups: tiles
 // of a group of the average size, plus half a tile where that is no small part of one.
 struct DirectForm { int TM, TN, resident; float alone, busy, over, even; };       // even: the part of a chunk's time that goes with the rows a tile has (rows evenly over the tiles)
-// rounds: a CU whose tiles are no whole number of `resident` ones has the rest at the pace of a tile alone, and five pieces are looked at too where six put a second tile on a CU (126 x 512 x
-// 2048 in bf16: 8.3 in six, 8.9 in five).  us before / so (halves of 32-bit activations, with their split and the sum): 200 x 6144 x 4096 46.8 / 39.8 (768 tiles of 64 x 128 on 512 places
-// / 240 of 128 x 256 in five pieces), 256 52.9 / 43.2, 160 x 4096 x 4096 28.7 / 27.4; of 152 sizes the 12 whose plan changes are 0.8 .. 1.02 of the time before.
-static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats, bool rounds = false) {
+// rounds > 0 (one matrix): a second estimate has a CU's last tiles, where they are no whole number of `resident` ones, at the pace of a tile alone, and looks at five pieces where six put a second
+// tile on a CU.  What it names is taken where it puts the plan of the first estimate behind by that factor, and `us` stays the first estimate's (the lines between these forms and others are drawn with
+// it).  The second estimate is no better than a few per cent: taken wherever it differs, of 250 sizes each it was up to 13 % behind in bfloat16, up to 26 % in gated units, up to 9 % with halves
+// (158 x 2048 x 7488); from 1.05, 1.05 and 1.08 on never by more than 2 %.  Those that are taken, us before / so: bfloat16 700 x 4096 x 14336 97 / 88, 1500 x 4096 x 14336 229 / 179, gated 1181 x 7488 x 7488
+// 212 / 172; halves of 32-bit activations (with their split and the sum) 200 x 6144 x 4096 46.8 / 39.8 (768 tiles of 64 x 128 on 512 places / 240 of 128 x 256 in five pieces), 256 52.9 / 43.2,
+// 443 x 6240 x 7488 130 / 109, gated 262 x 8192 x 7488 136 / 111.
+static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats, float rounds = 0.0f) {
     static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
-    TilePlan best{0, 1, 1e30f};
+    TilePlan best{0, 1, 1e30f}, other = best;
+    float best_too = 0.0f;                          // the second estimate of `best`
     const int chunks = (K + chunk - 1) / chunk;
     for (int i = 0; i < n_forms; ++i) {
         const float mean = (float)rows / groups / f[i].TM;
@@ -301,17 +305,21 @@ static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int row
         const float tiles = row_tiles * ((N + f[i].TN - 1) / f[i].TN);
         for (int s : counts) {
             if (s > 1 && ((long long)s * rows * N > scratch_floats || chunks < 4 * s)) break;
-            if (s == 5 && (!rounds || tiles * 6.0f <= 256.0f)) continue;
-            const int n = (int)((tiles * s + 255.0f) / 256.0f);
+            const int n = (int)((tiles * s + 255.0f) / 256.0f), rest = n % f[i].resident;
             const float full = 1.0f - f[i].even * (1.0f - std::min(1.0f, mean / row_tiles));
-            const int rest = rounds ? n % f[i].resident : n == 1 ? 1 : 0;
-            float us = (float)((chunks + s - 1) / s) * full * ((n - rest) * f[i].busy + (rest ? std::max(f[i].alone, rest * f[i].busy) : 0.0f)) + f[i].over * ((n + f[i].resident - 1) / f[i].resident);
-            if (s > 1) us += 3.0f + (float)(s + 1) * rows * N * 4.0f / 7e6f;
-            if (us < best.us) best = TilePlan{i, s, us};
+            const float each = (float)((chunks + s - 1) / s) * full;
+            float beside = f[i].over * ((n + f[i].resident - 1) / f[i].resident);
+            if (s > 1) beside += 3.0f + (float)(s + 1) * rows * N * 4.0f / 7e6f;
+            const float us = each * (n == 1 ? f[i].alone : n * f[i].busy) + beside;
+            const float too = each * (n == 1 ? f[i].alone : (n - rest) * f[i].busy + (rest ? std::max(f[i].alone, rest * f[i].busy) : 0.0f)) + beside;
+            if (s != 5 && us < best.us) { best = TilePlan{i, s, us}; best_too = too; }
+            if ((s != 5 || tiles * 6.0f > 256.0f) && too < other.us) other = TilePlan{i, s, too};
         }
     }
+    if (rounds > 0.0f && other.us * rounds <= best_too) { best.form = other.form; best.splits = other.splits; }
     return best;
 }
+static void tell_plan(const DirectForm& f, const TilePlan& p, int* plan) { plan[0] = f.TM; plan[1] = f.TN; plan[2] = f.resident; plan[3] = p.splits; }
 
 // the pieces of several matrices' columns side by side, in order, into each one's own results
 template <int V>

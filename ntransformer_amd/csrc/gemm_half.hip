@@ -138,9 +138,9 @@ __global__ __launch_bounds__(1024) void half_norm_split_kernel(const HalfNormArg
 }
 
 // two matrix instructions a product: constants as for bf16 (plan_direct), from 16 .. 200 rows, 1024 .. 28672 outputs, 4096 .. 14336 inputs
-static TilePlan plan_direct_half(int rows, int N, int K, long long room) {
-    static const DirectForm forms[] = {{128, 256, 1, 1.65f, 1.65f, 12.0f, 0.6f}, {64, 128, 2, 0.82f, 0.495f, 5.0f, 0.0f}, {64, 64, 2, 0.47f, 0.315f, 4.0f, 0.0f}};
-    return plan_direct(forms, 3, 64, rows, 1, N, K, room, true);
+static const DirectForm kFormsHalf[] = {{128, 256, 1, 1.65f, 1.65f, 12.0f, 0.6f}, {64, 128, 2, 0.82f, 0.495f, 5.0f, 0.0f}, {64, 64, 2, 0.47f, 0.315f, 4.0f, 0.0f}};
+static TilePlan plan_direct_half(int rows, int N, int K, long long room, bool gated = false) {
+    return plan_direct(kFormsHalf, 3, 64, rows, 1, N, K, room, gated ? 1.02f : 1.08f);
 }
 template <int GLU>
 static int launch_direct_half(const DirectArgs& d, const TilePlan& p, hipStream_t s, bool sum = true) {
@@ -211,7 +211,7 @@ static int half_many(const ntk_half_desc* d, bool ready, ntk_gemm_partials* defe
         a.X16 = halves; a.x_row = (uint32_t)K * 2; a.plane = plane * 2;
         const long long left = (char*)d->workspace + d->workspace_bytes - behind;
         const long long room = d->silu || left < 0 ? 0 : left / (long long)sizeof(float);
-        const TilePlan p = plan_direct_half(n, (int)N, K, room);
+        const TilePlan p = plan_direct_half(n, (int)N, K, room, d->silu != 0);
         if (d->silu) {
             t.W = std::min(w0, w1); a.gate_at = (uint32_t)(w0 - (const char*)t.W); a.up_at = (uint32_t)(w1 - (const char*)t.W);
             a.glu_ff = d->out[0];
@@ -226,6 +226,13 @@ static int half_many(const ntk_half_desc* d, bool ready, ntk_gemm_partials* defe
     return last_launch_status();
 }
 int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) { return half_many(d, false, nullptr, stream); }
+int ntk_gemm_half_plan(int rows, int N, int K, int gated, long long room, int* plan) {
+    if (!plan) return NTK_E_NULL;
+    if (rows <= 0 || N <= 0 || K <= 0) return NTK_E_SHAPE;
+    const TilePlan p = plan_direct_half(rows, N, K, room, gated != 0);
+    tell_plan(kFormsHalf[p.form], p, plan);
+    return NTK_OK;
+}
 
 // ---- a norm's halves from the launch that sums the projection in front of it (include/ntk_engine.h) ----
 int ntk_half_norm_takes(int n_tokens, int width, size_t workspace_bytes) {
@@ -281,7 +288,9 @@ static int gemm_half(float* Y, const void* W, const float* X, int n_tokens, int 
     // The halves formed once, in the workspace, where that is estimated to be ahead: every pass of the rows that it holds reads the weights again, and what the halves take is lost to
     // partial sums.  us over tiles that convert, over halves in a workspace for a third / two thirds / all of the rows / ten times as much: 14336 x 4096, 200 tokens 105, 151 / 89 / 67 / 66;
     // 1024 x 4096, 100 tokens 21 (20 with room for pieces), 145 / 73 / 39 / 18; 4096 x 14336, 200 tokens 207 (112), 426 / 221 / 116 / 69; 2000 tokens 712, 892 / 630 / 463 / 456.  A twentieth in
-    // hand for the estimates, a tenth with several passes, a third where the halves leave fewer pieces (1024 x 8192, 2000 tokens: 168 in one piece, 126 in three).  Over 99 sizes and nine workspaces none is behind the tiles.
+    // hand for the estimates, a tenth with several passes, a third where the halves leave fewer pieces (1024 x 8192, 2000 tokens: 168 in one piece, 126 in three).  Of 10000 sizes (9 .. 2000
+    // rows, 64 .. 28672 outputs) and workspaces with the estimate as it is, those from 1024 inputs on are ahead or within 3 % but for 50, 16 % behind at most (two passes of rows that leave a tile
+    // partly empty, 64 outputs); at 256 and 512 inputs, where the launch that forms the halves takes as long as the product, a third of them are behind, by up to 4 us of 12.
     if (vec && workspace && !((uintptr_t)workspace & 15) && in_features % 64 == 0 && in_features < 1 << 22 && workspace_bytes >= ntk_gemm_half_many_bytes(n_tokens, in_features)) {
         const int per = half_pass_rows(n_tokens, in_features, workspace_bytes), passes = (n_tokens + per - 1) / per;
         const long long left = (long long)workspace_bytes - 4LL * per * in_features - (long long)half_max_bytes(per);

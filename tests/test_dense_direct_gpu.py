@@ -186,3 +186,15 @@ def test_gates_that_leave_rounded_rows(T, n, per_head):
     assert _rounded_near(Lr.gate_rows_16(x, g, n, per_head), x[:, :n] * s)
     with pytest.raises(Exception):
         Lr.gate_rows_16(x, g, 3, 0)
+
+
+@pytest.mark.parametrize("T,N,K,tile", [(129, 2048, 2112, (64, 64, 3)), (70, 6240, 2560, (64, 128, 2)), (70, 6240, 4096, (128, 128, 1)), (200, 6144, 4096, (128, 128, 2))])
+def test_five_pieces_of_k_by_their_plans(T, N, K, tile):
+    """every tile that takes five pieces, chunks of 64 that they do not share evenly (33, 40 and 64): the plan is asked for, so that another choice does not leave the form untested"""
+    from ntransformer_amd import layers as Lr
+    import ctypes as C
+    plan, f = (C.c_int * 4)(), Lr._bind().ntk_dense_direct_plan
+    f.argtypes, f.restype = [C.c_int] * 4 + [C.c_longlong, C.POINTER(C.c_int)], C.c_int
+    assert f(T, 1, N, K, 16 * T * N, plan) == 0 and tuple(plan) == tile + (5,)
+    x, w = _case(np.random.default_rng(T), T, N, K)
+    _close(Lr.dense_direct(x, w, scratch_floats=16 * T * N), x, w)
