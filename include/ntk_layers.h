@@ -78,6 +78,9 @@ typedef struct ntk_direct_desc {
     void* y16; int ldy16;
 } ntk_direct_desc;
 int ntk_dense_direct_takes(int wdtype, int T, int x16_rows, int N, int K);
+/* 1: a bfloat16 product of one matrix is ahead over T rows that the launch in front of it, a norm or (gate != 0) a gate, leaves as bfloat16 (ntk_dense_direct with scratch_bytes of scratch), of
+ * ntk_dense over F32 rows; else 0 */
+int ntk_dense_direct_ahead(int T, int N, int K, int gate, size_t scratch_bytes);
 /* how ntk_dense_direct does a bfloat16 product of `rows` rows in `groups` groups with room floats of scratch (0: gated or grouped): plan = {rows, columns of a tile, tiles a CU holds at once, pieces of K} */
 int ntk_dense_direct_plan(int rows, int groups, int N, int K, long long room, int* plan);
 int ntk_dense_direct(const ntk_dense_desc* d, const ntk_direct_desc* e, void* stream);

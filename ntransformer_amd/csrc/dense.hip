@@ -797,6 +797,17 @@ int ntk_dense_unit_direct(int wdtype, int rows, int groups, int tokens, int widt
     return direct < (groups > 1 ? 0.95f : plain ? 0.9f : 0.85f) * tiles;
 }
 
+// The launch in front of a product can leave its rows as bfloat16, for the direct form, or as F32, for ntk_dense.  Of 450 sizes each (9 .. 1000 rows, 512 .. 4096 outputs, 256 .. 4096 inputs; a norm, a
+// gate, a norm and gate in front, both launches in a graph) always direct was behind by more than 2 % in 43, 62 and 68: fewer than eight chunks, which cost less than a direct tile's first requests
+// (65 x 2048 x 256 7.2 us / 6.4 over F32 rows; many rows are ahead again, 1000 x 2048 x 256 by 15 %), and behind a gate, whose launch gains less, up to 1024 inputs that the tiles cut into pieces and
+// this form does not (48 x 512 x 768 8.9 / 8.2, behind a norm 9.1 / 9.1).  So in none, at 0.81, 0.89 and 0.89 of the time over F32 rows: 150 x 1024 x 2048 12.5 / 15.9, 12 x 4096 x 4096 15.2 / 24.3.
+int ntk_dense_direct_ahead(int T, int N, int K, int gate, size_t scratch_bytes) {
+    if (!ntk_dense_direct_takes(NTK_DT_BF16, T, T, N, K)) return 0;
+    const long long room = T > 65535 ? 0 : (long long)(scratch_bytes / sizeof(float));
+    const TilePlan q = plan_direct_bf16(T, 1, N, K, room), p = plan_tiles_bf16(T, 1, N, K, room);
+    if (K < 512) return T >= 500 || q.us < p.us + 2.5f;
+    return !(gate && K < 1024 && p.splits > 1 && q.splits == 1 && q.us >= p.us + 1.15f);
+}
 int ntk_dense_direct_plan(int rows, int groups, int N, int K, long long room, int* plan) {
     if (!plan) return NTK_E_NULL;
     if (rows <= 0 || groups <= 0 || N <= 0 || K <= 0) return NTK_E_SHAPE;

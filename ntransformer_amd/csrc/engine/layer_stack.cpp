@@ -1101,7 +1101,7 @@ int LayerStackModel::run_mixer(const StackLayer& L, float* cache, int T, int pos
         // many rows: the query latent's norm leaves the bfloat16 rows that its product reads, instead of F32 ones that the product's tiles convert: 1024 x 768 x 3072 18.9 -> 15.0 us, 1999 rows
         // 37.7 (as two portions) -> 20.5
         int st = NTK_E_ALIGN;
-        if (rounded(m.uq, T)) {
+        if (rounded_ahead(m.uq, T, false)) {
             st = ntk_rmsnorm_offset_16(nullptr, cq_, m.q_norm, nullptr, nullptr, nullptr, m.q_rank, a_, na, T, m.q_rank, eps_, 0.0f, stream_);
             if (st != NTK_E_ALIGN) LS_TRY(st);
         }
@@ -1492,10 +1492,14 @@ int LayerStackModel::linear(float* Y, int ldy, const float* X, int ldx, const vo
     return product(d);
 }
 
-// A product over rows that the launch in front of it leaves as bfloat16: where they go -- the front of the products' room, its pieces lie behind them; NULL: that product takes F32 rows
-// or has no room -- and the product.
+// A product over rows that the launch in front of it leaves as bfloat16: whether that is ahead, where they go -- the front of the products' room, its pieces lie behind them; NULL: that product
+// takes F32 rows or has no room -- and the product.
+bool LayerStackModel::rounded_ahead(const DenseW& w, int T, bool gate) const {
+    const size_t image = gate ? (size_t)T * w.in_f * 2 : 0;       // (a gate's rows lie in the products' room)
+    return rounded(w, T) && ntk_dense_direct_ahead(T, (int)w.out_f, (int)w.in_f, gate, pscratch_bytes_ > image ? pscratch_bytes_ - image : 0) != 0;
+}
 void* LayerStackModel::rounded_rows(const DenseW& w, int T) const {
-    return rounded(w, T) && (size_t)T * w.in_f * 2 <= pscratch_bytes_ ? (void*)pscratch_ : nullptr;
+    return rounded_ahead(w, T, true) && (size_t)T * w.in_f * 2 <= pscratch_bytes_ ? (void*)pscratch_ : nullptr;
 }
 int LayerStackModel::rounded_product(float* Y, const DenseW& w, int T) {
     const size_t image = ((size_t)T * w.in_f * 2 + 15) & ~(size_t)15;

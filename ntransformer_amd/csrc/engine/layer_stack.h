@@ -353,6 +353,7 @@ private:
     bool rounded(const MoeFeedForward& M, int T) const;
     int product(ntk_dense_desc& d);
     int wait_for_stream();
+    bool rounded_ahead(const DenseW& w, int T, bool gate) const;
     void* rounded_rows(const DenseW& w, int T) const;
     int rounded_product(float* Y, const DenseW& w, int T);
     int linear(float* Y, int ldy, const float* X, int ldx, const void* W, int wdtype, int T, int N, int K, int accumulate);

@@ -92,3 +92,13 @@ def test_room_bounds_the_pieces():
     for rows, N, K in SIZES:
         for pieces in (0, 1, 2, 5, 7):
             assert bf16(rows, 1, N, K, pieces * rows * N)[3] <= max(pieces, 1) and half(rows, N, K, 0, pieces * rows * N)[3] <= max(pieces, 1)
+
+
+@pytest.mark.parametrize("T,N,K,norm,gate", [(65, 2048, 256, 0, 0), (24, 4096, 256, 0, 0), (300, 1024, 256, 0, 0), (1000, 2048, 256, 1, 1), (48, 512, 768, 1, 0), (24, 1024, 768, 1, 0), (24, 1024, 1024, 1, 1),
+                                             (12, 4096, 4096, 1, 1), (150, 1024, 2048, 1, 1), (128, 4096, 1024, 1, 1), (1024, 3072, 768, 1, 1), (1999, 2048, 2048, 1, 1), (8, 4096, 4096, 0, 0),
+                                             (65, 2048, 2050, 0, 0)])
+def test_rows_left_as_bfloat16_where_that_is_ahead(T, N, K, norm, gate):
+    """(up to 8 rows, and rows of no whole chunks, the direct form does not take at all)"""
+    f = _lib.lib().ntk_dense_direct_ahead
+    f.argtypes, f.restype = [C.c_int] * 4 + [C.c_size_t], C.c_int
+    assert (f(T, N, K, 0, 64 << 20), f(T, N, K, 1, 64 << 20)) == (norm, gate)
