@@ -334,7 +334,7 @@ int ntk_debug_sclk_begin(unsigned* d_flag, unsigned long long* d_out2, void* sid
 int ntk_debug_sclk_end(unsigned* d_flag, void* other_stream);
 
 /* test instrumentation: after this call nt_hip_malloc hands out at most `bytes` more device bytes and then fails like an exhausted device
- * (NULL + the reference's message); bytes < 0 removes the budget.  Process-wide; tests only (the load-time repack's "does not fit" path). */
+ * (NULL + the reference's message), where what is freed of them counts again; bytes < 0 removes the budget.  Process-wide; tests only (the load-time repack's "does not fit" path). */
 void ntk_debug_malloc_budget(long long bytes);
 /* test instrumentation: how often the process has waited for a stream (ntk_stream_synchronize) */
 long long ntk_debug_stream_waits(void);

@@ -923,16 +923,62 @@ int LayerStackModel::load(const std::string& dir, const SeqLoadOptions& opt) {
 }
 
 int LayerStackModel::alloc_buffers() {
-    const int W = info_.width;
+    const size_t ctx = (size_t)opt_.max_context;
+    out_row_.alloc((size_t)info_.vocab);                     // (none: a copy of the runtime's)
+    // what every slot holds per layer run: cache rows per position, the recurrent state, the convolutions' last inputs (mixer's, then feed-forward's)
+    for (auto& r : runs_) {
+        const StackLayer& L = layers_[(size_t)r.layer];
+        const size_t row = (size_t)L.cache_row();
+        if (L.kv_from() >= 0) {
+            r.cache = runs_[(size_t)L.kv_from()].cache;       // (such a form has no repeated span: run i is layer i)
+        } else if (row) {
+            r.cache = (float*)dev_alloc((size_t)opt_.slots * ctx * row * sizeof(float));
+            if (!r.cache) return fail(NTK_E_NOMEM, "out of device memory (cache)");
+        }
+        if (L.state_floats()) {
+            r.state = (float*)dev_alloc((size_t)opt_.slots * L.state_floats() * sizeof(float));
+            if (!r.state) return fail(NTK_E_NOMEM, "out of device memory (state)");
+        }
+        if (form_.sequential && taps_ > 1) {
+            r.conv = (float*)dev_alloc((size_t)opt_.slots * 2 * (taps_ - 1) * info_.width * sizeof(float));
+            if (!r.conv) return fail(NTK_E_NOMEM, "out of device memory (state)");
+        }
+    }
     // Tokens of an internal pass: every launch of a layer runs once a pass, so a prompt cut in two pays its launches, its weights' way to the matrix cores and each launch's last wave twice.
     // us a prompt, passes of 1024 / 2048 / 4096 tokens: attention, recurrence and latents in bfloat16 (2048 wide, four layers), 1100 tokens 1698 / 1382 / 1376, 1999 2345 / 1972 / 1972, 2500
     // 3194 / 2763 / 2508, 8000 10578 / 8640 / 8261; in float32, 1999 tokens 7535 / 7180 / 7172; two layers of 32 experts, 1100 tokens 1127 / 823 / 823, 2500 2021 / 1700 / 1463, 8000 7014 /
     // 5476 / 5070.  (The workspaces go with it: about a gigabyte at these widths.)  A token's choices of experts are rows of their own, and rows a grid's second dimension.
+    // A long pass is a matter of speed alone: where its buffers do not fit, take more than a quarter of what is left or leave no room for the attention's image, it is halved, down to the 1024 tokens that a
+    // model cannot do without.
     chunk_ = 4096;
     for (const auto& L : layers_)
         if (L.mlp_kind == kMlpMoe) while (chunk_ > 1024 && (long long)chunk_ * L.mlp.top > 32768) chunk_ /= 2;
     chunk_ = std::min(opt_.max_context, chunk_);
+    for (const size_t mark = allocs_.size();;) {
+        const bool last = chunk_ <= 1024;
+        size_t before = 0, left = 0, total = 0;
+        const bool known = ntk_device_mem_info(&before, &total) == NTK_OK;
+        const bool fits = alloc_pass();
+        if (last && !fits) return fail(NTK_E_NOMEM, "out of device memory (activation buffers)");
+        const size_t visible = max_hqd_ > 0 ? ctx * (size_t)(max_hdn_ + max_hdv_) * sizeof(float) : 0;      // (of the buffers, what goes with the context)
+        if (fits && known && ntk_device_mem_info(&left, &total) == NTK_OK && (last || before <= left + visible + before / 4)) {
+            // behind everything that the model cannot run without, and no more than a quarter of what is left: the attention has a form without
+            if (image_bytes_ && image_bytes_ <= left / 4) image_ = nt_hip_malloc(image_bytes_);
+            if (image_ || !image_bytes_) return NTK_OK;
+        }
+        if (last) break;
+        for (; allocs_.size() > mark; allocs_.pop_back()) nt_hip_free(allocs_.back());
+        chunk_ = chunk_ > 2048 ? 2048 : 1024;
+    }
+    image_bytes_ = 0;
+    return NTK_OK;
+}
+
+// what a pass of chunk_ tokens works in
+bool LayerStackModel::alloc_pass() {
+    const int W = info_.width;
     size_t sc = 0, wsc = 0, lsc = 0, rsc = 0;
+    image_bytes_ = 0;
     // what a portion's attention sees at most, in pieces: the portion and a window ahead of it (and the positions that stay visible), or everything
     auto seen = [&](int window, int keep, int kv_heads, int dk, int dv) {
         const long long n = window > 0 ? std::min<long long>((long long)window + chunk_ + keep + 64, opt_.max_context) : opt_.max_context;
@@ -1023,43 +1069,18 @@ int LayerStackModel::alloc_buffers() {
     ok = ok && fl(&pscratch_, pscratch_bytes_ / sizeof(float));
     if (wdtype_ == NTK_DT_BF16) ok = ok && (h1_16_ = dev_alloc(C * W * 2)) && (h2_16_ = dev_alloc(C * W * 2));
     if (max_mid_ > 0) ok = ok && fl(&mid_, (size_t)ntk_dense_few_rows() * max_mid_);
+    if (h_stage_) nt_hip_free_host(h_stage_);
     h_stage_ = (int*)nt_hip_malloc_host(4 * C * sizeof(int));
     ok = ok && h_stage_ != nullptr;
-    out_row_.alloc((size_t)info_.vocab);                     // (none: a copy of the runtime's)
     if (max_top_ > 0) {
         const size_t P = C * max_top_;
         ok = ok && in(&ids_, P) && fl(&wts_, P) && fl(&sg_, C) && in(&offsets_, (size_t)max_e_ + 1) && in(&order_, P) && in(&where_, P) && fl(&gu_, P * max_ff2_) &&
              fl(&act_, P * (max_ff2_ / 2)) && fl(&dn_, P * W);
         if (max_sff2_ > 0) ok = ok && fl(&sgu_, C * max_sff2_) && fl(&sact_, C * (max_sff2_ / 2)) && fl(&sdn_, C * W);
     }
-    if (!ok) return fail(NTK_E_NOMEM, "out of device memory (activation buffers)");
-    // what every slot holds per layer run: cache rows per position, the recurrent state, the convolutions' last inputs (mixer's, then feed-forward's)
-    for (auto& r : runs_) {
-        const StackLayer& L = layers_[(size_t)r.layer];
-        const size_t row = (size_t)L.cache_row();
-        if (L.kv_from() >= 0) {
-            r.cache = runs_[(size_t)L.kv_from()].cache;       // (such a form has no repeated span: run i is layer i)
-        } else if (row) {
-            r.cache = (float*)dev_alloc((size_t)opt_.slots * ctx * row * sizeof(float));
-            if (!r.cache) return fail(NTK_E_NOMEM, "out of device memory (cache)");
-        }
-        if (L.state_floats()) {
-            r.state = (float*)dev_alloc((size_t)opt_.slots * L.state_floats() * sizeof(float));
-            if (!r.state) return fail(NTK_E_NOMEM, "out of device memory (state)");
-        }
-        if (form_.sequential && taps_ > 1) {
-            r.conv = (float*)dev_alloc((size_t)opt_.slots * 2 * (taps_ - 1) * W * sizeof(float));
-            if (!r.conv) return fail(NTK_E_NOMEM, "out of device memory (state)");
-        }
-    }
-    // behind everything that the model cannot run without, and no more than a quarter of what is left: the attention has a form without
-    size_t left = 0, total = 0;
-    if (image_bytes_ && ntk_device_mem_info(&left, &total) == NTK_OK && image_bytes_ <= left / 4) image_ = nt_hip_malloc(image_bytes_);
-    if (!image_) image_bytes_ = 0;
-    return NTK_OK;
+    return ok;
 }
 
-// an allocation during a run: it goes ahead of the attention's image
 void* LayerStackModel::late_alloc(size_t bytes) {
     void* p = nt_hip_malloc(bytes);
     if (p || !image_) return p;

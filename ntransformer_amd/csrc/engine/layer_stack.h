@@ -328,6 +328,7 @@ private:
     int upload_vector(const ModelFolder& f, const std::string& name, int64_t n, float** out);
     int upload_matrix(const ModelFolder& f, const std::vector<std::string>& names, int64_t in_f, DenseW& out, int count = 1);
     int alloc_buffers();
+    bool alloc_pass();
     void* dev_alloc(size_t bytes);
     void* late_alloc(size_t bytes);
     int portion(int slot, const int* tokens_dev, int token, int prev_token, int T, int pos0, const int* want_dev, int n_want, bool want_last, float* logits_out);

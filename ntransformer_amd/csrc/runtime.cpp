@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <unordered_map>
 #include "../../include/ntk_engine.h"
 #include <atomic>
 
@@ -161,8 +162,17 @@ int ntk_event_elapsed_ms(void* start, void* end, float* ms) {
 }
 
 // test instrumentation (ntk_debug_malloc_budget): nt_hip_malloc fails like an exhausted device once the budget is used up; < 0 = no budget
+// (what is freed of it can be had again, as on a device)
 static std::atomic<long long> g_malloc_budget{-1};
-void ntk_debug_malloc_budget(long long bytes) { g_malloc_budget.store(bytes); }
+static std::atomic<size_t> g_budgeted{0};
+static std::mutex g_budget_mu;
+static std::unordered_map<void*, size_t> g_budget_of;
+void ntk_debug_malloc_budget(long long bytes) {
+    std::lock_guard<std::mutex> lk(g_budget_mu);
+    g_budget_of.clear();
+    g_budgeted.store(0);
+    g_malloc_budget.store(bytes);
+}
 void* nt_hip_malloc(size_t size) {
     if (ensure_ready() != NTK_OK) { fprintf(stderr, "ntk: no GPU available for hipMalloc\n"); return nullptr; }
     void* p = nullptr;
@@ -170,7 +180,12 @@ void* nt_hip_malloc(size_t size) {
     long long left = g_malloc_budget.load();
     if (left < 0 || (long long)size <= left) {
         e = hipMalloc(&p, size ? size : 1);
-        if (e == hipSuccess && left >= 0) g_malloc_budget.fetch_sub((long long)size);
+        if (e == hipSuccess && left >= 0) {
+            std::lock_guard<std::mutex> lk(g_budget_mu);
+            g_malloc_budget.fetch_sub((long long)size);
+            g_budget_of[p] = size;
+            g_budgeted.store(g_budget_of.size());
+        }
     }
     if (e != hipSuccess) {   // reference device.cu:154-162: message + NULL
         fprintf(stderr, "hipMalloc failed (%zu bytes): %s\n", size, hipGetErrorString(e));
@@ -179,7 +194,19 @@ void* nt_hip_malloc(size_t size) {
     }
     return p;
 }
-void nt_hip_free(void* p) { if (p) (void)hipFree(p); }
+void nt_hip_free(void* p) {
+    if (!p) return;
+    if (g_budgeted.load()) {
+        std::lock_guard<std::mutex> lk(g_budget_mu);
+        const auto it = g_budget_of.find(p);
+        if (it != g_budget_of.end()) {
+            if (g_malloc_budget.load() >= 0) g_malloc_budget.fetch_add((long long)it->second);
+            g_budget_of.erase(it);
+            g_budgeted.store(g_budget_of.size());
+        }
+    }
+    (void)hipFree(p);
+}
 void nt_hip_memcpy_h2d(void* d, const void* s, size_t n) { if (n) (void)hipMemcpy(d, s, n, hipMemcpyHostToDevice); }
 void nt_hip_memcpy_d2h(void* d, const void* s, size_t n) { if (n) (void)hipMemcpy(d, s, n, hipMemcpyDeviceToHost); }
 // Device-to-device copies and fills run on the legacy stream and may return before they have executed; the library's own streams are NON-blocking

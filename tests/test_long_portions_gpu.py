@@ -1,5 +1,6 @@
 """Prompts longer than one internal pass of the model folders (4096 tokens), whole and in portions that end elsewhere, against each family's oracle: what a pass leaves for the next -- cache rows,
 states, carried convolution inputs, blended values, the pair in front of a pass's first token."""
+import ctypes as C
 import functools
 import os
 import sys
@@ -51,3 +52,55 @@ def test_a_prompt_beyond_one_internal_pass(tmp_path, monkeypatch, family):
     e.seq_forward(s, toks[:130], want=[])
     assert rel(e.seq_forward(s, toks[130:], want=[PASS - 1, PASS, N - 131]), [PASS + 129, PASS + 130, N - 1]) < TOL
     e.close()
+
+
+def _left_of(L, most):
+    """what is left of the malloc budget, to the byte"""
+    left, held = 0, []
+    for bit in range(most.bit_length(), -1, -1):
+        p = L.nt_hip_malloc(1 << bit)
+        if p:
+            left += 1 << bit
+            held.append(p)
+    for p in held:
+        L.nt_hip_free(p)
+    return left
+
+
+def test_a_pass_yields_to_memory(tmp_path):
+    """a long pass is a matter of speed: with a budget that its buffers do not fit the folder loads with passes half as long, down to 1024 tokens, and computes the same; below those it is refused"""
+    from ntransformer_amd import _lib
+    from ntransformer_amd.engine import Engine
+    L, O = _lib.lib(), fabolorn_oracle
+    L.ntk_debug_malloc_budget.argtypes, L.ntk_debug_malloc_budget.restype = [C.c_longlong], None
+    L.nt_hip_malloc.argtypes, L.nt_hip_malloc.restype, L.nt_hip_free.argtypes = [C.c_size_t], C.c_void_p, [C.c_void_p]
+    cfg = O.small_config(layers=("latent_attention", "latent_attention_2"), dim=72, ff=256, shared_ff=192)
+    w = O.random_weights(cfg, 3)
+    O.save_model(str(tmp_path / "m"), cfg, w)
+    toks = [int(t) for t in np.random.default_rng(4).integers(0, cfg["vocab"], 2500)]
+    want = [0, 1023, 1024, 2047, 2048, 2499]
+    ref = np.asarray(O.forward(cfg, w, toks), np.float64)[want]
+    whole, used = 1 << 30, []
+
+    def load(budget):
+        L.ntk_debug_malloc_budget(budget)
+        try:
+            e = Engine()
+            e.load_folder(str(tmp_path / "m"), max_context=4400, dtype="float32")
+            used.append(budget - _left_of(L, budget))
+        finally:
+            L.ntk_debug_malloc_budget(-1)
+        got = e.seq_forward(e.seq_acquire(), toks, want=want)
+        e.close()
+        assert np.sqrt(np.mean((got - ref) ** 2)) < TOL * np.sqrt(np.mean(ref ** 2))
+    image = L.ntk_prompt_attention_image_bytes
+    image.argtypes, image.restype = [C.c_int] * 4, C.c_size_t
+    room = image(4400, cfg["layers"][0]["mixer"]["heads"], 72 + 8, 24)
+    load(whole)
+    load(used[0] - 1)                                  # (the image alone does not fit: the pass yields before it does)
+    load(used[0] - room - 1)
+    load(used[1] - 1)
+    assert used[1] == used[2] < used[0] - room and used[3] < used[1] and used[1] - used[3] < used[0] - used[1]
+    load(used[3] - 1)                                  # passes of 1024, no image
+    with pytest.raises(Exception):
+        load(used[4] - 1)
