@@ -1871,7 +1871,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
     }
     if (capture_) {
         const size_t cf = runs_.size() * (size_t)n * info_.width;
-        if (n > std::min(chunk_, 1024)) { err_ = "capture: the portion must fit one internal pass"; return nullptr; }
+        if (n > std::min(chunk_, kCaptureTokens)) { err_ = "capture: a portion of at most " + std::to_string(std::min(chunk_, kCaptureTokens)) + " tokens"; return nullptr; }
         if (cf > capture_floats_) {
             ntk_stream_synchronize(stream_);
             if (capture_buf_) nt_hip_free(capture_buf_);
@@ -1889,6 +1889,7 @@ float* LayerStackModel::forward(int slot, const int* tokens, int n, const int* w
         std::vector<int> rel((size_t)std::max(w1 - done_want, 1));
         for (int i = done_want; i < w1; ++i) rel[(size_t)(i - done_want)] = want[i] - at;
         const int nw = w1 - done_want;
+        if (nw > chunk_) { err_ = "forward: more than " + std::to_string(chunk_) + " wanted places in one internal pass"; return nullptr; }      // (places may repeat: the gathered rows' room)
         int* const want_dev = tokens_dev_ + T;
         // (a decoded token goes with the launch of its embedding, where that is the plain table's)
         const bool alone = T == 1 && nw <= 1 && tokens[at] >= 0 && info_.width % 4 == 0 && !((uintptr_t)embed_.ptr & 15) && !(form_.gated || form_.post_norm || buckets_ > 0);

@@ -295,6 +295,7 @@ public:
     int sync() override;
     void* stream() const override { return stream_; }
     static constexpr int kSharedRows = 8;     // up to this many tokens per portion take the decode form of the mixer (and the GEMV form of the products)
+    static constexpr int kCaptureTokens = 1024;   // a captured portion's (its stream after every layer run is kept)
 
 private:
     struct Run { int layer; bool enters; float* cache; float* state; float* conv; };   // per slot: cache rows, recurrent state, [2][taps - 1][width] last inputs

@@ -52,3 +52,22 @@ def test_prompts_one_after_the_other(tmp_path):
         assert off(one(p, at), r[at]) < 2e-4
         assert one(p, []).shape[0] == 0
     e.close()
+
+
+def test_limits(tmp_path):
+    """a captured portion beyond 1024 tokens, and more (repeated) wanted places than a pass has room for, are refused; what is at the bound runs"""
+    e, cfg, w = engine(tmp_path, 1100)
+    toks = [int(t) for t in np.random.default_rng(8).integers(0, cfg["vocab"], 1100)]
+    s = e.seq_acquire()
+    e.seq_capture(True)
+    with pytest.raises(Exception):
+        e.seq_forward(s, toks, want=[0])
+    e.seq_forward(s, toks[:1024], want=[0])
+    assert np.isfinite(e.seq_captured(1024)).all()
+    e.seq_capture(False)
+    e.seq_truncate(s, 0)
+    with pytest.raises(Exception):
+        e.seq_forward(s, toks[:40], want=[39] * 1101)
+    got = e.seq_forward(s, toks[:40], want=[39] * 1100)
+    assert (got == got[0]).all()
+    e.close()
