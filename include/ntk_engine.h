@@ -241,6 +241,8 @@ int ntk_rows_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials
  *                                 workspace's area of partial sums at which this launch's begin (a multiple of 4), so that several launches may leave theirs to one consumer
  * n_tokens <= 32, rows a multiple of 32 (NTK_E_SHAPE), 16-byte aligned pointers (NTK_E_ALIGN).  `workspace` must not be the one partials lie in.  Stream ordered, no allocation. */
 int ntk_gemm_short_takes(const int* rows, int nseg, int n_tokens, int in_features, int dtype);
+/* how it takes them: 1 the planes in LDS, 2 in registers (K-quants, many rows, up to 16 tokens); 0 not at all */
+int ntk_gemm_short_form(const int* rows, int nseg, int n_tokens, int in_features, int dtype, int repacked);
 int ntk_short_prepare_x(const float* X, int n_tokens, int in_features, void* workspace, void* stream);
 int ntk_short_norm_prepare_x(float* hidden, const ntk_gemm_partials* partials, const float* weight, int n_tokens, int hidden_size, void* workspace, void* stream);
 int ntk_short_silu_mul_prepare_x(const ntk_gemm_partials* partials, void* workspace, void* stream);

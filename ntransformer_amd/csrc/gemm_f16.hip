@@ -2410,6 +2410,22 @@ static int short_takes(const int* rows, int nseg, int T, int in) {
     return kslice_plan<DT>(rows, nseg, T, in).n > 0;
 }
 
+// gemm_short.hip's plan for matrices whose slices are `plan` with the planes in LDS: 1 .. 16 tokens, many rows; never in more slices than there, so that its sums fit where that one's do
+template <int DT>
+static ShortStreamPlan stream_plan(const int* rows, int nseg, int T, int in, const KSlicePlan& plan) {
+    if constexpr (DeqI<DT>::RP) {
+        int total = 0;
+        for (int i = 0; i < nseg; ++i) total += rows[i];
+        if (T <= SS_TOKENS && plan.n > 0) return short_stream_plan(DT - GB_RP, in / 256, total / 16, plan.n, plan.jobs * plan.ups * DeqI<kslice_dt<DT>()>::SPU * plan.rt);
+    }
+    return ShortStreamPlan{};
+}
+template <int DT>
+static int short_form(const int* rows, int nseg, int T, int in) {
+    const KSlicePlan plan = kslice_plan<DT>(rows, nseg, T, in);
+    return plan.n == 0 ? 0 : stream_plan<DT>(rows, nseg, T, in, plan).n > 0 ? 2 : 1;
+}
+
 // gemm_short.hip's launch over the planes of workspace wsb; parts: where each matrix's sums of slices lie
 template <int DT>
 static void stream_params(ShortStreamParams* q, const HostSeg* segs, int nseg, int T, int in, const ShortStreamPlan& sp, uint8_t* wsb, const ShortArgs& sh, const float* resid, const float** parts) {
@@ -2476,8 +2492,7 @@ static int launch_gemm_f16(const HostSeg* segs, int nseg, const float* X, int T,
     const KSlicePlan plan = kslice_plan<DT>(outs, nseg, T, in);
     if (sh.on && (plan.n == 0 || sh.part_at + (size_t)plan.n * T * (size_t)out_total > sh.part_cap)) return NTK_E_SHAPE;   // (nothing launched: the planes were there)
     if constexpr (D::RP) {
-        // 2 .. 16 tokens, many rows: the planes in registers (gemm_short.hip); never in more slices than the form below, so that its sums fit where that one's do
-        const ShortStreamPlan sp = sh.on && T <= SS_TOKENS ? short_stream_plan(DT - GB_RP, in / 256, (int)(out_total / 16), plan.n, plan.jobs * plan.ups * KD::SPU * plan.rt) : ShortStreamPlan{};
+        const ShortStreamPlan sp = sh.on ? stream_plan<DT>(outs, nseg, T, in, plan) : ShortStreamPlan{};
         if (sp.n > 0) {
             ShortStreamParams q{};
             const float* parts[GB_MAX_SEG] = {};
@@ -2813,6 +2828,15 @@ int ntk_gemm_short_takes(const int* rows, int nseg, int n_tokens, int in_feature
         default: return 0;
     }
 }
+int ntk_gemm_short_form(const int* rows, int nseg, int n_tokens, int in_features, int dtype, int repacked) {
+    if (!ntk_gemm_short_takes(rows, nseg, std::max(n_tokens, 2), in_features, dtype) || n_tokens < 1) return 0;
+    switch (dtype + (repacked ? ntk::GB_RP : 0)) {
+        case NTK_DT_Q4_K + ntk::GB_RP: return ntk::short_form<NTK_DT_Q4_K + ntk::GB_RP>(rows, nseg, n_tokens, in_features);
+        case NTK_DT_Q5_K + ntk::GB_RP: return ntk::short_form<NTK_DT_Q5_K + ntk::GB_RP>(rows, nseg, n_tokens, in_features);
+        case NTK_DT_Q6_K + ntk::GB_RP: return ntk::short_form<NTK_DT_Q6_K + ntk::GB_RP>(rows, nseg, n_tokens, in_features);
+        default: return repacked ? 0 : 1;
+    }
+}
 int ntk_gemm_short(const ntk_gemm_desc* d, int normed, float eps, size_t part_at, void* stream) {
     if (!d) return NTK_E_NULL;
     if (d->n_tokens < 1 || d->n_tokens > ntk::GB_SHORT || d->in_features <= 0 || part_at % 4 != 0) return NTK_E_SHAPE;
@@ -2844,7 +2868,7 @@ bool pair_side(const ntk_gemm_desc* d, PairSide* o) {
     o->nseg = d->nseg; o->dt = DT;
     o->lds = ntk::kslice_plan<DT + ntk::GB_RP>(outs, d->nseg, d->n_tokens, d->in_features);
     if (o->lds.n == 0) return false;
-    o->own = ntk::short_stream_plan(DT, d->in_features / 256, o->rows / 16, o->lds.n, o->lds.jobs * o->lds.ups * ntk::DeqI<DT + ntk::GB_RP>::SPU * o->lds.rt);
+    o->own = ntk::stream_plan<DT + ntk::GB_RP>(outs, d->nseg, d->n_tokens, d->in_features, o->lds);
     return true;
 }
 bool pair_side(const ntk_gemm_desc* d, PairSide* o) {

@@ -7,8 +7,11 @@
 //     (mask, exponent), (1024 + q) sc - 1024 sc one v_pk_fma with an exact result; a high nibble stays where it is, at sixteen times its value.
 //   * Q6_K: (q - 32) sc takes 13 bits.  Four lane groups exchange dwords (v_permlane32_swap, v_permlane16_swap), after which a product lies within sixteen columns and its sum takes the scale.
 // The integers are given to the matrix cores as normal numbers: as FP16 subnormals (q 2^-24, no instruction at all) products come out exact, but their sums are aligned by the nominal exponent and lose
-// up to ten bits (root mean square of the error 1.45e-7 -> 2.5e-7, beside towering channels 2.3e-7 -> 1.8e-6).  Sums run over two products (the first pieces) or four (the second ones) and are added
-// up outside: in one chain over a unit they are 1.7e-7.  So: Q4_K 1.45e-7, Q5_K 1.53e-7, Q6_K 1.12e-7 of the products' size, the other form's 1.45e-7, 1.51e-7, 1.10e-7 (16 x 8192 x 4096, three seeds).
+// up to ten bits (root mean square of the error 1.45e-7 -> 2.5e-7, beside towering channels 2.3e-7 -> 1.8e-6).  A product of 22 bits an entry is rounded as it is summed, which the other form's (weights
+// of 4 or 5 bits) is not, so the rest of the way is short: no product's sum is the start of another (but for the second pieces), a unit's and a slice's sums are added up as trees (Q6_K, whose products
+// are exact: a chain of eight a half of a unit, units in order).  Root mean square of the error over the products' size, this form / the other, 16 x 28672 x 4096: Q4_K 1.393e-7 / 1.476e-7, with eight
+// channels a hundred times the others' (24 choices of them) 1.772 / 1.808; Q5_K 1.425 / 1.501, 1.732 / 1.804; Q6_K 1.039 / 1.122, 1.071 / 1.162.  With products in chains of two and units in order it was 2 % more
+// beside such channels (and a launch of 57344 x 8192 in Q5_K took 47.0 us instead of 48.5).
 // us, 28672 x 4096 in Q4_K: without the planes' way 1.2 less, without any product 3.6 less; three items under way 0.5 .. 1 ahead of four, three ahead of six (4 us).
 #include "gemm_short.hip.h"
 #include <algorithm>
@@ -38,8 +41,31 @@ __device__ __forceinline__ void ss_turn(uint32_t (&r)[4]) {
     r[0] = c[0]; r[1] = c[1]; r[2] = d[0]; r[3] = d[1];
 }
 
-// Workgroup (x, slice): eight waves, wave = (row group wave / ups, unit slice * ups + wave % ups of 256 columns), tiles (x + k wgx) * groups + row group for k = 0, 1, ...
 typedef f32x4 SsSums[SS_AHEAD * SS_WAVES][64];
+// the sums of a slice's units (a tree: all requested at once; behind the last: zeros)
+template <int N>
+__device__ __forceinline__ f32x4 ss_tree(const f32x4 (*of)[64], int n, int lane) {
+    f32x4 v[N];
+#pragma unroll
+    for (int w = 0; w < N; ++w) v[w] = of[min(w, n - 1)][lane];
+#pragma unroll
+    for (int w = 1; w < N; ++w)
+        if (w >= n) v[w] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int step = 1; step < N; step *= 2)
+#pragma unroll
+        for (int w = 0; w + step < N; w += 2 * step) v[w] += v[w + step];
+    return v[0];
+}
+template <bool TREE>
+__device__ __forceinline__ f32x4 ss_units(const f32x4 (*of)[64], int n, int lane) {
+    if constexpr (TREE) return n > 4 ? ss_tree<8>(of, n, lane) : n > 2 ? ss_tree<4>(of, n, lane) : ss_tree<2>(of, n, lane);
+    f32x4 y = of[0][lane];
+    for (int w = 1; w < n; ++w) y += of[w][lane];
+    return y;
+}
+
+// Workgroup (x, slice): eight waves, wave = (row group wave / ups, unit slice * ups + wave % ups of 256 columns), tiles (x + k wgx) * groups + row group for k = 0, 1, ...
 template <int DT>
 __device__ __forceinline__ void short_stream(const ShortStreamParams& p, const int bx, const int slice, const int wgx, const int slices, SsSums (&sums)[2]) {
     using R = Sp<DT>;
@@ -142,7 +168,7 @@ __device__ __forceinline__ void short_stream(const ShortStreamParams& p, const i
     auto multiply = [&](const SsItem<DT>& it) {
         f32x4 y;
         if constexpr (FOLD) {
-            f32x4 acc[2][2] = {{zero, zero}, {zero, zero}}, low0 = zero, low1 = zero;        // [s][h] of the first pieces
+            f32x4 acc[2][2][2], low0 = zero, low1 = zero;        // [s][h][t] of the first pieces
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 // the sub-blocks' scales of this lane's columns as FP16, (low nibbles, high nibbles): 1024 + sc, less 1024; a high nibble stands at sixteen times its value, and so do those products
@@ -165,9 +191,9 @@ __device__ __forceinline__ void short_stream(const ShortStreamParams& p, const i
                         hi[2 * c] = ss_mul(h0, s1, n1); hi[2 * c + 1] = ss_mul(h1, s1, n1);
                     }
                     const f16x8 wl = ss_op(lo[0], lo[1], lo[2], lo[3]), wh = ss_op(hi[0], hi[1], hi[2], hi[3]);
-                    acc[s][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[0][4 * s + t]), wl, acc[s][0], 0, 0, 0);
+                    acc[s][0][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[0][4 * s + t]), wl, zero, 0, 0, 0);
                     low0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[1][4 * s + t]), wl, low0, 0, 0, 0);
-                    acc[s][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[0][4 * s + 2 + t]), wh, acc[s][1], 0, 0, 0);
+                    acc[s][1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[0][4 * s + 2 + t]), wh, zero, 0, 0, 0);
                     low1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x[1][4 * s + 2 + t]), wh, low1, 0, 0, 0);
                 }
             }
@@ -184,9 +210,12 @@ __device__ __forceinline__ void short_stream(const ShortStreamParams& p, const i
             }
             const float d = h2f((uint16_t)(it.dd & 0xFFFFu)), dm = h2f((uint16_t)(it.dd >> 16)) * -64.0f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = fmaf(dm, mn[e], d * fmaf(0.0625f, (acc[0][1][e] + acc[1][1][e]) + low1[e], (acc[0][0][e] + acc[1][0][e]) + low0[e]));
+            for (int e = 0; e < 4; ++e) {
+                auto first = [&](int h) { return (acc[0][h][0][e] + acc[0][h][1][e]) + (acc[1][h][0][e] + acc[1][h][1][e]); };
+                y[e] = fmaf(d, fmaf(0.0625f, first(1) + low1[e], first(0) + low0[e]), dm * mn[e]);
+            }
         } else {
-            y = zero;
+            f32x4 half[2] = {zero, zero};                 // a chain of eight a half of the unit
             const float d = h2f((uint16_t)it.dd);
             const f16x2 off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
 #pragma unroll
@@ -215,9 +244,10 @@ __device__ __forceinline__ void short_stream(const ShortStreamParams& p, const i
                         }
                         const float sc = d * (float)(int)(int8_t)(scw >> (8 * k));
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) y[e] = fmaf(sc, c[e], y[e]);
+                        for (int e = 0; e < 4; ++e) half[s][e] = fmaf(sc, c[e], half[s][e]);
                     }
                 }
+            y = half[0] + half[1];
         }
         return y * ginv;
     };
@@ -235,8 +265,7 @@ __device__ __forceinline__ void short_stream(const ShortStreamParams& p, const i
         for (int l = wave; l < SS_AHEAD * p.groups; l += SS_WAVES) {
             const int a = l / p.groups, gr = l - a * p.groups, tile = (bx + (k0 + a) * wgx) * p.groups + gr;
             if (k0 + a >= turns || tile >= p.tiles) continue;
-            f32x4 y = buf[a * SS_WAVES + gr * p.ups][lane];
-            for (int w = 1; w < here; ++w) y += buf[a * SS_WAVES + gr * p.ups + w][lane];
+            const f32x4 y = ss_units<FOLD>(&buf[a * SS_WAVES + gr * p.ups], here, lane);
             int sg = 0;
             if (p.nseg > 1 && tile >= p.seg[1].tile0) sg = 1;
             if (p.nseg > 2 && tile >= p.seg[2].tile0) sg = 2;

@@ -327,3 +327,43 @@ def test_two_formats_over_one_workspace(qa, qb, T, ra, rb, inf):
             else:
                 got = y.numpy(np.float32).reshape(T, n).astype(np.float64)
             close(got, W, n64)
+
+
+# root mean square of the error over the products' size of the form with its planes in LDS, on these values: (normal ones, two draws; with eight channels a
+# hundred times the others', 24 draws: how far off such a sum is depends on which products the channels fall into)
+LDS_ERROR = {"Q4_K": (1.477e-7, 1.808e-7), "Q5_K": (1.501e-7, 1.805e-7), "Q6_K": (1.122e-7, 1.163e-7)}
+
+
+@pytest.mark.parametrize("qname", ["Q4_K", "Q5_K", "Q6_K"])
+def test_planes_in_registers_lose_no_precision(qname):
+    """the form with its planes in registers against 64 bits, by the mean over half a million products a draw: no further off than the other one"""
+    import torch
+    from ntransformer_amd import ops
+    T, rows, inf = 16, 28672, 4096
+    gt = getattr(G, "GGML_" + qname)
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[7, gt]))
+    dt = G.GGML_TO_DT[gt]
+    L.ntk_gemm_short_form.argtypes = [C.POINTER(C.c_int)] + [C.c_int] * 5
+    assert L.ntk_gemm_short_form((C.c_int * 1)(rows), 1, T, inf, dt, 1) == 2
+    raw, W, _ = weights(r, gt, rows, inf)
+    w = ops.rp_pack(DB.from_numpy(raw), rows, inf, dt)
+    W = torch.from_numpy(W).cuda()
+    nbytes = L.ntk_gemm_quant_workspace_bytes(inf, rows)
+    ws, y = DB.zeros(nbytes), DB.zeros(T * rows * 4)
+    square = [[], []]
+    for towers in [False] * 2 + [True] * 24:
+        X = r.standard_normal((T, inf)).astype(np.float32)
+        if towers:
+            X[:, r.permutation(inf)[:8]] *= np.float32(100)
+        Xd = DB.from_numpy(X)
+        _lib.check(L.ntk_short_prepare_x(Xd.ptr, T, inf, ws.ptr, None), "short_prepare_x")
+        segs = (_lib.GemvSeg * 1)()
+        segs[0].W, segs[0].y, segs[0].rows, segs[0].dtype = w.ptr, y.ptr, rows, dt
+        d = _lib.GemmDesc()
+        d.segs, d.nseg, d.n_tokens, d.in_features, d.weights_repacked, d.workspace, d.workspace_bytes = segs, 1, T, inf, 1, ws.ptr, nbytes
+        _lib.check(L.ntk_gemm_short(C.byref(d), 0, 0.0, 0, None), "gemm_short")
+        x = torch.from_numpy(X.astype(np.float64)).cuda()
+        err = (torch.from_numpy(y.numpy(np.float32).reshape(T, rows).astype(np.float64)).cuda() - x @ W.T) / torch.sqrt((x * x) @ (W * W).T)
+        square[towers].append(float((err * err).mean()))
+    got = [float(np.sqrt(np.mean(v))) for v in square]
+    assert got[0] <= LDS_ERROR[qname][0] and got[1] <= LDS_ERROR[qname][1], got
