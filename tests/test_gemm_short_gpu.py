@@ -367,3 +367,37 @@ def test_planes_in_registers_lose_no_precision(qname):
         square[towers].append(float((err * err).mean()))
     got = [float(np.sqrt(np.mean(v))) for v in square]
     assert got[0] <= LDS_ERROR[qname][0] and got[1] <= LDS_ERROR[qname][1], got
+
+
+@pytest.mark.parametrize("qname", ["Q4_K", "Q5_K", "Q6_K"])
+@pytest.mark.parametrize("rows,inf,form", [(33024, 1024, 2), (48, 1024, 1)])
+def test_values_that_are_none_stay_in_their_token(qname, rows, inf, form):
+    """NaN and infinities in some tokens, with the planes in registers and in LDS: those tokens' results are none either, the others' bits do not change"""
+    from ntransformer_amd import ops
+    T, gt = 9, getattr(G, "GGML_" + qname)
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[rows, gt]))
+    dt = G.GGML_TO_DT[gt]
+    L.ntk_gemm_short_form.argtypes = [C.POINTER(C.c_int)] + [C.c_int] * 5
+    assert L.ntk_gemm_short_form((C.c_int * 1)(rows), 1, T, inf, dt, 1) == form
+    raw = np.frombuffer(G.synth_tensor(r, gt, rows, inf), np.uint8)
+    w = ops.rp_pack(DB.from_numpy(raw), rows, inf, dt)
+    nbytes = L.ntk_gemm_quant_workspace_bytes(inf, rows)
+    ws, y = DB.zeros(nbytes), DB.zeros(T * rows * 4)
+
+    def go(X):
+        Xd = DB.from_numpy(X)
+        _lib.check(L.ntk_short_prepare_x(Xd.ptr, T, inf, ws.ptr, None), "short_prepare_x")
+        segs = (_lib.GemvSeg * 1)()
+        segs[0].W, segs[0].y, segs[0].rows, segs[0].dtype = w.ptr, y.ptr, rows, dt
+        d = _lib.GemmDesc()
+        d.segs, d.nseg, d.n_tokens, d.in_features, d.weights_repacked, d.workspace, d.workspace_bytes = segs, 1, T, inf, 1, ws.ptr, nbytes
+        _lib.check(L.ntk_gemm_short(C.byref(d), 0, 0.0, 0, None), "gemm_short")
+        return y.numpy(np.float32).reshape(T, rows)
+    X = r.standard_normal((T, inf)).astype(np.float32)
+    plain = go(X)
+    X[2, 700], X[4, 3], X[4, 4], X[8, inf - 1] = np.nan, np.inf, -np.inf, -np.inf
+    got = go(X)
+    bad = [2, 4, 8]
+    assert not np.isfinite(got[bad]).any()
+    good = [t for t in range(T) if t not in bad]
+    assert np.array_equal(got[good], plain[good])
