@@ -239,6 +239,7 @@ int ntk_rows_silu_mul_prepare_x(float* output, const ntk_gemm_partials* partials
  *   ntk_short_silu_mul_prepare_x  planes of silu(gate) * up of a deferred gate | up launch
  *   ntk_gemm_short                ntk_gemm_quant_f16 over such planes (desc->X and reuse_x are not looked at; NTK_E_SHAPE where ntk_gemm_short_takes says 0).  part_at: floats into the
  *                                 workspace's area of partial sums at which this launch's begin (a multiple of 4), so that several launches may leave theirs to one consumer
+ *                                 (ntk_gemm_short_form 2: a repack's results are summed in another order than its tensor's, else they are the same bits)
  * n_tokens <= 32, rows a multiple of 32 (NTK_E_SHAPE), 16-byte aligned pointers (NTK_E_ALIGN).  `workspace` must not be the one partials lie in.  Stream ordered, no allocation. */
 int ntk_gemm_short_takes(const int* rows, int nseg, int n_tokens, int in_features, int dtype);
 /* how it takes them: 1 the planes in LDS, 2 in registers (K-quants, many rows, up to 16 tokens); 0 not at all */

@@ -705,9 +705,11 @@ int Model::layers_short(int T, int start_pos, int first, int last_layer) {
     float* up_buf = gate_buf + (size_t)T * I;
     void* ws = gemm_ws_;
     auto other = [&]() { ws = ws == gemm_ws_ ? gemm_ws2_ : gemm_ws_; return ws; };
+    // (the repack wherever it is there, the file's blocks beside it or not: up to 16 tokens of many rows are multiplied in another order from it, and a prompt's bits are to be the same either way.
+    // us, both copies resident, 16 tokens, sixteen 8B layers in Q4_K_M 1542 / 1329, eight in Q6_K 953 / 800)
     auto repacked = [&](const DevTensor* const* Ws, int n) {
         bool rp = true;
-        for (int i = 0; i < n; ++i) rp = rp && !Ws[i]->ptr && Ws[i]->rp && Ws[i]->dtype != NTK_DT_Q8_0 && Ws[i]->dtype != NTK_DT_Q4_0;
+        for (int i = 0; i < n; ++i) rp = rp && Ws[i]->rp && Ws[i]->dtype != NTK_DT_Q8_0 && Ws[i]->dtype != NTK_DT_Q4_0;
         return rp;
     };
     auto describe = [&](const DevTensor* const* Ws, float* const* Ys, int n, const float* resid, ntk_gemm_partials* pt, bool rp, ntk_gemv_seg (&segs)[3]) {
