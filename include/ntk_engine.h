@@ -251,6 +251,8 @@ int ntk_gemm_short(const ntk_gemm_desc* desc, int normed, float eps, size_t part
 /* ntk_gemm_short of a, then of b with its partial sums behind a's: matrices of two formats over the same planes, in one launch where one of them has many rows and that is estimated to be ahead
  * (repacked K-quants, sums left) */
 int ntk_gemm_short_two(const ntk_gemm_desc* a, const ntk_gemm_desc* b, int normed, float eps, size_t part_at, void* stream);
+/* 1: it does these two in one launch, 0: one after the other */
+int ntk_gemm_short_two_joins(const ntk_gemm_desc* a, const ntk_gemm_desc* b, size_t part_at);
 /* A prompt of at most 32 tokens from position 0 on: ntk_reduce_rope_kv_store, ntk_attention_prefill and ntk_short_prepare_x of its result in one launch.  sums / splits: of q, k and v as in
  * ntk_reduce_rope_kv_store; angles: ntk_short_angles' table (ntk_short_angles_bytes, 16-byte aligned), formed once a model.  head_dim 128, an even number of heads (NTK_E_SHAPE). */
 size_t ntk_short_angles_bytes(int head_dim);

@@ -2892,36 +2892,48 @@ static size_t left_behind(const ntk_gemm_partials* p) {
         for (int i = 0; i < p->nseg; ++i) n += (size_t)p->nsplit * p->n_tokens * p->rows[i];
     return n;
 }
-int ntk_gemm_short_two(const ntk_gemm_desc* a, const ntk_gemm_desc* b, int normed, float eps, size_t part_at, void* stream) {
-    if (!a || !b) return NTK_E_NULL;
+// one launch for both: what it is launched with (false: one launch after the other)
+extern "C++" { namespace {
+struct PairLaunch { PairSide sa, sb; bool turned; ntk::ShortStreamPlan plo, phi; size_t cap; };
+bool pair_launch(const ntk_gemm_desc* a, const ntk_gemm_desc* b, size_t part_at, PairLaunch* o) {
     const int T = a->n_tokens, in = a->in_features;
     const bool like = a->segs && b->segs && a->nseg >= 1 && b->nseg >= 1 && a->nseg <= ntk::GB_MAX_SEG && b->nseg <= ntk::GB_MAX_SEG && a->weights_repacked && b->weights_repacked && a->partials &&
                       b->partials && !a->resid && !b->resid && a->workspace && a->workspace == b->workspace && a->workspace_bytes == b->workspace_bytes && b->n_tokens == T && b->in_features == in &&
                       T >= 2 && T <= ntk::SS_TOKENS && in > 0 && in % 256 == 0 && part_at % 4 == 0 && !(reinterpret_cast<uintptr_t>(a->workspace) & 15);
-    PairSide sa, sb;
     // (where one of them takes gemm_short.hip's form by itself: matrices too small for that keep the other form, whose sums are the same from a tensor and from its repack)
-    if (like && pair_side(a, &sa) && pair_side(b, &sb) && sa.dt != sb.dt && (sa.own.n > 0 || sb.own.n > 0)) {
-        const bool turned = sa.dt > sb.dt;
-        PairSide &lo = turned ? sb : sa, &hi = turned ? sa : sb;
-        ntk::ShortStreamPlan plo, phi;
-        const size_t head = ntk::ws_part_offset((in + 31) / 32 * 32), cap = a->workspace_bytes > head ? (a->workspace_bytes - head) / sizeof(float) : 0;
-        if (a->workspace_bytes >= ntk_gemm_quant_workspace_bytes(in, sa.rows + sb.rows) &&
-            ntk::short_stream_plan_two(lo.dt, hi.dt, in / 256, lo.rows / 16, hi.rows / 16, std::min(lo.lds.n, hi.lds.n), lo.own.us + hi.own.us, &plo, &phi) &&
-            part_at + (size_t)plo.n * T * (size_t)(sa.rows + sb.rows) <= cap) {
-            ntk::ShortArgs sh;
-            sh.on = true; sh.norm = normed != 0; sh.eps = eps; sh.part_at = part_at; sh.part_cap = cap;
-            ntk::ShortStreamParams q[2] = {};
-            const float* parts[2][ntk::GB_MAX_SEG] = {};
-            uint8_t* ws = static_cast<uint8_t*>(a->workspace);
-            pair_params(lo, &q[0], T, in, plo, ws, sh, parts[0]);
-            if (plo.n > 1) sh.part_at += (size_t)plo.n * T * (size_t)lo.rows;
-            pair_params(hi, &q[1], T, in, phi, ws, sh, parts[1]);
-            hipStream_t st = ntk::resolve_stream(stream);
-            const int rc = ntk::short_stream_launch_two(lo.dt, hi.dt, q[0], q[1], plo, phi, st);
-            if (rc != NTK_OK) return rc;
-            ntk::leave_slices(lo.segs, lo.nseg, parts[0], plo.n, T, nullptr, (turned ? b : a)->partials, st);
-            return ntk::leave_slices(hi.segs, hi.nseg, parts[1], phi.n, T, nullptr, (turned ? a : b)->partials, st);
-        }
+    if (!like || !pair_side(a, &o->sa) || !pair_side(b, &o->sb) || o->sa.dt == o->sb.dt || (o->sa.own.n == 0 && o->sb.own.n == 0)) return false;
+    o->turned = o->sa.dt > o->sb.dt;
+    const PairSide &lo = o->turned ? o->sb : o->sa, &hi = o->turned ? o->sa : o->sb;
+    const size_t head = ntk::ws_part_offset((in + 31) / 32 * 32);
+    o->cap = a->workspace_bytes > head ? (a->workspace_bytes - head) / sizeof(float) : 0;
+    return a->workspace_bytes >= ntk_gemm_quant_workspace_bytes(in, lo.rows + hi.rows) &&
+           ntk::short_stream_plan_two(lo.dt, hi.dt, in / 256, lo.rows / 16, hi.rows / 16, std::min(lo.lds.n, hi.lds.n), lo.own.us + hi.own.us, &o->plo, &o->phi) &&
+           part_at + (size_t)o->plo.n * T * (size_t)(lo.rows + hi.rows) <= o->cap;
+}
+} }  // namespace
+int ntk_gemm_short_two_joins(const ntk_gemm_desc* a, const ntk_gemm_desc* b, size_t part_at) {
+    PairLaunch pl;
+    return a && b && pair_launch(a, b, part_at, &pl) ? 1 : 0;
+}
+int ntk_gemm_short_two(const ntk_gemm_desc* a, const ntk_gemm_desc* b, int normed, float eps, size_t part_at, void* stream) {
+    if (!a || !b) return NTK_E_NULL;
+    PairLaunch pl;
+    if (pair_launch(a, b, part_at, &pl)) {
+        const PairSide &lo = pl.turned ? pl.sb : pl.sa, &hi = pl.turned ? pl.sa : pl.sb;
+        const int T = a->n_tokens, in = a->in_features;
+        ntk::ShortArgs sh;
+        sh.on = true; sh.norm = normed != 0; sh.eps = eps; sh.part_at = part_at; sh.part_cap = pl.cap;
+        ntk::ShortStreamParams q[2] = {};
+        const float* parts[2][ntk::GB_MAX_SEG] = {};
+        uint8_t* ws = static_cast<uint8_t*>(a->workspace);
+        pair_params(lo, &q[0], T, in, pl.plo, ws, sh, parts[0]);
+        if (pl.plo.n > 1) sh.part_at += (size_t)pl.plo.n * T * (size_t)lo.rows;
+        pair_params(hi, &q[1], T, in, pl.phi, ws, sh, parts[1]);
+        hipStream_t st = ntk::resolve_stream(stream);
+        const int rc = ntk::short_stream_launch_two(lo.dt, hi.dt, q[0], q[1], pl.plo, pl.phi, st);
+        if (rc != NTK_OK) return rc;
+        ntk::leave_slices(lo.segs, lo.nseg, parts[0], pl.plo.n, T, nullptr, (pl.turned ? b : a)->partials, st);
+        return ntk::leave_slices(hi.segs, hi.nseg, parts[1], pl.phi.n, T, nullptr, (pl.turned ? a : b)->partials, st);
     }
     const int rc = ntk_gemm_short(a, normed, eps, part_at, stream);
     return rc != NTK_OK ? rc : ntk_gemm_short(b, normed, eps, part_at + left_behind(a->partials), stream);

@@ -401,3 +401,55 @@ def test_values_that_are_none_stay_in_their_token(qname, rows, inf, form):
     assert not np.isfinite(got[bad]).any()
     good = [t for t in range(T) if t not in bad]
     assert np.array_equal(got[good], plain[good])
+
+
+@pytest.mark.parametrize("qa,qb", [("Q4_K", "Q6_K"), ("Q4_K", "Q5_K"), ("Q5_K", "Q6_K")])
+@pytest.mark.parametrize("turned", [False, True])
+@pytest.mark.parametrize("T,ra,rb,inf,at,joins", [(16, (4096, 1024), (1024,), 4096, 0, 1), (2, (4096, 1024), (1040,), 4096, 512, 1), (16, (64,), (32,), 512, 0, 0), (17, (4096, 1024), (1024,), 4096, 64, 0)])
+def test_two_formats_in_one_launch(qa, qb, turned, T, ra, rb, inf, at, joins):
+    """every pair of formats in both orders: in one launch and, for matrices too small and for 17 tokens, in two -- asked for, so that the launch is not left untested; sums behind others in their area"""
+    from ntransformer_amd import ops
+    L, r = lib(), np.random.Generator(np.random.Philox(key=[T + at, sum(ra) + inf]))
+    L.ntk_gemm_short_two.argtypes = [C.POINTER(_lib.GemmDesc)] * 2 + [C.c_int, C.c_float, C.c_size_t, VP]
+    L.ntk_gemm_short_two_joins.argtypes = [C.POINTER(_lib.GemmDesc)] * 2 + [C.c_size_t]
+    if turned:
+        qa, qb = qb, qa
+    nbytes = L.ntk_gemm_quant_workspace_bytes(inf, 4 * (sum(ra) + sum(rb)))
+    ws, eps = DB.zeros(nbytes), 1e-5
+    X, nw = r.standard_normal((T, inf)).astype(np.float32), (1.0 + 0.1 * r.standard_normal(inf)).astype(np.float32)
+    xd, nd = DB.from_numpy(X), DB.from_numpy(nw)
+    _lib.check(L.ntk_short_norm_prepare_x(xd.ptr, None, nd.ptr, T, inf, ws.ptr, None), "short_norm")
+    x64 = X.astype(np.float64)
+    n64 = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + eps) * nw
+    sides, keep = [], []
+    for q, rows in ((qa, ra), (qb, rb)):
+        mats, pt, segs = [], _lib.GemmPartials(), (_lib.GemvSeg * len(rows))()
+        for s, n in zip(segs, rows):
+            raw, W, dt = weights(r, getattr(G, "GGML_" + q), n, inf)
+            w, y = ops.rp_pack(DB.from_numpy(raw), n, inf, dt), DB.from_numpy(np.full((T, n), 7.0, np.float32))
+            s.W, s.y, s.rows, s.dtype = w.ptr, y.ptr, n, dt
+            mats.append((W, y, n))
+            keep.append(w)
+        if not L.ntk_gemm_short_takes((C.c_int * len(rows))(*rows), len(rows), T, inf, dt):
+            assert T > 16 and q == "Q6_K"
+            pytest.skip("32 tokens of the format that scales per 16 columns")
+        d = _lib.GemmDesc()
+        d.segs, d.nseg, d.n_tokens, d.in_features, d.weights_repacked = segs, len(rows), T, inf, 1
+        d.workspace, d.workspace_bytes, d.partials = ws.ptr, nbytes, C.pointer(pt)
+        sides.append((d, pt, mats, segs))
+    a, b = C.byref(sides[0][0]), C.byref(sides[1][0])
+    assert L.ntk_gemm_short_two_joins(a, b, at) == joins
+    before = ws.numpy(np.float32)
+    _lib.check(L.ntk_gemm_short_two(a, b, 1, eps, at, None), "gemm_short_two")
+    whole, first = ws.numpy(np.float32), None
+    for d, pt, mats, _ in sides:
+        for k, (W, y, n) in enumerate(mats):
+            if pt.nsplit > 1:
+                place = (pt.part[k] - ws.ptr) // 4
+                first = place if first is None else min(first, place)
+                got = whole[place:place + pt.nsplit * T * n].reshape(pt.nsplit, T, n).astype(np.float64).sum(0)
+            else:
+                got = y.numpy(np.float32).reshape(T, n).astype(np.float64)
+            close(got, W, n64)
+    if first is not None and at:
+        assert np.array_equal(whole[first - at:first], before[first - at:first])      # (what lies in front in that area)
