@@ -225,7 +225,8 @@ struct SharedArgs {
 // counts where many rows walk a long context.  us with the merge, 8 tokens of 64 heads at 8000 positions, tile in LDS / so: 32 + 8 121 / 43, 256 + 32 157 / 95, 512 + 64 400 / 193.
 // ROUTE: the first `beside` rows of the grid's workgroups choose a token's experts each (route_token), which waits for nothing that attention leaves.  Attention of one token leaves most
 // CUs idle and takes about as long: us, 16 heads, 512 + 64, 1100 positions, and a router of 32 experts of 2048 inputs: 9.6 + 8.7 in two launches, 10.8 so (12.5 with four rows
-// of the router a wave, requested behind the norm).
+// of the router a wave, requested behind the norm).  Five rows a wave are one round for up to 40 rows; with more the launch gains less, but it gains: with the unfolding behind it, two launches / so, 16 .. 39
+// experts 1.5, 64 23.8 / 16.5, 128 29.2 / 23.8, 256 39.7 / 35.1; of 4096 inputs 256 57.4 / 56.2; over 1, 2 and 8 tokens at 40, 1100 and 8000 positions 1.00 .. 1.60.
 struct NoRoute {};
 struct RouteBeside { RouteJob job; int T, rows; };
 constexpr int kRouteBesideInputs = 4096;

@@ -180,13 +180,24 @@ __device__ __forceinline__ void route_token(const RouteJob& j, long long t, floa
         if (e < E) z[e] = s;
         else if (j.sgate) j.sgate[t] = 1.0f / (1.0f + expf(-s));
     };
-    if (vec) {
+    if (vec && EA == 1) {
+        for (int e = wave; e < rows; e += WAVES) {
+            const float* w = row(e);
+            float s = 0.0f;
+#pragma unroll 4
+            for (int k = lane * 4; k < n; k += 256) {
+                const float4 a4 = *reinterpret_cast<const float4*>(w + k), x4 = *reinterpret_cast<const float4*>(xs + k);
+                s = fmaf(a4.x, x4.x, s); s = fmaf(a4.y, x4.y, s); s = fmaf(a4.z, x4.z, s); s = fmaf(a4.w, x4.w, s);
+            }
+            leave(e, s);
+        }
+    } else if (vec) {
         for (int e0 = wave; e0 < rows; e0 += EA * WAVES) {       // (uniform over the wave)
             float s[EA];
 #pragma unroll
             for (int i = 0; i < EA; ++i) s[i] = 0.0f;
             for (int k0 = lane * 4; k0 < n; k0 += 256 * KA) {
-                if (EA == 1 || e0 > wave || k0 > lane * 4) request(e0, k0);
+                if (e0 > wave || k0 > lane * 4) request(e0, k0);
 #pragma unroll
                 for (int u = 0; u < KA; ++u) {
                     if (k0 + 256 * u >= n) break;
