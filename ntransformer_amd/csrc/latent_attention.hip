@@ -254,13 +254,24 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
     const int last_row = min(row0 + SROWS, n_rows) - 1;
     const int pmin = a.pos0 + row0 / a.H, pmax = a.pos0 + last_row / a.H;
     const int jlo = a.window > 0 ? max(0, pmin - a.window + 1) : 0, jhi = pmax;
-    auto four = [](const float* p, int at, int end) -> f4 {         // entries at .. at + 3 of a row of `end`, zero behind it
+    // entries at .. at + 3 of a row of `end`, zero behind it: asked for, and what was asked for as it is used.  As they lie (V); else every request goes out unconditionally and what does not count is moved or zeroed
+    // when it is used: keys of up to 128 entries one by one, past the end the last one again; longer ones in fours, a row's last entries with the four that end it.  (Requests under conditions were waited
+    // for one after the other.  us with merge and unfolding, the tile in LDS / those / so: 9 entries at 172 positions 10.6 / 12.9 / 11.5, 255 + 30 at 128 17.2 / 15.0 / 13.8)
+    constexpr bool SINGLE = !V && KS == 2;
+    auto ask = [](const float* p, int at, int end) -> f4 {
         f4 v{0.f, 0.f, 0.f, 0.f};
         if constexpr (V) { if (at < end) v = *reinterpret_cast<const f4*>(p + at); }
-        else if (at + 4 <= end) v = *reinterpret_cast<const f4_anywhere*>(p + at);
-        else if (at < end)
-            for (int c = 0; c < 4; ++c) if (at + c < end) v[c] = p[at + c];
+        else if constexpr (!SINGLE) v = *reinterpret_cast<const f4_anywhere*>(p + min(at, max(end, 4) - 4));          // (end < 4: a rank beside rotated entries, which are four at least together)
+        else
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = p[min(at + c, end - 1)];
         return v;
+    };
+    auto put = [](const f4& w, int at, int end) -> f4 {
+        if constexpr (V) return w;
+        else if constexpr (SINGLE) return f4{at < end ? w[0] : 0.f, at + 1 < end ? w[1] : 0.f, at + 2 < end ? w[2] : 0.f, at + 3 < end ? w[3] : 0.f};
+        const int back = at - min(at, max(end, 4) - 4);                 // (past a rank below four: columns that nothing reads)
+        return back == 0 ? w : back == 1 ? f4{w[1], w[2], w[3], 0.f} : back == 2 ? f4{w[2], w[3], 0.f, 0.f} : back == 3 ? f4{w[3], 0.f, 0.f, 0.f} : f4{0.f, 0.f, 0.f, 0.f};
     };
     // (keys past the last re-read it; their weight is zero)
     f4 qf[KS], kf[KS][2], vf[2][4];
@@ -269,7 +280,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
 #pragma unroll
         for (int u = 0; u < KS; ++u) {
             const int st = wave + NW * u;
-            if (st < steps) { kf[u][0] = four(k0, 16 * st + 4 * g4, DK); kf[u][1] = four(k1, 16 * st + 4 * g4, DK); }
+            if (st < steps) { kf[u][0] = ask(k0, 16 * st + 4 * g4, DK); kf[u][1] = ask(k1, 16 * st + 4 * g4, DK); }
         }
     };
     const bool sums = 64 * wave < a.R;             // (uniform over the wave)
@@ -278,7 +289,7 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
 #pragma unroll
         for (int e = 0; e < 2; ++e)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) vf[e][c] = four(a.cache + (long long)min(j0 + 16 * e + 4 * g4 + c, jhi) * a.row, col, a.R);
+            for (int c = 0; c < 4; ++c) vf[e][c] = ask(a.cache + (long long)min(j0 + 16 * e + 4 * g4 + c, jhi) * a.row, col, a.R);
     };
     int j0 = jlo + KB * part;
     const int hop = KB * a.splits;
@@ -287,9 +298,13 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
         const float* q = a.q + (long long)(r / a.H) * a.ldq + (long long)(r % a.H) * DK;
 #pragma unroll
         for (int u = 0; u < KS; ++u)
-            if (wave + NW * u < steps) qf[u] = four(q, 16 * (wave + NW * u) + 4 * g4, DK);
+            if (wave + NW * u < steps) qf[u] = ask(q, 16 * (wave + NW * u) + 4 * g4, DK);
     }
     if (j0 <= jhi) { load_keys(j0); load_values(j0); }
+    if constexpr (!V)
+#pragma unroll
+        for (int u = 0; u < KS; ++u)
+            if (wave + NW * u < steps) qf[u] = put(qf[u], 16 * (wave + NW * u) + 4 * g4, DK);
     if (tid < SROWS) { ms[tid] = -INFINITY; ls[tid] = 0.0f; }
     const int srow = tid / TPR, sub = tid % TPR;
     const int rpos = row0 + srow < n_rows ? a.pos0 + (row0 + srow) / a.H : -1;
@@ -304,10 +319,12 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
 #pragma unroll
         for (int u = 0; u < KS; ++u) {
             if (wave + NW * u >= steps) continue;  // (uniform over the wave)
+            const int at = 16 * (wave + NW * u) + 4 * g4;
+            const f4 k0 = put(kf[u][0], at, DK), k1 = put(kf[u][1], at, DK);
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], kf[u][0][c], s0, 0, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], kf[u][1][c], s1, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], k0[c], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[u][c], k1[c], s1, 0, 0, 0);
             }
         }
         if (more) load_keys(j0 + hop);
@@ -366,12 +383,14 @@ __global__ __launch_bounds__(64 * NW) void latent_attention_shared_kernel(const 
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[t][r] *= corr[r];
 #pragma unroll
-            for (int c = 0; c < 4; ++c)            // component c of the weights belongs to key 4 g4 + c
+            for (int c = 0; c < 4; ++c) {          // component c of the weights belongs to key 4 g4 + c
+                const f4 v0 = put(vf[0][c], col, a.R), v1 = put(vf[1][c], col, a.R);
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[c], vf[0][c][t], acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[c], vf[1][c][t], acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p0[c], v0[t], acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[c], v1[t], acc[t], 0, 0, 0);
                 }
+            }
             if (more) load_values(j0 + hop);
         }
     }

@@ -164,3 +164,10 @@ def test_latent_values_that_are_not_finite_stay_with_the_rows_that_see_them(what
     hit = np.zeros(got.shape, bool)
     hit[77 - pos0:77 - pos0 + 42, 1, 20] = True
     assert np.abs(got[~hit] - want[~hit]).max() < 2e-5 * np.abs(clean).max() and not np.isfinite(got[hit]).any()
+
+
+@pytest.mark.parametrize("R,dr", [(1, 0), (2, 2), (3, 0), (3, 126), (2, 400), (9, 0), (31, 6), (125, 3), (127, 2), (255, 30), (510, 30), (511, 300)])
+@pytest.mark.parametrize("T,H,pos0,window", [(1, 3, 0, 0), (2, 8, 33, 0), (3, 5, 700, 90)])
+def test_shared_latents_of_rows_off_four_entries(R, dr, H, T, pos0, window):
+    """rows that are no whole fours: entry by entry (up to 128) and in fours with the last ones moved, ranks below four beside rotated entries"""
+    test_decoded_tokens_over_shared_latents_at_the_edges(R, dr, H, T, pos0, window)
