@@ -530,8 +530,7 @@ def test_other_sizes(tmp_path, name):
 
 
 def test_long_decoding_and_a_prompt_longer_than_one_internal_pass(tmp_path):
-    """1100 tokens are two internal passes: the blended values are those of each pass's own tokens, the convolutions and the state carry across; then 200 tokens
-    one by one across several chunk edges"""
+    """1100 tokens in one internal pass (beyond one: test_long_portions_gpu.py); then 200 tokens one by one across several chunk edges, the convolutions and the state carried"""
     cfg = O.config([O.attention_layer(size=88), O.delta_layer(), O.attention_layer(size=200), O.latent_layer(ff=0)])
     folder, w = make(tmp_path, cfg, seed=9)
     toks = tokens_for(cfg, 1100, seed=10)

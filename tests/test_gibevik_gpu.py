@@ -647,7 +647,7 @@ def test_other_sizes(tmp_path, name):
 
 
 def test_long_decoding_and_a_prompt_longer_than_one_internal_pass(tmp_path):
-    """1100 tokens are two internal passes: positions, temperature and latents of the second go on from the first; then 200 tokens one by one"""
+    """1100 tokens in one internal pass (beyond one: test_long_portions_gpu.py); then 200 tokens one by one: positions, temperature and latents go on from the prompt's"""
     cfg = O.config([O.layer_attention(every=100, mlp=O.dense()), O.layer_latent(mlp=O.moe(4, 2, 12, identity=1, shared=12)), O.layer_latent(kv_from=1, heads=2)])
     folder, w = make(tmp_path, cfg, seed=9)
     toks = tokens_for(cfg, 1100, seed=10)

@@ -54,6 +54,47 @@ def test_a_prompt_beyond_one_internal_pass(tmp_path, monkeypatch, family):
     e.close()
 
 
+# What the first ones leave out: a mixture and a layer over another's latents, a layer without cache rows of its own at the end, a window on latents, a token's choices that halve the pass (9 of 12 experts: 2048
+# tokens).  bfloat16: sizes of whole chunks, so that norms and gates leave rounded rows and products read them (ntk_dense_direct_ahead), over a whole pass and across its edge.
+MORE = {
+    "gibevik": ("float32", gibevik_oracle, lambda O: O.config([O.layer_attention(every=100, mlp=O.dense()), O.layer_latent(mlp=O.moe(4, 2, 12, identity=1, shared=12)), O.layer_latent(kv_from=1, heads=2)])),
+    "zalazen": ("float32", zalazen_oracle, lambda O: O.config([O.layer(size=88, kept=4), O.layer(size=200, kept=1), O.layer(size=30, kept=7, kv_from=0), O.layer(size=0, kv_from=1, ff=0)])),
+    "fabolorn": ("float32", fabolorn_oracle, lambda O: O.small_config(window=70, layers=("latent_attention", "latent_attention_2"))),
+    "fabolorn, nine choices": ("float32", fabolorn_oracle, lambda O: O.small_config(window=70, experts=12, top=9)),
+    "fifotar, bfloat16": ("bfloat16", fifotar_oracle, lambda O: O.config([O.attention_layer(size=88, dim=16, vdim=16, ff=64), O.delta_layer(dim=16, vdim=16, ff=64),
+                                                                         O.latent_layer(heads=4, dim=16, vdim=16, rot_dim=8, kv_rank=64, q_rank=64, ff=64)], width=64)),
+    "fabolorn, bfloat16": ("bfloat16", fabolorn_oracle, lambda O: O.small_config(window=70, heads=4, dim=16, vdim=16, kv_rank=64, q_rank=64, mlp_on=(False, False))),
+}
+
+
+@pytest.mark.parametrize("case", list(MORE))
+def test_a_prompt_beyond_one_internal_pass_and_tokens_behind_it(tmp_path, case):
+    from ntransformer_amd import _lib
+    from ntransformer_amd.engine import Engine
+    dtype, O, config = MORE[case]
+    cfg = config(O)
+    w = O.random_weights(cfg, 9)
+    O.save_model(str(tmp_path / "m"), cfg, w)
+    toks = [int(t) for t in np.random.default_rng(11).integers(0, cfg["vocab"], N + 4)]
+    ref = O.forward(cfg, w, toks)
+    ref = np.asarray(ref[0] if isinstance(ref, tuple) else ref, np.float64)
+    tol = TOL if dtype == "float32" else 4e-2          # (the families' own)
+    if dtype == "bfloat16":
+        f = _lib.lib().ntk_dense_direct_ahead
+        f.argtypes, f.restype = [C.c_int] * 4 + [C.c_size_t], C.c_int
+        assert f(PASS, 64, 64, 0, 1 << 24) == f(PASS, 64, 64, 1, 1 << 24) == 1
+    rel = lambda got, at: float(np.sqrt(np.mean((got - ref[at]) ** 2)) / np.sqrt(np.mean(ref[at] ** 2)))
+    want = [0, 1023, 1024, 2047, 2048, PASS - 1, PASS, N - 1]
+    e = Engine()
+    e.load_folder(str(tmp_path / "m"), max_context=4400, dtype=dtype)
+    s = e.seq_acquire()
+    got = e.seq_forward(s, toks[:N], want=want)
+    assert max(rel(got[k:k + 1], at) for k, at in enumerate(want)) < 3 * tol and rel(got, want) < tol
+    for k in range(N, N + 4):
+        assert rel(e.seq_forward(s, [toks[k]]), [k]) < 3 * tol
+    e.close()
+
+
 def _left_of(L, most):
     """what is left of the malloc budget, to the byte"""
     left, held = 0, []

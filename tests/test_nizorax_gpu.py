@@ -519,7 +519,7 @@ def test_long_decoding_from_one_token(tmp_path):
 
 
 def test_a_long_prompt_in_several_internal_passes(tmp_path):
-    """more tokens than one internal pass holds: the cache rows, the recurrent state and the convolution inputs go from pass to pass"""
+    """1100 tokens in one internal pass (beyond one: test_long_portions_gpu.py): rows on both sides of 1024"""
     cfg = O.small_config(layers=("attention", "lightning"), mlps=("dense", None), window=200, width=32, ff=40, vocab=40)
     folder, w = make(tmp_path, cfg, seed=19)
     e = engine_for(folder, ctx=1400)

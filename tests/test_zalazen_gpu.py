@@ -468,7 +468,7 @@ def test_other_sizes(tmp_path, name):
 
 
 def test_long_decoding_and_a_prompt_longer_than_one_internal_pass(tmp_path):
-    """1100 tokens are two internal passes: the token before the second pass, the shared rows and the kept positions come from the first; then 200 tokens one by one
+    """1100 tokens in one internal pass (beyond one: test_long_portions_gpu.py); then 200 tokens one by one
     far behind the kept positions, several windows long"""
     cfg = O.config([O.layer(size=88, kept=4), O.layer(size=200, kept=1), O.layer(size=30, kept=7, kv_from=0), O.layer(size=0, kv_from=1, ff=0)])
     folder, w = make(tmp_path, cfg, seed=9)
