@@ -339,15 +339,7 @@ __global__ __launch_bounds__(64) void store_words_kernel(int* __restrict__ a, in
     if (i < na) a[i] = w.v[i];
     else b[i - na] = w.v[i];
 }
-__global__ __launch_bounds__(256) void copy_out_kernel(uint32_t* __restrict__ out, const uint32_t* __restrict__ src, size_t words, int wide) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (wide) {
-        if (4 * i + 3 < words) *reinterpret_cast<uint4*>(out + 4 * i) = *reinterpret_cast<const uint4*>(src + 4 * i);
-        else
-            for (size_t k = 4 * i; k < words; ++k) out[k] = src[k];
-    } else if (i < words) out[i] = src[i];
-}
-// a piece a workgroup: its stores are out (system scope) in front of its word
+// a piece a workgroup: its stores are out (system scope) in front of its word (there NULL: no words, the stream is waited for)
 __global__ __launch_bounds__(256) void copy_out_pieces_kernel(uint32_t* __restrict__ out, const uint32_t* __restrict__ src, size_t words, int wide, unsigned* __restrict__ there, unsigned turn, int* __restrict__ bump) {
     const size_t at = (size_t)blockIdx.x * NTK_COPY_OUT_PIECE, end = min(words, at + NTK_COPY_OUT_PIECE);
     if (bump && blockIdx.x == 0 && threadIdx.x == 0) *bump += 1;
@@ -359,6 +351,7 @@ __global__ __launch_bounds__(256) void copy_out_pieces_kernel(uint32_t* __restri
         }
     } else
         for (size_t i = at + threadIdx.x; i < end; i += 256) out[i] = src[i];
+    if (!there) return;
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(there + blockIdx.x, turn, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -382,9 +375,8 @@ int ntk_copy_out(void* pinned, const void* src, size_t size, void* stream) {
     if (size % 4 || size / 4 > (size_t)0x7FFFFFFF * 256) return NTK_E_SHAPE;
     if (at & 3) return NTK_E_ALIGN;
     if (size == 0) return NTK_OK;
-    const int wide = (at & 15) == 0;
-    const size_t words = size / 4, threads = wide ? (words + 3) / 4 : words;
-    hipLaunchKernelGGL(copy_out_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, resolve_stream(stream), static_cast<uint32_t*>(pinned), static_cast<const uint32_t*>(src), words, wide);
+    hipLaunchKernelGGL(copy_out_pieces_kernel, dim3((unsigned)ntk_copy_out_words(size / 4)), dim3(256), 0, resolve_stream(stream), static_cast<uint32_t*>(pinned), static_cast<const uint32_t*>(src),
+                       size / 4, (int)((at & 15) == 0), static_cast<unsigned*>(nullptr), 0u, static_cast<int*>(nullptr));
     return last_launch_status();
 }
 
