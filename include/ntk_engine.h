@@ -287,8 +287,8 @@ typedef struct ntk_half_desc {
 } ntk_half_desc;
 size_t ntk_gemm_half_many_bytes(int n_tokens, int in_features);
 int ntk_gemm_half_many(const ntk_half_desc* d, void* stream);
-/* how one pass of it goes, with room floats behind the halves (silu: gated, 0): plan = {rows, columns of a tile, tiles a CU holds at once, pieces of K} */
-int ntk_gemm_half_plan(int rows, int N, int K, int gated, long long room, int* plan);
+/* how one pass of it goes, with room floats behind the halves (silu: 0): plan = {rows, columns of a tile, tiles a CU holds at once, pieces of K} */
+int ntk_gemm_half_plan(int rows, int N, int K, long long room, int* plan);
 /* ... with a norm between two of them and no row in between.  ntk_gemm_half_defer: ntk_gemm_half with accumulate that may leave its pieces of K to the launch behind it (partials: as those of
  * ntk_gemm_quant_f16; they lie in the workspace).  ntk_half_norm_split: hidden += that projection (partials; NULL: hidden as it lies), and the halves of its RMSNorm into `workspace` (another one), from
  * which ntk_gemm_half_normed is ntk_gemm_half_many (X, row_max not looked at; no unit's sums are left).  ntk_half_norm_takes: 1 where the workspace holds all tokens (width a multiple of 64, up to 16384), else 0. */

@@ -724,7 +724,7 @@ constexpr float kRoundUs = 3.5f, kRoundRate = 4e6f;     // the launch that round
 static const DirectForm kFormsBf16[] = {{256, 256, 1, 1.45f, 1.45f, 12.0f}, {256, 128, 1, 0.84f, 0.84f, 9.0f}, {128, 256, 1, 0.85f, 0.85f, 9.0f}, {128, 128, 2, 0.72f, 0.475f, 7.0f},
                                         {128, 128, 1, 0.50f, 0.57f, 7.0f}, {64, 128, 2, 0.42f, 0.35f, 5.0f}, {64, 64, 3, 0.33f, 0.22f, 4.0f}};
 static TilePlan plan_direct_bf16(int rows, int groups, int N, int K, long long room) {
-    return plan_direct(kFormsBf16, 7, 64, rows, groups, N, K, room, groups == 1 ? 1.05f : 0.0f);
+    return plan_direct(kFormsBf16, 7, 64, rows, groups, N, K, room, groups == 1);
 }
 // float32: K in chunks of 32; one form, ahead of larger and smaller tiles and other splits of the tile over waves at the sizes they were tried at (12 .. 200 rows, 900 in 32 groups).  Over 337
 // grouped sizes it takes 0.89 of gemm_tile.hip.h's time on average and is 3 .. 17 % behind it at about eleven (40 rows in 128 groups, 300 in 8 or 16).  us, the form of gemm_tile.hip.h

@@ -288,13 +288,14 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void gemm_direct_kernel(const D
 // that come from memory; the estimate is within a sixth there, and the choice within a tenth of the best form but for uneven small groups.  Rows of several groups: tiles
 // of a group of the average size, plus half a tile where that is no small part of one.
 struct DirectForm { int TM, TN, resident; float alone, busy, over, even; };       // even: the part of a chunk's time that goes with the rows a tile has (rows evenly over the tiles)
-// rounds > 0 (one matrix): a second estimate has a CU's last tiles, where they are no whole number of `resident` ones, at the pace of a tile alone, and looks at five pieces where six put a second
-// tile on a CU.  What it names is taken where it puts the plan of the first estimate behind by that factor, and `us` stays the first estimate's (the lines between these forms and others are drawn with
-// it).  The second estimate is no better than a few per cent: taken wherever it differs, of 250 sizes each it was up to 13 % behind in bfloat16, up to 26 % in gated units, up to 9 % with halves
-// (158 x 2048 x 7488); from 1.05, 1.05 and 1.08 on never by more than 2 %.  Those that are taken, us before / so: bfloat16 700 x 4096 x 14336 97 / 88, 1500 x 4096 x 14336 229 / 179, gated 1181 x 7488 x 7488
-// 212 / 172; halves of 32-bit activations (with their split and the sum) 200 x 6144 x 4096 46.8 / 39.8 (768 tiles of 64 x 128 on 512 places / 240 of 128 x 256 in five pieces), 256 52.9 / 43.2,
-// 443 x 6240 x 7488 130 / 109, gated 262 x 8192 x 7488 136 / 111.
-static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats, float rounds = 0.0f) {
+// rounds (one matrix): a second estimate has a CU's last tiles, where they are no whole number of `resident` ones, at the pace of a tile alone, and looks at five pieces where six put a second tile
+// on a CU.  `us` stays the first estimate's (the lines between these forms and others are drawn with it); the plan is the second one's where that has the same tile in fewer pieces, or is ahead by a
+// tenth.  Both plans were measured wherever they differ.  bfloat16, 1080 sizes of 9 .. 2000 rows: the same tile in fewer pieces takes 0.88 of the time on average and never more (150 x 2048 x 2048 in
+// five for eight 12.7 -> 10.7), a tenth ahead 0.94 (700 x 4096 x 14336 90 -> 80; 15 of 161 are behind by more than 2 %, half of those where 256 x 256 tiles replace two of 128 x 128 a CU, 9 % there and
+// 12 % at most); up to a twentieth ahead it is no better than chance, between the two 23 of 64 are behind, by up to 19 %.  Halves of 32-bit activations, 437 sizes (with their split and the sum):
+// 0.93 (2 of 24 behind, by 3 %) and 0.955 (6 of 147, 6 % at most); gated 0.90 (4 of 31, 5 %).  Before, where these plans were the first estimate's: 200 x 6144 x 4096 46.8 -> 39.8 (768 tiles of
+// 64 x 128 on 512 places / 240 of 128 x 256 in five pieces), gated bfloat16 1181 x 7488 x 7488 212 -> 172.
+static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int rows, int groups, int N, int K, long long scratch_floats, bool rounds = false) {
     static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
     TilePlan best{0, 1, 1e30f}, other = best;
     float best_too = 0.0f;                          // the second estimate of `best`
@@ -316,7 +317,7 @@ static TilePlan plan_direct(const DirectForm* f, int n_forms, int chunk, int row
             if ((s != 5 || tiles * 6.0f > 256.0f) && too < other.us) other = TilePlan{i, s, too};
         }
     }
-    if (rounds > 0.0f && other.us * rounds <= best_too) { best.form = other.form; best.splits = other.splits; }
+    if (rounds && ((other.form == best.form && other.splits < best.splits) || other.us * 1.1f <= best_too)) { best.form = other.form; best.splits = other.splits; }
     return best;
 }
 static void tell_plan(const DirectForm& f, const TilePlan& p, int* plan) { plan[0] = f.TM; plan[1] = f.TN; plan[2] = f.resident; plan[3] = p.splits; }

@@ -139,8 +139,8 @@ __global__ __launch_bounds__(1024) void half_norm_split_kernel(const HalfNormArg
 
 // two matrix instructions a product: constants as for bf16 (plan_direct), from 16 .. 200 rows, 1024 .. 28672 outputs, 4096 .. 14336 inputs
 static const DirectForm kFormsHalf[] = {{128, 256, 1, 1.65f, 1.65f, 12.0f, 0.6f}, {64, 128, 2, 0.82f, 0.495f, 5.0f, 0.0f}, {64, 64, 2, 0.47f, 0.315f, 4.0f, 0.0f}};
-static TilePlan plan_direct_half(int rows, int N, int K, long long room, bool gated = false) {
-    return plan_direct(kFormsHalf, 3, 64, rows, 1, N, K, room, gated ? 1.02f : 1.08f);
+static TilePlan plan_direct_half(int rows, int N, int K, long long room) {
+    return plan_direct(kFormsHalf, 3, 64, rows, 1, N, K, room, true);
 }
 template <int GLU>
 static int launch_direct_half(const DirectArgs& d, const TilePlan& p, hipStream_t s, bool sum = true) {
@@ -211,7 +211,7 @@ static int half_many(const ntk_half_desc* d, bool ready, ntk_gemm_partials* defe
         a.X16 = halves; a.x_row = (uint32_t)K * 2; a.plane = plane * 2;
         const long long left = (char*)d->workspace + d->workspace_bytes - behind;
         const long long room = d->silu || left < 0 ? 0 : left / (long long)sizeof(float);
-        const TilePlan p = plan_direct_half(n, (int)N, K, room, d->silu != 0);
+        const TilePlan p = plan_direct_half(n, (int)N, K, room);
         if (d->silu) {
             t.W = std::min(w0, w1); a.gate_at = (uint32_t)(w0 - (const char*)t.W); a.up_at = (uint32_t)(w1 - (const char*)t.W);
             a.glu_ff = d->out[0];
@@ -226,10 +226,10 @@ static int half_many(const ntk_half_desc* d, bool ready, ntk_gemm_partials* defe
     return last_launch_status();
 }
 int ntk_gemm_half_many(const ntk_half_desc* d, void* stream) { return half_many(d, false, nullptr, stream); }
-int ntk_gemm_half_plan(int rows, int N, int K, int gated, long long room, int* plan) {
+int ntk_gemm_half_plan(int rows, int N, int K, long long room, int* plan) {
     if (!plan) return NTK_E_NULL;
     if (rows <= 0 || N <= 0 || K <= 0) return NTK_E_SHAPE;
-    const TilePlan p = plan_direct_half(rows, N, K, room, gated != 0);
+    const TilePlan p = plan_direct_half(rows, N, K, room);
     tell_plan(kFormsHalf[p.form], p, plan);
     return NTK_OK;
 }

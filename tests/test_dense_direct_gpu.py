@@ -188,9 +188,10 @@ def test_gates_that_leave_rounded_rows(T, n, per_head):
         Lr.gate_rows_16(x, g, 3, 0)
 
 
-@pytest.mark.parametrize("T,N,K,tile", [(129, 2048, 2112, (64, 64, 3)), (70, 6240, 2560, (64, 128, 2)), (70, 6240, 4096, (128, 128, 1)), (200, 6144, 4096, (128, 128, 2))])
+@pytest.mark.parametrize("T,N,K,tile", [(20, 3264, 2112, (64, 64, 3)), (14, 12320, 4096, (64, 128, 2)), (65, 5504, 6464, (128, 128, 1)), (65, 10976, 6464, (128, 256, 1)),
+                                        (200, 5408, 6464, (256, 128, 1)), (129, 10976, 6464, (256, 256, 1))])
 def test_five_pieces_of_k_by_their_plans(T, N, K, tile):
-    """every tile that takes five pieces, chunks of 64 that they do not share evenly (33, 40 and 64): the plan is asked for, so that another choice does not leave the form untested"""
+    """every tile that takes five pieces, chunks of 64 that they do not share evenly (33, 64 and 101): the plan is asked for, so that another choice does not leave the form untested"""
     from ntransformer_amd import layers as Lr
     import ctypes as C
     plan, f = (C.c_int * 4)(), Lr._bind().ntk_dense_direct_plan
